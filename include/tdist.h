@@ -505,6 +505,28 @@ int tdist_decode_fused(const void* q, const void* k_cache, const void* v_cache, 
                        int64_t table_stride, int dtype, int32_t* counters, int64_t n_counters, void* out,
                        int out_dtype, int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream);
 
+/* Decode of a whole batch in ONE launch that divides the keys itself: the result of tdist_decode_split_kv followed by
+ * tdist_decode_combine(mode 1), without partial results for the caller to hold.
+ *   replaces gqa_fwd_batch_decode                   kernels/nvidia/flash_decode.py:763-844 (split-KV + combine launches,
+ *   a fixed number of splits for every sequence)
+ * All sequences' blocks of keys are laid end to end and cut into equal ranges, one per wave and kv head, so the time
+ * goes with the sum of the lengths, not with the longest, and a short sequence is not cut at all. out [B,Hq,Dv] of
+ * out_dtype (strides out_stride_b, out_stride_h); lse_out fp32 [B,Hq] or NULL; a sequence of length 0 gets out = 0,
+ * lse = -inf. counters as for tdist_decode_fused (all zero on entry, left zero). workspace: plain device memory,
+ * 16-byte aligned, of at least tdist_decode_stream_workspace_bytes() bytes (-1: bad sizes); its contents do not matter
+ * before or after the call. Calls that share counters or workspace must not overlap. Head dimensions as
+ * for tdist_decode_split_kv, except that (576,512) is taken only where the value is the first 512 columns of the key (the
+ * same pointer and strides: latent attention, which then reads every row once); TDIST_ERR_UNSUPPORTED otherwise: use the
+ * two calls. */
+int64_t tdist_decode_stream_workspace_bytes(int batch, int q_heads, int kv_heads, int head_dim, int head_dim_v);
+int tdist_decode_stream(const void* q, const void* k_cache, const void* v_cache, float sm_scale, float soft_cap,
+                        const int32_t* block_table, const int32_t* kv_lens, int batch, int q_heads, int kv_heads,
+                        int head_dim, int head_dim_v, int page_size, int64_t q_stride_b, int64_t q_stride_h,
+                        int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
+                        int64_t v_stride_token, int64_t v_stride_head, int64_t table_stride, int dtype, int32_t* counters,
+                        int64_t n_counters, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                        int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream);
+
 /* LSE-weighted merge of P partial results per (b,h) — used for the splits of one shard and for the
  * shards of several ranks:
  *   m = max_j lse[j];  w_j = exp(lse[j]-m);  out = sum_j w_j*part[j] / sum_j w_j;  lse_out = m + log(sum_j w_j)

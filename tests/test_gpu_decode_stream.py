@@ -1,0 +1,84 @@
+"""The decode that divides a batch's keys itself (tdist_decode_stream) against the exact closed form, at the lengths where
+its ranges begin and end: blocks of 16 and 32 keys, sequences without keys, more sequences than lanes, one long sequence
+among short ones (its partial results merged over many ranges), batches whose units do not fill a workgroup."""
+import pytest
+import torch
+
+from oracle import golden
+from tests.conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+ATOL = 2e-3
+
+LENS = {
+    "one": [1], "block edges": [15, 16, 17, 32, 33, 64, 65], "none among some": [0, 40, 0, 0, 100, 7, 0], "no keys at all": [0, 0, 0],
+    "one long": [5, 9000, 64, 1, 300], "more than lanes": [(37 * i) % 90 for i in range(150)],
+}
+
+
+def check(cuda, num_heads, dims, dtype, kv_lens, page, soft_cap, latent, seed):
+    from triton_dist.kernels.amd.flash_decode import decode_stream
+    dk, dv = dims
+    Hq, Hkv = num_heads
+    B = len(kv_lens)
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randn((B, Hq, dk), generator=g).to(dtype)
+    k, v, table = golden.make_paged_kv(B, max(max(kv_lens), 1), Hkv, dk, page, dtype, g, v_head_dim=dv)
+    kd, td, lens = k.to(cuda), table.to(cuda), torch.tensor(kv_lens, dtype=torch.int32, device=cuda)
+    if latent:
+        v, vd = k[..., :dv], kd[..., :dv]
+    else:
+        vd = v.to(cuda)
+    scale = dk**-0.5
+    counters = torch.zeros(8192, dtype=torch.int32, device=cuda)
+    exact, exact_lse = golden.decode_exact(q, k, v, kv_lens, table, scale, soft_cap)
+    live = ~torch.isinf(exact_lse)
+    first = None
+    for _ in range(2):   # twice on the same counters
+        out = torch.full((B, Hq, dv + 4), float("nan"), dtype=torch.float32, device=cuda)[..., :dv]
+        lse = torch.full((B, Hq), float("nan"), dtype=torch.float32, device=cuda)
+        decode_stream(q.to(cuda), kd, vd, lens, td, scale, soft_cap, out, lse, counters=counters)
+        torch.cuda.synchronize()
+        assert int(counters.abs().sum()) == 0
+        assert (out.cpu().double() - exact).abs().max() <= ATOL
+        assert torch.equal(torch.isinf(lse.cpu()), ~live)
+        assert not live.any() or (lse.cpu().double()[live] - exact_lse[live]).abs().max() <= ATOL
+        assert first is None or torch.equal(first, out)   # whoever arrives last, the sums run in order
+        first = out
+    out16 = torch.full((B, Hq, dv), float("nan"), dtype=dtype, device=cuda)
+    decode_stream(q.to(cuda), kd, vd, lens, td, scale, soft_cap, out16)
+    torch.cuda.synchronize()
+    assert torch.equal(out16, first.to(dtype))
+
+
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("num_heads,dims,dtype,page,soft_cap", [
+    ((32, 8), (128, 128), torch.bfloat16, 16, 0), ((6, 1), (128, 128), torch.float16, 1, 30), ((40, 2), (64, 64), torch.bfloat16, 16, 0),
+    ((16, 16), (192, 128), torch.float16, 16, 0), ((12, 3), (256, 256), torch.bfloat16, 1, 0), ((10, 5), (96, 96), torch.bfloat16, 16, 0),
+    ((8, 2), (40, 40), torch.float16, 16, 0), ((8, 8), (160, 160), torch.bfloat16, 16, 50)])
+def test_ranges_against_the_exact_result(cuda, num_heads, dims, dtype, page, soft_cap, lens):
+    announce("decode stream heads=%s dims=%s %s page=%d cap=%s lens: %s" % (num_heads, dims, dtype, page, soft_cap, lens))
+    check(cuda, num_heads, dims, dtype, LENS[lens], page, soft_cap, False, len(lens) + dims[0])
+
+
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("num_heads,dtype,page,soft_cap", [((128, 1), torch.bfloat16, 16, 0), ((24, 1), torch.float16, 1, 30), ((4, 2), torch.bfloat16, 16, 0)])
+def test_latent_heads_against_the_exact_result(cuda, num_heads, dtype, page, soft_cap, lens):
+    """576 / 512 with the value a view of the key's first 512 columns."""
+    announce("decode stream latent heads=%s %s page=%d cap=%s lens: %s" % (num_heads, dtype, page, soft_cap, lens))
+    check(cuda, num_heads, (576, 512), dtype, LENS[lens], page, soft_cap, True, len(lens))
+
+
+def test_workspace_and_head_dimensions_are_checked(cuda):
+    from triton_dist import _lib
+    lib = _lib.load()
+    need = lib.tdist_decode_stream_workspace_bytes(3, 32, 8, 128, 128)
+    assert need > 0 and lib.tdist_decode_stream_workspace_bytes(3, 32, 5, 128, 128) == -1
+    p = torch.zeros(4096, dtype=torch.uint8, device=cuda).data_ptr()
+
+    def call(dk, dv, v, nbytes):
+        return lib.tdist_decode_stream(p, p, v, 1.0, 0.0, p, p, 3, 32, 8, dk, dv, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, _lib.TDIST_BF16, p,
+                                       1024, p, nbytes, p, _lib.TDIST_BF16, 0, 0, None, None)
+    assert call(128, 128, p, need - 1) == _lib.TDIST_ERR_WORKSPACE
+    assert call(576, 512, p + 16, 1 << 40) == _lib.TDIST_ERR_UNSUPPORTED

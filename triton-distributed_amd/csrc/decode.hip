@@ -27,6 +27,7 @@
 //
 // HBM traffic per launch: every K and V row of the split once (len * Hkv * (Dk + Dv) * 2 B per sequence).
 #include <stdlib.h>
+#include <type_traits>
 
 #include "common.h"
 
@@ -68,6 +69,10 @@ struct DecodeParams {
   float* final_lse;          // [B,Hq] or null
   int final_dtype;
   int64_t fo_sb, fo_sh;      // element strides of final_out
+  int fo_vec;                // its rows take 8-byte (16-bit types) / 16-byte (fp32) stores
+  int part_vec;              // the partial results take 16-byte stores
+  // streaming form: ranges the batch's blocks are cut into at most, and the fewest blocks of a range
+  int ranges, min_blocks;
 };
 
 struct MmaBF16 {
@@ -103,6 +108,8 @@ struct MmaF16 {
 // kWaveHeads: splits one workgroup may stream through (the results of all but the last wait in registers: D / 4 each).
 // `heavy`: the instances that already fill their registers (soft cap, fused merge, padded rows).
 constexpr int decode_max_splits_per_team(int d, bool heavy) { return d <= 64 ? 4 : d <= 128 ? (heavy ? 3 : 4) : 2; }
+// a head's row of a wave's result on its way through the LDS
+constexpr int decode_acc_row(int d) { return d + 4; }
 constexpr int kTableSlots = 8;  // ring of page-table rows per wave (>= 2P+2)
 
 // what the DMA lanes of a padded head dimension read for the dimensions that do not exist
@@ -110,7 +117,8 @@ static __device__ __align__(16) const unsigned char kZeroChunk[16] = {0};
 
 // KEYS = keys per block (16 or 32): one or two groups of 16 keys, a group being one MFMA tile of scores.
 // DM = value dimension = power-of-two part of the key dimension; DPE = the extra key dimensions (0 or 64).
-template <int DM, int DPE, int KEYS, int NST>
+// kAlias: the value is the first DM columns of the key (latent attention): one row set serves both.
+template <int DM, int DPE, int KEYS, int NST, bool kAlias = false>
 struct DecodeCfg {
   static constexpr int kGroups = KEYS / 16;
   static constexpr int kRowBytes = DM * 2;
@@ -124,9 +132,10 @@ struct DecodeCfg {
   static constexpr int kPeRowsPerInstr = 64 / kPeLanesPerRow;
   static constexpr int kPeInstr = DPE > 0 ? KEYS / kPeRowsPerInstr : 0;
   static constexpr int kPeBytes = KEYS * kPeRowBytes;
-  static constexpr int kPeBase = 2 * kTensorBytes;
-  static constexpr int kStageBytes = 2 * kTensorBytes + kPeBytes;
-  static constexpr int kLoadsPerGroup = 1 + 2 * kInstrPerTensor + kPeInstr;  // table row + K + V (+ extra K)
+  static constexpr int kVBase = kAlias ? 0 : kTensorBytes;
+  static constexpr int kPeBase = kVBase + kTensorBytes;
+  static constexpr int kStageBytes = kPeBase + kPeBytes;
+  static constexpr int kLoadsPerGroup = 1 + (kAlias ? 1 : 2) * kInstrPerTensor + kPeInstr;  // table row + K + V (+ extra K)
   static constexpr int kP = NST - 1;
   // LDS position of 16-byte chunk c of a row: K rows c ^ kswz(key), V rows c ^ vswz(key).
   // K operand reads: 16 lanes = 16 keys, same chunk      → spread over 16 positions: key & 15.
@@ -150,8 +159,14 @@ struct DecodeCfg {
   // key needs a new XOR term.
   static constexpr int kRowsPerWindow = kRowBytes >= 256 ? 1 : 256 / kRowBytes;
   static constexpr int kPeRowsPerWindow = DPE > 0 ? 256 / kPeRowBytes : 1;
-  __device__ static __forceinline__ int kswz(int key) { return (key / kRowsPerWindow) & kSwzMask; }
-  __device__ static __forceinline__ int vswz(int key) { return (((key / kRowsPerWindow) & 7) << 1) & kSwzMask; }
+  // (one row set for both: 16 keys, 16 positions, and 8 neighbouring keys at 8 pairs of chunks)
+  static_assert(!kAlias || (kSwzMask == 15 && kRowsPerWindow == 1), "shared rows: at least a bank window long");
+  __device__ static __forceinline__ int kswz(int key) {
+    return kAlias ? ((key & 7) << 1) | ((key >> 3) & 1) : (key / kRowsPerWindow) & kSwzMask;
+  }
+  __device__ static __forceinline__ int vswz(int key) {
+    return kAlias ? kswz(key) : (((key / kRowsPerWindow) & 7) << 1) & kSwzMask;
+  }
   __device__ static __forceinline__ int peswz(int key) { return (key / kPeRowsPerWindow) & kPeSwzMask; }
 };
 
@@ -182,6 +197,175 @@ template <bool kCoherent>
 __device__ __forceinline__ void store_partial4(float* p, float4v v) {
   if constexpr (kCoherent) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
   else *(float4v*)p = v;
+}
+
+__device__ __forceinline__ float load_elem(const unsigned char* base, int64_t idx, int dtype) {
+  if (dtype == TDIST_F32) return ((const float*)base)[idx];
+  const uint32_t bits = ((const unsigned short*)base)[idx];
+  return dtype == TDIST_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+}
+__device__ __forceinline__ void store_elem(unsigned char* base, int64_t idx, int dtype, float v) {
+  if (dtype == TDIST_F32) ((float*)base)[idx] = v;
+  else if (dtype == TDIST_BF16) ((unsigned short*)base)[idx] = (unsigned short)f32_to_bf16_bits(v);
+  else ((unsigned short*)base)[idx] = (unsigned short)(pack_f16x2(v, 0.f) & 0xffffu);
+}
+// Four consecutive elements; `vec`: their address takes one store.
+__device__ __forceinline__ void store_elem4(unsigned char* base, int64_t idx, int dtype, int vec, float4v v) {
+  if (!vec) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) store_elem(base, idx + e, dtype, v[e]);
+  } else if (dtype == TDIST_F32) {
+    *(float4v*)(base + idx * 4) = v;
+  } else {
+    const int2v w = dtype == TDIST_BF16 ? int2v{(int)pack_bf16x2(v[0], v[1]), (int)pack_bf16x2(v[2], v[3])}
+                                        : int2v{(int)pack_f16x2(v[0], v[1]), (int)pack_f16x2(v[2], v[3])};
+    *(int2v*)(base + idx * 2) = w;
+  }
+}
+
+// Workgroup i of n runs on XCD i % 8: its place when the workgroups are counted XCD by XCD.
+__device__ __forceinline__ int xcd_major(int i, int n) {
+  const int x = i & 7, q = n >> 3, rest = n & 7;
+  return x * q + min(x, rest) + (i >> 3);
+}
+
+// ---- streaming form: which blocks a range holds -----------------------------------------------------------
+constexpr int kStreamMaxParts = 64;   // ranges one sequence may be spread over (a merge weighs them one per lane)
+
+struct StreamRange {
+  int n;            // blocks in the range (0: the batch has fewer ranges)
+  int seq, block;   // the sequence its first block belongs to, and that block's number in the sequence
+  int first_block;  // that sequence's first block, numbered over the whole batch
+  int per;          // blocks per range
+};
+
+// All sequences' blocks laid end to end and cut into ranges of `per` blocks: the same answer in every wave, from one
+// load per 64 sequences and a scan over the lanes.
+template <int KEYS>
+__device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int range) {
+  const int lane = threadIdx.x & 63;
+  auto blocks = [&](int i) { return i < prm.B ? (max(prm.lens[i], 0) + KEYS - 1) / KEYS : 0; };
+  int nb = 0, sum = 0, mx = 0, total = 0;
+  auto scan = [&](int i0) {   // sum: this lane's sequence and the ones before it within the 64
+    nb = blocks(i0 + lane);
+    sum = nb;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(sum, o);
+      if (lane >= o) sum += t;
+    }
+  };
+  for (int i0 = 0; i0 < prm.B; i0 += 64) {
+    scan(i0);
+    mx = max(mx, nb);
+    total += __builtin_amdgcn_readlane(sum, 63);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
+  mx = __builtin_amdgcn_readfirstlane(mx);
+  StreamRange r;
+  // even shares, but no shorter than min_blocks and no more than kStreamMaxParts ranges to a sequence (a sequence of
+  // n blocks touches at most ceil(n / per) + 1 ranges)
+  r.per = max(max((total + prm.ranges - 1) / prm.ranges, prm.min_blocks), (mx + kStreamMaxParts - 2) / (kStreamMaxParts - 1));
+  const long long g0 = (long long)range * r.per;
+  r.seq = r.block = r.first_block = 0;
+  if (g0 >= total) {
+    r.n = 0;
+    return r;
+  }
+  r.n = min(r.per, total - (int)g0);
+  int base = 0;
+  for (int i0 = 0;; i0 += 64) {
+    if (prm.B > 64) scan(i0);
+    const unsigned long long past = __ballot(base + sum > (int)g0);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      r.seq = i0 + at;
+      r.first_block = base + __builtin_amdgcn_readlane(sum, at) - __builtin_amdgcn_readlane(nb, at);
+      r.block = (int)g0 - r.first_block;
+      return r;
+    }
+    base += __builtin_amdgcn_readlane(sum, 63);
+  }
+}
+
+// The merge of one sequence's partial results for one block of up to 16 heads, by NW waves (all of their workgroup, or a
+// wave alone): partial j is that of range first + j (the second slot of the range in which the sequence begins, the first
+// slot of the others). A lane weighs head lane & 15 of every fourth partial; every wave works out all weights for itself
+// (the same values to the same places of the LDS, `s`: 16 x kStreamMaxParts floats), so none waits. Then kB partials' rows
+// and kV 16-byte pieces per lane are in flight together. The sums run over the partials in order.
+template <int NW>
+__device__ __forceinline__ void stream_merge(const DecodeParams& prm, int seq, int first, int parts, int h0, int nvalid,
+                                             int Dout, TDIST_AS3 float* s) {
+  const int lane = threadIdx.x & 63;
+  const int tid = NW == 1 ? lane : (int)threadIdx.x;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  auto row = [&](int j) { return ((int64_t)(first + j) * 2 + (j == 0 ? 1 : 0)) * prm.Hq + h0; };
+  {
+    constexpr int kPer = kStreamMaxParts / 4;
+    const int h = lane & 15, j0 = lane >> 4;
+    float l[kPer];
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int j = j0 + 4 * i;
+      l[i] = j < parts && h < nvalid ? prm.lse[row(j) + h] : -INFINITY;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) M = fmaxf(M, l[i]);
+    M = fmaxf(M, __shfl_xor(M, 16));
+    M = fmaxf(M, __shfl_xor(M, 32));
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      l[i] = l[i] == -INFINITY ? 0.f : __expf(l[i] - M);
+      L += l[i];
+    }
+    L += __shfl_xor(L, 16);
+    L += __shfl_xor(L, 32);
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) s[h * kStreamMaxParts + j0 + 4 * i] = l[i] * inv;
+    if (prm.final_lse && tid < nvalid) prm.final_lse[(int64_t)seq * prm.Hq + h0 + h] = L > 0.f ? M + logf(L) : -INFINITY;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int vecs = nvalid * Dout / 4, per_head = Dout / 4;
+  auto sum_rows = [&](auto kv, auto kb) {
+    constexpr int kV = decltype(kv)::value, kB = decltype(kb)::value;
+    for (int v0 = 0; v0 < vecs; v0 += 64 * NW * kV) {
+      float4v acc[kV];
+      int at[kV], h[kV];
+#pragma unroll
+      for (int v = 0; v < kV; ++v) {
+        acc[v] = float4v{0.f, 0.f, 0.f, 0.f};
+        at[v] = min(v0 + v * 64 * NW + tid, vecs - 1);
+        h[v] = at[v] / per_head;
+      }
+      for (int j0 = 0; j0 < parts; j0 += kB) {
+        float4v r[kB][kV];
+#pragma unroll
+        for (int u = 0; u < kB; ++u) {
+          const float4v* src = (const float4v*)(prm.out + row(min(j0 + u, parts - 1)) * Dout);
+#pragma unroll
+          for (int v = 0; v < kV; ++v) r[u][v] = src[at[v]];
+        }
+#pragma unroll
+        for (int u = 0; u < kB; ++u)
+#pragma unroll
+          for (int v = 0; v < kV; ++v) {
+            const float w = j0 + u < parts ? s[h[v] * kStreamMaxParts + j0 + u] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[v][e] += w * r[u][v][e];
+          }
+      }
+#pragma unroll
+      for (int v = 0; v < kV; ++v)
+        if (v0 + v * 64 * NW + tid < vecs)
+          store_elem4(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)(h0 + h[v]) * prm.fo_sh + (at[v] - h[v] * per_head) * 4,
+                      prm.final_dtype, prm.fo_vec, acc[v]);
+    }
+  };
+  if (vecs <= 64 * NW * 2) sum_rows(std::integral_constant<int, 2>{}, std::integral_constant<int, 16>{});
+  else sum_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{});
 }
 
 // Are the B sequence lengths even enough for the form that hands a workgroup 8 kv heads of one (sequence, split)?
@@ -224,9 +408,19 @@ __device__ __forceinline__ bool decode_lens_even(const int32_t* lens, int B) {
 // sharing one kv head's keys: together they read whole stretches of the token rows (NW * 2 * D bytes of every row) at
 // the same time, and no wave waits for another: each writes its own heads' results. For at most 16 query heads per kv
 // head and a number of kv heads that is a multiple of NW.
-template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kFuse, bool kPadded, bool kWaveHeads>
+// kStream: see decode_stream_kernel; a wave's kv head and its blocks come from its place in the grid.
+// kStreamGroup: see decode_stream_group_kernel; likewise for a workgroup, whose waves share the blocks (b, start and end
+// are then the segment at hand).
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kFuse, bool kPadded, bool kWaveHeads,
+          bool kStream = false, bool kStreamGroup = false>
 __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
-  typedef DecodeCfg<D, DPE, KEYS, NST> C;
+  constexpr bool kAlias = kStreamGroup;
+  // kStreamGroup: two waves work on the same blocks of keys and take half of the value dimensions each (their sums would
+  // not leave room for the query beside them in one wave's registers, and one wave per SIMD hides no latency)
+  constexpr int kHalves = kStreamGroup ? 2 : 1;
+  constexpr int NK = NW / kHalves;      // streams of keys
+  constexpr int DT = D / 16 / kHalves;  // tiles of 16 value dimensions per wave
+  typedef DecodeCfg<D, DPE, KEYS, NST, kAlias> C;
   constexpr int G = C::kGroups;
   constexpr int DK = D + DPE;  // key (and query) dimensions; D is the value dimension
   static_assert(!kPadded || DPE == 0, "padded rows have no extra key dimensions");
@@ -239,29 +433,56 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   const int group = prm.Hq / prm.Hkv;
   const int head_blocks = (group + 15) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform for the compiler too
+  const int half = kStreamGroup ? wave & 1 : 0;
+  const int kwave = wave / kHalves;
   const int lane = threadIdx.x & 63;
-  const int kvh = kWaveHeads ? blockIdx.x * NW + wave : blockIdx.x / head_blocks;
-  const int hb = kWaveHeads ? 0 : blockIdx.x - kvh * head_blocks;
-  const int b = blockIdx.z;
+  // kStream: heads vary fastest over the grid's waves, then the range of blocks
+  // (kStreamGroup: among the workgroups of one XCD, which so share the keys of a range in their L2)
+  const int unit = kStreamGroup ? xcd_major(blockIdx.x, gridDim.x) : blockIdx.x * NW + wave;
+  const int range = kStream || kStreamGroup ? unit / (prm.Hkv * head_blocks) : 0;
+  const int head_unit = kStream || kStreamGroup ? unit - range * prm.Hkv * head_blocks : blockIdx.x;
+  const int kvh = kWaveHeads ? blockIdx.x * NW + wave : head_unit / head_blocks;
+  const int hb = kWaveHeads ? 0 : head_unit - kvh * head_blocks;
+  int b = blockIdx.z;
   const int h0 = kvh * group + hb * 16;
   const int nvalid = min(16, group - hb * 16);
   // threads that share the work of one (kv head, head block): the workgroup, or the wave
-  const int team_tid = kWaveHeads ? lane : (int)threadIdx.x;
-  constexpr int kTeam = kWaveHeads ? 64 : NW * 64;
+  const int team_tid = kWaveHeads || kStream ? lane : (int)threadIdx.x;
+  constexpr int kTeam = kWaveHeads || kStream ? 64 : NW * 64;
   const int g = lane >> 4;   // lane group 0..3
   const int x = lane & 15;   // head (score column) / dv within tile (V^T row) / key (K row)
 
-  const int len = prm.lens[b];
+  StreamRange sr{};
+  if constexpr (kStream || kStreamGroup) {
+    sr = stream_range<KEYS>(prm, range);
+    for (int i0 = 0; range == 0 && i0 < prm.B; i0 += 64) {
+      // sequences without keys: out = 0, lse = -inf
+      unsigned long long none = __ballot(i0 + lane < prm.B && prm.lens[min(i0 + lane, prm.B - 1)] <= 0);
+      for (; none; none &= none - 1) {
+        const int seq = i0 + __builtin_ctzll(none);
+        for (int j = team_tid; j < nvalid * Dout; j += kTeam) {
+          const int h = j / Dout;
+          store_elem(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)(h0 + h) * prm.fo_sh + (j - h * Dout), prm.final_dtype, 0.f);
+        }
+        if (prm.final_lse && team_tid < nvalid) prm.final_lse[(int64_t)seq * prm.Hq + h0 + team_tid] = -INFINITY;
+      }
+    }
+    if (sr.n == 0) return;
+  }
+
+  // (the lengths through the scalar cache: a vector load would wait for the stream behind which it is queued)
+  const auto lens = (const __attribute__((address_space(4))) int32_t*)(uintptr_t)prm.lens;
+  const int len = kStream || kStreamGroup ? 0 : prm.lens[b];
   const int per = (len + prm.S - 1) / prm.S;
   // kWaveHeads: the team streams through splits split .. split + n_splits - 1 of its sequence, one after the other
   const int split = kWaveHeads ? blockIdx.y * prm.splits_per_team : blockIdx.y;
   const int n_splits = kWaveHeads ? min(prm.splits_per_team, prm.S - split) : 1;
-  const int start = per * split;
-  const int end = min(start + per, len);
+  int start = per * split;
+  int end = min(start + per, len);
 
   float* out_base = prm.out + (((int64_t)b * prm.Hq + h0) * prm.S + split) * Dout;
   float* lse_base = prm.lse + ((int64_t)b * prm.Hq + h0) * prm.S + split;
-  if (end <= start) {
+  if (!kStream && !kStreamGroup && end <= start) {
     // empty split (and with it every later one): zeros and LSE = -inf so that any merge gives it weight 0
     for (int sp = 0; sp < n_splits; ++sp) {
       for (int i = team_tid; i < nvalid * Dout; i += kTeam) {
@@ -276,14 +497,14 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   typedef TDIST_AS3 unsigned char* lds_u8;  // explicit LDS pointers: a generic pointer would turn reads into
                                             // flat loads, which count on vmcnt and break the DMA accounting
   lds_u8 const smem3 = (lds_u8)smem;
-  lds_u8 const wbase = smem3 + wave * C::kWaveBytes;
+  lds_u8 const wbase = smem3 + kwave * C::kWaveBytes;
   lds_u8 const tbl_base = wbase + NST * C::kStageBytes;
 
   const int nb_total = (end - start + KEYS - 1) / KEYS;
   // this wave's blocks: every NW-th one of the kv head's; or all of its own kv head's, split after split (an empty
   // split at the sequence's end runs one block with every key masked, which writes its zeros)
   auto blocks_of = [&](int lo, int hi) { return max(1, (hi - lo + KEYS - 1) / KEYS); };
-  int n_w = nb_total > wave ? (nb_total - wave + NW - 1) / NW : 0;
+  int n_w = nb_total > kwave ? (nb_total - kwave + NK - 1) / NK : 0;
   if constexpr (kWaveHeads) {
     n_w = 0;
     for (int sp = 0; sp < n_splits; ++sp) n_w += blocks_of(start + sp * per, min(start + (sp + 1) * per, len));
@@ -291,63 +512,79 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
 
   // ---- Q fragments (B operand of the score MFMA): head x, dims 32s + 8g .. +8 -------------------
   typename MMA::frag8 qf[DK / 32];
-  {
-    const unsigned char* qrow = prm.q + (int64_t)b * prm.q_sb + (int64_t)(h0 + x) * prm.q_sh;
+  auto load_q = [&](int seq) {
+    const unsigned char* qrow = prm.q + (int64_t)seq * prm.q_sb + (int64_t)(h0 + x) * prm.q_sh;
 #pragma unroll
     for (int s = 0; s < DK / 32; ++s) {
       int4v raw = {0, 0, 0, 0};
       if (x < nvalid && (!kPadded || 4 * s + g < valid_chunks)) raw = *(const int4v*)(qrow + (32 * s + 8 * g) * 2);
       qf[s] = __builtin_bit_cast(typename MMA::frag8, raw);
     }
-  }
+    // Waited for here: a query fetched inside the stream would otherwise be waited for at every use in the loop, and
+    // with it (loads count in order) the whole stream behind it.
+    if constexpr (kStream || kStreamGroup) {
+#pragma unroll
+      for (int s = 0; s < DK / 32; ++s) {
+        int4v raw = __builtin_bit_cast(int4v, qf[s]);
+        asm volatile("" : "+v"(raw));
+        qf[s] = __builtin_bit_cast(typename MMA::frag8, raw);
+      }
+    }
+  };
+  if constexpr (!kStreamGroup && !kStream) load_q(b);
 
   constexpr float kLog2e = 1.4426950408889634f;
   const float scale_log2 = prm.sm_scale * kLog2e;
 
   float m_run = -INFINITY;  // running max (log2 domain) of head x, identical in the 4 lane groups
   float l_run = 0.f;        // this lane group's share of the running sum
-  float4v acc[D / 16];
+  float4v acc[DT];
 #pragma unroll
-  for (int d = 0; d < D / 16; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < DT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  // Loop-invariant LDS offsets (relative to the stage) of this lane's operand reads.
+  // Loop-invariant LDS offsets (relative to the stage) of this lane's operand reads. The swizzle moves a chunk within
+  // a window of kSwzMask + 1 chunks only, so the windows of a longer row share their offsets.
   // K (A operand of the scores): row = key x of group q, logical chunk 4s+g.
   // The extra key dimensions D + 32s' + 8g live in their own rows behind the K and V rows.
-  int koff[G][DK / 32];
+  constexpr int kWinChunks = C::kSwzMask + 1, kWinBytes = kWinChunks * 16;
+  constexpr int kKWin = kWinChunks / 4 < D / 32 ? kWinChunks / 4 : D / 32, kVWin = kWinChunks / 2 < DT ? kWinChunks / 2 : DT;
+  int koff[G][kKWin], peoff[G][DPE > 0 ? DPE / 32 : 1];
 #pragma unroll
-  for (int q = 0; q < G; ++q)
+  for (int q = 0; q < G; ++q) {
+    const int key = 16 * q + x;
 #pragma unroll
-    for (int s = 0; s < DK / 32; ++s) {
-      const int key = 16 * q + x;
-      if (s < D / 32) koff[q][s] = key * C::kRowBytes + (((4 * s + g) ^ C::kswz(key)) << 4);
-      else koff[q][s] = C::kPeBase + key * C::kPeRowBytes + (((4 * (s - D / 32) + g) ^ C::peswz(key)) << 4);
-    }
+    for (int s = 0; s < kKWin; ++s) koff[q][s] = key * C::kRowBytes + (((4 * s + g) ^ C::kswz(key)) << 4);
+#pragma unroll
+    for (int s = 0; s < DPE / 32; ++s) peoff[q][s] = C::kPeBase + key * C::kPeRowBytes + (((4 * s + g) ^ C::peswz(key)) << 4);
+  }
+  auto k_at = [&](int q, int s) { return s < D / 32 ? koff[q][s % kKWin] + s / kKWin * kWinBytes : peoff[q][s - D / 32]; };
   // V^T (A operand of the output MFMA) through the transposing LDS read: within a 16-lane block, lane x ends
   // up with elements x, 16+x, 32+x, 48+x of the 64 the block loads (lane s loads 4 consecutive ones), so lane s
   // supplies V[key 4g + s/4 of group q][dv 16d + 4(s%4) .. +3] and lane x receives V[4g+j][16d+x], j = 0..3.
-  int voff[G][D / 16];
+  int voff[G][kVWin];
 #pragma unroll
   for (int q = 0; q < G; ++q)
 #pragma unroll
-    for (int d = 0; d < D / 16; ++d) {
+    for (int d = 0; d < kVWin; ++d) {
       const int key = 16 * q + 4 * g + (x >> 2);
       const int chunk = 2 * d + ((x & 3) >> 1);
-      voff[q][d] = C::kTensorBytes + key * C::kRowBytes + ((chunk ^ C::vswz(key)) << 4) + (x & 1) * 8;
+      voff[q][d] = C::kVBase + half * DT * 32 + key * C::kRowBytes + ((chunk ^ C::vswz(key)) << 4) + (x & 1) * 8;
     }
+  static_assert(kHalves == 1 || (DT * 32) % kWinBytes == 0, "a half begins on a window");
 
   // A block: its first key and the key range [lo, hi) of its split. Keys outside the range are read as the nearest
   // key inside (and, for a split that is empty, as the sequence's last key) and masked in the scores.
-  struct Block { int key0, lo, hi; };
+  struct Block { int key0, lo, hi, seq; };
   auto clamp_key = [&](int n, const Block& blk) {
     n = max(min(n, blk.hi - 1), blk.lo);
     if constexpr (kWaveHeads) n = min(n, len - 1);
     return n;
   };
   // first key of the wave's j-th block where the workgroup shares one split
-  auto shared_block = [&](int j) { return Block{start + (wave + j * NW) * KEYS, start, end}; };
+  auto shared_block = [&](int j) { return Block{start + (kwave + j * NK) * KEYS, start, end, b}; };
   // kWaveHeads: a cursor over the team's blocks in order
   struct Cursor { Block blk; int left; };   // left: blocks of this split still to come, this one included
-  auto cursor_begin = [&]() { return Cursor{Block{start, start, end}, blocks_of(start, end)}; };
+  auto cursor_begin = [&]() { return Cursor{Block{start, start, end, b}, blocks_of(start, end)}; };
   auto cursor_next = [&](Cursor& c) {
     c.blk.key0 += KEYS;
     if (--c.left == 0) {
@@ -363,68 +600,127 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     if (lane < KEYS) {
       const int n = clamp_key(blk.key0 + lane, blk);
       const int e = (int)(((uint64_t)(uint32_t)n * prm.page_magic) >> prm.page_shift);
-      const int32_t* src = prm.table + (int64_t)b * prm.t_s + e;
+      const int32_t* src = prm.table + (int64_t)(kStream ? blk.seq : b) * prm.t_s + e;
       __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)src,
                                        (TDIST_AS3 void*)(tbl_base + (j % kTableSlots) * C::kTableSlotBytes), 4, 0, 0);
     }
   };
 
+  // (rows that the head blocks of a range fetch one after the other are worth keeping in the L2)
+  constexpr int kAux = kStreamGroup ? 0 : TDIST_KV_AUX;
   // K and V rows of block j → stage j % NST
+  // The byte offset of a row within its cache (page, place in the page, head) is worked out once per block, by one lane
+  // per row (K rows in lanes 0 .. KEYS-1, V rows in the next KEYS), and handed to the lanes that fetch the row's chunks.
   auto issue_rows = [&](int j, const Block& blk) {
-    const int key0 = blk.key0;
     const volatile TDIST_AS3 int32_t* tbl =
         (const volatile TDIST_AS3 int32_t*)(tbl_base + (j % kTableSlots) * C::kTableSlotBytes);
     lds_u8 const kst = wbase + (j % NST) * C::kStageBytes;
-    lds_u8 const vst = kst + C::kTensorBytes;
-    const int chunk = lane % C::kLanesPerRow;
-#pragma unroll
-    for (int i = 0; i < C::kInstrPerTensor; ++i) {
-      const int key = i * C::kRowsPerInstr + lane / C::kLanesPerRow;
-      const int n = clamp_key(key0 + key, blk);
-      const uint32_t page = (uint32_t)tbl[key];
-      const uint32_t in_page = (uint32_t)n - (uint32_t)(((uint64_t)(uint32_t)n * prm.page_magic) >> prm.page_shift) * (uint32_t)prm.page_size;
-      const unsigned char* ksrc = prm.k + (uint64_t)page * (uint64_t)prm.k_sp +
-                                  (in_page * (uint32_t)prm.k_st + (uint32_t)kvh * (uint32_t)prm.k_sh + ((chunk ^ C::kswz(key)) << 4));
-      const unsigned char* vsrc = prm.v + (uint64_t)page * (uint64_t)prm.v_sp +
-                                  (in_page * (uint32_t)prm.v_st + (uint32_t)kvh * (uint32_t)prm.v_sh + ((chunk ^ C::vswz(key)) << 4));
-      if constexpr (kPadded) {
-        if ((chunk ^ C::kswz(key)) >= valid_chunks) ksrc = kZeroChunk;
-        if ((chunk ^ C::vswz(key)) >= valid_chunks) vsrc = kZeroChunk;
-      }
-      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)ksrc, (TDIST_AS3 void*)(kst + i * 1024), 16, 0, TDIST_KV_AUX);
-      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)vsrc, (TDIST_AS3 void*)(vst + i * 1024), 16, 0, TDIST_KV_AUX);
+    lds_u8 const vst = kst + C::kVBase;
+    uint32_t off_lo, off_hi;
+    {
+      const int row = lane & (KEYS - 1);
+      const bool is_v = !kAlias && (lane & KEYS) != 0;
+      const uint32_t n = (uint32_t)clamp_key(blk.key0 + row, blk);
+      const uint32_t in_page = n - (uint32_t)(((uint64_t)n * prm.page_magic) >> prm.page_shift) * (uint32_t)prm.page_size;
+      const uint64_t off = (uint64_t)(uint32_t)tbl[row] * (uint64_t)(is_v ? prm.v_sp : prm.k_sp) +
+                           (in_page * (uint32_t)(is_v ? prm.v_st : prm.k_st) + (uint32_t)kvh * (uint32_t)(is_v ? prm.v_sh : prm.k_sh));
+      off_lo = (uint32_t)off;
+      off_hi = (uint32_t)(off >> 32);
     }
-    if constexpr (DPE > 0) {
-      lds_u8 const pst = kst + C::kPeBase;
-      const int pchunk = lane % C::kPeLanesPerRow;
+    // `row`: which lane's offset; the same for the whole wave where a row takes a whole instruction
+    auto row_offset = [&](int row, bool uniform) -> uint64_t {
+      const uint32_t lo = uniform ? __builtin_amdgcn_readlane(off_lo, row) : (uint32_t)__shfl((int)off_lo, row);
+      const uint32_t hi = uniform ? __builtin_amdgcn_readlane(off_hi, row) : (uint32_t)__shfl((int)off_hi, row);
+      return ((uint64_t)hi << 32) | lo;
+    };
+    constexpr bool kWholeRow = C::kRowsPerInstr == 1;
+    constexpr int kInstr = C::kInstrPerTensor / kHalves, kPe = C::kPeInstr / kHalves;
+    const int chunk = lane % C::kLanesPerRow, pchunk = lane % C::kPeLanesPerRow;
+    // all exchanges between lanes first, then the loads: the compiler would wait for each exchange at its load
+    uint64_t k_off[kInstr], v_off[kInstr], pe_off[kPe > 0 ? kPe : 1];
 #pragma unroll
-      for (int i = 0; i < C::kPeInstr; ++i) {
-        const int key = i * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow;
-        const int n = clamp_key(key0 + key, blk);
-        const uint32_t page = (uint32_t)tbl[key];
-        const uint32_t in_page = (uint32_t)n - (uint32_t)(((uint64_t)(uint32_t)n * prm.page_magic) >> prm.page_shift) * (uint32_t)prm.page_size;
-        const unsigned char* psrc = prm.k + (uint64_t)page * (uint64_t)prm.k_sp +
-                                    (in_page * (uint32_t)prm.k_st + (uint32_t)kvh * (uint32_t)prm.k_sh +
-                                     (uint32_t)(C::kRowBytes + ((pchunk ^ C::peswz(key)) << 4)));
-        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)psrc, (TDIST_AS3 void*)(pst + i * 1024), 16, 0, TDIST_KV_AUX);
+    for (int u = 0; u < kInstr; ++u) {
+      const int key = kWholeRow ? u * kHalves + half : (u * kHalves + half) * C::kRowsPerInstr + lane / C::kLanesPerRow;
+      k_off[u] = row_offset(key, kWholeRow);
+      if constexpr (!kAlias) v_off[u] = row_offset(KEYS + key, kWholeRow);
+    }
+#pragma unroll
+    for (int u = 0; u < kPe; ++u) pe_off[u] = row_offset((u * kHalves + half) * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow, false);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kInstr; ++u) {
+      const int i = u * kHalves + half;
+      const int key = kWholeRow ? i : i * C::kRowsPerInstr + lane / C::kLanesPerRow;
+      const int kchunk = chunk ^ C::kswz(key), vchunk = chunk ^ C::vswz(key);
+      const unsigned char* ksrc = prm.k + k_off[u] + (uint32_t)(kchunk << 4);
+      if (kPadded && kchunk >= valid_chunks) ksrc = kZeroChunk;
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)ksrc, (TDIST_AS3 void*)(kst + i * 1024), 16, 0, kAux);
+      if constexpr (!kAlias) {
+        const unsigned char* vsrc = prm.v + v_off[u] + (uint32_t)(vchunk << 4);
+        if (kPadded && vchunk >= valid_chunks) vsrc = kZeroChunk;
+        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)vsrc, (TDIST_AS3 void*)(vst + i * 1024), 16, 0, kAux);
       }
+    }
+#pragma unroll
+    for (int u = 0; u < kPe; ++u) {
+      const int i = u * kHalves + half;
+      const int key = i * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow;
+      const unsigned char* psrc = prm.k + pe_off[u] + (uint32_t)(C::kRowBytes + ((pchunk ^ C::peswz(key)) << 4));
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)psrc, (TDIST_AS3 void*)(kst + C::kPeBase + i * 1024), 16, 0, kAux);
     }
   };
 
   auto compute = [&](int j, const Block& blk) {
     const int key0 = blk.key0;
     lds_u8 const st = wbase + (j % NST) * C::kStageBytes;
+    // Operand reads run kAhead tiles ahead of their products: two groups of registers in turn.
     // scores: A = K rows (key x of group q, dims 32s+8g..), B = Q  →  sc[q][i]: key 16q+4g+i, head x
+    constexpr int kAhead = 4;
+    static_assert(DT % kAhead == 0 && kAhead * G < 16, "whole groups of tiles; lgkmcnt counts to 15");
     float4v sc[G];
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       sc[q] = float4v{0.f, 0.f, 0.f, 0.f};
+      int4v kb[2][kAhead];
+      auto read_k = [&](int s0, int4v(&to)[kAhead]) {
 #pragma unroll
-      for (int s = 0; s < DK / 32; ++s) {
-        const int4v raw = *(const TDIST_AS3 int4v*)(st + koff[q][s]);
-        sc[q] = MMA::mma32(__builtin_bit_cast(typename MMA::frag8, raw), qf[s], sc[q]);
+        for (int u = 0; u < kAhead; ++u)
+          if (s0 + u < DK / 32) to[u] = *(const TDIST_AS3 int4v*)(st + k_at(q, s0 + u));
+      };
+      read_k(0, kb[0]);
+#pragma unroll
+      for (int s0 = 0; s0 < DK / 32; s0 += kAhead) {
+        if (s0 + kAhead < DK / 32) read_k(s0 + kAhead, kb[(s0 / kAhead + 1) & 1]);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+          if (s0 + u < DK / 32) sc[q] = MMA::mma32(__builtin_bit_cast(typename MMA::frag8, kb[(s0 / kAhead) & 1][u]), qf[s0 + u], sc[q]);
       }
     }
+    // (the first V tiles are on their way while the probabilities are worked out)
+    // The transposing reads and the waits for them are written out: for the builtin the compiler waits until every load
+    // into the LDS is done, the ones in flight for later blocks included.
+    int2v vb[2][kAhead][G];
+    const uint32_t v_base = (uint32_t)(uintptr_t)st;
+    auto read_v = [&](int d0, int2v(&to)[kAhead][G]) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+          if (d0 + u < DT)
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
+                         : "=v"(to[u][q])
+                         : "v"(v_base + (uint32_t)voff[q][(d0 + u) % kVWin]), "n"((d0 + u) / kVWin * kWinBytes)
+                         : "memory");
+    };
+    auto wait_v = [&](int later, int2v(&of)[kAhead][G]) {   // all but the `later` youngest LDS reads are back
+      if (later == 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kAhead * G) : "memory");
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+        for (int q = 0; q < G; ++q) asm volatile("" : "+v"(of[u][q]));
+    };
+    read_v(0, vb[0]);
     float t[G][4];
     float mx = -INFINITY;
 #pragma unroll
@@ -441,14 +737,18 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
         t[q][i] = valid ? v : -INFINITY;
         mx = fmaxf(mx, t[q][i]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float m_new = fmaxf(m_run, mx);
-    if (__any(m_new > m_run)) {
+    // The sums are kept relative to m_run, which is raised only when a score lies kSlack above it: their values then stay
+    // below 2^kSlack, which costs no precision, and the lanes of a head compare notes and the sums are rescaled a few
+    // times per stream instead of per block.
+    constexpr float kSlack = 8.f;
+    if (__any(mx > m_run + kSlack)) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float m_new = fmaxf(m_run, mx);
       const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
 #pragma unroll
-      for (int d = 0; d < D / 16; ++d) acc[d] *= alpha;
+      for (int d = 0; d < DT; ++d) acc[d] *= alpha;
       m_run = m_new;
     }
     const float m_safe = (m_run == -INFINITY) ? 0.f : m_run;
@@ -467,29 +767,162 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     }
     // O^T tiles: A = V^T (dv 16d+x; k slots as above), B = P^T
 #pragma unroll
-    for (int d = 0; d < D / 16; ++d) {
-      if (G == 2) {
-        const short4v v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TDIST_AS3 short4v*)(st + voff[0][d]));
-        const short4v v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TDIST_AS3 short4v*)(st + voff[G - 1][d]));
-        const int2v a0 = __builtin_bit_cast(int2v, v0), a1 = __builtin_bit_cast(int2v, v1);
-        const int4v vt = {a0[0], a0[1], a1[0], a1[1]};
-        const int4v ph = {(int)hi[0][0], (int)hi[0][1], (int)hi[G - 1][0], (int)hi[G - 1][1]};
-        const int4v pl = {(int)lo[0][0], (int)lo[0][1], (int)lo[G - 1][0], (int)lo[G - 1][1]};
-        const typename MMA::frag8 vf = __builtin_bit_cast(typename MMA::frag8, vt);
-        acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, ph), acc[d]);
-        acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, pl), acc[d]);
-      } else {
-        const short4v v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TDIST_AS3 short4v*)(st + voff[0][d]));
-        const int2v ph = {(int)hi[0][0], (int)hi[0][1]};
-        const int2v pl = {(int)lo[0][0], (int)lo[0][1]};
-        const typename MMA::frag4 vf = __builtin_bit_cast(typename MMA::frag4, v0);
-        acc[d] = MMA::mma16(vf, __builtin_bit_cast(typename MMA::frag4, ph), acc[d]);
-        acc[d] = MMA::mma16(vf, __builtin_bit_cast(typename MMA::frag4, pl), acc[d]);
+    for (int d0 = 0; d0 < DT; d0 += kAhead) {
+      if (d0 + kAhead < DT) read_v(d0 + kAhead, vb[(d0 / kAhead + 1) & 1]);
+      wait_v(d0 + kAhead < DT ? 1 : 0, vb[(d0 / kAhead) & 1]);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int d = d0 + u;
+        const auto& v = vb[(d0 / kAhead) & 1][u];
+        if constexpr (G == 2) {
+          const int2v a0 = v[0], a1 = v[G - 1];
+          const int4v vt = {a0[0], a0[1], a1[0], a1[1]};
+          const int4v ph = {(int)hi[0][0], (int)hi[0][1], (int)hi[G - 1][0], (int)hi[G - 1][1]};
+          const int4v pl = {(int)lo[0][0], (int)lo[0][1], (int)lo[G - 1][0], (int)lo[G - 1][1]};
+          const typename MMA::frag8 vf = __builtin_bit_cast(typename MMA::frag8, vt);
+          acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, ph), acc[d]);
+          acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, pl), acc[d]);
+        } else if constexpr (kAlias) {
+          // both halves of the probabilities in one product over 32 k slots: the same 4 keys of a lane twice
+          const int2v a0 = v[0];
+          const int4v vt = {a0[0], a0[1], a0[0], a0[1]};
+          const int4v p4 = {(int)hi[0][0], (int)hi[0][1], (int)lo[0][0], (int)lo[0][1]};
+          acc[d] = MMA::mma32(__builtin_bit_cast(typename MMA::frag8, vt), __builtin_bit_cast(typename MMA::frag8, p4), acc[d]);
+        } else {
+          const int2v ph = {(int)hi[0][0], (int)hi[0][1]};
+          const int2v pl = {(int)lo[0][0], (int)lo[0][1]};
+          const typename MMA::frag4 vf = __builtin_bit_cast(typename MMA::frag4, v[0]);
+          acc[d] = MMA::mma16(vf, __builtin_bit_cast(typename MMA::frag4, ph), acc[d]);
+          acc[d] = MMA::mma16(vf, __builtin_bit_cast(typename MMA::frag4, pl), acc[d]);
+        }
       }
     }
   };
 
   constexpr float kLn2 = 0.6931471805599453f;
+  if constexpr (kStream) {
+    static_assert(!C::kWaitFirst, "a kv head per wave: several groups in flight");
+    // One pipeline over the range's blocks, across the sequences in it.
+    struct Walk { Block blk; int left, rem; };   // left / rem: blocks of this sequence / of the range, this one included
+    auto walk_begin = [&]() {
+      const int hi = lens[sr.seq];
+      return Walk{Block{sr.block * KEYS, 0, hi, sr.seq}, min((hi + KEYS - 1) / KEYS - sr.block, sr.n), sr.n};
+    };
+    auto walk_next = [&](Walk& w) {   // (stays on the last block)
+      if (w.rem == 1) return;
+      --w.rem;
+      w.blk.key0 += KEYS;
+      if (--w.left == 0) {
+        do w.blk.hi = lens[++w.blk.seq];
+        while (w.blk.hi <= 0);
+        w.blk.key0 = 0;
+        w.left = min((w.blk.hi + KEYS - 1) / KEYS, w.rem);
+      }
+    };
+    Walk w_tbl = walk_begin(), w_rows = w_tbl, w_cmp = w_tbl;
+    int j_tbl = 0;
+    for (; j_tbl <= C::kP; ++j_tbl) {
+      issue_table(j_tbl, w_tbl.blk);
+      walk_next(w_tbl);
+    }
+    load_q(sr.seq);   // (one trip to memory with the page-table rows)
+    wait_vmcnt<0>();
+    for (int gi = 0; gi < C::kP; ++gi) {
+      if (gi < sr.n) {
+        issue_table(j_tbl++, w_tbl.blk);
+        walk_next(w_tbl);
+        issue_rows(gi, w_rows.blk);
+        walk_next(w_rows);
+      }
+    }
+    // The range's first sequence may have begun in an earlier range (its partial result waits in registers for the
+    // end of the stream) and its last may go on in the next one; all between are whole and stored when they end.
+    bool begun_here = sr.block == 0;
+    int seq_first = sr.first_block;   // global number of the current sequence's first block
+    float4v held[DT];
+    float held_lse = 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) held[d] = float4v{0.f, 0.f, 0.f, 0.f};
+    int part_seq[2] = {-1, -1}, part_first[2] = {0, 0};
+    auto part_row = [&](int rg, int slot) { return ((int64_t)rg * 2 + slot) * prm.Hq + h0; };
+    auto store_part = [&](int slot, const float4v(&val)[DT], float val_lse) {
+      if (x < nvalid) {
+        float* o = prm.out + (part_row(range, slot) + x) * Dout + 4 * g;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+          if (!kPadded || 16 * d + 4 * g < Dout) store_partial4<true>(o + 16 * d, val[d]);
+        if (g == 0) store_partial<true>(prm.lse + part_row(range, slot) + x, val_lse);
+      }
+    };
+    for (int i = 0; i < sr.n; ++i) {
+      if (i + C::kP < sr.n) {
+        issue_table(j_tbl++, w_tbl.blk);
+        walk_next(w_tbl);
+        issue_rows(i + C::kP, w_rows.blk);
+        walk_next(w_rows);
+      }
+      wait_groups<C::kLoadsPerGroup>(min(C::kP, sr.n - 1 - i));
+      compute(i, w_cmp.blk);
+      if (w_cmp.left == 1) {
+        float L = l_run + __shfl_xor(l_run, 16);
+        L += __shfl_xor(L, 32);
+        const float inv = L > 0.f ? 1.f / L : 0.f;
+        const float r_lse = L > 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
+        const bool ends = w_cmp.blk.key0 + KEYS >= w_cmp.blk.hi;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) acc[d] *= inv;
+        if (begun_here && ends) {
+          if (x < nvalid) {
+            const int64_t o = (int64_t)w_cmp.blk.seq * prm.fo_sb + (int64_t)(h0 + x) * prm.fo_sh + 4 * g;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+              if (!kPadded || 16 * d + 4 * g < Dout) store_elem4(prm.final_out, o + 16 * d, prm.final_dtype, prm.fo_vec, acc[d]);
+            if (prm.final_lse && g == 0) prm.final_lse[(int64_t)w_cmp.blk.seq * prm.Hq + h0 + x] = r_lse;
+          }
+        } else {
+          const int slot = begun_here ? 1 : 0;
+          part_seq[slot] = w_cmp.blk.seq;
+          part_first[slot] = seq_first;
+          if (i == sr.n - 1) {
+            store_part(slot, acc, r_lse);
+          } else {
+            held_lse = r_lse;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) held[d] = acc[d];
+          }
+        }
+        if (i < sr.n - 1) {
+          seq_first += (w_cmp.blk.hi + KEYS - 1) / KEYS;
+          begun_here = true;
+          m_run = -INFINITY;
+          l_run = 0.f;
+#pragma unroll
+          for (int d = 0; d < DT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
+          walk_next(w_cmp);
+          load_q(w_cmp.blk.seq);
+          continue;
+        }
+      }
+      walk_next(w_cmp);
+    }
+    if (part_seq[0] >= 0 && w_cmp.blk.seq != part_seq[0]) store_part(0, held, held_lse);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the partial results are where every XCD sees them
+#pragma unroll
+    for (int slot = 0; slot < 2; ++slot) {
+      if (part_seq[slot] < 0) continue;
+      const int seq = part_seq[slot];
+      const int nb = (lens[seq] + KEYS - 1) / KEYS;
+      const int first = part_first[slot] / sr.per, parts = (part_first[slot] + nb - 1) / sr.per - first + 1;
+      int32_t* const ctr = prm.counters + ((int64_t)seq * prm.Hkv + kvh) * head_blocks + hb;
+      int last = 0;
+      if (lane == 0) {
+        last = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (__builtin_amdgcn_readfirstlane(last)) stream_merge<1>(prm, seq, first, parts, h0, nvalid, Dout, (TDIST_AS3 float*)wbase);
+    }
+    return;
+  }
   if constexpr (kWaveHeads) {
     static_assert(!C::kWaitFirst, "a kv head per wave: several groups in flight");
     // One pipeline over all blocks of the team's splits: the loads of the next split's first blocks are in flight
@@ -512,13 +945,13 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     }
     // results of the splits before the team's last one, held until the stream ends
     constexpr int kMaxHeld = decode_max_splits_per_team(D, kSoftCap || kFuse || kPadded) - 1;
-    float4v held[kMaxHeld][D / 16];
+    float4v held[kMaxHeld][DT];
     float held_lse[kMaxHeld];
 #pragma unroll
     for (int u = 0; u < kMaxHeld; ++u) {
       held_lse[u] = 0.f;
 #pragma unroll
-      for (int d = 0; d < D / 16; ++d) held[u][d] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int d = 0; d < DT; ++d) held[u][d] = float4v{0.f, 0.f, 0.f, 0.f};
     }
     int sp = 0;
     for (int i = 0; i < n_w; ++i) {
@@ -534,17 +967,17 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
         // the split's last block: this lane holds dimensions 16d + 4g .. + 3 of head x
         float L = l_run + __shfl_xor(l_run, 16);
         L += __shfl_xor(L, 32);
-        float4v r[D / 16];
+        float4v r[DT];
 #pragma unroll
-        for (int d = 0; d < D / 16; ++d)
+        for (int d = 0; d < DT; ++d)
 #pragma unroll
           for (int e = 0; e < 4; ++e) r[d][e] = L > 0.f ? acc[d][e] / L : 0.f;
         const float r_lse = L > 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
-        auto store_split = [&](int which, const float4v(&val)[D / 16], float val_lse) {
+        auto store_split = [&](int which, const float4v(&val)[DT], float val_lse) {
           if (x < nvalid) {
             float* o = out_base + ((int64_t)x * prm.S + which) * Dout + 4 * g;
 #pragma unroll
-            for (int d = 0; d < D / 16; ++d)
+            for (int d = 0; d < DT; ++d)
               if (!kPadded || 16 * d + 4 * g < Dout) store_partial4<kFuse>(o + 16 * d, val[d]);
             if (g == 0) store_partial<kFuse>(lse_base + (int64_t)x * prm.S + which, val_lse);
           }
@@ -563,7 +996,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
           for (int u = 0; u < kMaxHeld; ++u)
             if (sp == u) {
 #pragma unroll
-              for (int d = 0; d < D / 16; ++d) held[u][d] = r[d];
+              for (int d = 0; d < DT; ++d) held[u][d] = r[d];
               held_lse[u] = r_lse;
             }
         }
@@ -571,67 +1004,161 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
         m_run = -INFINITY;
         l_run = 0.f;
 #pragma unroll
-        for (int d = 0; d < D / 16; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < DT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
       }
       cursor_next(c_cmp);
     }
     return;
   }
 
-  if (n_w > 0) {
-    // page-table rows of the first P+1 blocks, then the first P row groups
-    for (int j = 0; j <= C::kP; ++j) issue_table(j, shared_block(j));
-    wait_vmcnt<0>();
-    for (int gi = -C::kP; gi < 0; ++gi) {
-      if (gi + C::kP < n_w) {
-        issue_table(gi + 2 * C::kP + 1, shared_block(gi + 2 * C::kP + 1));
-        issue_rows(gi + C::kP, shared_block(gi + C::kP));
+  // kStreamGroup: the range's segments (a sequence's part in it), one after the other; else the one split
+  int seg_left = sr.n, seg_block = sr.block, seg_first = sr.first_block;
+  int part_seq[2] = {-1, -1}, part_first[2] = {0, 0};
+  b = kStreamGroup ? sr.seq : b;
+  for (;;) {
+    float* seg_out = out_base;   // rows of the 16 heads, seg_row floats apart; LSEs seg_lse_row apart
+    float* seg_lse = lse_base;
+    int64_t seg_row = (int64_t)prm.S * Dout, seg_lse_row = prm.S;
+    bool whole = false;
+    int seg_n = 0;
+    if constexpr (kStreamGroup) {
+      const int seq_len = lens[b], nb = (seq_len + KEYS - 1) / KEYS;
+      seg_n = min(nb - seg_block, seg_left);
+      start = seg_block * KEYS;
+      end = min(start + seg_n * KEYS, seq_len);
+      whole = seg_n == nb;
+      const int slot = seg_block == 0 ? 1 : 0;
+      seg_out = prm.out + (((int64_t)range * 2 + slot) * prm.Hq + h0) * Dout;
+      seg_lse = prm.lse + ((int64_t)range * 2 + slot) * prm.Hq + h0;
+      seg_row = Dout;
+      seg_lse_row = 1;
+      if (!whole) part_seq[slot] = b, part_first[slot] = seg_first;
+      n_w = seg_n > kwave ? (seg_n - kwave + NK - 1) / NK : 0;
+      m_run = -INFINITY;
+      l_run = 0.f;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
+    }
+    constexpr int kLoads = 1 + (C::kLoadsPerGroup - 1) / kHalves;   // this wave's share of a block's
+    // (kStreamGroup: the waves of a pair bring each other's rows, so all waves step together)
+    const int steps = kStreamGroup ? (seg_n + NK - 1) / NK : n_w;
+    auto step_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (n_w > 0) {
+      // page-table rows of the first P+1 blocks, then the first P row groups
+      for (int j = 0; j <= C::kP; ++j) issue_table(j, shared_block(j));
+      if constexpr (kStreamGroup) load_q(b);   // (one trip to memory with the page-table rows)
+      wait_vmcnt<0>();
+      for (int gi = -C::kP; gi < 0; ++gi) {
+        if (gi + C::kP < n_w) {
+          issue_table(gi + 2 * C::kP + 1, shared_block(gi + 2 * C::kP + 1));
+          issue_rows(gi + C::kP, shared_block(gi + C::kP));
+        }
       }
     }
-    for (int i = 0; i < n_w; ++i) {
+    for (int i = 0; i < steps; ++i) {
       if constexpr (C::kWaitFirst) wait_vmcnt<0>();
       if (i + C::kP < n_w) {
         issue_table(i + 2 * C::kP + 1, shared_block(i + 2 * C::kP + 1));
         issue_rows(i + C::kP, shared_block(i + C::kP));
       }
-      if constexpr (!C::kWaitFirst) wait_groups<C::kLoadsPerGroup>(min(C::kP, n_w - 1 - i));
-      compute(i, shared_block(i));
+      if constexpr (!C::kWaitFirst) wait_groups<kLoads>(min(C::kP, n_w - 1 - i));
+      if constexpr (kStreamGroup) step_barrier();
+      if (!kStreamGroup || i < n_w) compute(i, shared_block(i));
+      if constexpr (kStreamGroup) step_barrier();
     }
-  }
 
-  // ---- merge the waves' partial states ---------------------------------------------------------
-  l_run += __shfl_xor(l_run, 16);
-  l_run += __shfl_xor(l_run, 32);
-  wait_vmcnt<0>();
-  __syncthreads();  // every wave is done with its ring; reuse it
-  TDIST_AS3 float* s_m = (TDIST_AS3 float*)(wbase);  // [16]
-  TDIST_AS3 float* s_l = s_m + 16;                   // [16]
-  TDIST_AS3 float* s_acc = s_l + 16;                 // [D][16]
-  if (lane < 16) {
-    s_m[lane] = m_run;
-    s_l[lane] = l_run;
-  }
-#pragma unroll
-  for (int d = 0; d < D / 16; ++d)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s_acc[(16 * d + 4 * g + i) * 16 + x] = acc[d][i];
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < nvalid * Dout; idx += NW * 64) {
-    const int h = idx / Dout, dv = idx - h * Dout;
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, ((const TDIST_AS3 float*)(smem3 + w * C::kWaveBytes))[h]);
-    float L = 0.f, O = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const TDIST_AS3 float* wm = (const TDIST_AS3 float*)(smem3 + w * C::kWaveBytes);
-      const float mw = wm[h];
-      const float sc = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-      L += wm[16 + h] * sc;
-      O += wm[32 + dv * 16 + h] * sc;
+    // ---- merge the waves' partial states ---------------------------------------------------------
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    wait_vmcnt<0>();
+    __syncthreads();  // every wave is done with its ring; reuse it
+    TDIST_AS3 float* s_m = (TDIST_AS3 float*)(wbase);  // [16]
+    TDIST_AS3 float* s_l = s_m + 16;                   // [16]
+    TDIST_AS3 float* s_acc = s_l + 16;                 // [16][kAccRow]: the 4 floats between rows spread them over the banks
+    constexpr int kAccRow = decode_acc_row(D);
+    if (lane < 16) {
+      s_m[lane] = m_run;
+      s_l[lane] = l_run;
     }
-    store_partial<kFuse>(out_base + (int64_t)h * prm.S * Dout + dv, O / L);
-    if (dv == 0) store_partial<kFuse>(lse_base + (int64_t)h * prm.S, (M + log2f(L)) * kLn2);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) *(TDIST_AS3 float4v*)(s_acc + x * kAccRow + 16 * (half * DT + d) + 4 * g) = acc[d];
+    __syncthreads();
+    // What each stream of keys counts for in each head: lane l works it out for stream l / 16 and head l % 16 (in every
+    // wave: nobody waits), and the LDS hands it round.
+    static_assert(kWaveHeads || kStream || NK <= 4, "one lane per stream of keys and head");
+    float r_lse16;
+    TDIST_AS3 float* const s_w = s_acc + 16 * kAccRow + (kHalves == 1 ? 0 : half * 64);   // this wave's [4][16]
+    {
+      const int w = lane >> 4, h = lane & 15;
+      const TDIST_AS3 float* wm = (const TDIST_AS3 float*)(smem3 + min(w, NK - 1) * C::kWaveBytes);
+      const float mw = w < NK ? wm[h] : -INFINITY;
+      float M = fmaxf(mw, __shfl_xor(mw, 16));
+      M = fmaxf(M, __shfl_xor(M, 32));
+      const float sc = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+      float L = w < NK ? wm[16 + h] * sc : 0.f;
+      L += __shfl_xor(L, 16);
+      L += __shfl_xor(L, 32);
+      s_w[lane] = sc / L;
+      r_lse16 = (M + log2f(L)) * kLn2;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int vecs = Dout / 4;
+    for (int idx = threadIdx.x; idx < nvalid * vecs; idx += NW * 64) {
+      const int h = idx / vecs, dv = (idx - h * vecs) * 4;
+      float4v O = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NK; ++w) {
+        const float4v a4 = *(const TDIST_AS3 float4v*)((const TDIST_AS3 float*)(smem3 + w * C::kWaveBytes) + 32 + h * kAccRow + dv);
+        const float sc = s_w[w * 16 + h];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[e] += a4[e] * sc;
+      }
+      if (kStreamGroup && whole) {
+        store_elem4(prm.final_out, (int64_t)b * prm.fo_sb + (int64_t)(h0 + h) * prm.fo_sh + dv, prm.final_dtype, prm.fo_vec, O);
+      } else {
+        float* o = seg_out + h * seg_row + dv;
+        if (kStreamGroup || prm.part_vec) {
+          store_partial4<kFuse>(o, O);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) store_partial<kFuse>(o + e, O[e]);
+        }
+      }
+    }
+    if (threadIdx.x < nvalid) {
+      if (!kStreamGroup || !whole) store_partial<kFuse>(seg_lse + threadIdx.x * seg_lse_row, r_lse16);
+      else if (prm.final_lse) prm.final_lse[(int64_t)b * prm.Hq + h0 + threadIdx.x] = r_lse16;
+    }
+    if constexpr (!kStreamGroup) break;
+    seg_left -= seg_n;
+    if (seg_left == 0) break;
+    seg_first += (lens[b] + KEYS - 1) / KEYS;
+    do ++b;
+    while (lens[b] <= 0);
+    seg_block = 0;
+    __syncthreads();   // the merge has read its rings
+  }
+  if constexpr (kStreamGroup) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's partial results are where every XCD sees them
+    __syncthreads();
+    TDIST_AS3 int* const s_last = (TDIST_AS3 int*)smem3;
+#pragma unroll
+    for (int slot = 0; slot < 2; ++slot) {
+      if (part_seq[slot] < 0) continue;
+      const int seq = part_seq[slot];
+      const int nb = (lens[seq] + KEYS - 1) / KEYS;
+      const int first = part_first[slot] / sr.per, parts = (part_first[slot] + nb - 1) / sr.per - first + 1;
+      if (threadIdx.x == 0) {
+        int32_t* const ctr = prm.counters + ((int64_t)seq * prm.Hkv + kvh) * head_blocks + hb;
+        const int last = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *s_last = last;
+      }
+      __syncthreads();
+      const int last = __builtin_amdgcn_readfirstlane(*s_last);
+      if (last) stream_merge<NW>(prm, seq, first, parts, h0, nvalid, Dout, (TDIST_AS3 float*)(smem3 + 64));
+      __syncthreads();
+    }
   }
 }
 
@@ -648,17 +1175,6 @@ struct CombineParams {
   int64_t l_sp, l_sb, l_sh;
   int64_t o_sb, o_sh;
 };
-
-__device__ __forceinline__ float load_elem(const unsigned char* base, int64_t idx, int dtype) {
-  if (dtype == TDIST_F32) return ((const float*)base)[idx];
-  const uint32_t bits = ((const unsigned short*)base)[idx];
-  return dtype == TDIST_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
-}
-__device__ __forceinline__ void store_elem(unsigned char* base, int64_t idx, int dtype, float v) {
-  if (dtype == TDIST_F32) ((float*)base)[idx] = v;
-  else if (dtype == TDIST_BF16) ((unsigned short*)base)[idx] = (unsigned short)f32_to_bf16_bits(v);
-  else ((unsigned short*)base)[idx] = (unsigned short)(pack_f16x2(v, 0.f) & 0xffffu);
-}
 
 // One wave per (b,h); lanes stride over Dv. Partial j is weighted by exp(lse_j - max).
 // Lane j holds the LSE of partial j (one load per lane instead of a loop of loads in every lane; -inf where the
@@ -846,7 +1362,7 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kv_kernel(const DecodePa
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kFuse, bool kPadded, bool kWaveHeads = false>
 static int launch_decode_cfg(const DecodeParams& prm, int head_blocks, hipStream_t stream) {
   typedef DecodeCfg<D, DPE, KEYS, NST> C;
-  static_assert((32 + D * 16) * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
+  static_assert((32 + 16 * decode_acc_row(D) + 128) * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
   const size_t lds = (size_t)NW * C::kWaveBytes;
   static_assert((size_t)NW * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
   auto kern = decode_split_kv_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap, kFuse, kPadded, kWaveHeads>;
@@ -860,6 +1376,77 @@ static int launch_decode_cfg(const DecodeParams& prm, int head_blocks, hipStream
             kWaveHeads ? (prm.S + prm.splits_per_team - 1) / prm.splits_per_team : prm.S, prm.B);
   hipLaunchKernelGGL(kern, grid, dim3(NW * 64), lds, stream, prm);
   return launch_status(kFuse ? "tdist_decode_fused" : "tdist_decode_split_kv");
+}
+
+// Streaming form: the whole batch in one launch that fills the chip once. All sequences' blocks of KEYS keys are laid
+// end to end and cut into equal ranges; a wave takes one kv head (and up to 16 of its query heads) over one range,
+// whatever the lengths are. A sequence that lies in one range is finished by its wave; one that is spread over several
+// leaves partial results (at most two per range), and the last of its waves to arrive merges them, so nobody waits.
+// What bounds it: the K/V stream from HBM (B 32, 64 / 8 heads, 32768 keys: 650 us, 6.6 TB/s), and for little work the
+// chain lens -> table -> rows -> merge (B 1, 32 / 8 heads, 64 keys: 9 us). Against 32 splits per sequence, a combine launch
+// and the form for even lengths behind which the other one was queued, whole calls: 48 sequences of 128 to 8192 keys, f16,
+// 64 / 8 heads 205 -> 85 us; B 32 x 32768 715 -> 652 us. Eight waves of two stages: the same where the stream is long,
+// 15 % behind where it is short (B 64 x 256 keys).
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kPadded>
+__global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodeParams prm) {
+  const int group = prm.Hq / prm.Hkv;
+  if ((int)(blockIdx.x * NW + (threadIdx.x >> 6)) >= prm.ranges * prm.Hkv * ((group + 15) >> 4)) return;
+  decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, false, kPadded, false, true>(prm);
+}
+
+// The same for heads that share one key and whose value is a part of it (latent attention, 576 / 512): a workgroup takes
+// a block of 16 query heads over one range, its pairs of waves every fourth block of keys, merged through the LDS where a
+// sequence ends; only the key rows are fetched, and the head blocks of a range run on one XCD, whose L2 then fetches them once.
+// What bounds it: LDS reads of the operands (53 KB per block and wave pair; the scores are worked out in both waves of a
+// pair) and, at a few blocks per stream, the fixed work at a segment's ends. B 16, 128 / 1 heads, 64 to 4096 keys: 388 us
+// with 32 splits and their combine (eight head blocks fetching both row sets, 134 MB of partial results) -> 66 us.
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
+__global__ __launch_bounds__(NW * 64) void decode_stream_group_kernel(const DecodeParams prm) {
+  decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, true, false, false, false, true>(prm);
+}
+
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
+static int launch_stream_group_cfg(DecodeParams& prm, int head_blocks, hipStream_t stream) {
+  typedef DecodeCfg<D, DPE, KEYS, NST, true> C;
+  static_assert((32 + 16 * decode_acc_row(D) + 128) * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
+  static_assert(64 + 16 * kStreamMaxParts * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
+  const size_t lds = (size_t)(NW / 2) * C::kWaveBytes;
+  static_assert((size_t)(NW / 2) * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
+  auto kern = decode_stream_group_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return fail(TDIST_ERR_LAUNCH, "decode: cannot reserve %zu B of LDS: %s", lds, hipGetErrorString(e));
+    attr_set = true;
+  }
+  prm.min_blocks = NW;   // two steps of every stream of keys
+  hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)prm.ranges * prm.Hkv * head_blocks)), dim3(NW * 64), lds, stream, prm);
+  return launch_status("tdist_decode_stream");
+}
+
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kPadded>
+static int launch_stream_cfg(DecodeParams& prm, int head_blocks, hipStream_t stream) {
+  typedef DecodeCfg<D, DPE, KEYS, NST> C;
+  static_assert(16 * kStreamMaxParts * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
+  const size_t lds = (size_t)NW * C::kWaveBytes;
+  static_assert((size_t)NW * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
+  auto kern = decode_stream_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap, kPadded>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return fail(TDIST_ERR_LAUNCH, "decode: cannot reserve %zu B of LDS: %s", lds, hipGetErrorString(e));
+    attr_set = true;
+  }
+  prm.min_blocks = 64 / KEYS;
+  const int64_t waves = (int64_t)prm.ranges * prm.Hkv * head_blocks;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((waves + NW - 1) / NW)), dim3(NW * 64), lds, stream, prm);
+  return launch_status("tdist_decode_stream");
+}
+
+template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kPadded>
+static int launch_stream(DecodeParams& prm, int head_blocks, hipStream_t stream) {
+  return prm.soft_cap > 0.f ? launch_stream_cfg<MMA, D, DPE, KEYS, NW, NST, true, kPadded>(prm, head_blocks, stream)
+                            : launch_stream_cfg<MMA, D, DPE, KEYS, NW, NST, false, kPadded>(prm, head_blocks, stream);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kPadded = false>
@@ -896,7 +1483,12 @@ struct DecodeCall {
   float* lse_out;
   void* stream;
   const char* who;
+  // streaming form
+  void* workspace;
+  int64_t workspace_bytes;
 };
+
+enum DecodeForm { kFormSplit, kFormFused, kFormStream };
 
 static int64_t decode_fused_counters(int batch, int q_heads, int kv_heads) {
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0) return -1;
@@ -904,9 +1496,36 @@ static int64_t decode_fused_counters(int batch, int q_heads, int kv_heads) {
   return (int64_t)batch * kv_heads * ((group + 15) / 16);
 }
 
-static int run_decode(const DecodeCall& c, bool fuse) {
+// Streaming form: how many ranges the batch is cut into. `units` waves (kv heads x blocks of query heads) share a
+// range, and `slots` waves are resident at a time: as many ranges as fill them once, or, where the units alone nearly
+// fill or overfill them, the number of ranges whose last round of waves is the fullest.
+static int stream_ranges(int64_t units, int64_t slots) {
+  if (units * 4 <= slots) return (int)(slots / units);
+  int best = 1;
+  double best_cost = 0;
+  for (int r = 1; r <= 16; ++r) {
+    const double cost = (double)((units * r + slots - 1) / slots) / r;
+    if (r == 1 || cost < best_cost * 0.97) best_cost = cost, best = r;
+  }
+  return best;
+}
+// Units of the streaming form on one compute unit: four waves with rings of up to four stages (as much in flight as
+// eight waves of two, half the fixed work and half the partial results), or one workgroup for latent attention.
+static int stream_waves(int head_dim) { return head_dim > 256 ? 1 : 4; }
+constexpr int kLatentWaves = 8;   // waves of a workgroup of the form for latent attention, one workgroup per compute unit
+static int64_t stream_workspace_bytes(int batch, int q_heads, int kv_heads, int head_dim, int head_dim_v) {
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || head_dim_v <= 0) return -1;
+  const int64_t units = (int64_t)kv_heads * ((q_heads / kv_heads + 15) / 16);
+  const int cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
+  // two partial results per range: rows of head_dim_v floats and one LSE per query head
+  return 2ll * stream_ranges(units, (int64_t)cus * stream_waves(head_dim)) * q_heads * (head_dim_v + 1) * 4;
+}
+
+static int run_decode(const DecodeCall& c, DecodeForm form) {
   const char* who = c.who;
-  if (!c.q || !c.k_cache || !c.v_cache || !c.out_split || !c.lse_split || !c.block_table || !c.kv_lens)
+  const bool fuse = form != kFormSplit;
+  if (!c.q || !c.k_cache || !c.v_cache || !c.block_table || !c.kv_lens ||
+      (form == kFormStream ? !c.workspace : !c.out_split || !c.lse_split))
     return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
   if (c.batch <= 0 || c.q_heads <= 0 || c.kv_heads <= 0 || c.page_size <= 0 || c.num_splits <= 0)
     return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
@@ -941,6 +1560,7 @@ static int run_decode(const DecodeCall& c, bool fuse) {
   prm.Hkv = c.kv_heads;
   prm.S = c.num_splits;
   prm.d_valid = dk;
+  prm.part_vec = aligned16(c.out_split);
   prm.splits_per_team = 1;
   prm.when_lens = 0;
   prm.page_size = c.page_size;
@@ -964,7 +1584,8 @@ static int run_decode(const DecodeCall& c, bool fuse) {
   prm.fo_sb = prm.fo_sh = 0;
   if (fuse) {
     if (!c.counters || !c.out) return fail(TDIST_ERR_INVALID, "%s: null counters or output", who);
-    if (!aligned16(c.out_split)) return fail(TDIST_ERR_UNSUPPORTED, "%s: out_split must be 16-byte aligned", who);
+    if (!aligned16(form == kFormStream ? c.workspace : c.out_split))
+      return fail(TDIST_ERR_UNSUPPORTED, "%s: %s must be 16-byte aligned", who, form == kFormStream ? "workspace" : "out_split");
     if (c.out_dtype != TDIST_F32 && c.out_dtype != TDIST_BF16 && c.out_dtype != TDIST_F16)
       return fail(TDIST_ERR_UNSUPPORTED, "%s: output dtype %d", who, c.out_dtype);
     const int64_t need = decode_fused_counters(c.batch, c.q_heads, c.kv_heads);
@@ -976,12 +1597,43 @@ static int run_decode(const DecodeCall& c, bool fuse) {
     prm.final_dtype = c.out_dtype;
     prm.fo_sb = c.out_stride_b;
     prm.fo_sh = c.out_stride_h;
+    const int esz = c.out_dtype == TDIST_F32 ? 4 : 2;
+    prm.fo_vec = ((uintptr_t)c.out % (4 * esz)) == 0 && c.out_stride_b % 4 == 0 && c.out_stride_h % 4 == 0;
   }
   const int group = c.q_heads / c.kv_heads;
   const int head_blocks = (group + 15) / 16;
   if ((int64_t)c.kv_heads * head_blocks > 65535) return fail(TDIST_ERR_UNSUPPORTED, "%s: too many heads", who);
   hipStream_t st = (hipStream_t)c.stream;
   const bool bf = c.dtype == TDIST_BF16;
+  if (form == kFormStream) {
+    const bool latent = c.v_cache == c.k_cache && prm.v_sp == prm.k_sp && prm.v_st == prm.k_st && (prm.v_sh == prm.k_sh || c.kv_heads == 1);
+    if (dk > 256 && !latent)
+      return fail(TDIST_ERR_UNSUPPORTED, "%s: head dims (%d, %d) with a value that is no part of the key", who, dk, dv);
+    const int64_t need = stream_workspace_bytes(c.batch, c.q_heads, c.kv_heads, dk, dv);
+    if (c.workspace_bytes < need)
+      return fail(TDIST_ERR_WORKSPACE, "%s: %lld bytes of workspace given, %lld needed", who, (long long)c.workspace_bytes, (long long)need);
+    const int cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
+    prm.ranges = stream_ranges((int64_t)c.kv_heads * head_blocks, (int64_t)cus * stream_waves(dk));
+    prm.out = (float*)c.workspace;
+    prm.lse = prm.out + 2ll * prm.ranges * c.q_heads * dv;
+#define TDIST_STREAM(D_, DPE_, KEYS_, NW_, NST_, PAD_)                                                \
+  return bf ? launch_stream<MmaBF16, D_, DPE_, KEYS_, NW_, NST_, PAD_>(prm, head_blocks, st)         \
+            : launch_stream<MmaF16, D_, DPE_, KEYS_, NW_, NST_, PAD_>(prm, head_blocks, st);
+    if (dk > 256) {
+#define TDIST_LATENT(MMA_, CAP_) launch_stream_group_cfg<MMA_, 512, 64, 16, kLatentWaves, 2, CAP_>(prm, head_blocks, st)
+      if (prm.soft_cap > 0.f) return bf ? TDIST_LATENT(MmaBF16, true) : TDIST_LATENT(MmaF16, true);
+      return bf ? TDIST_LATENT(MmaBF16, false) : TDIST_LATENT(MmaF16, false);
+#undef TDIST_LATENT
+    }
+    if (dk == 64) TDIST_STREAM(64, 0, 32, 4, 4, false)
+    if (dk == 128) TDIST_STREAM(128, 0, 16, 4, 4, false)
+    if (dk == 192 && dv == 128) TDIST_STREAM(128, 64, 16, 4, 3, false)
+    if (dk == 256) TDIST_STREAM(256, 0, 16, 4, 2, false)
+    if (dk < 64) TDIST_STREAM(64, 0, 32, 4, 4, true)
+    if (dk < 128) TDIST_STREAM(128, 0, 16, 4, 4, true)
+    TDIST_STREAM(256, 0, 16, 4, 2, true)
+#undef TDIST_STREAM
+  }
   // <dtype, Dv, extra key dims, keys per block, waves, stages>:
   // LDS = waves * (stages * keys * (Dk + Dv) * 2 B + tables) <= 160 KB
 #define TDIST_DEC(D_, DPE_, KEYS_, NW_, NST_)                                             \
@@ -1088,8 +1740,8 @@ int tdist_decode_split_kv(const void* q, const void* k_cache, const void* v_cach
   DecodeCall c = {q, k_cache, v_cache, out_split, lse_split, sm_scale, soft_cap, block_table, kv_lens, batch, q_heads,
                   kv_heads, head_dim, head_dim_v, page_size, num_splits, q_stride_b, q_stride_h, k_stride_page,
                   k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, table_stride, dtype,
-                  nullptr, 0, nullptr, TDIST_F32, 0, 0, nullptr, stream, "tdist_decode_split_kv"};
-  return run_decode(c, false);
+                  nullptr, 0, nullptr, TDIST_F32, 0, 0, nullptr, stream, "tdist_decode_split_kv", nullptr, 0};
+  return run_decode(c, kFormSplit);
 }
 
 int64_t tdist_decode_fused_counters(int batch, int q_heads, int kv_heads) {
@@ -1107,8 +1759,27 @@ int tdist_decode_fused(const void* q, const void* k_cache, const void* v_cache, 
                   kv_heads, head_dim, head_dim_v, page_size, num_splits, q_stride_b, q_stride_h, k_stride_page,
                   k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, table_stride, dtype,
                   counters, n_counters, out, out_dtype, out_stride_b, out_stride_h, lse_out, stream,
-                  "tdist_decode_fused"};
-  return run_decode(c, true);
+                  "tdist_decode_fused", nullptr, 0};
+  return run_decode(c, kFormFused);
+}
+
+int64_t tdist_decode_stream_workspace_bytes(int batch, int q_heads, int kv_heads, int head_dim, int head_dim_v) {
+  return stream_workspace_bytes(batch, q_heads, kv_heads, head_dim, head_dim_v);
+}
+
+int tdist_decode_stream(const void* q, const void* k_cache, const void* v_cache, float sm_scale, float soft_cap,
+                        const int32_t* block_table, const int32_t* kv_lens, int batch, int q_heads, int kv_heads,
+                        int head_dim, int head_dim_v, int page_size, int64_t q_stride_b, int64_t q_stride_h,
+                        int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
+                        int64_t v_stride_token, int64_t v_stride_head, int64_t table_stride, int dtype, int32_t* counters,
+                        int64_t n_counters, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                        int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream) {
+  DecodeCall c = {q, k_cache, v_cache, nullptr, nullptr, sm_scale, soft_cap, block_table, kv_lens, batch, q_heads,
+                  kv_heads, head_dim, head_dim_v, page_size, 1, q_stride_b, q_stride_h, k_stride_page,
+                  k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, table_stride, dtype,
+                  counters, n_counters, out, out_dtype, out_stride_b, out_stride_h, lse_out, stream,
+                  "tdist_decode_stream", workspace, workspace_bytes};
+  return run_decode(c, kFormStream);
 }
 
 int tdist_decode_combine(const void* part, int part_dtype, const float* lse, int num_partials, int mode,

@@ -115,6 +115,40 @@ def decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num
     return out, out_split, lse_split
 
 
+_STREAM_PLANS = {}   # (batch, q heads, kv heads, head dims, device) -> workspace bytes
+
+
+def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, out, lse_out=None, counters=None):
+    """tdist_decode_stream: the whole decode in one launch that divides the keys itself. ``out`` [B,Hq,Dv] (bf16 / f16 /
+    fp32), ``lse_out`` contiguous fp32 [B,Hq] or None. ``counters`` as in _counters_for. The 576 / 512 heads take this
+    form where the value is a view of the key's first columns; with a value cache of its own they run as a fixed number
+    of splits and their combine. Returns ``out``."""
+    kv_lens, block_table = _check_inputs(q, k_cache, v_cache, kv_lens, block_table)
+    batch, q_heads, dk = q.shape
+    _, page_size, kv_heads, dv = v_cache.shape
+    assert out.stride(-1) == 1 and (lse_out is None or (lse_out.dtype == torch.float32 and lse_out.is_contiguous()))
+    qs, ks, vs, os = q.stride(), k_cache.stride(), v_cache.stride(), out.stride()
+    if dk > 256 and (k_cache.data_ptr() != v_cache.data_ptr() or ks != vs):
+        S = DEFAULT_KV_SPLITS
+        part, lse, kv_lens = _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, S)
+        return decode_combine(part, lse, S, 1, kv_lens, batch, q_heads, dv, (part.stride(2), part.stride(0), part.stride(1)),
+                              (lse.stride(2), lse.stride(0), lse.stride(1)), out, lse_out)
+    key = (batch, q_heads, kv_heads, dk, dv, q.device.index)
+    need = _STREAM_PLANS.get(key)
+    if need is None:
+        if len(_STREAM_PLANS) >= 1024:
+            _STREAM_PLANS.clear()
+        need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv)
+    counters, n_counters = _counters_for(q, kv_heads, counters)
+    workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    _lib.call("tdist_decode_stream", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), scale, soft_cap,
+              block_table.data_ptr(), kv_lens.data_ptr(), batch, q_heads, kv_heads, dk, dv, page_size, qs[0], qs[1], ks[0],
+              ks[1], ks[2], vs[0], vs[1], vs[2], block_table.stride(0), _lib.dtype_code(q.dtype), counters.data_ptr(),
+              n_counters, workspace.data_ptr(), need, out.data_ptr(), _lib.dtype_code(out.dtype), os[0], os[1],
+              _lib.ptr(lse_out), _lib.stream_ptr())
+    return out
+
+
 def decode_combine(part, lse, num_partials, mode, lens, batch, q_heads, dv, part_strides, lse_strides, out,
                    lse_out=None):
     """tdist_decode_combine with explicit element strides (p, b, h) for ``part`` and ``lse``."""
@@ -131,19 +165,13 @@ def gqa_fwd_batch_decode(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_
 
     q [B,Hq,D]; k_cache / v_cache [num_pages, page_size, Hkv, D]; kv_lens int32[B]; block_table int32
     [B, max_pages]. ``workspace`` and ``q_lens`` are accepted and unused, as in the reference.
-    ``output_split`` is ignored (partials are fp32 internally). Returns ``output_combine`` [B,Hq,Dv]
-    (default dtype: q's; the reference hard-codes float16, :784)."""
-    num_splits = DEFAULT_KV_SPLITS if kv_split == -1 else kv_split
-    out_split, lse_split, kv_lens = _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num_splits)
-    batch, q_heads, _ = q.shape
-    dv = v_cache.shape[-1]
+    ``output_split`` is ignored: one launch divides the keys of the whole batch evenly over the chip, whatever the
+    lengths (``kv_split``, the reference's fixed number of splits per sequence, is accepted for its signature and
+    changes nothing in the result). Returns ``output_combine`` [B,Hq,Dv] (default dtype: q's; the reference hard-codes
+    float16, :784)."""
     if output_combine is None:
-        output_combine = torch.empty((batch, q_heads, dv), dtype=q.dtype, device=q.device)
-    assert output_combine.stride(-1) == 1
-    decode_combine(out_split, lse_split, num_splits, 1, kv_lens, batch, q_heads, dv,
-                   (out_split.stride(2), out_split.stride(0), out_split.stride(1)),
-                   (lse_split.stride(2), lse_split.stride(0), lse_split.stride(1)), output_combine)
-    return output_combine
+        output_combine = torch.empty((q.shape[0], q.shape[1], v_cache.shape[-1]), dtype=q.dtype, device=q.device)
+    return decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, output_combine)
 
 
 def gqa_fwd_batch_decode_persistent(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_table, scale, soft_cap=0.0,
@@ -153,12 +181,14 @@ def gqa_fwd_batch_decode_persistent(q, k_cache, v_cache, workspace, q_lens, kv_l
     ``workspace`` (the reference's barrier buffer) and ``q_lens`` are accepted and unused: nothing says what a
     caller's buffer holds or who else uses it, and a counter that does not start at zero makes a merge fire early or
     never, so the arrival counters are the library's own (zeroed, cached per device and stream, left zero by every
-    call). ``output_split`` is ignored (partials are fp32 internally)."""
-    num_splits = DEFAULT_KV_SPLITS if kv_split == -1 else kv_split
+    call). ``output_split`` is ignored (partials are fp32 internally). ``kv_split`` = -1: the launch divides the keys
+    itself, as gqa_fwd_batch_decode does; otherwise every sequence is cut into that many splits."""
     batch, q_heads, _ = q.shape
     if output_combine is None:
         output_combine = torch.empty((batch, q_heads, v_cache.shape[-1]), dtype=q.dtype, device=q.device)
-    decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num_splits, output_combine)
+    if kv_split == -1:
+        return decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, output_combine)
+    decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, kv_split, output_combine)
     return output_combine
 
 
@@ -170,16 +200,14 @@ def gqa_fwd_batch_decode_intra_rank(q, k_cache, v_cache, workspace, q_lens, kv_l
     fp32 (out [B,Hq,Dv], lse [B,Hq]) pair the merge produced. ``workspace`` and ``q_lens`` are accepted and unused, as
     in the reference; ``counters`` (keyword only in spirit: an addition) hands in zeroed arrival counters of the
     caller's own, see _counters_for."""
-    num_splits = DEFAULT_KV_SPLITS if kv_split == -1 else kv_split
     batch, q_heads, _ = q.shape
     dv = v_cache.shape[-1]
     if output_combine is None:
         output_combine = torch.empty((batch, q_heads, dv + 1), dtype=torch.float32, device=q.device)
     out32 = torch.empty((batch, q_heads, dv), dtype=torch.float32, device=q.device)
     lse32 = torch.empty((batch, q_heads), dtype=torch.float32, device=q.device)
-    # split-KV and the merge of the splits (keeping the LSE) in one launch
-    decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num_splits, out32, lse32,
-                 workspace=counters)
+    # the keys divided and merged (keeping the LSE) in one launch
+    decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, out32, lse32, counters=counters)
     output_combine[..., :dv].copy_(out32)
     output_combine[..., dv].copy_(lse32)
     if return_lse:

@@ -9,8 +9,7 @@ the gather has nobody to talk to: the partial results of the other ranks are pas
 import torch
 
 from triton_dist import _lib
-from triton_dist.kernels.amd.flash_decode import (gqa_fwd_batch_decode_intra_rank,
-                                                   gqa_fwd_batch_decode_inter_rank_combine)
+from triton_dist.kernels.amd.flash_decode import decode_stream, gqa_fwd_batch_decode_inter_rank_combine
 
 
 class SpGQAFlashDecodeAttention(torch.nn.Module):
@@ -30,7 +29,8 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         self.q_head_dim, self.v_head_dim = q_head_dim, v_head_dim
         self.page_size = page_size
         self.scale, self.soft_cap = scale, soft_cap
-        self.kv_split = 32                    # splits of the local shard (the reference fixes 32, :59)
+        self.kv_split = 32                    # recorded (the reference cuts every sequence into 32, :59; here the launch
+                                              # divides the batch's keys itself)
         self.max_allowed_batch = max_allowed_batch
         # the fused decode keeps its arrival counters per layer, so that two layers may run on two streams
         self.workspace = None
@@ -53,19 +53,21 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         if self.workspace is None or self.workspace.device != q.device:
             n = _lib.load().tdist_decode_fused_counters(self.max_allowed_batch, self.num_q_heads, self.num_kv_heads)
             self.workspace = torch.zeros(max(int(n), 1), dtype=torch.int32, device=q.device)
-        _, out32, lse32 = gqa_fwd_batch_decode_intra_rank(q, k_cache, v_cache, None, [1] * batch,
-                                                          global_kv_lens[self.rank], block_table, self.scale,
-                                                          soft_cap=self.soft_cap, kv_split=self.kv_split,
-                                                          return_lse=True, counters=self.workspace)
         if self.num_ranks == 1:
-            all_out, all_lse = out32.unsqueeze(0), lse32.unsqueeze(0)
+            all_out = torch.empty((1, batch, self.num_q_heads, self.v_head_dim), dtype=torch.float32, device=q.device)
+            all_lse = torch.empty((1, batch, self.num_q_heads), dtype=torch.float32, device=q.device)
         else:
             if peer_partials is None:
                 raise RuntimeError("one GPU holds a single rank: pass the other ranks' (out, lse) as peer_partials")
             all_out, all_lse = peer_partials
             assert all_out.shape == (self.num_ranks, batch, self.num_q_heads, self.v_head_dim)
             assert all_lse.shape == (self.num_ranks, batch, self.num_q_heads)
-            # the local copy into the gather buffer (reference :133-135)
-            all_out[self.rank].copy_(out32)
-            all_lse[self.rank].copy_(lse32)
+        # the own result goes straight into its place in the gather buffers (reference :133-135 copies it there)
+        own_out, own_lse = all_out[self.rank], all_lse[self.rank]
+        lse = own_lse if own_lse.dtype == torch.float32 and own_lse.is_contiguous() else torch.empty_like(
+            own_lse, dtype=torch.float32, memory_format=torch.contiguous_format)
+        decode_stream(q, k_cache, v_cache, global_kv_lens[self.rank], block_table, self.scale, self.soft_cap, own_out, lse,
+                      counters=self.workspace)
+        if lse is not own_lse:
+            own_lse.copy_(lse)
         return gqa_fwd_batch_decode_inter_rank_combine(all_out, all_lse, global_kv_lens, out_dtype=q.dtype)
