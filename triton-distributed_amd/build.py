@@ -21,7 +21,7 @@ INCLUDE = os.path.join(ROOT, "include")
 OUT_DIR = os.path.join(HERE, "triton_dist", "_lib")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_NAME = "libtdist_hip.so"
-SOURCES = ["gemm.hip", "decode.hip", "moe.hip", "lib.hip", "reduce.hip"]
+SOURCES = ["gemm.hip", "gemm_small.hip", "decode.hip", "moe.hip", "lib.hip", "reduce.hip"]
 BENCH_SOURCES = ["bench_probes.hip"]   # libtdist_bench.so: measurement helpers, not part of the product library
 BENCH_LIB_NAME = "libtdist_bench.so"
 
@@ -57,7 +57,7 @@ def _hipcc():
 
 def _inputs():
     files = [os.path.join(CSRC, s) for s in SOURCES + BENCH_SOURCES]
-    files += [os.path.join(CSRC, "common.h"), os.path.join(INCLUDE, "tdist.h"), os.path.join(INCLUDE, "tdist_bench.h")]
+    files += [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_small.h"), os.path.join(INCLUDE, "tdist.h"), os.path.join(INCLUDE, "tdist_bench.h")]
     return files
 
 

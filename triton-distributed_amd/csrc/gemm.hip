@@ -30,6 +30,7 @@
 #include <utility>
 
 #include "common.h"
+#include "gemm_small.h"
 
 namespace tdist {
 
@@ -53,6 +54,10 @@ struct GemmParams {
   int gate_rows;     // rows per flag word: m_per_chunk, or (ragged chunks, walked in row order) any positive number:
                      // a tile then waits for every flag its rows touch
   int k_tail_bytes;  // bytes of K in the last K tile when K is not a whole number of them (128 x 128 tile only), else 0
+  // Split ring, K no whole number of 128-byte tiles: bytes of K in the FIRST K tile, else 0. A, A_local and B then point
+  // 128 - k_head_bytes before their first row, so that K tile 0 ends where the rest begins and every later tile is whole:
+  // only the loads of tile 0, which lie outside the K loop, need to know (their lanes in front of the row fetch zeros).
+  int k_head_bytes;
   int chunks_per_rank;
   int wait_value;
   int rank, world_size;
@@ -116,6 +121,8 @@ struct GemmParams {
 // Workspace header, in int32 words
 constexpr int kSkCtrlEpoch = 0;          // tag base of the next launch
 constexpr int kSkCtrlDone = 1;           // workgroups of the running launch that have left
+constexpr int kSkSmallOff = 16;          // [kSkSmallTiles] arrival counters of gemm_small.hip's tiles, zero between launches
+constexpr int kSkSmallTiles = 1024 - kSkSmallOff;
 constexpr int kSkMaxWorkgroups = 1024;
 constexpr int kSkFlagsOff = 1024;        // [kSkMaxWorkgroups] tag of the partial in the slot
 constexpr int kSkAcksOff = 2048;         // [kSkMaxWorkgroups] readers that are done with the slot, ever
@@ -367,7 +374,7 @@ __device__ __forceinline__ int chunk_of(const GemmParams& p, int oc) {
 
 // kPlain: an instance for calls without flags and without a local shard (the GEMM-RS producer, plain GEMMs): no gating
 // code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly).
-template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false>
+template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams p) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
   typedef TDIST_AS3 unsigned char* lds_u8;
@@ -743,6 +750,25 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       const unsigned char* src = chunk * 16 < p.k_tail_bytes ? sbase + voff : kZeroChunk;
       __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)src, (TDIST_AS3 void*)dst, 16, 0, 0);
     };
+    // the same for a ragged FIRST K tile of the split ring (k_head_bytes), whose lanes in front of the row fetch zeros
+    auto dma16_first = [&](const unsigned char* sbase, uint32_t voff, int r, lds_u8 dst, bool ragged) {
+      if (!ragged) {
+        dma16(sbase, voff, dst);
+        return;
+      }
+      const int chunk = dma_pos ^ swz<KB>(r);
+      const unsigned char* src = chunk * 16 >= KB - p.k_head_bytes ? sbase + voff : kZeroChunk;
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)src, (TDIST_AS3 void*)dst, 16, 0, 0);
+    };
+    auto issue_first = [&](const unsigned char* abase, const unsigned char* bbase, bool ragged) {   // A(0), B(0)
+#pragma unroll
+      for (int t = 0; t < C::kAInstr; ++t)
+        dma16_first(abase, a_off[t], (wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row, smem + (wave * C::kAInstr + t) * 1024, ragged);
+#pragma unroll
+      for (int u = 0; u < C::kBInstr; ++u)
+        dma16_first(bbase, b_off[u], (wave * C::kBInstr + u) * C::kRowsPerInstr + dma_row,
+                    smem + C::kAStages * C::kABytes + (wave * C::kBInstr + u) * 1024, ragged);
+    };
     auto issue_a = [&](int kt, int t) {
       lds_u8 const dst = a_stage(kt) + (wave * C::kAInstr + t) * 1024;
       if constexpr (!C::kSplit) {
@@ -908,10 +934,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         acc_clear<kAccRegs>();
         wait_tiles_and_barrier<kEarly ? C::kBInstr + kEpiStores + C::kAInstr : 0>();
       } else {
-#pragma unroll
-        for (int t = 0; t < C::kAInstr; ++t) issue_a(0, t);
-#pragma unroll
-        for (int u = 0; u < C::kBInstr; ++u) issue_b(0, u);
+        issue_first(a_base, b_base, kHead && p.k_head_bytes != 0 && ka == 0);
 #pragma unroll
         for (int t = 0; t < C::kAInstr; ++t) issue_a(1, t);
 #pragma unroll
@@ -999,10 +1022,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         acc_clear<kAccRegs>();
         wait_tiles_and_barrier<kEarly ? C::kBInstr + kEpiStores + C::kAInstr : 0>();
       } else {
-#pragma unroll
-        for (int t = 0; t < C::kAInstr; ++t) issue_a(0, t);
-#pragma unroll
-        for (int u = 0; u < C::kBInstr; ++u) issue_b(0, u);
+        issue_first(a_base, b_base, kHead && p.k_head_bytes != 0 && ka == 0);
 #pragma unroll
         for (int t = 0; t < C::kAInstr; ++t) issue_a(1, t);
 #pragma unroll
@@ -1181,11 +1201,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       // and once everything older than them has landed (the loads the K loop issued beyond the tile's end, which may
       // point anywhere in the ring) the A stages 1 and 2 are free for staging
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-      for (int t = 0; t < C::kAInstr; ++t) dma16(a_base_n, a_off[t], smem + (wave * C::kAInstr + t) * 1024);
-#pragma unroll
-      for (int u = 0; u < C::kBInstr; ++u)
-        dma16(b_base_n, b_off[u], smem + C::kAStages * C::kABytes + (wave * C::kBInstr + u) * 1024);
+      issue_first(a_base_n, b_base_n, kHead && p.k_head_bytes != 0);
 #pragma unroll
       for (int u = 0; u < C::kBInstr; ++u)
         dma16(b_base_n + KB, b_off[u], smem + C::kAStages * C::kABytes + C::kBBytes + (wave * C::kBInstr + u) * 1024);
@@ -1665,6 +1681,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
 
 // ---- host side ------------------------------------------------------------------------------------
 enum GemmElem { kElemBF16, kElemF16, kElemFP8 };
+constexpr int kNumLargeTiles = 5;   // the tiles of this file; TDIST_DEBUG_GEMM_TILE counts gemm_small.hip's behind them
 
 struct GemmCall {
   const void* A;
@@ -1692,10 +1709,10 @@ struct GemmCall {
   const char* who;
 };
 
-template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false>
+template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
 static int launch_gemm_cfg(const GemmParams& prm, int grid, hipStream_t stream, const char* who) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
-  auto kern = gemm_kernel<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain>;
+  auto kern = gemm_kernel<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain, kHead>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes);
@@ -1741,6 +1758,81 @@ static void sk_attach(GemmParams& p, void* ws, int mode) {
 // tile's fp32 accumulators and reads as much back)
 static double sk_handover_k_tiles(int bm, int bn) { return 2.0 + 6.0 * bm * bn / 65536.0; }
 
+// The GEMM on the small tiles (gemm_small.hip): the tile and the number of workgroups that share one along K, by an
+// estimate in microseconds (us = 0: this call does not qualify). The estimate is a fit to measured times (bf16 and e4m3 alike:
+// what a K tile of 128 bytes costs is its LDS traffic): a K tile takes 0.5 / 0.7 us while a compute unit has one workgroup
+// (64 / 128 rows) and 0.72 / 1.15 us with two, a round of workgroups 1.5 us beside, a launch 3 us, and handing pieces
+// over 2 us + 0.25 us per piece + their bytes at 2.7 TB/s.
+// (Pieces of at least kSmallMinPiece K tiles: shorter ones cost more than they save, and a short K's sums then run in the
+// order of the large tiles', bit for bit.)
+constexpr int kSmallMinPiece = 8;
+struct SmallPlan {
+  int tile, splits, tiles_per_split;
+  bool deep;
+  double us;
+};
+static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
+  SmallPlan best = {0, 0, 0, false, 0};
+  if (c.flags || c.A_local || (int64_t)c.M * c.lda * esz >= (1ll << 31) || (int64_t)c.N * c.ldb * esz >= (1ll << 31)) return best;
+  const int k_tiles = (int)ceil_div((int64_t)c.K * esz, 128);
+  const int forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE) - kNumLargeTiles, sk = debug_get(TDIST_DEBUG_GEMM_SPLIT_K);
+  // (a capped grid and a forced split of a last round are the large tiles')
+  if ((c.max_workgroups > 0 && c.max_workgroups < cus) || (sk == 1 && forced_tile < 0)) return best;
+  for (int t = 0; t < kNumSmallTiles; ++t) {
+    if (forced_tile >= 0 && forced_tile != t) continue;
+    const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn;
+    if (c.scatter_bufs && (c.world_size <= 0 || c.M % c.world_size != 0 || (c.M / c.world_size) % bm != 0)) continue;
+    const int64_t tiles = ceil_div(c.M, bm) * ceil_div(c.N, bn);
+    for (int s = 1; s <= kSmallMaxSplits; s *= 2) {
+      if (s > 1 && (sk == 0 || tiles > kSkSmallTiles || k_tiles / s < (sk > 1 ? 2 : kSmallMinPiece) || c.sk_workspace == nullptr ||
+                    c.sk_workspace_bytes < kSkHeaderBytes + tiles * s * bm * bn * 4)) break;
+      if (sk > 1 && s != sk) continue;
+      const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
+      const int64_t units = tiles * pieces;
+      const bool deep = units <= cus;
+      double us = 3.0;
+      if (deep) us += per * (t == 0 ? 0.5 : 0.7) + 1.0;
+      else us += (double)ceil_div(units, 2 * cus) * (per * (t == 0 ? 0.72 : 1.15) + 1.5);
+      if (pieces > 1) us += 2.0 + 0.25 * pieces + (double)units * bm * bn * 4 / 2.7e6;
+      if (best.us == 0 || us < best.us) best = {t, pieces, per, deep, us};
+    }
+  }
+  return best;
+}
+
+static int run_small(const GemmCall& c, GemmElem elem, int esz, const SmallPlan& plan, const DeviceInfo& di) {
+  SmallGemmParams q;
+  q.A = (const unsigned char*)c.A;
+  q.B = (const unsigned char*)c.B;
+  q.C = (unsigned char*)c.C;
+  q.scatter_bufs = c.scatter_bufs;
+  q.row_scale = c.row_scale;
+  q.col_scale = c.col_scale;
+  q.lda_b = c.lda * esz;
+  q.ldb_b = c.ldb * esz;
+  q.ldc = c.ldc;
+  q.M = c.M;
+  q.N = c.N;
+  q.k_bytes = c.K * esz;
+  q.m_per_rank = c.scatter_bufs ? c.M / c.world_size : c.M;
+  q.rank = c.rank;
+  q.splits = plan.splits;
+  q.tiles_per_split = plan.tiles_per_split;
+  q.partials = plan.splits > 1 ? (float*)((unsigned char*)c.sk_workspace + kSkHeaderBytes) : nullptr;
+  q.counters = plan.splits > 1 ? (int32_t*)c.sk_workspace + kSkSmallOff : nullptr;
+  q.l2_local = di.xcd_round_robin == 1 && di.num_xcds == 8 && debug_get(TDIST_DEBUG_GEMM_SK_COHERENT) != 1;
+  return launch_gemm_small(q, elem == kElemBF16 ? kSmallBF16 : elem == kElemF16 ? kSmallF16 : kSmallFP8, plan.tile, plan.deep, c.stream, c.who);
+}
+
+static void set_k_head(GemmParams& p, bool split_ring, int64_t k_bytes) {
+  p.k_head_bytes = split_ring ? (int)(k_bytes % 128) : 0;
+  if (p.k_head_bytes == 0) return;
+  const int back = 128 - p.k_head_bytes;
+  p.A -= back;
+  p.B -= back;
+  if (p.A_local) p.A_local -= back;
+}
+
 static int run_gemm(const GemmCall& c, GemmElem elem) {
   const char* who = c.who;
   const int esz = elem == kElemFP8 ? 1 : 2;
@@ -1764,29 +1856,28 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   if (int rc = sk_workspace_check(c.sk_workspace, c.sk_workspace_bytes, who)) return rc;
   const DeviceInfo& di = device_info();
   if (di.ok != 1) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
-
   // Tile configuration. The 256-row tiles (256x256 and 256x128, both on the split ring) need the call's row blocks
-  // (chunks, rank slices, the local shard) to be multiples of 256 rows and K to be a multiple of 128 bytes; the
+  // (chunks, rank slices, the local shard) to be multiples of 256 rows; the
   // 128x256 and 128x192 tiles (split ring as well, waves of 64 x 128 and 64 x 96: for row blocks of 128·odd rows, and
   // three quarters of a 256x128 tile's work for shapes whose larger tiles would leave a quarter of the chip without
-  // one) need whole 128-byte K tiles; the 128x128 tile takes everything else. Among the admissible ones the cheapest estimate wins: rounds of the grid times the tile's work
+  // one) need more than 128 bytes of K; the 128x128 tile takes everything else. Among the admissible ones the cheapest estimate wins: rounds of the grid times the tile's work
   // over its measured relative efficiency.
   bool rows256 = true;
   if (c.scatter_bufs && c.world_size > 0 && (c.M % c.world_size != 0 || (c.M / c.world_size) % 256 != 0)) rows256 = false;
   if (!c.scatter_bufs && c.flags && c.m_per_chunk % 256 != 0) rows256 = false;
-  if (k_tail_bytes != 0) rows256 = false;
   if (c.A_local && (c.local_row_begin % 256 != 0 || c.local_rows % 256 != 0)) rows256 = false;
-  if (((int64_t)c.K * esz) % 128 != 0) rows256 = false;  // the split ring steps through K 128 bytes at a time
+  // the split ring steps through K 128 bytes at a time; a ragged K (see k_head_bytes) takes at least two K tiles
+  const bool k128 = ((int64_t)c.K * esz) % 128 == 0 || (int64_t)c.K * esz > 128;
+  if (!k128) rows256 = false;
   int cap_wgs = di.num_cus;
   if (c.max_workgroups > 0 && c.max_workgroups < cap_wgs) cap_wgs = c.max_workgroups;
   struct TileChoice { int bm, bn; double eff; };
-  constexpr int kNumChoices = 5;
+  constexpr int kNumChoices = kNumLargeTiles;
   // (rates relative to the 256x256 tile, measured on 8192 x 6144 x 3584 bf16: 1425, 1255, 774, 1078 and 1178
   // TFLOP/s; the 128x192 tile is entered below its multi-round rate because a tile's prologue and epilogue weigh
   // more the smaller it is: one round of 256 of them takes 50.5 us on 4096 x 1536 x 4096 where 192 tiles of 256x128
   // take 48.3 and 192 tiles of 128x256 53.1)
   static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.88}, {128, 128, 0.54}, {128, 192, 0.65}, {128, 256, 0.8}};
-  const bool k128 = ((int64_t)c.K * esz) % 128 == 0;
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
   // With a workspace, a last round that fills at most half of the grid is split along K (see GemmParams): it then
@@ -1808,9 +1899,20 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
-      const double cost_sk = ((double)(tiles / cap_wgs) * kt + (double)kt / split + sk_handover_k_tiles(bm, bn)) * per_k_tile;
+      // (and 10 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
+      const double cost_sk = ((double)(tiles / cap_wgs) * kt + (double)kt / split + sk_handover_k_tiles(bm, bn)) * per_k_tile +
+                             10.0 / 1.2 * 65536.0;
       if (cost_sk < 0.95 * best || (sk_mode == 1 && (!use_sk || cost_sk < best))) best = cost_sk, pick = t, use_sk = true;
     }
+  }
+  // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
+  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more (10 of them in its estimate already)
+  // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 21 us on 512 of 64 x 128; 200 x 1536 x 4096 bf16:
+  // 26 -> 16 us; 4096 x 1536 x 4096 stays on the large tiles, 45 us against 63).
+  if (const SmallPlan plan = small_plan(c, esz, di.num_cus); plan.us > 0) {
+    const int forced = debug_get(TDIST_DEBUG_GEMM_TILE);
+    const double large_us = 8.0 + best / 65536.0 * 1.2 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 15.0 : 0.0);
+    if (forced >= kNumLargeTiles || (forced < 0 && plan.us < 0.95 * large_us)) return run_small(c, elem, esz, plan, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,
   // 4 = 128x256; a tile that the call's row blocks or K do not admit is not taken.
@@ -1877,6 +1979,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   p.sched_rounds = 0; p.sched_tpc_magic = 0; p.sched_ws_magic = 0;
   p.group_s = 1; p.group_rows_shift = 0; p.cm_shift = 0;
   p.k_tail_bytes = k_tail_bytes;
+  set_k_head(p, pick != 2, (int64_t)c.K * esz);
 
   if (c.scatter_bufs) {
     if (c.world_size <= 0 || c.rank < 0 || c.rank >= c.world_size)
@@ -1982,14 +2085,17 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
 
   // 256-row tiles: 2 x 2 waves on the split ring (3 A stages + 2 B stages), 16-row MFMA blocks
   if (BM == 256 && BN == 256 && p.flags == nullptr && p.A_local == nullptr) {
-    // no flags, no local shard: the instances without gating code (the GEMM-RS producer's, the headline shape's)
+    // no flags, no local shard: the instances without gating code (the GEMM-RS producer's, the headline shape's), with
+    // and without a ragged first K tile (the test for one costs the headline shape 0.5 %)
+#define TDIST_PLAIN(E_, SC_)                                                                                        \
+  (p.k_head_bytes != 0 ? launch_gemm_cfg<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, true>(p, grid, c.stream, who)    \
+                       : launch_gemm_cfg<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, false>(p, grid, c.stream, who))
     switch (elem) {
-      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 256, 256, 128, 2, 2, 5, false, false, true>(p, grid, c.stream, who);
-      case kElemF16: return launch_gemm_cfg<ElemF16N, 256, 256, 128, 2, 2, 5, false, false, true>(p, grid, c.stream, who);
-      default:
-        return scales ? launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, true, false, true>(p, grid, c.stream, who)
-                      : launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, false, false, true>(p, grid, c.stream, who);
+      case kElemBF16: return TDIST_PLAIN(ElemBF16N, false);
+      case kElemF16: return TDIST_PLAIN(ElemF16N, false);
+      default: return scales ? TDIST_PLAIN(ElemFP8N, true) : TDIST_PLAIN(ElemFP8N, false);
     }
+#undef TDIST_PLAIN
   }
   if (BM == 256 && BN == 256) {
     switch (elem) {
@@ -2069,8 +2175,8 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
     return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
   if (c.block_size != 128 && c.block_size != 256)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: block_size %d (the row blocks of the align / sort step must be 128 or 256 rows)", who, c.block_size);
-  if (((int64_t)c.K * esz) % 64 != 0)
-    return fail(TDIST_ERR_UNSUPPORTED, "%s: K*elem_size = %lld must be a multiple of 64 bytes", who, (long long)c.K * esz);
+  if (((int64_t)c.K * esz) % 16 != 0 || (((int64_t)c.K * esz) % 64 != 0 && (int64_t)c.K * esz <= 128))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: K*elem_size = %lld must be a multiple of 64 bytes (above 128: of 16)", who, (long long)c.K * esz);
   if (!aligned16(c.A) || !aligned16(c.B) || (c.A_local && !aligned16(c.A_local)) || (c.lda * esz) % 16 || (c.ldb * esz) % 16 ||
       (c.expert_stride * esz) % 16 || (c.A_local && (c.lda_local * esz) % 16))
     return fail(TDIST_ERR_UNSUPPORTED, "%s: A/B bases and strides must be 16-byte aligned", who);
@@ -2134,8 +2240,9 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   p.gate_rows = p.m_per_chunk;
   p.k_tail_bytes = 0;
 
-  const bool k128 = ((int64_t)c.K * esz) % 128 == 0;
+  const bool k128 = ((int64_t)c.K * esz) % 128 == 0 || (int64_t)c.K * esz > 128;
   const int BN = (c.block_size == 256 || k128) ? 256 : 128;
+  set_k_head(p, k128, (int64_t)c.K * esz);
   const int64_t sched = (int64_t)c.num_blocks * ceil_div(c.N, BN);
   if (sched > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: too many tiles", who);
   int cap_wgs = di.num_cus;
@@ -2145,7 +2252,7 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   // workspace at hand the kernel splits the last round along K whenever it fills at most half of the grid.
   {
     const int bm = c.block_size == 256 ? 256 : 128;
-    const int64_t kt = (int64_t)c.K * esz / (c.block_size == 256 || k128 ? 128 : 64);
+    const int64_t kt = ceil_div((int64_t)c.K * esz, c.block_size == 256 || k128 ? 128 : 64);
     if (sk_env() != 0 && kt >= 2 * kSkMinPiece && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, BN)) {
       grid = cap_wgs;
       sk_attach(p, c.sk_workspace, 1);

@@ -1,0 +1,35 @@
+// GEMMs that do not fill the chip with large tiles: what run_gemm (gemm.hip) hands to gemm_small.hip.
+#pragma once
+#include "common.h"
+
+namespace tdist {
+
+struct SmallGemmParams {
+  const unsigned char* A;
+  const unsigned char* B;
+  unsigned char* C;           // plain output (scatter_bufs == NULL)
+  void* const* scatter_bufs;  // GEMM-RS: rows of owner o go to scatter_bufs[o] from row rank * m_per_rank on
+  const float* row_scale;     // e4m3 inputs: fp32 scales or NULL
+  const float* col_scale;
+  int64_t lda_b, ldb_b;  // byte strides; M * lda_b and N * ldb_b below 2^31
+  int64_t ldc;           // elements
+  int M, N;
+  int k_bytes;  // a multiple of 16
+  int m_per_rank, rank;
+  int splits;         // workgroups that share a tile along K
+  int tiles_per_split;  // K tiles of 128 bytes per workgroup
+  float* partials;    // splits > 1: fp32 accumulators, a tile per workgroup
+  int32_t* counters;  // splits > 1: one per tile, zero, left zero
+  int l2_local;       // workgroup i has been seen to run on XCD i % 8: the pieces of a tile meet in that XCD's L2
+};
+
+enum SmallGemmElem { kSmallBF16, kSmallF16, kSmallFP8 };
+struct SmallGemmTile { int bm, bn; };
+constexpr int kNumSmallTiles = 2;
+constexpr SmallGemmTile kSmallTiles[kNumSmallTiles] = {{64, 128}, {128, 128}};
+constexpr int kSmallMaxSplits = 16;
+
+// `deep`: six stages instead of three, one workgroup per compute unit
+int launch_gemm_small(const SmallGemmParams& p, SmallGemmElem elem, int tile, bool deep, hipStream_t stream, const char* who);
+
+}  // namespace tdist
