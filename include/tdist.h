@@ -63,8 +63,10 @@ int tdist_num_cus(void);
  * kernels take their variants from autotune configs, e.g. kernels/amd/all_gather_gemm.py:103-137). */
 typedef enum tdist_debug_key {
   TDIST_DEBUG_GEMM_TILE = 0,       /* 0..4: force the 256x256, 256x128, 128x128, 128x192 or 128x256 tile where the
-                                      call's row blocks and K admit it */
-  TDIST_DEBUG_GEMM_SPLIT_K = 1,    /* 0: whole tiles only; 1: split a last round wherever the workspace allows */
+                                      call's row blocks and K admit it; 5, 6: the small 64x128 or 128x128 tile where
+                                      the call has no flags and no local shard */
+  TDIST_DEBUG_GEMM_SPLIT_K = 1,    /* 0: whole tiles only; 1: split a last round wherever the workspace allows;
+                                      2, 4, 8, 16: workgroups per tile of the small tiles */
   TDIST_DEBUG_GEMM_SK_COHERENT = 2,/* 1: the split-round exchange always through device-coherent stores */
   TDIST_DEBUG_GEMM_SCHEDULE = 3,   /* 0: every workgroup takes its tiles in the static order; 1: in arrival
                                       order (the default for gated calls, see tdist_gemm_chunk_gated_bf16) */
@@ -101,9 +103,10 @@ int tdist_debug_get(int key);
  *   max_workgroups  upper bound on the persistent grid; <= 0: one workgroup per compute unit. A producer
  *         whose copies run on this same GPU needs compute units of its own while the GEMM spins on a flag:
  *         leave it 32 (pass tdist_num_cus() - 32). Not needed when the rows arrive from a peer's copy engine.
- * Requirements: K, lda and ldb multiples of 8 (16 for fp8) elements and 16-byte aligned bases. The large tiles are
- * taken when K * element size is a multiple of 128 bytes and the row blocks (m_per_chunk, the local shard) are
- * multiples of 256 rows; a K that ends inside a 64-byte K tile is filled up with zeros on its way in.
+ * Requirements: K, lda and ldb multiples of 8 (16 for fp8) elements and 16-byte aligned bases. The 256-row tiles are
+ * taken when the row blocks (m_per_chunk, the local shard) are multiples of 256 rows; a K that is no whole number of
+ * K tiles is filled up with zeros on its way in. Calls without flags and local shard that would leave most of the
+ * chip idle run on small tiles, several workgroups to a tile along K where sk_workspace allows.
  * m_per_chunk may be any positive number of rows: when it is not a multiple of 128, a tile waits for every chunk its
  * rows touch (the reference's per-segment wait, kernels/nvidia/allgather_gemm.py:222-224), tiles are visited in row
  * order starting inside the own rank's rows, chunk_order must be NULL and the local shard must either start and end
@@ -175,6 +178,14 @@ int tdist_producer_push_peers(void* workspace, const void* const* peer_src, int 
                               int64_t rank_bytes, int64_t chunk_bytes, int32_t* flags, int flag_value,
                               int32_t* counters, const int32_t* held, const uint64_t* stamp, int64_t ns_per_chunk,
                               uint32_t delay_seed, int64_t max_delay_ns, int workgroups_per_peer, void* stream);
+
+/* The shards of all ranks into the workspace in one launch on `stream`, without flags: what an all-gather of few rows
+ * needs whose GEMM is queued behind it on the same stream (no counterpart in the reference, where every peer pushes for
+ * itself). Shard r lands at workspace + r*rank_bytes; peer_src: device array of world_size device pointers (entry `rank`
+ * unused: the own shard is read from `own`). rank_bytes a multiple of 16, all addresses 16-byte aligned. status not NULL:
+ * the same launch retires it into first_error, as tdist_status_retire does. */
+int tdist_gather_shards(void* workspace, const void* const* peer_src, const void* own, int world_size, int rank,
+                        int64_t rank_bytes, int32_t* status, int32_t* first_error, void* stream);
 
 /* Link pacing for the one-GPU producer (no counterpart in the reference, whose chunks arrive over xGMI at the
  * link's rate: ~153 GB/s per peer). tdist_producer_mark stores the device's constant-rate wall clock into *stamp

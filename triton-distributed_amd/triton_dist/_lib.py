@@ -46,6 +46,7 @@ PROTOTYPES = {
     "tdist_gemm_chunk_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_producer_push_chunk": (_I, [_P, _P, _L, _P, _P, _I, _P]),
     "tdist_producer_push_peers": (_I, [_P, _P, _I, _I, _L, _L, _P, _I, _P, _P, _P, _L, ctypes.c_uint32, _L, _I, _P]),
+    "tdist_gather_shards": (_I, [_P, _P, _P, _I, _I, _L, _P, _P, _P]),
     "tdist_producer_mark": (_I, [_P, _P]),
     "tdist_producer_wait_until": (_I, [_P, _L, _P]),
     "tdist_flag_set": (_I, [_P, _I, _P]),
@@ -161,8 +162,9 @@ def ptr(t):
 
 def stream_ptr(stream=None):
     import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())   # (without a Stream object: 0.2 us for 1.3)
 
 
 def dtype_code(dtype):
