@@ -179,13 +179,14 @@ int tdist_producer_push_peers(void* workspace, const void* const* peer_src, int 
                               int32_t* counters, const int32_t* held, const uint64_t* stamp, int64_t ns_per_chunk,
                               uint32_t delay_seed, int64_t max_delay_ns, int workgroups_per_peer, void* stream);
 
-/* The shards of all ranks into the workspace in one launch on `stream`, without flags: what an all-gather of few rows
- * needs whose GEMM is queued behind it on the same stream (no counterpart in the reference, where every peer pushes for
- * itself). Shard r lands at workspace + r*rank_bytes; peer_src: device array of world_size device pointers (entry `rank`
- * unused: the own shard is read from `own`). rank_bytes a multiple of 16, all addresses 16-byte aligned. status not NULL:
+/* The shards of all ranks into the workspace in one launch on `stream`, without flags: what an all-gather needs whose
+ * GEMM is queued behind it on the same stream (no counterpart in the reference, where every peer pushes for itself).
+ * Shard r lands at workspace + r*rank_bytes; shards: HOST array of world_size (at most TDIST_GATHER_MAX_RANKS) device
+ * pointers, read before the call returns. rank_bytes a multiple of 16, all addresses 16-byte aligned. status not NULL:
  * the same launch retires it into first_error, as tdist_status_retire does. */
-int tdist_gather_shards(void* workspace, const void* const* peer_src, const void* own, int world_size, int rank,
-                        int64_t rank_bytes, int32_t* status, int32_t* first_error, void* stream);
+#define TDIST_GATHER_MAX_RANKS 64
+int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
+                        int32_t* first_error, void* stream);
 
 /* Link pacing for the one-GPU producer (no counterpart in the reference, whose chunks arrive over xGMI at the
  * link's rate: ~153 GB/s per peer). tdist_producer_mark stores the device's constant-rate wall clock into *stamp

@@ -373,7 +373,8 @@ __device__ __forceinline__ int chunk_of(const GemmParams& p, int oc) {
 }
 
 // kPlain: an instance for calls without flags and without a local shard (the GEMM-RS producer, plain GEMMs): no gating
-// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly).
+// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly; not the grouped
+// ones, whose row addresses are a load away).
 template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams p) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
@@ -623,7 +624,14 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         sidx = round_base + wg_pos;
         if (sidx >= total_sched) continue;
       }
-      if (!kGrouped && p.group_s > 1) {
+      if (kGrouped && kPlain && p.group_s > 1) {
+        // row blocks group_s at a time; the last group holds what is left of those in use
+        const int tpg = p.group_s * num_pid_n;
+        const int og = sidx / tpg, win = sidx - og * tpg;
+        const int rows_g = min(p.group_s, n_chunks - og * p.group_s);
+        within = win / rows_g;
+        oc = og * p.group_s + (win - within * rows_g);
+      } else if (!kGrouped && p.group_s > 1) {
         const int rows_g = p.group_s * cm, tpg = rows_g * num_pid_n;
         const int og = sidx / tpg, win = sidx - og * tpg;
         const int pn = win >> p.group_rows_shift, j = win & (rows_g - 1);
@@ -2258,20 +2266,39 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
       sk_attach(p, c.sk_workspace, 1);
     }
   }
-#define TDIST_GROUPED(EB, EH, E8, BM_, BN_, KB_, NST_)                                                          \
-  switch (elem) {                                                                                               \
-    case kElemBF16: return launch_gemm_cfg<EB, BM_, BN_, KB_, 2, 2, NST_, false, true>(p, grid, c.stream, who); \
-    case kElemF16: return launch_gemm_cfg<EH, BM_, BN_, KB_, 2, 2, NST_, false, true>(p, grid, c.stream, who);  \
-    default: return launch_gemm_cfg<E8, BM_, BN_, KB_, 2, 2, NST_, false, true>(p, grid, c.stream, who);        \
+#define TDIST_GROUPED(EB, EH, E8, BM_, BN_, KB_, NST_, PL_)                                                          \
+  switch (elem) {                                                                                                    \
+    case kElemBF16: return launch_gemm_cfg<EB, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who); \
+    case kElemF16: return launch_gemm_cfg<EH, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who);  \
+    default: return launch_gemm_cfg<E8, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who);        \
+  }
+  const bool plain = k128 && c.flags == nullptr && c.A_local == nullptr;
+  if (plain) {
+    // Nothing to wait for: an XCD's workgroups walk a block of tiles of few operand panels (rows + columns of tiles),
+    // as in an ungated GEMM, instead of one row block after the other (16 column tiles: 4 x 8 tiles, 12 panels, instead
+    // of 2 x 16, 18 panels). A group that spans experts fetches no more than single rows would.
+    const int per_xcd = di.num_xcds > 0 && cap_wgs % di.num_xcds == 0 ? cap_wgs / di.num_xcds : cap_wgs;
+    const int tiles_n = (int)ceil_div(c.N, BN);
+    double best = 0;
+    for (int rows = 1; rows <= 8; rows *= 2) {
+      const double cols = per_xcd / rows < tiles_n ? per_xcd / rows : tiles_n;
+      const double cost = (double)per_xcd / cols * c.block_size + cols * BN;
+      if (best == 0 || cost < 0.99 * best) {
+        best = cost;
+        p.group_s = rows;
+      }
+    }
   }
   if (c.block_size == 256) {
     if (!k128) return fail(TDIST_ERR_UNSUPPORTED, "%s: 256-row blocks need K*elem_size to be a multiple of 128 bytes", who);
-    TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 256, 256, 128, 5)
+    if (plain) TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 256, 256, 128, 5, true)
+    TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 256, 256, 128, 5, false)
   }
+  if (plain) TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 128, 256, 128, 5, true)
   if (k128) {  // 64 x 128 per wave on the split ring
-    TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 128, 256, 128, 5)
+    TDIST_GROUPED(ElemBF16N, ElemF16N, ElemFP8N, 128, 256, 128, 5, false)
   }
-  TDIST_GROUPED(ElemBF16, ElemF16, ElemFP8, 128, 128, 64, 4)
+  TDIST_GROUPED(ElemBF16, ElemF16, ElemFP8, 128, 128, 64, 4, false)
 #undef TDIST_GROUPED
 }
 

@@ -263,16 +263,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(24))) void prod
 // flight per lane. Bound by the launch at the sizes it is for (1.6 MB: 3 us); 64 MB: 25 us.
 struct GatherParams {
   unsigned char* workspace;
-  const unsigned char* const* peer_src;
-  const unsigned char* own;
+  const unsigned char* src[TDIST_GATHER_MAX_RANKS];   // (by value: no table in memory to keep in step, none to load first)
   long long rank_bytes;
-  int rank;
   int32_t *status, *first_error;   // optional: retired as by tdist_status_retire
 };
 __global__ __launch_bounds__(256) void gather_shards_kernel(const GatherParams p) {
   if (p.status != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) retire_status(p.status, p.first_error);
   const int r = blockIdx.y;
-  const int4v* const src = (const int4v*)(r == p.rank ? p.own : p.peer_src[r]);
+  const int4v* const src = (const int4v*)p.src[r];
   int4v* const dst = (int4v*)(p.workspace + r * p.rank_bytes);
   const long long n = p.rank_bytes / 16, step = (long long)gridDim.x * 1024;
   for (long long i0 = (long long)blockIdx.x * 1024 + threadIdx.x; i0 < n; i0 += step) {
@@ -292,14 +290,24 @@ using namespace tdist;
 
 extern "C" {
 
-int tdist_gather_shards(void* workspace, const void* const* peer_src, const void* own, int world_size, int rank, int64_t rank_bytes,
-                        int32_t* status, int32_t* first_error, void* stream) {
+int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
+                        int32_t* first_error, void* stream) {
   const char* who = "tdist_gather_shards";
-  if (!workspace || !peer_src || !own) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
-  if (world_size < 1 || rank < 0 || rank >= world_size) return fail(TDIST_ERR_INVALID, "%s: rank %d / world_size %d", who, rank, world_size);
-  if (rank_bytes <= 0 || rank_bytes % 16 != 0 || !aligned16(workspace) || !aligned16(own))
+  if (!workspace || !shards) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (world_size < 1 || world_size > TDIST_GATHER_MAX_RANKS)
+    return fail(TDIST_ERR_INVALID, "%s: world_size %d (1 .. %d)", who, world_size, TDIST_GATHER_MAX_RANKS);
+  if (rank_bytes <= 0 || rank_bytes % 16 != 0 || !aligned16(workspace))
     return fail(TDIST_ERR_UNSUPPORTED, "%s: shards of whole 16-byte pieces, 16-byte aligned", who);
-  GatherParams p = {(unsigned char*)workspace, (const unsigned char* const*)peer_src, (const unsigned char*)own, rank_bytes, rank, status, first_error};
+  GatherParams p = {};
+  p.workspace = (unsigned char*)workspace;
+  for (int r = 0; r < world_size; ++r) {
+    if (!shards[r]) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+    if (!aligned16(shards[r])) return fail(TDIST_ERR_UNSUPPORTED, "%s: shards of whole 16-byte pieces, 16-byte aligned", who);
+    p.src[r] = (const unsigned char*)shards[r];
+  }
+  p.rank_bytes = rank_bytes;
+  p.status = status;
+  p.first_error = first_error;
   const int64_t blocks = ceil_div(rank_bytes, 16 * 1024);
   hipLaunchKernelGGL(gather_shards_kernel, dim3((unsigned)(blocks < 256 ? blocks : 256), (unsigned)world_size), dim3(256), 0, (hipStream_t)stream, p);
   return launch_status(who);

@@ -46,7 +46,7 @@ PROTOTYPES = {
     "tdist_gemm_chunk_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_producer_push_chunk": (_I, [_P, _P, _L, _P, _P, _I, _P]),
     "tdist_producer_push_peers": (_I, [_P, _P, _I, _I, _L, _L, _P, _I, _P, _P, _P, _L, ctypes.c_uint32, _L, _I, _P]),
-    "tdist_gather_shards": (_I, [_P, _P, _P, _I, _I, _L, _P, _P, _P]),
+    "tdist_gather_shards": (_I, [_P, _P, _I, _L, _P, _P, _P]),
     "tdist_producer_mark": (_I, [_P, _P]),
     "tdist_producer_wait_until": (_I, [_P, _L, _P]),
     "tdist_flag_set": (_I, [_P, _I, _P]),
@@ -165,6 +165,23 @@ def stream_ptr(stream=None):
     if stream is not None:
         return stream.cuda_stream
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())   # (without a Stream object: 0.2 us for 1.3)
+
+
+GATHER_MAX_RANKS = 64
+
+
+def shard_table(own, peer_shards, rank, num_ranks):
+    """The host table of every rank's shard for tdist_gather_shards, or None where a shard is missing or does not lie on 16
+    bytes (the copies of the flag-gated path take any address)."""
+    if num_ranks > GATHER_MAX_RANKS or own.data_ptr() % 16 != 0:
+        return None
+    table = (ctypes.c_void_p * num_ranks)()
+    for r in range(num_ranks):
+        t = own if r == rank else peer_shards.get(r)
+        if t is None or t.data_ptr() % 16 != 0:
+            return None
+        table[r] = t.data_ptr()
+    return table
 
 
 def dtype_code(dtype):

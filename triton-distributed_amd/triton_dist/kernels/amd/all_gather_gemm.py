@@ -429,10 +429,10 @@ def _rows_are_at_hand(a, ctx):
     """Whether nothing asks for arrivals one chunk at a time: no pacing, no order, delays or withheld chunks, no copy engine
     and no producer kernel. The peers' shards then lie in this GPU's memory, complete, when the call is made."""
     return not (ctx.serial or ctx.preset_flags or ctx.producer_kernel or ctx.use_sdma or ctx.link_gbps > 0 or ctx.arrival_order is not None
-                or ctx.held_chunks or ctx.late_chunks_us or ctx.random_delay_us > 0) and ctx.peer_ptrs is not None and a.is_contiguous()
+                or ctx.held_chunks or ctx.late_chunks_us or ctx.random_delay_us > 0) and a.is_contiguous()
 
 
-def _gather_and_multiply(a, b, c, ctx, row_scale, col_scale):
+def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
     """One launch brings every rank's rows into the workspace, the next multiplies them, on one stream. With the rows at
     hand a gather at HBM speed is the shortest part of the call (C3's 134 MB: 45 us in front of 605), and a GEMM that shares
     the chip with copies, keeps 32 compute units free for them or waits for flags costs more than that at every size:
@@ -446,8 +446,8 @@ def _gather_and_multiply(a, b, c, ctx, row_scale, col_scale):
     stream = ctx.gemm_stream.cuda_stream
     if stream != current:
         ctx.gemm_stream.wait_stream(torch.cuda.current_stream())
-    _lib.call("tdist_gather_shards", workspace.data_ptr(), ctx.peer_ptrs.data_ptr(), a.data_ptr(), num_ranks, rank,
-              M_per_rank * K * a.element_size(), ctx.status.data_ptr(), ctx.status.data_ptr() + 8, stream)
+    _lib.call("tdist_gather_shards", workspace.data_ptr(), shards, num_ranks, M_per_rank * K * a.element_size(),
+              ctx.status.data_ptr(), ctx.status.data_ptr() + 8, stream)
     gated_gemm(workspace if workspace.shape[0] == M else workspace[:M], None, 0, b, c, None, 0, rank, num_ranks, row_scale=row_scale,
                col_scale=col_scale, sk_workspace=ctx.sk_workspace, stream=ctx.gemm_stream)
     if stream != current:
@@ -481,10 +481,11 @@ def ag_gemm_intra_node(a, b, transe_b, ctx, *, row_scale=None, col_scale=None):
     out_dtype = a.dtype if a.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
     C = torch.empty([ctx.num_ranks * M_per_rank, N_per_rank], dtype=out_dtype, device=a.device)
 
-    if ctx.num_ranks > 1 and _rows_are_at_hand(a, ctx) and len(ctx.peer_shards) == ctx.num_ranks - 1:
+    shards = _lib.shard_table(a, ctx.peer_shards, ctx.rank, ctx.num_ranks) if ctx.num_ranks > 1 and _rows_are_at_hand(a, ctx) else None
+    if shards is not None and (M_per_rank * a.shape[1] * a.element_size()) % 16 == 0:
         assert a.shape[1] == b.shape[1], "Incompatible dimensions"
         assert a.dtype == b.dtype, "Incompatible dtypes"
-        _gather_and_multiply(a, b, C, ctx, row_scale, col_scale)
+        _gather_and_multiply(a, b, C, ctx, shards, row_scale, col_scale)
         return C
     ag_gemm_intra_node_op(a, b, C, ctx.rank, ctx.num_ranks, ctx.workspace_tensors, ctx.one, ctx.barrier_tensors,
                           ctx.comm_buf_ptr, ag_streams=ctx.ag_streams, gemm_stream=ctx.gemm_stream, serial=ctx.serial,

@@ -14,7 +14,8 @@ from typing import Dict, List, Optional
 import torch
 
 from triton_dist import _lib
-from triton_dist.kernels.amd.allgather_group_gemm import group_gemm_gated, sort_topk_ids_align_block_size
+from triton_dist.kernels.amd.allgather_group_gemm import (LocalRowBlocks, group_gemm_gated, local_row_blocks,
+                                                          sort_topk_ids_align_block_size)
 from triton_dist.kernels.amd.low_latency_all_to_all import moe_weighted_combine
 
 
@@ -49,6 +50,7 @@ class MoEAgScatterGroupGemmPrecomputeContext:
     TOP_K: int = 0
     BLOCK_M: int = 0
     num_tokens_per_rank: int = 0
+    local_blocks: Optional[LocalRowBlocks] = None   # the same rows in blocks without rank segments, for this GPU's GEMM
 
 
 def precompute_context_helper(pg, num_ranks, topk, num_tokens_per_rank, num_experts, input_dtype, device, router_logits,
@@ -104,6 +106,7 @@ def create_moe_rs_context(pg, local_rank, world_size, local_world_size, max_toke
     assert num_tokens_per_rank * world_size <= max_token_num and max_token_num % world_size == 0
     pre = precompute_context_helper(pg, world_size, topk, num_tokens_per_rank, num_experts, input_dtype, device,
                                     router_logits, BLOCK_M=moe_block_size, peer_router_logits=peer_router_logits, rank=rank)
+    pre.local_blocks = local_row_blocks(pre.full_topk_ids, num_experts, hidden_dim, pre.full_sorted_token_ids)
     M = num_tokens_per_rank * world_size
     rs_buffers: List[Optional[torch.Tensor]] = [None] * world_size
     rs_buffers[rank] = torch.zeros([max_token_num, hidden_dim], dtype=output_dtype, device=device)
@@ -137,11 +140,17 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     assert a.shape[0] == M * topk and a.dtype == b.dtype and a.shape[1] == b.shape[1]
     hidden = b.shape[2]
     out = ctx.final_output_buffer[:M * topk, :hidden]
-    flags = None
-    # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local
-    group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
-                     pre.block_wait_barriers, pre.full_num_tokens_post_padded_list, pre.BLOCK_M, pre.full_numel, 1,
-                     pre.num_tokens_per_rank * topk, 0, flags, rank, sk_workspace=ctx.sk_workspace)
+    blocks = pre.local_blocks
+    # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local, and
+    # blocks that run across the rank segments hold less padding
+    if blocks is not None and blocks.stand_for(pre.full_sorted_token_ids, a.shape[1] * a.element_size()):
+        group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, blocks.sorted_ids, blocks.expert_ids, blocks.segment_ids,
+                         blocks.num_tokens_post_padded, blocks.block_size, pre.full_numel, 1, M * topk, 0, None, rank,
+                         sk_workspace=ctx.sk_workspace)
+    else:
+        group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
+                         pre.block_wait_barriers, pre.full_num_tokens_post_padded_list, pre.BLOCK_M, pre.full_numel, 1,
+                         pre.num_tokens_per_rank * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
     y = moe_weighted_combine(None, out, None, ctx.identity_index, ctx.topk_weight_f32, from_slots=False)   # [M, hidden]
     m_per = M // world_size
     buf = ctx.rs_buffers[ctx.rank]
