@@ -331,6 +331,12 @@ int tdist_moe_dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, co
                                        int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
                                        int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
                                        int32_t* gather_idx, void* stream);
+/* The same from 64-bit ids as torch.topk gives them (their low words count, as after a conversion to 32 bits). */
+int tdist_moe_dispatch_tokens_from_ids64(const void* tokens, int64_t row_bytes, const float* token_scales,
+                                         const int64_t* ids, int topk, int64_t n_tokens, int world_size,
+                                         int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
+                                         int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
+                                         int32_t* gather_idx, void* stream);
 
 /* Compaction of the slots into one [sum, row_bytes] tensor in destination order
  * (all_to_all_post_process, low_latency_all_to_all.py:251-270): output row p comes from slot row

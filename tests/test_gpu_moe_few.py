@@ -1,0 +1,55 @@
+"""MoE dispatch from expert ids where rows are shared by several waves (few tokens), and align / sort where padding outweighs
+the entries: bit-exact against the oracle."""
+import pytest
+import torch
+
+from oracle import golden
+from tests.conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+# one token; whole and broken workgroups; windows of 1 to 7 KB with a last one that is empty, partial or a single piece;
+# rows without 16-byte pieces; the last size that is cut finer and the first that is not (1024 tokens of one window)
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("T,topk,G,W,H", [(1, 8, 256, 32, 7168), (2, 1, 8, 2, 1024), (15, 3, 16, 4, 1040), (16, 8, 64, 8, 2048), (17, 8, 64, 8, 5120),
+                                          (128, 8, 256, 32, 7168), (33, 5, 8, 2, 8208), (31, 4, 8, 2, 16384), (3, 2, 4, 2, 100000),
+                                          (9, 3, 4, 4, 52), (40, 2, 4, 4, 3001), (1007, 2, 32, 8, 1040), (1009, 2, 32, 8, 1040)])
+def test_dispatch_from_few_ids(cuda, wide, T, topk, G, W, H):
+    from triton_dist.kernels.amd import create_all_to_all_context, fast_all_to_all
+    announce("dispatch from few ids T=%d topk=%d G=%d W=%d H=%d wide=%s" % (T, topk, G, W, H, wide))
+    g = torch.Generator().manual_seed(T + H)
+    ids = golden.random_distinct_experts(T, G, topk, g)
+    x = torch.randint(0, 256, (T, H), generator=g, dtype=torch.uint8)
+    scale = torch.rand(T, generator=g)
+    max_m = T * topk
+    ctx = create_all_to_all_context(max_m, H, 0, G, W, G // W, dtype=torch.float8_e4m3fn)
+    ctx.recv_buf.view(torch.uint8).fill_(0xAB)
+    dev_ids = ids.to(torch.int64 if wide else torch.int32).to(cuda)
+    splits, recv, scales = fast_all_to_all(ctx, x.to(cuda).view(torch.float8_e4m3fn), None, scale.to(cuda), expert_ids=dev_ids)
+    torch.cuda.synchronize()
+    w_splits, w_cumsum, w_scatter, w_gather, _ = golden.moe_preprocess(ids, G)
+    for got, want in zip(ctx.last_index, (w_splits, w_cumsum, w_scatter, w_gather)):
+        assert torch.equal(got.cpu(), want)
+    assert torch.equal(splits.cpu(), w_splits)
+    recv, scales, rows = recv.view(torch.uint8).cpu(), scales.cpu(), x[w_gather.long()]
+    for d in range(W):
+        lo, hi = int(w_cumsum[d * (G // W)]), int(w_cumsum[(d + 1) * (G // W)])
+        assert torch.equal(recv[d * max_m:d * max_m + hi - lo], rows[lo:hi])
+        assert torch.equal(scales[d * max_m:d * max_m + hi - lo], scale[w_gather.long()][lo:hi])
+        assert (recv[d * max_m + hi - lo:(d + 1) * max_m] == 0xAB).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("R,T,topk,E,BS", [(8, 1, 8, 256, 128), (8, 125, 8, 256, 128), (1, 3, 2, 16, 256), (8, 2, 2, 64, 1024), (4, 1031, 3, 100, 64)])
+def test_align_sort_with_more_padding_than_entries(cuda, dtype, R, T, topk, E, BS):
+    from triton_dist.kernels.amd import sort_topk_ids_align_block_size
+    announce("align R=%d T=%d topk=%d E=%d BS=%d" % (R, T, topk, E, BS))
+    ids = golden.random_distinct_experts(R * T, E, topk, torch.Generator().manual_seed(T))
+    want = golden.sort_topk_ids_align_block_size(ids, E, R, T, BS)
+    got = sort_topk_ids_align_block_size(ids.to(dtype).to(cuda), E, R, T, BS)
+    nb = want[4] // BS
+    assert int(got[4].item()) == want[4]
+    assert torch.equal(got[0].cpu(), want[0])   # the whole buffer, padding included
+    assert torch.equal(got[1].cpu()[:nb], want[1]) and torch.equal(got[2].cpu()[:nb], want[2])
+    assert torch.equal(got[3].cpu(), want[3])

@@ -301,6 +301,7 @@ __global__ __launch_bounds__(kThreads) void moe_index_fused_kernel(const int32_t
 #pragma unroll
     for (int u = 0; u < kVecBatch; ++u) {
       const int64_t vi = v0 + (int64_t)u * kThreads;
+      if (vi - lane >= n_vec) break;   // (nothing left for this wave)
       int32_t* const row = s_out + (vi * 4 < own_lo ? 0 : G);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -669,16 +670,23 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(const unsigned
 // entries, workgroup 0 the splits and cumsum.
 // A workgroup is kFdWaves waves; wave w stands for (token, 8 KB window) unit w of the workgroup, as in
 // moe_dispatch_tokens_kernel. The window-0 wave of a token counts and ranks that token's ids.
+// Few tokens: windows of `vecs` < 8 KB, so that a row is shared by several waves and the rows by more workgroups. What 16
+// whole rows per workgroup cost a decode step of 128 tokens x 8 copies of 7168 B is eight compute units storing 7.3 MB:
+// 14.5 us, against 12.2 us with eight waves to a row (64 workgroups; what is left is the chain ids, counts, scan, stores).
+// 64-bit ids are read as they are (a conversion of 1024 of them in front: 3 us and a launch).
 constexpr int kFdWaves = 16, kFdThreads = kFdWaves * 64;
 constexpr int64_t kFusedDispatchMaxIds = 65536;
 
-template <bool kVec16>
+// kFew: windows of less than 8 KB (the others' code is left without the tests for them: they cost a prefill's 4096 rows
+// and combine 9 of 110 us). kWide: 64-bit ids, of which the low words count.
+template <bool kVec16, bool kFew, bool kWide>
 __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
     const unsigned char* __restrict__ tokens, int64_t row_bytes, const float* __restrict__ scales,
     const int32_t* __restrict__ ids, int topk, int64_t n_tokens, int G, int nbits, int W, int Er, int max_m, int windows,
-    unsigned char* __restrict__ slot_rows, float* __restrict__ slot_scales, int32_t* __restrict__ splits_out,
+    int few_vecs, unsigned char* __restrict__ slot_rows, float* __restrict__ slot_scales, int32_t* __restrict__ splits_out,
     int32_t* __restrict__ splits, int32_t* __restrict__ cumsum, int32_t* __restrict__ scatter_idx,
     int32_t* __restrict__ gather_idx) {
+  const int vecs = kFew ? few_vecs : 8;   // 16-byte loads per lane and window
   // [3][G] counters: ids in front of this workgroup's range, its own, ids behind it; [G + 1] expert starts (cumsum);
   // then this workgroup's own ids in flat order, padded to a multiple of four with -1
   extern __shared__ int32_t s_fd[];
@@ -700,7 +708,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   const int64_t own_lo = (int64_t)blockIdx.x * own_n, own_hi = own_lo + own_n;
   const int own_f = (wave / windows) * topk + lane;   // this lane's entry among the workgroup's own, in flat order
   int e = -1;
-  if (live && lane < topk) e = ids[t * topk + lane];
+  if (live && lane < topk) e = ids[(t * topk + lane) << (kWide ? 1 : 0)];
   if (e < 0 || e >= G) e = -1;
   constexpr int kBatch = 8;
   const int64_t n_vec = (n + 3) / 4;
@@ -712,9 +720,16 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
       const int64_t vi = v0 + (int64_t)u * kFdThreads;
       q[u] = int4v{-1, -1, -1, -1};
       if (vi < n_vec) {
-        if (vec_ok && vi * 4 + 3 < n) q[u] = ((const int4v*)ids)[vi];
-        else
-          for (int j = 0; j < 4; ++j) q[u][j] = vi * 4 + j < n ? ids[vi * 4 + j] : -1;
+        if (vec_ok && vi * 4 + 3 < n) {
+          if constexpr (kWide) {
+            const int4v lo = ((const int4v*)ids)[2 * vi], hi = ((const int4v*)ids)[2 * vi + 1];
+            q[u] = int4v{lo[0], lo[2], hi[0], hi[2]};
+          } else {
+            q[u] = ((const int4v*)ids)[vi];
+          }
+        } else {
+          for (int j = 0; j < 4; ++j) q[u][j] = vi * 4 + j < n ? ids[(vi * 4 + j) << (kWide ? 1 : 0)] : -1;
+        }
       }
     }
   };
@@ -725,6 +740,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int64_t vi = v0 + (int64_t)u * kFdThreads;
+      if (kFew && vi - lane >= n_vec) break;   // (nothing left for this wave)
       const int64_t i0 = vi * 4;
       if (i0 + 3 < own_lo || i0 >= own_hi) {
         int32_t* const row = i0 < own_lo ? s_before : s_behind;
@@ -747,14 +763,14 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   // the row's loads go out behind the ids' (loads return in order, and the counting only needs the ids: it runs while
   // the row is on its way)
   const int n16 = (int)(row_bytes >> 4);
-  const int base = win * 512;
+  const int base = win * vecs * 64;
   int4v v[8];
   if (kVec16 && live) {
     const int4v* s16 = (const int4v*)(tokens + t * row_bytes);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int c = base + j * 64 + lane;
-      if (c < n16) v[j] = s16[c];
+      if ((!kFew || j < vecs) && c < n16) v[j] = s16[c];
     }
   }
   for (int g = threadIdx.x; g < 3 * G; g += kFdThreads) s_fd[g] = 0;
@@ -833,7 +849,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int c = base + j * 64 + lane;
-        if (c < n16) __builtin_nontemporal_store(v[j], d16 + c);
+        if ((!kFew || j < vecs) && c < n16) __builtin_nontemporal_store(v[j], d16 + c);
       }
     }
   } else {
@@ -842,7 +858,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
       const int32_t dst_row = __shfl(my_dst, k);
       if (dst_row < 0) continue;
       unsigned char* dst = slot_rows + (int64_t)dst_row * row_bytes;
-      for (int64_t c = (int64_t)win * 8192 + lane; c < row_bytes && c < (int64_t)(win + 1) * 8192; c += 64) dst[c] = src[c];
+      for (int64_t c = (int64_t)base * 16 + lane; c < row_bytes && c < ((int64_t)base + vecs * 64) * 16; c += 64) dst[c] = src[c];
     }
   }
 }
@@ -1174,6 +1190,10 @@ __global__ __launch_bounds__(kPlaceThreads) void moe_align_place_kernel(
 // own, those behind), works out the padded prefix over the G = R * E groups for itself and places its own entries;
 // the padding positions, the per-block expert / segment ids and the positions behind the padded total (up to fill_n)
 // are shared out among the blocks, groups in turn; block 0 writes the blocks per segment and the padded total.
+// Many groups of few entries: the padding is the larger part (1000 tokens x 8, 256 experts x 8 segments, blocks of 128:
+// 260 000 positions for 8000 entries), so the launch has a block per kAlignFillPerBlock positions even where the entries
+// alone need fewer: blocks beyond the entries count like the others and only fill (16 blocks 20.9 us, 131 blocks 12.1).
+constexpr int kAlignFillPerBlock = 2048;
 template <int kThreads, int kPerWave, bool kIds64>
 __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
     const void* __restrict__ ids_v, int64_t n, int per_iter, int E, int R, int nbits, int block_size,
@@ -1248,6 +1268,7 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
 #pragma unroll
     for (int u = 0; u < kVecBatch; ++u) {
       const int64_t vi = v0 + (int64_t)u * kThreads;
+      if (vi - lane >= n_vec) break;   // (nothing left for this wave)
       int32_t* const row = s_out + (vi * 4 < own_lo ? 0 : G);
       const uint32_t i0 = (uint32_t)(vi * 4);
       const uint32_t seg = __umulhi(i0, seg_magic);
@@ -1556,12 +1577,10 @@ int tdist_moe_dispatch_tokens(const void* tokens, int64_t row_bytes, const float
   return launch_status("tdist_moe_dispatch_tokens");
 }
 
-int tdist_moe_dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const float* token_scales,
-                                       const int32_t* ids, int topk, int64_t n_tokens, int world_size,
-                                       int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
-                                       int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
-                                       int32_t* gather_idx, void* stream) {
-  const char* who = "tdist_moe_dispatch_tokens_from_ids";
+static int dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const float* token_scales, const int32_t* ids,
+                                    int ids_wide, int topk, int64_t n_tokens, int world_size, int experts_per_rank, int max_m,
+                                    void* slot_rows, float* slot_scales, int32_t* splits_out, int32_t* splits, int32_t* cumsum,
+                                    int32_t* scatter_idx, int32_t* gather_idx, void* stream, const char* who) {
   if (!tokens || !ids || !slot_rows || !cumsum || !scatter_idx || !gather_idx) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
   if ((token_scales != nullptr) != (slot_scales != nullptr))
     return fail(TDIST_ERR_INVALID, "%s: token_scales and slot_scales go together", who);
@@ -1572,27 +1591,60 @@ int tdist_moe_dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, co
   if (G64 > kMoeMaxExperts) return fail(TDIST_ERR_UNSUPPORTED, "%s: num_experts %lld > %d", who, (long long)G64, kMoeMaxExperts);
   if ((int64_t)world_size * max_m > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: world_size * max_m too large", who);
   const int G = (int)G64;
-  const int windows = (int)ceil_div(row_bytes, 8192);
+  int windows = (int)ceil_div(row_bytes, 8192);
   const int64_t lds = ((int64_t)3 * G + ((G + 1 + 3) & ~3) + kFdWaves * topk + 8 + 64) * 4;   // (+ a word per lane for what is not counted)
   if (n_tokens * topk > kFusedDispatchMaxIds || windows > kFdWaves || kFdWaves % windows != 0 || lds > 160 * 1024 - 256)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: more than %lld ids, rows above %d bytes (or no power-of-two number of 8 KB windows), or too "
                 "many experts for one workgroup's counters: use tdist_moe_scatter_index + tdist_moe_dispatch_tokens", who,
                 (long long)kFusedDispatchMaxIds, kFdWaves * 8192);
+  // Few tokens: smaller windows, as long as there are fewer workgroups than a quarter of the compute units (every
+  // workgroup counts all ids, so more of them is not free) and a window holds a KB.
+  int vecs = 8;
+  const DeviceInfo& di = device_info();
+  const int64_t cus = di.ok == 1 ? di.num_cus : 256;
+  while (windows < kFdWaves && vecs > 1 && ceil_div(n_tokens * windows, kFdWaves) * 4 < cus) {
+    windows *= 2;
+    vecs = (int)ceil_div(row_bytes, (int64_t)windows * 1024);
+  }
   const int64_t units = (n_tokens > 0 ? n_tokens : 1) * windows;
   const int64_t blocks = ceil_div(units, kFdWaves);
   const bool vec = (row_bytes % 16 == 0) && aligned16(tokens) && aligned16(slot_rows);
-  auto kern = vec ? moe_dispatch_fused_kernel<true> : moe_dispatch_fused_kernel<false>;
-  static bool attr_set[2] = {false, false};
-  if (!attr_set[vec]) {
+  const bool few = vecs < 8;
+  auto kern = !vec ? (ids_wide ? moe_dispatch_fused_kernel<false, true, true> : moe_dispatch_fused_kernel<false, true, false>)
+            : few  ? (ids_wide ? moe_dispatch_fused_kernel<true, true, true> : moe_dispatch_fused_kernel<true, true, false>)
+                   : (ids_wide ? moe_dispatch_fused_kernel<true, false, true> : moe_dispatch_fused_kernel<true, false, false>);
+  static bool attr_set[6] = {false, false, false, false, false, false};
+  const int which = (!vec ? 0 : few ? 2 : 4) + ids_wide;
+  if (!attr_set[which]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256) != hipSuccess)
       return fail(TDIST_ERR_LAUNCH, "%s: cannot reserve LDS", who);
-    attr_set[vec] = true;
+    attr_set[which] = true;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kFdThreads), (size_t)lds, (hipStream_t)stream,
                      (const unsigned char*)tokens, row_bytes, token_scales, ids, topk, n_tokens, G, id_bits(G), world_size,
-                     experts_per_rank, max_m, windows, (unsigned char*)slot_rows, slot_scales, splits_out, splits, cumsum,
+                     experts_per_rank, max_m, windows, vecs, (unsigned char*)slot_rows, slot_scales, splits_out, splits, cumsum,
                      scatter_idx, gather_idx);
   return launch_status(who);
+}
+
+int tdist_moe_dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const float* token_scales,
+                                       const int32_t* ids, int topk, int64_t n_tokens, int world_size,
+                                       int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
+                                       int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
+                                       int32_t* gather_idx, void* stream) {
+  return dispatch_tokens_from_ids(tokens, row_bytes, token_scales, ids, 0, topk, n_tokens, world_size, experts_per_rank, max_m,
+                                  slot_rows, slot_scales, splits_out, splits, cumsum, scatter_idx, gather_idx, stream,
+                                  "tdist_moe_dispatch_tokens_from_ids");
+}
+
+int tdist_moe_dispatch_tokens_from_ids64(const void* tokens, int64_t row_bytes, const float* token_scales,
+                                         const int64_t* ids, int topk, int64_t n_tokens, int world_size,
+                                         int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
+                                         int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
+                                         int32_t* gather_idx, void* stream) {
+  return dispatch_tokens_from_ids(tokens, row_bytes, token_scales, (const int32_t*)ids, 1, topk, n_tokens, world_size,
+                                  experts_per_rank, max_m, slot_rows, slot_scales, splits_out, splits, cumsum, scatter_idx,
+                                  gather_idx, stream, "tdist_moe_dispatch_tokens_from_ids64");
 }
 
 int tdist_moe_post_process(const void* slot_rows, int64_t row_bytes, const float* slot_scales, const int32_t* splits,
@@ -1742,7 +1794,9 @@ int tdist_moe_align_block_size(const void* topk_ids, int ids_int64, int64_t n_to
           return fail(TDIST_ERR_LAUNCH, "%s: cannot reserve LDS for the align kernel", who);
         attr_set[which] = true;
       }
-      const int64_t nblk = ceil_div(n1, form == 1 ? kFusedThreads : 2 * kFusedThreads);
+      const int64_t for_entries = ceil_div(n1, form == 1 ? kFusedThreads : 2 * kFusedThreads), cus = device_info().num_cus;
+      const int64_t for_fill = ceil_div(sorted_fill, kAlignFillPerBlock) < cus ? ceil_div(sorted_fill, kAlignFillPerBlock) : cus;
+      const int64_t nblk = for_entries > for_fill ? for_entries : for_fill;
       hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kFusedThreads), (size_t)kRows * G * 4 + 256, st, topk_ids, n_total,
                          (int)per_iter, num_experts, num_iterations, id_bits((int)G), block_size, sorted_token_ids, sorted_fill,
                          expert_ids, block_barrier_ids, rank_block_num, total_tokens_post_pad, seg_magic);

@@ -315,7 +315,8 @@ def _fast_all_to_all_from_ids(ctx, send_tensor, send_scale, expert_ids):
         ctx.last_index = (splits_i, cumsum, scatter, gather)
         return fast_all_to_all(ctx, send_tensor, cumsum, send_scale, scatter_index=scatter)
     _ensure_index_sets(ctx, T, topk, G, send_tensor.device)
-    ids = _staged_ids(ctx, expert_ids)
+    wide = expert_ids.dtype == torch.int64 and expert_ids.is_contiguous()   # (torch.topk's ids, read as they are)
+    ids = expert_ids if wide else _staged_ids(ctx, expert_ids)
     which = ctx.index_calls % 2
     ctx.index_calls += 1
     splits_i, cumsum, scatter, gather, _ = ctx.index_sets[which]
@@ -329,7 +330,7 @@ def _fast_all_to_all_from_ids(ctx, send_tensor, send_scale, expert_ids):
     recv = ctx.recv_buf[act_pos * rows:(act_pos + 1) * rows, :]
     scale_recv = ctx.scale_recv_buf[act_pos * rows:(act_pos + 1) * rows]
     splits = ctx.split_recv_buf[act_pos * G:(act_pos + 1) * G]
-    _lib.call("tdist_moe_dispatch_tokens_from_ids", send_tensor.data_ptr(), row_bytes, _lib.ptr(send_scale), ids.data_ptr(),
+    _lib.call("tdist_moe_dispatch_tokens_from_ids64" if wide else "tdist_moe_dispatch_tokens_from_ids", send_tensor.data_ptr(), row_bytes, _lib.ptr(send_scale), ids.data_ptr(),
               topk, T, ctx.WORLD_SIZE, ctx.experts_per_rank, ctx.max_m, recv.data_ptr(),
               scale_recv.data_ptr() if with_scale else None, splits.data_ptr(), splits_i.data_ptr(), cumsum.data_ptr(),
               scatter.data_ptr(), gather.data_ptr(), _lib.stream_ptr())
