@@ -74,6 +74,7 @@ struct GemmParams {
   const int32_t* post_pad;       // device scalar: rows of the sorted space in use (a multiple of BM)
   int64_t b_expert_stride_b;     // bytes between the experts' weight matrices
   int num_valid, topk, first_block, a_rows;
+  uint32_t topk_magic;   // kPlain: ceil(2^32 / topk); the host takes those instances while num_valid * topk < 2^32
   // Split rounds (sk_ctrl != NULL: the caller handed in a workspace). A tile may be cut along K into s = 2, 4 or 8
   // equal pieces (at least kSkMinPiece K tiles each), one per workgroup: workgroups s*t .. s*t+s-1 of the round share
   // tile t. Every piece writes its fp32 accumulators (register order) to slot [workgroup] of sk_partials and raises
@@ -373,8 +374,7 @@ __device__ __forceinline__ int chunk_of(const GemmParams& p, int oc) {
 }
 
 // kPlain: an instance for calls without flags and without a local shard (the GEMM-RS producer, plain GEMMs): no gating
-// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly; not the grouped
-// ones, whose row addresses are a load away).
+// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly).
 template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams p) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
@@ -572,11 +572,68 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
   // and waits for A(0) and B(0) alone: the epilogue's stores, issued behind those loads, are still on their way then
   // and have the whole first K tile to be acknowledged (loads and stores retire in order through one counter, so a
   // prologue that issues its loads behind the stores waits for every store of the tile before it).
-  constexpr bool kEarly = kPlain && C::kSplit && !kGrouped && kFixedAcc && C::kWaves <= 4 && C::kRowPieces == C::kEpiChunks &&
+  constexpr bool kEarly = kPlain && C::kSplit && kFixedAcc && C::kWaves <= 4 && C::kRowPieces == C::kEpiChunks &&
                           2 * C::kABytes >= C::kWaves * 64 * C::kEpiPitch && C::kAInstr == C::kBInstr;
   constexpr int kEpiStores = (C::kWaveM / 32) * 32 * C::kEpiChunks / 64;   // 16-byte stores per wave and tile
   static_assert(!kEarly || C::kBInstr + kEpiStores + C::kAInstr < 64, "vmcnt is a 6-bit counter");
   bool prefetched = false;   // this tile's A(0), B(0), B(1) were issued by the tile before
+  // Grouped, nothing to wait for (kFlat): a tile's row ids, its rows' offsets and its expert, carried over from the tile
+  // before where that has fetched them for its early loads, so that such a tile starts without a trip to memory. A lane
+  // holds the ids of rows `lane` (and 64 + lane) of its wave's rows; the epilogue gets a row's id from there by a
+  // permutation. With early loads padding reads the row of the block's first id and stores there: the same bits to the
+  // same place, so that no store is conditional (which the wait behind those loads could not count); without, it reads
+  // its segment's first row, its id is -1 and it stores nothing.
+  // 16384 x 1792 x 4096 / 16384 x 4096 x 1792 over 8 experts, 256 x 256 tiles: 210 -> 197 and 260 -> 232 us.
+  constexpr bool kFlat = kGrouped && kPlain;
+  constexpr bool kFlatSkips = kFlat && !kEarly;
+  constexpr int kIdRegs = kFlat ? C::kWaveM / 64 : 1;
+  int row_id[kIdRegs] = {0};
+  uint32_t a_off_carried[kFlat ? C::kAInstr : 1] = {0};
+  int first_id = 0, tile_expert = 0;
+  auto flat_token = [&](int sid, int first, int padding_token) -> int {
+    if (sid >= p.num_valid) {
+      if (kFlatSkips || first >= p.num_valid) return padding_token;   // (or a block without a valid first row)
+      sid = first;
+    }
+    return p.topk == 1 ? sid : (int)__umulhi((uint32_t)sid, p.topk_magic);
+  };
+  // block and columns of the tile behind schedule index sidx
+  auto flat_locate = [&](int sidx, int& block, int& column) {
+    int oc;
+    if (p.group_s > 1) {
+      // row blocks group_s at a time; the last group holds what is left of those in use
+      const int tpg = p.group_s * num_pid_n;
+      const int og = sidx / tpg, win = sidx - og * tpg;
+      const int rows_g = min(p.group_s, n_chunks - og * p.group_s);
+      column = win / rows_g;
+      oc = og * p.group_s + (win - column * rows_g);
+    } else {
+      oc = sidx / num_pid_n;
+      column = sidx - oc * num_pid_n;
+    }
+    block = (oc + p.first_block) % n_chunks;
+  };
+  auto flat_fetch = [&](int block, int& first, int& expert, int (&ids)[kIdRegs], uint32_t (&off)[kFlat ? C::kAInstr : 1]) {
+    const int32_t* const bids = p.sorted_ids + (int64_t)block * BM;
+    int raw[kFlat ? C::kAInstr : 1];
+#pragma unroll
+    for (int t = 0; t < (kFlat ? C::kAInstr : 1); ++t) raw[t] = bids[(wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row];
+#pragma unroll
+    for (int q = 0; q < kIdRegs; ++q) ids[q] = bids[wm * C::kWaveM + q * 64 + lane];
+    first = __builtin_amdgcn_readfirstlane(bids[0]);
+    expert = __builtin_amdgcn_readfirstlane(p.block_expert[block]);
+    int padding_token = 0;
+    if (kFlatSkips || first >= p.num_valid) padding_token = p.block_segment[block] * p.m_per_rank;
+#pragma unroll
+    for (int q = 0; q < kIdRegs; ++q)
+      if (ids[q] >= p.num_valid) ids[q] = kFlatSkips ? -1 : first;
+#pragma unroll
+    for (int t = 0; t < (kFlat ? C::kAInstr : 1); ++t) {
+      const int r = (wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row;
+      const int gr = min(max(flat_token(raw[t], first, padding_token), 0), p.a_rows - 1);
+      off[t] = (uint32_t)gr * (uint32_t)p.lda_b + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
+    }
+  };
   // tile of C behind schedule index sidx (ungated calls)
   auto locate = [&](int sidx, int& tm0, int& tn0) -> bool {
     const int toc = sidx / tiles_per_chunk, twithin = sidx - toc * tiles_per_chunk;
@@ -624,13 +681,8 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         sidx = round_base + wg_pos;
         if (sidx >= total_sched) continue;
       }
-      if (kGrouped && kPlain && p.group_s > 1) {
-        // row blocks group_s at a time; the last group holds what is left of those in use
-        const int tpg = p.group_s * num_pid_n;
-        const int og = sidx / tpg, win = sidx - og * tpg;
-        const int rows_g = min(p.group_s, n_chunks - og * p.group_s);
-        within = win / rows_g;
-        oc = og * p.group_s + (win - within * rows_g);
+      if constexpr (kFlat) {
+        flat_locate(sidx, oc, within);   // (oc: the row block itself)
       } else if (!kGrouped && p.group_s > 1) {
         const int rows_g = p.group_s * cm, tpg = rows_g * num_pid_n;
         const int og = sidx / tpg, win = sidx - og * tpg;
@@ -643,13 +695,15 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       }
     }
     const int KTp = kb - ka;
-    const int chunk = kGrouped ? (oc + p.first_block) % n_chunks : arr_chunk >= 0 ? arr_chunk : chunk_of(p, oc);
+    const int chunk = kFlat ? oc : kGrouped ? (oc + p.first_block) % n_chunks : arr_chunk >= 0 ? arr_chunk : chunk_of(p, oc);
     const int pid_m = chunk * cm + within % cm;
     const int pid_n = within / cm;
     if (pid_m >= num_pid_m) continue;
     const int m0 = pid_m * BM, n0 = pid_n * BN;
     int segment = 0;  // grouped: rank segment of this row block
-    if constexpr (kGrouped) {
+    if constexpr (kFlat) {
+      if (!(kEarly && prefetched)) flat_fetch(pid_m, first_id, tile_expert, row_id, a_off_carried);
+    } else if constexpr (kGrouped) {
       if (m0 >= __builtin_nontemporal_load(p.post_pad)) continue;  // (written by an earlier kernel of the stream)
       segment = p.block_segment[pid_m];
     }
@@ -705,11 +759,15 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     const int a_g0 = kGrouped ? 0 : min(m0 - a_row_off, a_row_max), b_g0 = min(n0, p.N - 1);
     const unsigned char* const a_base = Arows + (int64_t)a_g0 * a_ld + (int64_t)ka * KB;
     const unsigned char* b_base_ = p.B + (int64_t)b_g0 * p.ldb_b + (int64_t)ka * KB;
-    if constexpr (kGrouped) b_base_ += (int64_t)p.block_expert[pid_m] * p.b_expert_stride_b;
+    if constexpr (kGrouped) b_base_ += (int64_t)(kFlat ? tile_expert : p.block_expert[pid_m]) * p.b_expert_stride_b;
     const unsigned char* const b_base = b_base_;
     uint32_t a_off[C::kAInstr], b_off[C::kBInstr];
 #pragma unroll
     for (int t = 0; t < C::kAInstr; ++t) {
+      if constexpr (kFlat) {
+        a_off[t] = a_off_carried[t];
+        continue;
+      }
       const int r = (wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row;  // row within the tile
       int gr;
       if constexpr (kGrouped) {
@@ -1182,10 +1240,30 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     bool early = false;
     const unsigned char* a_base_n = a_base;
     const unsigned char* b_base_n = b_base;
+    int row_id_n[kIdRegs] = {0}, first_id_n = 0, tile_expert_n = 0;
+    if constexpr (kEarly && kFlat) {
+      if (sk_s == 1 && KT >= 2 && sbase < total_sched && !(sk_split > 1 && sbase + G > total_sched) && sbase + wg_pos < total_sched &&
+          first_id < p.num_valid && n0 + BN <= p.N && p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0) {
+        int nblock, ncolumn;
+        flat_locate(sbase + wg_pos, nblock, ncolumn);
+        nblock = __builtin_amdgcn_readfirstlane(nblock);
+        ncolumn = __builtin_amdgcn_readfirstlane(ncolumn);
+        if (ncolumn * BN + BN <= p.N) {
+          flat_fetch(nblock, first_id_n, tile_expert_n, row_id_n, a_off_carried);
+          if (first_id_n < p.num_valid) {
+            early = true;
+#pragma unroll
+            for (int t = 0; t < C::kAInstr; ++t) a_off[t] = a_off_carried[t];
+            a_base_n = p.A;
+            b_base_n = p.B + (int64_t)(ncolumn * BN) * p.ldb_b + (int64_t)tile_expert_n * p.b_expert_stride_b;
+          }
+        }
+      }
+    }
     if constexpr (kEarly) {
       int nm0 = 0, nn0 = 0;
       const bool next_whole_round = !arrival && sbase < total_sched && !(sk_split > 1 && sbase + G > total_sched) && sbase + wg_pos < total_sched;
-      if (p.flags == nullptr && p.A_local == nullptr && sk_s == 1 && KT >= 2 && next_whole_round && m0 + BM <= p.M &&
+      if (!kFlat && p.flags == nullptr && p.A_local == nullptr && sk_s == 1 && KT >= 2 && next_whole_round && m0 + BM <= p.M &&
           n0 + BN <= p.N && p.ldc % 8 == 0 && locate(sbase + wg_pos, nm0, nn0) && nm0 + BM <= p.M && nn0 + BN <= p.N) {
         bool c_aligned = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;
         if (p.scatter_bufs != nullptr) c_aligned = (reinterpret_cast<uintptr_t>(p.scatter_bufs[m0 / p.m_per_rank]) & 15) == 0;
@@ -1516,8 +1594,8 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     // per lane for the whole tile (uniform base + constant row step) and no per-store bounds arithmetic. The scales
     // of the whole wave tile are fetched up front, in one round trip.
     bool stored = false;
-    if constexpr (C::kWaves <= 4 && !kGrouped && kFullRows) {
-      if (m0 + BM <= p.M && n0 + BN <= p.N && n_vec_ok) {
+    if constexpr (C::kWaves <= 4 && (!kGrouped || kFlat) && kFullRows) {
+      if (m0 + BM <= p.M && n0 + BN <= p.N && n_vec_ok && (!kFlat || kFlatSkips || first_id < p.num_valid)) {
         stored = true;
         constexpr int kPasses = 32 / kRowsPerPass;
         static_assert(2 * kPasses == kGroups, "one read or store per column group of a row block");
@@ -1563,11 +1641,19 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         arr_issue(kRowBlocks * kPasses);
         __builtin_amdgcn_sched_barrier(0);
         int4v v[kPasses];
+        int dst_id[kFlat ? kPasses : 1];   // kFlat: the row each piece goes to
+        unsigned char* const flat_dst = Cbase + (n0 + wn * C::kWaveN) * 2 + ec * 16;
         auto read_piece = [&](int i, int u) {
+          if constexpr (kFlat) {
+            const int row = 32 * i + u * kRowsPerPass;
+            dst_id[u] = __shfl(row_id[kIdRegs > 1 ? row / 64 : 0], row % 64 + er);
+          }
           v[u] = *(const TDIST_AS3 int4v*)(rbase[u % kReadPhases] + (32 * (blocks_in_turn ? i % 2 : i) + u * kRowsPerPass) * C::kEpiPitch);
         };
         auto store_fast = [&](int i, int u) {
-          TDIST_AS1 int4v* dst = (TDIST_AS1 int4v*)(tile_dst + (int64_t)(32 * i + u * kRowsPerPass) * row_bytes + lane_off);
+          TDIST_AS1 int4v* dst = (TDIST_AS1 int4v*)(kFlat ? flat_dst + (int64_t)dst_id[kFlat ? u : 0] * row_bytes
+                                                          : tile_dst + (int64_t)(32 * i + u * kRowsPerPass) * row_bytes + lane_off);
+          if (kFlatSkips && dst_id[kFlat ? u : 0] < 0) return;
           if (streaming) __builtin_nontemporal_store(v[u], dst);
           else *dst = v[u];
         };
@@ -1670,6 +1756,14 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     // the next tile's prologue overwrites the ring: every wave must be done reading its staging area
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (kEarly) prefetched = early;
+    if constexpr (kEarly && kFlat) {
+      if (early) {
+#pragma unroll
+        for (int q = 0; q < kIdRegs; ++q) row_id[q] = row_id_n[q];
+        first_id = first_id_n;
+        tile_expert = tile_expert_n;
+      }
+    }
   }
   // ---- the last workgroup out advances the workspace's tag base for the next launch --------------------------
   if (p.sk_mode != 0 && threadIdx.x == 0) {
@@ -1979,7 +2073,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   p.chunks_per_rank = 1;
   p.sorted_ids = p.block_expert = p.block_segment = p.post_pad = nullptr;
   p.b_expert_stride_b = 0;
-  p.num_valid = p.topk = p.first_block = p.a_rows = 0;
+  p.num_valid = p.topk = p.first_block = p.a_rows = 0; p.topk_magic = 0;
   p.sk_ctrl = nullptr;
   p.sk_partials = nullptr;
   p.sk_mode = 0;
@@ -2237,6 +2331,7 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   p.b_expert_stride_b = c.expert_stride * esz;
   p.num_valid = c.num_valid;
   p.topk = c.topk;
+  p.topk_magic = (uint32_t)(((1ull << 32) + c.topk - 1) / c.topk);
   p.first_block = c.first_block;
   p.a_rows = c.a_rows;
   p.sk_ctrl = nullptr;
@@ -2272,15 +2367,18 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
     case kElemF16: return launch_gemm_cfg<EH, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who);  \
     default: return launch_gemm_cfg<E8, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who);        \
   }
-  const bool plain = k128 && c.flags == nullptr && c.A_local == nullptr;
+  const bool plain = k128 && c.flags == nullptr && c.A_local == nullptr && (int64_t)c.num_valid * c.topk < (1ll << 32);
   if (plain) {
     // Nothing to wait for: an XCD's workgroups walk a block of tiles of few operand panels (rows + columns of tiles),
     // as in an ungated GEMM, instead of one row block after the other (16 column tiles: 4 x 8 tiles, 12 panels, instead
-    // of 2 x 16, 18 panels). A group that spans experts fetches no more than single rows would.
+    // of 2 x 16, 18 panels: 16384 x 4096 x 1792 over 8 experts 267 -> 260 us). Where an expert has a block or two only, the
+    // blocks of a group share no weights and rows one by one are 1 % ahead. (Groups: what the capacity of the blocks allows
+    // for; every group pads block_size - 1 rows at most.)
     const int per_xcd = di.num_xcds > 0 && cap_wgs % di.num_xcds == 0 ? cap_wgs / di.num_xcds : cap_wgs;
     const int tiles_n = (int)ceil_div(c.N, BN);
     double best = 0;
-    for (int rows = 1; rows <= 8; rows *= 2) {
+    const int64_t groups = ((int64_t)c.num_blocks * c.block_size - c.num_valid) / (c.block_size - 1) + 1;
+    for (int rows = 1; rows <= 8 && (rows == 1 || c.num_valid >= 2 * groups * c.block_size); rows *= 2) {
       const double cols = per_xcd / rows < tiles_n ? per_xcd / rows : tiles_n;
       const double cost = (double)per_xcd / cols * c.block_size + cols * BN;
       if (best == 0 || cost < 0.99 * best) {
