@@ -41,9 +41,9 @@ MEASURED_TRAFFIC_BYTES = {
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
-    "decode.hip": "5f65cc9c7465e64c",
-    "gemm.hip": "5b1de058c7b76344",
-    "moe.hip": "3ab3dfd4ffc67cea",
+    "decode.hip": "66b59d440f8eb3d5",
+    "gemm.hip": "7e89d4f745c84dd9",
+    "moe.hip": "213a47764ff3bfc4",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")

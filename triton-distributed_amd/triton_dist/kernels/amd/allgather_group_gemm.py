@@ -104,8 +104,8 @@ def _row_block(entries, num_experts, n, cus):
     """Rows per block for ``entries`` (token, k) pairs spread over the experts, ``n`` output columns: every expert with rows
     pads half a block on average, and fewer tiles than compute units leave some idle whatever the tile. 256 from 192
     rows per expert on, where the chip is full (2 x 8192 entries over 8 experts, the two products of a 4096 x 1792 layer
-    through their entry points: 223 and 304 us against 251 and 341 with 128; 174 rows by 6 over 64 experts, 4352 x 1024:
-    132 and 205 against 125 and 161)."""
+    through their entry points: 214 and 279 us against 235 and 315 with 128; 2 x 174 rows by 6 over 64 experts, 4352 x 1024:
+    131 and 180 against 124 and 151)."""
     used, cols = min(num_experts, entries), -(-n // 256)
     return min(_BLOCK_COST, key=lambda b: max(1.0, (entries / b + 0.5 * used) * cols / cus) * _BLOCK_COST[b])
 
