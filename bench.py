@@ -43,7 +43,7 @@ MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
     "decode.hip": "66b59d440f8eb3d5",
     "gemm.hip": "7e89d4f745c84dd9",
-    "moe.hip": "213a47764ff3bfc4",
+    "moe.hip": "178cbc1874360811",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")

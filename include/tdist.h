@@ -285,6 +285,12 @@ int tdist_moe_splits_cumsum(const int32_t* ids, int64_t n_ids, int num_experts, 
 int tdist_moe_scatter_index(const int32_t* ids, int64_t n_ids, int topk, int num_experts, int32_t* splits,
                             int32_t* cumsum, int32_t* scatter_idx, int32_t* gather_idx, int32_t* topk_idx,
                             void* workspace, int64_t workspace_bytes, void* stream);
+/* The same from 64-bit ids as torch.topk gives them (their low words count, as after a conversion to 32 bits). Where the one
+ * launch does not apply (more than 65536 ids, not 16-byte aligned, too many experts for its counters, another form asked
+ * for): TDIST_ERR_UNSUPPORTED, nothing launched; convert the ids and call tdist_moe_scatter_index. */
+int tdist_moe_scatter_index64(const int64_t* ids, int64_t n_ids, int topk, int num_experts, int32_t* splits,
+                            int32_t* cumsum, int32_t* scatter_idx, int32_t* gather_idx, int32_t* topk_idx,
+                            void* workspace, int64_t workspace_bytes, void* stream);
 
 /* tdist_moe_scatter_index for callers that cannot allocate (code under HIP graph capture, serving loops, harnesses
  * that forbid hipMalloc). It has no counterpart in the reference. Same arguments and same results, without the

@@ -53,3 +53,30 @@ def test_align_sort_with_more_padding_than_entries(cuda, dtype, R, T, topk, E, B
     assert torch.equal(got[0].cpu(), want[0])   # the whole buffer, padding included
     assert torch.equal(got[1].cpu()[:nb], want[1]) and torch.equal(got[2].cpu()[:nb], want[2])
     assert torch.equal(got[3].cpu(), want[3])
+
+
+# 64-bit ids: both block sizes of the one launch, remainders of a vector of four, ids that are not 16-byte aligned, not
+# contiguous, out of range, and more of them than the one launch takes
+@pytest.mark.parametrize("T,topk,G,how", [(1, 1, 1, ""), (1, 8, 256, ""), (63, 3, 7, ""), (4096, 8, 256, ""), (4097, 8, 64, ""), (8192, 8, 64, ""), (9000, 8, 64, ""),
+                                          (101, 3, 40, "misaligned"), (50, 4, 16, "strided"), (77, 5, 12, "out of range"), (16, 2, 4096, "")])
+def test_index_from_64_bit_ids(cuda, T, topk, G, how):
+    from triton_dist.kernels.amd import create_all_to_all_context, moe_dispatch_preprocess
+    announce("index from 64-bit ids T=%d topk=%d G=%d %s" % (T, topk, G, how))
+    g = torch.Generator().manual_seed(T + G)
+    ids = torch.randint(-1 if how == "out of range" else 0, G + (1 if how == "out of range" else 0), (T, topk), generator=g)
+    if how == "misaligned":
+        dev = torch.empty(T * topk + 1, dtype=torch.int64, device=cuda)[1:].view(T, topk).copy_(ids)
+    elif how == "strided":
+        dev = torch.empty((T, topk + 2), dtype=torch.int64, device=cuda)[:, :topk].copy_(ids)
+    else:
+        dev = ids.to(cuda)
+    ctx = create_all_to_all_context(8, 16, 0, G, 1, G, dtype=torch.float8_e4m3fn)
+    want = [t.clone() for t in moe_dispatch_preprocess(ids.int().to(cuda), G, want_topk_index=True)]
+    got = moe_dispatch_preprocess(dev, G, want_topk_index=True, ctx=ctx)
+    valid = int(want[1][-1])
+    for name, a, b in zip(("splits", "cumsum", "scatter", "gather", "topk"), got, want):
+        n = valid if name in ("gather", "topk") else a.numel()
+        assert torch.equal(a.reshape(-1)[:n], b.reshape(-1)[:n]), name
+    if how != "out of range":
+        for a, b in zip(got, golden.moe_preprocess(ids, G)[:4]):
+            assert torch.equal(a.cpu(), b)

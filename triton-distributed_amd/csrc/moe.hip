@@ -247,7 +247,9 @@ constexpr int kFusedThreads = 512, kFusedPerWave = 256, kFusedItems = kFusedThre
 // The work grows with blocks x ids, so the host takes this form up to kRecountMaxBlocks blocks of 1024 ids only.
 constexpr int kRecountMaxBlocks = 64;
 
-template <int kThreads, int kPerWave, bool kRecount>
+// kWide: 64-bit ids (torch.topk's), of which the low words count: read as they are instead of converted by a launch of their
+// own in front (8000 ids: 3.2 us).
+template <int kThreads, int kPerWave, bool kRecount, bool kWide = false>
 __global__ __launch_bounds__(kThreads) void moe_index_fused_kernel(const int32_t* __restrict__ ids, int64_t n, int topk,
                                                                   int G, int nbits, int32_t* hist, int32_t* ctrl,
                                                                   int32_t* __restrict__ splits,
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void moe_index_fused_kernel(const int32_t
 #pragma unroll
   for (int u = 0; u < kPasses; ++u) {
     const int64_t i = wbase + u * 64 + lane;
-    e_of[u] = i < n ? ids[i] : -1;
+    e_of[u] = i < n ? ids[i << (kWide ? 1 : 0)] : -1;
   }
   // kRecount: the other blocks' ids, four per load, kVecBatch loads in flight (the ranges are multiples of four ids,
   // so a vector lies on one side of this block's range or inside it). The first batch (all of a decode step's ids)
@@ -288,9 +290,16 @@ __global__ __launch_bounds__(kThreads) void moe_index_fused_kernel(const int32_t
       const bool mine = vi * 4 >= own_lo && vi * 4 < own_hi;
       q[u] = int4v{-1, -1, -1, -1};
       if (vi < n_vec && !mine) {
-        if (vi * 4 + 3 < n) q[u] = ((const int4v*)ids)[vi];
-        else
-          for (int j = 0; j < 4; ++j) q[u][j] = vi * 4 + j < n ? ids[vi * 4 + j] : -1;
+        if (vi * 4 + 3 < n) {
+          if constexpr (kWide) {
+            const int4v lo = ((const int4v*)ids)[2 * vi], hi = ((const int4v*)ids)[2 * vi + 1];
+            q[u] = int4v{lo[0], lo[2], hi[0], hi[2]};
+          } else {
+            q[u] = ((const int4v*)ids)[vi];
+          }
+        } else {
+          for (int j = 0; j < 4; ++j) q[u][j] = vi * 4 + j < n ? ids[(vi * 4 + j) << (kWide ? 1 : 0)] : -1;
+        }
       }
     }
   };
@@ -1395,7 +1404,7 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
 
 static int moe_index_common(const int32_t* ids, int64_t n_ids, int topk, int G, int32_t* splits, int32_t* cumsum,
                             int32_t* scatter_idx, int32_t* gather_idx, int32_t* topk_idx, void* workspace,
-                            int64_t workspace_bytes, hipStream_t stream, bool want_index, const char* who) {
+                            int64_t workspace_bytes, hipStream_t stream, bool want_index, const char* who, bool wide = false) {
   if (!ids || !cumsum) return fail(TDIST_ERR_INVALID, "%s: null ids or cumsum", who);
   if (want_index && (!scatter_idx || !gather_idx)) return fail(TDIST_ERR_INVALID, "%s: null index output", who);
   if (n_ids < 0 || G <= 0 || (want_index && topk <= 0)) return fail(TDIST_ERR_INVALID, "%s: bad sizes", who);
@@ -1427,24 +1436,30 @@ static int moe_index_common(const int32_t* ids, int64_t n_ids, int topk, int G, 
   const bool can_recount = form_dbg != 2 && kRowsRecount * G * 4 + 256 <= kLdsLimit && aligned16(ids);
   // 0: blocks of 2048 ids that exchange their histograms; 1 / 2: blocks of 512 / 1024 ids that count everything
   const int form = !can_recount ? 0 : ceil_div(n1, kSmall) <= kRecountMaxBlocks ? 1 : ceil_div(n1, 2 * kSmall) <= kRecountMaxBlocks ? 2 : 0;
+  if (wide && (form == 0 || form_dbg == 2 || form_dbg == 3))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: 64-bit ids are for the one-launch form that counts them all (16-byte aligned, at most "
+                "%d of them, counters that fit the LDS): convert them and call tdist_moe_scatter_index", who, kRecountMaxBlocks * 2 * kSmall);
   if (di.ok == 1 && fused_blocks <= di.num_cus && form_dbg != 3 && (form != 0 || form_dbg == 2)) {
-    auto kern = form == 1 ? moe_index_fused_kernel<kFusedThreads, kSmall / 8, true>
-              : form == 2 ? moe_index_fused_kernel<kFusedThreads, kSmall / 4, true>
+    auto kern = form == 1 ? (wide ? moe_index_fused_kernel<kFusedThreads, kSmall / 8, true, true>
+                                  : moe_index_fused_kernel<kFusedThreads, kSmall / 8, true>)
+              : form == 2 ? (wide ? moe_index_fused_kernel<kFusedThreads, kSmall / 4, true, true>
+                                  : moe_index_fused_kernel<kFusedThreads, kSmall / 4, true>)
                           : moe_index_fused_kernel<kFusedThreads, kFusedPerWave, false>;
     const int64_t blocks = form == 1 ? ceil_div(n1, kSmall) : form == 2 ? ceil_div(n1, 2 * kSmall) : fused_blocks;
     const int rows = form != 0 ? kRowsRecount : kRowsPlain;
-    static bool attr_set[3] = {false, false, false};
-    if (!attr_set[form]) {
+    static bool attr_set[2][3] = {{false, false, false}, {false, false, false}};
+    if (!attr_set[wide][form]) {
       const int most = rows * kMoeMaxExperts * 4 < kLdsLimit ? rows * kMoeMaxExperts * 4 : kLdsLimit;
       if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess)
         return fail(TDIST_ERR_LAUNCH, "%s: cannot reserve LDS for the index kernel", who);
-      attr_set[form] = true;
+      attr_set[wide][form] = true;
     }
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kFusedThreads), (size_t)rows * G * 4 + (form != 0 ? 256 : 0), stream,
                        ids, n_ids, want_index ? topk : 1, G, id_bits(G), hist, scan_counter, splits, cumsum,
                        want_index ? scatter_idx : nullptr, gather_idx, topk_idx);
     return launch_status(who);
   }
+  if (wide) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
   hipLaunchKernelGGL(moe_hist_kernel, dim3(num_blocks), dim3(kMoeThreads), (size_t)G * 4, stream, ids, n_ids, G, hist,
                      scan_counter);
   hipLaunchKernelGGL(moe_scan_kernel, dim3((G + kScanCols - 1) / kScanCols), dim3(kScanThreads), 0, stream, hist, num_blocks,
@@ -1531,6 +1546,13 @@ int tdist_moe_scatter_index(const int32_t* ids, int64_t n_ids, int topk, int num
                             void* workspace, int64_t workspace_bytes, void* stream) {
   return moe_index_common(ids, n_ids, topk, num_experts, splits, cumsum, scatter_idx, gather_idx, topk_idx, workspace,
                           workspace_bytes, (hipStream_t)stream, true, "tdist_moe_scatter_index");
+}
+
+int tdist_moe_scatter_index64(const int64_t* ids, int64_t n_ids, int topk, int num_experts, int32_t* splits,
+                            int32_t* cumsum, int32_t* scatter_idx, int32_t* gather_idx, int32_t* topk_idx,
+                            void* workspace, int64_t workspace_bytes, void* stream) {
+  return moe_index_common((const int32_t*)ids, n_ids, topk, num_experts, splits, cumsum, scatter_idx, gather_idx, topk_idx, workspace,
+                          workspace_bytes, (hipStream_t)stream, true, "tdist_moe_scatter_index64", true);
 }
 
 int tdist_moe_dispatch(const void* rows, int64_t row_bytes, const float* scales, const int32_t* gather_idx,

@@ -183,16 +183,21 @@ def moe_dispatch_preprocess(exp_indices: torch.Tensor, num_experts: int, want_to
     if ctx is not None:
         _ensure_index_sets(ctx, T, topk, num_experts, dev)
         # the context has seen this shape: its tensors' addresses are at hand and the host does next to nothing (the
-        # index kernel takes ~9 us on the device; a general path costs more than that on the host). Ids that are not
-        # contiguous int32 (torch.topk gives int64) are converted into the context's staging tensor: one copy kernel,
-        # no allocation.
-        exp_indices = _staged_ids(ctx, exp_indices)
+        # index kernel takes ~9 us on the device; a general path costs more than that on the host). Contiguous int64 ids
+        # (torch.topk's) are read as they are where the one-launch form takes them; others that are not contiguous
+        # int32 are converted into the context's staging tensor: one copy kernel, no allocation.
         which = ctx.index_calls % 2
         ctx.index_calls += 1
         out = ctx.index_sets[which]
         head, tail = ctx.index_args[which]
-        _lib.call("tdist_moe_scatter_index", exp_indices.data_ptr(), *head, _lib.ptr(out[4] if want_topk_index else None),
-                  *tail, _lib.stream_ptr())
+        args = (*head, _lib.ptr(out[4] if want_topk_index else None), *tail, _lib.stream_ptr())
+        rc = _lib.TDIST_ERR_UNSUPPORTED
+        if exp_indices.dtype == torch.int64 and exp_indices.is_contiguous():
+            rc = _lib.load().tdist_moe_scatter_index64(exp_indices.data_ptr(), *args)
+        if rc == _lib.TDIST_ERR_UNSUPPORTED:
+            exp_indices = _staged_ids(ctx, exp_indices)
+            rc = _lib.load().tdist_moe_scatter_index(exp_indices.data_ptr(), *args)
+        _lib.check(rc)
         return out if want_topk_index else out[:4]
     if exp_indices.dtype != torch.int32:
         exp_indices = exp_indices.to(torch.int32)
