@@ -214,18 +214,30 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 
   // ---- epilogue: lane holds columns 4g .. 4g+3 of row x of each block; staged through the LDS so that stores are whole
   // 16-byte pieces of a row
+  // (the scales in one round trip, in front of the packing: a load per element and row block in between took longer than a
+  // short K's products: 2048 x 1024 x 3328 e4m3 37 -> 26 us per call)
+  float4v cs[kScales ? C::kTN : 1];
+  float rs[kScales ? C::kTM : 1];
+  if constexpr (kScales) {
+#pragma unroll
+    for (int j = 0; j < C::kTN; ++j) {
+      const int col = n0 + wn * (BN / 2) + j * 16 + 4 * g;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) cs[j][e] = p.col_scale ? p.col_scale[min(col + e, p.N - 1)] : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < C::kTM; ++i) rs[i] = p.row_scale ? p.row_scale[min(m0 + wm * (BM / 2) + i * 16 + x, p.M - 1)] : 1.f;
+  }
 #pragma unroll
   for (int i = 0; i < C::kTM; ++i) {
     const int row = wm * (BM / 2) + i * 16 + x;
-    float rs = 1.f;
-    if (kScales && p.row_scale) rs = p.row_scale[min(m0 + row, p.M - 1)];
 #pragma unroll
     for (int j = 0; j < C::kTN; ++j) {
       const int col = wn * (BN / 2) + j * 16 + 4 * g;
       float4v v = acc[j][i];
       if constexpr (kScales) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= rs * (p.col_scale ? p.col_scale[min(n0 + col + e, p.N - 1)] : 1.f);
+        for (int e = 0; e < 4; ++e) v[e] *= rs[i] * cs[j][e];
       }
       *(TDIST_AS3 int2v*)(ring + row * C::kEpiPitch + col * 2) = int2v{(int)E::pack(v[0], v[1]), (int)E::pack(v[2], v[3])};
     }
