@@ -82,3 +82,29 @@ def test_workspace_and_head_dimensions_are_checked(cuda):
                                        1024, p, nbytes, p, _lib.TDIST_BF16, 0, 0, None, None)
     assert call(128, 128, p, need - 1) == _lib.TDIST_ERR_WORKSPACE
     assert call(576, 512, p + 16, 1 << 40) == _lib.TDIST_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,lens,dtype", [(1, 64, 8, 128, [6016], torch.bfloat16), (5, 32, 8, 96, [6001, 17, 300, 0, 2048], torch.float16),
+                                                   (12, 6, 1, 128, [6100] + [33] * 11, torch.bfloat16), (8, 6, 1, 72, [1] * 8, torch.float16)])
+def test_few_long_sequences_take_either_form_with_one_result(cuda, B, Hq, Hkv, D, lens, dtype):
+    """A page table with room for more than 6000 keys sends few sequences to the split form; the lengths are the same behind
+    a narrow table, which the streaming form takes. Both hold fp32 partial results: they differ by one rounding of the output."""
+    from triton_dist.kernels.amd import flash_decode as fd
+    announce("few long sequences B=%d heads %d/%d D=%d" % (B, Hq, Hkv, D))
+    g = torch.Generator().manual_seed(B + D)
+    page, pages = 16, 400
+    k = torch.randn((pages, page, Hkv, D), generator=g).to(dtype).to(cuda)
+    v = torch.randn((pages, page, Hkv, D), generator=g).to(dtype).to(cuda)
+    q = torch.randn((B, Hq, D), generator=g).to(dtype).to(cuda)
+    need = max(1, -(-max(lens) // page))
+    table = torch.randint(0, pages, (B, max(need, 376)), generator=g, dtype=torch.int32).to(cuda)
+    kv_lens = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    assert fd._few_long_sequences(B, Hq, Hkv, D, table.shape[1] * page)
+    got = fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, table, D ** -0.5)
+    rule, fd._few_long_sequences = fd._few_long_sequences, lambda *a: False
+    try:
+        want = fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, table, D ** -0.5)
+    finally:
+        fd._few_long_sequences = rule
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert ((got.float() - want.float()).abs() <= 2 * eps * want.float().abs() + 1e-5).all()
