@@ -99,6 +99,25 @@ def test_null_pointers_are_rejected_without_touching_the_gpu():
     assert lib.tdist_moe_workspace_bytes(32768, 256) == (128 + 1) * 256 * 4 + 256
 
 
+@pytest.mark.parametrize("entry,scales", [("tdist_gemm_rs_scatter_bf16", []), ("tdist_gemm_rs_scatter_f16", []),
+                                          ("tdist_gemm_rs_scatter_fp8e4m3", [None, None])])
+@pytest.mark.parametrize("rows_per_rank", [128, 64, 192, 320, 2048])
+def test_scatter_checks_rank_and_rows_whatever_tile_would_be_taken(entry, scales, rows_per_rank):
+    """A rank outside the world would scatter in front of or behind the owners' buffers, and a slice must be a multiple of
+    128 rows: both are refused before the device is looked at, for sizes of the small tiles and of the large ones alike."""
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(4096 + 256)
+    p = (ctypes.addressof(buf) + 255) & ~255
+
+    def call(rank, world):
+        return getattr(lib, entry)(p, 512, p, 512, p, 512, 4 * rows_per_rank, 512, 512, *scales, rank, world, None, 0, None)
+    for rank, world in ((-1, 4), (4, 4), (7, 4), (0, 0), (0, -4)):
+        assert call(rank, world) == _lib.TDIST_ERR_INVALID and "rank" in _lib.last_error(), (rank, world)
+    if rows_per_rank % 128 != 0:
+        assert call(0, 4) == _lib.TDIST_ERR_UNSUPPORTED and "128" in _lib.last_error()
+    assert call(0, 7) == _lib.TDIST_ERR_UNSUPPORTED   # (rows that are no multiple of the ranks)
+
+
 def test_debug_switches_default_to_automatic_and_ignore_the_environment(monkeypatch):
     """The library's test and measurement switches: -1 (the library decides) until tdist_debug_set says otherwise,
     a negative value puts a key back, unknown keys are rejected, and nothing is read from the environment."""

@@ -1868,6 +1868,9 @@ static double sk_handover_k_tiles(int bm, int bn) { return 2.0 + 6.0 * bm * bn /
 // (Pieces of at least kSmallMinPiece K tiles: shorter ones cost more than they save, and a short K's sums then run in the
 // order of the large tiles', bit for bit.)
 constexpr int kSmallMinPiece = 8;
+// Rows of a rank's slice in a scatter call come in whole multiples of this: every tile but the 256-row ones (which are
+// taken for multiples of their own only) then lies inside one slice.
+constexpr int kScatterRows = 128;
 struct SmallPlan {
   int tile, splits, tiles_per_split;
   bool deep;
@@ -1883,7 +1886,6 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
   for (int t = 0; t < kNumSmallTiles; ++t) {
     if (forced_tile >= 0 && forced_tile != t) continue;
     const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn;
-    if (c.scatter_bufs && (c.world_size <= 0 || c.M % c.world_size != 0 || (c.M / c.world_size) % bm != 0)) continue;
     const int64_t tiles = ceil_div(c.M, bm) * ceil_div(c.N, bn);
     for (int s = 1; s <= kSmallMaxSplits; s *= 2) {
       if (s > 1 && (sk == 0 || tiles > kSkSmallTiles || k_tiles / s < (sk > 1 ? 2 : kSmallMinPiece) || c.sk_workspace == nullptr ||
@@ -1940,6 +1942,14 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   const int esz = elem == kElemFP8 ? 1 : 2;
   if (!c.A || !c.B || (!c.C && !c.scatter_bufs)) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
   if (c.M <= 0 || c.N <= 0 || c.K <= 0) return fail(TDIST_ERR_INVALID, "%s: M, N, K must be positive", who);
+  if (c.scatter_bufs) {
+    // (in front of any choice of tiles: every kernel takes the owner and its row from these)
+    if (c.world_size <= 0 || c.rank < 0 || c.rank >= c.world_size)
+      return fail(TDIST_ERR_INVALID, "%s: rank %d / world_size %d", who, c.rank, c.world_size);
+    if (c.M % c.world_size != 0 || (c.M / c.world_size) % kScatterRows != 0)
+      return fail(TDIST_ERR_UNSUPPORTED, "%s: M = %d must be world_size = %d times a multiple of %d rows", who, c.M, c.world_size,
+                  kScatterRows);
+  }
   if (((int64_t)c.K * esz) % 16 != 0)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: K*elem_size = %lld must be a multiple of 16 bytes", who, (long long)c.K * esz);
   if (!aligned16(c.A) || !aligned16(c.B) || (c.A_local && !aligned16(c.A_local)) || (c.lda * esz) % 16 ||
@@ -1965,7 +1975,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // one) need more than 128 bytes of K; the 128x128 tile takes everything else. Among the admissible ones the cheapest estimate wins: rounds of the grid times the tile's work
   // over its measured relative efficiency.
   bool rows256 = true;
-  if (c.scatter_bufs && c.world_size > 0 && (c.M % c.world_size != 0 || (c.M / c.world_size) % 256 != 0)) rows256 = false;
+  if (c.scatter_bufs && (c.M / c.world_size) % 256 != 0) rows256 = false;
   if (!c.scatter_bufs && c.flags && c.m_per_chunk % 256 != 0) rows256 = false;
   if (c.A_local && (c.local_row_begin % 256 != 0 || c.local_rows % 256 != 0)) rows256 = false;
   // the split ring steps through K 128 bytes at a time; a ragged K (see k_head_bytes) takes at least two K tiles
@@ -2084,11 +2094,6 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   set_k_head(p, pick != 2, (int64_t)c.K * esz);
 
   if (c.scatter_bufs) {
-    if (c.world_size <= 0 || c.rank < 0 || c.rank >= c.world_size)
-      return fail(TDIST_ERR_INVALID, "%s: rank %d / world_size %d", who, c.rank, c.world_size);
-    if (c.M % c.world_size != 0 || (c.M / c.world_size) % BM != 0)
-      return fail(TDIST_ERR_UNSUPPORTED, "%s: M/world_size = %d must be a multiple of the %d-row tile", who,
-                  c.M / c.world_size, BM);
     p.m_per_rank = c.M / c.world_size;
     p.m_per_chunk = p.m_per_rank;
     p.n_chunks = c.world_size;
