@@ -173,14 +173,15 @@ GATHER_MAX_RANKS = 64
 
 
 def shard_table(own, peer_shards, rank, num_ranks):
-    """The host table of every rank's shard for tdist_gather_shards, or None where a shard is missing or does not lie on 16
-    bytes (the copies of the flag-gated path take any address)."""
+    """The host table of every rank's shard for tdist_gather_shards, or None where a shard is missing, lies on another device
+    (a kernel reads it: nothing says that peer access is enabled) or not on 16 bytes. The copies of the flag-gated path
+    take any device and any address."""
     if num_ranks > GATHER_MAX_RANKS or own.data_ptr() % 16 != 0:
         return None
     table = (ctypes.c_void_p * num_ranks)()
     for r in range(num_ranks):
         t = own if r == rank else peer_shards.get(r)
-        if t is None or t.data_ptr() % 16 != 0:
+        if t is None or t.device != own.device or t.data_ptr() % 16 != 0:
             return None
         table[r] = t.data_ptr()
     return table
