@@ -41,7 +41,7 @@ MEASURED_TRAFFIC_BYTES = {
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
-    "decode.hip": "66b59d440f8eb3d5",
+    "decode.hip": "b4ea45912b78b068",
     "gemm.hip": "f5e3c8dbadd4a963",
     "moe.hip": "178cbc1874360811",
     "reduce.hip": "469689d34df1b205",

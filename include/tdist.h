@@ -529,16 +529,18 @@ int tdist_decode_fused(const void* q, const void* k_cache, const void* v_cache, 
                        int64_t table_stride, int dtype, int32_t* counters, int64_t n_counters, void* out,
                        int out_dtype, int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream);
 
-/* Decode of a whole batch in ONE launch that divides the keys itself: the result of tdist_decode_split_kv followed by
+/* Decode of a whole batch that divides the keys itself: the result of tdist_decode_split_kv followed by
  * tdist_decode_combine(mode 1), without partial results for the caller to hold.
  *   replaces gqa_fwd_batch_decode                   kernels/nvidia/flash_decode.py:763-844 (split-KV + combine launches,
  *   a fixed number of splits for every sequence)
  * All sequences' blocks of keys are laid end to end and cut into equal ranges, one per wave and kv head, so the time
- * goes with the sum of the lengths, not with the longest, and a short sequence is not cut at all. out [B,Hq,Dv] of
+ * goes with the sum of the lengths, not with the longest, and a short sequence is not cut at all; a second launch merges
+ * the sequences that are spread over several ranges. out [B,Hq,Dv] of
  * out_dtype (strides out_stride_b, out_stride_h); lse_out fp32 [B,Hq] or NULL; a sequence of length 0 gets out = 0,
- * lse = -inf. counters as for tdist_decode_fused (all zero on entry, left zero). workspace: plain device memory,
+ * lse = -inf. counters, n_counters: not used (NULL, 0). workspace: plain device memory,
  * 16-byte aligned, of at least tdist_decode_stream_workspace_bytes() bytes (-1: bad sizes); its contents do not matter
- * before or after the call. Calls that share counters or workspace must not overlap. Head dimensions as
+ * before or after the call: nothing is kept between calls, which may be captured and replayed in any order. Calls that
+ * share a workspace must not overlap. Head dimensions as
  * for tdist_decode_split_kv, except that (576,512) is taken only where the value is the first 512 columns of the key (the
  * same pointer and strides: latent attention, which then reads every row once); TDIST_ERR_UNSUPPORTED otherwise: use the
  * two calls. */

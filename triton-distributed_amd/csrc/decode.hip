@@ -71,8 +71,9 @@ struct DecodeParams {
   int64_t fo_sb, fo_sh;      // element strides of final_out
   int fo_vec;                // its rows take 8-byte (16-bit types) / 16-byte (fp32) stores
   int part_vec;              // the partial results take 16-byte stores
-  // streaming form: ranges the batch's blocks are cut into at most, and the fewest blocks of a range
-  int ranges, min_blocks;
+  // streaming form: ranges the batch's blocks are cut into at most, the fewest blocks of a range, and (for the merge) the
+  // width of a result's row
+  int ranges, min_blocks, dv;
 };
 
 struct MmaBF16 {
@@ -230,7 +231,7 @@ __device__ __forceinline__ int xcd_major(int i, int n) {
 }
 
 // ---- streaming form: which blocks a range holds -----------------------------------------------------------
-constexpr int kStreamMaxParts = 64;   // ranges one sequence may be spread over (a merge weighs them one per lane)
+constexpr int kStreamMaxParts = 64;   // ranges one sequence may be spread over
 
 struct StreamRange {
   int n;            // blocks in the range (0: the batch has fewer ranges)
@@ -238,6 +239,12 @@ struct StreamRange {
   int first_block;  // that sequence's first block, numbered over the whole batch
   int per;          // blocks per range
 };
+
+// Blocks per range, from the batch's blocks and its longest sequence's: even shares, but no shorter than min_blocks and no
+// more than kStreamMaxParts ranges to a sequence (a sequence of n blocks touches at most ceil(n / per) + 1 ranges).
+__device__ __forceinline__ int stream_blocks_per_range(const DecodeParams& prm, int total, int longest) {
+  return max(max((total + prm.ranges - 1) / prm.ranges, prm.min_blocks), (longest + kStreamMaxParts - 2) / (kStreamMaxParts - 1));
+}
 
 // All sequences' blocks laid end to end and cut into ranges of `per` blocks: the same answer in every wave, from one
 // load per 64 sequences and a scan over the lanes.
@@ -264,9 +271,7 @@ __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int
   for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
   mx = __builtin_amdgcn_readfirstlane(mx);
   StreamRange r;
-  // even shares, but no shorter than min_blocks and no more than kStreamMaxParts ranges to a sequence (a sequence of
-  // n blocks touches at most ceil(n / per) + 1 ranges)
-  r.per = max(max((total + prm.ranges - 1) / prm.ranges, prm.min_blocks), (mx + kStreamMaxParts - 2) / (kStreamMaxParts - 1));
+  r.per = stream_blocks_per_range(prm, total, mx);
   const long long g0 = (long long)range * r.per;
   r.seq = r.block = r.first_block = 0;
   if (g0 >= total) {
@@ -289,83 +294,26 @@ __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int
   }
 }
 
-// The merge of one sequence's partial results for one block of up to 16 heads, by NW waves (all of their workgroup, or a
-// wave alone): partial j is that of range first + j (the second slot of the range in which the sequence begins, the first
-// slot of the others). A lane weighs head lane & 15 of every fourth partial; every wave works out all weights for itself
-// (the same values to the same places of the LDS, `s`: 16 x kStreamMaxParts floats), so none waits. Then kB partials' rows
-// and kV 16-byte pieces per lane are in flight together. The sums run over the partials in order.
-template <int NW>
-__device__ __forceinline__ void stream_merge(const DecodeParams& prm, int seq, int first, int parts, int h0, int nvalid,
-                                             int Dout, TDIST_AS3 float* s) {
+// One sequence: its first block, numbered over the whole batch, and the blocks per range. The loads of all lengths are
+// independent of each other.
+template <int KEYS>
+__device__ __forceinline__ void stream_sequence(const DecodeParams& prm, int seq, int& first_block, int& per) {
   const int lane = threadIdx.x & 63;
-  const int tid = NW == 1 ? lane : (int)threadIdx.x;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  auto row = [&](int j) { return ((int64_t)(first + j) * 2 + (j == 0 ? 1 : 0)) * prm.Hq + h0; };
-  {
-    constexpr int kPer = kStreamMaxParts / 4;
-    const int h = lane & 15, j0 = lane >> 4;
-    float l[kPer];
-    float M = -INFINITY, L = 0.f;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int j = j0 + 4 * i;
-      l[i] = j < parts && h < nvalid ? prm.lse[row(j) + h] : -INFINITY;
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) M = fmaxf(M, l[i]);
-    M = fmaxf(M, __shfl_xor(M, 16));
-    M = fmaxf(M, __shfl_xor(M, 32));
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      l[i] = l[i] == -INFINITY ? 0.f : __expf(l[i] - M);
-      L += l[i];
-    }
-    L += __shfl_xor(L, 16);
-    L += __shfl_xor(L, 32);
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) s[h * kStreamMaxParts + j0 + 4 * i] = l[i] * inv;
-    if (prm.final_lse && tid < nvalid) prm.final_lse[(int64_t)seq * prm.Hq + h0 + h] = L > 0.f ? M + logf(L) : -INFINITY;
+  int total = 0, before = 0, mx = 0;
+  for (int i = lane; i < prm.B; i += 64) {
+    const int nb = (max(prm.lens[i], 0) + KEYS - 1) / KEYS;
+    total += nb;
+    before += i < seq ? nb : 0;
+    mx = max(mx, nb);
   }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  const int vecs = nvalid * Dout / 4, per_head = Dout / 4;
-  auto sum_rows = [&](auto kv, auto kb) {
-    constexpr int kV = decltype(kv)::value, kB = decltype(kb)::value;
-    for (int v0 = 0; v0 < vecs; v0 += 64 * NW * kV) {
-      float4v acc[kV];
-      int at[kV], h[kV];
 #pragma unroll
-      for (int v = 0; v < kV; ++v) {
-        acc[v] = float4v{0.f, 0.f, 0.f, 0.f};
-        at[v] = min(v0 + v * 64 * NW + tid, vecs - 1);
-        h[v] = at[v] / per_head;
-      }
-      for (int j0 = 0; j0 < parts; j0 += kB) {
-        float4v r[kB][kV];
-#pragma unroll
-        for (int u = 0; u < kB; ++u) {
-          const float4v* src = (const float4v*)(prm.out + row(min(j0 + u, parts - 1)) * Dout);
-#pragma unroll
-          for (int v = 0; v < kV; ++v) r[u][v] = src[at[v]];
-        }
-#pragma unroll
-        for (int u = 0; u < kB; ++u)
-#pragma unroll
-          for (int v = 0; v < kV; ++v) {
-            const float w = j0 + u < parts ? s[h[v] * kStreamMaxParts + j0 + u] : 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[v][e] += w * r[u][v][e];
-          }
-      }
-#pragma unroll
-      for (int v = 0; v < kV; ++v)
-        if (v0 + v * 64 * NW + tid < vecs)
-          store_elem4(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)(h0 + h[v]) * prm.fo_sh + (at[v] - h[v] * per_head) * 4,
-                      prm.final_dtype, prm.fo_vec, acc[v]);
-    }
-  };
-  if (vecs <= 64 * NW * 2) sum_rows(std::integral_constant<int, 2>{}, std::integral_constant<int, 16>{});
-  else sum_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{});
+  for (int o = 32; o > 0; o >>= 1) {
+    total += __shfl_xor(total, o);
+    before += __shfl_xor(before, o);
+    mx = max(mx, __shfl_xor(mx, o));
+  }
+  first_block = __builtin_amdgcn_readfirstlane(before);
+  per = stream_blocks_per_range(prm, __builtin_amdgcn_readfirstlane(total), __builtin_amdgcn_readfirstlane(mx));
 }
 
 // Are the B sequence lengths even enough for the form that hands a workgroup 8 kv heads of one (sequence, split)?
@@ -838,20 +786,19 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     // The range's first sequence may have begun in an earlier range (its partial result waits in registers for the
     // end of the stream) and its last may go on in the next one; all between are whole and stored when they end.
     bool begun_here = sr.block == 0;
-    int seq_first = sr.first_block;   // global number of the current sequence's first block
     float4v held[DT];
     float held_lse = 0.f;
 #pragma unroll
     for (int d = 0; d < DT; ++d) held[d] = float4v{0.f, 0.f, 0.f, 0.f};
-    int part_seq[2] = {-1, -1}, part_first[2] = {0, 0};
+    bool any_held = false;
     auto part_row = [&](int rg, int slot) { return ((int64_t)rg * 2 + slot) * prm.Hq + h0; };
     auto store_part = [&](int slot, const float4v(&val)[DT], float val_lse) {
       if (x < nvalid) {
         float* o = prm.out + (part_row(range, slot) + x) * Dout + 4 * g;
 #pragma unroll
         for (int d = 0; d < DT; ++d)
-          if (!kPadded || 16 * d + 4 * g < Dout) store_partial4<true>(o + 16 * d, val[d]);
-        if (g == 0) store_partial<true>(prm.lse + part_row(range, slot) + x, val_lse);
+          if (!kPadded || 16 * d + 4 * g < Dout) store_partial4<false>(o + 16 * d, val[d]);
+        if (g == 0) prm.lse[part_row(range, slot) + x] = val_lse;
       }
     };
     for (int i = 0; i < sr.n; ++i) {
@@ -879,20 +826,15 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
               if (!kPadded || 16 * d + 4 * g < Dout) store_elem4(prm.final_out, o + 16 * d, prm.final_dtype, prm.fo_vec, acc[d]);
             if (prm.final_lse && g == 0) prm.final_lse[(int64_t)w_cmp.blk.seq * prm.Hq + h0 + x] = r_lse;
           }
-        } else {
-          const int slot = begun_here ? 1 : 0;
-          part_seq[slot] = w_cmp.blk.seq;
-          part_first[slot] = seq_first;
-          if (i == sr.n - 1) {
-            store_part(slot, acc, r_lse);
-          } else {
-            held_lse = r_lse;
+        } else if (i == sr.n - 1) {
+          store_part(begun_here ? 1 : 0, acc, r_lse);
+        } else {   // (it began in an earlier range and ends here)
+          any_held = true;
+          held_lse = r_lse;
 #pragma unroll
-            for (int d = 0; d < DT; ++d) held[d] = acc[d];
-          }
+          for (int d = 0; d < DT; ++d) held[d] = acc[d];
         }
         if (i < sr.n - 1) {
-          seq_first += (w_cmp.blk.hi + KEYS - 1) / KEYS;
           begun_here = true;
           m_run = -INFINITY;
           l_run = 0.f;
@@ -905,22 +847,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       }
       walk_next(w_cmp);
     }
-    if (part_seq[0] >= 0 && w_cmp.blk.seq != part_seq[0]) store_part(0, held, held_lse);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the partial results are where every XCD sees them
-#pragma unroll
-    for (int slot = 0; slot < 2; ++slot) {
-      if (part_seq[slot] < 0) continue;
-      const int seq = part_seq[slot];
-      const int nb = (lens[seq] + KEYS - 1) / KEYS;
-      const int first = part_first[slot] / sr.per, parts = (part_first[slot] + nb - 1) / sr.per - first + 1;
-      int32_t* const ctr = prm.counters + ((int64_t)seq * prm.Hkv + kvh) * head_blocks + hb;
-      int last = 0;
-      if (lane == 0) {
-        last = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (__builtin_amdgcn_readfirstlane(last)) stream_merge<1>(prm, seq, first, parts, h0, nvalid, Dout, (TDIST_AS3 float*)wbase);
-    }
+    if (any_held) store_part(0, held, held_lse);
     return;
   }
   if constexpr (kWaveHeads) {
@@ -1012,8 +939,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   }
 
   // kStreamGroup: the range's segments (a sequence's part in it), one after the other; else the one split
-  int seg_left = sr.n, seg_block = sr.block, seg_first = sr.first_block;
-  int part_seq[2] = {-1, -1}, part_first[2] = {0, 0};
+  int seg_left = sr.n, seg_block = sr.block;
   b = kStreamGroup ? sr.seq : b;
   for (;;) {
     float* seg_out = out_base;   // rows of the 16 heads, seg_row floats apart; LSEs seg_lse_row apart
@@ -1032,7 +958,6 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       seg_lse = prm.lse + ((int64_t)range * 2 + slot) * prm.Hq + h0;
       seg_row = Dout;
       seg_lse_row = 1;
-      if (!whole) part_seq[slot] = b, part_first[slot] = seg_first;
       n_w = seg_n > kwave ? (seg_n - kwave + NK - 1) / NK : 0;
       m_run = -INFINITY;
       l_run = 0.f;
@@ -1132,33 +1057,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     if constexpr (!kStreamGroup) break;
     seg_left -= seg_n;
     if (seg_left == 0) break;
-    seg_first += (lens[b] + KEYS - 1) / KEYS;
     do ++b;
     while (lens[b] <= 0);
     seg_block = 0;
     __syncthreads();   // the merge has read its rings
-  }
-  if constexpr (kStreamGroup) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's partial results are where every XCD sees them
-    __syncthreads();
-    TDIST_AS3 int* const s_last = (TDIST_AS3 int*)smem3;
-#pragma unroll
-    for (int slot = 0; slot < 2; ++slot) {
-      if (part_seq[slot] < 0) continue;
-      const int seq = part_seq[slot];
-      const int nb = (lens[seq] + KEYS - 1) / KEYS;
-      const int first = part_first[slot] / sr.per, parts = (part_first[slot] + nb - 1) / sr.per - first + 1;
-      if (threadIdx.x == 0) {
-        int32_t* const ctr = prm.counters + ((int64_t)seq * prm.Hkv + kvh) * head_blocks + hb;
-        const int last = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *s_last = last;
-      }
-      __syncthreads();
-      const int last = __builtin_amdgcn_readfirstlane(*s_last);
-      if (last) stream_merge<NW>(prm, seq, first, parts, h0, nvalid, Dout, (TDIST_AS3 float*)(smem3 + 64));
-      __syncthreads();
-    }
   }
 }
 
@@ -1378,10 +1280,107 @@ static int launch_decode_cfg(const DecodeParams& prm, int head_blocks, hipStream
   return launch_status(kFuse ? "tdist_decode_fused" : "tdist_decode_split_kv");
 }
 
+// The second launch of the streaming form: the partial results of every sequence that is spread over several ranges into its
+// result. A workgroup takes 64 16-byte pieces of one sequence's [Hq, Dv] plane; partial j of the sequence lies in the second
+// slot of the range in which it begins (j = 0) and in the first slot of the others; a wave takes a run of them, kBatch rows and
+// LSEs in flight per lane, and the LDS brings the waves' sums together in order: the result repeats bit for bit.
+// Where the batch has fewer sequences than ranges a workgroup asks for its sequence, else for the one that crosses the boundary
+// behind range `at` and begins in it (nothing to do at the other boundaries).
+// A launch of its own, not the work of the last range to arrive: nobody counts arrivals, so the call holds no state that outlives
+// it, and the partials of a long sequence are read by as many waves as its result has pieces.
+// What bounds it: the launch and two trips to memory (lengths; rows and LSEs). Against the merge by the last wave to arrive, whole
+// calls: 1 x 1320 keys, 32 / 8 heads 16.8 -> 16.0 us; latent heads, 16 up to 4096 keys 60.4 -> 57.7; 48 up to 8192 74.9 -> 75.7;
+// 32 x 32768 660 -> 664.
+template <int KEYS, int NW>
+__global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm) {
+  constexpr int kBatch = 16;
+  __shared__ float4v s_acc[NW][64];
+  __shared__ float s_max[NW][64], s_sum[NW][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row_vecs = prm.dv / 4, vecs = prm.Hq * row_vecs, pieces = (vecs + 63) / 64;
+  const int at = blockIdx.x / pieces, piece = blockIdx.x - at * pieces;
+  int seq = at, first_block, per;
+  if (prm.B < prm.ranges) {
+    stream_sequence<KEYS>(prm, seq, first_block, per);
+  } else {
+    const StreamRange r = stream_range<KEYS>(prm, at + 1);
+    if (r.n == 0 || r.block == 0 || r.first_block / r.per != at) return;
+    seq = r.seq;
+    first_block = r.first_block;
+    per = r.per;
+  }
+  const int nb = (max(prm.lens[seq], 0) + KEYS - 1) / KEYS;
+  if (nb == 0) return;   // (zeros, stored by the first launch)
+  const int first = first_block / per, parts = (first_block + nb - 1) / per - first + 1;
+  if (parts == 1) return;
+
+  const int at_vec = min(piece * 64 + lane, vecs - 1), h = at_vec / row_vecs;
+  const int64_t plane = (int64_t)prm.Hq * prm.dv;
+  auto slot_of = [&](int j) { return ((int64_t)first + j) * 2 + (j == 0 ? 1 : 0); };
+  const int share = (parts + NW - 1) / NW, j_end = min(parts, (wave + 1) * share);
+  float m = -INFINITY, l = 0.f;
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+  for (int j0 = wave * share; j0 < j_end; j0 += kBatch) {
+    float4v r[kBatch];
+    float w[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int64_t slot = slot_of(min(j0 + u, j_end - 1));
+      r[u] = *((const float4v*)(prm.out + slot * plane) + at_vec);
+      w[u] = prm.lse[slot * prm.Hq + h];
+    }
+    float m_new = m;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) m_new = fmaxf(m_new, w[u]);
+    const float scale = m == -INFINITY ? 0.f : __expf(m - m_new);
+    m = m_new;
+    l *= scale;
+    acc *= scale;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float p = j0 + u < j_end && w[u] != -INFINITY ? __expf(w[u] - m) : 0.f;
+      l += p;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += p * r[u][e];
+    }
+  }
+  s_acc[wave][lane] = acc;
+  s_max[wave][lane] = m;
+  s_sum[wave][lane] = l;
+  __syncthreads();
+  if (wave != 0 || piece * 64 + lane >= vecs) return;
+  float M = s_max[0][lane];
+#pragma unroll
+  for (int v = 1; v < NW; ++v) M = fmaxf(M, s_max[v][lane]);
+  float L = 0.f;
+  acc = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < NW; ++v) {
+    const float p = s_max[v][lane] == -INFINITY ? 0.f : __expf(s_max[v][lane] - M);
+    L += p * s_sum[v][lane];
+    const float4v a = s_acc[v][lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += p * a[e];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = L > 0.f ? acc[e] / L : 0.f;
+  const int d = (at_vec - h * row_vecs) * 4;
+  store_elem4(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)h * prm.fo_sh + d, prm.final_dtype, prm.fo_vec, acc);
+  if (prm.final_lse && d == 0) prm.final_lse[(int64_t)seq * prm.Hq + h] = L > 0.f ? M + logf(L) : -INFINITY;
+}
+
+template <int KEYS>
+static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
+  if (prm.ranges == 1) return TDIST_OK;   // every sequence lies in the one range
+  const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
+  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 4>), dim3((unsigned)(places * pieces)), dim3(256), 0, stream, prm);
+  return launch_status("tdist_decode_stream");
+}
+
 // Streaming form: the whole batch in one launch that fills the chip once. All sequences' blocks of KEYS keys are laid
 // end to end and cut into equal ranges; a wave takes one kv head (and up to 16 of its query heads) over one range,
 // whatever the lengths are. A sequence that lies in one range is finished by its wave; one that is spread over several
-// leaves partial results (at most two per range), and the last of its waves to arrive merges them, so nobody waits.
+// leaves partial results (at most two per range), which the next launch merges (decode_stream_merge_kernel).
 // What bounds it: the K/V stream from HBM (B 32, 64 / 8 heads, 32768 keys: 650 us, 6.6 TB/s), and for little work the
 // chain lens -> table -> rows -> merge (B 1, 32 / 8 heads, 64 keys: 9 us). Against 32 splits per sequence, a combine launch
 // and the form for even lengths behind which the other one was queued, whole calls: 48 sequences of 128 to 8192 keys, f16,
@@ -1402,14 +1401,13 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodePara
 // with 32 splits and their combine (eight head blocks fetching both row sets, 134 MB of partial results) -> 66 us.
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
 __global__ __launch_bounds__(NW * 64) void decode_stream_group_kernel(const DecodeParams prm) {
-  decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, true, false, false, false, true>(prm);
+  decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, false, false, false, false, true>(prm);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
 static int launch_stream_group_cfg(DecodeParams& prm, int head_blocks, hipStream_t stream) {
   typedef DecodeCfg<D, DPE, KEYS, NST, true> C;
   static_assert((32 + 16 * decode_acc_row(D) + 128) * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
-  static_assert(64 + 16 * kStreamMaxParts * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
   const size_t lds = (size_t)(NW / 2) * C::kWaveBytes;
   static_assert((size_t)(NW / 2) * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
   auto kern = decode_stream_group_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap>;
@@ -1421,13 +1419,13 @@ static int launch_stream_group_cfg(DecodeParams& prm, int head_blocks, hipStream
   }
   prm.min_blocks = NW;   // two steps of every stream of keys
   hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)prm.ranges * prm.Hkv * head_blocks)), dim3(NW * 64), lds, stream, prm);
-  return launch_status("tdist_decode_stream");
+  if (int rc = launch_status("tdist_decode_stream")) return rc;
+  return launch_stream_merge<KEYS>(prm, stream);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kPadded>
 static int launch_stream_cfg(DecodeParams& prm, int head_blocks, hipStream_t stream) {
   typedef DecodeCfg<D, DPE, KEYS, NST> C;
-  static_assert(16 * kStreamMaxParts * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
   const size_t lds = (size_t)NW * C::kWaveBytes;
   static_assert((size_t)NW * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
   auto kern = decode_stream_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap, kPadded>;
@@ -1440,7 +1438,8 @@ static int launch_stream_cfg(DecodeParams& prm, int head_blocks, hipStream_t str
   prm.min_blocks = 64 / KEYS;
   const int64_t waves = (int64_t)prm.ranges * prm.Hkv * head_blocks;
   hipLaunchKernelGGL(kern, dim3((unsigned)((waves + NW - 1) / NW)), dim3(NW * 64), lds, stream, prm);
-  return launch_status("tdist_decode_stream");
+  if (int rc = launch_status("tdist_decode_stream")) return rc;
+  return launch_stream_merge<KEYS>(prm, stream);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kPadded>
@@ -1523,7 +1522,8 @@ static int64_t stream_workspace_bytes(int batch, int q_heads, int kv_heads, int 
 
 static int run_decode(const DecodeCall& c, DecodeForm form) {
   const char* who = c.who;
-  const bool fuse = form != kFormSplit;
+  const bool whole = form != kFormSplit;   // the call's output is the merged result
+  const bool fuse = form == kFormFused;
   if (!c.q || !c.k_cache || !c.v_cache || !c.block_table || !c.kv_lens ||
       (form == kFormStream ? !c.workspace : !c.out_split || !c.lse_split))
     return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
@@ -1559,6 +1559,7 @@ static int run_decode(const DecodeCall& c, DecodeForm form) {
   prm.Hq = c.q_heads;
   prm.Hkv = c.kv_heads;
   prm.S = c.num_splits;
+  prm.dv = dv;
   prm.d_valid = dk;
   prm.part_vec = aligned16(c.out_split);
   prm.splits_per_team = 1;
@@ -1582,16 +1583,18 @@ static int run_decode(const DecodeCall& c, DecodeForm form) {
   prm.final_lse = nullptr;
   prm.final_dtype = TDIST_F32;
   prm.fo_sb = prm.fo_sh = 0;
-  if (fuse) {
-    if (!c.counters || !c.out) return fail(TDIST_ERR_INVALID, "%s: null counters or output", who);
+  if (whole) {
+    if ((fuse && !c.counters) || !c.out) return fail(TDIST_ERR_INVALID, "%s: null counters or output", who);
     if (!aligned16(form == kFormStream ? c.workspace : c.out_split))
       return fail(TDIST_ERR_UNSUPPORTED, "%s: %s must be 16-byte aligned", who, form == kFormStream ? "workspace" : "out_split");
     if (c.out_dtype != TDIST_F32 && c.out_dtype != TDIST_BF16 && c.out_dtype != TDIST_F16)
       return fail(TDIST_ERR_UNSUPPORTED, "%s: output dtype %d", who, c.out_dtype);
-    const int64_t need = decode_fused_counters(c.batch, c.q_heads, c.kv_heads);
-    if (c.n_counters < need)
-      return fail(TDIST_ERR_WORKSPACE, "%s: %lld counters given, %lld needed", who, (long long)c.n_counters, (long long)need);
-    prm.counters = c.counters;
+    if (fuse) {
+      const int64_t need = decode_fused_counters(c.batch, c.q_heads, c.kv_heads);
+      if (c.n_counters < need)
+        return fail(TDIST_ERR_WORKSPACE, "%s: %lld counters given, %lld needed", who, (long long)c.n_counters, (long long)need);
+      prm.counters = c.counters;
+    }
     prm.final_out = (unsigned char*)c.out;
     prm.final_lse = c.lse_out;
     prm.final_dtype = c.out_dtype;
@@ -1771,13 +1774,13 @@ int tdist_decode_stream(const void* q, const void* k_cache, const void* v_cache,
                         const int32_t* block_table, const int32_t* kv_lens, int batch, int q_heads, int kv_heads,
                         int head_dim, int head_dim_v, int page_size, int64_t q_stride_b, int64_t q_stride_h,
                         int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
-                        int64_t v_stride_token, int64_t v_stride_head, int64_t table_stride, int dtype, int32_t* counters,
-                        int64_t n_counters, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                        int64_t v_stride_token, int64_t v_stride_head, int64_t table_stride, int dtype, int32_t* /*counters*/,
+                        int64_t /*n_counters*/, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
                         int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream) {
   DecodeCall c = {q, k_cache, v_cache, nullptr, nullptr, sm_scale, soft_cap, block_table, kv_lens, batch, q_heads,
                   kv_heads, head_dim, head_dim_v, page_size, 1, q_stride_b, q_stride_h, k_stride_page,
                   k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, table_stride, dtype,
-                  counters, n_counters, out, out_dtype, out_stride_b, out_stride_h, lse_out, stream,
+                  nullptr, 0, out, out_dtype, out_stride_b, out_stride_h, lse_out, stream,
                   "tdist_decode_stream", workspace, workspace_bytes};
   return run_decode(c, kFormStream);
 }

@@ -78,18 +78,22 @@ def _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num_sp
 _fused_counters = {}   # (device index, stream handle) -> zero-initialised int32 counters (the kernel leaves them zero)
 
 
+def _check_counters(q, kv_heads, counters):
+    """``counters``: a contiguous int32 device tensor of at least tdist_decode_fused_counters(...) entries; that many."""
+    need = _lib.load().tdist_decode_fused_counters(q.shape[0], q.shape[1], kv_heads)
+    if counters is not None and not (isinstance(counters, torch.Tensor) and counters.is_cuda and counters.dtype == torch.int32
+                                     and counters.is_contiguous() and counters.numel() >= need):
+        raise ValueError("counters: a contiguous int32 device tensor of at least %d zeroed entries" % need)
+    return need
+
+
 def _counters_for(q, kv_heads, counters):
-    """Arrival counters of the fused launch. ``counters`` (an explicit opt-in of this module's own callers: the layer,
-    the tests): a contiguous int32 device tensor of at least tdist_decode_fused_counters(...) entries that is ALL ZERO
-    and shared with no launch that may overlap this one; the kernel leaves it zero. None: a zeroed buffer cached per
-    (device, current stream): launches on one stream are ordered, so they may share it, and launches on different
+    """Arrival counters of the fused launch. ``counters`` (an explicit opt-in of decode_fused's callers): see _check_counters;
+    ALL ZERO and shared with no launch that may overlap this one; the kernel leaves it zero. None: a zeroed buffer cached
+    per (device, current stream): launches on one stream are ordered, so they may share it, and launches on different
     streams never do."""
-    batch, q_heads, _ = q.shape
-    need = _lib.load().tdist_decode_fused_counters(batch, q_heads, kv_heads)
+    need = _check_counters(q, kv_heads, counters)
     if counters is not None:
-        if not (isinstance(counters, torch.Tensor) and counters.is_cuda and counters.dtype == torch.int32
-                and counters.is_contiguous() and counters.numel() >= need):
-            raise ValueError("counters: a contiguous int32 device tensor of at least %d zeroed entries" % need)
         return counters, counters.numel()
     key = (q.device.index, torch.cuda.current_stream(q.device).cuda_stream)
     buf = _fused_counters.get(key)
@@ -131,9 +135,9 @@ def _few_long_sequences(batch, q_heads, kv_heads, dk, keys):
 
 
 def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, out, lse_out=None, counters=None):
-    """tdist_decode_stream: the whole decode in one launch that divides the keys itself. ``out`` [B,Hq,Dv] (bf16 / f16 /
-    fp32), ``lse_out`` contiguous fp32 [B,Hq] or None. ``counters`` as in _counters_for. The 576 / 512 heads take this
-    form where the value is a view of the key's first columns; with a value cache of its own, and for few long sequences
+    """tdist_decode_stream: a launch that divides the batch's keys itself and one that merges the sequences it spread over
+    several places. ``out`` [B,Hq,Dv] (bf16 / f16 / fp32), ``lse_out`` contiguous fp32 [B,Hq] or None. No state outlives the
+    call (``counters`` is checked and not used). The 576 / 512 heads take this form where the value is a view of the key's first columns; with a value cache of its own, and for few long sequences
     (_few_long_sequences), the call runs as a fixed number of splits and their combine. Returns ``out``."""
     kv_lens, block_table = _check_inputs(q, k_cache, v_cache, kv_lens, block_table)
     batch, q_heads, dk = q.shape
@@ -152,12 +156,13 @@ def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, ou
         if len(_STREAM_PLANS) >= 1024:
             _STREAM_PLANS.clear()
         need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv)
-    counters, n_counters = _counters_for(q, kv_heads, counters)
+    if counters is not None:
+        _check_counters(q, kv_heads, counters)
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     _lib.call("tdist_decode_stream", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), scale, soft_cap,
               block_table.data_ptr(), kv_lens.data_ptr(), batch, q_heads, kv_heads, dk, dv, page_size, qs[0], qs[1], ks[0],
-              ks[1], ks[2], vs[0], vs[1], vs[2], block_table.stride(0), _lib.dtype_code(q.dtype), counters.data_ptr(),
-              n_counters, workspace.data_ptr(), need, out.data_ptr(), _lib.dtype_code(out.dtype), os[0], os[1],
+              ks[1], ks[2], vs[0], vs[1], vs[2], block_table.stride(0), _lib.dtype_code(q.dtype), None, 0,
+              workspace.data_ptr(), need, out.data_ptr(), _lib.dtype_code(out.dtype), os[0], os[1],
               _lib.ptr(lse_out), _lib.stream_ptr())
     return out
 
@@ -178,7 +183,7 @@ def gqa_fwd_batch_decode(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_
 
     q [B,Hq,D]; k_cache / v_cache [num_pages, page_size, Hkv, D]; kv_lens int32[B]; block_table int32
     [B, max_pages]. ``workspace`` and ``q_lens`` are accepted and unused, as in the reference.
-    ``output_split`` is ignored: one launch divides the keys of the whole batch evenly over the chip, whatever the
+    ``output_split`` is ignored: the keys of the whole batch are divided evenly over the chip, whatever the
     lengths (``kv_split``, the reference's fixed number of splits per sequence, is accepted for its signature and
     changes nothing in the result). Returns ``output_combine`` [B,Hq,Dv] (default dtype: q's; the reference hard-codes
     float16, :784)."""
@@ -189,13 +194,13 @@ def gqa_fwd_batch_decode(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_
 
 def gqa_fwd_batch_decode_persistent(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_table, scale, soft_cap=0.0,
                                     output_split=None, output_combine=None, kv_split=-1):
-    """Same result as gqa_fwd_batch_decode in one launch (reference :931-1004: split-KV, a grid barrier on
-    ``workspace``, then the combine). Here the last workgroup to finish a (sequence, head block) merges its splits.
-    ``workspace`` (the reference's barrier buffer) and ``q_lens`` are accepted and unused: nothing says what a
-    caller's buffer holds or who else uses it, and a counter that does not start at zero makes a merge fire early or
-    never, so the arrival counters are the library's own (zeroed, cached per device and stream, left zero by every
-    call). ``output_split`` is ignored (partials are fp32 internally). ``kv_split`` = -1: the launch divides the keys
-    itself, as gqa_fwd_batch_decode does; otherwise every sequence is cut into that many splits."""
+    """Same result as gqa_fwd_batch_decode (reference :931-1004: split-KV, a grid barrier on ``workspace``, then the
+    combine). ``kv_split`` = -1: as gqa_fwd_batch_decode. Otherwise every sequence is cut into that many splits in one
+    launch, in which the last workgroup to finish a (sequence, head block) merges its splits. ``workspace`` (the
+    reference's barrier buffer) and ``q_lens`` are accepted and unused: nothing says what a caller's buffer holds or who
+    else uses it, and a counter that does not start at zero makes a merge fire early or never, so the arrival counters
+    are the library's own (zeroed, cached per device and stream, left zero by every call). ``output_split`` is ignored
+    (partials are fp32 internally)."""
     batch, q_heads, _ = q.shape
     if output_combine is None:
         output_combine = torch.empty((batch, q_heads, v_cache.shape[-1]), dtype=q.dtype, device=q.device)
@@ -211,15 +216,14 @@ def gqa_fwd_batch_decode_intra_rank(q, k_cache, v_cache, workspace, q_lens, kv_l
     :847-928). Returns ``output_combine`` [B,Hq,Dv+1] with the LSE in column Dv, fp32 unless the caller
     passes a buffer of another dtype (the reference uses q's dtype). With ``return_lse`` also returns the
     fp32 (out [B,Hq,Dv], lse [B,Hq]) pair the merge produced. ``workspace`` and ``q_lens`` are accepted and unused, as
-    in the reference; ``counters`` (keyword only in spirit: an addition) hands in zeroed arrival counters of the
-    caller's own, see _counters_for."""
+    in the reference; ``counters`` (keyword only in spirit: an addition) likewise, if it is what _check_counters asks for."""
     batch, q_heads, _ = q.shape
     dv = v_cache.shape[-1]
     if output_combine is None:
         output_combine = torch.empty((batch, q_heads, dv + 1), dtype=torch.float32, device=q.device)
     out32 = torch.empty((batch, q_heads, dv), dtype=torch.float32, device=q.device)
     lse32 = torch.empty((batch, q_heads), dtype=torch.float32, device=q.device)
-    # the keys divided and merged (keeping the LSE) in one launch
+    # the keys divided and merged, keeping the LSE
     decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, out32, lse32, counters=counters)
     output_combine[..., :dv].copy_(out32)
     output_combine[..., dv].copy_(lse32)

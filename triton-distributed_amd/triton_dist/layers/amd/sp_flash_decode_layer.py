@@ -8,7 +8,6 @@ the gather has nobody to talk to: the partial results of the other ranks are pas
 """
 import torch
 
-from triton_dist import _lib
 from triton_dist.kernels.amd.flash_decode import decode_stream, gqa_fwd_batch_decode_inter_rank_combine
 
 
@@ -29,11 +28,10 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         self.q_head_dim, self.v_head_dim = q_head_dim, v_head_dim
         self.page_size = page_size
         self.scale, self.soft_cap = scale, soft_cap
-        self.kv_split = 32                    # recorded (the reference cuts every sequence into 32, :59; here the launch
+        self.kv_split = 32                    # recorded (the reference cuts every sequence into 32, :59; here the call
                                               # divides the batch's keys itself)
         self.max_allowed_batch = max_allowed_batch
-        # the fused decode keeps its arrival counters per layer, so that two layers may run on two streams
-        self.workspace = None
+        self.workspace = None                 # (the reference's workspace; a call keeps nothing here)
         self.stages = stages
         self.shrink_buffer_threshold = thrink_buffer_threshold
 
@@ -50,9 +48,6 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         assert global_kv_lens.shape[0] == self.num_ranks
         assert global_kv_lens.shape[1] == batch
         assert batch <= self.max_allowed_batch, f"Only support {self.max_allowed_batch} queries decode now"
-        if self.workspace is None or self.workspace.device != q.device:
-            n = _lib.load().tdist_decode_fused_counters(self.max_allowed_batch, self.num_q_heads, self.num_kv_heads)
-            self.workspace = torch.zeros(max(int(n), 1), dtype=torch.int32, device=q.device)
         if self.num_ranks == 1:
             all_out = torch.empty((1, batch, self.num_q_heads, self.v_head_dim), dtype=torch.float32, device=q.device)
             all_lse = torch.empty((1, batch, self.num_q_heads), dtype=torch.float32, device=q.device)
@@ -66,8 +61,7 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         own_out, own_lse = all_out[self.rank], all_lse[self.rank]
         lse = own_lse if own_lse.dtype == torch.float32 and own_lse.is_contiguous() else torch.empty_like(
             own_lse, dtype=torch.float32, memory_format=torch.contiguous_format)
-        decode_stream(q, k_cache, v_cache, global_kv_lens[self.rank], block_table, self.scale, self.soft_cap, own_out, lse,
-                      counters=self.workspace)
+        decode_stream(q, k_cache, v_cache, global_kv_lens[self.rank], block_table, self.scale, self.soft_cap, own_out, lse)
         if lse is not own_lse:
             own_lse.copy_(lse)
         return gqa_fwd_batch_decode_inter_rank_combine(all_out, all_lse, global_kv_lens, out_dtype=q.dtype)
