@@ -41,7 +41,7 @@ MEASURED_TRAFFIC_BYTES = {
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
-    "decode.hip": "b4ea45912b78b068",
+    "decode.hip": "7741974f667a3d5e",
     "gemm.hip": "f5e3c8dbadd4a963",
     "moe.hip": "178cbc1874360811",
     "reduce.hip": "469689d34df1b205",

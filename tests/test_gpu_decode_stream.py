@@ -87,8 +87,9 @@ def test_workspace_and_head_dimensions_are_checked(cuda):
 @pytest.mark.parametrize("B,Hq,Hkv,D,lens,dtype", [(1, 64, 8, 128, [6016], torch.bfloat16), (5, 32, 8, 96, [6001, 17, 300, 0, 2048], torch.float16),
                                                    (12, 6, 1, 128, [6100] + [33] * 11, torch.bfloat16), (8, 6, 1, 72, [1] * 8, torch.float16)])
 def test_few_long_sequences_take_either_form_with_one_result(cuda, B, Hq, Hkv, D, lens, dtype):
-    """A page table with room for more than 6000 keys sends few sequences to the split form; the lengths are the same behind
-    a narrow table, which the streaming form takes. Both hold fp32 partial results: they differ by one rounding of the output."""
+    """A fixed number of splits and their combine on the same inputs. Both hold fp32 partial results: they differ by one
+    rounding of the output. And the room a page table has beyond the sequences' pages changes nothing, not even the route:
+    the same bits behind a narrow table and one four times as wide."""
     from triton_dist.kernels.amd import flash_decode as fd
     announce("few long sequences B=%d heads %d/%d D=%d" % (B, Hq, Hkv, D))
     g = torch.Generator().manual_seed(B + D)
@@ -97,14 +98,27 @@ def test_few_long_sequences_take_either_form_with_one_result(cuda, B, Hq, Hkv, D
     v = torch.randn((pages, page, Hkv, D), generator=g).to(dtype).to(cuda)
     q = torch.randn((B, Hq, D), generator=g).to(dtype).to(cuda)
     need = max(1, -(-max(lens) // page))
-    table = torch.randint(0, pages, (B, max(need, 376)), generator=g, dtype=torch.int32).to(cuda)
+    wide = torch.randint(0, pages, (B, 4 * max(need, 376)), generator=g, dtype=torch.int32).to(cuda)
     kv_lens = torch.tensor(lens, dtype=torch.int32, device=cuda)
-    assert fd._few_long_sequences(B, Hq, Hkv, D, table.shape[1] * page)
-    got = fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, table, D ** -0.5)
-    rule, fd._few_long_sequences = fd._few_long_sequences, lambda *a: False
-    try:
-        want = fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, table, D ** -0.5)
-    finally:
-        fd._few_long_sequences = rule
+    got = fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, wide, D ** -0.5)
+    assert torch.equal(got, fd.gqa_fwd_batch_decode(q, k, v, None, [1] * B, kv_lens, wide[:, :need], D ** -0.5))
+    S = fd.DEFAULT_KV_SPLITS
+    part, lse, _ = fd._split_kv(q, k, v, kv_lens, wide, D ** -0.5, 0.0, S)
+    want = fd.decode_combine(part, lse, S, 1, kv_lens, B, Hq, D, (part.stride(2), part.stride(0), part.stride(1)),
+                             (lse.stride(2), lse.stride(0), lse.stride(1)), torch.empty_like(got))
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     assert ((got.float() - want.float()).abs() <= 2 * eps * want.float().abs() + 1e-5).all()
+
+
+# one sequence over 1024, 512, 341, 256 and 128 ranges (merged by 16 waves a workgroup above 256, by four below), alone and
+# beside short ones
+@pytest.mark.parametrize("lens", [[21000], [3, 0, 21000, 700]])
+@pytest.mark.parametrize("num_heads,D", [((6, 1), 128), ((10, 2), 64), ((24, 3), 96), ((16, 4), 128), ((16, 8), 64), ((20, 1), 256)])
+def test_a_long_sequence_over_many_ranges(cuda, num_heads, D, lens):
+    announce("decode stream, many ranges, heads=%s D=%d lens=%s" % (num_heads, D, lens))
+    check(cuda, num_heads, (D, D), torch.bfloat16, lens, 16, 0, False, D + len(lens))
+
+
+def test_a_long_latent_sequence(cuda):
+    announce("decode stream, many ranges, latent heads")
+    check(cuda, (16, 1), (576, 512), torch.bfloat16, [21000, 40], 16, 0, True, 5)

@@ -231,8 +231,6 @@ __device__ __forceinline__ int xcd_major(int i, int n) {
 }
 
 // ---- streaming form: which blocks a range holds -----------------------------------------------------------
-constexpr int kStreamMaxParts = 64;   // ranges one sequence may be spread over
-
 struct StreamRange {
   int n;            // blocks in the range (0: the batch has fewer ranges)
   int seq, block;   // the sequence its first block belongs to, and that block's number in the sequence
@@ -240,10 +238,9 @@ struct StreamRange {
   int per;          // blocks per range
 };
 
-// Blocks per range, from the batch's blocks and its longest sequence's: even shares, but no shorter than min_blocks and no
-// more than kStreamMaxParts ranges to a sequence (a sequence of n blocks touches at most ceil(n / per) + 1 ranges).
-__device__ __forceinline__ int stream_blocks_per_range(const DecodeParams& prm, int total, int longest) {
-  return max(max((total + prm.ranges - 1) / prm.ranges, prm.min_blocks), (longest + kStreamMaxParts - 2) / (kStreamMaxParts - 1));
+// Blocks per range, from the batch's blocks: even shares, but no shorter than min_blocks.
+__device__ __forceinline__ int stream_blocks_per_range(const DecodeParams& prm, int total) {
+  return max((total + prm.ranges - 1) / prm.ranges, prm.min_blocks);
 }
 
 // All sequences' blocks laid end to end and cut into ranges of `per` blocks: the same answer in every wave, from one
@@ -252,7 +249,7 @@ template <int KEYS>
 __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int range) {
   const int lane = threadIdx.x & 63;
   auto blocks = [&](int i) { return i < prm.B ? (max(prm.lens[i], 0) + KEYS - 1) / KEYS : 0; };
-  int nb = 0, sum = 0, mx = 0, total = 0;
+  int nb = 0, sum = 0, total = 0;
   auto scan = [&](int i0) {   // sum: this lane's sequence and the ones before it within the 64
     nb = blocks(i0 + lane);
     sum = nb;
@@ -264,14 +261,10 @@ __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int
   };
   for (int i0 = 0; i0 < prm.B; i0 += 64) {
     scan(i0);
-    mx = max(mx, nb);
     total += __builtin_amdgcn_readlane(sum, 63);
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
-  mx = __builtin_amdgcn_readfirstlane(mx);
   StreamRange r;
-  r.per = stream_blocks_per_range(prm, total, mx);
+  r.per = stream_blocks_per_range(prm, total);
   const long long g0 = (long long)range * r.per;
   r.seq = r.block = r.first_block = 0;
   if (g0 >= total) {
@@ -299,21 +292,19 @@ __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int
 template <int KEYS>
 __device__ __forceinline__ void stream_sequence(const DecodeParams& prm, int seq, int& first_block, int& per) {
   const int lane = threadIdx.x & 63;
-  int total = 0, before = 0, mx = 0;
+  int total = 0, before = 0;
   for (int i = lane; i < prm.B; i += 64) {
     const int nb = (max(prm.lens[i], 0) + KEYS - 1) / KEYS;
     total += nb;
     before += i < seq ? nb : 0;
-    mx = max(mx, nb);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     total += __shfl_xor(total, o);
     before += __shfl_xor(before, o);
-    mx = max(mx, __shfl_xor(mx, o));
   }
   first_block = __builtin_amdgcn_readfirstlane(before);
-  per = stream_blocks_per_range(prm, __builtin_amdgcn_readfirstlane(total), __builtin_amdgcn_readfirstlane(mx));
+  per = stream_blocks_per_range(prm, __builtin_amdgcn_readfirstlane(total));
 }
 
 // Are the B sequence lengths even enough for the form that hands a workgroup 8 kv heads of one (sequence, split)?
@@ -1280,6 +1271,8 @@ static int launch_decode_cfg(const DecodeParams& prm, int head_blocks, hipStream
   return launch_status(kFuse ? "tdist_decode_fused" : "tdist_decode_split_kv");
 }
 
+constexpr int kMergeBatch = 16;   // partial results in flight per lane of the merge
+
 // The second launch of the streaming form: the partial results of every sequence that is spread over several ranges into its
 // result. A workgroup takes 64 16-byte pieces of one sequence's [Hq, Dv] plane; partial j of the sequence lies in the second
 // slot of the range in which it begins (j = 0) and in the first slot of the others; a wave takes a run of them, kBatch rows and
@@ -1290,10 +1283,12 @@ static int launch_decode_cfg(const DecodeParams& prm, int head_blocks, hipStream
 // it, and the partials of a long sequence are read by as many waves as its result has pieces.
 // What bounds it: the launch and two trips to memory (lengths; rows and LSEs). Against the merge by the last wave to arrive, whole
 // calls: 1 x 1320 keys, 32 / 8 heads 16.8 -> 16.0 us; latent heads, 16 up to 4096 keys 60.4 -> 57.7; 48 up to 8192 74.9 -> 75.7;
-// 32 x 32768 660 -> 664.
+// 32 x 32768 660 -> 664. One wave could merge 63 ranges of a sequence at most; without that limit 1 x 131072 keys take 36 us
+// instead of 156 with 6 / 1 heads and 87 instead of 155 with 32 / 8 (32 splits and their combine: 90, 91).
+// 16 waves a workgroup where a sequence may have more partials than four waves hold in flight.
 template <int KEYS, int NW>
 __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm) {
-  constexpr int kBatch = 16;
+  constexpr int kBatch = kMergeBatch;
   __shared__ float4v s_acc[NW][64];
   __shared__ float s_max[NW][64], s_sum[NW][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1373,7 +1368,10 @@ template <int KEYS>
 static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
   if (prm.ranges == 1) return TDIST_OK;   // every sequence lies in the one range
   const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
-  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 4>), dim3((unsigned)(places * pieces)), dim3(256), 0, stream, prm);
+  if (prm.ranges > 4 * kMergeBatch * 4)
+    hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 16>), dim3((unsigned)(places * pieces)), dim3(1024), 0, stream, prm);
+  else
+    hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 4>), dim3((unsigned)(places * pieces)), dim3(256), 0, stream, prm);
   return launch_status("tdist_decode_stream");
 }
 

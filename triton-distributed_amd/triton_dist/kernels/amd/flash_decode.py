@@ -122,30 +122,18 @@ def decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num
 _STREAM_PLANS = {}   # (batch, q heads, kv heads, head dims, device) -> workspace bytes
 
 
-def _few_long_sequences(batch, q_heads, kv_heads, dk, keys):
-    """Whether a fixed number of splits and their combine are the faster form: few sequences of up to ``keys`` keys, so that
-    each is spread over as many ranges as the streaming form allows (63) and one wave's merge of those takes as long as their
-    streams. Measured with 64 < dk <= 128 (us, streaming / splits + combine): 1 x 7310 keys, 64 / 8 heads 34.5 / 29.3; 4 up to
-    7415, 32 / 8 32.4 / 29.2; 5 up to 11667 40 / 34.6; 12 up to 8873, 6 / 1 heads 30-35 / 28.5; 3 up to 7351, 6 / 1
-    33.2 / 28.2. Beyond the lines: 1 x 1320
-    keys 16.9 / 27.3; 4 up to 5596, 16 / 16 (64 units) 32.9 / 39.5; 2 up to 7289, 6 / 1 (2 units) 27.1 / 29.4; 64-wide heads
-    1 x 9233 27.3 / 28.9. The host knows no length, only how many keys the page table has room for."""
-    units = batch * kv_heads * ((q_heads // kv_heads + 15) // 16)
-    return 64 < dk <= 128 and 3 <= units <= 40 and keys > 6000
-
-
 def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, out, lse_out=None, counters=None):
     """tdist_decode_stream: a launch that divides the batch's keys itself and one that merges the sequences it spread over
     several places. ``out`` [B,Hq,Dv] (bf16 / f16 / fp32), ``lse_out`` contiguous fp32 [B,Hq] or None. No state outlives the
-    call (``counters`` is checked and not used). The 576 / 512 heads take this form where the value is a view of the key's first columns; with a value cache of its own, and for few long sequences
-    (_few_long_sequences), the call runs as a fixed number of splits and their combine. Returns ``out``."""
+    call (``counters`` is checked and not used). The 576 / 512 heads take
+    this form where the value is a view of the key's first columns; with a value cache of its own the call runs as a fixed
+    number of splits and their combine. Returns ``out``."""
     kv_lens, block_table = _check_inputs(q, k_cache, v_cache, kv_lens, block_table)
     batch, q_heads, dk = q.shape
     _, page_size, kv_heads, dv = v_cache.shape
     assert out.stride(-1) == 1 and (lse_out is None or (lse_out.dtype == torch.float32 and lse_out.is_contiguous()))
     qs, ks, vs, os = q.stride(), k_cache.stride(), v_cache.stride(), out.stride()
-    if (dk > 256 and (k_cache.data_ptr() != v_cache.data_ptr() or ks != vs)) or _few_long_sequences(
-            batch, q_heads, kv_heads, dk, block_table.shape[1] * page_size):
+    if dk > 256 and (k_cache.data_ptr() != v_cache.data_ptr() or ks != vs):
         S = DEFAULT_KV_SPLITS
         part, lse, kv_lens = _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, S)
         return decode_combine(part, lse, S, 1, kv_lens, batch, q_heads, dv, (part.stride(2), part.stride(0), part.stride(1)),
