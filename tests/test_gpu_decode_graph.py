@@ -1,6 +1,7 @@
 """Decode under HIP graphs, as it is served: one graph per batch size, captured one after the other on torch's capture
-stream, replayed in any order and from several streams, on lengths that change between the replays. A call keeps nothing
-that outlives it, so no graph depends on another's having run, or on eager calls."""
+stream, replayed in any order and from several streams, on lengths that change between the replays. A captured call keeps nothing
+that outlives it, so no graph depends on another's having run, or on eager calls. Likewise the align / sort in the form that
+goes through scratch memory."""
 import pytest
 import torch
 
@@ -41,7 +42,8 @@ class Served:
         assert (self.out.cpu().double() - exact).abs().max() <= ATOL
 
 
-@pytest.mark.parametrize("entry,split", [("gqa_fwd_batch_decode", -1), ("gqa_fwd_batch_decode_persistent", -1)])
+@pytest.mark.parametrize("entry,split", [("gqa_fwd_batch_decode", -1), ("gqa_fwd_batch_decode_persistent", -1),
+                                         ("gqa_fwd_batch_decode_persistent", 16)])
 @pytest.mark.parametrize("heads,dims,latent", [((32, 8), (128, 128), False), ((128, 1), (576, 512), True)])
 def test_graphs_of_two_batch_sizes_in_reverse_order_and_on_two_streams(cuda, entry, split, heads, dims, latent):
     from triton_dist.kernels.amd import flash_decode
@@ -87,3 +89,40 @@ def test_layer_captured_twice(cuda):
         exact, _ = golden.decode_exact(s.q, s.k, s.v, lens, s.table, s.scale, 0)
         # the layer's result is bf16: its rounding step beside the bar
         assert ((s.out.cpu().double() - exact).abs() <= ATOL + 2.0 ** -8 * exact.abs()).all()
+
+
+def test_sort_in_two_graphs_at_once(cuda):
+    """More entries than the one-launch form takes: three launches through a scratch tensor, which eager calls share per
+    stream and captured ones must not."""
+    from triton_dist import _lib
+    from triton_dist.kernels.amd import sort_topk_ids_align_block_size
+    announce("align / sort graphs")
+    E, block = 16, 128
+    made = []
+    for tokens, seed in ((9000, 1), (20000, 2)):
+        ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(seed * 100000 + t))[:8] for t in range(64)])
+        ids = ids.repeat(-(-tokens // 64), 1)[:tokens].contiguous()
+        ids_d = ids.to(cuda)
+        sort_topk_ids_align_block_size(ids_d, E, 1, tokens, block)
+        graph = torch.cuda.CUDAGraph()
+        before = dict(_lib._zero_scratch)
+        with torch.cuda.graph(graph):
+            out = sort_topk_ids_align_block_size(ids_d, E, 1, tokens, block)
+        assert {k: v.data_ptr() for k, v in _lib._zero_scratch.items()} == {k: v.data_ptr() for k, v in before.items()}
+        want = golden.sort_topk_ids_align_block_size(ids, E, 1, tokens, block)
+        made.append((graph, ids_d, out, want))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(3):
+        for _, _, out, _ in made:
+            for t in out:
+                t.fill_(-5)
+        torch.cuda.synchronize()
+        for (graph, *_), stream in zip(reversed(made), streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+        torch.cuda.synchronize()
+        for _, _, out, want in made:
+            total = int(out[4].item())
+            assert total == int(want[4])
+            assert torch.equal(out[0][:total].cpu(), want[0][:total].to(torch.int32))
+            assert torch.equal(out[1][:total // block].cpu(), want[1][:total // block].to(torch.int32))

@@ -242,24 +242,33 @@ def new_split_k_workspace(device=None):
         return torch.zeros(nbytes, dtype=torch.uint8, device="cuda:%d" % dev)
 
 
+def zeros_per_stream(pool, n, least, dtype, device):
+    """``n`` zeroed elements that the kernels of the call leave at zero: allocated zero-filled once per (device, current
+    stream), ``least`` elements or more, kept in ``pool`` and handed out again on later calls, so a call allocates nothing.
+    Launches on one stream are ordered and may share them; launches on different streams never do. A call that is being
+    captured gets elements of its own, with their clearing as a kernel in front: its graph may be replayed on any stream,
+    before or beside any other graph, long after the pool has moved on to a larger buffer."""
+    import torch
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(max(int(n), 1), dtype=dtype, device=device).zero_()
+    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    buf = pool.get(key)
+    if buf is None or buf.numel() < n:
+        buf = pool[key] = torch.zeros(max(int(n), least), dtype=dtype, device=device)
+    return buf
+
+
 _zero_scratch = {}   # (device index, stream handle) -> uint8 tensor whose control words the kernels keep at zero
 
 
 def zeroed_scratch(nbytes, device):
     """A scratch tensor of at least ``nbytes`` for entry points whose workspace starts with control words that must be
-    zero on first use and are left zero by every call (the MoE index build, the align / sort): allocated zero-filled
-    once per (device, current stream) and handed out again on later calls, so a call allocates nothing. Launches on
-    one stream are ordered and may share it; launches on different streams never do."""
+    zero on first use and are left zero by every call (the MoE index build, the align / sort); see zeros_per_stream."""
     import torch
     device = torch.device(device)
     if device.index is None:
         device = torch.device("cuda", torch.cuda.current_device())
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    buf = _zero_scratch.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.zeros(max(int(nbytes), 1 << 20), dtype=torch.uint8, device=device)
-        _zero_scratch[key] = buf
-    return buf
+    return zeros_per_stream(_zero_scratch, nbytes, 1 << 20, torch.uint8, device)
 
 
 def workspace_args(ws):

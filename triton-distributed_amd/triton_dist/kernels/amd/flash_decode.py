@@ -89,18 +89,12 @@ def _check_counters(q, kv_heads, counters):
 
 def _counters_for(q, kv_heads, counters):
     """Arrival counters of the fused launch. ``counters`` (an explicit opt-in of decode_fused's callers): see _check_counters;
-    ALL ZERO and shared with no launch that may overlap this one; the kernel leaves it zero. None: a zeroed buffer cached
-    per (device, current stream): launches on one stream are ordered, so they may share it, and launches on different
-    streams never do."""
+    ALL ZERO and shared with no launch that may overlap this one; the kernel leaves it zero. None: the library's own, a
+    zeroed buffer per device and stream (_lib.zeros_per_stream)."""
     need = _check_counters(q, kv_heads, counters)
-    if counters is not None:
-        return counters, counters.numel()
-    key = (q.device.index, torch.cuda.current_stream(q.device).cuda_stream)
-    buf = _fused_counters.get(key)
-    if buf is None or buf.numel() < need:
-        buf = torch.zeros(max(int(need), 4096), dtype=torch.int32, device=q.device)
-        _fused_counters[key] = buf
-    return buf, buf.numel()
+    if counters is None:
+        counters = _lib.zeros_per_stream(_fused_counters, need, 4096, torch.int32, q.device)
+    return counters, counters.numel()
 
 
 def decode_fused(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, num_splits, out, lse_out=None,
@@ -187,7 +181,7 @@ def gqa_fwd_batch_decode_persistent(q, k_cache, v_cache, workspace, q_lens, kv_l
     launch, in which the last workgroup to finish a (sequence, head block) merges its splits. ``workspace`` (the
     reference's barrier buffer) and ``q_lens`` are accepted and unused: nothing says what a caller's buffer holds or who
     else uses it, and a counter that does not start at zero makes a merge fire early or never, so the arrival counters
-    are the library's own (zeroed, cached per device and stream, left zero by every call). ``output_split`` is ignored
+    are the library's own (_lib.zeros_per_stream). ``output_split`` is ignored
     (partials are fp32 internally)."""
     batch, q_heads, _ = q.shape
     if output_combine is None:
