@@ -43,7 +43,7 @@ MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
     "decode.hip": "7741974f667a3d5e",
     "gemm.hip": "f5e3c8dbadd4a963",
-    "moe.hip": "178cbc1874360811",
+    "moe.hip": "97f23dc5aa4ab792",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")

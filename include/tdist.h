@@ -407,6 +407,25 @@ int tdist_moe_align_block_size(const void* topk_ids, int ids_int64, int64_t n_to
                                int32_t* block_barrier_ids, int32_t* rank_block_num, int32_t* total_tokens_post_pad,
                                void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The row blocks of the align / sort without their rank segments, for a grouped GEMM that has every rank's rows at hand: the
+ * valid entries (0 <= id < num_valid_tokens) of all blocks of an expert end to end, in the order of the blocks, padded with
+ * num_valid_tokens to whole blocks of out_block rows; experts in order. num_blocks: capacity of expert_ids (sorted_token_ids
+ * holds num_blocks * block_size ids), of which *num_tokens_post_padded / block_size are in use. out_sorted_ids has out_rows
+ * entries (num_valid_tokens + num_experts * (out_block - 1) suffice where no entry is in two blocks; more than fit are dropped),
+ * out_expert_ids and out_segment_ids (all 0) out_rows / out_block, out_post_padded one. One launch, no state; block_size <= 512,
+ * num_experts <= 4096, at most about 32 000 blocks: TDIST_ERR_UNSUPPORTED otherwise. */
+int tdist_moe_join_blocks(const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* num_tokens_post_padded, int num_blocks, int block_size, int num_valid_tokens,
+                          int num_experts, int out_block, int32_t* out_sorted_ids, int64_t out_rows,
+                          int32_t* out_expert_ids, int32_t* out_segment_ids, int32_t* out_post_padded, void* stream);
+/* tdist_gather_shards and tdist_moe_join_blocks in one launch: what a grouped GEMM needs whose rows are all at hand. */
+int tdist_moe_gather_and_join(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes,
+                              int32_t* status, int32_t* first_error, const int32_t* sorted_token_ids,
+                              const int32_t* expert_ids, const int32_t* num_tokens_post_padded, int num_blocks,
+                              int block_size, int num_valid_tokens, int num_experts, int out_block,
+                              int32_t* out_sorted_ids, int64_t out_rows, int32_t* out_expert_ids,
+                              int32_t* out_segment_ids, int32_t* out_post_padded, void* stream);
+
 /* Chunk-gated grouped GEMM of the MoE tensor-parallel path: the consumer of the align / sort step.
  *   replaces kernel_consumer_m_parallel_scatter_group_gemm   kernels/nvidia/allgather_group_gemm.py:238-314
  *   as launched by rowise_intranode_ag_scatter_group_gemm    kernels/nvidia/allgather_group_gemm.py:317-403

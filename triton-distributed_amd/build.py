@@ -57,7 +57,8 @@ def _hipcc():
 
 def _inputs():
     files = [os.path.join(CSRC, s) for s in SOURCES + BENCH_SOURCES]
-    files += [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_small.h"), os.path.join(INCLUDE, "tdist.h"), os.path.join(INCLUDE, "tdist_bench.h")]
+    files += [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_small.h"), os.path.join(CSRC, "gather.h"),
+              os.path.join(INCLUDE, "tdist.h"), os.path.join(INCLUDE, "tdist_bench.h")]
     return files
 
 

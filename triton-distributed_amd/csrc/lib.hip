@@ -7,7 +7,7 @@
 #include <atomic>
 #include <mutex>
 
-#include "common.h"
+#include "gather.h"
 
 namespace tdist {
 
@@ -116,16 +116,6 @@ __global__ void flag_fill_kernel(int32_t* flags, int n, int value) {
   if (i < n) __hip_atomic_store(flags + i, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// status[0..1] of the launch before → first_error[0..1] if that is still clear; status cleared for the next launch
-__device__ __forceinline__ void retire_status(int32_t* status, int32_t* first_error) {
-  const int32_t code = status[0];
-  if (code != 0 && first_error != nullptr && first_error[0] == 0) {
-    first_error[1] = status[1];
-    first_error[0] = code;
-  }
-  status[1] = 0;
-  status[0] = 0;
-}
 __global__ void status_retire_kernel(int32_t* status, int32_t* first_error) {
   if (threadIdx.x == 0) retire_status(status, first_error);
 }
@@ -261,27 +251,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(24))) void prod
 // All ranks' rows into the workspace at once, the own ones among them: what a call does whose rows are few enough that
 // a launch in front of the GEMM costs less than flags, streams and events. A block row per rank, four 16-byte loads in
 // flight per lane. Bound by the launch at the sizes it is for (1.6 MB: 3 us); 64 MB: 25 us.
-struct GatherParams {
-  unsigned char* workspace;
-  const unsigned char* src[TDIST_GATHER_MAX_RANKS];   // (by value: no table in memory to keep in step, none to load first)
-  long long rank_bytes;
-  int32_t *status, *first_error;   // optional: retired as by tdist_status_retire
-};
 __global__ __launch_bounds__(256) void gather_shards_kernel(const GatherParams p) {
   if (p.status != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) retire_status(p.status, p.first_error);
-  const int r = blockIdx.y;
-  const int4v* const src = (const int4v*)p.src[r];
-  int4v* const dst = (int4v*)(p.workspace + r * p.rank_bytes);
-  const long long n = p.rank_bytes / 16, step = (long long)gridDim.x * 1024;
-  for (long long i0 = (long long)blockIdx.x * 1024 + threadIdx.x; i0 < n; i0 += step) {
-    int4v v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u * 256 < n) v[u] = __builtin_nontemporal_load(src + i0 + u * 256);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u * 256 < n) dst[i0 + u * 256] = v[u];   // (read again right away, by the GEMM)
-  }
+  gather_rows<256>(p, blockIdx.y, blockIdx.x, gridDim.x);
 }
 
 }  // namespace tdist
@@ -293,21 +265,8 @@ extern "C" {
 int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
                         int32_t* first_error, void* stream) {
   const char* who = "tdist_gather_shards";
-  if (!workspace || !shards) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
-  if (world_size < 1 || world_size > TDIST_GATHER_MAX_RANKS)
-    return fail(TDIST_ERR_INVALID, "%s: world_size %d (1 .. %d)", who, world_size, TDIST_GATHER_MAX_RANKS);
-  if (rank_bytes <= 0 || rank_bytes % 16 != 0 || !aligned16(workspace))
-    return fail(TDIST_ERR_UNSUPPORTED, "%s: shards of whole 16-byte pieces, 16-byte aligned", who);
-  GatherParams p = {};
-  p.workspace = (unsigned char*)workspace;
-  for (int r = 0; r < world_size; ++r) {
-    if (!shards[r]) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
-    if (!aligned16(shards[r])) return fail(TDIST_ERR_UNSUPPORTED, "%s: shards of whole 16-byte pieces, 16-byte aligned", who);
-    p.src[r] = (const unsigned char*)shards[r];
-  }
-  p.rank_bytes = rank_bytes;
-  p.status = status;
-  p.first_error = first_error;
+  GatherParams p;
+  if (int rc = gather_params(p, workspace, shards, world_size, rank_bytes, status, first_error, who)) return rc;
   const int64_t blocks = ceil_div(rank_bytes, 16 * 1024);
   hipLaunchKernelGGL(gather_shards_kernel, dim3((unsigned)(blocks < 256 ? blocks : 256), (unsigned)world_size), dim3(256), 0, (hipStream_t)stream, p);
   return launch_status(who);

@@ -15,7 +15,7 @@
 
 #include <mutex>
 
-#include "common.h"
+#include "gather.h"
 
 namespace tdist {
 
@@ -1504,6 +1504,170 @@ int moe_static_scratch_init() {
   return moe_static_scratch(&ptr, "tdist_init");
 }
 
+// ---- row blocks without rank segments ------------------------------------------------------------------------
+// The align / sort ends its row blocks with their rank segment, which is what a GEMM needs that starts on one rank's rows while
+// the others' are on their way. For a GEMM that has all rows at hand this joins them: the valid entries of all blocks of an
+// expert end to end, in the order of the blocks, padded to whole blocks of `out_block` rows. It reads the blocks as they are
+// when it runs, so whatever has been written to them since they were sorted is what the GEMM multiplies.
+// Every workgroup counts the entries of all blocks (a wave per block, 32 loads per lane in flight) and so knows every expert's
+// place; blocks and experts are then shared out among the waves of the grid. The first batch, the experts, the padded total
+// and the ids of the first block that a wave will place are all on their way before anything is waited for.
+// What bounds it: the launch, one trip to memory, four barriers. 64 blocks 4.5 us a launch with 4 waves to a workgroup (5.9 with
+// 16), 160 blocks 6.4 and 512 blocks 8.7 with 16 (half as much again with 4): 4 waves up to kJoinFewBlocks, 16 beyond. (A launch
+// that does nothing: 2.1 us.)
+constexpr int kJoinFewBlocks = 96, kJoinMaxBlock = 512, kJoinCountBits = 10;
+constexpr int64_t kJoinLdsLimit = 160 * 1024 - 256;
+struct JoinParams {
+  const int32_t *sorted_ids, *expert_ids, *post_pad;
+  int num_blocks, block_size, num_valid, E, out_block, out_rows;
+  int32_t *out_ids, *out_experts, *out_segments, *out_padded;
+};
+// Workgroup `block` of `blocks`. kChunks: 64 rows each to a block; 0: any number.
+template <int kThreads, int kChunks>
+__device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int blocks) {
+  const int32_t* __restrict__ const sorted_ids = p.sorted_ids;
+  const int32_t* __restrict__ const expert_ids = p.expert_ids;
+  int32_t* __restrict__ const out_ids = p.out_ids;
+  const int num_blocks = p.num_blocks, block_size = p.block_size, num_valid = p.num_valid, E = p.E, out_block = p.out_block,
+            out_rows = p.out_rows;
+  constexpr int kWaves = kThreads / 64, kCountMask = (1 << kJoinCountBits) - 1, kMine = kChunks > 0 ? kChunks : 1,
+                kBatch = 32 / kMine;   // blocks of a wave in flight
+  extern __shared__ int32_t s_mem[];
+  int32_t* const s_total = s_mem;           // [E] entries per expert
+  int32_t* const s_start = s_mem + E;       // [E] its first row
+  int32_t* const s_block = s_mem + 2 * E;   // [num_blocks] expert and number of entries of each block
+  __shared__ int32_t s_part[kWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int chunks = kChunks > 0 ? kChunks : (block_size + 63) / 64;
+  const int gwave = block * kWaves + wave, waves = blocks * kWaves;
+  auto valid = [&](int id) { return (uint32_t)id < (uint32_t)num_valid; };
+  // (a block beyond the last of `limit` reads that one again, so that no load depends on a branch; nobody looks at its count)
+  auto load = [&](int b, int c, int limit) {
+    const int r = c * 64 + lane;
+    const int id = sorted_ids[(int64_t)min(b, limit - 1) * block_size + (kChunks > 0 ? r : min(r, block_size - 1))];
+    return kChunks > 0 || r < block_size ? id : -1;
+  };
+  const int total_rows = p.post_pad[0];
+  int ids[kBatch][kMine], mine[kMine], expert0 = threadIdx.x < num_blocks ? expert_ids[threadIdx.x] : 0;
+  auto load_batch = [&](int b0, int c0, int limit) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+      for (int c = 0; c < kMine; ++c) ids[u][c] = load(b0 + u * kWaves, c0 + c, limit);
+  };
+  load_batch(wave, 0, num_blocks);
+#pragma unroll
+  for (int c = 0; c < kMine; ++c) mine[c] = load(gwave, c, num_blocks);
+  for (int e = threadIdx.x; e < E; e += kThreads) s_total[e] = 0;
+  const int used = __builtin_amdgcn_readfirstlane(max(min(total_rows / block_size, num_blocks), 0));
+  for (int b = threadIdx.x; b < used; b += kThreads) {
+    s_block[b] = min(max(expert0, 0), E - 1) << kJoinCountBits;
+    expert0 = b + kThreads < used ? expert_ids[b + kThreads] : 0;
+  }
+  __syncthreads();
+  for (int b0 = wave; b0 < used; b0 += kWaves * kBatch) {
+    int n = 0;   // lane u's block is b0 + u * kWaves
+    for (int c0 = 0; c0 < chunks; c0 += kMine) {
+      if (b0 != wave || c0 != 0) load_batch(b0, c0, used);
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        int count = 0;
+#pragma unroll
+        for (int c = 0; c < kMine; ++c) count += __popcll(__ballot(valid(ids[u][c])));
+        n = lane == u ? n + count : n;
+      }
+    }
+    const int b = b0 + lane * kWaves;
+    if (lane < kBatch && b < used) {
+      const int e = s_block[b] >> kJoinCountBits;
+      s_block[b] = e << kJoinCountBits | n;
+      atomicAdd(&s_total[e], n);
+    }
+  }
+  __syncthreads();
+  // exclusive prefix of the experts' padded sizes: a thread takes `per` neighbours
+  const int per = (E + kThreads - 1) / kThreads;
+  auto padded = [&](int n) { return (n + out_block - 1) / out_block * out_block; };
+  int own = 0;
+  for (int i = 0; i < per; ++i) {
+    const int e = threadIdx.x * per + i;
+    if (e < E) own += padded(s_total[e]);
+  }
+  int sum = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(sum, o);
+    if (lane >= o) sum += t;
+  }
+  if (lane == 63) s_part[wave] = sum;
+  __syncthreads();
+  int at = sum - own, all = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) at += s_part[w];
+    all += s_part[w];
+  }
+  for (int i = 0; i < per; ++i) {
+    const int e = threadIdx.x * per + i;
+    if (e < E) {
+      s_start[e] = at;
+      at += padded(s_total[e]);
+    }
+  }
+  if (block == 0 && threadIdx.x == 0) p.out_padded[0] = min(all, out_rows / out_block * out_block);
+  __syncthreads();
+  for (int b = gwave; b < used; b += waves) {
+    const int e = s_block[b] >> kJoinCountBits;
+    int before = 0;   // entries of the expert's earlier blocks
+    for (int i = lane; i < b; i += 64) {
+      const int v = s_block[i];
+      before += v >> kJoinCountBits == e ? v & kCountMask : 0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+    int row = s_start[e] + before;
+    auto place = [&](int id) {
+      const unsigned long long is = __ballot(valid(id));
+      const int to = row + __popcll(is & ((1ull << lane) - 1));
+      if (valid(id) && to < out_rows) out_ids[to] = id;
+      row += __popcll(is);
+    };
+    if (kChunks > 0 && b == gwave) {
+#pragma unroll
+      for (int c = 0; c < kMine; ++c) place(mine[c]);
+    } else {
+      for (int c = 0; c < chunks; ++c) place(load(b, c, used));
+    }
+  }
+  for (int e = gwave; e < E; e += waves) {
+    const int total = s_total[e], lo = s_start[e], hi = min(lo + padded(total), out_rows);
+    for (int r = lo + total + lane; r < hi; r += 64) out_ids[r] = num_valid;
+    for (int b = lo / out_block + lane; b < hi / out_block; b += 64) {
+      p.out_experts[b] = e;
+      p.out_segments[b] = 0;
+    }
+  }
+}
+
+template <int kThreads, int kChunks>
+__global__ __launch_bounds__(kThreads) void moe_join_blocks_kernel(const JoinParams p) {
+  join_blocks<kThreads, kChunks>(p, blockIdx.x, gridDim.x);
+}
+
+// The same beside the gather of the rows that the GEMM behind will read: the first `join_grid` workgroups join, and are done before
+// the rows are there (8 x 1024 rows by 4096: 25 us for both, 23 + 8 us as two launches).
+template <int kThreads, int kChunks>
+__global__ __launch_bounds__(kThreads) void moe_gather_and_join_kernel(const GatherParams g, const JoinParams p, int join_grid, int per_rank) {
+  const int block = blockIdx.x;
+  if (block < join_grid) {
+    if (g.status != nullptr && block == 0 && threadIdx.x == 0) retire_status(g.status, g.first_error);
+    join_blocks<kThreads, kChunks>(p, block, join_grid);
+  } else {
+    const int r = (block - join_grid) / per_rank;
+    gather_rows<kThreads>(g, r, block - join_grid - r * per_rank, per_rank);
+  }
+}
+
 }  // namespace tdist
 
 using namespace tdist;
@@ -1838,5 +2002,76 @@ int tdist_moe_align_block_size(const void* topk_ids, int ids_int64, int64_t n_to
                      block_barrier_ids, rank_block_num, total_tokens_post_pad);
   return launch_status(who);
 }
+
+#define TDIST_JOIN_ARGS                                                                                                        \
+  const int32_t *sorted_token_ids, const int32_t *expert_ids, const int32_t *num_tokens_post_padded, int num_blocks,           \
+      int block_size, int num_valid_tokens, int num_experts, int out_block, int32_t *out_sorted_ids, int64_t out_rows,         \
+      int32_t *out_expert_ids, int32_t *out_segment_ids, int32_t *out_post_padded
+#define TDIST_JOIN_NAMES                                                                                                        \
+  sorted_token_ids, expert_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, num_experts, out_block,      \
+      out_sorted_ids, out_rows, out_expert_ids, out_segment_ids, out_post_padded
+
+// Checks the arguments of a join and fills `p`, the LDS it takes, its threads and workgroups.
+struct JoinLaunch {
+  JoinParams p;
+  int64_t lds;
+  int threads, grid;
+};
+static int join_launch(JoinLaunch& j, const char* who, TDIST_JOIN_ARGS) {
+  if (!sorted_token_ids || !expert_ids || !num_tokens_post_padded || !out_sorted_ids || !out_expert_ids || !out_segment_ids ||
+      !out_post_padded)
+    return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (num_blocks <= 0 || block_size <= 0 || num_valid_tokens < 0 || num_experts <= 0 || out_block <= 0 || out_rows < out_block)
+    return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
+  j.lds = (2ll * num_experts + num_blocks) * 4;
+  if (block_size > kJoinMaxBlock || num_experts > kMoeMaxExperts || j.lds > kJoinLdsLimit || out_rows > 0x7fffffffll)
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: %d blocks of %d rows, %d experts", who, num_blocks, block_size, num_experts);
+  j.p = {sorted_token_ids, expert_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, num_experts, out_block,
+         (int)out_rows, out_sorted_ids, out_expert_ids, out_segment_ids, out_post_padded};
+  j.threads = num_blocks <= kJoinFewBlocks ? 256 : 1024;
+  const int64_t items = ceil_div(num_blocks > num_experts ? num_blocks : num_experts, j.threads / 64);
+  j.grid = (int)(items < 32 ? items : 32);
+  return TDIST_OK;
+}
+
+// The instance for the launch: the block sizes that the grouped GEMMs take, or any other.
+#define TDIST_JOIN_PICK(NAME)                                                                                                 \
+  const int which = (j.threads == 256 ? 0 : 3) + (block_size == 128 ? 0 : block_size == 256 ? 1 : 2);                         \
+  auto kern = which == 0 ? NAME<256, 2> : which == 1 ? NAME<256, 4> : which == 2 ? NAME<256, 0>                               \
+            : which == 3 ? NAME<1024, 2> : which == 4 ? NAME<1024, 4> : NAME<1024, 0>;                                        \
+  static bool attr_set[6] = {false, false, false, false, false, false};                                                       \
+  if (!attr_set[which]) {                                                                                                     \
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kJoinLdsLimit) != hipSuccess)  \
+      return fail(TDIST_ERR_LAUNCH, "%s: cannot reserve LDS", who);                                                           \
+    attr_set[which] = true;                                                                                                   \
+  }
+
+int tdist_moe_join_blocks(TDIST_JOIN_ARGS, void* stream) {
+  const char* who = "tdist_moe_join_blocks";
+  JoinLaunch j;
+  if (int rc = join_launch(j, who, TDIST_JOIN_NAMES)) return rc;
+  TDIST_JOIN_PICK(moe_join_blocks_kernel)
+  hipLaunchKernelGGL(kern, dim3((unsigned)j.grid), dim3(j.threads), (size_t)j.lds, (hipStream_t)stream, j.p);
+  return launch_status(who);
+}
+
+int tdist_moe_gather_and_join(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
+                              int32_t* first_error, TDIST_JOIN_ARGS, void* stream) {
+  const char* who = "tdist_moe_gather_and_join";
+  GatherParams g;
+  if (int rc = gather_params(g, workspace, shards, world_size, rank_bytes, status, first_error, who)) return rc;
+  JoinLaunch j;
+  if (int rc = join_launch(j, who, TDIST_JOIN_NAMES)) return rc;
+  TDIST_JOIN_PICK(moe_gather_and_join_kernel)
+  // (four 16-byte loads per lane and turn; at most two million lanes)
+  const int64_t wanted = ceil_div(rank_bytes, 16 * 4 * j.threads), most = 2048 * 1024 / j.threads / world_size;
+  const int per_rank = (int)(wanted < most ? wanted : most);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(j.grid + per_rank * world_size)), dim3(j.threads), (size_t)j.lds, (hipStream_t)stream, g, j.p,
+                     j.grid, per_rank);
+  return launch_status(who);
+}
+#undef TDIST_JOIN_PICK
+#undef TDIST_JOIN_ARGS
+#undef TDIST_JOIN_NAMES
 
 }  // extern "C"

@@ -110,31 +110,55 @@ def _row_block(entries, num_experts, n, cus):
     return min(_BLOCK_COST, key=lambda b: max(1.0, (entries / b + 0.5 * used) * cols / cus) * _BLOCK_COST[b])
 
 
-@dataclasses.dataclass
-class LocalRowBlocks:
-    """The row blocks of a grouped GEMM that waits for nobody: experts in order, with no rank segments in between.
-
-    Blocks that end with their rank segment are what a GEMM needs that starts on the rows of one rank while the others' are
-    on their way; with all rows there they only add padding (Mixtral's 8 experts x 8 ranks at 16384 entries: 160 blocks of
-    128 rows for 128 that are full, and no 256-row ones)."""
-    sorted_ids: torch.Tensor
-    expert_ids: torch.Tensor
-    segment_ids: torch.Tensor
-    num_tokens_post_padded: torch.Tensor
-    block_size: int
-    made_for: torch.Tensor   # the segmented blocks these stand for ...
-    version: int             # ... as they were then
-
-    def stand_for(self, segmented, row_bytes):
-        """Whether they (still) hold what ``segmented`` holds, and the GEMM takes rows of ``row_bytes`` in such blocks."""
-        return self.made_for is segmented and self.version == segmented._version and (row_bytes % 128 == 0 or row_bytes > 128)
+def _join_plan(entries, num_experts, n):
+    """Rows per joined block and the most blocks they can be."""
+    block = _row_block(entries, num_experts, n, _lib.load().tdist_num_cus())
+    return block, (entries + num_experts * (block - 1)) // block
 
 
-def local_row_blocks(topk_ids, num_experts, n, segmented):
-    """LocalRowBlocks of ``topk_ids`` [tokens, topk] for a GEMM with ``n`` output columns."""
-    block = _row_block(topk_ids.numel(), num_experts, n, _lib.load().tdist_num_cus())
-    ids, experts, segments, _, padded = sort_topk_ids_align_block_size(topk_ids, num_experts, 1, topk_ids.shape[0], block)
-    return LocalRowBlocks(ids, experts, segments, padded, block, segmented, segmented._version)
+class RowBlocks:
+    """Addresses of a grouped GEMM's row blocks (sorted ids, an expert and a segment per block, the padded total), their
+    number and their rows; ``memory``: the tensor they lie in."""
+    __slots__ = ("sorted_ids", "experts", "segments", "padded", "num_blocks", "block_size", "memory")
+
+    def __init__(self, sorted_ids, experts, segments, padded, num_blocks, block_size, memory=None):
+        self.sorted_ids, self.experts, self.segments, self.padded = sorted_ids, experts, segments, padded
+        self.num_blocks, self.block_size, self.memory = num_blocks, block_size, memory
+
+
+def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, block_size, entries, num_experts, n, row_bytes, stream, gather=None):
+    """The rows of ``sorted_ids`` in blocks without rank segments, for a grouped GEMM with ``n`` output columns that waits for
+    nobody: RowBlocks, or None where the GEMM does not take rows of ``row_bytes`` in such blocks or the sizes are beyond
+    tdist_moe_join_blocks (nothing has been launched then).
+
+    Blocks that end with their rank segment only add padding where all rows are there (Mixtral's 8 experts x 8 ranks at
+    16384 entries: 160 blocks of 128 rows for 128 that are full, and no 256-row ones), also where the chip has room for all
+    of them: fewer tiles are cut along K (8 x 28 tokens by 4 over 8 experts, a layer of 5248 x 1280: 111 us joined, 198 as sorted).
+    They are joined on every call, from what the tensors hold then: a caller may replace or rewrite any of them, also between
+    the replays of a graph. (Kept from call to call they cost 7 to 14 us less a layer, and a rewritten routing went unseen.)
+    ``made``: the context's memory for them, a RowBlocks per size (a graph may hold the address of any of them).
+    ``gather``: the arguments of tdist_gather_shards but its stream; the same launch then gathers."""
+    if not (row_bytes % 128 == 0 or row_bytes > 128):
+        return None
+    _lib.require_cuda(sorted_ids, expert_ids, num_tokens_post_padded)
+    key = (entries, num_experts, n)
+    out = made.get(key)
+    if out is None:
+        block, n_blocks = _join_plan(entries, num_experts, n)
+        rows = n_blocks * block
+        memory = torch.empty(rows + 2 * n_blocks + 1, dtype=torch.int32, device=sorted_ids.device)
+        base = memory.data_ptr()
+        out = made[key] = RowBlocks(base, base + 4 * rows, base + 4 * (rows + n_blocks), base + 4 * (rows + 2 * n_blocks), n_blocks, block,
+                                    memory)
+    args = (sorted_ids.data_ptr(), expert_ids.data_ptr(), num_tokens_post_padded.data_ptr(),
+            min(expert_ids.numel(), sorted_ids.numel() // block_size), block_size, entries, num_experts, out.block_size, out.sorted_ids,
+            out.num_blocks * out.block_size, out.experts, out.segments, out.padded, stream)
+    lib = _lib.load()
+    rc = lib.tdist_moe_join_blocks(*args) if gather is None else lib.tdist_moe_gather_and_join(*gather, *args)
+    if rc == _lib.TDIST_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc)
+    return out
 
 
 _GROUP_GEMM_ENTRY = {
@@ -149,19 +173,27 @@ def group_gemm_gated(a_ws, a_local, local_row_begin, b_nk, c, sorted_token_ids, 
                      *, wait_value=1, spin_limit=0, status=None, max_workgroups=0, sk_workspace=None, stream=None):
     """Thin wrapper over tdist_group_gemm_gated_*. ``a_ws`` [tokens, K] gathered rows, ``a_local`` the own shard or
     None, ``b_nk`` [E, N, K] (K contiguous), ``c`` [num_valid_tokens, N]."""
-    _lib.require_cuda(a_ws, b_nk, c, sorted_token_ids, expert_ids, block_barrier_ids, num_tokens_post_padded)
+    _lib.require_cuda(sorted_token_ids, expert_ids, block_barrier_ids, num_tokens_post_padded)
+    blocks = RowBlocks(sorted_token_ids.data_ptr(), expert_ids.data_ptr(), block_barrier_ids.data_ptr(), num_tokens_post_padded.data_ptr(),
+                       min(expert_ids.numel(), sorted_token_ids.numel() // block_size), int(block_size))
+    return _group_gemm(a_ws, a_local, local_row_begin, b_nk, c, blocks, num_valid_tokens, topk, tokens_per_rank, first_block, flags, rank,
+                       wait_value, spin_limit, status, max_workgroups, sk_workspace, stream)
+
+
+def _group_gemm(a_ws, a_local, local_row_begin, b_nk, c, blocks, num_valid_tokens, topk, tokens_per_rank, first_block, flags, rank,
+                wait_value=1, spin_limit=0, status=None, max_workgroups=0, sk_workspace=None, stream=None):
+    _lib.require_cuda(a_ws, b_nk, c)
     if a_ws.dtype not in _GROUP_GEMM_ENTRY:
         raise TypeError("unsupported grouped GEMM dtype %s" % a_ws.dtype)
     if a_ws.stride(1) != 1 or b_nk.stride(2) != 1 or c.stride(1) != 1:
         raise ValueError("A, B ([E, N, K]) and C need a contiguous last dimension")
     E, N, K = b_nk.shape
     assert a_ws.shape[1] == K and c.shape[1] == N
-    num_blocks = min(expert_ids.numel(), sorted_token_ids.numel() // block_size)
     _lib.call(_GROUP_GEMM_ENTRY[a_ws.dtype], a_ws.data_ptr(), a_ws.stride(0), _lib.ptr(a_local),
               a_local.stride(0) if a_local is not None else 0, int(local_row_begin),
               a_local.shape[0] if a_local is not None else 0, b_nk.data_ptr(), b_nk.stride(1), b_nk.stride(0), c.data_ptr(),
-              c.stride(0), a_ws.shape[0], N, K, sorted_token_ids.data_ptr(), expert_ids.data_ptr(),
-              block_barrier_ids.data_ptr(), num_tokens_post_padded.data_ptr(), num_blocks, int(block_size),
+              c.stride(0), a_ws.shape[0], N, K, blocks.sorted_ids, blocks.experts, blocks.segments, blocks.padded, blocks.num_blocks,
+              blocks.block_size,
               int(num_valid_tokens), int(topk), int(tokens_per_rank), int(first_block), _lib.ptr(flags), int(wait_value),
               int(rank), int(spin_limit), _lib.ptr(status), int(max_workgroups), *_lib.workspace_args(sk_workspace),
               _lib.stream_ptr(stream))
@@ -203,7 +235,10 @@ class MoE_AllGatherGroupGEMMTensorParallelContext:
     weight_nk: Optional[torch.Tensor] = None   # [E, N, K] copy of a [E, K, N] weight, made once per weight tensor
     weight_key: Optional[tuple] = None
     sk_workspace: Optional[torch.Tensor] = None   # the context's GEMM workspace (split of a last round along K); None = off
-    local_blocks: Optional[LocalRowBlocks] = None # row blocks for calls that have every rank's rows at hand
+    # False: the other ranks' rows come by copies beside a GEMM that waits for their flags also where they are at hand and
+    # one launch could gather them in front of it
+    gather_rows: bool = True
+    joined: dict = dataclasses.field(default_factory=dict)   # memory for the row blocks of a call, see joined_row_blocks
 
     def set_peer_shards(self, shards):
         """``shards``: dict rank -> [M_per_rank, K] tensor (or a list; the own entry is ignored): the token rows that
@@ -268,28 +303,32 @@ def create_ag_group_gemm_intra_node_context(tp_pg, tensor_A, tensor_B, full_topk
         group_gemm_stream=group_gemm_stream, BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, BLOCK_K=BLOCK_K,
         GROUP_SIZE_M=GROUP_SIZE_M, stages=stages, warps=warps, rank_block_num=rank_block_num, first_block=first_block,
         one=torch.ones((16, ), dtype=torch.int32, device=device), status=torch.zeros((4, ), dtype=torch.int32, device=device),
-        sk_workspace=_lib.new_split_k_workspace(device) if split_k else None,
-        local_blocks=local_row_blocks(full_topk_ids, num_experts, tensor_B.shape[2], sorted_ids))
+        sk_workspace=_lib.new_split_k_workspace(device) if split_k else None)
 
 
 def _gather_and_multiply(a, b_nk, c, ctx, shards):
-    """With every rank's rows at hand: one launch brings them into the workspace, the next multiplies them, on one stream, in
-    row blocks without rank segments. Against copies beside a flag-gated GEMM on 32 compute units less, in blocks that end
-    with their segment (8 x 1024 tokens by 4096, top 2 of 8 experts, 1792 columns): 323 -> 221 us."""
+    """With every rank's rows at hand: one launch brings them into the workspace and joins the row blocks across the rank
+    segments, the next multiplies them, on one stream. Against copies beside a flag-gated GEMM on 32 compute units less, in
+    blocks that end with their segment (8 x 1024 tokens by 4096, top 2 of 8 experts, 1792 columns): 323 -> 222 us. False
+    where the blocks cannot be joined (nothing has been launched then)."""
     M_per_rank, K = a.shape
-    workspace, blocks = ctx.workspace_tensors[ctx.rank], ctx.local_blocks
+    workspace = ctx.workspace_tensors[ctx.rank]
     M = M_per_rank * ctx.num_ranks
     current = _lib.stream_ptr()
     stream = current if ctx.group_gemm_stream is None else ctx.group_gemm_stream.cuda_stream
     if stream != current:
         ctx.group_gemm_stream.wait_stream(torch.cuda.current_stream())
-    _lib.call("tdist_gather_shards", workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * K * a.element_size(),
-              ctx.status.data_ptr(), ctx.status.data_ptr() + 8, stream)
-    group_gemm_gated(workspace[:M], None, 0, b_nk, c, blocks.sorted_ids, blocks.expert_ids, blocks.segment_ids,
-                     blocks.num_tokens_post_padded, blocks.block_size, ctx.full_num_tokens, ctx.topk, M, 0, None, ctx.rank,
-                     sk_workspace=ctx.sk_workspace, stream=ctx.group_gemm_stream)
+    status = ctx.status.data_ptr()
+    blocks = joined_row_blocks(ctx.joined, ctx.sorted_topk_ids, ctx.aligned_expert_ids, ctx.aligned_num_tokens, ctx.BLOCK_M, ctx.full_num_tokens,
+                               b_nk.shape[0], b_nk.shape[1], K * a.element_size(), stream,
+                               gather=(workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * K * a.element_size(), status, status + 8))
+    if blocks is None:
+        return False
+    _group_gemm(workspace[:M], None, 0, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, M, 0, None, ctx.rank,
+                sk_workspace=ctx.sk_workspace, stream=ctx.group_gemm_stream)
     if stream != current:
         torch.cuda.current_stream().wait_stream(ctx.group_gemm_stream)
+    return True
 
 
 def _weight_nk(ctx, b):
@@ -321,11 +360,9 @@ def ag_group_gemm_intra_node(a, b, ctx=None, full_topk_ids=None, num_experts=Non
     out_dtype = a.dtype if a.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
     C = torch.empty([ctx.topk * M_per_rank * W, N_per_rank], dtype=out_dtype, device=a.device)
     b_nk = _weight_nk(ctx, b)
-    if (W > 1 and not ctx.held_ranks and a.is_contiguous() and (M_per_rank * K * a.element_size()) % 16 == 0 and
-            ctx.local_blocks is not None and ctx.local_blocks.stand_for(ctx.sorted_topk_ids, K * a.element_size())):
+    if W > 1 and ctx.gather_rows and not ctx.held_ranks and a.is_contiguous() and (M_per_rank * K * a.element_size()) % 16 == 0:
         shards = _lib.shard_table(a, ctx.peer_shards, rank, W)
-        if shards is not None:
-            _gather_and_multiply(a, b_nk, C, ctx, shards)
+        if shards is not None and _gather_and_multiply(a, b_nk, C, ctx, shards):
             return C
     workspace, barrier = ctx.workspace_tensors[rank], ctx.barrier_tensors[rank]
     current = torch.cuda.current_stream()

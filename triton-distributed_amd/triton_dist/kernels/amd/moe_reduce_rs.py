@@ -14,7 +14,7 @@ from typing import Dict, List, Optional
 import torch
 
 from triton_dist import _lib
-from triton_dist.kernels.amd.allgather_group_gemm import (LocalRowBlocks, group_gemm_gated, local_row_blocks,
+from triton_dist.kernels.amd.allgather_group_gemm import (_group_gemm, group_gemm_gated, joined_row_blocks,
                                                           sort_topk_ids_align_block_size)
 from triton_dist.kernels.amd.low_latency_all_to_all import moe_weighted_combine
 
@@ -50,7 +50,6 @@ class MoEAgScatterGroupGemmPrecomputeContext:
     TOP_K: int = 0
     BLOCK_M: int = 0
     num_tokens_per_rank: int = 0
-    local_blocks: Optional[LocalRowBlocks] = None   # the same rows in blocks without rank segments, for this GPU's GEMM
 
 
 def precompute_context_helper(pg, num_ranks, topk, num_tokens_per_rank, num_experts, input_dtype, device, router_logits,
@@ -81,6 +80,7 @@ class MoEReduceRSContext:
     weight_nk: Optional[torch.Tensor] = None
     weight_key: Optional[tuple] = None
     sk_workspace: Optional[torch.Tensor] = None   # the context's GEMM workspace; None = off
+    joined: dict = dataclasses.field(default_factory=dict)   # memory for the row blocks of a call, see joined_row_blocks
 
     def set_peer_partials(self, partials):
         """``partials``: dict rank -> [tokens_per_rank, hidden]: what rank r computed (over its share of the intermediate
@@ -106,7 +106,6 @@ def create_moe_rs_context(pg, local_rank, world_size, local_world_size, max_toke
     assert num_tokens_per_rank * world_size <= max_token_num and max_token_num % world_size == 0
     pre = precompute_context_helper(pg, world_size, topk, num_tokens_per_rank, num_experts, input_dtype, device,
                                     router_logits, BLOCK_M=moe_block_size, peer_router_logits=peer_router_logits, rank=rank)
-    pre.local_blocks = local_row_blocks(pre.full_topk_ids, num_experts, hidden_dim, pre.full_sorted_token_ids)
     M = num_tokens_per_rank * world_size
     rs_buffers: List[Optional[torch.Tensor]] = [None] * world_size
     rs_buffers[rank] = torch.zeros([max_token_num, hidden_dim], dtype=output_dtype, device=device)
@@ -140,13 +139,12 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     assert a.shape[0] == M * topk and a.dtype == b.dtype and a.shape[1] == b.shape[1]
     hidden = b.shape[2]
     out = ctx.final_output_buffer[:M * topk, :hidden]
-    blocks = pre.local_blocks
     # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local, and
     # blocks that run across the rank segments hold less padding
-    if blocks is not None and blocks.stand_for(pre.full_sorted_token_ids, a.shape[1] * a.element_size()):
-        group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, blocks.sorted_ids, blocks.expert_ids, blocks.segment_ids,
-                         blocks.num_tokens_post_padded, blocks.block_size, pre.full_numel, 1, M * topk, 0, None, rank,
-                         sk_workspace=ctx.sk_workspace)
+    blocks = joined_row_blocks(ctx.joined, pre.full_sorted_token_ids, pre.full_token_expert_ids, pre.full_num_tokens_post_padded_list, pre.BLOCK_M,
+                               pre.full_numel, b.shape[0], hidden, a.shape[1] * a.element_size(), _lib.stream_ptr())
+    if blocks is not None:
+        _group_gemm(a, None, 0, _weight_nk(ctx, b), out, blocks, pre.full_numel, 1, M * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
     else:
         group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
                          pre.block_wait_barriers, pre.full_num_tokens_post_padded_list, pre.BLOCK_M, pre.full_numel, 1,
