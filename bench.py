@@ -42,7 +42,7 @@ MEASURED_TRAFFIC_BYTES = {
 MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
     "decode.hip": "7741974f667a3d5e",
-    "gemm.hip": "f5e3c8dbadd4a963",
+    "gemm.hip": "e637df29a212e7ee",
     "moe.hip": "97f23dc5aa4ab792",
     "reduce.hip": "469689d34df1b205",
 }

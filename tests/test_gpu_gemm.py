@@ -838,3 +838,25 @@ def test_chunks_that_are_no_whole_tiles(cuda, world, mpc, rank):
     # a local shard that is no whole number of tiles cannot be handed in beside such chunks
     with pytest.raises(_lib.TdistError, match="local shard"):
         gated_gemm(a_d, a_d[rank * mpc:(rank + 1) * mpc], rank * mpc, b_d, c, flags, mpc, rank, world)
+
+
+# 5, 9, 13 and 17 row tiles by columns for which whole groups of 4 or 8 row tiles would take a round more (walked one, two or four
+# row tiles at a time), a single row tile, and one over 16
+@pytest.mark.parametrize("tile,M,N", [(0, 1280, 9472), (0, 2300, 7680), (1, 1280, 4736), (1, 3200, 2176), (4, 1152, 13696), (4, 2176, 7936), (3, 1664, 3648),
+                                      (2, 640, 4736), (0, 200, 16640), (4, 2100, 4000)])
+def test_walks_of_an_ungated_gemm(cuda, switches, tile, M, N):
+    from triton_dist import _lib
+    from triton_dist.kernels.amd import gated_gemm
+    announce("gemm walk tile %d %dx%d" % (tile, M, N))
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randint(-2, 3, (M, 192), generator=g).to(torch.bfloat16).to(cuda)
+    b = torch.randint(-2, 3, (N, 192), generator=g).to(torch.bfloat16).to(cuda)
+    want = (a.float() @ b.float().t()).to(torch.bfloat16)   # (|sums| <= 768: exact in fp32, rounded once)
+    switches(_lib.TDIST_DEBUG_GEMM_TILE, tile)
+    ws = _lib.new_split_k_workspace(cuda)
+    for split in (0, 1):
+        switches(_lib.TDIST_DEBUG_GEMM_SPLIT_K, split)
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+        gated_gemm(a, None, 0, b, c, None, 0, 0, 1, sk_workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(c, want), split

@@ -2,19 +2,18 @@
 import types
 
 import pytest
-import torch
 
 from triton_dist import _lib
 
 
-def shard(address, device="cuda:0"):
-    return types.SimpleNamespace(data_ptr=lambda: address, device=torch.device(device))
+def shard(address, device=0):
+    return types.SimpleNamespace(data_ptr=lambda: address, get_device=lambda: device)   # (-1: host memory)
 
 
 @pytest.mark.parametrize("peers,taken", [
     ({0: shard(0x2000), 2: shard(0x3000)}, True),
-    ({0: shard(0x2000), 2: shard(0x3000, "cuda:1")}, False),   # another GPU: the copies' business
-    ({0: shard(0x2000), 2: shard(0x3000, "cpu")}, False),
+    ({0: shard(0x2000), 2: shard(0x3000, 1)}, False),   # another GPU: the copies' business
+    ({0: shard(0x2000), 2: shard(0x3000, -1)}, False),
     ({0: shard(0x2000), 2: shard(0x3008)}, False),
     ({0: shard(0x2000)}, False),
 ])

@@ -26,6 +26,7 @@
 //    compact block of tiles so they share A rows and B rows in that XCD's L2.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <mutex>
 #include <utility>
 
@@ -1992,39 +1993,98 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.88}, {128, 128, 0.54}, {128, 192, 0.65}, {128, 256, 0.8}};
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
+  // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
+  // operand rows of rows + cols panels for it: the rows of such a block, a little more where a side does not
+  // divide the tile count (the blocks then wrap around the matrix's edge and their panels are shared by fewer tiles);
+  // 0 if the XCD's workgroups do not make whole rows.
+  const int per_xcd = di.num_xcds > 0 && cap_wgs % di.num_xcds == 0 ? cap_wgs / di.num_xcds : cap_wgs;
+  // (32-bit divisions, few of them: a call of a few microseconds waits for this choice)
+  auto xcd_block_cost = [&](int bm, int bn, int tiles_m, int tiles_n, int rows) -> double {
+    if (rows <= 0 || per_xcd % rows != 0) return 0;
+    const int cols = per_xcd / rows;
+    return ((double)rows * bm + (double)cols * bn) * (1.0 + (tiles_n % cols != 0 ? 0.125 : 0.0) + (tiles_m % rows != 0 ? 0.125 : 0.0));
+  };
+  // The walk over tile t's grid: rounds times what a K tile of a round takes, in the units below, with the last round split
+  // along K or whole; and for an ungated call the row tiles that are walked as a group. Such a call's last group is walked to
+  // its end whether there are row tiles or not, so that large groups may cost a round (1152 x 13696 x 7680 bf16, 9 row tiles of
+  // 128 by 54: 648 positions in groups of 4 or 8, three rounds, 345-376 us; 486 one by one, two rounds, 280; 212 on the 256 x 256
+  // tiles, which the estimate takes since it counts this); small groups make an XCD's block long and narrow: 3 % more at 2 x 16 tiles of 256 x 256 and 9 % at 1 x 32 than at 8 x 4 (16384 x 7168 x 8192 e4m3;
+  // 4 x 8 there, 28 column tiles, constant operands: 472 us against 455), and no round is faster than its panels come from the
+  // memory-side cache, 7.5 TB/s to all XCDs (128 x 256 tiles one row at a time: 1.2 us a K tile instead of 0.75).
+  struct Walk { double cost; int rows; };
+  auto walk = [&](int t, bool split_last) -> Walk {
+    const int bm = kChoices[t].bm, bn = kChoices[t].bn;
+    const int tiles_m = (c.M + bm - 1) / bm, tiles_n = (c.N + bn - 1) / bn;
+    const double per_k_tile = (double)bm * bn / kChoices[t].eff;
+    auto rounds = [&](int64_t positions) -> double {
+      const int64_t full = positions < 0x7fffffff ? (int)positions / cap_wgs : positions / cap_wgs, tail = positions - full * cap_wgs;
+      if (tail == 0 || !split_last) return (double)(full + (tail != 0));
+      const int64_t kt = ceil_div((int64_t)c.K * esz, k_tile_bytes(t));
+      return (double)full + 1.0 / sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff));
+    };
+    if (c.flags || c.scatter_bufs) return {rounds((int64_t)tiles_m * tiles_n) * per_k_tile, 0};
+    constexpr int kGroups[] = {4, 8, 2, 16, 1};
+    double panels[5], fewest = 0;
+    for (int i = 0; i < 5; ++i) {
+      panels[i] = xcd_block_cost(bm, bn, tiles_m, tiles_n, kGroups[i]);
+      if (panels[i] > 0 && (fewest == 0 || panels[i] < fewest)) fewest = panels[i];
+    }
+    Walk best = {0, 1};
+    for (int i = 0; i < 5; ++i) {
+      const int rows = kGroups[i];
+      if (panels[i] == 0) continue;
+      const double fetched = ((double)rows * bm + (double)(per_xcd / rows) * bn) * k_tile_bytes(t) * di.num_xcds;
+      const double k_tile = std::max(per_k_tile * (1.0 + 0.05 * (panels[i] / fewest - 1.0)), fetched / 7.5e6 / 1.2 * 65536.0);
+      const double cost = rounds((int64_t)((tiles_m + rows - 1) & -rows) * tiles_n) * k_tile;   // (rows: a power of two)
+      if (best.cost == 0 || cost < best.cost) best = {cost, rows};
+    }
+    return best;
+  };
   // With a workspace, a last round that fills at most half of the grid is split along K (see GemmParams): it then
   // costs 1/s of a round plus one exchange of the tile's accumulators, and that form is taken where it beats whole
   // tiles by a margin.
-  const int sk_mode = sk_env();
-  int pick = 2;
-  bool use_sk = false;
-  double best = 0;
+  const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
+  // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
+  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more (10 of them in its estimate already)
+  // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 21 us on 512 of 64 x 128; 200 x 1536 x 4096 bf16:
+  // 26 -> 16 us; 4096 x 1536 x 4096 stays on the large tiles, 45 us against 63). Most calls that take them are told by a
+  // bound that needs no walk (a microsecond of host time less): every tile's work at its rate, no hand-over, no last round.
+  const SmallPlan small = small_plan(c, esz, di.num_cus);
+  if (small.us > 0 && forced_tile < 0) {
+    double least = 0;
+    for (int t = 0; t < kNumChoices; ++t) {
+      const int bm = kChoices[t].bm, bn = kChoices[t].bn;
+      const double tiles = (double)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn), rounds = std::max(tiles / cap_wgs, 1.0 / kSkMaxSplit);
+      const double cost = rounds * bm * bn / kChoices[t].eff * c.K * esz / 128.0;
+      if (admissible(t) && (least == 0 || cost < least)) least = cost;
+    }
+    if (small.us < 0.95 * (8.0 + least / 65536.0 * 1.2)) return run_small(c, elem, esz, small, di);
+  }
+  int pick = 2, pick_split = -1;
+  double whole = 0, split_last = 0;
   for (int t = 0; t < kNumChoices; ++t) {
     if (!admissible(t)) continue;
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int64_t tiles = ceil_div(c.M, bm) * ceil_div(c.N, bn);
     const int64_t kt = ceil_div((int64_t)c.K * esz, k_tile_bytes(t));
-    const double per_k_tile = (double)bm * bn / kChoices[t].eff;
-    const double cost = (double)ceil_div(tiles, cap_wgs) * kt * per_k_tile;
-    if (best == 0 || cost < best) best = cost, pick = t, use_sk = false;
+    const double cost = walk(t, false).cost * kt;
+    if (whole == 0 || cost < whole) whole = cost, pick = t;
     const int64_t tail = tiles % cap_wgs;
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
       // (and 10 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
-      const double cost_sk = ((double)(tiles / cap_wgs) * kt + (double)kt / split + sk_handover_k_tiles(bm, bn)) * per_k_tile +
-                             10.0 / 1.2 * 65536.0;
-      if (cost_sk < 0.95 * best || (sk_mode == 1 && (!use_sk || cost_sk < best))) best = cost_sk, pick = t, use_sk = true;
+      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / kChoices[t].eff) + 10.0 / 1.2 * 65536.0;
+      if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
   }
-  // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
-  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more (10 of them in its estimate already)
-  // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 21 us on 512 of 64 x 128; 200 x 1536 x 4096 bf16:
-  // 26 -> 16 us; 4096 x 1536 x 4096 stays on the large tiles, 45 us against 63).
-  if (const SmallPlan plan = small_plan(c, esz, di.num_cus); plan.us > 0) {
-    const int forced = debug_get(TDIST_DEBUG_GEMM_TILE);
+  // (the margin lies between whole tiles and a split round, not between two tiles' split rounds)
+  bool use_sk = pick_split >= 0 && (sk_mode == 1 || split_last < 0.95 * whole);
+  if (use_sk) pick = pick_split;
+  const double best = use_sk ? split_last : whole;
+  if (small.us > 0) {
     const double large_us = 8.0 + best / 65536.0 * 1.2 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 15.0 : 0.0);
-    if (forced >= kNumLargeTiles || (forced < 0 && plan.us < 0.95 * large_us)) return run_small(c, elem, esz, plan, di);
+    if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < 0.95 * large_us)) return run_small(c, elem, esz, small, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,
   // 4 = 128x256; a tile that the call's row blocks or K do not admit is not taken.
@@ -2042,18 +2102,6 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   }
   const int BM = kChoices[pick].bm;
   const int BN = kChoices[pick].bn;
-  // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
-  // operand rows of rows + cols panels for it: the bytes of such a block per tile, a little more where a side does not
-  // divide the tile count (the blocks then wrap around the matrix's edge and their panels are shared by fewer tiles);
-  // 0 if the XCD's workgroups do not make whole rows.
-  auto xcd_block_cost = [&](int rows) -> double {
-    const int per_xcd = di.num_xcds > 0 && cap_wgs % di.num_xcds == 0 ? cap_wgs / di.num_xcds : cap_wgs;
-    if (rows <= 0 || per_xcd % rows != 0) return 0;
-    const int cols = per_xcd / rows;
-    const int tiles_m = (int)ceil_div(c.M, BM), tiles_n = (int)ceil_div(c.N, BN);
-    return ((double)rows * BM + (double)cols * BN) * (1.0 + (tiles_n % cols != 0 ? 0.125 : 0.0) + (tiles_m % rows != 0 ? 0.125 : 0.0));
-  };
-
   GemmParams p;
   p.A = (const unsigned char*)c.A;
   p.A_local = (const unsigned char*)c.A_local;
@@ -2136,7 +2184,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       double best = 0;
       for (int cand = 1; cand * cmh <= 16; cand *= 2) {
         if (p.n_chunks % cand != 0 || (cand > 1 && p.order_mode == 1 && c.world_size % cand != 0)) continue;
-        const double cost = xcd_block_cost(cand * cmh);
+        const double cost = xcd_block_cost(BM, BN, (int)ceil_div(c.M, BM), (int)ceil_div(c.N, BN), cand * cmh);
         if (cost > 0 && (best == 0 || cost < best)) {
           best = cost;
           gs = cand;
@@ -2150,19 +2198,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       }
     }
   } else {
-    // ungated GEMM: scheduled in groups of row tiles, of the size that gives an XCD's block of tiles its best shape
-    // (16384 x 7168 x 8192 e4m3, 28 column tiles, constant operands: 472 us in blocks of 4 x 8, 455 in blocks of 8 x 4)
-    int rows_per_group = 4;
-    {
-      double best = 0;
-      for (int rows : {4, 8, 2, 16}) {
-        const double cost = xcd_block_cost(rows);
-        if (cost > 0 && (best == 0 || cost < best)) {
-          best = cost;
-          rows_per_group = rows;
-        }
-      }
-    }
+    // ungated GEMM: scheduled in groups of row tiles (see walk)
+    const int rows_per_group = walk(pick, use_sk).rows;
     p.m_per_chunk = BM * rows_per_group;
     p.n_chunks = (int)ceil_div(c.M, p.m_per_chunk);
     p.order_mode = 0;

@@ -180,10 +180,10 @@ def shard_table(own, peer_shards, rank, num_ranks):
     take any device and any address."""
     if num_ranks > GATHER_MAX_RANKS or own.data_ptr() % 16 != 0:
         return None
-    table = (ctypes.c_void_p * num_ranks)()
+    table, device = (ctypes.c_void_p * num_ranks)(), own.get_device()
     for r in range(num_ranks):
         t = own if r == rank else peer_shards.get(r)
-        if t is None or t.device != own.device or t.data_ptr() % 16 != 0:
+        if t is None or t.get_device() != device or t.data_ptr() % 16 != 0:
             return None
         table[r] = t.data_ptr()
     return table
