@@ -155,3 +155,13 @@ def test_ops_fail_loudly_without_gpu():
         create_gemm_rs_intra_node_context(1024, 256, torch.bfloat16, 0, 8, None)
     with pytest.raises(RuntimeError):
         moe_dispatch_preprocess(torch.zeros((4, 2), dtype=torch.int32), 8)
+
+
+@pytest.mark.parametrize("entry", ["gqa_fwd_batch_decode", "gqa_fwd_batch_decode_persistent", "gqa_fwd_batch_decode_intra_rank"])
+def test_decode_refuses_what_is_no_number_of_splits(entry):
+    """Also where the launch divides the keys itself and the number changes nothing; looked at before the tensors are."""
+    from triton_dist.kernels.amd import flash_decode
+    for kv_split, code in ((0, _lib.TDIST_ERR_INVALID), (-2, _lib.TDIST_ERR_INVALID), (65536, _lib.TDIST_ERR_UNSUPPORTED)):
+        with pytest.raises(_lib.TdistError) as e:
+            getattr(flash_decode, entry)(None, None, None, None, None, None, None, 1.0, kv_split=kv_split)
+        assert e.value.code == code

@@ -25,6 +25,12 @@ def head_dims_supported(dk, dv):
     return (dk, dv) in SUPPORTED_HEAD_DIMS or (dk == dv and 0 < dk <= 256 and dk % 8 == 0)
 
 
+def _check_kv_split(kv_split):
+    """A number of splits, or -1 for the library's choice; refused otherwise, also where the number changes nothing."""
+    if kv_split != -1 and not 1 <= kv_split <= 65535:
+        raise _lib.TdistError(_lib.TDIST_ERR_INVALID if kv_split < 1 else _lib.TDIST_ERR_UNSUPPORTED, "kv_split %d" % kv_split)
+
+
 def _check_inputs(q, k_cache, v_cache, kv_lens, block_table):
     _lib.require_cuda(q, k_cache, v_cache, kv_lens, block_table)
     batch, q_heads, q_head_dim = q.shape
@@ -169,6 +175,7 @@ def gqa_fwd_batch_decode(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_
     lengths (``kv_split``, the reference's fixed number of splits per sequence, is accepted for its signature and
     changes nothing in the result). Returns ``output_combine`` [B,Hq,Dv] (default dtype: q's; the reference hard-codes
     float16, :784)."""
+    _check_kv_split(kv_split)
     if output_combine is None:
         output_combine = torch.empty((q.shape[0], q.shape[1], v_cache.shape[-1]), dtype=q.dtype, device=q.device)
     return decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, output_combine)
@@ -183,6 +190,7 @@ def gqa_fwd_batch_decode_persistent(q, k_cache, v_cache, workspace, q_lens, kv_l
     else uses it, and a counter that does not start at zero makes a merge fire early or never, so the arrival counters
     are the library's own (_lib.zeros_per_stream). ``output_split`` is ignored
     (partials are fp32 internally)."""
+    _check_kv_split(kv_split)
     batch, q_heads, _ = q.shape
     if output_combine is None:
         output_combine = torch.empty((batch, q_heads, v_cache.shape[-1]), dtype=q.dtype, device=q.device)
@@ -199,6 +207,7 @@ def gqa_fwd_batch_decode_intra_rank(q, k_cache, v_cache, workspace, q_lens, kv_l
     passes a buffer of another dtype (the reference uses q's dtype). With ``return_lse`` also returns the
     fp32 (out [B,Hq,Dv], lse [B,Hq]) pair the merge produced. ``workspace`` and ``q_lens`` are accepted and unused, as
     in the reference; ``counters`` (keyword only in spirit: an addition) likewise, if it is what _check_counters asks for."""
+    _check_kv_split(kv_split)
     batch, q_heads, _ = q.shape
     dv = v_cache.shape[-1]
     if output_combine is None:
