@@ -81,14 +81,31 @@ def run_ag_gemm(cuda, shards, b, rank, m_per_chunk, **ctx_kw):
     return ctx
 
 
-def test_ag_gemm_config1(cuda):
-    """4 chunks of [1024, 4096] bf16, B [1536, 4096], flags released by the copy streams."""
+def copies_and_flags(ctx, rank, world, chunks=1):
+    """Has the peers' rows come as chunk copies that release flags, in the default order of the copy producer (without an
+    order of its own, a context whose rows are at hand takes the gather in front of an ungated product)."""
+    ctx.arrival_order = [((rank + i) % world, c) for i in range(1, world) for c in range(chunks)]
+    return ctx
+
+
+@pytest.fixture
+def no_gather(monkeypatch):
+    """Called in a leg that is about the flags: the gather fails the test if it is taken."""
+    from triton_dist.kernels.amd import all_gather_gemm
+    return lambda: monkeypatch.setattr(all_gather_gemm, "_gather_and_multiply", lambda *_: pytest.fail("took the gather"))
+
+
+def test_ag_gemm_config1(cuda, no_gather):
+    """4 chunks of [1024, 4096] bf16, B [1536, 4096], the rows gathered, then flags released by the copy
+    streams."""
     from triton_dist.kernels.amd import ag_gemm_intra_node
     announce("ag_gemm C1")
     shards, b = make_ag_case(4, 1024, 4096, 1536, torch.bfloat16, seed=3 + 0)
     ref = golden.ag_gemm_fp32(shards, b)
     gold = golden.torch_ag_gemm(shards, b)
-    for rank, order in [(0, None), (2, [(3, 0), (1, 0), (0, 0)])]:
+    for rank, order in [(0, None), (0, [(1, 0), (2, 0), (3, 0)]), (2, [(3, 0), (1, 0), (0, 0)])]:
+        if order is not None:
+            no_gather()
         ctx = run_ag_gemm(cuda, shards, b, rank, 1024, arrival_order=order)
         for it in range(2):   # flags are reset between calls
             c = ag_gemm_intra_node(shards[rank].to(cuda), b.to(cuda), False, ctx)
@@ -439,10 +456,12 @@ def test_gemm_rs_config2_full_size(cuda):
     assert torch.allclose(out.float().cpu(), ref, rtol=2.0**-6, atol=2e-3 * float(ref.abs().max()))
 
 
-def test_fp8_ag_gemm_config3_full_size(cuda):
-    """8 chunks of [2048, 8192] e4m3, B [7168, 8192] e4m3, per-row and per-column fp32 scales."""
+@pytest.mark.parametrize("gathered", [True, False])
+def test_fp8_ag_gemm_config3_full_size(cuda, no_gather, gathered):
+    """8 chunks of [2048, 8192] e4m3, B [7168, 8192] e4m3, per-row and per-column fp32 scales. With the
+    rows gathered and with chunk copies that release flags."""
     from triton_dist.kernels.amd import ag_gemm_intra_node
-    announce("fp8 ag_gemm C3 full size")
+    announce("fp8 ag_gemm C3 full size, gathered %s" % gathered)
     world, rank, m_per_rank, K, N = 8, 0, 2048, 8192, 7168
     g = torch.Generator().manual_seed(3 + 2)
     shards = [torch.randn((m_per_rank, K), generator=g).to(torch.float8_e4m3fn) for _ in range(world)]
@@ -450,6 +469,9 @@ def test_fp8_ag_gemm_config3_full_size(cuda):
     sa = torch.rand(world * m_per_rank, generator=g) * 0.09 + 0.01
     sb = torch.rand(N, generator=g) * 0.009 + 0.001
     ctx = run_ag_gemm(cuda, shards, b, rank, 2048)
+    if not gathered:
+        copies_and_flags(ctx, rank, world)
+        no_gather()
     c = ag_gemm_intra_node(shards[rank].to(cuda), b.to(cuda), False, ctx, row_scale=sa.to(cuda), col_scale=sb.to(cuda))
     ctx.check_status()
     assert c.shape == (16384, 7168) and c.dtype == torch.bfloat16
@@ -624,11 +646,11 @@ def test_paced_arrivals_hold_the_chunks_back(cuda):
     assert start.elapsed_time(stop) < 200
 
 
-@pytest.mark.parametrize("producer_kernel,link_gbps", [(False, 0.0), (True, 0.0), (True, 50.0)])
-def test_ag_gemm_kernel_producer_and_graph_replay(cuda, producer_kernel, link_gbps):
+@pytest.mark.parametrize("producer_kernel,link_gbps", [(False, 0.0), (True, 0.0), (True, 50.0), (None, 0.0)])
+def test_ag_gemm_kernel_producer_and_graph_replay(cuda, no_gather, producer_kernel, link_gbps):
     """The whole op (producer on its stream, gated GEMM, flag reset) captured into a HIP graph and replayed three
     times with eager work in between: every replay must reproduce the eager result from a poisoned workspace. Runs
-    with the copy producer and with the one-launch kernel producer (unpaced and paced)."""
+    with the copy producer, with the one-launch kernel producer (unpaced and paced) and, for None, with the gather."""
     from triton_dist.kernels.amd import ag_gemm_intra_node, create_ag_gemm_intra_node_context
     announce("ag-gemm graph replay, kernel producer %s, link %s" % (producer_kernel, link_gbps))
     world, rank, mpr, K, N = 4, 2, 512, 1024, 640
@@ -638,7 +660,11 @@ def test_ag_gemm_kernel_producer_and_graph_replay(cuda, producer_kernel, link_gb
                                             M_PER_CHUNK=256, gemm_stream=torch.cuda.Stream(),
                                             ag_streams=[torch.cuda.Stream(), torch.cuda.Stream()])
     ctx.set_peer_shards({r: s.to(cuda) for r, s in enumerate(shards) if r != rank})
-    ctx.producer_kernel, ctx.link_gbps = producer_kernel, link_gbps
+    ctx.producer_kernel, ctx.link_gbps = bool(producer_kernel), link_gbps
+    if producer_kernel is False:
+        copies_and_flags(ctx, rank, world, chunks=2)
+    if producer_kernel is not None:
+        no_gather()
     a_d, b_d = shards[rank].to(cuda), b.to(cuda)
     want = ag_gemm_intra_node(a_d, b_d, False, ctx).clone()
     ctx.check_status()
@@ -712,7 +738,7 @@ def test_for_correctness_context_delays_its_producer(cuda):
 
 
 @pytest.mark.parametrize("m_per,K", [(256, 256), (200, 320), (72, 96)])
-def test_nvidia_side_signatures(cuda, m_per, K):
+def test_nvidia_side_signatures(cuda, no_gather, m_per, K):
     """The NVIDIA-side entry points of the reference (kernels/nvidia/allgather_gemm.py:785-882,
     gemm_reduce_scatter.py:77-88, 468-538): context from the local tensors, one flag per rank segment, M_per_rank padded
     to BLOCK_M for the reduce-scatter."""
@@ -737,7 +763,10 @@ def test_nvidia_side_signatures(cuda, m_per, K):
     actx = create_ag_gemm_intra_node_context(shards[rank].to(cuda), bb.to(cuda), rank, W)
     assert actx.barrier_tensors[rank].numel() == W and actx.M_PER_CHUNK == m_per
     actx.set_peer_shards({r: s.to(cuda) for r, s in enumerate(shards) if r != rank})
-    for _ in range(2):   # (the second call finds the flags reset by the first)
+    for call in range(3):   # the gather, then the flags twice (the second time they are the ones that the first reset)
+        if call == 1:
+            copies_and_flags(actx, rank, W)
+            no_gather()
         actx.workspace_tensors[rank].view(torch.uint8).fill_(0x7B)
         c = ag_gemm_intra_node(shards[rank].to(cuda), bb.to(cuda), actx)
         actx.check_status()

@@ -37,9 +37,19 @@ def run(cuda, shards, w, ids, rank, E, block, **ctx_kw):
     return ctx, c
 
 
+@pytest.fixture(params=["gathered", "flags"])
+def rows(request, monkeypatch):
+    """How the ranks' rows come: gathered in front of joined row blocks, or as copies that release the flag of each rank's
+    blocks. Gives the context's switch; the flags' leg fails if it takes the gather."""
+    if request.param == "flags":
+        from triton_dist.kernels.amd import allgather_group_gemm
+        monkeypatch.setattr(allgather_group_gemm, "_gather_and_multiply", lambda *_: pytest.fail("took the gather"))
+    return {"gather_rows": request.param == "gathered"}
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("block,K", [(128, 256), (256, 512), (128, 96)])
-def test_exact_on_integer_inputs(cuda, dtype, block, K):
+def test_exact_on_integer_inputs(cuda, rows, dtype, block, K):
     """Integer-valued tokens and weights: the fp32 sums are exact, only the final rounding remains. K = 96 elements of
     16 bits is an odd number of 64-byte halves and takes the 128 x 128 tile."""
     if dtype == torch.float8_e4m3fn:
@@ -48,18 +58,18 @@ def test_exact_on_integer_inputs(cuda, dtype, block, K):
     announce("group gemm exact %s block %d K %d" % (dtype, block, K))
     shards, w, ids = make_case(world, mpr, K, N, E, topk, dtype, seed=block + K, integer=True)
     for rank in (0, 3):
-        ctx, c = run(cuda, shards, w, ids, rank, E, block)
+        ctx, c = run(cuda, shards, w, ids, rank, E, block, **rows)
         ctx.check_status()
         ref = golden.ag_group_gemm_fp32(shards, w, ids)
         assert torch.equal(c.float().cpu(), ref.to(c.dtype).float()), "rank %d" % rank
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_random_inputs_and_the_reference_golden(cuda, dtype):
+def test_random_inputs_and_the_reference_golden(cuda, rows, dtype):
     world, mpr, K, N, E, topk = 8, 256, 1024, 768, 16, 4
     announce("group gemm random %s" % dtype)
     shards, w, ids = make_case(world, mpr, K, N, E, topk, dtype, seed=5)
-    ctx, c = run(cuda, shards, w, ids, 2, E, 128)
+    ctx, c = run(cuda, shards, w, ids, 2, E, 128, **rows)
     ctx.check_status()
     ref = golden.ag_group_gemm_fp32(shards, w, ids)
     assert golden.max_rel_err(c.float().cpu(), ref) <= 1e-2
@@ -79,7 +89,7 @@ def run_again(cuda, ctx, shards, w, rank):
     return c
 
 
-def test_skewed_routing_and_unused_experts(cuda):
+def test_skewed_routing_and_unused_experts(cuda, rows):
     """All tokens of one rank go to one expert, some experts get nothing, topk = 1: blocks of very different counts
     per segment, and segments with a single block."""
     world, mpr, K, N, E = 4, 200, 256, 256, 8
@@ -89,7 +99,7 @@ def test_skewed_routing_and_unused_experts(cuda):
     w = torch.randint(-2, 3, (E, K, N), generator=g).float().bfloat16()
     ids = torch.cat([torch.full((mpr, 1), 7), torch.randint(0, 2, (mpr, 1), generator=g), torch.full((mpr, 1), 3),
                      torch.randint(4, 6, (mpr, 1), generator=g)]).long()
-    ctx, c = run(cuda, shards, w, ids, 1, E, 128)
+    ctx, c = run(cuda, shards, w, ids, 1, E, 128, **rows)
     ctx.check_status()
     assert torch.equal(c.float().cpu(), golden.ag_group_gemm_fp32(shards, w, ids).bfloat16().float())
 
