@@ -33,16 +33,23 @@ PEAK = {"bf16": 2.5e15, "fp8": 5.0e15, "hbm": 8.0e12}  # MI355X published dense 
 # the summaries are kept under profiles/. Each figure names the kernel sources it was measured on, and
 # MEASURED_SOURCE_DIGEST holds those sources' digests at the time: a figure whose sources have changed since is
 # reported as null, not as a measurement (tests/test_bench_constants.py fails until it is measured again).
+GEMM_SOURCES = ("gemm.hip", "gemm_small.hip", "gemm_small.h", "common.h")   # (the small tiles take part in the choice of a tile)
 MEASURED_TRAFFIC_BYTES = {
-    "c2_gemm": (840.0e6, ("gemm.hip", "common.h")), "c2_reduce": (151.0e6, ("reduce.hip", "common.h")),
-    "c1_gemm": (130.4e6, ("gemm.hip", "common.h")), "c3_gemm": (1646.0e6, ("gemm.hip", "common.h")),
+    "c2_gemm": (840.0e6, GEMM_SOURCES), "c2_reduce": (151.0e6, ("reduce.hip", "common.h")),
+    "c1_gemm": (130.4e6, GEMM_SOURCES), "c3_gemm": (1646.0e6, GEMM_SOURCES),
+    "c3_gather": (268.4e6, ("lib.hip", "gather.h", "common.h")),
     "c4_dispatch": (265.8e6, ("moe.hip", "common.h")), "c4_dispatch_from_ids": (267.4e6, ("moe.hip", "common.h")),
     "c4_combine": (296.7e6, ("moe.hip", "common.h")), "c5_split_kv": (4318.1e6, ("decode.hip", "common.h")),
+    "c5_stream": (4302.1e6, ("decode.hip", "common.h")),
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "29a71d5d51010d68",
     "decode.hip": "7741974f667a3d5e",
+    "gather.h": "efd413b797d8716f",
     "gemm.hip": "e637df29a212e7ee",
+    "gemm_small.h": "6e8a49fb30ce162c",
+    "gemm_small.hip": "bbc3652da8a55a10",
+    "lib.hip": "f0a1cb9af6a3eaba",
     "moe.hip": "97f23dc5aa4ab792",
     "reduce.hip": "469689d34df1b205",
 }
@@ -113,12 +120,27 @@ def time_launches(fn, steps, warmup):
 
 def time_live_ag_gemm(call, ctx, steps, warmup):
     """Times the AG-GEMM with its producer running, in the reference's order (producer queued first, then the gated
-    GEMM); a bounded flag wait that expired is an error. Returns (seconds, order)."""
+    GEMM): the context's kernel producer, or chunk copies that release flags, which an explicit arrival order asks for
+    (the default one: peers rank + 1, rank + 2, ..., chunks in order); a bounded flag wait that expired is an error.
+    Returns (seconds, order)."""
+    if not ctx.producer_kernel:
+        chunks = ctx.barrier_tensors[ctx.rank].numel() // ctx.num_ranks
+        ctx.arrival_order = [((ctx.rank + i) % ctx.num_ranks, c) for i in range(1, ctx.num_ranks) for c in range(chunks)]
     call()
     ctx.check_status()
     s = time_launches(call, steps, warmup)
     ctx.check_status()
+    ctx.arrival_order = None
     return s, "copies_first"
+
+
+def rows_gathered(call, ctx, steps, warmup, traffic=None):
+    """The same call in a context that asks for no arrivals: every peer's shard is at hand, so one launch gathers the rows
+    and the product runs ungated behind it. ``traffic``: the measured HBM-side bytes of the gather launch."""
+    call()
+    s = time_launches(call, steps, warmup)
+    ctx.check_status()
+    return dict({"us": round(s * 1e6, 2)}, **({} if traffic is None else {"gather_traffic": traffic}))
 
 
 XGMI_LINK_GBPS = 153.0   # one xGMI link of MI355X: the rate at which one peer's rows arrive
@@ -276,9 +298,10 @@ def bench_c1(dev, steps, warmup):
     ctx.set_peer_shards({r: s.to(dev) for r, s in enumerate(shards) if r != rank})
     a_d, b_d = shards[rank].to(dev), b.to(dev)
     flops = 2.0 * world * mpr * N * K
-    live_s, live_order = None, None
+    live_s, live_order, at_hand = None, None, None
     if LIVE_PRODUCER:
         live_s, live_order = time_live_ag_gemm(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx), ctx, steps, warmup)
+        at_hand = rows_gathered(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx), ctx, steps, warmup)
         c = ag_gemm_intra_node(a_d, b_d, False, ctx)
         ctx.check_status()
         err = golden.max_rel_err(c.float().cpu(), golden.ag_gemm_fp32(shards, b))
@@ -294,6 +317,7 @@ def bench_c1(dev, steps, warmup):
                          "sample": "the whole config once (torch golden: cat + matmul), %.2f s" % cs}
     r["with_live_producer_us"] = round(live_s * 1e6, 2) if live_s is not None else None
     r["live_producer_order"] = live_order
+    r["rows_gathered"] = at_hand
     if LIVE_PRODUCER:
         r["paced_xgmi_%dGBps" % XGMI_LINK_GBPS] = paced_ag_gemm(
             lambda c: (lambda: ag_gemm_intra_node(a_d, b_d, False, c)), world, rank, mpr, N, K, torch.bfloat16,
@@ -316,10 +340,12 @@ def bench_c3(dev, steps, warmup):
     ctx.set_peer_shards({r: s.to(dev) for r, s in enumerate(shards) if r != rank})
     a_d, b_d = shards[rank].to(dev), b.to(dev)
     flops = 2.0 * world * mpr * N * K
-    live_s, live_order = None, None
+    live_s, live_order, at_hand = None, None, None
     if LIVE_PRODUCER:
         live_s, live_order = time_live_ag_gemm(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb),
                                                ctx, steps, warmup)
+        at_hand = rows_gathered(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb), ctx, steps,
+                                warmup, measured_traffic("c3_gather"))
         c = ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb)
         ctx.check_status()
         rows = slice(5 * mpr + 11, 5 * mpr + 75)
@@ -339,6 +365,7 @@ def bench_c3(dev, steps, warmup):
                          "sample": "1024 of the 16384 rows (fp32 up-cast golden with scales), %.2f s" % cs}
     r["with_live_producer_us"] = round(live_s * 1e6, 2) if live_s is not None else None
     r["live_producer_order"] = live_order
+    r["rows_gathered"] = at_hand
     if LIVE_PRODUCER:
         r["paced_xgmi_%dGBps" % XGMI_LINK_GBPS] = paced_ag_gemm(
             lambda c: (lambda: ag_gemm_intra_node(a_d, b_d, False, c, row_scale=sa, col_scale=sb)), world, rank, mpr, N, K,
@@ -456,6 +483,14 @@ def bench_c5(dev, steps, warmup):
     final = torch.empty((B, Hq, D), dtype=torch.bfloat16, device=dev)
     rank_s = time_launches(lambda: gqa_fwd_batch_decode_inter_rank_combine(all_out, all_lse, all_lens, final), steps, warmup)
     kv_bytes = 2 * B * L * Hkv * D * 2
+    # what the entry points launch: the keys of the whole batch in equal ranges, then the merge of the ranges
+    from triton_dist.kernels.amd import gqa_fwd_batch_decode
+    entry_out = torch.empty_like(merged)
+    entry_s = time_launches(lambda: gqa_fwd_batch_decode(q, k, v, None, None, lens, table, scale, output_combine=entry_out),
+                            steps, warmup)
+    if float((entry_out.float() - merged.float()).abs().max()) > 2.0**-8 * float(merged.float().abs().max()):
+        raise RuntimeError("the entry point's decode differs from split + combine")
+    entry_bytes = kv_bytes + q.numel() * 2 + table.numel() * 4 + merged.numel() * 2
     split_bytes = kv_bytes + q.numel() * 2 + table.numel() * 4 + out_split.numel() * 4 + lse_split.numel() * 4
     r = roof("hbm", split_bytes, split_s, "hbm", measured_traffic("c5_split_kv"))
     from oracle import golden
@@ -467,6 +502,8 @@ def bench_c5(dev, steps, warmup):
                          "sample": "one of the 32 sequences (torch golden ref_paged_attn, 32768 keys), %.2f s" % cs}
     r["combine_us"] = round(comb_s * 1e6, 2)
     r["split_then_combine_us"] = round(both_s * 1e6, 2)
+    r["entry_point"] = {"us": round(entry_s * 1e6, 2), "achieved_GBps": round(entry_bytes / entry_s / 1e9, 1),
+                        "frac": round(entry_bytes / entry_s / PEAK["hbm"], 4), "traffic": measured_traffic("c5_stream")}
     r["fused_split_and_combine_us"] = round(fused_s * 1e6, 2)
     r["inter_rank_combine_us"] = round(rank_s * 1e6, 2)
     # the reference layer's defaults (layers/nvidia/sp_flash_decode_layer.py:45,61): 32 splits, and pages of one token
@@ -507,8 +544,10 @@ def bench_group_gemm(dev, steps, warmup):
                                                   num_ranks=world)
     ctx.set_peer_shards({r: s.to(dev) for r, s in enumerate(shards) if r != rank})
     flops = 2.0 * world * mpr * topk * K * N
-    live_s = None
+    live_s, at_hand = None, None
     if LIVE_PRODUCER:
+        at_hand = rows_gathered(lambda: ag_group_gemm_intra_node(a_d, w, ctx), ctx, steps, warmup)
+        ctx.gather_rows = False   # rank segments that arrive one by one: copies that release flags, the GEMM gated by them
         c = ag_group_gemm_intra_node(a_d, w, ctx)
         ctx.check_status()
         rows = torch.arange(5 * mpr * topk + 3, 5 * mpr * topk + 67)
@@ -526,6 +565,7 @@ def bench_group_gemm(dev, steps, warmup):
     r = roof("mfma", flops, pre_s, "bf16")
     r["workload"] = "8192 tokens x top-2 of 8 experts, K 14336, N 512 per rank, row blocks of 128 (128 x 256 tiles)"
     r["with_live_producer_us"] = round(live_s * 1e6, 2) if live_s is not None else None
+    r["rows_gathered"] = at_hand
     return r
 
 
