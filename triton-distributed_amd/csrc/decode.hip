@@ -1380,9 +1380,9 @@ static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
 // whatever the lengths are. A sequence that lies in one range is finished by its wave; one that is spread over several
 // leaves partial results (at most two per range), which the next launch merges (decode_stream_merge_kernel).
 // What bounds it: the K/V stream from HBM (B 32, 64 / 8 heads, 32768 keys: 650 us, 6.6 TB/s), and for little work the
-// chain lens -> table -> rows -> merge (B 1, 32 / 8 heads, 64 keys: 9 us). Against 32 splits per sequence, a combine launch
-// and the form for even lengths behind which the other one was queued, whole calls: 48 sequences of 128 to 8192 keys, f16,
-// 64 / 8 heads 205 -> 85 us; B 32 x 32768 715 -> 652 us. Eight waves of two stages: the same where the stream is long,
+// chain lens -> table -> rows -> merge. Against 32 splits per sequence, a combine launch and the form for even lengths behind
+// which the other one was queued, whole calls: 48 sequences of 128 to 8192 keys, f16, 64 / 8 heads 205 -> 72-76 us; B 32 x
+// 32768 712 -> 661 us (merge with 7 other ranks' partials included). Eight waves of two stages: the same where the stream is long,
 // 15 % behind where it is short (B 64 x 256 keys).
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kPadded>
 __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodeParams prm) {
@@ -1395,8 +1395,9 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodePara
 // a block of 16 query heads over one range, its pairs of waves every fourth block of keys, merged through the LDS where a
 // sequence ends; only the key rows are fetched, and the head blocks of a range run on one XCD, whose L2 then fetches them once.
 // What bounds it: LDS reads of the operands (53 KB per block and wave pair; the scores are worked out in both waves of a
-// pair) and, at a few blocks per stream, the fixed work at a segment's ends. B 16, 128 / 1 heads, 64 to 4096 keys: 388 us
-// with 32 splits and their combine (eight head blocks fetching both row sets, 134 MB of partial results) -> 66 us.
+// pair) and, at a few blocks per stream, the fixed work at a segment's ends. B 16, 128 / 1 heads, 64 to 4096 keys: 387 us
+// with 32 splits and their combine (eight head blocks fetching both row sets, 134 MB of partial results) -> 58-63 us, of
+// which 49 are this kernel (its matrix cores busy 7 % of the time, 28 % of the LDS cycles lost to bank conflicts) and 15 the merge.
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
 __global__ __launch_bounds__(NW * 64) void decode_stream_group_kernel(const DecodeParams prm) {
   decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, false, false, false, false, true>(prm);

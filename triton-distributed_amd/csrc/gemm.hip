@@ -2008,9 +2008,11 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // along K or whole; and for an ungated call the row tiles that are walked as a group. Such a call's last group is walked to
   // its end whether there are row tiles or not, so that large groups may cost a round (1152 x 13696 x 7680 bf16, 9 row tiles of
   // 128 by 54: 648 positions in groups of 4 or 8, three rounds, 345-376 us; 486 one by one, two rounds, 280; 212 on the 256 x 256
-  // tiles, which the estimate takes since it counts this); small groups make an XCD's block long and narrow: 3 % more at 2 x 16 tiles of 256 x 256 and 9 % at 1 x 32 than at 8 x 4 (16384 x 7168 x 8192 e4m3;
-  // 4 x 8 there, 28 column tiles, constant operands: 472 us against 455), and no round is faster than its panels come from the
-  // memory-side cache, 7.5 TB/s to all XCDs (128 x 256 tiles one row at a time: 1.2 us a K tile instead of 0.75).
+  // tiles, which the estimate takes since it counts this; 1536 x 4480 x 14848 bf16 286 -> 157 us for the same reason); small
+  // groups make an XCD's block long and narrow: 3 % more at 2 x 16 tiles of 256 x 256 and 9 % at 1 x 32 than at 8 x 4
+  // (16384 x 7168 x 8192 e4m3; 4 x 8 there, 28 column tiles, constant operands: 472 us against 455), and no round is faster
+  // than its panels come from the memory-side cache, 7.5 TB/s to all XCDs (128 x 256 tiles one row at a time: 1.2 us a K tile
+  // instead of 0.75). Over 300 shapes the tile and walk taken are 1 % from the best ones on average, 4 % before.
   struct Walk { double cost; int rows; };
   auto walk = [&](int t, bool split_last) -> Walk {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
@@ -2045,7 +2047,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // tiles by a margin.
   const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
   // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
-  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more (10 of them in its estimate already)
+  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more
+  // (10 of them in its estimate already)
   // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 21 us on 512 of 64 x 128; 200 x 1536 x 4096 bf16:
   // 26 -> 16 us; 4096 x 1536 x 4096 stays on the large tiles, 45 us against 63). Most calls that take them are told by a
   // bound that needs no walk (a microsecond of host time less): every tile's work at its rate, no hand-over, no last round.

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(24))) void prod
 
 // All ranks' rows into the workspace at once, the own ones among them: what a call does whose rows are few enough that
 // a launch in front of the GEMM costs less than flags, streams and events. A block row per rank, four 16-byte loads in
-// flight per lane. Bound by the launch at the sizes it is for (1.6 MB: 3 us); 64 MB: 25 us.
+// flight per lane. Bound by the launch at the sizes it is for (1.6 MB: 3 us); 64 MB: 23 us, 134 MB: 42 us.
 __global__ __launch_bounds__(256) void gather_shards_kernel(const GatherParams p) {
   if (p.status != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) retire_status(p.status, p.first_error);
   gather_rows<256>(p, blockIdx.y, blockIdx.x, gridDim.x);

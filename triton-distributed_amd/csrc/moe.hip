@@ -1512,9 +1512,9 @@ int moe_static_scratch_init() {
 // Every workgroup counts the entries of all blocks (a wave per block, 32 loads per lane in flight) and so knows every expert's
 // place; blocks and experts are then shared out among the waves of the grid. The first batch, the experts, the padded total
 // and the ids of the first block that a wave will place are all on their way before anything is waited for.
-// What bounds it: the launch, one trip to memory, four barriers. 64 blocks 4.5 us a launch with 4 waves to a workgroup (5.9 with
-// 16), 160 blocks 6.4 and 512 blocks 8.7 with 16 (half as much again with 4): 4 waves up to kJoinFewBlocks, 16 beyond. (A launch
-// that does nothing: 2.1 us.)
+// What bounds it: the launch, one trip to memory, four barriers. 64 blocks 4.5 us a launch with 4 waves to a workgroup (6.4 with
+// 16), 160 blocks 6.4 and 512 blocks 8.7 with 16 (7.2 and 14.6 with 4): 4 waves up to kJoinFewBlocks, 16 beyond. (In a graph,
+// where a launch that does nothing takes 2.1 us.)
 constexpr int kJoinFewBlocks = 96, kJoinMaxBlock = 512, kJoinCountBits = 10;
 constexpr int64_t kJoinLdsLimit = 160 * 1024 - 256;
 struct JoinParams {
@@ -1655,7 +1655,7 @@ __global__ __launch_bounds__(kThreads) void moe_join_blocks_kernel(const JoinPar
 }
 
 // The same beside the gather of the rows that the GEMM behind will read: the first `join_grid` workgroups join, and are done before
-// the rows are there (8 x 1024 rows by 4096: 25 us for both, 23 + 8 us as two launches).
+// the rows are there (8 x 1024 rows by 4096: 26 us for both, 23 + 8 us as two launches).
 template <int kThreads, int kChunks>
 __global__ __launch_bounds__(kThreads) void moe_gather_and_join_kernel(const GatherParams g, const JoinParams p, int join_grid, int per_rank) {
   const int block = blockIdx.x;

@@ -434,9 +434,9 @@ def _rows_are_at_hand(a, ctx):
 
 def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
     """One launch brings every rank's rows into the workspace, the next multiplies them, on one stream. With the rows at
-    hand a gather at HBM speed is the shortest part of the call (C3's 134 MB: 45 us in front of 605), and a GEMM that shares
+    hand a gather at HBM speed is the shortest part of the call (C3's 134 MB: 42 us in front of 593), and a GEMM that shares
     the chip with copies, keeps 32 compute units free for them or waits for flags costs more than that at every size:
-    C3 711 -> 652 us, 8 x 1024 x 4096 rows by 4096 294 -> 212 us, 4 x 1024 x 4096 by 1536 127 -> 60 us, 4 x 50 rows 128 -> 20 us
+    C3 700 -> 630 us, 8 x 1024 x 4096 rows by 4096 267 -> 204 us, 4 x 1024 x 4096 by 1536 126 -> 60 us, 4 x 50 rows 135 -> 21 us
     (fourteen copies, five events and a flag fill less)."""
     rank, num_ranks = ctx.rank, ctx.num_ranks
     M_per_rank, K = a.shape

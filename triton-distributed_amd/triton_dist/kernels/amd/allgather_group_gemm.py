@@ -103,9 +103,8 @@ _BLOCK_COST = {256: 1.0, 128: 0.625}
 def _row_block(entries, num_experts, n, cus):
     """Rows per block for ``entries`` (token, k) pairs spread over the experts, ``n`` output columns: every expert with rows
     pads half a block on average, and fewer tiles than compute units leave some idle whatever the tile. 256 from 192
-    rows per expert on, where the chip is full (2 x 8192 entries over 8 experts, the two products of a 4096 x 1792 layer
-    through their entry points: 214 and 279 us against 235 and 315 with 128; 2 x 174 rows by 6 over 64 experts, 4352 x 1024:
-    131 and 180 against 124 and 151)."""
+    rows per expert on, where the chip is full (2 x 8192 entries over 8 experts, a whole layer of 4096 x 1792: 513 us against
+    637 with 128; 2 x 174 rows by 6 over 64 experts, 4352 x 1024: 347 against 288)."""
     used, cols = min(num_experts, entries), -(-n // 256)
     return min(_BLOCK_COST, key=lambda b: max(1.0, (entries / b + 0.5 * used) * cols / cus) * _BLOCK_COST[b])
 
@@ -133,7 +132,7 @@ def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, bloc
 
     Blocks that end with their rank segment only add padding where all rows are there (Mixtral's 8 experts x 8 ranks at
     16384 entries: 160 blocks of 128 rows for 128 that are full, and no 256-row ones), also where the chip has room for all
-    of them: fewer tiles are cut along K (8 x 28 tokens by 4 over 8 experts, a layer of 5248 x 1280: 111 us joined, 198 as sorted).
+    of them: fewer tiles are cut along K (8 x 28 tokens by 4 over 8 experts, a layer of 5248 x 1280: 107 us joined, 198 as sorted).
     They are joined on every call, from what the tensors hold then: a caller may replace or rewrite any of them, also between
     the replays of a graph. (Kept from call to call they cost 7 to 14 us less a layer, and a rewritten routing went unseen.)
     ``made``: the context's memory for them, a RowBlocks per size (a graph may hold the address of any of them).
@@ -309,7 +308,7 @@ def create_ag_group_gemm_intra_node_context(tp_pg, tensor_A, tensor_B, full_topk
 def _gather_and_multiply(a, b_nk, c, ctx, shards):
     """With every rank's rows at hand: one launch brings them into the workspace and joins the row blocks across the rank
     segments, the next multiplies them, on one stream. Against copies beside a flag-gated GEMM on 32 compute units less, in
-    blocks that end with their segment (8 x 1024 tokens by 4096, top 2 of 8 experts, 1792 columns): 323 -> 222 us. False
+    blocks that end with their segment (8 x 1024 tokens by 4096, top 2 of 8 experts, 1792 columns): 339 -> 219 us. False
     where the blocks cannot be joined (nothing has been launched then)."""
     M_per_rank, K = a.shape
     workspace = ctx.workspace_tensors[ctx.rank]
