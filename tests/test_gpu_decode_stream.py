@@ -70,6 +70,22 @@ def test_latent_heads_against_the_exact_result(cuda, num_heads, dtype, page, sof
     check(cuda, num_heads, (576, 512), dtype, LENS[lens], page, soft_cap, True, len(lens))
 
 
+# a workgroup's 16 or 32 heads filled, overfilled by one and shared by two kv heads; lengths around its blocks of 32 keys, and
+# sequences of several blocks that share a range with others
+@pytest.mark.parametrize("num_heads", [(16, 1), (17, 1), (32, 1), (33, 1), (48, 1), (40, 2)])
+@pytest.mark.parametrize("lens", [[31, 32, 33, 63, 64, 65, 95, 96, 97], [1, 0, 130, 0, 31, 700, 2]])
+def test_latent_head_sets_and_blocks(cuda, num_heads, lens):
+    announce("decode stream latent heads=%s lens: %s" % (num_heads, lens))
+    check(cuda, num_heads, (576, 512), torch.bfloat16, lens, 16, 0, True, num_heads[0] + len(lens))
+
+
+# sequences with few partials each (a wave merges all of them) and batches on both sides of that rule
+@pytest.mark.parametrize("B,num_heads,D", [(7, (32, 8), 64), (8, (32, 8), 64), (9, (32, 8), 128), (33, (6, 1), 128), (65, (6, 1), 96)])
+def test_merge_of_few_partials(cuda, B, num_heads, D):
+    announce("decode stream merge B=%d heads=%s D=%d" % (B, num_heads, D))
+    check(cuda, num_heads, (D, D), torch.bfloat16, [(97 * i) % 701 + 400 for i in range(B)], 16, 0, False, B + D)
+
+
 def test_workspace_and_head_dimensions_are_checked(cuda):
     from triton_dist import _lib
     lib = _lib.load()

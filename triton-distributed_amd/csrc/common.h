@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 #include "tdist.h"
 
 #define TDIST_AS1 __attribute__((address_space(1)))
@@ -113,6 +115,17 @@ __device__ __forceinline__ void e4m3x4_to_f32(uint32_t w, float* out) {
 // lds_base must be wave-uniform. Completion is tracked by vmcnt.
 __device__ __forceinline__ void load_lds_16(const void* gptr, void* lds_base) {
   __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)gptr, (TDIST_AS3 void*)lds_base, 16, 0, 0);
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): a loop whose index is a constant in every trip
+// without leaning on the unroller (which gives up on bodies as long as a K step's schedule)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 template <int N>

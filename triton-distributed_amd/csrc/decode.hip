@@ -26,7 +26,6 @@
 //    partials. No workgroup ever waits for another, so nothing depends on the grid being co-resident.
 //
 // HBM traffic per launch: every K and V row of the split once (len * Hkv * (Dk + Dv) * 2 B per sequence).
-#include <stdlib.h>
 #include <type_traits>
 
 #include "common.h"
@@ -118,8 +117,7 @@ static __device__ __align__(16) const unsigned char kZeroChunk[16] = {0};
 
 // KEYS = keys per block (16 or 32): one or two groups of 16 keys, a group being one MFMA tile of scores.
 // DM = value dimension = power-of-two part of the key dimension; DPE = the extra key dimensions (0 or 64).
-// kAlias: the value is the first DM columns of the key (latent attention): one row set serves both.
-template <int DM, int DPE, int KEYS, int NST, bool kAlias = false>
+template <int DM, int DPE, int KEYS, int NST>
 struct DecodeCfg {
   static constexpr int kGroups = KEYS / 16;
   static constexpr int kRowBytes = DM * 2;
@@ -133,10 +131,10 @@ struct DecodeCfg {
   static constexpr int kPeRowsPerInstr = 64 / kPeLanesPerRow;
   static constexpr int kPeInstr = DPE > 0 ? KEYS / kPeRowsPerInstr : 0;
   static constexpr int kPeBytes = KEYS * kPeRowBytes;
-  static constexpr int kVBase = kAlias ? 0 : kTensorBytes;
+  static constexpr int kVBase = kTensorBytes;
   static constexpr int kPeBase = kVBase + kTensorBytes;
   static constexpr int kStageBytes = kPeBase + kPeBytes;
-  static constexpr int kLoadsPerGroup = 1 + (kAlias ? 1 : 2) * kInstrPerTensor + kPeInstr;  // table row + K + V (+ extra K)
+  static constexpr int kLoadsPerGroup = 1 + 2 * kInstrPerTensor + kPeInstr;  // table row + K + V (+ extra K)
   static constexpr int kP = NST - 1;
   // LDS position of 16-byte chunk c of a row: K rows c ^ kswz(key), V rows c ^ vswz(key).
   // K operand reads: 16 lanes = 16 keys, same chunk      → spread over 16 positions: key & 15.
@@ -160,13 +158,11 @@ struct DecodeCfg {
   // key needs a new XOR term.
   static constexpr int kRowsPerWindow = kRowBytes >= 256 ? 1 : 256 / kRowBytes;
   static constexpr int kPeRowsPerWindow = DPE > 0 ? 256 / kPeRowBytes : 1;
-  // (one row set for both: 16 keys, 16 positions, and 8 neighbouring keys at 8 pairs of chunks)
-  static_assert(!kAlias || (kSwzMask == 15 && kRowsPerWindow == 1), "shared rows: at least a bank window long");
   __device__ static __forceinline__ int kswz(int key) {
-    return kAlias ? ((key & 7) << 1) | ((key >> 3) & 1) : (key / kRowsPerWindow) & kSwzMask;
+    return (key / kRowsPerWindow) & kSwzMask;
   }
   __device__ static __forceinline__ int vswz(int key) {
-    return kAlias ? kswz(key) : (((key / kRowsPerWindow) & 7) << 1) & kSwzMask;
+    return (((key / kRowsPerWindow) & 7) << 1) & kSwzMask;
   }
   __device__ static __forceinline__ int peswz(int key) { return (key / kPeRowsPerWindow) & kPeSwzMask; }
 };
@@ -348,18 +344,11 @@ __device__ __forceinline__ bool decode_lens_even(const int32_t* lens, int B) {
 // the same time, and no wave waits for another: each writes its own heads' results. For at most 16 query heads per kv
 // head and a number of kv heads that is a multiple of NW.
 // kStream: see decode_stream_kernel; a wave's kv head and its blocks come from its place in the grid.
-// kStreamGroup: see decode_stream_group_kernel; likewise for a workgroup, whose waves share the blocks (b, start and end
-// are then the segment at hand).
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kFuse, bool kPadded, bool kWaveHeads,
-          bool kStream = false, bool kStreamGroup = false>
+          bool kStream = false>
 __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
-  constexpr bool kAlias = kStreamGroup;
-  // kStreamGroup: two waves work on the same blocks of keys and take half of the value dimensions each (their sums would
-  // not leave room for the query beside them in one wave's registers, and one wave per SIMD hides no latency)
-  constexpr int kHalves = kStreamGroup ? 2 : 1;
-  constexpr int NK = NW / kHalves;      // streams of keys
-  constexpr int DT = D / 16 / kHalves;  // tiles of 16 value dimensions per wave
-  typedef DecodeCfg<D, DPE, KEYS, NST, kAlias> C;
+  constexpr int DT = D / 16;  // tiles of 16 value dimensions
+  typedef DecodeCfg<D, DPE, KEYS, NST> C;
   constexpr int G = C::kGroups;
   constexpr int DK = D + DPE;  // key (and query) dimensions; D is the value dimension
   static_assert(!kPadded || DPE == 0, "padded rows have no extra key dimensions");
@@ -372,14 +361,11 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   const int group = prm.Hq / prm.Hkv;
   const int head_blocks = (group + 15) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform for the compiler too
-  const int half = kStreamGroup ? wave & 1 : 0;
-  const int kwave = wave / kHalves;
   const int lane = threadIdx.x & 63;
   // kStream: heads vary fastest over the grid's waves, then the range of blocks
-  // (kStreamGroup: among the workgroups of one XCD, which so share the keys of a range in their L2)
-  const int unit = kStreamGroup ? xcd_major(blockIdx.x, gridDim.x) : blockIdx.x * NW + wave;
-  const int range = kStream || kStreamGroup ? unit / (prm.Hkv * head_blocks) : 0;
-  const int head_unit = kStream || kStreamGroup ? unit - range * prm.Hkv * head_blocks : blockIdx.x;
+  const int unit = blockIdx.x * NW + wave;
+  const int range = kStream ? unit / (prm.Hkv * head_blocks) : 0;
+  const int head_unit = kStream ? unit - range * prm.Hkv * head_blocks : blockIdx.x;
   const int kvh = kWaveHeads ? blockIdx.x * NW + wave : head_unit / head_blocks;
   const int hb = kWaveHeads ? 0 : head_unit - kvh * head_blocks;
   int b = blockIdx.z;
@@ -392,7 +378,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   const int x = lane & 15;   // head (score column) / dv within tile (V^T row) / key (K row)
 
   StreamRange sr{};
-  if constexpr (kStream || kStreamGroup) {
+  if constexpr (kStream) {
     sr = stream_range<KEYS>(prm, range);
     for (int i0 = 0; range == 0 && i0 < prm.B; i0 += 64) {
       // sequences without keys: out = 0, lse = -inf
@@ -411,7 +397,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
 
   // (the lengths through the scalar cache: a vector load would wait for the stream behind which it is queued)
   const auto lens = (const __attribute__((address_space(4))) int32_t*)(uintptr_t)prm.lens;
-  const int len = kStream || kStreamGroup ? 0 : prm.lens[b];
+  const int len = kStream ? 0 : prm.lens[b];
   const int per = (len + prm.S - 1) / prm.S;
   // kWaveHeads: the team streams through splits split .. split + n_splits - 1 of its sequence, one after the other
   const int split = kWaveHeads ? blockIdx.y * prm.splits_per_team : blockIdx.y;
@@ -421,7 +407,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
 
   float* out_base = prm.out + (((int64_t)b * prm.Hq + h0) * prm.S + split) * Dout;
   float* lse_base = prm.lse + ((int64_t)b * prm.Hq + h0) * prm.S + split;
-  if (!kStream && !kStreamGroup && end <= start) {
+  if (!kStream && end <= start) {
     // empty split (and with it every later one): zeros and LSE = -inf so that any merge gives it weight 0
     for (int sp = 0; sp < n_splits; ++sp) {
       for (int i = team_tid; i < nvalid * Dout; i += kTeam) {
@@ -436,14 +422,14 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   typedef TDIST_AS3 unsigned char* lds_u8;  // explicit LDS pointers: a generic pointer would turn reads into
                                             // flat loads, which count on vmcnt and break the DMA accounting
   lds_u8 const smem3 = (lds_u8)smem;
-  lds_u8 const wbase = smem3 + kwave * C::kWaveBytes;
+  lds_u8 const wbase = smem3 + wave * C::kWaveBytes;
   lds_u8 const tbl_base = wbase + NST * C::kStageBytes;
 
   const int nb_total = (end - start + KEYS - 1) / KEYS;
   // this wave's blocks: every NW-th one of the kv head's; or all of its own kv head's, split after split (an empty
   // split at the sequence's end runs one block with every key masked, which writes its zeros)
   auto blocks_of = [&](int lo, int hi) { return max(1, (hi - lo + KEYS - 1) / KEYS); };
-  int n_w = nb_total > kwave ? (nb_total - kwave + NK - 1) / NK : 0;
+  int n_w = nb_total > wave ? (nb_total - wave + NW - 1) / NW : 0;
   if constexpr (kWaveHeads) {
     n_w = 0;
     for (int sp = 0; sp < n_splits; ++sp) n_w += blocks_of(start + sp * per, min(start + (sp + 1) * per, len));
@@ -461,7 +447,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     }
     // Waited for here: a query fetched inside the stream would otherwise be waited for at every use in the loop, and
     // with it (loads count in order) the whole stream behind it.
-    if constexpr (kStream || kStreamGroup) {
+    if constexpr (kStream) {
 #pragma unroll
       for (int s = 0; s < DK / 32; ++s) {
         int4v raw = __builtin_bit_cast(int4v, qf[s]);
@@ -470,7 +456,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       }
     }
   };
-  if constexpr (!kStreamGroup && !kStream) load_q(b);
+  if constexpr (!kStream) load_q(b);
 
   constexpr float kLog2e = 1.4426950408889634f;
   const float scale_log2 = prm.sm_scale * kLog2e;
@@ -507,9 +493,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     for (int d = 0; d < kVWin; ++d) {
       const int key = 16 * q + 4 * g + (x >> 2);
       const int chunk = 2 * d + ((x & 3) >> 1);
-      voff[q][d] = C::kVBase + half * DT * 32 + key * C::kRowBytes + ((chunk ^ C::vswz(key)) << 4) + (x & 1) * 8;
+      voff[q][d] = C::kVBase + key * C::kRowBytes + ((chunk ^ C::vswz(key)) << 4) + (x & 1) * 8;
     }
-  static_assert(kHalves == 1 || (DT * 32) % kWinBytes == 0, "a half begins on a window");
 
   // A block: its first key and the key range [lo, hi) of its split. Keys outside the range are read as the nearest
   // key inside (and, for a split that is empty, as the sequence's last key) and masked in the scores.
@@ -520,7 +505,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     return n;
   };
   // first key of the wave's j-th block where the workgroup shares one split
-  auto shared_block = [&](int j) { return Block{start + (kwave + j * NK) * KEYS, start, end, b}; };
+  auto shared_block = [&](int j) { return Block{start + (wave + j * NW) * KEYS, start, end, b}; };
   // kWaveHeads: a cursor over the team's blocks in order
   struct Cursor { Block blk; int left; };   // left: blocks of this split still to come, this one included
   auto cursor_begin = [&]() { return Cursor{Block{start, start, end, b}, blocks_of(start, end)}; };
@@ -545,8 +530,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     }
   };
 
-  // (rows that the head blocks of a range fetch one after the other are worth keeping in the L2)
-  constexpr int kAux = kStreamGroup ? 0 : TDIST_KV_AUX;
+  constexpr int kAux = TDIST_KV_AUX;
   // K and V rows of block j → stage j % NST
   // The byte offset of a row within its cache (page, place in the page, head) is worked out once per block, by one lane
   // per row (K rows in lanes 0 .. KEYS-1, V rows in the next KEYS), and handed to the lanes that fetch the row's chunks.
@@ -558,7 +542,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     uint32_t off_lo, off_hi;
     {
       const int row = lane & (KEYS - 1);
-      const bool is_v = !kAlias && (lane & KEYS) != 0;
+      const bool is_v = (lane & KEYS) != 0;
       const uint32_t n = (uint32_t)clamp_key(blk.key0 + row, blk);
       const uint32_t in_page = n - (uint32_t)(((uint64_t)n * prm.page_magic) >> prm.page_shift) * (uint32_t)prm.page_size;
       const uint64_t off = (uint64_t)(uint32_t)tbl[row] * (uint64_t)(is_v ? prm.v_sp : prm.k_sp) +
@@ -573,39 +557,35 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       return ((uint64_t)hi << 32) | lo;
     };
     constexpr bool kWholeRow = C::kRowsPerInstr == 1;
-    constexpr int kInstr = C::kInstrPerTensor / kHalves, kPe = C::kPeInstr / kHalves;
+    constexpr int kInstr = C::kInstrPerTensor, kPe = C::kPeInstr;
     const int chunk = lane % C::kLanesPerRow, pchunk = lane % C::kPeLanesPerRow;
     // all exchanges between lanes first, then the loads: the compiler would wait for each exchange at its load
     uint64_t k_off[kInstr], v_off[kInstr], pe_off[kPe > 0 ? kPe : 1];
 #pragma unroll
     for (int u = 0; u < kInstr; ++u) {
-      const int key = kWholeRow ? u * kHalves + half : (u * kHalves + half) * C::kRowsPerInstr + lane / C::kLanesPerRow;
+      const int key = kWholeRow ? u : u * C::kRowsPerInstr + lane / C::kLanesPerRow;
       k_off[u] = row_offset(key, kWholeRow);
-      if constexpr (!kAlias) v_off[u] = row_offset(KEYS + key, kWholeRow);
+      v_off[u] = row_offset(KEYS + key, kWholeRow);
     }
 #pragma unroll
-    for (int u = 0; u < kPe; ++u) pe_off[u] = row_offset((u * kHalves + half) * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow, false);
+    for (int u = 0; u < kPe; ++u) pe_off[u] = row_offset(u * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow, false);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kInstr; ++u) {
-      const int i = u * kHalves + half;
-      const int key = kWholeRow ? i : i * C::kRowsPerInstr + lane / C::kLanesPerRow;
+      const int key = kWholeRow ? u : u * C::kRowsPerInstr + lane / C::kLanesPerRow;
       const int kchunk = chunk ^ C::kswz(key), vchunk = chunk ^ C::vswz(key);
       const unsigned char* ksrc = prm.k + k_off[u] + (uint32_t)(kchunk << 4);
       if (kPadded && kchunk >= valid_chunks) ksrc = kZeroChunk;
-      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)ksrc, (TDIST_AS3 void*)(kst + i * 1024), 16, 0, kAux);
-      if constexpr (!kAlias) {
-        const unsigned char* vsrc = prm.v + v_off[u] + (uint32_t)(vchunk << 4);
-        if (kPadded && vchunk >= valid_chunks) vsrc = kZeroChunk;
-        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)vsrc, (TDIST_AS3 void*)(vst + i * 1024), 16, 0, kAux);
-      }
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)ksrc, (TDIST_AS3 void*)(kst + u * 1024), 16, 0, kAux);
+      const unsigned char* vsrc = prm.v + v_off[u] + (uint32_t)(vchunk << 4);
+      if (kPadded && vchunk >= valid_chunks) vsrc = kZeroChunk;
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)vsrc, (TDIST_AS3 void*)(vst + u * 1024), 16, 0, kAux);
     }
 #pragma unroll
     for (int u = 0; u < kPe; ++u) {
-      const int i = u * kHalves + half;
-      const int key = i * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow;
+      const int key = u * C::kPeRowsPerInstr + lane / C::kPeLanesPerRow;
       const unsigned char* psrc = prm.k + pe_off[u] + (uint32_t)(C::kRowBytes + ((pchunk ^ C::peswz(key)) << 4));
-      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)psrc, (TDIST_AS3 void*)(kst + C::kPeBase + i * 1024), 16, 0, kAux);
+      __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)psrc, (TDIST_AS3 void*)(kst + C::kPeBase + u * 1024), 16, 0, kAux);
     }
   };
 
@@ -721,12 +701,6 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
           const typename MMA::frag8 vf = __builtin_bit_cast(typename MMA::frag8, vt);
           acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, ph), acc[d]);
           acc[d] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, pl), acc[d]);
-        } else if constexpr (kAlias) {
-          // both halves of the probabilities in one product over 32 k slots: the same 4 keys of a lane twice
-          const int2v a0 = v[0];
-          const int4v vt = {a0[0], a0[1], a0[0], a0[1]};
-          const int4v p4 = {(int)hi[0][0], (int)hi[0][1], (int)lo[0][0], (int)lo[0][1]};
-          acc[d] = MMA::mma32(__builtin_bit_cast(typename MMA::frag8, vt), __builtin_bit_cast(typename MMA::frag8, p4), acc[d]);
         } else {
           const int2v ph = {(int)hi[0][0], (int)hi[0][1]};
           const int2v pl = {(int)lo[0][0], (int)lo[0][1]};
@@ -929,130 +903,82 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     return;
   }
 
-  // kStreamGroup: the range's segments (a sequence's part in it), one after the other; else the one split
-  int seg_left = sr.n, seg_block = sr.block;
-  b = kStreamGroup ? sr.seq : b;
-  for (;;) {
-    float* seg_out = out_base;   // rows of the 16 heads, seg_row floats apart; LSEs seg_lse_row apart
-    float* seg_lse = lse_base;
-    int64_t seg_row = (int64_t)prm.S * Dout, seg_lse_row = prm.S;
-    bool whole = false;
-    int seg_n = 0;
-    if constexpr (kStreamGroup) {
-      const int seq_len = lens[b], nb = (seq_len + KEYS - 1) / KEYS;
-      seg_n = min(nb - seg_block, seg_left);
-      start = seg_block * KEYS;
-      end = min(start + seg_n * KEYS, seq_len);
-      whole = seg_n == nb;
-      const int slot = seg_block == 0 ? 1 : 0;
-      seg_out = prm.out + (((int64_t)range * 2 + slot) * prm.Hq + h0) * Dout;
-      seg_lse = prm.lse + ((int64_t)range * 2 + slot) * prm.Hq + h0;
-      seg_row = Dout;
-      seg_lse_row = 1;
-      n_w = seg_n > kwave ? (seg_n - kwave + NK - 1) / NK : 0;
-      m_run = -INFINITY;
-      l_run = 0.f;
-#pragma unroll
-      for (int d = 0; d < DT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
-    }
-    constexpr int kLoads = 1 + (C::kLoadsPerGroup - 1) / kHalves;   // this wave's share of a block's
-    // (kStreamGroup: the waves of a pair bring each other's rows, so all waves step together)
-    const int steps = kStreamGroup ? (seg_n + NK - 1) / NK : n_w;
-    auto step_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    if (n_w > 0) {
-      // page-table rows of the first P+1 blocks, then the first P row groups
-      for (int j = 0; j <= C::kP; ++j) issue_table(j, shared_block(j));
-      if constexpr (kStreamGroup) load_q(b);   // (one trip to memory with the page-table rows)
-      wait_vmcnt<0>();
-      for (int gi = -C::kP; gi < 0; ++gi) {
-        if (gi + C::kP < n_w) {
-          issue_table(gi + 2 * C::kP + 1, shared_block(gi + 2 * C::kP + 1));
-          issue_rows(gi + C::kP, shared_block(gi + C::kP));
-        }
-      }
-    }
-    for (int i = 0; i < steps; ++i) {
-      if constexpr (C::kWaitFirst) wait_vmcnt<0>();
-      if (i + C::kP < n_w) {
-        issue_table(i + 2 * C::kP + 1, shared_block(i + 2 * C::kP + 1));
-        issue_rows(i + C::kP, shared_block(i + C::kP));
-      }
-      if constexpr (!C::kWaitFirst) wait_groups<kLoads>(min(C::kP, n_w - 1 - i));
-      if constexpr (kStreamGroup) step_barrier();
-      if (!kStreamGroup || i < n_w) compute(i, shared_block(i));
-      if constexpr (kStreamGroup) step_barrier();
-    }
-
-    // ---- merge the waves' partial states ---------------------------------------------------------
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
+  if (n_w > 0) {
+    // page-table rows of the first P+1 blocks, then the first P row groups
+    for (int j = 0; j <= C::kP; ++j) issue_table(j, shared_block(j));
     wait_vmcnt<0>();
-    __syncthreads();  // every wave is done with its ring; reuse it
-    TDIST_AS3 float* s_m = (TDIST_AS3 float*)(wbase);  // [16]
-    TDIST_AS3 float* s_l = s_m + 16;                   // [16]
-    TDIST_AS3 float* s_acc = s_l + 16;                 // [16][kAccRow]: the 4 floats between rows spread them over the banks
-    constexpr int kAccRow = decode_acc_row(D);
-    if (lane < 16) {
-      s_m[lane] = m_run;
-      s_l[lane] = l_run;
-    }
-#pragma unroll
-    for (int d = 0; d < DT; ++d) *(TDIST_AS3 float4v*)(s_acc + x * kAccRow + 16 * (half * DT + d) + 4 * g) = acc[d];
-    __syncthreads();
-    // What each stream of keys counts for in each head: lane l works it out for stream l / 16 and head l % 16 (in every
-    // wave: nobody waits), and the LDS hands it round.
-    static_assert(kWaveHeads || kStream || NK <= 4, "one lane per stream of keys and head");
-    float r_lse16;
-    TDIST_AS3 float* const s_w = s_acc + 16 * kAccRow + (kHalves == 1 ? 0 : half * 64);   // this wave's [4][16]
-    {
-      const int w = lane >> 4, h = lane & 15;
-      const TDIST_AS3 float* wm = (const TDIST_AS3 float*)(smem3 + min(w, NK - 1) * C::kWaveBytes);
-      const float mw = w < NK ? wm[h] : -INFINITY;
-      float M = fmaxf(mw, __shfl_xor(mw, 16));
-      M = fmaxf(M, __shfl_xor(M, 32));
-      const float sc = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-      float L = w < NK ? wm[16 + h] * sc : 0.f;
-      L += __shfl_xor(L, 16);
-      L += __shfl_xor(L, 32);
-      s_w[lane] = sc / L;
-      r_lse16 = (M + log2f(L)) * kLn2;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int vecs = Dout / 4;
-    for (int idx = threadIdx.x; idx < nvalid * vecs; idx += NW * 64) {
-      const int h = idx / vecs, dv = (idx - h * vecs) * 4;
-      float4v O = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < NK; ++w) {
-        const float4v a4 = *(const TDIST_AS3 float4v*)((const TDIST_AS3 float*)(smem3 + w * C::kWaveBytes) + 32 + h * kAccRow + dv);
-        const float sc = s_w[w * 16 + h];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) O[e] += a4[e] * sc;
-      }
-      if (kStreamGroup && whole) {
-        store_elem4(prm.final_out, (int64_t)b * prm.fo_sb + (int64_t)(h0 + h) * prm.fo_sh + dv, prm.final_dtype, prm.fo_vec, O);
-      } else {
-        float* o = seg_out + h * seg_row + dv;
-        if (kStreamGroup || prm.part_vec) {
-          store_partial4<kFuse>(o, O);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) store_partial<kFuse>(o + e, O[e]);
-        }
+    for (int gi = -C::kP; gi < 0; ++gi) {
+      if (gi + C::kP < n_w) {
+        issue_table(gi + 2 * C::kP + 1, shared_block(gi + 2 * C::kP + 1));
+        issue_rows(gi + C::kP, shared_block(gi + C::kP));
       }
     }
-    if (threadIdx.x < nvalid) {
-      if (!kStreamGroup || !whole) store_partial<kFuse>(seg_lse + threadIdx.x * seg_lse_row, r_lse16);
-      else if (prm.final_lse) prm.final_lse[(int64_t)b * prm.Hq + h0 + threadIdx.x] = r_lse16;
-    }
-    if constexpr (!kStreamGroup) break;
-    seg_left -= seg_n;
-    if (seg_left == 0) break;
-    do ++b;
-    while (lens[b] <= 0);
-    seg_block = 0;
-    __syncthreads();   // the merge has read its rings
   }
+  for (int i = 0; i < n_w; ++i) {
+    if constexpr (C::kWaitFirst) wait_vmcnt<0>();
+    if (i + C::kP < n_w) {
+      issue_table(i + 2 * C::kP + 1, shared_block(i + 2 * C::kP + 1));
+      issue_rows(i + C::kP, shared_block(i + C::kP));
+    }
+    if constexpr (!C::kWaitFirst) wait_groups<C::kLoadsPerGroup>(min(C::kP, n_w - 1 - i));
+    compute(i, shared_block(i));
+  }
+
+  // ---- merge the waves' partial states ---------------------------------------------------------
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+  wait_vmcnt<0>();
+  __syncthreads();  // every wave is done with its ring; reuse it
+  TDIST_AS3 float* s_m = (TDIST_AS3 float*)(wbase);  // [16]
+  TDIST_AS3 float* s_l = s_m + 16;                   // [16]
+  TDIST_AS3 float* s_acc = s_l + 16;                 // [16][kAccRow]: the 4 floats between rows spread them over the banks
+  constexpr int kAccRow = decode_acc_row(D);
+  if (lane < 16) {
+    s_m[lane] = m_run;
+    s_l[lane] = l_run;
+  }
+#pragma unroll
+  for (int d = 0; d < DT; ++d) *(TDIST_AS3 float4v*)(s_acc + x * kAccRow + 16 * d + 4 * g) = acc[d];
+  __syncthreads();
+  // What each wave counts for in each head: lane l works it out for wave l / 16 and head l % 16 (in every
+  // wave: nobody waits), and the LDS hands it round.
+  static_assert(kWaveHeads || kStream || NW <= 4, "one lane per wave and head");
+  float r_lse16;
+  TDIST_AS3 float* const s_w = s_acc + 16 * kAccRow;   // this wave's [4][16]
+  {
+    const int w = lane >> 4, h = lane & 15;
+    const TDIST_AS3 float* wm = (const TDIST_AS3 float*)(smem3 + min(w, NW - 1) * C::kWaveBytes);
+    const float mw = w < NW ? wm[h] : -INFINITY;
+    float M = fmaxf(mw, __shfl_xor(mw, 16));
+    M = fmaxf(M, __shfl_xor(M, 32));
+    const float sc = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+    float L = w < NW ? wm[16 + h] * sc : 0.f;
+    L += __shfl_xor(L, 16);
+    L += __shfl_xor(L, 32);
+    s_w[lane] = sc / L;
+    r_lse16 = (M + log2f(L)) * kLn2;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int vecs = Dout / 4;
+  for (int idx = threadIdx.x; idx < nvalid * vecs; idx += NW * 64) {
+    const int h = idx / vecs, dv = (idx - h * vecs) * 4;
+    float4v O = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float4v a4 = *(const TDIST_AS3 float4v*)((const TDIST_AS3 float*)(smem3 + w * C::kWaveBytes) + 32 + h * kAccRow + dv);
+      const float sc = s_w[w * 16 + h];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) O[e] += a4[e] * sc;
+    }
+    float* o = out_base + (int64_t)h * prm.S * Dout + dv;
+    if (prm.part_vec) {
+      store_partial4<kFuse>(o, O);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) store_partial<kFuse>(o + e, O[e]);
+    }
+  }
+  if (threadIdx.x < nvalid) store_partial<kFuse>(lse_base + (int64_t)threadIdx.x * prm.S, r_lse16);
 }
 
 // ---- combine --------------------------------------------------------------------------------------
@@ -1286,13 +1212,19 @@ constexpr int kMergeBatch = 16;   // partial results in flight per lane of the m
 // 32 x 32768 660 -> 664. One wave could merge 63 ranges of a sequence at most; without that limit 1 x 131072 keys take 36 us
 // instead of 156 with 6 / 1 heads and 87 instead of 155 with 32 / 8 (32 splits and their combine: 90, 91).
 // 16 waves a workgroup where a sequence may have more partials than four waves hold in flight.
-template <int KEYS, int NW>
+// kAlone: every wave takes 64 pieces of its own and all partials of them, eight in flight, and there is nothing to bring together:
+// for batches whose sequences have few partials each (16 on average at most), where the other form's four waves share a handful and
+// there are four times as many workgroups, each with its trip for the lengths: latent heads, 16 up to 4096 keys 39.2 -> 31.2 us a
+// call, 53 x 100 keys 26.7 -> 18.9, 48 up to 8192 keys with 64 / 8 heads 83.7 -> 80.6, 32 x 32768 655 -> 650. A sequence of many
+// partials beside short ones is read eight partials a trip: 4 uneven sequences up to 21874 keys, 256 ranges, 41.2 us with four
+// waves to a piece, 45.5 alone, hence the bound.
+template <int KEYS, int NW, bool kAlone>
 __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm) {
-  constexpr int kBatch = kMergeBatch;
-  __shared__ float4v s_acc[NW][64];
-  __shared__ float s_max[NW][64], s_sum[NW][64];
+  constexpr int kBatch = kAlone ? kMergeBatch / 2 : kMergeBatch, kPieces = kAlone ? NW * 64 : 64;   // 16-byte pieces of a workgroup
+  __shared__ float4v s_acc[kAlone ? 1 : NW][64];
+  __shared__ float s_max[kAlone ? 1 : NW][64], s_sum[kAlone ? 1 : NW][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row_vecs = prm.dv / 4, vecs = prm.Hq * row_vecs, pieces = (vecs + 63) / 64;
+  const int row_vecs = prm.dv / 4, vecs = prm.Hq * row_vecs, pieces = (vecs + kPieces - 1) / kPieces;
   const int at = blockIdx.x / pieces, piece = blockIdx.x - at * pieces;
   int seq = at, first_block, per;
   if (prm.B < prm.ranges) {
@@ -1309,13 +1241,13 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   const int first = first_block / per, parts = (first_block + nb - 1) / per - first + 1;
   if (parts == 1) return;
 
-  const int at_vec = min(piece * 64 + lane, vecs - 1), h = at_vec / row_vecs;
+  const int my_vec = piece * kPieces + (kAlone ? wave * 64 : 0) + lane, at_vec = min(my_vec, vecs - 1), h = at_vec / row_vecs;
   const int64_t plane = (int64_t)prm.Hq * prm.dv;
   auto slot_of = [&](int j) { return ((int64_t)first + j) * 2 + (j == 0 ? 1 : 0); };
-  const int share = (parts + NW - 1) / NW, j_end = min(parts, (wave + 1) * share);
+  const int share = kAlone ? parts : (parts + NW - 1) / NW, j_begin = kAlone ? 0 : wave * share, j_end = min(parts, j_begin + share);
   float m = -INFINITY, l = 0.f;
   float4v acc = {0.f, 0.f, 0.f, 0.f};
-  for (int j0 = wave * share; j0 < j_end; j0 += kBatch) {
+  for (int j0 = j_begin; j0 < j_end; j0 += kBatch) {
     float4v r[kBatch];
     float w[kBatch];
 #pragma unroll
@@ -1339,24 +1271,28 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
       for (int e = 0; e < 4; ++e) acc[e] += p * r[u][e];
     }
   }
-  s_acc[wave][lane] = acc;
-  s_max[wave][lane] = m;
-  s_sum[wave][lane] = l;
-  __syncthreads();
-  if (wave != 0 || piece * 64 + lane >= vecs) return;
-  float M = s_max[0][lane];
+  float M = m, L = l;
+  if constexpr (!kAlone) {
+    s_acc[wave][lane] = acc;
+    s_max[wave][lane] = m;
+    s_sum[wave][lane] = l;
+    __syncthreads();
+    if (wave != 0) return;
+    M = s_max[0][lane];
 #pragma unroll
-  for (int v = 1; v < NW; ++v) M = fmaxf(M, s_max[v][lane]);
-  float L = 0.f;
-  acc = float4v{0.f, 0.f, 0.f, 0.f};
+    for (int v = 1; v < NW; ++v) M = fmaxf(M, s_max[v][lane]);
+    L = 0.f;
+    acc = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int v = 0; v < NW; ++v) {
-    const float p = s_max[v][lane] == -INFINITY ? 0.f : __expf(s_max[v][lane] - M);
-    L += p * s_sum[v][lane];
-    const float4v a = s_acc[v][lane];
+    for (int v = 0; v < NW; ++v) {
+      const float p = s_max[v][lane] == -INFINITY ? 0.f : __expf(s_max[v][lane] - M);
+      L += p * s_sum[v][lane];
+      const float4v a = s_acc[v][lane];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += p * a[e];
+      for (int e = 0; e < 4; ++e) acc[e] += p * a[e];
+    }
   }
+  if (my_vec >= vecs) return;
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = L > 0.f ? acc[e] / L : 0.f;
   const int d = (at_vec - h * row_vecs) * 4;
@@ -1364,16 +1300,24 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   if (prm.final_lse && d == 0) prm.final_lse[(int64_t)seq * prm.Hq + h] = L > 0.f ? M + logf(L) : -INFINITY;
 }
 
+template <int KEYS, int NW, bool kAlone>
+static int launch_merge_cfg(const DecodeParams& prm, hipStream_t stream) {
+  const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), kAlone ? NW * 64 : 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
+  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone>), dim3((unsigned)(places * pieces)), dim3(NW * 64), 0, stream, prm);
+  return launch_status("tdist_decode_stream");
+}
 template <int KEYS>
 static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
   if (prm.ranges == 1) return TDIST_OK;   // every sequence lies in the one range
-  const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
-  if (prm.ranges > 4 * kMergeBatch * 4)
-    hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 16>), dim3((unsigned)(places * pieces)), dim3(1024), 0, stream, prm);
-  else
-    hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, 4>), dim3((unsigned)(places * pieces)), dim3(256), 0, stream, prm);
-  return launch_status("tdist_decode_stream");
+  if (prm.ranges <= 16 * prm.B) return launch_merge_cfg<KEYS, 4, true>(prm, stream);
+  return prm.ranges > 4 * kMergeBatch * 4 ? launch_merge_cfg<KEYS, 16, false>(prm, stream) : launch_merge_cfg<KEYS, 4, false>(prm, stream);
 }
+
+// Latent attention: blocks of 16 query heads that share a workgroup (a second one is free where the heads fill more than one: the rows
+// come in once for both), and the fewest blocks of 32 keys of a range (1 x 1000 keys, 128 heads: 17.0 us with 2, 18.6 with 4, 21.3
+// with 8; longer batches have more in any case).
+static int latent_head_blocks(int group) { return group <= 16 ? 1 : 2; }
+constexpr int kLatentMinBlocks = 2;
 
 // Streaming form: the whole batch in one launch that fills the chip once. All sequences' blocks of KEYS keys are laid
 // end to end and cut into equal ranges; a wave takes one kv head (and up to 16 of its query heads) over one range,
@@ -1391,35 +1335,392 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodePara
   decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, false, kPadded, false, true>(prm);
 }
 
-// The same for heads that share one key and whose value is a part of it (latent attention, 576 / 512): a workgroup takes
-// a block of 16 query heads over one range, its pairs of waves every fourth block of keys, merged through the LDS where a
-// sequence ends; only the key rows are fetched, and the head blocks of a range run on one XCD, whose L2 then fetches them once.
-// What bounds it: LDS reads of the operands (53 KB per block and wave pair; the scores are worked out in both waves of a
-// pair) and, at a few blocks per stream, the fixed work at a segment's ends. B 16, 128 / 1 heads, 64 to 4096 keys: 387 us
-// with 32 splits and their combine (eight head blocks fetching both row sets, 134 MB of partial results) -> 58-63 us, of
-// which 49 are this kernel (its matrix cores busy 7 % of the time, 28 % of the LDS cycles lost to bank conflicts) and 15 the merge.
-template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
-__global__ __launch_bounds__(NW * 64) void decode_stream_group_kernel(const DecodeParams prm) {
-  decode_split_body<MMA, D, DPE, KEYS, NW, NST, kSoftCap, false, false, false, false, true>(prm);
+// The same for heads that share one key and whose value is the first 512 of its 576 columns (latent attention). A workgroup
+// takes HB blocks of 16 query heads over one range, 32 keys at a time, in two kinds of waves that work side by side, one
+// block of keys apart, and meet once per block:
+//  * HB waves work out the scores and probabilities of 16 heads each (query in registers, 36 MFMAs and the softmax), so that a
+//    head's running maximum and sum concern one wave alone, and leave the probabilities (hi + lo) in the LDS as their lanes
+//    hold them, which is the layout that the output product reads;
+//  * four waves own 128 value columns of all heads each (a value is read from the LDS once per workgroup) and rescale their sums
+//    where a maximum was raised;
+//  * two waves bring the rows in: four stages, two blocks in flight.
+// The head blocks of a range run on one XCD, whose L2 fetches its rows once.
+// What bounds it: at a few blocks per range the launch, the chain lens -> table -> rows -> scores -> output, and the partial
+// results (64 KB a workgroup); in a long stream the instructions of a block, about 1 us for 32 keys by 32 heads (0.5 of it beside
+// the products: softmax, exchange, meeting), and with up to 32 heads HBM. Whole calls, against 16 heads a workgroup with eight
+// waves that each took every fourth block (scores worked out twice, merged through the LDS; 28 % of the LDS cycles lost to bank
+// conflicts, none here): 128 / 1 heads, 16 sequences of 64 to 4096 keys 56.6 -> 27.1 us; 16 x 16384 keys 296 -> 144; 64 x 300
+// 44 -> 24; 1 x 1000 19.9 -> 17.0; 16 / 1 heads, 16 x 16384 68.5 -> 63 (4.8 TB/s). The output waves bringing the rows in as well:
+// 16 x 16384 166 us; 64 heads a workgroup: 132, but twice the partial results (the batch of 16 uneven ones 45 us against 41).
+template <int HB>
+struct LatentCfg {
+  static constexpr int kKeys = 32, kDK = 576, kDV = 512;
+  static constexpr int kLoaders = 2, kThreads = (4 + HB + kLoaders) * 64;
+  static constexpr int kSteps = kDK / 32;        // MFMA steps of a score
+  static constexpr int kTiles = kDV / 16 / 4;    // tiles of 16 value columns per wave
+  static constexpr int kRow = kDV * 2, kPeRow = (kDK - kDV) * 2;
+  // rows of a stage: the first 1024 bytes of the keys, which the output product reads a block after the scores, in four places, the
+  // other 128 in three
+  static constexpr int kStage = kKeys * kRow, kPeStage = kKeys * kPeRow, kStages = 4, kPeStages = 3;
+  static constexpr int kPe = kStages * kStage, kProbs = kPe + kPeStages * kPeStage, kProbBlock = HB * 2048;
+  static constexpr int kAlpha = kProbs + 2 * kProbBlock, kEnd = kAlpha + 2 * HB * 64, kRaised = kEnd + 2 * HB * 128;
+  static constexpr int kTable = kRaised + 32, kTableSlots = 4, kLds = kTable + kTableSlots * kKeys * 4;
+  static constexpr int kRows = kKeys / kLoaders, kLoads = kRows + kRows / 8;   // rows of a loading wave per block, and its loads of them
+  static_assert(kLds <= 160 * 1024, "LDS of one CU");
+  // 16-byte chunk c of a row's first 1024 bytes sits at c ^ swz(key), of the other 128 at c ^ peswz(key). A score's operand read takes
+  // one chunk (or, in half of its lanes, the neighbouring one) of 16 keys, a transposing read two neighbouring chunks of 8 keys:
+  // both spread over all banks (no conflict by the counter).
+  __host__ __device__ static constexpr int swz(int key) { return ((((key & 7) ^ ((key & 8) >> 1)) << 1) | ((key >> 3) & 1)); }
+  __device__ static __forceinline__ int peswz(int key) { return (key >> 1) & 7; }
+};
+
+template <typename MMA, int HB, bool kSoftCap>
+__global__ __launch_bounds__(LatentCfg<HB>::kThreads) void decode_latent_kernel(const DecodeParams prm) {
+  typedef LatentCfg<HB> C;
+  constexpr int KEYS = C::kKeys, DV = C::kDV;
+  typedef TDIST_AS3 unsigned char* lds_u8;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  lds_u8 const lds = (lds_u8)smem;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int x = lane & 15, g = lane >> 4;
+  const int group = prm.Hq / prm.Hkv, head_sets = (group + HB * 16 - 1) / (HB * 16);
+  const int unit = xcd_major(blockIdx.x, gridDim.x);
+  const int range = unit / (prm.Hkv * head_sets), head_unit = unit - range * prm.Hkv * head_sets;
+  const int kvh = head_unit / head_sets, first_head = (head_unit - kvh * head_sets) * HB * 16;
+  const int h0 = kvh * group + first_head, nvalid = min(HB * 16, group - first_head);
+
+  const StreamRange sr = stream_range<KEYS>(prm, range);
+  for (int i0 = 0; range == 0 && i0 < prm.B; i0 += 64) {
+    // sequences without keys: out = 0, lse = -inf
+    unsigned long long none = __ballot(i0 + lane < prm.B && prm.lens[min(i0 + lane, prm.B - 1)] <= 0);
+    for (; none; none &= none - 1) {
+      const int seq = i0 + __builtin_ctzll(none);
+      for (int j = threadIdx.x; j < nvalid * DV; j += C::kThreads)
+        store_elem(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)(h0 + j / DV) * prm.fo_sh + j % DV, prm.final_dtype, 0.f);
+      if (prm.final_lse && (int)threadIdx.x < nvalid) prm.final_lse[(int64_t)seq * prm.Hq + h0 + threadIdx.x] = -INFINITY;
+    }
+  }
+  if (sr.n == 0) return;
+
+  // blocks of the range in order, across the sequences in it
+  const auto lens = (const __attribute__((address_space(4))) int32_t*)(uintptr_t)prm.lens;
+  struct Walk { int key0, hi, seq, left, rem; };   // left / rem: blocks of this sequence / of the range, this one included
+  auto walk_begin = [&]() {
+    const int hi = lens[sr.seq];
+    return Walk{sr.block * KEYS, hi, sr.seq, min((hi + KEYS - 1) / KEYS - sr.block, sr.n), sr.n};
+  };
+  auto walk_next = [&](Walk& w) {   // (stays on the last block)
+    if (w.rem == 1) return;
+    --w.rem;
+    w.key0 += KEYS;
+    if (--w.left == 0) {
+      do w.hi = lens[++w.seq];
+      while (w.hi <= 0);
+      w.key0 = 0;
+      w.left = min((w.hi + KEYS - 1) / KEYS, w.rem);
+    }
+  };
+  constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+  TDIST_AS3 float* const s_alpha = (TDIST_AS3 float*)(lds + C::kAlpha);   // [2][HB][16]
+  TDIST_AS3 float* const s_end = (TDIST_AS3 float*)(lds + C::kEnd);       // [2][HB][16] pairs: 1 / sum, lse
+  TDIST_AS3 int* const s_raised = (TDIST_AS3 int*)(lds + C::kRaised);     // [2][4]
+  lds_u8 const s_p = lds + C::kProbs + lane * 16;                         // [2][HB][2 key groups][64]
+  // Step s: the scores of block s and the output product of block s - 1. Blocks 0 .. n - 1, steps 0 .. n: every wave meets n + 1 times.
+  if (wave >= 4 && wave < 4 + HB) {
+    const int hb = wave - 4;
+    const float scale_log2 = prm.sm_scale * kLog2e;
+    // query: head x, columns 32s + 8g .. + 7; operand reads relative to the stage: chunk 4s + g of key x
+    typename MMA::frag8 qf[C::kSteps];
+    const int h = min(hb * 16 + x, nvalid - 1);
+    int koff[4], peoff[2];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) koff[s] = x * C::kRow + (((4 * s + g) ^ C::swz(x)) << 4);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) peoff[s] = x * C::kPeRow + (((4 * s + g) ^ C::peswz(x)) << 4);
+    float m_run = -INFINITY, l_run = 0.f;   // log2 domain; the sum over this lane's keys
+    bool begins = true;
+    Walk w = walk_begin();
+    for (int i = 0; i < sr.n; ++i) {
+      if (begins) {
+        const unsigned char* row = prm.q + (int64_t)w.seq * prm.q_sb + (int64_t)(h0 + h) * prm.q_sh + 16 * g;
+#pragma unroll
+        for (int s = 0; s < C::kSteps; ++s) qf[s] = __builtin_bit_cast(typename MMA::frag8, *(const int4v*)(row + 64 * s));
+        m_run = -INFINITY;
+        l_run = 0.f;
+        begins = false;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      lds_u8 const st = lds + (i & 3) * C::kStage, pe = lds + C::kPe + i % 3 * C::kPeStage;
+      // four chains of products: sc[q], sc[2 + q] for key group q
+      float4v sc[4] = {float4v{0.f, 0.f, 0.f, 0.f}, float4v{0.f, 0.f, 0.f, 0.f}, float4v{0.f, 0.f, 0.f, 0.f}, float4v{0.f, 0.f, 0.f, 0.f}};
+      // operand n (step n / 2, key group n % 2) is read kAhead products before its own: a step's time is this chain's
+      constexpr int kAhead = 12;
+      int4v kb[kAhead];
+      auto read_k = [&](int n) {
+        const int u = n >> 1, q = n & 1;
+        return *(const TDIST_AS3 int4v*)(u < 16 ? st + koff[u & 3] + (u >> 2) * 256 + q * 16 * C::kRow : pe + peoff[u & 1] + q * 16 * C::kPeRow);
+      };
+#pragma unroll
+      for (int n = 0; n < kAhead; ++n) kb[n] = read_k(n);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 2 * C::kSteps; ++n) {
+        sc[n & 3] = MMA::mma32(__builtin_bit_cast(typename MMA::frag8, kb[n % kAhead]), qf[n >> 1], sc[n & 3]);
+        if (n + kAhead < 2 * C::kSteps) kb[n % kAhead] = read_k(n + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      sc[0] += sc[2];
+      sc[1] += sc[3];
+      // sc[q][e]: key 16q + 4g + e, head x
+      float t[2][4], mx = -INFINITY;
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          t[q][e] = kSoftCap ? prm.soft_cap * tanhf(sc[q][e] * prm.sm_scale / prm.soft_cap) * kLog2e : sc[q][e] * scale_log2;
+      if (w.key0 + KEYS > w.hi) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) t[q][e] = w.key0 + 16 * q + 4 * g + e < w.hi ? t[q][e] : -INFINITY;
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, t[q][e]);
+      // The sums are kept relative to m_run, which is raised only when a score lies kSlack above it: their values then stay
+      // below 2^kSlack, which costs no precision, and are rescaled a few times per stream instead of per block.
+      constexpr float kSlack = 8.f;
+      const int raised = __any(mx > m_run + kSlack);
+      if (raised) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+        if (g == 0) s_alpha[((i & 1) * HB + hb) * 16 + x] = alpha;
+        l_run *= alpha;
+        m_run = m_new;
+      }
+      if (lane == 0) s_raised[(i & 1) * 4 + hb] = raised;
+      const float m_safe = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float p[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          p[e] = __builtin_amdgcn_exp2f(t[q][e] - m_safe);
+          l_run += p[e];
+        }
+        uint32_t hi[2], lo[2];
+        MMA::split(p[0], p[1], hi[0], lo[0]);
+        MMA::split(p[2], p[3], hi[1], lo[1]);
+        *(TDIST_AS3 int4v*)(s_p + (i & 1) * C::kProbBlock + hb * 2048 + q * 1024) = int4v{(int)hi[0], (int)hi[1], (int)lo[0], (int)lo[1]};
+      }
+      if (w.left == 1) {
+        // the sequence's last block in this range
+        float L = l_run + __shfl_xor(l_run, 16);
+        L += __shfl_xor(L, 32);
+        if (g == 0) {
+          TDIST_AS3 float* e = s_end + (((i & 1) * HB + hb) * 16 + x) * 2;
+          e[0] = L > 0.f ? 1.f / L : 0.f;
+          e[1] = L > 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
+        }
+        begins = true;
+      }
+      walk_next(w);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    return;
+  }
+
+  if (wave >= 4 + HB) {
+    // Half of a block's rows each; four lanes work out the place of one. Keys behind the end are read as the last one (their
+    // probabilities are 0).
+    const int first = (wave - 4 - HB) * C::kRows;
+    lds_u8 const table = lds + C::kTable + first * 4;
+    auto page_slot = [&](uint32_t n) { return (uint32_t)(((uint64_t)n * prm.page_magic) >> prm.page_shift); };
+    auto issue_table = [&](int j, const Walk& w) {
+      if (lane < C::kRows) {
+        const uint32_t n = (uint32_t)min(w.key0 + first + lane, w.hi - 1);
+        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)(prm.table + (int64_t)w.seq * prm.t_s + page_slot(n)),
+                                         (TDIST_AS3 void*)(table + j % C::kTableSlots * (KEYS * 4)), 4, 0, 0);
+      }
+    };
+    auto issue_rows = [&](int j, const Walk& w) {
+      const int mine = lane / (64 / C::kRows);
+      const uint32_t n = (uint32_t)min(w.key0 + first + mine, w.hi - 1), in_page = n - page_slot(n) * (uint32_t)prm.page_size;
+      const uint32_t page = (uint32_t)((const volatile TDIST_AS3 int32_t*)(table + j % C::kTableSlots * (KEYS * 4)))[mine];
+      const uint64_t row = (uint64_t)(uintptr_t)prm.k + (uint64_t)page * (uint64_t)prm.k_sp + (in_page * (uint32_t)prm.k_st + (uint32_t)kvh * (uint32_t)prm.k_sh);
+      const uint32_t row_lo = (uint32_t)row, row_hi = (uint32_t)(row >> 32);
+      lds_u8 const st = lds + (j & 3) * C::kStage + first * C::kRow, pe = lds + C::kPe + j % 3 * C::kPeStage + first * C::kPeRow;
+      // (a lane number that the compiler takes for a new one: offsets kept from block to block would be added as 64-bit vectors)
+      int l = lane;
+      asm volatile("" : "+v"(l));
+#pragma unroll
+      for (int u = 0; u < C::kRows; ++u) {
+        const uint64_t at = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)row_hi, u * (64 / C::kRows)) << 32) |
+                            (uint32_t)__builtin_amdgcn_readlane((int)row_lo, u * (64 / C::kRows));
+        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)((const unsigned char*)(uintptr_t)at + (uint32_t)((l ^ C::swz(u & 15)) << 4)),
+                                         (TDIST_AS3 void*)(st + u * C::kRow), 16, 0, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < C::kRows / 8; ++u) {
+        const int key = u * 8 + (l >> 3);
+        const uint32_t lo = (uint32_t)__shfl((int)row_lo, key * (64 / C::kRows)), hi = (uint32_t)__shfl((int)row_hi, key * (64 / C::kRows));
+        const uint64_t at = ((uint64_t)hi << 32) | lo;
+        __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)((const unsigned char*)(uintptr_t)at + (uint32_t)(C::kRow + (((l & 7) ^ C::peswz(key)) << 4))),
+                                         (TDIST_AS3 void*)(pe + u * 1024), 16, 0, 0);
+      }
+    };
+    static_assert(C::kRows % 16 == 0, "a wave's rows begin a group of 16");
+    Walk w_table = walk_begin(), w_rows = w_table;
+    for (int j = 0; j < C::kTableSlots; ++j) {
+      issue_table(j, w_table);
+      walk_next(w_table);
+    }
+    wait_vmcnt<0>();
+    for (int j = 0; j < 2 && j < sr.n; ++j) {
+      issue_rows(j, w_rows);
+      walk_next(w_rows);
+    }
+    for (int s = 0; s <= sr.n; ++s) {
+      // block s has landed (and with it the table of block s + 2, which was fetched before); block s + 1 may be on its way
+      if (s + 1 < sr.n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::kLoads) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (s + 2 < sr.n) {
+        issue_table(s + 4, w_table);
+        walk_next(w_table);
+        issue_rows(s + 2, w_rows);
+        walk_next(w_rows);
+      }
+    }
+    return;
+  }
+
+  // transposing reads relative to the stage: chunks of tile d in keys 4g + x / 4
+  int voff[C::kTiles];
+#pragma unroll
+  for (int d = 0; d < C::kTiles; ++d) {
+    const int key = 4 * g + (x >> 2);
+    voff[d] = key * C::kRow + wave * 256 + (((2 * d + ((x & 3) >> 1)) ^ C::swz(key)) << 4) + (x & 1) * 8;
+  }
+  static_assert(C::kTiles == 8, "a wave's value columns are one window of 16 chunks");
+  float4v acc[C::kTiles][HB];   // value columns wave * 128 + 16d + 4g .. + 3 of head b * 16 + x
+  auto reset = [&]() {
+#pragma unroll
+    for (int d = 0; d < C::kTiles; ++d)
+#pragma unroll
+      for (int b = 0; b < HB; ++b) acc[d][b] = float4v{0.f, 0.f, 0.f, 0.f};
+  };
+  reset();
+
+  Walk w_out = walk_begin();
+  bool begun_here = sr.block == 0;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int j = 0; j < sr.n; ++j) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int par = j & 1;
+    const uint32_t v_base = (uint32_t)(uintptr_t)(lds + (j & 3) * C::kStage);
+    // The transposing reads and the waits for them are written out: for the builtin the compiler waits until every load
+    // into the LDS is done, the ones in flight for later blocks included.
+    constexpr int kAhead = 6;
+    int2v vb[kAhead][2];
+    auto read_v = [&](int d) {
+      const uint32_t at = v_base + (uint32_t)voff[d];
+      asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(vb[d % kAhead][0]) : "v"(at) : "memory");
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(vb[d % kAhead][1]) : "v"(at), "n"(16 * C::kRow) : "memory");
+    };
+    const int4v raised = *(const TDIST_AS3 int4v*)(s_raised + par * 4);
+    int4v pa[HB], pc[HB];
+#pragma unroll
+    for (int b = 0; b < HB; ++b) {
+      pa[b] = *(const TDIST_AS3 int4v*)(s_p + par * C::kProbBlock + b * 2048);
+      pc[b] = *(const TDIST_AS3 int4v*)(s_p + par * C::kProbBlock + b * 2048 + 1024);
+    }
+    int any = raised[0];
+#pragma unroll
+    for (int b = 1; b < HB; ++b) any |= raised[b];
+    if (__builtin_amdgcn_readfirstlane(any)) {
+#pragma unroll
+      for (int b = 0; b < HB; ++b) {
+        const float alpha = __builtin_amdgcn_readfirstlane(raised[b]) ? s_alpha[(par * HB + b) * 16 + x] : 1.f;
+#pragma unroll
+        for (int d = 0; d < C::kTiles; ++d) acc[d][b] *= alpha;
+      }
+    }
+    int4v ph[HB], pl[HB];
+#pragma unroll
+    for (int b = 0; b < HB; ++b) {
+      ph[b] = int4v{pa[b][0], pa[b][1], pc[b][0], pc[b][1]};
+      pl[b] = int4v{pa[b][2], pa[b][3], pc[b][2], pc[b][3]};
+    }
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d) read_v(d);
+    static_for<C::kTiles>([&](auto tile) {
+      constexpr int d = decltype(tile)::value, later = C::kTiles - 1 - d;   // tiles read behind this one
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * (later < kAhead - 1 ? later : kAhead - 1)) : "memory");
+      int2v(&v)[2] = vb[d % kAhead];
+      asm volatile("" : "+v"(v[0]), "+v"(v[1]));
+      const typename MMA::frag8 vf = __builtin_bit_cast(typename MMA::frag8, int4v{v[0][0], v[0][1], v[1][0], v[1][1]});
+#pragma unroll
+      for (int b = 0; b < HB; ++b) acc[d][b] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, ph[b]), acc[d][b]);
+#pragma unroll
+      for (int b = 0; b < HB; ++b) acc[d][b] = MMA::mma32(vf, __builtin_bit_cast(typename MMA::frag8, pl[b]), acc[d][b]);
+      if constexpr (d + kAhead < C::kTiles) read_v(d + kAhead);
+    });
+
+    if (w_out.left == 1) {
+      // the sequence's last block in this range: its result, or its part of it
+      const bool whole = begun_here && w_out.key0 + KEYS >= w_out.hi;
+      const int64_t part = ((int64_t)range * 2 + (begun_here ? 1 : 0)) * prm.Hq + h0;
+#pragma unroll
+      for (int b = 0; b < HB; ++b) {
+        const TDIST_AS3 float* e = s_end + ((par * HB + b) * 16 + x) * 2;
+        const float inv = e[0], lse = e[1];
+        const int h = b * 16 + x, col = wave * 128 + 4 * g;
+        if (h < nvalid) {
+          if (whole) {
+            const int64_t o = (int64_t)w_out.seq * prm.fo_sb + (int64_t)(h0 + h) * prm.fo_sh + col;
+#pragma unroll
+            for (int d = 0; d < C::kTiles; ++d) store_elem4(prm.final_out, o + 16 * d, prm.final_dtype, prm.fo_vec, acc[d][b] * inv);
+            if (prm.final_lse && wave == 0 && g == 0) prm.final_lse[(int64_t)w_out.seq * prm.Hq + h0 + h] = lse;
+          } else {
+            float* o = prm.out + (part + h) * DV + col;
+#pragma unroll
+            for (int d = 0; d < C::kTiles; ++d) *(float4v*)(o + 16 * d) = acc[d][b] * inv;
+            if (wave == 0 && g == 0) prm.lse[part + h] = lse;
+          }
+        }
+      }
+      begun_here = true;
+      reset();
+    }
+    walk_next(w_out);
+  }
 }
 
-template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap>
-static int launch_stream_group_cfg(DecodeParams& prm, int head_blocks, hipStream_t stream) {
-  typedef DecodeCfg<D, DPE, KEYS, NST, true> C;
-  static_assert((32 + 16 * decode_acc_row(D) + 128) * 4 <= C::kWaveBytes, "merge scratch must fit in a wave's ring");
-  const size_t lds = (size_t)(NW / 2) * C::kWaveBytes;
-  static_assert((size_t)(NW / 2) * C::kWaveBytes <= 160 * 1024, "LDS of one CU");
-  auto kern = decode_stream_group_kernel<MMA, D, DPE, KEYS, NW, NST, kSoftCap>;
+template <typename MMA, int HB, bool kSoftCap>
+static int launch_latent_cfg(DecodeParams& prm, hipStream_t stream) {
+  typedef LatentCfg<HB> C;
+  auto kern = decode_latent_kernel<MMA, HB, kSoftCap>;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail(TDIST_ERR_LAUNCH, "decode: cannot reserve %zu B of LDS: %s", lds, hipGetErrorString(e));
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
+    if (e != hipSuccess) return fail(TDIST_ERR_LAUNCH, "decode: cannot reserve %d B of LDS: %s", C::kLds, hipGetErrorString(e));
     attr_set = true;
   }
-  prm.min_blocks = NW;   // two steps of every stream of keys
-  hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)prm.ranges * prm.Hkv * head_blocks)), dim3(NW * 64), lds, stream, prm);
+  prm.min_blocks = kLatentMinBlocks;
+  const int64_t sets = ceil_div(prm.Hq / prm.Hkv, HB * 16);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)prm.ranges * prm.Hkv * sets)), dim3(C::kThreads), C::kLds, stream, prm);
   if (int rc = launch_status("tdist_decode_stream")) return rc;
-  return launch_stream_merge<KEYS>(prm, stream);
+  return launch_stream_merge<C::kKeys>(prm, stream);
+}
+
+template <typename MMA>
+static int launch_latent(DecodeParams& prm, hipStream_t stream) {
+  const bool few = latent_head_blocks(prm.Hq / prm.Hkv) == 1;
+  if (prm.soft_cap > 0.f) return few ? launch_latent_cfg<MMA, 1, true>(prm, stream) : launch_latent_cfg<MMA, 2, true>(prm, stream);
+  return few ? launch_latent_cfg<MMA, 1, false>(prm, stream) : launch_latent_cfg<MMA, 2, false>(prm, stream);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kSoftCap, bool kPadded>
@@ -1507,16 +1808,18 @@ static int stream_ranges(int64_t units, int64_t slots) {
   }
   return best;
 }
-// Units of the streaming form on one compute unit: four waves with rings of up to four stages (as much in flight as
-// eight waves of two, half the fixed work and half the partial results), or one workgroup for latent attention.
-static int stream_waves(int head_dim) { return head_dim > 256 ? 1 : 4; }
-constexpr int kLatentWaves = 8;   // waves of a workgroup of the form for latent attention, one workgroup per compute unit
+// Ranges for a call, given its head counts and key dimension. Four waves with rings of up to four stages per compute unit (as much
+// in flight as eight waves of two, half the fixed work and half the partial results), a kv head and a block of 16 query heads each;
+// or, for latent attention, two workgroups, each a set of head blocks.
+static int stream_ranges_for(int q_heads, int kv_heads, int head_dim) {
+  const int group = q_heads / kv_heads, cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
+  if (head_dim > 256) return stream_ranges((int64_t)kv_heads * ceil_div(group, 16 * latent_head_blocks(group)), 1ll * cus);
+  return stream_ranges((int64_t)kv_heads * ceil_div(group, 16), 4ll * cus);
+}
 static int64_t stream_workspace_bytes(int batch, int q_heads, int kv_heads, int head_dim, int head_dim_v) {
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || head_dim_v <= 0) return -1;
-  const int64_t units = (int64_t)kv_heads * ((q_heads / kv_heads + 15) / 16);
-  const int cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
   // two partial results per range: rows of head_dim_v floats and one LSE per query head
-  return 2ll * stream_ranges(units, (int64_t)cus * stream_waves(head_dim)) * q_heads * (head_dim_v + 1) * 4;
+  return 2ll * stream_ranges_for(q_heads, kv_heads, head_dim) * q_heads * (head_dim_v + 1) * 4;
 }
 
 static int run_decode(const DecodeCall& c, DecodeForm form) {
@@ -1614,19 +1917,13 @@ static int run_decode(const DecodeCall& c, DecodeForm form) {
     const int64_t need = stream_workspace_bytes(c.batch, c.q_heads, c.kv_heads, dk, dv);
     if (c.workspace_bytes < need)
       return fail(TDIST_ERR_WORKSPACE, "%s: %lld bytes of workspace given, %lld needed", who, (long long)c.workspace_bytes, (long long)need);
-    const int cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
-    prm.ranges = stream_ranges((int64_t)c.kv_heads * head_blocks, (int64_t)cus * stream_waves(dk));
+    prm.ranges = stream_ranges_for(c.q_heads, c.kv_heads, dk);
     prm.out = (float*)c.workspace;
     prm.lse = prm.out + 2ll * prm.ranges * c.q_heads * dv;
 #define TDIST_STREAM(D_, DPE_, KEYS_, NW_, NST_, PAD_)                                                \
   return bf ? launch_stream<MmaBF16, D_, DPE_, KEYS_, NW_, NST_, PAD_>(prm, head_blocks, st)         \
             : launch_stream<MmaF16, D_, DPE_, KEYS_, NW_, NST_, PAD_>(prm, head_blocks, st);
-    if (dk > 256) {
-#define TDIST_LATENT(MMA_, CAP_) launch_stream_group_cfg<MMA_, 512, 64, 16, kLatentWaves, 2, CAP_>(prm, head_blocks, st)
-      if (prm.soft_cap > 0.f) return bf ? TDIST_LATENT(MmaBF16, true) : TDIST_LATENT(MmaF16, true);
-      return bf ? TDIST_LATENT(MmaBF16, false) : TDIST_LATENT(MmaF16, false);
-#undef TDIST_LATENT
-    }
+    if (dk > 256) return bf ? launch_latent<MmaBF16>(prm, st) : launch_latent<MmaF16>(prm, st);
     if (dk == 64) TDIST_STREAM(64, 0, 32, 4, 4, false)
     if (dk == 128) TDIST_STREAM(128, 0, 16, 4, 4, false)
     if (dk == 192 && dv == 128) TDIST_STREAM(128, 64, 16, 4, 3, false)

@@ -299,17 +299,6 @@ struct GemmCfg {
   static_assert(kWaveM % 32 == 0 && kWaveN % 32 == 0, "wave tile");
 };
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): a loop whose index is a constant in every trip
-// without leaning on the unroller (which gives up on bodies as long as a K step's schedule)
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // Waits until at most `kOutstanding` of this wave's DMA loads are in flight and for its LDS reads, then joins
 // the workgroup barrier.
 template <int kOutstanding>
