@@ -188,6 +188,18 @@ int tdist_producer_push_peers(void* workspace, const void* const* peer_src, int 
 int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
                         int32_t* first_error, void* stream);
 
+/* C = the gathered rows x B^T for an all-gather whose shards all lie on this GPU: tdist_gather_shards and an ungated
+ * tdist_gemm_chunk_gated_* in one call, of which the gather is left out where the GEMM can read the rows where they lie
+ * (at most 16 shards of at least 2 rows within 4 GiB of each other, world_size * rows_per_rank^2 < 2^32). dtype: of the shards and B
+ * (TDIST_BF16, TDIST_F16, TDIST_F8E4M3; C is bf16 for e4m3, with optional fp32 scales per row and column, else NULL).
+ * shards: HOST array of world_size device pointers to [rows_per_rank, K] rows, 16-byte aligned. workspace: room for the
+ * gathered rows [world_size*rows_per_rank, K]; what it holds afterwards is unspecified. status / first_error: retired as by
+ * tdist_gather_shards. Other arguments, alignment and errors as for those two. */
+int tdist_ag_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, void* workspace,
+                       const void* B, int64_t ldb, void* C, int64_t ldc, int N, int K, const float* row_scale,
+                       const float* col_scale, int32_t* status, int32_t* first_error, void* sk_workspace,
+                       int64_t sk_workspace_bytes, void* stream);
+
 /* Link pacing for the one-GPU producer (no counterpart in the reference, whose chunks arrive over xGMI at the
  * link's rate: ~153 GB/s per peer). tdist_producer_mark stores the device's constant-rate wall clock into *stamp
  * (device uint64); tdist_producer_wait_until holds `stream` until that clock is offset_ns (0 .. 100 ms) past the
@@ -467,6 +479,15 @@ int tdist_group_gemm_gated_fp8e4m3(const void* A, int64_t lda, const void* A_loc
                                    int first_block, const int32_t* flags, int wait_value, int rank, int spin_limit,
                                    int32_t* status, int max_workgroups,
     void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
+
+/* The same without flags for gathered rows that are read where they lie: token t is row t % rows_per_rank of shard
+ * t / rows_per_rank (shards, dtype, limits, status and first_error as for tdist_ag_gemm_rows; TDIST_ERR_UNSUPPORTED beyond them, or where K rows are
+ * of 128 bytes or fewer: gather the rows then). */
+int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+                          int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids,
+                          const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,
+                          int num_blocks, int block_size, int num_valid_tokens, int topk, int32_t* status,
+                          int32_t* first_error, void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Workspace of the GEMM entry points above (tdist_gemm_chunk_gated_*, tdist_gemm_rs_scatter_*,

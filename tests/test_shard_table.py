@@ -27,3 +27,27 @@ def test_own_shard_off_16_bytes_and_too_many_ranks():
     assert _lib.shard_table(shard(0x1004), {1: shard(0x2000)}, 0, 2) is None
     n = _lib.GATHER_MAX_RANKS + 1
     assert _lib.shard_table(shard(0x1000), {r: shard(0x1000 * (r + 1)) for r in range(1, n)}, 0, n) is None
+
+
+@pytest.mark.parametrize("addresses,rows,row_bytes,taken", [
+    ([0x1000, 0x2000], 16, 64, True),
+    ([1 << 33, (1 << 33) + (1 << 32) - 65536], 16, 64, True),
+    ([1 << 33, (1 << 33) + (1 << 32) - 4096], 16, 64, False),   # the last shard's end is out of 32 bits' reach
+    ([1 << 33, 1 << 34], 16, 64, False),
+    ([0x1000 * (r + 1) for r in range(17)], 16, 64, False),
+    ([1 << 20, 1 << 21], 46341, 16, False),                     # 2 * 46341^2 >= 2^32: the division by multiplication ends there
+    ([1 << 20, 1 << 21], 46340, 16, True),
+    ([1 << 20, 1 << 21], 1, 64, False),                         # 2^32 / 1 is no 32-bit factor
+])
+def test_shards_read_where_they_lie(addresses, rows, row_bytes, taken):
+    assert _lib.shards_in_reach(addresses, rows, row_bytes) == taken
+
+
+@pytest.mark.parametrize("rows,world", [(2, 16), (3, 16), (50, 4), (2048, 8), (4095, 16), (16383, 16), (46340, 2)])
+def test_division_by_a_shards_rows(rows, world):
+    """The kernel divides by the high word of a product: exact for every row it may meet."""
+    magic = ((1 << 32) + rows - 1) // rows
+    assert world * rows * rows < 1 << 32 and magic < 1 << 32
+    for shard in range(world):
+        for row in (shard * rows, shard * rows + rows - 1, shard * rows + rows // 2):
+            assert (row * magic) >> 32 == row // rows

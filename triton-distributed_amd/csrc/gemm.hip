@@ -31,12 +31,13 @@
 #include <utility>
 
 #include "common.h"
+#include "gather.h"
 #include "gemm_small.h"
 
 namespace tdist {
 
 struct GemmParams {
-  const unsigned char* A;        // gathered workspace
+  const unsigned char* A;        // gathered workspace, or the lowest shard where the rows lie in shards
   const unsigned char* A_local;  // own shard or NULL
   const unsigned char* B;
   unsigned char* C;              // plain output (scatter_bufs == NULL)
@@ -46,6 +47,8 @@ struct GemmParams {
   const int32_t* flags;
   const int32_t* chunk_order;
   int32_t* status;
+  ShardRows shards;                   // rows != 0: A's rows lie in shards, at these offsets from A (no flags, no local shard)
+  uint32_t shard_magic;               // grouped: see gather.h (0 where the rows lie in one piece)
   int64_t lda_b, lda_local_b, ldb_b;  // byte strides
   int64_t ldc;                         // elements
   int M, N, K;
@@ -398,6 +401,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       asm volatile("" : "+v"(frag_lane_a[q]), "+v"(frag_lane_a_hi[q]), "+v"(frag_lane_b[q]));
     }
   }
+  if constexpr (!kGrouped || kPlain) retire_beside(p.shards);
   const int num_pid_m = (p.M + BM - 1) / BM;
   const int num_pid_n = (p.N + BN - 1) / BN;
   const int cm = p.m_per_chunk / BM;                 // row tiles per chunk
@@ -575,6 +579,11 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
   // its segment's first row, its id is -1 and it stores nothing.
   // 16384 x 1792 x 4096 / 16384 x 4096 x 1792 over 8 experts, 256 x 256 tiles: 210 -> 197 and 260 -> 232 us.
   constexpr bool kFlat = kGrouped && kPlain;
+  // (rows in shards: lane r holds shard r's offset from A)
+  int shard_off = 0;
+  if constexpr (kFlat) {
+    if (p.shards.rows != 0) shard_off = (int)p.shards.off[lane % kMaxShards];
+  }
   constexpr bool kFlatSkips = kFlat && !kEarly;
   constexpr int kIdRegs = kFlat ? C::kWaveM / 64 : 1;
   int row_id[kIdRegs] = {0};
@@ -621,7 +630,9 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     for (int t = 0; t < (kFlat ? C::kAInstr : 1); ++t) {
       const int r = (wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row;
       const int gr = min(max(flat_token(raw[t], first, padding_token), 0), p.a_rows - 1);
-      off[t] = (uint32_t)gr * (uint32_t)p.lda_b + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
+      // (rows in one piece: shard 0 at offset 0)
+      const int shard = (int)__umulhi((uint32_t)gr, p.shard_magic);
+      off[t] = (uint32_t)__shfl(shard_off, shard) + (uint32_t)(gr - shard * p.shards.rows) * (uint32_t)p.lda_b + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
     }
   };
   // tile of C behind schedule index sidx (ungated calls)
@@ -631,6 +642,20 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     tm0 = tpid_m * BM;
     tn0 = (twithin / cm) * BN;
     return tpid_m < num_pid_m;
+  };
+
+  // Rows in shards: the tile's lane offsets from A. Its shards (one or two, more where they are short) one after the other, their offsets
+  // by scalar loads, each for the rows from its first on.
+  auto shard_offsets = [&](int tm0, uint32_t (&off)[C::kAInstr]) {
+    const int rows = p.shards.rows, last = min(tm0 + BM, p.M) - 1;
+    for (int s = __builtin_amdgcn_readfirstlane(tm0 / rows), first = s * rows; first <= last; ++s, first += rows) {
+      const uint32_t at = p.shards.off[s] - (uint32_t)first * (uint32_t)p.lda_b;
+#pragma unroll
+      for (int t = 0; t < C::kAInstr; ++t) {
+        const int r = (wave * C::kAInstr + t) * C::kRowsPerInstr + dma_row, row = min(tm0 + r, p.M - 1);
+        if (row >= first) off[t] = at + (uint32_t)row * (uint32_t)p.lda_b + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
+      }
+    }
   };
 
   int sbase = 0;
@@ -746,7 +771,8 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     // DMA sources: a wave-uniform base (first row of the tile, advanced along K in scalar registers) plus a
     // 32-bit per-lane offset, so that the load takes its address as SGPR base + VGPR offset and the K loop
     // carries no vector address arithmetic for it
-    const int a_g0 = kGrouped ? 0 : min(m0 - a_row_off, a_row_max), b_g0 = min(n0, p.N - 1);
+    const bool in_shards = !kGrouped && p.shards.rows != 0;
+    const int a_g0 = kGrouped || in_shards ? 0 : min(m0 - a_row_off, a_row_max), b_g0 = min(n0, p.N - 1);
     const unsigned char* const a_base = Arows + (int64_t)a_g0 * a_ld + (int64_t)ka * KB;
     const unsigned char* b_base_ = p.B + (int64_t)b_g0 * p.ldb_b + (int64_t)ka * KB;
     if constexpr (kGrouped) b_base_ += (int64_t)(kFlat ? tile_expert : p.block_expert[pid_m]) * p.b_expert_stride_b;
@@ -769,6 +795,9 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         gr = min(m0 + r - a_row_off, a_row_max);
       }
       a_off[t] = (uint32_t)(gr - a_g0) * (uint32_t)a_ld + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
+    }
+    if constexpr (!kGrouped) {
+      if (in_shards) shard_offsets(m0, a_off);
     }
 #pragma unroll
     for (int t = 0; t < C::kBInstr; ++t) {
@@ -1259,8 +1288,9 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
         if (p.scatter_bufs != nullptr) c_aligned = (reinterpret_cast<uintptr_t>(p.scatter_bufs[m0 / p.m_per_rank]) & 15) == 0;
         if (c_aligned) {
           early = true;
-          a_base_n = p.A + (int64_t)nm0 * p.lda_b;
+          a_base_n = in_shards ? p.A : p.A + (int64_t)nm0 * p.lda_b;
           b_base_n = p.B + (int64_t)nn0 * p.ldb_b;
+          if (in_shards) shard_offsets(nm0, a_off);
         }
       }
       // (wave-uniform by construction; said so to the compiler, which otherwise carries them in vector registers)
@@ -1799,6 +1829,7 @@ struct GemmCall {
   int64_t sk_workspace_bytes;
   hipStream_t stream;
   const char* who;
+  ShardRows shards;   // rows != 0: A's rows lie in shards
 };
 
 template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
@@ -1897,6 +1928,7 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
 static int run_small(const GemmCall& c, GemmElem elem, int esz, const SmallPlan& plan, const DeviceInfo& di) {
   SmallGemmParams q;
   q.A = (const unsigned char*)c.A;
+  q.shards = c.shards;
   q.B = (const unsigned char*)c.B;
   q.C = (unsigned char*)c.C;
   q.scatter_bufs = c.scatter_bufs;
@@ -2096,6 +2128,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   const int BN = kChoices[pick].bn;
   GemmParams p;
   p.A = (const unsigned char*)c.A;
+  p.shards = c.shards;
+  p.shard_magic = 0;
   p.A_local = (const unsigned char*)c.A_local;
   p.B = (const unsigned char*)c.B;
   p.C = (unsigned char*)c.C;
@@ -2300,6 +2334,7 @@ struct GroupGemmCall {
   int64_t sk_workspace_bytes;
   hipStream_t stream;
   const char* who;
+  ShardRows shards;   // rows != 0: A's rows lie in shards (calls without flags only)
 };
 
 static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
@@ -2319,7 +2354,7 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   if (c.lda < c.K || c.ldb < c.K || c.ldc < c.N) return fail(TDIST_ERR_INVALID, "%s: leading dimension smaller than row", who);
   // rows are addressed as a scalar base plus a 32-bit byte offset: the gathered A (and the own shard) must stay
   // below 4 GiB, as must one expert's B panel
-  if ((int64_t)c.a_rows * c.lda * esz >= (1ll << 32) || (c.A_local && (int64_t)c.local_rows * c.lda_local * esz >= (1ll << 32)) ||
+  if ((c.shards.rows == 0 && (int64_t)c.a_rows * c.lda * esz >= (1ll << 32)) || (c.A_local && (int64_t)c.local_rows * c.lda_local * esz >= (1ll << 32)) ||
       c.ldb * esz > (1 << 22))
     return fail(TDIST_ERR_UNSUPPORTED, "%s: A above 4 GiB or B row stride above 4 MiB", who);
   if ((int64_t)c.num_blocks * c.block_size > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: too many rows", who);
@@ -2331,6 +2366,8 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
 
   GemmParams p;
   p.A = (const unsigned char*)c.A;
+  p.shards = c.shards;
+  p.shard_magic = c.shards.rows != 0 ? shard_magic(c.shards.rows) : 0;
   p.A_local = (const unsigned char*)c.A_local;
   p.B = (const unsigned char*)c.B;
   p.C = (unsigned char*)c.C;
@@ -2402,6 +2439,7 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
     default: return launch_gemm_cfg<E8, BM_, BN_, KB_, 2, 2, NST_, false, true, PL_>(p, grid, c.stream, who);        \
   }
   const bool plain = k128 && c.flags == nullptr && c.A_local == nullptr && (int64_t)c.num_valid * c.topk < (1ll << 32);
+  if (c.shards.rows != 0 && !plain) return fail(TDIST_ERR_UNSUPPORTED, "%s: rows in shards need K*elem_size above 128 bytes and no flags", who);
   if (plain) {
     // Nothing to wait for: an XCD's workgroups walk a block of tiles of few operand panels (rows + columns of tiles),
     // as in an ungated GEMM, instead of one row block after the other (16 column tiles: 4 x 8 tiles, 12 panels, instead
@@ -2440,6 +2478,7 @@ using namespace tdist;
 
 #define TDIST_GATED_BODY(ELEM, RS, CS, WHO)                                                                         \
   GemmCall c;                                                                                                       \
+  c.shards.rows = 0;                                                                                                \
   c.A = A; c.lda = lda; c.A_local = A_local; c.lda_local = lda_local;                                               \
   c.local_row_begin = local_row_begin; c.local_rows = local_rows;                                                   \
   c.B = B; c.ldb = ldb; c.C = C; c.scatter_bufs = nullptr; c.ldc = ldc; c.M = M; c.N = N; c.K = K;                  \
@@ -2488,6 +2527,7 @@ static int gemm_rs_scatter(GemmElem elem, const void* A, int64_t lda, const void
                            const float* row_scale = nullptr, const float* col_scale = nullptr) {
   if (!scatter_bufs) return fail(TDIST_ERR_INVALID, "%s: null scatter_bufs", who);
   GemmCall c;
+  c.shards.rows = 0;
   c.A = A; c.lda = lda; c.A_local = nullptr; c.lda_local = 0; c.local_row_begin = 0; c.local_rows = 0;
   c.B = B; c.ldb = ldb; c.C = nullptr; c.scatter_bufs = scatter_bufs; c.ldc = ldc; c.M = M; c.N = N; c.K = K;
   c.row_scale = row_scale; c.col_scale = col_scale; c.flags = nullptr; c.m_per_chunk = 0; c.wait_value = 0;
@@ -2518,8 +2558,46 @@ int tdist_gemm_rs_scatter_fp8e4m3(const void* A, int64_t lda, const void* B, int
                          sk_workspace_bytes, stream, "tdist_gemm_rs_scatter_fp8e4m3", row_scale, col_scale);
 }
 
+static int elem_of(int dtype, GemmElem& elem, const char* who) {
+  switch (dtype) {
+    case TDIST_BF16: elem = kElemBF16; return TDIST_OK;
+    case TDIST_F16: elem = kElemF16; return TDIST_OK;
+    case TDIST_F8E4M3: elem = kElemFP8; return TDIST_OK;
+    default: return fail(TDIST_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
+  }
+}
+
+int tdist_ag_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, void* workspace, const void* B, int64_t ldb,
+                       void* C, int64_t ldc, int N, int K, const float* row_scale, const float* col_scale, int32_t* status,
+                       int32_t* first_error, void* sk_workspace, int64_t sk_workspace_bytes, void* stream) {
+  const char* who = "tdist_ag_gemm_rows";
+  GemmElem elem;
+  if (int rc = elem_of(dtype, elem, who)) return rc;
+  if (rows_per_rank <= 0 || K <= 0 || (int64_t)world_size * rows_per_rank > 0x7fffffff) return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
+  if (dtype != TDIST_F8E4M3 && (row_scale || col_scale)) return fail(TDIST_ERR_INVALID, "%s: scales are for e4m3 inputs", who);
+  const int64_t rank_bytes = (int64_t)rows_per_rank * K * (dtype == TDIST_F8E4M3 ? 1 : 2);
+  GatherParams g;   // (checks the shards; used only where they are gathered)
+  if (int rc = gather_params(g, workspace, shards, world_size, rank_bytes, status, first_error, who)) return rc;
+  GemmCall c = {};
+  const unsigned char* base;
+  c.shards.rows = 0;
+  if (shards_in_reach(shards, world_size, rows_per_rank, rank_bytes, c.shards, base)) {
+    c.A = base;
+    c.shards.status = status;
+    c.shards.first_error = first_error;
+  } else {
+    if (int rc = tdist_gather_shards(workspace, shards, world_size, rank_bytes, status, first_error, stream)) return rc;
+    c.A = workspace;
+  }
+  c.lda = K; c.B = B; c.ldb = ldb; c.C = C; c.ldc = ldc; c.M = world_size * rows_per_rank; c.N = N; c.K = K;
+  c.row_scale = row_scale; c.col_scale = col_scale; c.world_size = world_size;
+  c.sk_workspace = sk_workspace; c.sk_workspace_bytes = sk_workspace_bytes; c.stream = (hipStream_t)stream; c.who = who;
+  return run_gemm(c, elem);
+}
+
 #define TDIST_GROUP_GEMM_BODY(ELEM, WHO)                                                                              \
   GroupGemmCall c;                                                                                                    \
+  c.shards.rows = 0;                                                                                                  \
   c.A = A; c.lda = lda; c.A_local = A_local; c.lda_local = lda_local; c.local_row_begin = local_row_begin;            \
   c.local_rows = local_rows; c.B = B; c.ldb = ldb; c.expert_stride = expert_stride; c.C = C; c.ldc = ldc;             \
   c.a_rows = a_rows; c.N = N; c.K = K; c.sorted_ids = sorted_token_ids; c.expert_ids = expert_ids;                    \
@@ -2542,6 +2620,32 @@ int tdist_group_gemm_gated_bf16(TDIST_GROUP_GEMM_ARGS) { TDIST_GROUP_GEMM_BODY(k
 int tdist_group_gemm_gated_f16(TDIST_GROUP_GEMM_ARGS) { TDIST_GROUP_GEMM_BODY(kElemF16, "tdist_group_gemm_gated_f16") }
 int tdist_group_gemm_gated_fp8e4m3(TDIST_GROUP_GEMM_ARGS) {
   TDIST_GROUP_GEMM_BODY(kElemFP8, "tdist_group_gemm_gated_fp8e4m3")
+}
+
+int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+                          int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded, int num_blocks, int block_size,
+                          int num_valid_tokens, int topk, int32_t* status, int32_t* first_error, void* sk_workspace,
+                          int64_t sk_workspace_bytes, void* stream) {
+  const char* who = "tdist_group_gemm_rows";
+  GemmElem elem;
+  if (int rc = elem_of(dtype, elem, who)) return rc;
+  if (rows_per_rank <= 0 || K <= 0 || (int64_t)world_size * rows_per_rank > 0x7fffffff) return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
+  const int64_t rank_bytes = (int64_t)rows_per_rank * K * (dtype == TDIST_F8E4M3 ? 1 : 2);
+  GroupGemmCall c = {};
+  const unsigned char* base;
+  for (int r = 0; shards && r < world_size; ++r)
+    if (!shards[r] || !aligned16(shards[r])) return fail(shards[r] ? TDIST_ERR_UNSUPPORTED : TDIST_ERR_INVALID, "%s: shard %d: null or not 16-byte aligned", who, r);
+  if (!shards) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (!shards_in_reach(shards, world_size, rows_per_rank, rank_bytes, c.shards, base))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: at most %d shards within 4 GiB of each other, world_size * rows_per_rank^2 below 2^32", who, kMaxShards);
+  c.shards.status = status; c.shards.first_error = first_error;
+  c.A = base; c.lda = K; c.B = B; c.ldb = ldb; c.expert_stride = expert_stride; c.C = C; c.ldc = ldc;
+  c.a_rows = world_size * rows_per_rank; c.N = N; c.K = K; c.sorted_ids = sorted_token_ids; c.expert_ids = expert_ids;
+  c.block_segment = block_barrier_ids; c.post_pad = num_tokens_post_padded; c.num_blocks = num_blocks; c.block_size = block_size;
+  c.num_valid = num_valid_tokens; c.topk = topk; c.tokens_per_rank = c.a_rows;
+  c.sk_workspace = sk_workspace; c.sk_workspace_bytes = sk_workspace_bytes; c.stream = (hipStream_t)stream; c.who = who;
+  return run_group_gemm(c, elem);
 }
 
 }  // extern "C"

@@ -1,17 +1,19 @@
 // GEMMs that do not fill the chip with large tiles: what run_gemm (gemm.hip) hands to gemm_small.hip.
 #pragma once
 #include "common.h"
+#include "gather.h"
 
 namespace tdist {
 
 struct SmallGemmParams {
   const unsigned char* A;
+  ShardRows shards;           // rows != 0: A's rows lie in shards, at these offsets from A
   const unsigned char* B;
   unsigned char* C;           // plain output (scatter_bufs == NULL)
   void* const* scatter_bufs;  // GEMM-RS: rows of owner o go to scatter_bufs[o] from row rank * m_per_rank on
   const float* row_scale;     // e4m3 inputs: fp32 scales or NULL
   const float* col_scale;
-  int64_t lda_b, ldb_b;  // byte strides; M * lda_b and N * ldb_b below 2^31
+  int64_t lda_b, ldb_b;  // byte strides; M * lda_b (of rows in one piece) and N * ldb_b below 2^31
   int64_t ldc;           // elements
   int M, N;
   int k_bytes;  // a multiple of 16

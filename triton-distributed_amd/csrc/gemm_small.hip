@@ -53,7 +53,8 @@ struct SmallCfg {
   static_assert((NST - 2) * kLoads < 64, "vmcnt is 6 bits");
 };
 
-template <typename E, int BM, int BN, int NST, bool kScales>
+// kShards: A's rows lie in shards (an instance of its own: the test for them alone costs the other calls 0.3 us of 21)
+template <typename E, int BM, int BN, int NST, bool kScales, bool kShards>
 __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParams p) {
   typedef SmallCfg<BM, BN, NST> C;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   const int tiles_m = (p.M + BM - 1) / BM, tiles = tiles_m * ((p.N + BN - 1) / BN);
   const int xcd = blockIdx.x & 7, of_xcd = blockIdx.x >> 3;
   const int mine = of_xcd / p.splits, piece = of_xcd - mine * p.splits;
+  if constexpr (kShards) retire_beside(p.shards);
   if (mine >= (tiles >> 3) + (xcd < (tiles & 7))) return;
   const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + mine;
   const int tm = tile % tiles_m, tn = tile / tiles_m;
@@ -84,6 +86,18 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     const int r = (i * 4 + wave) * 8 + (lane >> 3);
     chunk_a[i] = (lane & 7) ^ ((r >> 1) & 7);
     aoff[i] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.lda_b + chunk_a[i] * 16;
+  }
+  if constexpr (kShards) {
+    // rows in shards: the tile's few shards one after the other (their offsets by scalar loads), each for the rows from its first on
+    const int rows = p.shards.rows, last = min(m0 + BM, p.M) - 1;
+    for (int s = m0 / rows, first = s * rows; first <= last; ++s, first += rows) {
+      const uint32_t off = p.shards.off[s] - (uint32_t)first * (uint32_t)p.lda_b;
+#pragma unroll
+      for (int i = 0; i < C::kAInstr; ++i) {
+        const int row = min(m0 + (i * 4 + wave) * 8 + (lane >> 3), p.M - 1);
+        if (row >= first) aoff[i] = off + (uint32_t)row * (uint32_t)p.lda_b + chunk_a[i] * 16;
+      }
+    }
   }
 #pragma unroll
   for (int i = 0; i < C::kBInstr; ++i) {
@@ -267,10 +281,10 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   }
 }
 
-template <typename E, int BM, int BN, int NST, bool kScales>
-static int launch_cfg(const SmallGemmParams& p, hipStream_t stream, const char* who) {
+template <typename E, int BM, int BN, int NST, bool kScales, bool kShards>
+static int launch_shards(const SmallGemmParams& p, hipStream_t stream, const char* who) {
   typedef SmallCfg<BM, BN, NST> C;
-  auto kern = gemm_small_kernel<E, BM, BN, NST, kScales>;
+  auto kern = gemm_small_kernel<E, BM, BN, NST, kScales, kShards>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes);
@@ -280,6 +294,11 @@ static int launch_cfg(const SmallGemmParams& p, hipStream_t stream, const char* 
   const int64_t grid = 8 * ceil_div(ceil_div(p.M, BM) * ceil_div(p.N, BN), 8) * p.splits;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), C::kLdsBytes, stream, p);
   return launch_status(who);
+}
+
+template <typename E, int BM, int BN, int NST, bool kScales>
+static int launch_cfg(const SmallGemmParams& p, hipStream_t stream, const char* who) {
+  return p.shards.rows != 0 ? launch_shards<E, BM, BN, NST, kScales, true>(p, stream, who) : launch_shards<E, BM, BN, NST, kScales, false>(p, stream, who);
 }
 
 template <int BM, int BN, int NST>

@@ -46,6 +46,7 @@ PROTOTYPES = {
     "tdist_gemm_chunk_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_producer_push_chunk": (_I, [_P, _P, _L, _P, _P, _I, _P]),
     "tdist_producer_push_peers": (_I, [_P, _P, _I, _I, _L, _L, _P, _I, _P, _P, _P, _L, ctypes.c_uint32, _L, _I, _P]),
+    "tdist_ag_gemm_rows": (_I, [_I, _P, _I, _I, _P, _P, _L, _P, _L, _I, _I, _P, _P, _P, _P, _P, _L, _P]),
     "tdist_gather_shards": (_I, [_P, _P, _I, _L, _P, _P, _P]),
     "tdist_producer_mark": (_I, [_P, _P]),
     "tdist_producer_wait_until": (_I, [_P, _L, _P]),
@@ -76,6 +77,7 @@ PROTOTYPES = {
     "tdist_group_gemm_gated_bf16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_f16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
+    "tdist_group_gemm_rows": (_I, [_I, _P, _I, _I, _P, _L, _L, _P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _L, _P]),
     "tdist_gemm_split_k_workspace_bytes": (_L, []),
     "tdist_decode_split_kv": (_I, [_P, _P, _P, _P, _P, _F, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I,
                                    _L, _L, _L, _L, _L, _L, _L, _L, _L, _I, _P]),
@@ -187,6 +189,11 @@ def shard_table(own, peer_shards, rank, num_ranks):
             return None
         table[r] = t.data_ptr()
     return table
+
+
+def shards_in_reach(table, rows, row_bytes):
+    """Whether tdist_group_gemm_rows takes these shards where they lie (a host table of shard_table): see gather.h."""
+    return len(table) <= 16 and rows >= 2 and len(table) * rows * rows < 1 << 32 and max(table) - min(table) + rows * row_bytes < (1 << 32) - 4096
 
 
 def dtype_code(dtype):

@@ -129,7 +129,7 @@ class AllGatherGEMMTensorParallelContext:
     autotune: bool = False
     # ---- one-GPU additions -------------------------------------------------------------------
     # With none of the producer settings below in use the peers' rows are simply there when the call is made, and
-    # ag_gemm_intra_node gathers them in one launch in front of an ungated GEMM (_gather_and_multiply). Setting one of them
+    # ag_gemm_intra_node multiplies them in an ungated GEMM that reads them where they lie (_gather_and_multiply). Setting one of them
     # (a link rate, an arrival order, delays, withheld chunks, the copy engines, the producer kernel) brings the rows in
     # chunk by chunk beside the GEMM, which waits for each chunk's flag.
     output_dtype: torch.dtype = torch.bfloat16
@@ -433,23 +433,29 @@ def _rows_are_at_hand(a, ctx):
 
 
 def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
-    """One launch brings every rank's rows into the workspace, the next multiplies them, on one stream. With the rows at
-    hand a gather at HBM speed is the shortest part of the call (C3's 134 MB: 42 us in front of 593), and a GEMM that shares
-    the chip with copies, keeps 32 compute units free for them or waits for flags costs more than that at every size:
-    C3 700 -> 630 us, 8 x 1024 x 4096 rows by 4096 267 -> 204 us, 4 x 1024 x 4096 by 1536 126 -> 60 us, 4 x 50 rows 135 -> 21 us
-    (fourteen copies, five events and a flag fill less)."""
+    """The product of every rank's rows, read where they lie, in one launch; where they lie too far apart, one launch brings them into
+    the workspace first (tdist_ag_gemm_rows). With the rows at hand a GEMM that shares the chip with copies, keeps 32 compute units
+    free for them or waits for flags is behind at every size (C3 700 us against 630, 4 x 50 rows 135 against 21), and so is one
+    with a gather in front: the workspace is scratch here, and what it holds afterwards is unspecified."""
     rank, num_ranks = ctx.rank, ctx.num_ranks
     M_per_rank, K = a.shape
     workspace = ctx.workspace_tensors[rank]
-    M = M_per_rank * num_ranks
+    if b.stride(1) != 1:
+        raise ValueError("A, B and C must be row-major with a contiguous last dimension")
+    if (row_scale is not None or col_scale is not None) and a.dtype != torch.float8_e4m3fn:
+        raise ValueError("scales are only defined for fp8 inputs")
+    if a.dtype not in _GEMM_ENTRY:
+        raise TypeError("unsupported GEMM dtype %s" % a.dtype)
+    if workspace.numel() < num_ranks * M_per_rank * K:
+        raise ValueError("the context was created for fewer rows or columns than %d x %d" % (num_ranks * M_per_rank, K))
     current = _lib.stream_ptr()
     stream = ctx.gemm_stream.cuda_stream
     if stream != current:
         ctx.gemm_stream.wait_stream(torch.cuda.current_stream())
-    _lib.call("tdist_gather_shards", workspace.data_ptr(), shards, num_ranks, M_per_rank * K * a.element_size(),
-              ctx.status.data_ptr(), ctx.status.data_ptr() + 8, stream)
-    gated_gemm(workspace if workspace.shape[0] == M else workspace[:M], None, 0, b, c, None, 0, rank, num_ranks, row_scale=row_scale,
-               col_scale=col_scale, sk_workspace=ctx.sk_workspace, stream=ctx.gemm_stream)
+    status = ctx.status.data_ptr()
+    _lib.call("tdist_ag_gemm_rows", _lib.dtype_code(a.dtype), shards, num_ranks, M_per_rank, workspace.data_ptr(), b.data_ptr(), b.stride(0),
+              c.data_ptr(), c.stride(0), b.shape[0], K, _lib.ptr(row_scale), _lib.ptr(col_scale), status, status + 8,
+              *_lib.workspace_args(ctx.sk_workspace), stream)
     if stream != current:
         torch.cuda.current_stream().wait_stream(ctx.gemm_stream)
 

@@ -306,10 +306,11 @@ def create_ag_group_gemm_intra_node_context(tp_pg, tensor_A, tensor_B, full_topk
 
 
 def _gather_and_multiply(a, b_nk, c, ctx, shards):
-    """With every rank's rows at hand: one launch brings them into the workspace and joins the row blocks across the rank
-    segments, the next multiplies them, on one stream. Against copies beside a flag-gated GEMM on 32 compute units less, in
-    blocks that end with their segment (8 x 1024 tokens by 4096, top 2 of 8 experts, 1792 columns): 339 -> 219 us. False
-    where the blocks cannot be joined (nothing has been launched then)."""
+    """With every rank's rows at hand: one launch joins the row blocks across the rank segments (and brings the rows into the
+    workspace where they lie too far apart to be read where they are), the next multiplies them, on one stream. Against
+    copies beside a flag-gated GEMM on 32 compute units less, in blocks that end with their segment (8 x 1024 tokens by 4096,
+    top 2 of 8 experts, 1792 columns): 339 -> 219 us with the gather. False where the blocks cannot be joined (nothing has been
+    launched then). The workspace is scratch here."""
     M_per_rank, K = a.shape
     workspace = ctx.workspace_tensors[ctx.rank]
     M = M_per_rank * ctx.num_ranks
@@ -317,14 +318,25 @@ def _gather_and_multiply(a, b_nk, c, ctx, shards):
     stream = current if ctx.group_gemm_stream is None else ctx.group_gemm_stream.cuda_stream
     if stream != current:
         ctx.group_gemm_stream.wait_stream(torch.cuda.current_stream())
+    row_bytes = K * a.element_size()
+    in_place = a.dtype in _GROUP_GEMM_ENTRY and _lib.shards_in_reach(shards, M_per_rank, row_bytes)
     status = ctx.status.data_ptr()
     blocks = joined_row_blocks(ctx.joined, ctx.sorted_topk_ids, ctx.aligned_expert_ids, ctx.aligned_num_tokens, ctx.BLOCK_M, ctx.full_num_tokens,
-                               b_nk.shape[0], b_nk.shape[1], K * a.element_size(), stream,
-                               gather=(workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * K * a.element_size(), status, status + 8))
+                               b_nk.shape[0], b_nk.shape[1], row_bytes, stream,
+                               gather=None if in_place else (workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * row_bytes, status, status + 8))
     if blocks is None:
         return False
-    _group_gemm(workspace[:M], None, 0, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, M, 0, None, ctx.rank,
-                sk_workspace=ctx.sk_workspace, stream=ctx.group_gemm_stream)
+    if in_place:
+        if b_nk.stride(2) != 1 or c.stride(1) != 1:
+            raise ValueError("A, B ([E, N, K]) and C need a contiguous last dimension")
+        assert b_nk.shape[2] == K and c.shape[1] == b_nk.shape[1]
+        _lib.call("tdist_group_gemm_rows", _lib.dtype_code(a.dtype), shards, ctx.num_ranks, M_per_rank, b_nk.data_ptr(), b_nk.stride(1),
+                  b_nk.stride(0), c.data_ptr(), c.stride(0), b_nk.shape[1], K, blocks.sorted_ids, blocks.experts, blocks.segments,
+                  blocks.padded, blocks.num_blocks, blocks.block_size, int(ctx.full_num_tokens), int(ctx.topk),
+                  status, status + 8, *_lib.workspace_args(ctx.sk_workspace), stream)
+    else:
+        _group_gemm(workspace[:M], None, 0, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, M, 0, None, ctx.rank,
+                    sk_workspace=ctx.sk_workspace, stream=ctx.group_gemm_stream)
     if stream != current:
         torch.cuda.current_stream().wait_stream(ctx.group_gemm_stream)
     return True
