@@ -38,6 +38,27 @@ def test_each_tile_with_ragged_k(cuda, switches, dtype, tile, pieces):
             assert torch.equal(c, want)
 
 
+# the ring of two, three, four or six stages (whether the tiles fill the chip twice chooses) filled in part, just filled and gone round,
+# with a whole and a ragged first K tile; pieces of one to four K tiles whose last is shorter
+@pytest.mark.parametrize("tile", [5, 6])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("M,N,pieces", [(130, 200, 1), (130, 200, 3), (130, 200, 7), (2300, 2200, 1)])
+def test_every_number_of_k_tiles(cuda, switches, dtype, tile, M, N, pieces):
+    from triton_dist import _lib
+    from triton_dist.kernels.amd import gated_gemm
+    announce("gemm small tile %d %s %dx%d pieces %d, K tiles 1 to 14" % (tile, dtype, M, N, pieces))
+    ws = _lib.new_split_k_workspace(cuda)
+    switches(_lib.TDIST_DEBUG_GEMM_TILE, tile)
+    switches(_lib.TDIST_DEBUG_GEMM_SPLIT_K, pieces)
+    esz = 1 if dtype == torch.float8_e4m3fn else 2
+    g = torch.Generator().manual_seed(M + pieces)
+    for k_bytes in [128 * n for n in range(1, 15)] + [128 * n + 48 for n in range(1, 14, 3)]:
+        a, b = poisoned(M, k_bytes // esz, dtype, g, cuda), poisoned(N, k_bytes // esz, dtype, g, cuda)
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+        gated_gemm(a, None, 0, b, c, None, 0, 0, 1, sk_workspace=ws)
+        assert torch.equal(c, (a.float() @ b.float().t()).to(torch.bfloat16)), k_bytes
+
+
 @pytest.mark.parametrize("coherent", [0, 1])
 def test_pieces_meet_in_the_l2_and_through_memory_alike(cuda, switches, coherent):
     from triton_dist import _lib

@@ -1882,13 +1882,14 @@ static void sk_attach(GemmParams& p, void* ws, int mode) {
 static double sk_handover_k_tiles(int bm, int bn) { return 2.0 + 6.0 * bm * bn / 65536.0; }
 
 // The GEMM on the small tiles (gemm_small.hip): the tile and the number of workgroups that share one along K, by an
-// estimate in microseconds (us = 0: this call does not qualify). The estimate is a fit to measured times (bf16 and e4m3 alike:
-// what a K tile of 128 bytes costs is its LDS traffic): a K tile takes 0.5 / 0.7 us while a compute unit has one workgroup
-// (64 / 128 rows) and 0.72 / 1.15 us with two, a round of workgroups 1.5 us beside, a launch 3 us, and handing pieces
-// over 2 us + 0.25 us per piece + their bytes at 2.7 TB/s.
-// (Pieces of at least kSmallMinPiece K tiles: shorter ones cost more than they save, and a short K's sums then run in the
-// order of the large tiles', bit for bit.)
-constexpr int kSmallMinPiece = 8;
+// estimate in microseconds (us = 0: this call does not qualify). The estimate is a fit to measured times (bf16 and e4m3 alike: what a
+// K tile of 128 bytes costs is its way into the LDS): a K tile takes 0.225 / 0.315 us while a compute unit has one workgroup (64 / 128
+// rows), or what its bytes take at 24 TB/s to all compute units, and 0.5 / 0.85 us a pair with two; a round of workgroups 1.5 us beside, a
+// launch 3 us, and handing pieces over 1.2 us + 0.25 / 0.6 us per piece + their bytes at 3 TB/s. Over 200 shapes the tile and number of
+// pieces taken, the large tiles among them, are 2 to 3 % behind the best on average.
+// (Pieces of at least kSmallMinPiece K tiles: shorter ones cost more than they save; 76 x 1568 x 1600 bf16 is 8.3 us in 4 pieces of 7
+// and 9.0 whole.)
+constexpr int kSmallMinPiece = 4;
 // Rows of a rank's slice in a scatter call come in whole multiples of this: every tile but the 256-row ones (which are
 // taken for multiples of their own only) then lies inside one slice.
 constexpr int kScatterRows = 128;
@@ -1916,9 +1917,10 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
       const int64_t units = tiles * pieces;
       const bool deep = units <= cus;
       double us = 3.0;
-      if (deep) us += per * (t == 0 ? 0.5 : 0.7) + 1.0;
-      else us += (double)ceil_div(units, 2 * cus) * (per * (t == 0 ? 0.72 : 1.15) + 1.5);
-      if (pieces > 1) us += 2.0 + 0.25 * pieces + (double)units * bm * bn * 4 / 2.7e6;
+      const double alone = t == 0 ? 0.225 : 0.315, stage_mb = (bm + bn) * 128 * 1e-6;
+      if (deep) us += per * std::max(alone, units * stage_mb / 24.0) + 1.0;
+      else us += (double)ceil_div(units, 2 * cus) * (per * (t == 0 ? 0.5 : 0.85) + 1.5);
+      if (pieces > 1) us += 1.2 + (t == 0 ? 0.25 : 0.6) * pieces + (double)units * bm * bn * 4 / 3.0e6;
       if (best.us == 0 || us < best.us) best = {t, pieces, per, deep, us};
     }
   }
@@ -2007,11 +2009,11 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   if (c.max_workgroups > 0 && c.max_workgroups < cap_wgs) cap_wgs = c.max_workgroups;
   struct TileChoice { int bm, bn; double eff; };
   constexpr int kNumChoices = kNumLargeTiles;
-  // (rates relative to the 256x256 tile, measured on 8192 x 6144 x 3584 bf16: 1425, 1255, 774, 1078 and 1178
-  // TFLOP/s; the 128x192 tile is entered below its multi-round rate because a tile's prologue and epilogue weigh
-  // more the smaller it is: one round of 256 of them takes 50.5 us on 4096 x 1536 x 4096 where 192 tiles of 256x128
-  // take 48.3 and 192 tiles of 128x256 53.1)
-  static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.88}, {128, 128, 0.54}, {128, 192, 0.65}, {128, 256, 0.8}};
+  // (rates relative to the 256x256 tile, fitted to the times of every tile on 45 ungated shapes of 340 to 15040 rows: the tile taken is
+  // 1 % behind the best on average with these, 6 % with the rates of one large problem, 0.88, 0.54, 0.65 and 0.8, that were here
+  // before: 2048 x 4304 x 3040 f16 79 -> 57 us, 7168 x 7128 x 3792 e4m3 241 -> 179; the smaller tiles fetch more operand bytes
+  // per product, and the 256x256 tile alone has an instance without gating code)
+  static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.70}, {128, 128, 0.48}, {128, 192, 0.62}, {128, 256, 0.70}};
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
   // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
@@ -2068,11 +2070,12 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // tiles by a margin.
   const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
   // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
-  // 256 x 256 tile takes 1.2 us, a launch with one tile's prologue and epilogue 8 us, handing over a split round 25 us more
-  // (10 of them in its estimate already)
-  // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 21 us on 512 of 64 x 128; 200 x 1536 x 4096 bf16:
-  // 26 -> 16 us; 4096 x 1536 x 4096 stays on the large tiles, 45 us against 63). Most calls that take them are told by a
-  // bound that needs no walk (a microsecond of host time less): every tile's work at its rate, no hand-over, no last round.
+  // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us, handing over a split round 25 us more
+  // (15 of them in its estimate already)
+  // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 14 us on 256 of 128 x 128; 200 x 1536 x 4096 bf16: 26 -> 12 us;
+  // 768 x 4952 x 2448 f16 37 -> 26, 2560 x 776 x 5936 68 -> 56; 2048 x 2104 x 4080 stays on the large tiles, 53 us against 70). Most
+  // calls that take them are told by a bound that needs no walk (a microsecond of host time less): every tile's work at its rate,
+  // no hand-over, no last round.
   const SmallPlan small = small_plan(c, esz, di.num_cus);
   if (small.us > 0 && forced_tile < 0) {
     double least = 0;
@@ -2082,7 +2085,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       const double cost = rounds * bm * bn / kChoices[t].eff * c.K * esz / 128.0;
       if (admissible(t) && (least == 0 || cost < least)) least = cost;
     }
-    if (small.us < 0.95 * (8.0 + least / 65536.0 * 1.2)) return run_small(c, elem, esz, small, di);
+    if (small.us < 0.95 * (6.0 + least / 65536.0 * 1.1)) return run_small(c, elem, esz, small, di);
   }
   int pick = 2, pick_split = -1;
   double whole = 0, split_last = 0;
@@ -2097,8 +2100,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
-      // (and 10 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
-      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / kChoices[t].eff) + 10.0 / 1.2 * 65536.0;
+      // (and 15 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
+      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / kChoices[t].eff) + 15.0 / 1.2 * 65536.0;
       if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
   }
@@ -2107,7 +2110,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   if (use_sk) pick = pick_split;
   const double best = use_sk ? split_last : whole;
   if (small.us > 0) {
-    const double large_us = 8.0 + best / 65536.0 * 1.2 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 15.0 : 0.0);
+    const double large_us = 6.0 + best / 65536.0 * 1.1 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
     if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < 0.95 * large_us)) return run_small(c, elem, esz, small, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,

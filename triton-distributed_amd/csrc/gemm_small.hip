@@ -2,14 +2,25 @@
 // prompts, narrow projections): tiles of 64 or 128 rows, two workgroups of four waves per compute unit, the K dimension
 // shared by several workgroups where the tiles alone are too few. Any K whose rows are a multiple of 16 bytes.
 //
-//  * A and B rows go to the LDS in K tiles of 128 bytes by LDS-DMA, three or four stages, one barrier per K tile; chunk c
+//  * A and B rows go to the LDS in K tiles of 128 bytes by LDS-DMA, two to six stages, one barrier per K tile; chunk c
 //    of row r sits at c ^ ((r >> 1) & 7), so that the 16 rows an operand read touches spread over the banks;
+//  * a wave reads the operands of its next products (the other half of the K tile, or the next tile) before the products at
+//    hand, and a load takes a scalar base and a lane offset that never changes: with one wave per SIMD nothing else hides an LDS
+//    read's latency or an address instruction;
+//  * a K that is no whole number of K tiles has the ragged one first (its lanes in front of the row fetch zeros), so that only
+//    loads outside the loop need to know;
+//  * what bounds it: the loads' way into the LDS (64 bytes a clock and compute unit; 24 KB a K tile of 64 x 128 in 0.222 us, 108 GB/s, of
+//    128 x 128 32 KB in 0.315 us), at short K the launch and the first trip to memory. Before operands were read ahead and loads went
+//    out one by one between products a K tile took 0.505 and 0.655 us whether its rows came from memory or from the L2: 200 x 1536 x 4096
+//    16.0 -> 12.1 us, 1024 x 4096 x 4096 47.6 -> 29.6, e4m3 64 x 1536 x 8192 33.7 -> 17.5;
 //  * v_mfma 16x16x32 (16-bit) / 16x16x128 (e4m3), D^T = B * A^T, so that a lane holds 4 consecutive columns;
 //  * with `splits` > 1 every workgroup leaves its fp32 accumulators in the workspace and bumps its tile's counter; the last
 //    to arrive adds the pieces up in their K order, so the result does not depend on timing and nobody waits. The pieces
 //    of a tile meet in one XCD's L2 where workgroup i is known to run on XCD i % 8 (written through to memory they cost
 //    12 us for 256 tiles of 64 x 128).
 #include "gemm_small.h"
+
+#include <type_traits>
 
 namespace tdist {
 
@@ -75,17 +86,15 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   const int tm = tile % tiles_m, tn = tile / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
   const int k_tiles = (p.k_bytes + kSmallKB - 1) / kSmallKB;
-  const int tail = p.k_bytes % kSmallKB;
+  const int back = k_tiles * kSmallKB - p.k_bytes;   // bytes of the first K tile in front of the rows
   int kt0 = piece * p.tiles_per_split, kt1 = min(kt0 + p.tiles_per_split, k_tiles), splits = p.splits;
 
   // DMA: instruction i of a wave brings rows (i * 4 + wave) * 8 .. + 7, lane = row * 8 + chunk position
   uint32_t aoff[C::kAInstr], boff[C::kBInstr];
-  int chunk_a[C::kAInstr], chunk_b[C::kBInstr];
 #pragma unroll
   for (int i = 0; i < C::kAInstr; ++i) {
     const int r = (i * 4 + wave) * 8 + (lane >> 3);
-    chunk_a[i] = (lane & 7) ^ ((r >> 1) & 7);
-    aoff[i] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.lda_b + chunk_a[i] * 16;
+    aoff[i] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.lda_b + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
   }
   if constexpr (kShards) {
     // rows in shards: the tile's few shards one after the other (their offsets by scalar loads), each for the rows from its first on
@@ -94,82 +103,150 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
       const uint32_t off = p.shards.off[s] - (uint32_t)first * (uint32_t)p.lda_b;
 #pragma unroll
       for (int i = 0; i < C::kAInstr; ++i) {
-        const int row = min(m0 + (i * 4 + wave) * 8 + (lane >> 3), p.M - 1);
-        if (row >= first) aoff[i] = off + (uint32_t)row * (uint32_t)p.lda_b + chunk_a[i] * 16;
+        const int r = (i * 4 + wave) * 8 + (lane >> 3), row = min(m0 + r, p.M - 1);
+        if (row >= first) aoff[i] = off + (uint32_t)row * (uint32_t)p.lda_b + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
       }
     }
   }
 #pragma unroll
   for (int i = 0; i < C::kBInstr; ++i) {
     const int r = (i * 4 + wave) * 8 + (lane >> 3);
-    chunk_b[i] = (lane & 7) ^ ((r >> 1) & 7);
-    boff[i] = (uint32_t)min(n0 + r, p.N - 1) * (uint32_t)p.ldb_b + chunk_b[i] * 16;
+    boff[i] = (uint32_t)min(n0 + r, p.N - 1) * (uint32_t)p.ldb_b + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
   }
-  auto dma = [](const unsigned char* src, lds_u8 dst) {
-    __builtin_amdgcn_global_load_lds((const TDIST_AS1 void*)src, (TDIST_AS3 void*)dst, 16, 0, 0);
+  // one load: scalar base + lane offset, M0 the LDS address (a register the compiler does not allocate, and nothing else here uses)
+  auto dma = [](const unsigned char* base, uint32_t off, lds_u8 dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"((uint32_t)(uintptr_t)dst) : "memory");
   };
-  auto issue = [&](int kt) {
-    lds_u8 const st = ring + (kt - kt0) % NST * C::kStageBytes + wave * 1024;
-    const unsigned char* a = p.A + (int64_t)kt * kSmallKB;
-    const unsigned char* b = p.B + (int64_t)kt * kSmallKB;
-    const bool cut = tail != 0 && kt == k_tiles - 1;
+  const uint32_t dma_lds = (uint32_t)(uintptr_t)ring + wave * 1024;
+  // load n of K tile kt into the stage at `stage` bytes
+  auto issue_one = [&](const unsigned char* a, const unsigned char* b, int stage, auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    lds_u8 const st = (lds_u8)(uintptr_t)(dma_lds + stage);
+    if constexpr (n < C::kAInstr) dma(a, aoff[n], st + n * 4096);
+    else dma(b, boff[n - C::kAInstr], st + BM * kSmallKB + (n - C::kAInstr) * 4096);
+  };
+  auto issue = [&](int kt, int stage) {
+    const int64_t at = (int64_t)kt * kSmallKB - back;
+    static_for<C::kLoads>([&](auto n_c) { issue_one(p.A + at, p.B + at, stage, n_c); });
+  };
+  // the first K tile where it is ragged: lanes in front of the row read zeros, the others what they read in any tile
+  auto issue_ragged = [&](int stage) {
+    lds_u8 const st = (lds_u8)(uintptr_t)(dma_lds + stage);
+    auto one = [&](const unsigned char* rows, uint32_t off, int r, lds_u8 dst) {
+      const unsigned char* src = rows - back + off;
+      if ((((lane & 7) ^ ((r >> 1) & 7)) << 4) < back) src = kZeroChunk16;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"((uint32_t)(uintptr_t)dst) : "memory");
+    };
 #pragma unroll
-    for (int i = 0; i < C::kAInstr; ++i) {
-      const unsigned char* src = a + aoff[i];
-      if (cut && chunk_a[i] * 16 >= tail) src = kZeroChunk16;
-      dma(src, st + i * 4096);
-    }
+    for (int i = 0; i < C::kAInstr; ++i) one(p.A, aoff[i], (i * 4 + wave) * 8 + (lane >> 3), st + i * 4096);
 #pragma unroll
-    for (int i = 0; i < C::kBInstr; ++i) {
-      const unsigned char* src = b + boff[i];
-      if (cut && chunk_b[i] * 16 >= tail) src = kZeroChunk16;
-      dma(src, st + BM * kSmallKB + i * 4096);
-    }
+    for (int i = 0; i < C::kBInstr; ++i) one(p.B, boff[i], (i * 4 + wave) * 8 + (lane >> 3), st + BM * kSmallKB + i * 4096);
   };
 
   float4v acc[C::kTN][C::kTM];
-  // operand reads: row x of block i, chunks of step s and lane group g
+  // operand reads: row x of block i, the chunks of a step (of 16-bit types; e4m3: chunks g and g + 4, the four groups of a read on
+  // consecutive chunks, and the order of gemm.hip's sums) and lane group g, relative to the stage; blocks are 16 rows apart, which
+  // leaves the swizzle alone
   const int a_row = wm * (BM / 2) + x, b_row = wn * (BN / 2) + x;
-  auto frag_at = [&](lds_u8 rows, int row, int step) -> typename E::frag {
-    const int sw = (row >> 1) & 7;   // (blocks are 16 rows apart: the same for all of them)
+  int a_at[2], b_at[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    a_at[c] = a_row * kSmallKB + (((4 * c + g) ^ ((a_row >> 1) & 7)) << 4);
+    b_at[c] = BM * kSmallKB + b_row * kSmallKB + (((4 * c + g) ^ ((b_row >> 1) & 7)) << 4);
+  }
+  auto read = [&](int stage, const int (&at)[2], int step, int i) -> typename E::frag {
     if constexpr (E::kVecs == 1) {
-      return *(const TDIST_AS3 int4v*)(rows + row * kSmallKB + (((step * 4 + g) ^ sw) << 4));
+      return *(const TDIST_AS3 int4v*)(ring + stage + at[step] + i * 16 * kSmallKB);
     } else {
-      // (chunks g and g + 4: the four groups of a read on consecutive chunks, and the order of gemm.hip's sums)
-      const int4v lo = *(const TDIST_AS3 int4v*)(rows + row * kSmallKB + ((g ^ sw) << 4));
-      const int4v hi = *(const TDIST_AS3 int4v*)(rows + row * kSmallKB + (((g + 4) ^ sw) << 4));
+      const int4v lo = *(const TDIST_AS3 int4v*)(ring + stage + at[0] + i * 16 * kSmallKB);
+      const int4v hi = *(const TDIST_AS3 int4v*)(ring + stage + at[1] + i * 16 * kSmallKB);
       return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   };
+  auto after = [](int stage) { return stage + C::kStageBytes == C::kLdsBytes ? 0 : stage + C::kStageBytes; };
 
   for (;;) {
+    // (nothing is outstanding here, and the compiler is told so: on the way round it would count loads of the other pieces, and
+    // then wait for every load into the LDS at the first use of a register in the loop below)
+    __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
     for (int j = 0; j < C::kTN; ++j)
 #pragma unroll
       for (int i = 0; i < C::kTM; ++i) acc[j][i] = float4v{0.f, 0.f, 0.f, 0.f};
     const int n_kt = kt1 - kt0;
 #pragma unroll
-    for (int i = 0; i < NST - 1; ++i)
-      if (i < n_kt) issue(kt0 + i);
-    for (int k = 0; k < n_kt; ++k) {
-      // this K tile has arrived (the younger ones may be on their way), and everyone is done with the one before
-      if (k + NST - 2 < n_kt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * C::kLoads) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (k + NST - 1 < n_kt) issue(kt0 + k + NST - 1);
-      lds_u8 const st = ring + k % NST * C::kStageBytes;
-#pragma unroll
-      for (int s = 0; s < E::kSteps; ++s) {
-        typename E::frag a[C::kTM], b[C::kTN];
-#pragma unroll
-        for (int i = 0; i < C::kTM; ++i) a[i] = frag_at(st, a_row + i * 16, s);
-#pragma unroll
-        for (int j = 0; j < C::kTN; ++j) b[j] = frag_at(st + BM * kSmallKB, b_row + j * 16, s);
-#pragma unroll
-        for (int j = 0; j < C::kTN; ++j)
-#pragma unroll
-          for (int i = 0; i < C::kTM; ++i) acc[j][i] = E::mma(b[j], a[i], acc[j][i]);
-      }
+    for (int i = 0; i < NST - 1; ++i) {
+      if (i >= n_kt) break;
+      if (back != 0 && kt0 + i == 0) issue_ragged(0);
+      else issue(kt0 + i, i * C::kStageBytes);
     }
+    // all but the `younger` youngest K tiles have arrived
+    auto wait_tiles = [&](int younger) {
+      static_for<NST - 1>([&](auto n_c) {
+        constexpr int n = NST - 2 - decltype(n_c)::value;
+        if (younger == n || (n == NST - 2 && younger > n)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n * C::kLoads) : "memory");
+      });
+    };
+    // everyone has read what they read before this, and everyone's loads that this wave has waited for have arrived
+    auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    // A tile's products come in two halves, 16-bit types by K and e4m3 by columns. Between a half's products the operands of the
+    // next half are read and, one by one, the loads of tile k + NST - 1 go out: a wave issues in order, and in a burst each
+    // would hold the products up until the one before it is through (64 x 128 bf16: 0.31 us a K tile in a burst).
+    // Behind the last tile whatever a stage holds is read, and not used: with the reads conditional the compiler would wait for
+    // them where the operands before them are used.
+    constexpr int kHalves = E::kSteps == 2 ? 1 : 2;             // column halves
+    constexpr int kCols = C::kTN / kHalves, kProducts = C::kTM * kCols;
+    constexpr int kFirstLoads = NST > 2 ? C::kLoads / 2 : C::kLoads;   // (two stages: the tile is waited for in this very trip)
+    typename E::frag a[3 - kHalves][C::kTM], b[2][kCols];       // (e4m3: the same rows for both halves)
+    int stage = 0, free_stage = (NST - 1) * C::kStageBytes;   // tile k's stage, and the one that tile k + NST - 1 goes to
+    auto half = [&](auto h_c, auto load_c, const unsigned char* ka, const unsigned char* kb, int load_stage) {
+      constexpr int h = decltype(h_c)::value;
+      constexpr int kLoad0 = h == 0 ? 0 : kFirstLoads, kLoadN = decltype(load_c)::value ? (h == 0 ? kFirstLoads : C::kLoads - kFirstLoads) : 0;
+      static_for<kProducts>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value, kNow = m * kLoadN / kProducts, kNext = (m + 1) * kLoadN / kProducts;
+        if constexpr (kHalves == 1) {
+          if constexpr (m < C::kTM) a[1 - h][m] = read(stage, a_at, 1 - h, m);
+          else if constexpr (m < C::kTM + kCols) b[1 - h][m - C::kTM] = read(stage, b_at, 1 - h, m - C::kTM);
+          constexpr int j = m / C::kTM, i = m % C::kTM;
+          acc[j][i] = E::mma(b[h][j], a[h][i], acc[j][i]);
+        } else {
+          // row by row: the next tile's row takes a row's place as soon as its products are out
+          if constexpr (m < kCols) b[1 - h][m] = read(stage, b_at, 0, (1 - h) * kCols + m);
+          constexpr int i = m / kCols, j = m % kCols;
+          acc[h * kCols + j][i] = E::mma(b[h][j], a[0][i], acc[h * kCols + j][i]);
+          if constexpr (h == 1 && j == kCols - 1) a[0][i] = read(stage, a_at, 0, i);
+        }
+        static_for<kNext - kNow>([&](auto u_c) { issue_one(ka, kb, load_stage, std::integral_constant<int, kLoad0 + kNow + decltype(u_c)::value>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    static_assert(kHalves == 2 || C::kTM + kCols <= kProducts, "a read per product");
+    constexpr std::integral_constant<int, 0> zero{};
+    constexpr std::integral_constant<int, 1> one{};
+    auto tile_of = [&](int k, auto load_c) {
+      constexpr bool kLoad = decltype(load_c)::value;
+      const int64_t at = (int64_t)(kt0 + k + NST - 1) * kSmallKB - back;
+      const unsigned char *ka = p.A + at, *kb = p.B + at;
+      const int load_stage = free_stage;
+      half(zero, load_c, ka, kb, load_stage);
+      // tile k + 1 has arrived
+      if constexpr (kLoad) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NST > 2 ? (NST - 3) * C::kLoads + kFirstLoads : 0) : "memory");
+      else wait_tiles(n_kt - 2 - k);
+      meet();
+      free_stage = stage;
+      stage = after(stage);
+      half(one, load_c, ka, kb, load_stage);
+    };
+    wait_tiles(n_kt - 1);
+    meet();
+#pragma unroll
+    for (int i = 0; i < C::kTM; ++i) a[0][i] = read(0, a_at, 0, i);
+#pragma unroll
+    for (int j = 0; j < kCols; ++j) b[0][j] = read(0, b_at, 0, j);
+    __builtin_amdgcn_sched_barrier(0);
+    int k = 0;
+    for (; k + NST - 1 < n_kt; ++k) tile_of(k, std::true_type{});
+    for (; k < n_kt; ++k) tile_of(k, std::false_type{});
     __syncthreads();
     if (splits == 1) break;
 
@@ -206,23 +283,42 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     }
     if (p.l2_local) asm volatile("buffer_inv sc0" ::: "memory");
     else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    // added in the pieces' order, eight accumulators of three other pieces in flight at a time; this workgroup's own piece is still
+    // in its registers
+    constexpr int kBatch = 3;
+    static_assert(kAccs % 8 == 0, "eight at a time");
+    static_for<kAccs / 8>([&](auto part_c) {
+      constexpr int u0 = decltype(part_c)::value * 8;
+      float4v total[8];
+      auto add_own = [&]() {
 #pragma unroll
-    for (int u = 0; u < kAccs; ++u) acc[u / C::kTM][u % C::kTM] = float4v{0.f, 0.f, 0.f, 0.f};
-    // two pieces in flight at a time, added in order
-    for (int z = 0; z < splits; z += 2) {
-      const float4v* src = slots + (int64_t)z * (kAccs * 256);
-      const float4v* src2 = slots + (int64_t)min(z + 1, splits - 1) * (kAccs * 256);
-      float4v v[2][kAccs];
+        for (int u = 0; u < 8; ++u) total[u] += acc[(u0 + u) / C::kTM][(u0 + u) % C::kTM];
+      };
 #pragma unroll
-      for (int u = 0; u < kAccs; ++u) v[0][u] = src[u * 256], v[1][u] = src2[u * 256];
+      for (int u = 0; u < 8; ++u) total[u] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int z0 = 0; z0 < splits - 1; z0 += kBatch) {   // z: the other pieces in order, own one left out
+        float4v v[kBatch][8];
 #pragma unroll
-      for (int u = 0; u < kAccs; ++u)
+        for (int w = 0; w < kBatch; ++w) {
+          const int z = min(z0 + w, splits - 2);
+          const float4v* src = slots + (int64_t)(z + (z >= piece)) * (kAccs * 256) + u0 * 256;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[u / C::kTM][u % C::kTM][e] += v[0][u][e];
-          if (z + 1 < splits) acc[u / C::kTM][u % C::kTM][e] += v[1][u][e];
+          for (int u = 0; u < 8; ++u) v[w][u] = src[u * 256];
         }
-    }
+#pragma unroll
+        for (int w = 0; w < kBatch; ++w) {
+          if (z0 + w == piece) add_own();
+          if (z0 + w < splits - 1) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) total[u] += v[w][u];
+          }
+        }
+      }
+      // (own the last, and not met above as the place behind the last batch)
+      if (piece == splits - 1 && (splits - 1) % kBatch == 0) add_own();
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc[(u0 + u) / C::kTM][(u0 + u) % C::kTM] = total[u];
+    });
     break;
   }
 
