@@ -141,7 +141,9 @@ def check(code):
 
 def call(name, *args):
     """Calls an entry point that returns a tdist_status and raises TdistError on failure."""
-    check(getattr(load(), name)(*args))
+    code = getattr(_lib or load(), name)(*args)
+    if code != TDIST_OK:
+        raise TdistError(code, last_error())
 
 
 class debug_switch:
@@ -260,7 +262,7 @@ def zeros_per_stream(pool, n, least, dtype, device):
     import torch
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(int(n), 1), dtype=dtype, device=device).zero_()
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, torch._C._cuda_getCurrentRawStream(device.index))
     buf = pool.get(key)
     if buf is None or buf.numel() < n:
         buf = pool[key] = torch.zeros(max(int(n), least), dtype=dtype, device=device)

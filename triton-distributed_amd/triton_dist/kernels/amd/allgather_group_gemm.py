@@ -68,8 +68,8 @@ def sort_topk_ids_align_block_size(
         plan = _ALIGN_PLANS[key] = (ws_bytes, at, tuple(starts), sizes)
     ws_bytes, n_flat, starts, sizes = plan
     flat = torch.empty(n_flat, dtype=torch.int32, device=dev)
-    sorted_ids, expert_ids, block_barrier_ids, rank_block_num, num_tokens_post_pad = (
-        flat[a:a + n] for a, n in zip(starts, sizes))
+    sorted_ids, expert_ids, block_barrier_ids, rank_block_num, num_tokens_post_pad = [
+        flat[a:a + n] for a, n in zip(starts, sizes)]
     base = flat.data_ptr()
     ids_ptr, ids_int64 = topk_ids.data_ptr(), 1 if topk_ids.dtype == torch.int64 else 0
 
@@ -78,13 +78,13 @@ def sort_topk_ids_align_block_size(
         # (sorted_ids.fill_(numel) of the reference, :103, is done inside the call)
         _lib.call("tdist_moe_align_block_size", ids_ptr, ids_int64, n_total, num_experts, num_ranks, n_per, block_size,
                   base + 4 * starts[0], sizes[0], base + 4 * starts[1], base + 4 * starts[2], base + 4 * starts[3],
-                  base + 4 * starts[4], workspace.data_ptr(), ws_bytes, stream.cuda_stream)
+                  base + 4 * starts[4], workspace.data_ptr(), ws_bytes, stream)
 
     if moe_stream is None:
-        launch(torch.cuda.current_stream())      # no stream switch, event or allocator bookkeeping to pay for
+        launch(_lib.stream_ptr())      # no stream switch, event, Stream object or allocator bookkeeping to pay for
     else:
         with torch.cuda.stream(moe_stream):
-            launch(moe_stream)
+            launch(moe_stream.cuda_stream)
         torch.cuda.current_stream().wait_stream(moe_stream)
     return (
         sorted_ids,

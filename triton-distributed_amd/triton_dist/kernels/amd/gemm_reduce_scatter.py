@@ -109,13 +109,13 @@ def matmul_fuse_scatter(a, b, scatter_bufs_ptr, rank, num_ranks, transpose_weigh
 
 def ring_reduce_after_scatter(rank, num_ranks, scatter_out, stream):
     """Sum of the num_ranks slices of ``scatter_out`` [M, N] in the order rank+1, rank+2, ... (reference
-    :264-286 / kernel :246-258), accumulated in fp32."""
+    :264-286 / kernel :246-258), accumulated in fp32. ``stream`` None: the current one."""
     M, N = scatter_out.shape
     assert scatter_out.is_contiguous()
     M_per_rank = M // num_ranks
     output = torch.empty((M_per_rank, N), dtype=scatter_out.dtype, device=scatter_out.device)
     _lib.call("tdist_reduce_slices", scatter_out.data_ptr(), M_per_rank * N, num_ranks, (rank + 1) % num_ranks,
-              M_per_rank * N, output.data_ptr(), _lib.dtype_code(scatter_out.dtype), stream.cuda_stream)
+              M_per_rank * N, output.data_ptr(), _lib.dtype_code(scatter_out.dtype), _lib.stream_ptr(stream))
     return output
 
 
@@ -135,13 +135,10 @@ def gemm_rs_intra_node_op(a, b, output_dtype, rank, num_ranks, scatter_bufs, sca
     if scatter_bufs[rank].dtype != partial_dtype:
         raise TypeError("the scatter buffers hold the GEMM's input dtype (reference :217-218; bf16 for e4m3 inputs): "
                         "ctx was created for %s, inputs are %s" % (scatter_bufs[rank].dtype, a.dtype))
-    current_stream = torch.cuda.current_stream()
+    own = scatter_bufs[rank]
     matmul_fuse_scatter(a, b, scatter_bufs_ptr, rank, num_ranks, transpose_weight=transpose_weight,
-                        ldc=scatter_bufs[rank].stride(0), stream=current_stream, sk_workspace=sk_workspace,
-                        row_scale=row_scale, col_scale=col_scale)
-    scatter_out = scatter_bufs[rank][:M]
-    output = ring_reduce_after_scatter(rank, num_ranks, scatter_out, current_stream)
-    return output
+                        ldc=own.stride(0), sk_workspace=sk_workspace, row_scale=row_scale, col_scale=col_scale)
+    return ring_reduce_after_scatter(rank, num_ranks, own if own.shape[0] == M else own[:M], None)
 
 
 def gemm_rs_intra_node(a, b, ctx, *, row_scale=None, col_scale=None):
