@@ -40,6 +40,12 @@ def test_dispatch_from_few_ids(cuda, wide, T, topk, G, W, H):
         assert (recv[d * max_m + hi - lo:(d + 1) * max_m] == 0xAB).all()
 
 
+# experts per rank that are one, odd, and as many as there can be: the rank of an expert is found by a multiplication
+@pytest.mark.parametrize("T,topk,G,W", [(37, 6, 21, 7), (37, 6, 21, 21), (5, 8, 381, 3), (5, 8, 4096, 1), (9, 4, 4095, 13)])
+def test_dispatch_with_any_number_of_experts_per_rank(cuda, T, topk, G, W):
+    test_dispatch_from_few_ids(cuda, False, T, topk, G, W, 1024)
+
+
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("R,T,topk,E,BS", [(8, 1, 8, 256, 128), (8, 125, 8, 256, 128), (1, 3, 2, 16, 256), (8, 2, 2, 64, 1024), (4, 1031, 3, 100, 64)])
 def test_align_sort_with_more_padding_than_entries(cuda, dtype, R, T, topk, E, BS):

@@ -681,7 +681,10 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(const unsigned
 // moe_dispatch_tokens_kernel. The window-0 wave of a token counts and ranks that token's ids.
 // Few tokens: windows of `vecs` < 8 KB, so that a row is shared by several waves and the rows by more workgroups. What 16
 // whole rows per workgroup cost a decode step of 128 tokens x 8 copies of 7168 B is eight compute units storing 7.3 MB:
-// 14.5 us, against 12.2 us with eight waves to a row (64 workgroups; what is left is the chain ids, counts, scan, stores).
+// 14.5 us, against 12.2 us with eight waves to a row (64 workgroups; twice as many: the same, four times: 18 for 13 us at 600
+// tokens). Up to the scan the launch takes 4.3 us; behind it, instructions and waits in a row are what counts, not bytes: 8.8 us
+// (from 12.1) since a token's scale is asked for at the start, the copies' rows and windows are the wave's (scalar branches
+// instead of eight tests a lane and copy) and the search among the workgroup's own entries has its reads in flight together.
 // 64-bit ids are read as they are (a conversion of 1024 of them in front: 3 us and a launch).
 constexpr int kFdWaves = 16, kFdThreads = kFdWaves * 64;
 constexpr int64_t kFusedDispatchMaxIds = 65536;
@@ -691,8 +694,8 @@ constexpr int64_t kFusedDispatchMaxIds = 65536;
 template <bool kVec16, bool kFew, bool kWide>
 __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
     const unsigned char* __restrict__ tokens, int64_t row_bytes, const float* __restrict__ scales,
-    const int32_t* __restrict__ ids, int topk, int64_t n_tokens, int G, int nbits, int W, int Er, int max_m, int windows,
-    int few_vecs, unsigned char* __restrict__ slot_rows, float* __restrict__ slot_scales, int32_t* __restrict__ splits_out,
+    const int32_t* __restrict__ ids, int topk, int64_t n_tokens, int G, int nbits, int W, int Er, uint32_t er_magic, int max_m,
+    int windows, int few_vecs, unsigned char* __restrict__ slot_rows, float* __restrict__ slot_scales, int32_t* __restrict__ splits_out,
     int32_t* __restrict__ splits, int32_t* __restrict__ cumsum, int32_t* __restrict__ scatter_idx,
     int32_t* __restrict__ gather_idx) {
   const int vecs = kFew ? few_vecs : 8;   // 16-byte loads per lane and window
@@ -703,9 +706,9 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   int32_t* const s_own = s_fd + G;
   int32_t* const s_behind = s_fd + 2 * G;
   int32_t* const s_start = s_fd + 3 * G;
-  int32_t* const s_ids = s_start + ((G + 1 + 3) & ~3);
+  int32_t* const s_ids = s_fd + 4 * G + 4;
   __shared__ int32_t s_part[kFdWaves];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int tokens_per_block = kFdWaves / windows;
   const int64_t unit = (int64_t)blockIdx.x * kFdWaves + wave;
   const int64_t t = unit / windows;
@@ -715,10 +718,12 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   const int64_t n = n_tokens * topk;
   const int own_n = tokens_per_block * topk;
   const int64_t own_lo = (int64_t)blockIdx.x * own_n, own_hi = own_lo + own_n;
-  const int own_f = (wave / windows) * topk + lane;   // this lane's entry among the workgroup's own, in flat order
+  const int own_first = (wave / windows) * topk;   // the token's first entry among the workgroup's own, in flat order
+  const int own_f = own_first + lane;              // and this lane's
   int e = -1;
   if (live && lane < topk) e = ids[(t * topk + lane) << (kWide ? 1 : 0)];
-  if (e < 0 || e >= G) e = -1;
+  float my_scale = 0.f;   // (asked for here: a load in front of the copies would hold them up for a trip to memory)
+  if (scales && live && win == 0) my_scale = scales[t];
   constexpr int kBatch = 8;
   const int64_t n_vec = (n + 3) / 4;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(ids) & 15u) == 0;
@@ -783,6 +788,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
     }
   }
   for (int g = threadIdx.x; g < 3 * G; g += kFdThreads) s_fd[g] = 0;
+  if ((uint32_t)e >= (uint32_t)G) e = -1;
   if (win == 0 && lane < topk) s_ids[own_f] = e;
   if (threadIdx.x < 4) s_ids[own_n + threadIdx.x] = -1;
   __syncthreads();
@@ -831,40 +837,44 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   // range, and the workgroup's own entries before this one in flat order; then its slot row
   int32_t my_dst = -1;
   if (e >= 0) {
+    // (the loop's bounds are the wave's, so that its reads go out several at a time)
     int32_t earlier = 0;
-    for (int f = 0; f < own_f; f += 4) {
+    const int32_t start = s_start[e], before = s_before[e];
+    const int d = er_magic != 0 ? (int)__umulhi((uint32_t)e, er_magic) : e;   // e / Er
+    const int32_t slot_start = s_start[d * Er];
+#pragma unroll 4
+    for (int f = 0; f < own_first + topk; f += 4) {
       const int4v o = *(const int4v*)(s_ids + f);
 #pragma unroll
       for (int j = 0; j < 4; ++j) earlier += (f + j < own_f && o[j] == e) ? 1 : 0;
     }
-    const int32_t p = s_start[e] + s_before[e] + earlier;
+    const int32_t p = start + before + earlier;
     if (win == 0) {
       scatter_idx[t * topk + lane] = p;
       gather_idx[p] = (int32_t)t;
     }
-    const int d = e / Er;
-    const int32_t in_slot = p - s_start[d * Er];
+    const int32_t in_slot = p - slot_start;
     if (in_slot < max_m) my_dst = d * max_m + in_slot;
-    if (win == 0 && my_dst >= 0 && scales) slot_scales[my_dst] = scales[t];
+    if (win == 0 && my_dst >= 0 && scales) slot_scales[my_dst] = my_scale;
   } else if (lane < topk && win == 0) {
     scatter_idx[t * topk + lane] = -1;
   }
-  // 5. the copies
+  // 5. the copies: row and window of a copy are the wave's, not the lane's (scalar branches, one address a lane)
   if (kVec16) {
     for (int k = 0; k < topk; ++k) {
-      const int32_t dst_row = __shfl(my_dst, k);
+      const int32_t dst_row = __builtin_amdgcn_readlane(my_dst, k);
       if (dst_row < 0) continue;
-      int4v* d16 = (int4v*)(slot_rows + (int64_t)dst_row * row_bytes);
+      int4v* const d16 = (int4v*)(slot_rows + (int64_t)dst_row * row_bytes) + base;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int c = base + j * 64 + lane;
-        if ((!kFew || j < vecs) && c < n16) __builtin_nontemporal_store(v[j], d16 + c);
+        if (kFew && j >= vecs) break;
+        if (lane < n16 - base - j * 64) __builtin_nontemporal_store(v[j], d16 + j * 64 + lane);
       }
     }
   } else {
     const unsigned char* src = tokens + t * row_bytes;
     for (int k = 0; k < topk; ++k) {
-      const int32_t dst_row = __shfl(my_dst, k);
+      const int32_t dst_row = __builtin_amdgcn_readlane(my_dst, k);
       if (dst_row < 0) continue;
       unsigned char* dst = slot_rows + (int64_t)dst_row * row_bytes;
       for (int64_t c = (int64_t)base * 16 + lane; c < row_bytes && c < ((int64_t)base + vecs * 64) * 16; c += 64) dst[c] = src[c];
@@ -1792,6 +1802,8 @@ static int dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const
     windows *= 2;
     vecs = (int)ceil_div(row_bytes, (int64_t)windows * 1024);
   }
+  // (expert / experts_per_rank by a multiplication: exact, both are at most kMoeMaxExperts; 0: the expert itself)
+  const uint32_t er_magic = experts_per_rank == 1 ? 0u : (uint32_t)(((1ull << 32) + experts_per_rank - 1) / experts_per_rank);
   const int64_t units = (n_tokens > 0 ? n_tokens : 1) * windows;
   const int64_t blocks = ceil_div(units, kFdWaves);
   const bool vec = (row_bytes % 16 == 0) && aligned16(tokens) && aligned16(slot_rows);
@@ -1808,7 +1820,7 @@ static int dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kFdThreads), (size_t)lds, (hipStream_t)stream,
                      (const unsigned char*)tokens, row_bytes, token_scales, ids, topk, n_tokens, G, id_bits(G), world_size,
-                     experts_per_rank, max_m, windows, vecs, (unsigned char*)slot_rows, slot_scales, splits_out, splits, cumsum,
+                     experts_per_rank, er_magic, max_m, windows, vecs, (unsigned char*)slot_rows, slot_scales, splits_out, splits, cumsum,
                      scatter_idx, gather_idx);
   return launch_status(who);
 }
