@@ -61,6 +61,15 @@ def test_align_sort_with_more_padding_than_entries(cuda, dtype, R, T, topk, E, B
     assert torch.equal(got[3].cpu(), want[3])
 
 
+# one and two passes of 64 entries per wave with many entries of one group in each (a wave's count of a group fills its byte
+# up to 128), four groups to a step and a remainder, as many groups as there can be, blocks of one row and of more than 32768
+@pytest.mark.parametrize("R,T,topk,E,BS", [(1, 600, 1, 1, 128), (1, 40000, 1, 2, 1), (2, 20001, 1, 1, 48), (3, 700, 2, 3, 5), (16, 130, 2, 256, 16),
+                                           (5, 97, 3, 819, 3), (2, 11, 2, 7, 40000)])
+def test_align_sort_counts(cuda, R, T, topk, E, BS):
+    test_align_sort_with_more_padding_than_entries(cuda, torch.int32, R, T, topk, E, BS)
+    test_align_sort_with_more_padding_than_entries(cuda, torch.int64, R, T, topk, E, BS)
+
+
 # 64-bit ids: both block sizes of the one launch, remainders of a vector of four, ids that are not 16-byte aligned, not
 # contiguous, out of range, and more of them than the one launch takes
 @pytest.mark.parametrize("T,topk,G,how", [(1, 1, 1, ""), (1, 8, 256, ""), (63, 3, 7, ""), (4096, 8, 256, ""), (4097, 8, 64, ""), (8192, 8, 64, ""), (9000, 8, 64, ""),

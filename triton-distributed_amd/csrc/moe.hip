@@ -1211,31 +1211,36 @@ __global__ __launch_bounds__(kPlaceThreads) void moe_align_place_kernel(
 // are shared out among the blocks, groups in turn; block 0 writes the blocks per segment and the padded total.
 // Many groups of few entries: the padding is the larger part (1000 tokens x 8, 256 experts x 8 segments, blocks of 128:
 // 260 000 positions for 8000 entries), so the launch has a block per kAlignFillPerBlock positions even where the entries
-// alone need fewer: blocks beyond the entries count like the others and only fill (16 blocks 20.9 us, 131 blocks 12.1).
-constexpr int kAlignFillPerBlock = 2048;
-template <int kThreads, int kPerWave, bool kIds64>
-__global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
+// alone need fewer: blocks beyond the entries count like the others and only fill (66 blocks 7.8 us, 131 6.8, 256 6.7).
+// What bounds it: two trips to memory and the work per group, of which there are thousands. The eight waves' counts of a
+// group are the bytes of one 64-bit word (a wave has at most 128 entries), so a group is 20 bytes to clear, to add up (four
+// groups a step, the bytes of a word by a sum of absolute differences) and to look up, and nothing is written back per
+// wave: the sizes above take 6.7 us, 12.4 with a row of counters per wave (of which 7 were clearing, sums and scan). With
+// 32768 entries 12.7 (of 64 groups 11.6): there it is the counting, 64 LDS atomics per thread.
+constexpr int kAlignFillPerBlock = 1024;
+constexpr int kAlignMostQuads = (kMoeMaxExperts / 4 + kFusedThreads - 1) / kFusedThreads;   // steps of four groups per thread
+static int64_t align_lds_bytes(int64_t G) { return 20 * ((G + 3) / 4 * 4) + 16 + 256; }
+template <int kPasses, bool kIds64>
+__global__ __launch_bounds__(kFusedThreads) void moe_align_fused_kernel(
     const void* __restrict__ ids_v, int64_t n, int per_iter, int E, int R, int nbits, int block_size,
     int32_t* __restrict__ sorted_ids, int64_t fill_n, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ block_barrier_ids, int32_t* __restrict__ rank_block_num, int32_t* __restrict__ total_post_pad,
-    uint32_t seg_magic) {
-  constexpr int kWaves = kThreads / 64, kItems = kWaves * kPerWave, kPasses = kPerWave / 64;
+    uint32_t seg_magic, uint32_t block_magic) {
+  constexpr int kThreads = kFusedThreads, kWaves = kThreads / 64, kPerWave = 64 * kPasses, kItems = kWaves * kPerWave;
+  static_assert(kWaves == 8 && kPerWave < 256, "a byte of a 64-bit word per wave");
   typedef __attribute__((__vector_size__(2 * sizeof(long long)))) long long long2v;
-  const int G = E * R;
-  extern __shared__ int32_t s_mem[];  // [kWaves][G] wave counters, [G] group sizes, [2][G] before / behind, then starts
-  int32_t* const s_cnt = s_mem;
-  int32_t* const s_col = s_mem + kWaves * G;
-  int32_t* const s_out = s_col + G;
-  int32_t* const s_start = s_out;     // [G + 1] padded exclusive prefix, once the two rows have been summed
+  const int G = E * R, Gp = (G + 3) & ~3;
+  extern __shared__ __attribute__((aligned(16))) int32_t s_mem[];
+  unsigned long long* const s_own = (unsigned long long*)s_mem;   // [Gp] entries of this block, a byte per wave
+  int32_t* const s_before = s_mem + 2 * Gp;                       // [Gp] entries in front of the block
+  int32_t* const s_behind = s_before + Gp;                        // [Gp] those behind it, later all of the group's
+  int32_t* const s_start = s_behind + Gp;                         // [Gp + 1] padded exclusive prefix
   __shared__ int32_t s_part[kWaves];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int B = gridDim.x, b = blockIdx.x;
   const int32_t* const ids32 = (const int32_t*)ids_v;
   const long long* const ids64 = (const long long*)ids_v;
   const uint32_t per = (uint32_t)per_iter;
-  auto key_of = [&](uint32_t i, long long id) -> int {
-    return (id >= 0 && id < E) ? (int)__umulhi(i, seg_magic) * E + (int)id : -1;
-  };
   // the wave's own entries first
   const int64_t wbase = (int64_t)b * kItems + (int64_t)wave * kPerWave;
   long long id_own[kPasses];
@@ -1250,10 +1255,11 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
   const int64_t n_vec = (n + 3) / 4;
   int4v q32[kIds64 ? 1 : kVecBatch];
   long2v q64[kIds64 ? 2 * kVecBatch : 1];
-  auto load_others = [&](int64_t v0) {
+  auto load_others = [&](int64_t v0) {   // (v0: the wave's first vector of the batch)
 #pragma unroll
     for (int u = 0; u < kVecBatch; ++u) {
-      const int64_t vi = v0 + (int64_t)u * kThreads;
+      if (v0 + (int64_t)u * kThreads >= n_vec) break;
+      const int64_t vi = v0 + (int64_t)u * kThreads + lane;
       const bool take = vi < n_vec && !(vi * 4 >= own_lo && vi * 4 < own_hi);
       const bool whole = vi * 4 + 3 < n;
       if constexpr (kIds64) {
@@ -1278,17 +1284,17 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
       }
     }
   };
-  // Counting is the kernel's longest phase (every lane counts n / kThreads entries), so an entry costs as few
-  // instructions as can be: the segment of a vector's first entry by a multiplication (seg_magic = ceil(2^32 / per),
-  // exact below 65536 entries), at most one segment boundary inside a vector (per >= 4), one unsigned compare for the
-  // id's range, and no branch: an id out of range counts into a word of its own lane behind the counters.
-  int32_t* const s_trash = s_mem + (kWaves + 3) * G + lane;
+  // Every lane counts n / kThreads entries, so an entry costs as few instructions as can be: the segment of a vector's
+  // first entry by a multiplication (seg_magic = ceil(2^32 / per), exact below 65536 entries), at most one segment
+  // boundary inside a vector (per >= 4), one unsigned compare for the id's range, and no branch: an id out of range
+  // counts into a word of its own lane behind the counters.
+  int32_t* const s_trash = s_start + Gp + 4 + lane;
   auto count_others = [&](int64_t v0) {
 #pragma unroll
     for (int u = 0; u < kVecBatch; ++u) {
-      const int64_t vi = v0 + (int64_t)u * kThreads;
-      if (vi - lane >= n_vec) break;   // (nothing left for this wave)
-      int32_t* const row = s_out + (vi * 4 < own_lo ? 0 : G);
+      if (v0 + (int64_t)u * kThreads >= n_vec) break;   // (nothing left for this wave)
+      const int64_t vi = v0 + (int64_t)u * kThreads + lane;
+      int32_t* const row = vi * 4 < own_lo ? s_before : s_behind;
       const uint32_t i0 = (uint32_t)(vi * 4);
       const uint32_t seg = __umulhi(i0, seg_magic);
       const uint32_t to_next = (seg + 1) * per - i0;   // entries of this vector that are still in segment `seg`
@@ -1310,44 +1316,76 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
       }
     }
   };
-  if (B > 1) load_others(threadIdx.x);
-  for (int g = threadIdx.x; g < (kWaves + 3) * G; g += kThreads) s_cnt[g] = 0;
-  __syncthreads();
-  int32_t* const my_cnt = s_cnt + wave * G;
-  int e_of[kPasses];
+  const int64_t first_vec = wave * 64;
+  if (B > 1) load_others(first_vec);
+  for (int g = threadIdx.x; g < Gp; g += kThreads) ((int4v*)s_mem)[g] = int4v{0, 0, 0, 0};   // 16 bytes a group
+  // the key of each own entry and its place among the wave's entries of that key: those of lower lanes, and of an earlier pass
+  int e_of[kPasses], within[kPasses];
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
   for (int u = 0; u < kPasses; ++u) {
-    e_of[u] = key_of((uint32_t)(wbase + u * 64 + lane), id_own[u]);
-    if (e_of[u] >= 0) atomicAdd(&my_cnt[e_of[u]], 1);
+    const uint32_t i = (uint32_t)(wbase + u * 64 + lane);
+    e_of[u] = id_own[u] >= 0 && id_own[u] < E ? (int)__umulhi(i, seg_magic) * E + (int)id_own[u] : -1;
+    uint64_t peers[kPasses];
+#pragma unroll
+    for (int v = 0; v <= u; ++v) peers[v] = __ballot(e_of[v] >= 0);
+    for (int bit = 0; bit < nbits; ++bit) {
+      const bool one = (e_of[u] >> bit) & 1;
+#pragma unroll
+      for (int v = 0; v <= u; ++v) {
+        const uint64_t m = __ballot((e_of[v] >> bit) & 1);
+        peers[v] &= one ? m : ~m;
+      }
+    }
+    within[u] = __popcll(peers[u] & lt_mask);
+#pragma unroll
+    for (int v = 0; v < u; ++v) within[u] += __popcll(peers[v]);
   }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPasses; ++u)
+    if (e_of[u] >= 0) atomicAdd(&s_own[e_of[u]], 1ull << (8 * wave));
   if (B > 1) {
-    count_others(threadIdx.x);
-    for (int64_t v0 = threadIdx.x + (int64_t)kVecBatch * kThreads; v0 < n_vec; v0 += (int64_t)kVecBatch * kThreads) {
+    count_others(first_vec);
+    for (int64_t v0 = first_vec + (int64_t)kVecBatch * kThreads; v0 < n_vec; v0 += (int64_t)kVecBatch * kThreads) {
       load_others(v0);
       count_others(v0);
     }
   }
   __syncthreads();
-  // group sizes; the waves' starts within their group (entries of the blocks in front, then of the earlier waves)
-  for (int g = threadIdx.x; g < G; g += kThreads) {
-    int32_t run = s_out[g], total = s_out[g] + s_out[G + g];
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const int32_t c = s_cnt[w * G + g];
-      s_cnt[w * G + g] = run;
-      run += c;
-      total += c;
-    }
-    s_col[g] = total;
-  }
-  __syncthreads();
-  // exclusive scan of the PADDED group sizes: consecutive groups per thread, then across threads and waves
-  const int per_thread = (G + kThreads - 1) / kThreads;
-  const int g0 = threadIdx.x * per_thread;
-  auto padded = [&](int32_t c) { return (c + block_size - 1) / block_size * block_size; };
+  // group sizes and the exclusive scan of the PADDED ones: consecutive groups per thread, then across threads and waves
+  // (whole blocks by a multiplication: exact up to 65536 entries and blocks of 32768; 0: by a division)
+  auto padded = [&](int32_t c) {
+    const uint32_t x = (uint32_t)(c + block_size - 1);
+    return (int32_t)(block_magic != 0 ? __umulhi(x, block_magic) : x / (uint32_t)block_size) * block_size;
+  };
+  auto sum_bytes = [](unsigned long long w, int32_t to) {
+    return (int32_t)__builtin_amdgcn_sad_u8((uint32_t)(w >> 32), 0u, __builtin_amdgcn_sad_u8((uint32_t)w, 0u, (uint32_t)to));
+  };
+  const int quads = Gp / 4, quads_each = (quads + kThreads - 1) / kThreads;
+  int4v size[kAlignMostQuads];   // padded
   int32_t local_total = 0;
-  for (int j = 0; j < per_thread; ++j)
-    if (g0 + j < G) local_total += padded(s_col[g0 + j]);
+#pragma unroll
+  for (int k = 0; k < kAlignMostQuads; ++k) {
+    const int at = threadIdx.x * quads_each + k;
+    size[k] = int4v{0, 0, 0, 0};
+    if (k < quads_each && at < quads) {
+      const int4v before = ((const int4v*)s_before)[at], behind = ((const int4v*)s_behind)[at];
+      const int4v own0 = ((const int4v*)s_own)[2 * at], own1 = ((const int4v*)s_own)[2 * at + 1];
+      int4v c = before + behind;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        c[j] = sum_bytes((unsigned long long)(uint32_t)own0[2 * j + 1] << 32 | (uint32_t)own0[2 * j], c[j]);
+        c[2 + j] = sum_bytes((unsigned long long)(uint32_t)own1[2 * j + 1] << 32 | (uint32_t)own1[2 * j], c[2 + j]);
+      }
+      ((int4v*)s_behind)[at] = c;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        size[k][j] = padded(c[j]);
+        local_total += size[k][j];
+      }
+    }
+  }
   int32_t incl = local_total;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -1356,32 +1394,51 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
   }
   if (lane == 63) s_part[wave] = incl;
   __syncthreads();
-  int32_t acc = incl - local_total;
+  int32_t acc = incl - local_total, total = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) acc += w < wave ? s_part[w] : 0;
-  for (int j = 0; j < per_thread; ++j) {
-    const int g = g0 + j;
-    if (g < G) {
-      s_start[g] = acc;
+  for (int w = 0; w < kWaves; ++w) {
+    const int32_t part = s_part[w];
+    acc += w < wave ? part : 0;
+    total += part;
+  }
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) s_cnt[w * G + g] += acc;
-      acc += padded(s_col[g]);
-      if (g == G - 1) s_start[G] = acc;
+  for (int k = 0; k < kAlignMostQuads; ++k) {
+    const int at = threadIdx.x * quads_each + k;
+    if (k < quads_each && at < quads) {
+      int4v from;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        from[j] = acc;
+        acc += size[k][j];
+      }
+      ((int4v*)s_start)[at] = from;
     }
   }
+  if (threadIdx.x == 0) s_start[Gp] = total;
   __syncthreads();
-  const int32_t total = s_start[G];
+  // the wave's entries
+#pragma unroll
+  for (int u = 0; u < kPasses; ++u) {
+    const int e = e_of[u];
+    if (e >= 0) {
+      const unsigned long long earlier_waves = s_own[e] & ((1ull << (8 * wave)) - 1);
+      sorted_ids[s_start[e] + sum_bytes(earlier_waves, s_before[e] + within[u])] = (int32_t)(wbase + u * 64 + lane);
+    }
+  }
   if (b == 0) {
     for (int r = threadIdx.x; r < R; r += kThreads) rank_block_num[r] = (s_start[(r + 1) * E] - s_start[r * E]) / block_size;
     if (threadIdx.x == 0) *total_post_pad = total;
   }
   // the groups this block looks after (a wave each, in turn): their padding positions and their blocks' ids
   for (int g = b + B * wave; g < G; g += B * kWaves) {
-    const int32_t st = s_start[g], c = s_col[g], pc = padded(c);
+    const int32_t st = s_start[g], c = s_behind[g], pc = padded(c);
     for (int32_t o = c + lane; o < pc; o += 64) sorted_ids[st + o] = (int32_t)n;
-    for (int32_t k = st / block_size + lane; k < (st + pc) / block_size; k += 64) {
-      expert_ids[k] = g % E;
-      block_barrier_ids[k] = g / E;
+    if (pc > 0) {
+      const int seg = g / E, expert = g - seg * E;
+      for (int32_t k = st / block_size + lane; k < (st + pc) / block_size; k += 64) {
+        expert_ids[k] = expert;
+        block_barrier_ids[k] = seg;
+      }
     }
   }
   // and its share of the positions behind the padded total
@@ -1389,26 +1446,6 @@ __global__ __launch_bounds__(kThreads) void moe_align_fused_kernel(
     const int64_t share = (fill_n - total + B - 1) / B;
     const int64_t lo = total + share * b, hi = lo + share < fill_n ? lo + share : fill_n;
     for (int64_t i = lo + threadIdx.x; i < hi; i += kThreads) sorted_ids[i] = (int32_t)n;
-  }
-  // the wave's entries in flat order, 64 at a time (as in moe_rank_kernel)
-  volatile int32_t* pos = my_cnt;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-#pragma unroll
-  for (int u = 0; u < kPasses; ++u) {
-    if (wbase + u * 64 >= n) break;
-    const int64_t i = wbase + u * 64 + lane;
-    const int e = e_of[u];
-    const bool valid = e >= 0;
-    uint64_t peers = __ballot(valid);
-    for (int bit = 0; bit < nbits; ++bit) {
-      const bool one = (e >> bit) & 1;
-      const uint64_t m = __ballot(valid && one);
-      peers &= one ? m : ~m;
-    }
-    if (valid) sorted_ids[pos[e] + __popcll(peers & lt_mask)] = (int32_t)i;
-    __builtin_amdgcn_wave_barrier();
-    if (valid && (peers & lt_mask) == 0) pos[e] = pos[e] + __popcll(peers);
-    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -1972,32 +2009,30 @@ int tdist_moe_align_block_size(const void* topk_ids, int ids_int64, int64_t n_to
   const int64_t blocks = ceil_div(n_total > 0 ? n_total : 1, 256);
   // Few entries: one launch in which every block counts all of them (see moe_align_fused_kernel).
   {
-    constexpr int kLdsLimit = 160 * 1024 - 256;
-    constexpr int kRows = kFusedThreads / 64 + 3;
     const int64_t n1 = n_total > 0 ? n_total : 1;
     const int form = ceil_div(n1, kFusedThreads) <= kRecountMaxBlocks ? 1 : ceil_div(n1, 2 * kFusedThreads) <= kRecountMaxBlocks ? 2 : 0;
     const int64_t per_iter = n_per_iteration > 0 ? n_per_iteration : 1;
     // (a vector of four entries may cross one segment boundary, not two; the segment of an entry by multiplication)
     const uint32_t seg_magic = per_iter >= 65536 ? 0u : (uint32_t)(((1ull << 32) + per_iter - 1) / per_iter);
-    if (form != 0 && device_info().ok == 1 && kRows * G * 4 + 256 <= kLdsLimit && aligned16(topk_ids) &&
-        (per_iter >= 4 || num_iterations == 1) && debug_get(TDIST_DEBUG_MOE_INDEX_FORM) != 3) {
-      auto kern = form == 1 ? (ids_int64 ? moe_align_fused_kernel<kFusedThreads, kFusedThreads / 8, true>
-                                         : moe_align_fused_kernel<kFusedThreads, kFusedThreads / 8, false>)
-                            : (ids_int64 ? moe_align_fused_kernel<kFusedThreads, kFusedThreads / 4, true>
-                                         : moe_align_fused_kernel<kFusedThreads, kFusedThreads / 4, false>);
+    const uint32_t block_magic = block_size > 1 && block_size <= 32768 ? (uint32_t)(((1ull << 32) + block_size - 1) / block_size) : 0u;
+    static_assert(20 * kMoeMaxExperts + 16 + 256 <= 160 * 1024 - 256, "any number of groups has room in the LDS");
+    if (form != 0 && device_info().ok == 1 && aligned16(topk_ids) && (per_iter >= 4 || num_iterations == 1) &&
+        debug_get(TDIST_DEBUG_MOE_INDEX_FORM) != 3) {
+      auto kern = form == 1 ? (ids_int64 ? moe_align_fused_kernel<1, true> : moe_align_fused_kernel<1, false>)
+                            : (ids_int64 ? moe_align_fused_kernel<2, true> : moe_align_fused_kernel<2, false>);
       static bool attr_set[4] = {false, false, false, false};
       const int which = (form - 1) * 2 + (ids_int64 ? 1 : 0);
       if (!attr_set[which]) {
-        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit) != hipSuccess)
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)align_lds_bytes(kMoeMaxExperts)) != hipSuccess)
           return fail(TDIST_ERR_LAUNCH, "%s: cannot reserve LDS for the align kernel", who);
         attr_set[which] = true;
       }
       const int64_t for_entries = ceil_div(n1, form == 1 ? kFusedThreads : 2 * kFusedThreads), cus = device_info().num_cus;
       const int64_t for_fill = ceil_div(sorted_fill, kAlignFillPerBlock) < cus ? ceil_div(sorted_fill, kAlignFillPerBlock) : cus;
       const int64_t nblk = for_entries > for_fill ? for_entries : for_fill;
-      hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kFusedThreads), (size_t)kRows * G * 4 + 256, st, topk_ids, n_total,
+      hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(kFusedThreads), (size_t)align_lds_bytes(G), st, topk_ids, n_total,
                          (int)per_iter, num_experts, num_iterations, id_bits((int)G), block_size, sorted_token_ids, sorted_fill,
-                         expert_ids, block_barrier_ids, rank_block_num, total_tokens_post_pad, seg_magic);
+                         expert_ids, block_barrier_ids, rank_block_num, total_tokens_post_pad, seg_magic, block_magic);
       return launch_status(who);
     }
   }
