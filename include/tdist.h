@@ -480,9 +480,15 @@ int tdist_group_gemm_gated_fp8e4m3(const void* A, int64_t lda, const void* A_loc
                                    int32_t* status, int max_workgroups,
     void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
 
+/* Rows per block (64, 128 or 256) that tdist_group_gemm_rows is the fastest with for `rows` rows over num_experts experts, N columns, k_bytes of K and
+ * a workspace of that size (0: none), by an estimate; 0 for sizes below 1 or without a device. Host only. */
+int tdist_group_gemm_row_block(int64_t rows, int num_experts, int N, int64_t k_bytes, int64_t sk_workspace_bytes);
+
 /* The same without flags for gathered rows that are read where they lie: token t is row t % rows_per_rank of shard
  * t / rows_per_rank (shards, dtype, limits, status and first_error as for tdist_ag_gemm_rows; TDIST_ERR_UNSUPPORTED beyond them, or where K rows are
  * of 128 bytes or fewer: gather the rows then). */
+/* (blocks of 64 rows are taken as well as of 128 and 256, for experts of few rows; one shard of rows in one piece may be of any length below 4 GiB, with
+ * status NULL) */
 int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
                           int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids,
                           const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,

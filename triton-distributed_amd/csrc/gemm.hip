@@ -24,6 +24,7 @@
 //  * persistent grid (one workgroup per CU). The tile schedule is chunk-major in arrival order, and
 //    within a round of concurrently running tiles the workgroups of one XCD (workgroup id mod 8) get a
 //    compact block of tiles so they share A rows and B rows in that XCD's L2.
+#include <cmath>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -1898,6 +1899,16 @@ struct SmallPlan {
   bool deep;
   double us;
 };
+constexpr double kSmallPairUs[kNumSmallTiles] = {0.5, 0.85};   // a K tile of each of two workgroups on a compute unit
+static double small_tiles_us(int t, int64_t units, int per, int pieces, int cus, const double* pair_us = kSmallPairUs) {
+  const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn;
+  const double alone = t == 0 ? 0.225 : 0.315, stage_mb = (bm + bn) * 128 * 1e-6;
+  double us = 3.0;
+  if (units <= cus) us += per * std::max(alone, units * stage_mb / 24.0) + 1.0;
+  else us += (double)ceil_div(units, 2 * cus) * (per * pair_us[t] + 1.5);
+  if (pieces > 1) us += 1.2 + (t == 0 ? 0.25 : 0.6) * pieces + (double)units * bm * bn * 4 / 3.0e6;
+  return us;
+}
 static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
   SmallPlan best = {0, 0, 0, false, 0};
   if (c.flags || c.A_local || (int64_t)c.M * c.lda * esz >= (1ll << 31) || (int64_t)c.N * c.ldb * esz >= (1ll << 31)) return best;
@@ -1915,13 +1926,8 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
       if (sk > 1 && s != sk) continue;
       const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
       const int64_t units = tiles * pieces;
-      const bool deep = units <= cus;
-      double us = 3.0;
-      const double alone = t == 0 ? 0.225 : 0.315, stage_mb = (bm + bn) * 128 * 1e-6;
-      if (deep) us += per * std::max(alone, units * stage_mb / 24.0) + 1.0;
-      else us += (double)ceil_div(units, 2 * cus) * (per * (t == 0 ? 0.5 : 0.85) + 1.5);
-      if (pieces > 1) us += 1.2 + (t == 0 ? 0.25 : 0.6) * pieces + (double)units * bm * bn * 4 / 3.0e6;
-      if (best.us == 0 || us < best.us) best = {t, pieces, per, deep, us};
+      const double us = small_tiles_us(t, units, per, pieces, cus);
+      if (best.us == 0 || us < best.us) best = {t, pieces, per, units <= cus, us};
     }
   }
   return best;
@@ -1931,6 +1937,7 @@ static int run_small(const GemmCall& c, GemmElem elem, int esz, const SmallPlan&
   SmallGemmParams q;
   q.A = (const unsigned char*)c.A;
   q.shards = c.shards;
+  q.sorted_ids = nullptr;
   q.B = (const unsigned char*)c.B;
   q.C = (unsigned char*)c.C;
   q.scatter_bufs = c.scatter_bufs;
@@ -2338,7 +2345,105 @@ struct GroupGemmCall {
   hipStream_t stream;
   const char* who;
   ShardRows shards;   // rows != 0: A's rows lie in shards (calls without flags only)
+  bool few_rows;      // blocks of kGroupedFewRows rows are taken as well (calls without flags or a local shard)
 };
+
+// ---- estimates for the grouped GEMM, in microseconds -------------------------------------------------------------
+// Fitted to the times of all four forms (64 x 128 and 128 x 128 small tiles, 128 x 256 and 256 x 256 large ones) on 70 problems of 16
+// to 18731 rows over 8 to 64 experts: the form taken is 0.3 % behind the best on average (the block sizes of before: 39 %). Beside
+// the tiles' work it is the way of the weights that counts: once from memory, again from the caches for an expert's other blocks.
+struct GroupShape {
+  int64_t rows;
+  double groups;   // experts, or what is known of their number
+  int N;
+  int64_t k_bytes;
+};
+static double groups_in_use(const GroupShape& g) {
+  return g.groups <= 1 || g.rows <= 0 ? 1 : -g.groups * std::expm1((double)g.rows * std::log1p(-1 / g.groups));
+}
+// blocks of `block` rows, rows evenly at random over the experts: sizes about the mean with its root as the deviation
+static int64_t group_blocks(const GroupShape& g, int block) {
+  const double used = std::max(1.0, groups_in_use(g)), mean = g.rows / used, dev = std::max(0.3, std::sqrt(mean));
+  double each = 1;
+  if (mean > 8.0 * block) each = mean / block + 0.5;
+  else
+    for (int k = 1; k * block < mean + 4 * dev; ++k) each += 0.5 * std::erfc((k * block + 0.5 - mean) / dev * 0.70710678);
+  return std::max<int64_t>(1, (int64_t)(used * each + 0.5));
+}
+static double group_panels_us(const GroupShape& g, double bytes, double cache_bytes_per_us) {
+  const double weights = groups_in_use(g) * g.N * g.k_bytes;
+  return weights / 5.5e6 + std::max(0.0, bytes - weights) / cache_bytes_per_us;
+}
+// On small tile t; `capacity`: blocks that there is room for. (A pair of workgroups takes longer than in an ungrouped GEMM: no two
+// of them share their weights.)
+static SmallPlan group_small_plan(const GroupShape& g, int t, int64_t capacity, int64_t workspace_bytes, int cus) {
+  constexpr double kPairUs[kNumSmallTiles] = {0.77, 1.18};
+  SmallPlan best = {t, 0, 0, false, 0};
+  const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn, k_tiles = (int)ceil_div(g.k_bytes, 128), sk = debug_get(TDIST_DEBUG_GEMM_SPLIT_K);
+  const int64_t tiles_n = ceil_div(g.N, bn), used = group_blocks(g, bm) * tiles_n, tiles = capacity * tiles_n;
+  const double panels = 4.2 + group_panels_us(g, (double)used * k_tiles * bn * 128, 10.6e6);
+  for (int s = 1; s <= kSmallMaxSplits; s *= 2) {
+    if (s > 1 && (sk == 0 || tiles > kSkSmallTiles || k_tiles / s < (sk > 1 ? 2 : kSmallMinPiece) ||
+                  workspace_bytes < kSkHeaderBytes + tiles * s * bm * bn * 4)) break;
+    if (sk > 1 && s != sk && s != 1) continue;   // (a forced number of pieces that K does not allow: whole)
+    const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
+    const double us = std::max(small_tiles_us(t, used * pieces, per, pieces, cus, kPairUs), panels);
+    if (best.us == 0 || us < best.us || (sk > 1 && s == sk)) best = {t, pieces, per, used * pieces <= cus, us};
+  }
+  return best;
+}
+// On the large tiles of `block` rows by 256 columns.
+static double group_large_us(const GroupShape& g, int block, bool split_last, int cus) {
+  const int k_tiles = (int)ceil_div(g.k_bytes, 128);
+  const int64_t tiles = group_blocks(g, block) * ceil_div(g.N, 256), full = tiles / cus, tail = tiles % cus;
+  const double k_tile = block == 256 ? 1.5 : 0.955;
+  double us = (double)(full + (tail != 0)) * k_tiles * k_tile;
+  const int s = split_last && tail != 0 && k_tiles >= 2 * kSkMinPiece ? sk_split_for(cus, (int)tail, k_tiles) : 1;
+  if (s > 1) us = (full + 1.0 / s) * k_tiles * k_tile + 24.0;
+  return 11.7 + std::max(us, group_panels_us(g, (double)tiles * k_tiles * (block + 256) * 128, 12.8e6));
+}
+
+// The small tiles' plan for a call whose blocks have a small tile's rows (us = 0: it does not qualify).
+static SmallPlan group_small_plan(const GroupGemmCall& c, const GroupShape& g, int esz, int cus) {
+  const int t = c.block_size == kSmallTiles[0].bm ? 0 : 1;
+  if (kSmallTiles[t].bm != c.block_size || c.flags || c.A_local || (c.max_workgroups > 0 && c.max_workgroups < cus) ||
+      (int64_t)c.N * c.ldb * esz >= (1ll << 31) || (int64_t)c.num_valid * c.topk >= (1ll << 32) ||
+      (c.num_blocks * ceil_div(c.N, kSmallTiles[t].bn) + 8) * kSmallMaxSplits > 0x7fffffff) return {t, 0, 0, false, 0};
+  return group_small_plan(g, t, c.num_blocks, c.sk_workspace ? c.sk_workspace_bytes : 0, cus);
+}
+
+static int run_group_small(const GroupGemmCall& c, GemmElem elem, int esz, const SmallPlan& plan, const DeviceInfo& di) {
+  SmallGemmParams q;
+  q.A = (const unsigned char*)c.A;
+  q.shards = c.shards;
+  q.sorted_ids = c.sorted_ids;
+  q.block_expert = c.expert_ids;
+  q.post_pad = c.post_pad;
+  q.b_expert_stride_b = c.expert_stride * esz;
+  q.num_blocks = c.num_blocks;
+  q.num_valid = c.num_valid;
+  q.a_rows = c.a_rows;
+  q.topk = c.topk;
+  q.topk_magic = (uint32_t)(((1ull << 32) + c.topk - 1) / c.topk);
+  q.B = (const unsigned char*)c.B;
+  q.C = (unsigned char*)c.C;
+  q.scatter_bufs = nullptr;
+  q.row_scale = q.col_scale = nullptr;
+  q.lda_b = c.lda * esz;
+  q.ldb_b = c.ldb * esz;
+  q.ldc = c.ldc;
+  q.M = c.num_blocks * c.block_size;
+  q.N = c.N;
+  q.k_bytes = c.K * esz;
+  q.m_per_rank = q.M;
+  q.rank = 0;
+  q.splits = plan.splits;
+  q.tiles_per_split = plan.tiles_per_split;
+  q.partials = plan.splits > 1 ? (float*)((unsigned char*)c.sk_workspace + kSkHeaderBytes) : nullptr;
+  q.counters = plan.splits > 1 ? (int32_t*)c.sk_workspace + kSkSmallOff : nullptr;
+  q.l2_local = di.xcd_round_robin == 1 && di.num_xcds == 8 && debug_get(TDIST_DEBUG_GEMM_SK_COHERENT) != 1;
+  return launch_gemm_small(q, elem == kElemBF16 ? kSmallBF16 : elem == kElemF16 ? kSmallF16 : kSmallFP8, plan.tile, plan.deep, c.stream, c.who);
+}
 
 static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   const char* who = c.who;
@@ -2347,7 +2452,8 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
     return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
   if (c.a_rows <= 0 || c.N <= 0 || c.K <= 0 || c.num_blocks <= 0 || c.topk <= 0 || c.num_valid < 0 || c.tokens_per_rank <= 0)
     return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
-  if (c.block_size != 128 && c.block_size != 256)
+  const bool few = c.few_rows && c.block_size == kGroupedFewRows;
+  if (c.block_size != 128 && c.block_size != 256 && !few)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: block_size %d (the row blocks of the align / sort step must be 128 or 256 rows)", who, c.block_size);
   if (((int64_t)c.K * esz) % 16 != 0 || (((int64_t)c.K * esz) % 64 != 0 && (int64_t)c.K * esz <= 128))
     return fail(TDIST_ERR_UNSUPPORTED, "%s: K*elem_size = %lld must be a multiple of 64 bytes (above 128: of 16)", who, (long long)c.K * esz);
@@ -2366,6 +2472,15 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   if (int rc = sk_workspace_check(c.sk_workspace, c.sk_workspace_bytes, who)) return rc;
   const DeviceInfo& di = device_info();
   if (di.ok != 1) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
+  // (experts: what the number of blocks leaves room for, every one pads block_size - 1 rows at most)
+  const GroupShape shape = {c.num_valid, (double)(((int64_t)c.num_blocks * c.block_size - c.num_valid) / (c.block_size - 1) + 1), c.N, (int64_t)c.K * esz};
+  const SmallPlan small = group_small_plan(c, shape, esz, di.num_cus);
+  const int forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
+  if (few && small.us == 0)
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: blocks of %d rows take an expert's weights below 2 GiB and no flags", who, c.block_size);
+  if (few || (small.us > 0 && (forced_tile >= kNumLargeTiles ||
+                               (forced_tile < 0 && sk_env() != 1 && small.us < group_large_us(shape, c.block_size, c.sk_workspace && sk_env() != 0, di.num_cus)))))
+    return run_group_small(c, elem, esz, small, di);
 
   GemmParams p;
   p.A = (const unsigned char*)c.A;
@@ -2601,6 +2716,7 @@ int tdist_ag_gemm_rows(int dtype, const void* const* shards, int world_size, int
 #define TDIST_GROUP_GEMM_BODY(ELEM, WHO)                                                                              \
   GroupGemmCall c;                                                                                                    \
   c.shards.rows = 0;                                                                                                  \
+  c.few_rows = false;                                                                                                 \
   c.A = A; c.lda = lda; c.A_local = A_local; c.lda_local = lda_local; c.local_row_begin = local_row_begin;            \
   c.local_rows = local_rows; c.B = B; c.ldb = ldb; c.expert_stride = expert_stride; c.C = C; c.ldc = ldc;             \
   c.a_rows = a_rows; c.N = N; c.K = K; c.sorted_ids = sorted_token_ids; c.expert_ids = expert_ids;                    \
@@ -2625,6 +2741,23 @@ int tdist_group_gemm_gated_fp8e4m3(TDIST_GROUP_GEMM_ARGS) {
   TDIST_GROUP_GEMM_BODY(kElemFP8, "tdist_group_gemm_gated_fp8e4m3")
 }
 
+int tdist_group_gemm_row_block(int64_t rows, int num_experts, int N, int64_t k_bytes, int64_t sk_workspace_bytes) {
+  const DeviceInfo& di = device_info();
+  if (di.ok != 1 || rows <= 0 || num_experts <= 0 || N <= 0 || k_bytes <= 0) return 0;
+  const int forced = debug_get(TDIST_DEBUG_GEMM_TILE);
+  if (forced >= kNumLargeTiles && forced < kNumLargeTiles + kNumSmallTiles) return kSmallTiles[forced - kNumLargeTiles].bm;
+  if (forced >= 0) return forced < 2 ? 256 : 128;
+  const GroupShape g = {rows, (double)num_experts, N, k_bytes};
+  const int64_t used = std::min<int64_t>(num_experts, rows);
+  int best = 256;
+  double us = group_large_us(g, 256, sk_workspace_bytes > 0, di.num_cus);
+  auto take = [&](int block, double t) { if (t < us) us = t, best = block; };
+  take(128, group_large_us(g, 128, sk_workspace_bytes > 0, di.num_cus));
+  for (int t = 0; t < kNumSmallTiles; ++t)
+    take(kSmallTiles[t].bm, group_small_plan(g, t, (rows + used * (kSmallTiles[t].bm - 1)) / kSmallTiles[t].bm, sk_workspace_bytes, di.num_cus).us);
+  return best;
+}
+
 int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
                           int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                           const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded, int num_blocks, int block_size,
@@ -2640,13 +2773,14 @@ int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, 
   for (int r = 0; shards && r < world_size; ++r)
     if (!shards[r] || !aligned16(shards[r])) return fail(shards[r] ? TDIST_ERR_UNSUPPORTED : TDIST_ERR_INVALID, "%s: shard %d: null or not 16-byte aligned", who, r);
   if (!shards) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
-  if (!shards_in_reach(shards, world_size, rows_per_rank, rank_bytes, c.shards, base))
+  if (world_size == 1 && status == nullptr) base = (const unsigned char*)shards[0];   // (rows in one piece, of any number)
+  else if (!shards_in_reach(shards, world_size, rows_per_rank, rank_bytes, c.shards, base))
     return fail(TDIST_ERR_UNSUPPORTED, "%s: at most %d shards within 4 GiB of each other, world_size * rows_per_rank^2 below 2^32", who, kMaxShards);
   c.shards.status = status; c.shards.first_error = first_error;
   c.A = base; c.lda = K; c.B = B; c.ldb = ldb; c.expert_stride = expert_stride; c.C = C; c.ldc = ldc;
   c.a_rows = world_size * rows_per_rank; c.N = N; c.K = K; c.sorted_ids = sorted_token_ids; c.expert_ids = expert_ids;
   c.block_segment = block_barrier_ids; c.post_pad = num_tokens_post_padded; c.num_blocks = num_blocks; c.block_size = block_size;
-  c.num_valid = num_valid_tokens; c.topk = topk; c.tokens_per_rank = c.a_rows;
+  c.num_valid = num_valid_tokens; c.topk = topk; c.tokens_per_rank = c.a_rows; c.few_rows = true;
   c.sk_workspace = sk_workspace; c.sk_workspace_bytes = sk_workspace_bytes; c.stream = (hipStream_t)stream; c.who = who;
   return run_group_gemm(c, elem);
 }

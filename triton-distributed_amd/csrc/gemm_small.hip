@@ -14,6 +14,10 @@
 //    out one by one between products a K tile took 0.505 and 0.655 us whether its rows came from memory or from the L2: 200 x 1536 x 4096
 //    16.0 -> 12.1 us, 1024 x 4096 x 4096 47.6 -> 29.6, e4m3 64 x 1536 x 8192 33.7 -> 17.5;
 //  * v_mfma 16x16x32 (16-bit) / 16x16x128 (e4m3), D^T = B * A^T, so that a lane holds 4 consecutive columns;
+//  * grouped (rows named by sorted ids, weights by a block's expert): for experts of few rows, where a call is a read of the
+//    weights. 64 experts of 72 rows in all, 2 x 512 x 2176: 51 us a launch on tiles of 128 x 256 cut along K (86 tiles, a third
+//    of their loads rows that are not there), 21 on 64 x 128, or 5.4 TB/s; 311 rows over 16 experts, 1280 x 3200: 62 -> 30;
+//    1454 rows over 16, 3584 x 896: 37 -> 25 on 128 x 128;
 //  * with `splits` > 1 every workgroup leaves its fp32 accumulators in the workspace and bumps its tile's counter; the last
 //    to arrive adds the pieces up in their K order, so the result does not depend on timing and nobody waits. The pieces
 //    of a tile meet in one XCD's L2 where workgroup i is known to run on XCD i % 8 (written through to memory they cost
@@ -64,8 +68,9 @@ struct SmallCfg {
   static_assert((NST - 2) * kLoads < 64, "vmcnt is 6 bits");
 };
 
-// kShards: A's rows lie in shards (an instance of its own: the test for them alone costs the other calls 0.3 us of 21)
-template <typename E, int BM, int BN, int NST, bool kScales, bool kShards>
+// kRows: where A's rows lie (instances of their own: the test for shards alone costs the other calls 0.3 us of 21)
+enum SmallRows { kRowsPlain, kRowsShards, kRowsGrouped };
+template <typename E, int BM, int BN, int NST, bool kScales, int kRows>
 __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParams p) {
   typedef SmallCfg<BM, BN, NST> C;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -77,10 +82,14 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   // Workgroup i runs on XCD i % 8 (checked once per device by tdist_init, and here by every tile's last workgroup): an XCD
   // takes a run of whole tiles, row tiles first, so that it fetches its columns' weights once and the pieces of a tile
   // meet in its L2.
-  const int tiles_m = (p.M + BM - 1) / BM, tiles = tiles_m * ((p.N + BN - 1) / BN);
+  // (grouped: of the blocks in use, a load in front of everything. Shared out with those that are not, the XCDs' parts differed by
+  // half: 6070 rows over 32 experts, 512 columns, 3712 deep 76 us.)
+  const int tiles_m = kRows == kRowsGrouped ? min(__builtin_amdgcn_readfirstlane(p.post_pad[0]) / BM, p.num_blocks) : (p.M + BM - 1) / BM;
+  const int tiles = tiles_m * ((p.N + BN - 1) / BN);
   const int xcd = blockIdx.x & 7, of_xcd = blockIdx.x >> 3;
   const int mine = of_xcd / p.splits, piece = of_xcd - mine * p.splits;
-  if constexpr (kShards) retire_beside(p.shards);
+  constexpr bool kShards = kRows == kRowsShards, kGrouped = kRows == kRowsGrouped;
+  if constexpr (kShards || kGrouped) retire_beside(p.shards);
   if (mine >= (tiles >> 3) + (xcd < (tiles & 7))) return;
   const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + mine;
   const int tm = tile % tiles_m, tn = tile / tiles_m;
@@ -91,10 +100,31 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 
   // DMA: instruction i of a wave brings rows (i * 4 + wave) * 8 .. + 7, lane = row * 8 + chunk position
   uint32_t aoff[C::kAInstr], boff[C::kBInstr];
+  const unsigned char* b_base = p.B;
+  if constexpr (kGrouped) {
+    int ids[C::kAInstr];
 #pragma unroll
-  for (int i = 0; i < C::kAInstr; ++i) {
-    const int r = (i * 4 + wave) * 8 + (lane >> 3);
-    aoff[i] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.lda_b + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    for (int i = 0; i < C::kAInstr; ++i) ids[i] = p.sorted_ids[m0 + (i * 4 + wave) * 8 + (lane >> 3)];
+    const int expert = __builtin_amdgcn_readfirstlane(p.block_expert[tm]);
+    b_base += (int64_t)expert * p.b_expert_stride_b;
+#pragma unroll
+    for (int i = 0; i < C::kAInstr; ++i) {
+      const int r = (i * 4 + wave) * 8 + (lane >> 3);
+      // (places without a row read the first one: the same lines for all of them, and what comes of it is not stored)
+      int row = (uint32_t)ids[i] < (uint32_t)p.num_valid ? (p.topk == 1 ? ids[i] : (int)__umulhi((uint32_t)ids[i], p.topk_magic)) : 0;
+      row = min(row, p.a_rows - 1);
+      uint32_t at = (uint32_t)row * (uint32_t)p.lda_b;
+      if (p.shards.rows != 0)
+        for (int s = 0, first = 0; first < p.a_rows; ++s, first += p.shards.rows)
+          if (row >= first) at = p.shards.off[s] + (uint32_t)(row - first) * (uint32_t)p.lda_b;
+      aoff[i] = at + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < C::kAInstr; ++i) {
+      const int r = (i * 4 + wave) * 8 + (lane >> 3);
+      aoff[i] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.lda_b + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
   }
   if constexpr (kShards) {
     // rows in shards: the tile's few shards one after the other (their offsets by scalar loads), each for the rows from its first on
@@ -127,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   };
   auto issue = [&](int kt, int stage) {
     const int64_t at = (int64_t)kt * kSmallKB - back;
-    static_for<C::kLoads>([&](auto n_c) { issue_one(p.A + at, p.B + at, stage, n_c); });
+    static_for<C::kLoads>([&](auto n_c) { issue_one(p.A + at, b_base + at, stage, n_c); });
   };
   // the first K tile where it is ragged: lanes in front of the row read zeros, the others what they read in any tile
   auto issue_ragged = [&](int stage) {
@@ -140,7 +170,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 #pragma unroll
     for (int i = 0; i < C::kAInstr; ++i) one(p.A, aoff[i], (i * 4 + wave) * 8 + (lane >> 3), st + i * 4096);
 #pragma unroll
-    for (int i = 0; i < C::kBInstr; ++i) one(p.B, boff[i], (i * 4 + wave) * 8 + (lane >> 3), st + BM * kSmallKB + i * 4096);
+    for (int i = 0; i < C::kBInstr; ++i) one(b_base, boff[i], (i * 4 + wave) * 8 + (lane >> 3), st + BM * kSmallKB + i * 4096);
   };
 
   float4v acc[C::kTN][C::kTM];
@@ -226,7 +256,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     auto tile_of = [&](int k, auto load_c) {
       constexpr bool kLoad = decltype(load_c)::value;
       const int64_t at = (int64_t)(kt0 + k + NST - 1) * kSmallKB - back;
-      const unsigned char *ka = p.A + at, *kb = p.B + at;
+      const unsigned char *ka = p.A + at, *kb = b_base + at;
       const int load_stage = free_stage;
       half(zero, load_c, ka, kb, load_stage);
       // tile k + 1 has arrived
@@ -322,6 +352,13 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     break;
   }
 
+  // grouped: the output rows of the pieces that this thread will store
+  constexpr int kPieces = BN / 8, kStores = BM * kPieces / 256;
+  int out_row[kGrouped ? kStores : 1];
+  if constexpr (kGrouped) {
+#pragma unroll
+    for (int u = 0; u < kStores; ++u) out_row[u] = p.sorted_ids[m0 + (u * 256 + threadIdx.x) / kPieces];
+  }
   // ---- epilogue: lane holds columns 4g .. 4g+3 of row x of each block; staged through the LDS so that stores are whole
   // 16-byte pieces of a row
   // (the scales in one round trip, in front of the packing: a load per element and row block in between took longer than a
@@ -353,6 +390,24 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     }
   }
   __syncthreads();
+  if constexpr (kGrouped) {
+    const bool vec = (p.ldc % 8) == 0 && ((uintptr_t)p.C & 15) == 0;
+#pragma unroll
+    for (int u = 0; u < kStores; ++u) {
+      const int idx = u * 256 + threadIdx.x, row = idx / kPieces, col = idx % kPieces * 8;
+      if ((uint32_t)out_row[u] >= (uint32_t)p.num_valid || n0 + col >= p.N) continue;
+      const int4v v = *(const TDIST_AS3 int4v*)(ring + row * C::kEpiPitch + col * 2);
+      unsigned short* dst = (unsigned short*)p.C + (int64_t)out_row[u] * p.ldc + n0 + col;
+      if (vec && n0 + col + 8 <= p.N) {
+        *(int4v*)dst = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (n0 + col + e < p.N) dst[e] = (unsigned short)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+    return;
+  }
   unsigned char* c_base = p.C;
   int row_shift = 0;
   if (p.scatter_bufs) {
@@ -361,7 +416,6 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     row_shift = (p.rank - owner) * p.m_per_rank;
   }
   const bool vec = (p.ldc % 8) == 0 && ((uintptr_t)c_base & 15) == 0;
-  constexpr int kPieces = BN / 8;
   for (int idx = threadIdx.x; idx < BM * kPieces; idx += 256) {
     const int row = idx / kPieces, col = idx % kPieces * 8;
     if (m0 + row >= p.M || n0 + col >= p.N) continue;
@@ -377,10 +431,10 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   }
 }
 
-template <typename E, int BM, int BN, int NST, bool kScales, bool kShards>
-static int launch_shards(const SmallGemmParams& p, hipStream_t stream, const char* who) {
+template <typename E, int BM, int BN, int NST, bool kScales, int kRows>
+static int launch_rows(const SmallGemmParams& p, hipStream_t stream, const char* who) {
   typedef SmallCfg<BM, BN, NST> C;
-  auto kern = gemm_small_kernel<E, BM, BN, NST, kScales, kShards>;
+  auto kern = gemm_small_kernel<E, BM, BN, NST, kScales, kRows>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes);
@@ -394,7 +448,9 @@ static int launch_shards(const SmallGemmParams& p, hipStream_t stream, const cha
 
 template <typename E, int BM, int BN, int NST, bool kScales>
 static int launch_cfg(const SmallGemmParams& p, hipStream_t stream, const char* who) {
-  return p.shards.rows != 0 ? launch_shards<E, BM, BN, NST, kScales, true>(p, stream, who) : launch_shards<E, BM, BN, NST, kScales, false>(p, stream, who);
+  if constexpr (!kScales)
+    if (p.sorted_ids) return launch_rows<E, BM, BN, NST, kScales, kRowsGrouped>(p, stream, who);
+  return p.shards.rows != 0 ? launch_rows<E, BM, BN, NST, kScales, kRowsShards>(p, stream, who) : launch_rows<E, BM, BN, NST, kScales, kRowsPlain>(p, stream, who);
 }
 
 template <int BM, int BN, int NST>

@@ -77,6 +77,7 @@ PROTOTYPES = {
     "tdist_group_gemm_gated_bf16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_f16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
+    "tdist_group_gemm_row_block": (_I, [_L, _I, _I, _L, _L]),
     "tdist_group_gemm_rows": (_I, [_I, _P, _I, _I, _P, _L, _L, _P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _L, _P]),
     "tdist_gemm_split_k_workspace_bytes": (_L, []),
     "tdist_decode_split_kv": (_I, [_P, _P, _P, _P, _P, _F, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I,
@@ -191,6 +192,11 @@ def shard_table(own, peer_shards, rank, num_ranks):
             return None
         table[r] = t.data_ptr()
     return table
+
+
+def address_table(tensor):
+    """A host table with the one address."""
+    return (ctypes.c_void_p * 1)(tensor.data_ptr())
 
 
 def shards_in_reach(table, rows, row_bytes):

@@ -96,7 +96,7 @@ def sort_topk_ids_align_block_size(
 
 
 # Relative time of a 256 x 256 and a 128 x 256 tile (the smaller one runs at 0.8 of the larger one's rate), for the choice
-# of the row block where the caller's is not asked for.
+# of the row block where neither the caller's is asked for nor _block_plan has one.
 _BLOCK_COST = {256: 1.0, 128: 0.625}
 
 
@@ -115,6 +115,13 @@ def _join_plan(entries, num_experts, n):
     return block, (entries + num_experts * (block - 1)) // block
 
 
+def _block_plan(entries, num_experts, n, row_bytes, sk_workspace):
+    """Rows per joined block and the most blocks they can be for tdist_group_gemm_rows, which knows more forms than
+    _row_block does and tells which one is the fastest (16 to 18731 rows over 8 to 64 experts: 39 % on average). None: it cannot."""
+    block = _lib.load().tdist_group_gemm_row_block(entries, num_experts, n, row_bytes, _lib.workspace_args(sk_workspace)[1])
+    return (block, (entries + min(num_experts, entries) * (block - 1)) // block) if block > 0 else None
+
+
 class RowBlocks:
     """Addresses of a grouped GEMM's row blocks (sorted ids, an expert and a segment per block, the padded total), their
     number and their rows; ``memory``: the tensor they lie in."""
@@ -125,7 +132,8 @@ class RowBlocks:
         self.num_blocks, self.block_size, self.memory = num_blocks, block_size, memory
 
 
-def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, block_size, entries, num_experts, n, row_bytes, stream, gather=None):
+def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, block_size, entries, num_experts, n, row_bytes, stream, gather=None,
+                      any_block=False, sk_workspace=None):
     """The rows of ``sorted_ids`` in blocks without rank segments, for a grouped GEMM with ``n`` output columns that waits for
     nobody: RowBlocks, or None where the GEMM does not take rows of ``row_bytes`` in such blocks or the sizes are beyond
     tdist_moe_join_blocks (nothing has been launched then).
@@ -136,14 +144,16 @@ def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, bloc
     They are joined on every call, from what the tensors hold then: a caller may replace or rewrite any of them, also between
     the replays of a graph. (Kept from call to call they cost 7 to 14 us less a layer, and a rewritten routing went unseen.)
     ``made``: the context's memory for them, a RowBlocks per size (a graph may hold the address of any of them).
-    ``gather``: the arguments of tdist_gather_shards but its stream; the same launch then gathers."""
+    ``gather``: the arguments of tdist_gather_shards but its stream; the same launch then gathers. ``any_block``: the caller's
+    GEMM is tdist_group_gemm_rows with ``sk_workspace``, whatever the block."""
     if not (row_bytes % 128 == 0 or row_bytes > 128):
         return None
     _lib.require_cuda(sorted_ids, expert_ids, num_tokens_post_padded)
-    key = (entries, num_experts, n)
+    key = (entries, num_experts, n, any_block and row_bytes)
     out = made.get(key)
     if out is None:
-        block, n_blocks = _join_plan(entries, num_experts, n)
+        plan = _block_plan(entries, num_experts, n, row_bytes, sk_workspace) if any_block else None
+        block, n_blocks = plan or _join_plan(entries, num_experts, n)
         rows = n_blocks * block
         memory = torch.empty(rows + 2 * n_blocks + 1, dtype=torch.int32, device=sorted_ids.device)
         base = memory.data_ptr()
@@ -196,6 +206,24 @@ def _group_gemm(a_ws, a_local, local_row_begin, b_nk, c, blocks, num_valid_token
               int(num_valid_tokens), int(topk), int(tokens_per_rank), int(first_block), _lib.ptr(flags), int(wait_value),
               int(rank), int(spin_limit), _lib.ptr(status), int(max_workgroups), *_lib.workspace_args(sk_workspace),
               _lib.stream_ptr(stream))
+    return c
+
+
+def any_block_fits(a_rows, row_bytes, b_nk, elem_size):
+    """Whether tdist_group_gemm_rows takes such operands in blocks of any size (its offsets are of 32 bits)."""
+    return a_rows * row_bytes < 1 << 32 and b_nk.shape[1] * b_nk.stride(1) * elem_size < 1 << 31
+
+
+def group_gemm_rows(dtype, shards, num_shards, rows_per_shard, b_nk, c, blocks, num_valid_tokens, topk, status=None, sk_workspace=None, stream=None):
+    """Thin wrapper over tdist_group_gemm_rows. ``shards``: addresses of the shards, or of all rows in one piece."""
+    if b_nk.stride(2) != 1 or c.stride(1) != 1:
+        raise ValueError("A, B ([E, N, K]) and C need a contiguous last dimension")
+    _, N, K = b_nk.shape
+    assert c.shape[1] == N
+    _lib.call("tdist_group_gemm_rows", _lib.dtype_code(dtype), shards, num_shards, rows_per_shard, b_nk.data_ptr(), b_nk.stride(1),
+              b_nk.stride(0), c.data_ptr(), c.stride(0), N, K, blocks.sorted_ids, blocks.experts, blocks.segments, blocks.padded,
+              blocks.num_blocks, blocks.block_size, int(num_valid_tokens), int(topk), status, None if status is None else status + 8,
+              *_lib.workspace_args(sk_workspace), stream)
     return c
 
 
@@ -319,21 +347,21 @@ def _gather_and_multiply(a, b_nk, c, ctx, shards):
     if stream != current:
         ctx.group_gemm_stream.wait_stream(torch.cuda.current_stream())
     row_bytes = K * a.element_size()
-    in_place = a.dtype in _GROUP_GEMM_ENTRY and _lib.shards_in_reach(shards, M_per_rank, row_bytes)
+    known = a.dtype in _GROUP_GEMM_ENTRY
+    in_place = known and _lib.shards_in_reach(shards, M_per_rank, row_bytes)
+    any_block = known and any_block_fits(M, row_bytes, b_nk, a.element_size())
     status = ctx.status.data_ptr()
     blocks = joined_row_blocks(ctx.joined, ctx.sorted_topk_ids, ctx.aligned_expert_ids, ctx.aligned_num_tokens, ctx.BLOCK_M, ctx.full_num_tokens,
                                b_nk.shape[0], b_nk.shape[1], row_bytes, stream,
-                               gather=None if in_place else (workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * row_bytes, status, status + 8))
+                               gather=None if in_place else (workspace.data_ptr(), shards, ctx.num_ranks, M_per_rank * row_bytes, status, status + 8),
+                               any_block=any_block, sk_workspace=ctx.sk_workspace)
     if blocks is None:
         return False
+    assert b_nk.shape[2] == K
     if in_place:
-        if b_nk.stride(2) != 1 or c.stride(1) != 1:
-            raise ValueError("A, B ([E, N, K]) and C need a contiguous last dimension")
-        assert b_nk.shape[2] == K and c.shape[1] == b_nk.shape[1]
-        _lib.call("tdist_group_gemm_rows", _lib.dtype_code(a.dtype), shards, ctx.num_ranks, M_per_rank, b_nk.data_ptr(), b_nk.stride(1),
-                  b_nk.stride(0), c.data_ptr(), c.stride(0), b_nk.shape[1], K, blocks.sorted_ids, blocks.experts, blocks.segments,
-                  blocks.padded, blocks.num_blocks, blocks.block_size, int(ctx.full_num_tokens), int(ctx.topk),
-                  status, status + 8, *_lib.workspace_args(ctx.sk_workspace), stream)
+        group_gemm_rows(a.dtype, shards, ctx.num_ranks, M_per_rank, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, status, ctx.sk_workspace, stream)
+    elif any_block:
+        group_gemm_rows(a.dtype, _lib.address_table(workspace), 1, M, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, None, ctx.sk_workspace, stream)
     else:
         _group_gemm(workspace[:M], None, 0, b_nk, c, blocks, ctx.full_num_tokens, ctx.topk, M, 0, None, ctx.rank,
                     sk_workspace=ctx.sk_workspace, stream=ctx.group_gemm_stream)

@@ -14,8 +14,8 @@ from typing import Dict, List, Optional
 import torch
 
 from triton_dist import _lib
-from triton_dist.kernels.amd.allgather_group_gemm import (_group_gemm, group_gemm_gated, joined_row_blocks,
-                                                          sort_topk_ids_align_block_size)
+from triton_dist.kernels.amd.allgather_group_gemm import (_group_gemm, any_block_fits, group_gemm_gated, group_gemm_rows,
+                                                          joined_row_blocks, sort_topk_ids_align_block_size)
 from triton_dist.kernels.amd.low_latency_all_to_all import moe_weighted_combine
 
 
@@ -141,12 +141,17 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     out = ctx.final_output_buffer[:M * topk, :hidden]
     # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local, and
     # blocks that run across the rank segments hold less padding
+    b_nk, row_bytes, stream = _weight_nk(ctx, b), a.shape[1] * a.element_size(), _lib.stream_ptr()
+    any_block = a.is_contiguous() and a.data_ptr() % 16 == 0 and any_block_fits(a.shape[0], row_bytes, b_nk, a.element_size())
     blocks = joined_row_blocks(ctx.joined, pre.full_sorted_token_ids, pre.full_token_expert_ids, pre.full_num_tokens_post_padded_list, pre.BLOCK_M,
-                               pre.full_numel, b.shape[0], hidden, a.shape[1] * a.element_size(), _lib.stream_ptr())
-    if blocks is not None:
-        _group_gemm(a, None, 0, _weight_nk(ctx, b), out, blocks, pre.full_numel, 1, M * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
+                               pre.full_numel, b.shape[0], hidden, row_bytes, stream, any_block=any_block,
+                               sk_workspace=ctx.sk_workspace)
+    if blocks is not None and any_block:
+        group_gemm_rows(a.dtype, _lib.address_table(a), 1, a.shape[0], b_nk, out, blocks, pre.full_numel, 1, None, ctx.sk_workspace, stream)
+    elif blocks is not None:
+        _group_gemm(a, None, 0, b_nk, out, blocks, pre.full_numel, 1, M * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
     else:
-        group_gemm_gated(a, None, 0, _weight_nk(ctx, b), out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
+        group_gemm_gated(a, None, 0, b_nk, out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
                          pre.block_wait_barriers, pre.full_num_tokens_post_padded_list, pre.BLOCK_M, pre.full_numel, 1,
                          pre.num_tokens_per_rank * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
     y = moe_weighted_combine(None, out, None, ctx.identity_index, ctx.topk_weight_f32, from_slots=False)   # [M, hidden]
