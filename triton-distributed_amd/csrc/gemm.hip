@@ -2077,13 +2077,15 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // tiles by a margin.
   const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
   // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
-  // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us, handing over a split round 25 us more
+  // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us (9 where the rows go to their owners' buffers:
+  // 1024 x 7424 x 768 bf16 22.7 us on 256 x 128, 16.1 on 128 x 128; over 60 scatter calls 0.7 % behind the best tile), handing over a split round 25 us more
   // (15 of them in its estimate already)
   // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 14 us on 256 of 128 x 128; 200 x 1536 x 4096 bf16: 26 -> 12 us;
   // 768 x 4952 x 2448 f16 37 -> 26, 2560 x 776 x 5936 68 -> 56; 2048 x 2104 x 4080 stays on the large tiles, 53 us against 70). Most
   // calls that take them are told by a bound that needs no walk (a microsecond of host time less): every tile's work at its rate,
   // no hand-over, no last round.
   const SmallPlan small = small_plan(c, esz, di.num_cus);
+  const double launch_us = c.scatter_bufs ? 9.0 : 6.0;
   if (small.us > 0 && forced_tile < 0) {
     double least = 0;
     for (int t = 0; t < kNumChoices; ++t) {
@@ -2092,7 +2094,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       const double cost = rounds * bm * bn / kChoices[t].eff * c.K * esz / 128.0;
       if (admissible(t) && (least == 0 || cost < least)) least = cost;
     }
-    if (small.us < 0.95 * (6.0 + least / 65536.0 * 1.1)) return run_small(c, elem, esz, small, di);
+    if (small.us < 0.95 * (launch_us + least / 65536.0 * 1.1)) return run_small(c, elem, esz, small, di);
   }
   int pick = 2, pick_split = -1;
   double whole = 0, split_last = 0;
@@ -2117,7 +2119,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   if (use_sk) pick = pick_split;
   const double best = use_sk ? split_last : whole;
   if (small.us > 0) {
-    const double large_us = 6.0 + best / 65536.0 * 1.1 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
+    const double large_us = launch_us + best / 65536.0 * 1.1 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
     if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < 0.95 * large_us)) return run_small(c, elem, esz, small, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,
