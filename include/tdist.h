@@ -378,6 +378,14 @@ int tdist_moe_combine(const void* slot_rows, int row_dtype, const float* slot_sc
                       int world_size, int experts_per_rank, int max_m, int scale_group_size, void* out_bf16,
                       void* stream);
 
+/* The weighted sum of bf16 rows (row t * topk + k with weight topk_w[t, k], fp32, sums in the order of k) and the reduction over the ranks behind it:
+ * sum t of another rank's token goes to sums [n_tokens, hidden] (what a rank sends on; its own rows there are not written); those of the
+ * n_tokens / world_size tokens that `rank` owns are left, rounded to bf16, in slice `rank` of partials [world_size, n_tokens / world_size, hidden], and
+ * out [n_tokens / world_size, hidden] is the sum of the slices in fp32, rank + 1 first. All bf16 but the weights, 16-byte aligned; hidden a multiple of 8,
+ * topk as for tdist_moe_combine. No two of the buffers may overlap. */
+int tdist_moe_combine_reduce(const void* rows, const float* topk_w, int64_t n_tokens, int topk, int hidden, int rank, int world_size, void* partials,
+                             void* sums, void* out, void* stream);
+
 /* Online e4m3 quantisation in groups of group_size = 128 columns.
  *   replaces _quant_kernel / quant_bf16_fp8   tutorials/04-deepseek-infer-all2all.py:309-360
  *   and the fused form in its dispatch kernel  tutorials/04-deepseek-infer-all2all.py:180-200

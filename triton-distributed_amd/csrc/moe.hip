@@ -1129,6 +1129,82 @@ __global__ __launch_bounds__(kCombineWaves * 64) void moe_combine_kernel(
   }
 }
 
+// Weighted sum of a token's rows as above (bf16 rows, row t * topk + k), and for the tokens that this rank owns the reduction over
+// the ranks' partial results right behind it: the wave that has a piece of such a row rounds it, leaves it in the rank's slice of
+// the partials, as the ranks with their own tokens' sums do, and adds the slices up in the order of tdist_reduce_slices, rank + 1 first.
+// Memory-bound: 8192 tokens x 2 of 4096 by 8 ranks 48 us, 5.6 TB/s; as three launches (sum, copy of the own slice, reduction) 58 us
+// and the gaps between them. The own tokens come first: their waves have the most to read.
+template <int kFirst>
+__device__ __forceinline__ void add_slices(float* acc, const int4v* own_chunk, int64_t slice16, int first, int rank, int W, const int4v& own) {
+  for (int i0 = 0; i0 < W; i0 += kFirst) {
+    int4v v[kFirst];
+#pragma unroll
+    for (int j = 0; j < kFirst; ++j) {
+      const int i = min(i0 + j, W - 1);
+      const int s = first + i < W ? first + i : first + i - W;
+      v[j] = own;
+      if (s != rank) v[j] = __builtin_nontemporal_load(own_chunk + (int64_t)s * slice16);
+    }
+#pragma unroll
+    for (int j = 0; j < kFirst; ++j) {
+      if (i0 + j < W) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[2 * q] += BF16::lo((uint32_t)v[j][q]);
+          acc[2 * q + 1] += BF16::hi((uint32_t)v[j][q]);
+        }
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kCombineWaves * 64) void moe_combine_reduce_kernel(
+    const unsigned char* __restrict__ rows, const float* __restrict__ topk_w, int n_tokens, int topk, int hidden, int n_windows, int rank,
+    int W, int m_per, unsigned char* __restrict__ partials, unsigned char* __restrict__ sums, unsigned char* __restrict__ out) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t gw = (int64_t)blockIdx.x * kCombineWaves + wave;
+  if (gw >= (int64_t)n_tokens * n_windows) return;
+  const int turn = (int)(gw / n_windows), win = (int)(gw - (int64_t)turn * n_windows);
+  const int t = turn + rank * m_per < n_tokens ? turn + rank * m_per : turn + rank * m_per - n_tokens;
+  const float coef = lane < topk ? topk_w[(int64_t)t * topk + lane] : 0.f;
+  const int64_t row16 = hidden / 8;
+  const int c = win * 64 + lane;
+  const bool active = c < row16;
+  const int4v* const src = (const int4v*)rows + (int64_t)t * topk * row16 + c;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < topk; k0 += 8) {
+    int4v v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = k0 + j < topk && active ? __builtin_nontemporal_load(src + (k0 + j) * row16) : int4v{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float cf = k0 + j < topk ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, coef), min(k0 + j, topk - 1))) : 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        acc[2 * q] += cf * BF16::lo((uint32_t)v[j][q]);
+        acc[2 * q + 1] += cf * BF16::hi((uint32_t)v[j][q]);
+      }
+    }
+  }
+  if (!active) return;
+  int4v w;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = (int)pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
+  if (turn >= m_per) {   // another rank's token
+    __builtin_nontemporal_store(w, (int4v*)sums + (int64_t)t * row16 + c);
+    return;
+  }
+  const int64_t slice16 = m_per * row16;
+  int4v* const mine = (int4v*)partials + turn * row16 + c;   // of slice 0
+  mine[rank * slice16] = w;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+  add_slices<8>(acc, mine, slice16, rank + 1 < W ? rank + 1 : 0, rank, W, w);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = (int)pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
+  __builtin_nontemporal_store(w, (int4v*)out + turn * row16 + c);
+}
+
 // ---- align / sort for the grouped GEMM ------------------------------------------------------------------
 // Follows moe_ag_scatter_align_block_size_kernel (csrc/lib/moe_utils.cu:60-165): per rank segment, entries grouped
 // by expert in flat order, every group padded to a multiple of block_size, groups and segments laid end to end.
@@ -1899,6 +1975,26 @@ int tdist_moe_post_process(const void* slot_rows, int64_t row_bytes, const float
                      (const unsigned char*)slot_rows, row_bytes, slot_scales, (const int32_t*)nullptr, splits, n_rows,
                      world_size, experts_per_rank, max_m, (unsigned char*)out_rows, out_scales, (int32_t*)nullptr);
   return launch_status("tdist_moe_post_process");
+}
+
+int tdist_moe_combine_reduce(const void* rows, const float* topk_w, int64_t n_tokens, int topk, int hidden, int rank, int world_size, void* partials,
+                             void* sums, void* out, void* stream) {
+  const char* who = "tdist_moe_combine_reduce";
+  if (!rows || !topk_w || !partials || !sums || !out) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (n_tokens < 0 || topk <= 0 || topk > kCombineMaxTopk || hidden <= 0)
+    return fail(TDIST_ERR_INVALID, "%s: bad sizes (topk <= %d)", who, kCombineMaxTopk);
+  if (world_size <= 0 || rank < 0 || rank >= world_size || n_tokens % world_size != 0)
+    return fail(TDIST_ERR_INVALID, "%s: rank %d / world_size %d, %lld tokens", who, rank, world_size, (long long)n_tokens);
+  if (hidden % 8 != 0 || !aligned16(rows) || !aligned16(partials) || !aligned16(sums) || !aligned16(out))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: hidden must be a multiple of 8 and buffers 16-byte aligned", who);
+  if (n_tokens == 0) return TDIST_OK;
+  const int n_windows = (hidden / 8 + 63) / 64;
+  const int64_t blocks = ceil_div(n_tokens * n_windows, kCombineWaves);
+  if (n_tokens > 0x3fffffff || blocks > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: too many tokens", who);
+  hipLaunchKernelGGL(moe_combine_reduce_kernel, dim3((unsigned)blocks), dim3(kCombineWaves * 64), 0, (hipStream_t)stream, (const unsigned char*)rows,
+                     topk_w, (int)n_tokens, topk, hidden, n_windows, rank, world_size, (int)(n_tokens / world_size), (unsigned char*)partials,
+                     (unsigned char*)sums, (unsigned char*)out);
+  return launch_status(who);
 }
 
 int tdist_moe_combine(const void* slot_rows, int row_dtype, const float* slot_scales, const int32_t* scatter_idx,

@@ -16,7 +16,6 @@ import torch
 from triton_dist import _lib
 from triton_dist.kernels.amd.allgather_group_gemm import (_group_gemm, any_block_fits, group_gemm_gated, group_gemm_rows,
                                                           joined_row_blocks, sort_topk_ids_align_block_size)
-from triton_dist.kernels.amd.low_latency_all_to_all import moe_weighted_combine
 
 
 def select_experts(pg, num_ranks, topk, input_dtype, device, router_logits, peer_router_logits=None, rank=0):
@@ -154,14 +153,19 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
         group_gemm_gated(a, None, 0, b_nk, out, pre.full_sorted_token_ids, pre.full_token_expert_ids,
                          pre.block_wait_barriers, pre.full_num_tokens_post_padded_list, pre.BLOCK_M, pre.full_numel, 1,
                          pre.num_tokens_per_rank * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
-    y = moe_weighted_combine(None, out, None, ctx.identity_index, ctx.topk_weight_f32, from_slots=False)   # [M, hidden]
     m_per = M // world_size
     buf = ctx.rs_buffers[ctx.rank]
-    buf[rank * m_per:(rank + 1) * m_per, :hidden].copy_(y[rank * m_per:(rank + 1) * m_per])
-    result = torch.empty((m_per, hidden), dtype=ctx.output_dtype, device=a.device)
-    slab = buf[:M, :hidden]
-    if not slab.is_contiguous():
+    if hidden != buf.shape[1] and not buf[:M, :hidden].is_contiguous():
         raise NotImplementedError("hidden must equal the context's hidden_dim")
-    _lib.call("tdist_reduce_slices", slab.data_ptr(), m_per * hidden, world_size, (rank + 1) % world_size, m_per * hidden,
-              result.data_ptr(), _lib.dtype_code(ctx.output_dtype), _lib.stream_ptr())
+    weight = ctx.topk_weight_f32
+    _lib.require_cuda(out, weight, buf)
+    assert weight.dtype == torch.float32 and weight.is_contiguous() and weight.shape == (M, topk)
+    if out.dtype != torch.bfloat16 or buf.dtype != torch.bfloat16 or not out.is_contiguous():
+        raise TypeError("the context's buffers hold contiguous bf16 rows")
+    # the top-k sums, this rank's slice of the partial results and their reduction in one launch; the sums of the other ranks'
+    # tokens are what this rank would send on
+    sums = torch.empty((M, hidden), dtype=torch.bfloat16, device=a.device)
+    result = torch.empty((m_per, hidden), dtype=ctx.output_dtype, device=a.device)
+    _lib.call("tdist_moe_combine_reduce", out.data_ptr(), weight.data_ptr(), M, topk, hidden, rank, world_size, buf.data_ptr(),
+              sums.data_ptr(), result.data_ptr(), stream)
     return result
