@@ -607,6 +607,19 @@ int tdist_decode_stream(const void* q, const void* k_cache, const void* v_cache,
                         int64_t n_counters, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
                         int64_t out_stride_b, int64_t out_stride_h, float* lse_out, void* stream);
 
+/* tdist_decode_stream of rank `rank`'s shard of the keys with the merge of all ranks' results behind it, in the stream's second launch where the batch
+ * has fewer sequences than the stream has ranges. rank_lens int32 [num_ranks, batch]: every rank's lengths (those of `rank` are the call's own; a rank
+ * without keys of a sequence is left out). rank_out [num_ranks, batch, q_heads, head_dim_v] (strides in elements, last one 1) and rank_lse (fp32,
+ * [batch, q_heads] contiguous per rank) hold the other ranks' results, and get this rank's in its place; out [batch, q_heads, head_dim_v] contiguous. The result has the
+ * bits of tdist_decode_stream followed by tdist_decode_combine in mode 2. */
+int tdist_decode_stream_ranks(const void* q, const void* k_cache, const void* v_cache, float sm_scale, float soft_cap,
+                              const int32_t* block_table, const int32_t* rank_lens, int rank, int num_ranks, int batch, int q_heads, int kv_heads,
+                              int head_dim, int head_dim_v, int page_size, int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_page,
+                              int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+                              int64_t v_stride_head, int64_t table_stride, int dtype, void* workspace, int64_t workspace_bytes, void* rank_out,
+                              int rank_out_dtype, int64_t out_stride_r, int64_t out_stride_b, int64_t out_stride_h, float* rank_lse,
+                              int64_t lse_stride_r, void* out, int out_dtype, void* stream);
+
 /* LSE-weighted merge of P partial results per (b,h) — used for the splits of one shard and for the
  * shards of several ranks:
  *   m = max_j lse[j];  w_j = exp(lse[j]-m);  out = sum_j w_j*part[j] / sum_j w_j;  lse_out = m + log(sum_j w_j)

@@ -73,6 +73,7 @@ struct DecodeParams {
   // streaming form: ranges the batch's blocks are cut into at most, the fewest blocks of a range, and (for the merge) the
   // width of a result's row
   int ranges, min_blocks, dv;
+  const struct RankParams* ranks;   // (host) the other ranks' results to merge with behind the stream, or null
 };
 
 struct MmaBF16 {
@@ -1070,6 +1071,20 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const CombineParams
   if (prm.lse_out && lane == 0) prm.lse_out[bh] = L > 0.f ? M + logf(L) : -INFINITY;
 }
 
+static int launch_combine(const CombineParams& prm, hipStream_t stream) {
+  const int64_t blocks = ceil_div((int64_t)prm.B * prm.Hq, 4);
+  if (blocks > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "tdist_decode_combine: grid too large");
+  auto kern = prm.Dv <= 128 ? decode_combine_kernel<2> : prm.Dv <= 256 ? decode_combine_kernel<4> : decode_combine_kernel<8>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, prm);
+  return launch_status("tdist_decode_combine");
+}
+
+// The merge with the other ranks' results that may follow a stream: rank `own`'s place in c.part and c.lse is the stream's output.
+struct RankParams {
+  CombineParams c;
+  int own, part_vec, out_vec;   // rows of four elements take one load / store
+};
+
 // Fused tail: publishes this team's partial result (the workgroup's, or with kWaveHeads the wave's); the last of the
 // S teams of a (sequence, head block) to get here merges their partials (same arithmetic, in the same order, as
 // decode_combine_kernel in mode 1) and puts the counter back to zero for the next launch.
@@ -1218,8 +1233,13 @@ constexpr int kMergeBatch = 16;   // partial results in flight per lane of the m
 // call, 53 x 100 keys 26.7 -> 18.9, 48 up to 8192 keys with 64 / 8 heads 83.7 -> 80.6, 32 x 32768 655 -> 650. A sequence of many
 // partials beside short ones is read eight partials a trip: 4 uneven sequences up to 21874 keys, 256 ranges, 41.2 us with four
 // waves to a piece, 45.5 alone, hence the bound.
-template <int KEYS, int NW, bool kAlone>
-__global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm) {
+// kRanks (1: 16-bit results, 2: fp32): the merge with the other ranks' results follows in the same launch, for which every sequence
+// has its workgroups: this rank's result goes to its place among the ranks' (or comes from there, where the first launch has left it), as
+// it is rounded there, and then the sums over the ranks as in decode_combine_kernel, in the same order and with the same bits.
+// The other ranks' rows and LSEs are asked for first. With that merge as a launch of its own (6 us) behind this one a sequence-parallel
+// layer of 1 x 1259 keys, 16 heads, 8 ranks took 27.6 us, 18.6 with it; 32 x 32768 keys 658 and 650.
+template <int KEYS, int NW, bool kAlone, int kRanks>
+__global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm, const RankParams rk) {
   constexpr int kBatch = kAlone ? kMergeBatch / 2 : kMergeBatch, kPieces = kAlone ? NW * 64 : 64;   // 16-byte pieces of a workgroup
   __shared__ float4v s_acc[kAlone ? 1 : NW][64];
   __shared__ float s_max[kAlone ? 1 : NW][64], s_sum[kAlone ? 1 : NW][64];
@@ -1227,7 +1247,7 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   const int row_vecs = prm.dv / 4, vecs = prm.Hq * row_vecs, pieces = (vecs + kPieces - 1) / kPieces;
   const int at = blockIdx.x / pieces, piece = blockIdx.x - at * pieces;
   int seq = at, first_block, per;
-  if (prm.B < prm.ranges) {
+  if (kRanks != 0 || prm.B < prm.ranges) {
     stream_sequence<KEYS>(prm, seq, first_block, per);
   } else {
     const StreamRange r = stream_range<KEYS>(prm, at + 1);
@@ -1237,17 +1257,45 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
     per = r.per;
   }
   const int nb = (max(prm.lens[seq], 0) + KEYS - 1) / KEYS;
-  if (nb == 0) return;   // (zeros, stored by the first launch)
-  const int first = first_block / per, parts = (first_block + nb - 1) / per - first + 1;
-  if (parts == 1) return;
+  if (kRanks == 0 && nb == 0) return;   // (zeros, stored by the first launch)
+  const int first = first_block / per, parts = nb == 0 ? 1 : (first_block + nb - 1) / per - first + 1;
+  if (kRanks == 0 && parts == 1) return;
 
   const int my_vec = piece * kPieces + (kAlone ? wave * 64 : 0) + lane, at_vec = min(my_vec, vecs - 1), h = at_vec / row_vecs;
   const int64_t plane = (int64_t)prm.Hq * prm.dv;
   auto slot_of = [&](int j) { return ((int64_t)first + j) * 2 + (j == 0 ? 1 : 0); };
   const int share = kAlone ? parts : (parts + NW - 1) / NW, j_begin = kAlone ? 0 : wave * share, j_end = min(parts, j_begin + share);
+  // the first ranks' results on their way
+  typedef std::conditional_t<kRanks == 2, float4v, int2v> piece_t;
+  constexpr int kRankBatch = kRanks != 0 ? 8 : 1;
+  const int d = (at_vec - h * row_vecs) * 4;
+  piece_t rank_x[kRankBatch];
+  float rank_lse[kRankBatch];
+  auto load_ranks = [&](int r0) {
+#pragma unroll
+    for (int u = 0; u < kRankBatch; ++u) {
+      const int r = min(r0 + u, rk.c.P - 1);
+      const unsigned char* at = rk.c.part + (r * rk.c.p_sp + seq * rk.c.p_sb + h * rk.c.p_sh + d) * (int64_t)(sizeof(piece_t) / 4);
+      if (rk.part_vec) {
+        rank_x[u] = *(const piece_t*)at;
+      } else if constexpr (kRanks == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rank_x[u][e] = ((const float*)at)[e];
+      } else {
+        const unsigned short* a = (const unsigned short*)at;
+        rank_x[u] = int2v{(int)(a[0] | (uint32_t)a[1] << 16), (int)(a[2] | (uint32_t)a[3] << 16)};
+      }
+      // (a rank without keys of the sequence is left out)
+      rank_lse[u] = r0 + u < rk.c.P && r != rk.own && rk.c.lens[(int64_t)r * prm.B + seq] != 0 ? rk.c.lse[r * rk.c.l_sp + seq * rk.c.l_sb + h * rk.c.l_sh] : -INFINITY;
+    }
+  };
+  if constexpr (kRanks != 0) {
+    if (parts == 1 && !kAlone && wave != 0) return;   // (nothing to bring together)
+    if (kAlone || wave == 0) load_ranks(0);
+  }
   float m = -INFINITY, l = 0.f;
   float4v acc = {0.f, 0.f, 0.f, 0.f};
-  for (int j0 = j_begin; j0 < j_end; j0 += kBatch) {
+  for (int j0 = kRanks != 0 && parts == 1 ? j_end : j_begin; j0 < j_end; j0 += kBatch) {
     float4v r[kBatch];
     float w[kBatch];
 #pragma unroll
@@ -1272,7 +1320,7 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
     }
   }
   float M = m, L = l;
-  if constexpr (!kAlone) {
+  if (!kAlone && !(kRanks != 0 && parts == 1)) {
     s_acc[wave][lane] = acc;
     s_max[wave][lane] = m;
     s_sum[wave][lane] = l;
@@ -1295,20 +1343,74 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   if (my_vec >= vecs) return;
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = L > 0.f ? acc[e] / L : 0.f;
-  const int d = (at_vec - h * row_vecs) * 4;
-  store_elem4(prm.final_out, (int64_t)seq * prm.fo_sb + (int64_t)h * prm.fo_sh + d, prm.final_dtype, prm.fo_vec, acc);
-  if (prm.final_lse && d == 0) prm.final_lse[(int64_t)seq * prm.Hq + h] = L > 0.f ? M + logf(L) : -INFINITY;
+  const int64_t final_at = (int64_t)seq * prm.fo_sb + (int64_t)h * prm.fo_sh + d;
+  float lse = L > 0.f ? M + logf(L) : -INFINITY;
+  if (kRanks == 0 || parts > 1) {
+    store_elem4(prm.final_out, final_at, prm.final_dtype, prm.fo_vec, acc);
+    if (prm.final_lse && d == 0) prm.final_lse[(int64_t)seq * prm.Hq + h] = lse;
+  }
+  if constexpr (kRanks != 0) {
+    auto value = [&](const piece_t& x, int e) -> float {
+      if constexpr (kRanks == 2) return x[e];
+      else {
+        const uint32_t bits = (uint32_t)x[e >> 1] >> (16 * (e & 1)) & 0xffffu;
+        return rk.c.part_dtype == TDIST_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+      }
+    };
+    if (parts == 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = load_elem(prm.final_out, final_at + e, prm.final_dtype);
+      lse = prm.final_lse[(int64_t)seq * prm.Hq + h];
+    } else if constexpr (kRanks == 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[e] = rk.c.part_dtype == TDIST_BF16 ? bf16_bits_to_f32(f32_to_bf16_bits(acc[e]) & 0xffffu) : f16_bits_to_f32(pack_f16x2(acc[e], 0.f) & 0xffffu);
+      }
+    }
+    const float own_lse = rk.c.lens[(int64_t)rk.own * prm.B + seq] != 0 ? lse : -INFINITY;
+    float top = own_lse;
+    for (int r0 = 0; r0 < rk.c.P; r0 += kRankBatch) {
+      if (r0 > 0) load_ranks(r0);
+#pragma unroll
+      for (int u = 0; u < kRankBatch; ++u) top = fmaxf(top, rank_lse[u]);
+    }
+    float sum = 0.f;
+    float4v out = {0.f, 0.f, 0.f, 0.f};
+    for (int r0 = 0; r0 < rk.c.P; r0 += kRankBatch) {
+      if (rk.c.P > kRankBatch) load_ranks(r0);
+#pragma unroll
+      for (int u = 0; u < kRankBatch; ++u) {
+        if (r0 + u >= rk.c.P) break;
+        const bool own = r0 + u == rk.own;
+        const float at = own ? own_lse : rank_lse[u];
+        const float w = at == -INFINITY ? 0.f : __expf(at - top);
+        sum += w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] += w * (at == -INFINITY ? 0.f : own ? acc[e] : value(rank_x[u], e));
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = sum > 0.f ? out[e] / sum : 0.f;
+    store_elem4(rk.c.out, (int64_t)seq * rk.c.o_sb + (int64_t)h * rk.c.o_sh + d, rk.c.out_dtype, rk.out_vec, out);
+  }
 }
 
 template <int KEYS, int NW, bool kAlone>
 static int launch_merge_cfg(const DecodeParams& prm, hipStream_t stream) {
   const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), kAlone ? NW * 64 : 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
-  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone>), dim3((unsigned)(places * pieces)), dim3(NW * 64), 0, stream, prm);
-  return launch_status("tdist_decode_stream");
+  const dim3 grid((unsigned)(places * pieces)), block(NW * 64);
+  if (prm.ranks && prm.B < prm.ranges) {
+    if (prm.final_dtype == TDIST_F32) hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 2>), grid, block, 0, stream, prm, *prm.ranks);
+    else hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 1>), grid, block, 0, stream, prm, *prm.ranks);
+    return launch_status("tdist_decode_stream");
+  }
+  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 0>), grid, block, 0, stream, prm, RankParams{});
+  if (int rc = launch_status("tdist_decode_stream")) return rc;
+  return prm.ranks ? launch_combine(prm.ranks->c, stream) : TDIST_OK;
 }
 template <int KEYS>
 static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
-  if (prm.ranges == 1) return TDIST_OK;   // every sequence lies in the one range
+  if (prm.ranges == 1) return prm.ranks ? launch_combine(prm.ranks->c, stream) : TDIST_OK;   // every sequence lies in the one range
   if (prm.ranges <= 16 * prm.B) return launch_merge_cfg<KEYS, 4, true>(prm, stream);
   return prm.ranges > 4 * kMergeBatch * 4 ? launch_merge_cfg<KEYS, 16, false>(prm, stream) : launch_merge_cfg<KEYS, 4, false>(prm, stream);
 }
@@ -1785,6 +1887,7 @@ struct DecodeCall {
   // streaming form
   void* workspace;
   int64_t workspace_bytes;
+  const RankParams* ranks = nullptr;
 };
 
 enum DecodeForm { kFormSplit, kFormFused, kFormStream };
@@ -1880,6 +1983,7 @@ static int run_decode(const DecodeCall& c, DecodeForm form) {
   prm.v_st = c.v_stride_token * 2;
   prm.v_sh = c.v_stride_head * 2;
   prm.t_s = c.table_stride;
+  prm.ranks = c.ranks;
   prm.counters = nullptr;
   prm.final_out = nullptr;
   prm.final_lse = nullptr;
@@ -2116,11 +2220,54 @@ int tdist_decode_combine(const void* part, int part_dtype, const float* lse, int
   prm.l_sh = lse_stride_h;
   prm.o_sb = out_stride_b;
   prm.o_sh = out_stride_h;
-  const int64_t blocks = ceil_div((int64_t)batch * q_heads, 4);
-  if (blocks > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "tdist_decode_combine: grid too large");
-  auto kern = head_dim_v <= 128 ? decode_combine_kernel<2> : head_dim_v <= 256 ? decode_combine_kernel<4> : decode_combine_kernel<8>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, prm);
-  return launch_status("tdist_decode_combine");
+  return launch_combine(prm, (hipStream_t)stream);
+}
+
+int tdist_decode_stream_ranks(const void* q, const void* k_cache, const void* v_cache, float sm_scale, float soft_cap,
+                              const int32_t* block_table, const int32_t* rank_lens, int rank, int num_ranks, int batch, int q_heads, int kv_heads,
+                              int head_dim, int head_dim_v, int page_size, int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_page,
+                              int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+                              int64_t v_stride_head, int64_t table_stride, int dtype, void* workspace, int64_t workspace_bytes, void* rank_out,
+                              int rank_out_dtype, int64_t out_stride_r, int64_t out_stride_b, int64_t out_stride_h, float* rank_lse,
+                              int64_t lse_stride_r, void* out, int out_dtype, void* stream) {
+  const char* who = "tdist_decode_stream_ranks";
+  if (!rank_lens || !rank_out || !rank_lse || !out) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (num_ranks <= 0 || rank < 0 || rank >= num_ranks || batch <= 0 || q_heads <= 0 || head_dim_v <= 0)
+    return fail(TDIST_ERR_INVALID, "%s: rank %d of %d, sizes must be positive", who, rank, num_ranks);
+  if ((rank_out_dtype != TDIST_F32 && rank_out_dtype != TDIST_BF16 && rank_out_dtype != TDIST_F16) ||
+      (out_dtype != TDIST_F32 && out_dtype != TDIST_BF16 && out_dtype != TDIST_F16) || head_dim_v > 512)
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: dtype, or head_dim_v %d > 512", who, head_dim_v);
+  const int esz = rank_out_dtype == TDIST_F32 ? 4 : 2, out_esz = out_dtype == TDIST_F32 ? 4 : 2;
+  RankParams r;
+  r.c.part = (const unsigned char*)rank_out;
+  r.c.lse = rank_lse;
+  r.c.lens = rank_lens;
+  r.c.out = (unsigned char*)out;
+  r.c.lse_out = nullptr;
+  r.c.P = num_ranks;
+  r.c.mode = 2;
+  r.c.B = batch;
+  r.c.Hq = q_heads;
+  r.c.Dv = head_dim_v;
+  r.c.part_dtype = rank_out_dtype;
+  r.c.out_dtype = out_dtype;
+  r.c.p_sp = out_stride_r;
+  r.c.p_sb = out_stride_b;
+  r.c.p_sh = out_stride_h;
+  r.c.l_sp = lse_stride_r;
+  r.c.l_sb = q_heads;
+  r.c.l_sh = 1;
+  r.c.o_sb = (int64_t)q_heads * head_dim_v;
+  r.c.o_sh = head_dim_v;
+  r.own = rank;
+  r.part_vec = (uintptr_t)rank_out % (4 * esz) == 0 && out_stride_r % 4 == 0 && out_stride_b % 4 == 0 && out_stride_h % 4 == 0;
+  r.out_vec = (uintptr_t)out % (4 * out_esz) == 0 && head_dim_v % 4 == 0;
+  DecodeCall c = {q, k_cache, v_cache, nullptr, nullptr, sm_scale, soft_cap, block_table, rank_lens + (int64_t)rank * batch, batch, q_heads,
+                  kv_heads, head_dim, head_dim_v, page_size, 1, q_stride_b, q_stride_h, k_stride_page,
+                  k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, table_stride, dtype,
+                  nullptr, 0, (unsigned char*)rank_out + rank * out_stride_r * esz, rank_out_dtype, out_stride_b, out_stride_h,
+                  rank_lse + rank * lse_stride_r, stream, who, workspace, workspace_bytes, &r};
+  return run_decode(c, kFormStream);
 }
 
 }  // extern "C"

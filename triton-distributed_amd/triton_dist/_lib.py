@@ -89,6 +89,8 @@ PROTOTYPES = {
     "tdist_decode_stream_workspace_bytes": (_L, [_I, _I, _I, _I, _I]),
     "tdist_decode_stream": (_I, [_P, _P, _P, _F, _F, _P, _P, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _L, _L, _L, _I,
                                  _P, _L, _P, _L, _P, _I, _L, _L, _P, _P]),
+    "tdist_decode_stream_ranks": (_I, [_P, _P, _P, _F, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _L, _L, _L, _I,
+                                       _P, _L, _P, _I, _L, _L, _L, _P, _L, _P, _I, _P]),
     "tdist_decode_combine": (_I, [_P, _I, _P, _I, _I, _P, _I, _I, _I, _L, _L, _L, _L, _L, _L, _P, _I, _L, _L, _P, _P]),
 }
 

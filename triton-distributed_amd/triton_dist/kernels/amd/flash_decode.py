@@ -138,12 +138,7 @@ def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, ou
         part, lse, kv_lens = _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, S)
         return decode_combine(part, lse, S, 1, kv_lens, batch, q_heads, dv, (part.stride(2), part.stride(0), part.stride(1)),
                               (lse.stride(2), lse.stride(0), lse.stride(1)), out, lse_out)
-    key = (batch, q_heads, kv_heads, dk, dv, q.device.index)
-    need = _STREAM_PLANS.get(key)
-    if need is None:
-        if len(_STREAM_PLANS) >= 1024:
-            _STREAM_PLANS.clear()
-        need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv)
+    need = _stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv, q.device.index)
     if counters is not None:
         _check_counters(q, kv_heads, counters)
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
@@ -152,6 +147,43 @@ def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, ou
               ks[1], ks[2], vs[0], vs[1], vs[2], block_table.stride(0), _lib.dtype_code(q.dtype), None, 0,
               workspace.data_ptr(), need, out.data_ptr(), _lib.dtype_code(out.dtype), os[0], os[1],
               _lib.ptr(lse_out), _lib.stream_ptr())
+    return out
+
+
+def _stream_workspace_bytes(*key):
+    need = _STREAM_PLANS.get(key)
+    if need is None:
+        if len(_STREAM_PLANS) >= 1024:
+            _STREAM_PLANS.clear()
+        need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(*key[:5])
+    return need
+
+
+def decode_stream_ranks(q, k_cache, v_cache, global_kv_lens, block_table, scale, soft_cap, rank, all_out, all_lse):
+    """tdist_decode_stream_ranks: decode_stream over rank ``rank``'s keys into its place in ``all_out`` [R,B,Hq,Dv] and ``all_lse``
+    (fp32 [R,B,Hq], contiguous per rank), and gqa_fwd_batch_decode_inter_rank_combine of all of them, a launch less. Returns
+    [B,Hq,Dv] in q's dtype, or None where the head dimensions have no streaming form (nothing has been launched then)."""
+    if global_kv_lens.dtype != torch.int32:
+        global_kv_lens = global_kv_lens.to(torch.int32)
+    global_kv_lens = global_kv_lens.contiguous()
+    _, block_table = _check_inputs(q, k_cache, v_cache, global_kv_lens, block_table)
+    batch, q_heads, dk = q.shape
+    _, page_size, kv_heads, dv = v_cache.shape
+    ks, vs = k_cache.stride(), v_cache.stride()
+    if dk > 256 and (k_cache.data_ptr() != v_cache.data_ptr() or ks != vs):
+        return None
+    R = all_out.shape[0]
+    _lib.require_cuda(all_out, all_lse)
+    assert all_lse.shape == (R, batch, q_heads) and all_out.stride(-1) == 1 and global_kv_lens.shape == (R, batch)
+    qs, os = q.stride(), all_out.stride()
+    need = _stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv, q.device.index)
+    workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    out = torch.empty((batch, q_heads, dv), dtype=q.dtype, device=q.device)
+    dtype = _lib.dtype_code(q.dtype)
+    _lib.call("tdist_decode_stream_ranks", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), scale, soft_cap, block_table.data_ptr(),
+              global_kv_lens.data_ptr(), rank, R, batch, q_heads, kv_heads, dk, dv, page_size, qs[0], qs[1], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2],
+              block_table.stride(0), dtype, workspace.data_ptr(), need, all_out.data_ptr(), _lib.dtype_code(all_out.dtype), os[0], os[1], os[2],
+              all_lse.data_ptr(), all_lse.stride(0), out.data_ptr(), dtype, _lib.stream_ptr())
     return out
 
 

@@ -8,7 +8,7 @@ the gather has nobody to talk to: the partial results of the other ranks are pas
 """
 import torch
 
-from triton_dist.kernels.amd.flash_decode import decode_stream, gqa_fwd_batch_decode_inter_rank_combine
+from triton_dist.kernels.amd.flash_decode import decode_stream, decode_stream_ranks, gqa_fwd_batch_decode_inter_rank_combine
 
 
 class SpGQAFlashDecodeAttention(torch.nn.Module):
@@ -57,6 +57,12 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
             all_out, all_lse = peer_partials
             assert all_out.shape == (self.num_ranks, batch, self.num_q_heads, self.v_head_dim)
             assert all_lse.shape == (self.num_ranks, batch, self.num_q_heads)
+        strides = all_lse.stride()
+        if all_lse.dtype == torch.float32 and strides[2] == 1 and strides[1] == self.num_q_heads:
+            # the own result into its place, and the merge of all ranks', in the stream's two launches
+            out = decode_stream_ranks(q, k_cache, v_cache, global_kv_lens, block_table, self.scale, self.soft_cap, self.rank, all_out, all_lse)
+            if out is not None:
+                return out
         # the own result goes straight into its place in the gather buffers (reference :133-135 copies it there)
         own_out, own_lse = all_out[self.rank], all_lse[self.rank]
         lse = own_lse if own_lse.dtype == torch.float32 and own_lse.is_contiguous() else torch.empty_like(
