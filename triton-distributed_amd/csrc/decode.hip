@@ -249,12 +249,7 @@ __device__ __forceinline__ StreamRange stream_range(const DecodeParams& prm, int
   int nb = 0, sum = 0, total = 0;
   auto scan = [&](int i0) {   // sum: this lane's sequence and the ones before it within the 64
     nb = blocks(i0 + lane);
-    sum = nb;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(sum, o);
-      if (lane >= o) sum += t;
-    }
+    sum = wave_scan_add(nb);
   };
   for (int i0 = 0; i0 < prm.B; i0 += 64) {
     scan(i0);
@@ -295,13 +290,8 @@ __device__ __forceinline__ void stream_sequence(const DecodeParams& prm, int seq
     total += nb;
     before += i < seq ? nb : 0;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    total += __shfl_xor(total, o);
-    before += __shfl_xor(before, o);
-  }
-  first_block = __builtin_amdgcn_readfirstlane(before);
-  per = stream_blocks_per_range(prm, __builtin_amdgcn_readfirstlane(total));
+  first_block = wave_sum(before);
+  per = stream_blocks_per_range(prm, wave_sum(total));
 }
 
 // Are the B sequence lengths even enough for the form that hands a workgroup 8 kv heads of one (sequence, split)?
@@ -662,8 +652,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     // times per stream instead of per block.
     constexpr float kSlack = 8.f;
     if (__any(mx > m_run + kSlack)) {
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      mx = max_lane_xor<32>(max_lane_xor<16>(mx));
       const float m_new = fmaxf(m_run, mx);
       const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
@@ -777,8 +766,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       wait_groups<C::kLoadsPerGroup>(min(C::kP, sr.n - 1 - i));
       compute(i, w_cmp.blk);
       if (w_cmp.left == 1) {
-        float L = l_run + __shfl_xor(l_run, 16);
-        L += __shfl_xor(L, 32);
+        const float L = sum_lane_xor<32>(sum_lane_xor<16>(l_run));
         const float inv = L > 0.f ? 1.f / L : 0.f;
         const float r_lse = L > 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
         const bool ends = w_cmp.blk.key0 + KEYS >= w_cmp.blk.hi;
@@ -858,8 +846,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
       compute(i, c_cmp.blk);
       if (c_cmp.left == 1) {
         // the split's last block: this lane holds dimensions 16d + 4g .. + 3 of head x
-        float L = l_run + __shfl_xor(l_run, 16);
-        L += __shfl_xor(L, 32);
+        const float L = sum_lane_xor<32>(sum_lane_xor<16>(l_run));
         float4v r[DT];
 #pragma unroll
         for (int d = 0; d < DT; ++d)
@@ -926,8 +913,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
   }
 
   // ---- merge the waves' partial states ---------------------------------------------------------
-  l_run += __shfl_xor(l_run, 16);
-  l_run += __shfl_xor(l_run, 32);
+  l_run = sum_lane_xor<32>(sum_lane_xor<16>(l_run));
   wait_vmcnt<0>();
   __syncthreads();  // every wave is done with its ring; reuse it
   TDIST_AS3 float* s_m = (TDIST_AS3 float*)(wbase);  // [16]
@@ -950,12 +936,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& prm) {
     const int w = lane >> 4, h = lane & 15;
     const TDIST_AS3 float* wm = (const TDIST_AS3 float*)(smem3 + min(w, NW - 1) * C::kWaveBytes);
     const float mw = w < NW ? wm[h] : -INFINITY;
-    float M = fmaxf(mw, __shfl_xor(mw, 16));
-    M = fmaxf(M, __shfl_xor(M, 32));
+    const float M = max_lane_xor<32>(max_lane_xor<16>(mw));
     const float sc = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
     float L = w < NW ? wm[16 + h] * sc : 0.f;
-    L += __shfl_xor(L, 16);
-    L += __shfl_xor(L, 32);
+    L = sum_lane_xor<32>(sum_lane_xor<16>(L));
     s_w[lane] = sc / L;
     r_lse16 = (M + log2f(L)) * kLn2;
   }
@@ -1595,8 +1579,7 @@ __global__ __launch_bounds__(LatentCfg<HB>::kThreads) void decode_latent_kernel(
       constexpr float kSlack = 8.f;
       const int raised = __any(mx > m_run + kSlack);
       if (raised) {
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = max_lane_xor<32>(max_lane_xor<16>(mx));
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
         if (g == 0) s_alpha[((i & 1) * HB + hb) * 16 + x] = alpha;
@@ -1620,8 +1603,7 @@ __global__ __launch_bounds__(LatentCfg<HB>::kThreads) void decode_latent_kernel(
       }
       if (w.left == 1) {
         // the sequence's last block in this range
-        float L = l_run + __shfl_xor(l_run, 16);
-        L += __shfl_xor(L, 32);
+        const float L = sum_lane_xor<32>(sum_lane_xor<16>(l_run));
         if (g == 0) {
           TDIST_AS3 float* e = s_end + (((i & 1) * HB + hb) * 16 + x) * 2;
           e[0] = L > 0.f ? 1.f / L : 0.f;

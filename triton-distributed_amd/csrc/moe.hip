@@ -415,12 +415,7 @@ __global__ __launch_bounds__(kThreads) void moe_index_fused_kernel(const int32_t
   int32_t local_total = 0;
   for (int j = 0; j < per; ++j)
     if (g0 + j < G) local_total += s_col[g0 + j];
-  int32_t incl = local_total;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int32_t t = __shfl_up(incl, off);
-    if (lane >= off) incl += t;
-  }
+  const int32_t incl = wave_scan_add(local_total);
   if (lane == 63) s_part[wave] = incl;
   __syncthreads();
   int32_t acc = incl - local_total;  // ids of the experts before this thread's first one
@@ -682,7 +677,7 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(const unsigned
 // Few tokens: windows of `vecs` < 8 KB, so that a row is shared by several waves and the rows by more workgroups. What 16
 // whole rows per workgroup cost a decode step of 128 tokens x 8 copies of 7168 B is eight compute units storing 7.3 MB:
 // 14.5 us, against 12.2 us with eight waves to a row (64 workgroups; twice as many: the same, four times: 18 for 13 us at 600
-// tokens). Up to the scan the launch takes 4.3 us; behind it, instructions and waits in a row are what counts, not bytes: 8.8 us
+// tokens). Up to the scan the launch takes 4.3 us; behind it, instructions and waits in a row are what counts, not bytes: 8.4 us
 // (from 12.1) since a token's scale is asked for at the start, the copies' rows and windows are the wave's (scalar branches
 // instead of eight tests a lane and copy) and the search among the workgroup's own entries has its reads in flight together.
 // 64-bit ids are read as they are (a conversion of 1024 of them in front: 3 us and a launch).
@@ -806,12 +801,7 @@ __global__ __launch_bounds__(kFdThreads) void moe_dispatch_fused_kernel(
   int32_t local_total = 0;
   for (int j = 0; j < per; ++j)
     if (g0 + j < G) local_total += s_before[g0 + j] + s_own[g0 + j] + s_behind[g0 + j];
-  int32_t incl = local_total;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int32_t up = __shfl_up(incl, off);
-    if (lane >= off) incl += up;
-  }
+  const int32_t incl = wave_scan_add(local_total);
   if (lane == 63) s_part[wave] = incl;
   __syncthreads();
   int32_t acc = incl - local_total;
@@ -1291,7 +1281,7 @@ __global__ __launch_bounds__(kPlaceThreads) void moe_align_place_kernel(
 // What bounds it: two trips to memory and the work per group, of which there are thousands. The eight waves' counts of a
 // group are the bytes of one 64-bit word (a wave has at most 128 entries), so a group is 20 bytes to clear, to add up (four
 // groups a step, the bytes of a word by a sum of absolute differences) and to look up, and nothing is written back per
-// wave: the sizes above take 6.7 us, 12.4 with a row of counters per wave (of which 7 were clearing, sums and scan). With
+// wave: the sizes above take 6.4 us, 12.4 with a row of counters per wave (of which 7 were clearing, sums and scan). With
 // 32768 entries 12.7 (of 64 groups 11.6): there it is the counting, 64 LDS atomics per thread.
 constexpr int kAlignFillPerBlock = 1024;
 constexpr int kAlignMostQuads = (kMoeMaxExperts / 4 + kFusedThreads - 1) / kFusedThreads;   // steps of four groups per thread
@@ -1462,12 +1452,7 @@ __global__ __launch_bounds__(kFusedThreads) void moe_align_fused_kernel(
       }
     }
   }
-  int32_t incl = local_total;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int32_t t = __shfl_up(incl, off);
-    if (lane >= off) incl += t;
-  }
+  const int32_t incl = wave_scan_add(local_total);
   if (lane == 63) s_part[wave] = incl;
   __syncthreads();
   int32_t acc = incl - local_total, total = 0;
@@ -1716,12 +1701,7 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
     const int e = threadIdx.x * per + i;
     if (e < E) own += padded(s_total[e]);
   }
-  int sum = own;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(sum, o);
-    if (lane >= o) sum += t;
-  }
+  const int sum = wave_scan_add(own);
   if (lane == 63) s_part[wave] = sum;
   __syncthreads();
   int at = sum - own, all = 0;
@@ -1746,8 +1726,7 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
       const int v = s_block[i];
       before += v >> kJoinCountBits == e ? v & kCountMask : 0;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+    before = wave_sum(before);
     int row = s_start[e] + before;
     auto place = [&](int id) {
       const unsigned long long is = __ballot(valid(id));
