@@ -1212,7 +1212,7 @@ constexpr int kMergeBatch = 16;   // partial results in flight per lane of the m
 // instead of 156 with 6 / 1 heads and 87 instead of 155 with 32 / 8 (32 splits and their combine: 90, 91).
 // 16 waves a workgroup where a sequence may have more partials than four waves hold in flight.
 // kAlone: every wave takes 64 pieces of its own and all partials of them, eight in flight, and there is nothing to bring together:
-// for batches whose sequences have few partials each (16 on average at most), where the other form's four waves share a handful and
+// for batches whose sequences have few partials each (kAloneMost), where the other form's four waves share a handful and
 // there are four times as many workgroups, each with its trip for the lengths: latent heads, 16 up to 4096 keys 39.2 -> 31.2 us a
 // call, 53 x 100 keys 26.7 -> 18.9, 48 up to 8192 keys with 64 / 8 heads 83.7 -> 80.6, 32 x 32768 655 -> 650. A sequence of many
 // partials beside short ones is read eight partials a trip: 4 uneven sequences up to 21874 keys, 256 ranges, 41.2 us with four
@@ -1379,6 +1379,11 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   }
 }
 
+// Ranges per sequence up to which every wave merges its pieces alone (see above): uneven sequences have several times the average.
+// 16 sequences up to 4000 keys, 32 / 8 heads, 8 ranges each: 23.4 us a call alone, 22.2 with four waves to a piece; 10 up to 15128 keys 42.3 and
+// 40.0; 30, 4.3 ranges each, 70.6 either way. Latent heads have four times the pieces: 12 sequences up to 4096 keys, 5.3 ranges each, 26.7 and 32.8;
+// 8 up to 16000 40.1 and 42.9.
+constexpr int kAloneMost = 5, kLatentAloneMost = 16;
 template <int KEYS, int NW, bool kAlone>
 static int launch_merge_cfg(const DecodeParams& prm, hipStream_t stream) {
   const int64_t pieces = ceil_div((int64_t)prm.Hq * (prm.dv / 4), kAlone ? NW * 64 : 64), places = prm.B < prm.ranges ? prm.B : prm.ranges - 1;
@@ -1393,9 +1398,9 @@ static int launch_merge_cfg(const DecodeParams& prm, hipStream_t stream) {
   return prm.ranks ? launch_combine(prm.ranks->c, stream) : TDIST_OK;
 }
 template <int KEYS>
-static int launch_stream_merge(const DecodeParams& prm, hipStream_t stream) {
+static int launch_stream_merge(const DecodeParams& prm, int alone_most, hipStream_t stream) {
   if (prm.ranges == 1) return prm.ranks ? launch_combine(prm.ranks->c, stream) : TDIST_OK;   // every sequence lies in the one range
-  if (prm.ranges <= 16 * prm.B) return launch_merge_cfg<KEYS, 4, true>(prm, stream);
+  if (prm.ranges <= alone_most * prm.B) return launch_merge_cfg<KEYS, 4, true>(prm, stream);
   return prm.ranges > 4 * kMergeBatch * 4 ? launch_merge_cfg<KEYS, 16, false>(prm, stream) : launch_merge_cfg<KEYS, 4, false>(prm, stream);
 }
 
@@ -1797,7 +1802,7 @@ static int launch_latent_cfg(DecodeParams& prm, hipStream_t stream) {
   const int64_t sets = ceil_div(prm.Hq / prm.Hkv, HB * 16);
   hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)prm.ranges * prm.Hkv * sets)), dim3(C::kThreads), C::kLds, stream, prm);
   if (int rc = launch_status("tdist_decode_stream")) return rc;
-  return launch_stream_merge<C::kKeys>(prm, stream);
+  return launch_stream_merge<C::kKeys>(prm, kLatentAloneMost, stream);
 }
 
 template <typename MMA>
@@ -1823,7 +1828,7 @@ static int launch_stream_cfg(DecodeParams& prm, int head_blocks, hipStream_t str
   const int64_t waves = (int64_t)prm.ranges * prm.Hkv * head_blocks;
   hipLaunchKernelGGL(kern, dim3((unsigned)((waves + NW - 1) / NW)), dim3(NW * 64), lds, stream, prm);
   if (int rc = launch_status("tdist_decode_stream")) return rc;
-  return launch_stream_merge<KEYS>(prm, stream);
+  return launch_stream_merge<KEYS>(prm, kAloneMost, stream);
 }
 
 template <typename MMA, int D, int DPE, int KEYS, int NW, int NST, bool kPadded>

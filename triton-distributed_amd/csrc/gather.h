@@ -50,7 +50,7 @@ struct ShardRows {
   uint32_t off[kMaxShards];           // bytes
   int32_t *status, *first_error;      // optional: retired by the kernel that reads the rows, as a gather's launch does
 };
-// What the first workgroup of that kernel does first.
+// What the first workgroup of that kernel does beside its tiles.
 __device__ __forceinline__ void retire_beside(const ShardRows& s) {
   if (s.rows != 0 && s.status != nullptr && blockIdx.x == 0 && threadIdx.x == 0) retire_status(s.status, s.first_error);
 }

@@ -402,7 +402,6 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       asm volatile("" : "+v"(frag_lane_a[q]), "+v"(frag_lane_a_hi[q]), "+v"(frag_lane_b[q]));
     }
   }
-  if constexpr (!kGrouped || kPlain) retire_beside(p.shards);
   const int num_pid_m = (p.M + BM - 1) / BM;
   const int num_pid_n = (p.N + BN - 1) / BN;
   const int cm = p.m_per_chunk / BM;                 // row tiles per chunk
@@ -1786,6 +1785,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       }
     }
   }
+  if constexpr (!kGrouped || kPlain) retire_beside(p.shards);   // (in front of the tiles its test held the first loads up: 0.4 of 53 us)
   // ---- the last workgroup out advances the workspace's tag base for the next launch --------------------------
   if (p.sk_mode != 0 && threadIdx.x == 0) {
     int32_t* const done = p.sk_ctrl + kSkCtrlDone;
@@ -2021,6 +2021,9 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // before: 2048 x 4304 x 3040 f16 79 -> 57 us, 7168 x 7128 x 3792 e4m3 241 -> 179; the smaller tiles fetch more operand bytes
   // per product, and the 256x256 tile alone has an instance without gating code)
   static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.70}, {128, 128, 0.48}, {128, 192, 0.62}, {128, 256, 0.70}};
+  // (behind flags the 256x256 tile has gating code too, and the 256x128 one is nearer to it: 4096 x 5208 x 3008 bf16 134 us on the large tile,
+  // 115 on three rounds of the other; 26 gated shapes are 0.9 % behind the best tile, 2.0 % with 0.70 and 5.5 % with 0.88)
+  auto rate = [&](int t) { return t == 1 && c.flags ? 0.80 : kChoices[t].eff; };
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
   // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
@@ -2047,7 +2050,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   auto walk = [&](int t, bool split_last) -> Walk {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int tiles_m = (c.M + bm - 1) / bm, tiles_n = (c.N + bn - 1) / bn;
-    const double per_k_tile = (double)bm * bn / kChoices[t].eff;
+    const double per_k_tile = (double)bm * bn / rate(t);
     auto rounds = [&](int64_t positions) -> double {
       const int64_t full = positions < 0x7fffffff ? (int)positions / cap_wgs : positions / cap_wgs, tail = positions - full * cap_wgs;
       if (tail == 0 || !split_last) return (double)(full + (tail != 0));
@@ -2091,7 +2094,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     for (int t = 0; t < kNumChoices; ++t) {
       const int bm = kChoices[t].bm, bn = kChoices[t].bn;
       const double tiles = (double)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn), rounds = std::max(tiles / cap_wgs, 1.0 / kSkMaxSplit);
-      const double cost = rounds * bm * bn / kChoices[t].eff * c.K * esz / 128.0;
+      const double cost = rounds * bm * bn / rate(t) * c.K * esz / 128.0;
       if (admissible(t) && (least == 0 || cost < least)) least = cost;
     }
     if (small.us < 0.95 * (launch_us + least / 65536.0 * 1.1)) return run_small(c, elem, esz, small, di);
@@ -2110,7 +2113,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
       // (and 15 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
-      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / kChoices[t].eff) + 15.0 / 1.2 * 65536.0;
+      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / rate(t)) + 15.0 / 1.2 * 65536.0;
       if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
   }
