@@ -33,24 +33,22 @@ PEAK = {"bf16": 2.5e15, "fp8": 5.0e15, "hbm": 8.0e12}  # MI355X published dense 
 # the summaries are kept under profiles/. Each figure names the kernel sources it was measured on, and
 # MEASURED_SOURCE_DIGEST holds those sources' digests at the time: a figure whose sources have changed since is
 # reported as null, not as a measurement (tests/test_bench_constants.py fails until it is measured again).
-GEMM_SOURCES = ("gemm.hip", "gemm_small.hip", "gemm_small.h", "common.h")   # (the small tiles take part in the choice of a tile)
+GEMM_SOURCES = ("gemm.hip", "gemm_small.hip", "gemm_small.h", "gather.h", "common.h")   # (the small tiles take part in the choice of a tile)
 MEASURED_TRAFFIC_BYTES = {
     "c2_gemm": (840.0e6, GEMM_SOURCES), "c2_reduce": (151.0e6, ("reduce.hip", "common.h")),
     "c1_gemm": (130.4e6, GEMM_SOURCES), "c3_gemm": (1646.0e6, GEMM_SOURCES),
-    "c3_gather": (268.4e6, ("lib.hip", "gather.h", "common.h")),
     "c4_dispatch": (265.8e6, ("moe.hip", "common.h")), "c4_dispatch_from_ids": (267.4e6, ("moe.hip", "common.h")),
     "c4_combine": (296.7e6, ("moe.hip", "common.h")), "c5_split_kv": (4318.1e6, ("decode.hip", "common.h")),
     "c5_stream": (4302.1e6, ("decode.hip", "common.h")),
 }
 MEASURED_SOURCE_DIGEST = {
-    "common.h": "29a71d5d51010d68",
-    "decode.hip": "7741974f667a3d5e",
-    "gather.h": "efd413b797d8716f",
-    "gemm.hip": "e637df29a212e7ee",
-    "gemm_small.h": "6e8a49fb30ce162c",
-    "gemm_small.hip": "bbc3652da8a55a10",
-    "lib.hip": "f0a1cb9af6a3eaba",
-    "moe.hip": "97f23dc5aa4ab792",
+    "common.h": "f5b639d6f2c93627",
+    "decode.hip": "5ea65a9c7115a3b6",
+    "gather.h": "3fd5e450cd06de4d",
+    "gemm.hip": "1a895ba16559069c",
+    "gemm_small.h": "ef635860051b59ae",
+    "gemm_small.hip": "9f3cf4730167f9a0",
+    "moe.hip": "b232f7830cc66aab",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")
@@ -134,13 +132,13 @@ def time_live_ag_gemm(call, ctx, steps, warmup):
     return s, "copies_first"
 
 
-def rows_gathered(call, ctx, steps, warmup, traffic=None):
-    """The same call in a context that asks for no arrivals: every peer's shard is at hand, so one launch gathers the rows
-    and the product runs ungated behind it. ``traffic``: the measured HBM-side bytes of the gather launch."""
+def rows_gathered(call, ctx, steps, warmup):
+    """The same call in a context that asks for no arrivals: every peer's shard is at hand, so the product runs ungated and
+    reads the rows where they lie."""
     call()
     s = time_launches(call, steps, warmup)
     ctx.check_status()
-    return dict({"us": round(s * 1e6, 2)}, **({} if traffic is None else {"gather_traffic": traffic}))
+    return {"us": round(s * 1e6, 2)}
 
 
 XGMI_LINK_GBPS = 153.0   # one xGMI link of MI355X: the rate at which one peer's rows arrive
@@ -344,8 +342,7 @@ def bench_c3(dev, steps, warmup):
     if LIVE_PRODUCER:
         live_s, live_order = time_live_ag_gemm(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb),
                                                ctx, steps, warmup)
-        at_hand = rows_gathered(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb), ctx, steps,
-                                warmup, measured_traffic("c3_gather"))
+        at_hand = rows_gathered(lambda: ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb), ctx, steps, warmup)
         c = ag_gemm_intra_node(a_d, b_d, False, ctx, row_scale=sa, col_scale=sb)
         ctx.check_status()
         rows = slice(5 * mpr + 11, 5 * mpr + 75)

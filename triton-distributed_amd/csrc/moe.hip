@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(kPlaceThreads) void moe_align_place_kernel(
 // group are the bytes of one 64-bit word (a wave has at most 128 entries), so a group is 20 bytes to clear, to add up (four
 // groups a step, the bytes of a word by a sum of absolute differences) and to look up, and nothing is written back per
 // wave: the sizes above take 6.4 us, 12.4 with a row of counters per wave (of which 7 were clearing, sums and scan). With
-// 32768 entries 12.7 (of 64 groups 11.6): there it is the counting, 64 LDS atomics per thread.
+// 32768 entries 12.7 (64 experts: 11.6): there it is the counting, 64 LDS atomics per thread.
 constexpr int kAlignFillPerBlock = 1024;
 constexpr int kAlignMostQuads = (kMoeMaxExperts / 4 + kFusedThreads - 1) / kFusedThreads;   // steps of four groups per thread
 static int64_t align_lds_bytes(int64_t G) { return 20 * ((G + 3) / 4 * 4) + 16 + 256; }

@@ -6,7 +6,7 @@ Keeps the interface of the reference's kernels/nvidia/moe_reduce_rs.py: ``select
 (:280-361) and ``moe_reduce_rs`` (:889-...). The three device steps are the library's grouped GEMM
 (kernel_producer_group_gemm_tp_scatter_input, :365-468), the weighted combine (the top-k sum of
 kernel_consumer_topk_reduce_scatter_intra_node, :471-546) and the ordered slice reduction (kernel_consumer_reduce,
-:549-587). With one GPU the other ranks' router logits and partial results are handed to the context
+:549-587), the last two in one launch. With one GPU the other ranks' router logits and partial results are handed to the context
 (``peer_router_logits=``, ``ctx.set_peer_partials``)."""
 import dataclasses
 from typing import Dict, List, Optional
