@@ -1824,7 +1824,10 @@ static int launch_stream_cfg(DecodeParams& prm, int head_blocks, hipStream_t str
     if (e != hipSuccess) return fail(TDIST_ERR_LAUNCH, "decode: cannot reserve %zu B of LDS: %s", lds, hipGetErrorString(e));
     attr_set = true;
   }
-  prm.min_blocks = 64 / KEYS;
+  // The fewest keys of a range: half of them in one wave are a shorter chain, twice the partial results are a little more to merge (launches of 1 x 1320
+  // keys, 32 / 8 heads: 64 keys 9.8 + 3.9 us, 32 7.5 + 4.6, 16 6.5 + 6.4; 2 x up to 1679 of 256-wide heads 16.2 + 4.0, 12.2 + 4.2, 10.3 + 6.6; 20 x up to 400
+  // 12.8 + 4.5, 9.2 + 5.1, 9.4 + 5.1).
+  prm.min_blocks = 32 / KEYS;
   const int64_t waves = (int64_t)prm.ranges * prm.Hkv * head_blocks;
   hipLaunchKernelGGL(kern, dim3((unsigned)((waves + NW - 1) / NW)), dim3(NW * 64), lds, stream, prm);
   if (int rc = launch_status("tdist_decode_stream")) return rc;
