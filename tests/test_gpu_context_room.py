@@ -1,0 +1,30 @@
+"""Calls whose rows the context has no room for are refused, on every route."""
+import pytest
+import torch
+
+from tests.conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _ag_gemm(cuda, made_for, dtype, m_per_rank, K, flags):
+    from triton_dist.kernels.amd import ag_gemm_intra_node, create_ag_gemm_intra_node_context
+    W, N = 2, 256
+    ctx = create_ag_gemm_intra_node_context(W * 128, N, 256, made_for, torch.bfloat16, 0, W, None, M_PER_CHUNK=128)
+    ctx.preset_flags = flags
+    shards = [torch.ones((m_per_rank, K), device=cuda).to(dtype) for _ in range(W)]
+    ctx.set_peer_shards({1: shards[1]})
+    return ag_gemm_intra_node(shards[0], torch.ones((N, K), device=cuda).to(dtype), False, ctx)
+
+
+@pytest.mark.parametrize("flags", [False, True])
+@pytest.mark.parametrize("made_for,dtype,m_per_rank,K", [
+    (torch.float8_e4m3fn, torch.bfloat16, 128, 256), (torch.bfloat16, torch.bfloat16, 256, 256), (torch.bfloat16, torch.bfloat16, 128, 264)])
+def test_ag_gemm_refuses_rows_beyond_the_workspace(cuda, flags, made_for, dtype, m_per_rank, K):
+    announce("ag_gemm: a workspace for less than %s %d x %d" % (dtype, m_per_rank, K))
+    with pytest.raises(ValueError):
+        _ag_gemm(cuda, made_for, dtype, m_per_rank, K, flags)
+    # what fits is taken: another type of the same size and (rows at hand) more columns of a narrower one
+    if not flags:
+        assert float(_ag_gemm(cuda, torch.bfloat16, torch.float16, 128, 256, flags)[0, 0]) == 256
+        assert float(_ag_gemm(cuda, torch.bfloat16, torch.float8_e4m3fn, 128, 512, flags)[0, 0]) == 512

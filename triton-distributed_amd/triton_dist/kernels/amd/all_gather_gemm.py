@@ -334,6 +334,9 @@ def ag_gemm_intra_node_op(a, b, c, rank, num_ranks, workspace_tensors, one, barr
     M_per_rank, K = a.shape
     M = M_per_rank * num_ranks
     workspace = workspace_tensors[rank]
+    _check_room(workspace, a, num_ranks)
+    if workspace.element_size() != a.element_size() or workspace.shape[1] != K:   # (the GEMM takes rows and type from it)
+        raise ValueError("the workspace holds rows of %d %s, not of %d %s" % (workspace.shape[1], workspace.dtype, K, a.dtype))
     barrier = barrier_tensors[rank]
     peer_shards = ctx.peer_shards if ctx is not None else {}
     if num_ranks > 1:
@@ -432,6 +435,13 @@ def _rows_are_at_hand(a, ctx):
                 or ctx.held_chunks or ctx.late_chunks_us or ctx.random_delay_us > 0) and a.is_contiguous()
 
 
+def _check_room(workspace, a, num_ranks):
+    """What a gather or the copies write is sized by ``a``: the context's workspace has to have room for it, in bytes."""
+    if workspace.nbytes < num_ranks * a.nbytes:
+        raise ValueError("the context's workspace of %d bytes has no room for %d shards of %d x %d %s"
+                         % (workspace.nbytes, num_ranks, *a.shape, a.dtype))
+
+
 def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
     """The product of every rank's rows, read where they lie, in one launch; where they lie too far apart, one launch brings them into
     the workspace first (tdist_ag_gemm_rows). With the rows at hand a GEMM that shares the chip with copies, keeps 32 compute units
@@ -446,8 +456,7 @@ def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
         raise ValueError("scales are only defined for fp8 inputs")
     if a.dtype not in _GEMM_ENTRY:
         raise TypeError("unsupported GEMM dtype %s" % a.dtype)
-    if workspace.numel() < num_ranks * M_per_rank * K:
-        raise ValueError("the context was created for fewer rows or columns than %d x %d" % (num_ranks * M_per_rank, K))
+    _check_room(workspace, a, num_ranks)
     current = _lib.stream_ptr()
     stream = ctx.gemm_stream.cuda_stream
     if stream != current:
