@@ -24,7 +24,9 @@ def test_ag_gemm_refuses_rows_beyond_the_workspace(cuda, flags, made_for, dtype,
     announce("ag_gemm: a workspace for less than %s %d x %d" % (dtype, m_per_rank, K))
     with pytest.raises(ValueError):
         _ag_gemm(cuda, made_for, dtype, m_per_rank, K, flags)
-    # what fits is taken: another type of the same size and (rows at hand) more columns of a narrower one
+    # what fits is taken: another type of the same size, (rows at hand) more columns of a narrower one, and bytes
     if not flags:
         assert float(_ag_gemm(cuda, torch.bfloat16, torch.float16, 128, 256, flags)[0, 0]) == 256
         assert float(_ag_gemm(cuda, torch.bfloat16, torch.float8_e4m3fn, 128, 512, flags)[0, 0]) == 512
+    as_bytes = _ag_gemm(cuda, torch.float8_e4m3fn, torch.uint8, 128, 256, flags)   # e4m3 bits: 1 is 2 ** -9
+    assert float(as_bytes[0, 0]) == 256 * 2.0**-18

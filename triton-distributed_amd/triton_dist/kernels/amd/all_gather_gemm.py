@@ -452,17 +452,19 @@ def _gather_and_multiply(a, b, c, ctx, shards, row_scale, col_scale):
     workspace = ctx.workspace_tensors[rank]
     if b.stride(1) != 1:
         raise ValueError("A, B and C must be row-major with a contiguous last dimension")
-    if (row_scale is not None or col_scale is not None) and a.dtype != torch.float8_e4m3fn:
+    # (bytes of a type that is none of the GEMM's are what the context was made for)
+    dtype = workspace.dtype if a.dtype not in _GEMM_ENTRY and a.element_size() == workspace.element_size() else a.dtype
+    if dtype not in _GEMM_ENTRY:
+        raise TypeError("unsupported GEMM dtype %s" % dtype)
+    if (row_scale is not None or col_scale is not None) and dtype != torch.float8_e4m3fn:
         raise ValueError("scales are only defined for fp8 inputs")
-    if a.dtype not in _GEMM_ENTRY:
-        raise TypeError("unsupported GEMM dtype %s" % a.dtype)
     _check_room(workspace, a, num_ranks)
     current = _lib.stream_ptr()
     stream = ctx.gemm_stream.cuda_stream
     if stream != current:
         ctx.gemm_stream.wait_stream(torch.cuda.current_stream())
     status = ctx.status.data_ptr()
-    _lib.call("tdist_ag_gemm_rows", _lib.dtype_code(a.dtype), shards, num_ranks, M_per_rank, workspace.data_ptr(), b.data_ptr(), b.stride(0),
+    _lib.call("tdist_ag_gemm_rows", _lib.dtype_code(dtype), shards, num_ranks, M_per_rank, workspace.data_ptr(), b.data_ptr(), b.stride(0),
               c.data_ptr(), c.stride(0), b.shape[0], K, _lib.ptr(row_scale), _lib.ptr(col_scale), status, status + 8,
               *_lib.workspace_args(ctx.sk_workspace), stream)
     if stream != current:
