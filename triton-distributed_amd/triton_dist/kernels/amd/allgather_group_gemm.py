@@ -397,6 +397,13 @@ def ag_group_gemm_intra_node(a, b, ctx=None, full_topk_ids=None, num_experts=Non
     if missing:
         raise RuntimeError("hand the other ranks' token rows to the context first (ctx.set_peer_shards); missing %s" % missing)
     out_dtype = a.dtype if a.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
+    # the routing names rows of C, the gather and the copies write what ``a`` is sized, and the GEMM reads b as a's type
+    if ctx.full_num_tokens > ctx.topk * M_per_rank * W:
+        raise ValueError("the context's routing is of %d rows, the call of %d" % (ctx.full_num_tokens, ctx.topk * M_per_rank * W))
+    if b.shape[1] != K or a.element_size() != b.element_size():
+        raise ValueError("Incompatible operands: %s %s and %s %s" % (tuple(a.shape), a.dtype, tuple(b.shape), b.dtype))
+    if ctx.workspace_tensors[rank].nbytes < W * a.nbytes:
+        raise ValueError("the context's workspace has no room for %d shards of %d x %d %s" % (W, M_per_rank, K, a.dtype))
     C = torch.empty([ctx.topk * M_per_rank * W, N_per_rank], dtype=out_dtype, device=a.device)
     b_nk = _weight_nk(ctx, b)
     if W > 1 and ctx.gather_rows and not ctx.held_ranks and a.is_contiguous() and (M_per_rank * K * a.element_size()) % 16 == 0:
@@ -404,6 +411,8 @@ def ag_group_gemm_intra_node(a, b, ctx=None, full_topk_ids=None, num_experts=Non
         if shards is not None and _gather_and_multiply(a, b_nk, C, ctx, shards):
             return C
     workspace, barrier = ctx.workspace_tensors[rank], ctx.barrier_tensors[rank]
+    if workspace.element_size() != a.element_size():   # (the GEMM takes rows and type from it)
+        raise ValueError("the workspace holds %s, not %s" % (workspace.dtype, a.dtype))
     current = torch.cuda.current_stream()
     gemm_stream = current if ctx.group_gemm_stream is None else ctx.group_gemm_stream
     fork = current.record_event()   # one event for both streams; a GEMM on the caller's own stream needs none
