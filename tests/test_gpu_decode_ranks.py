@@ -45,3 +45,24 @@ def test_like_stream_and_merge(cuda, R, lens, hq, hkv, dk, dv, part, room):
         got.append((out, all_out.contiguous(), all_lse))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_results_of_another_size_than_the_layer_is_for_are_refused(cuda):
+    """This rank's result is written into the caller's rows: they have to be of the cache's width, on either route."""
+    from triton_dist.kernels.amd.flash_decode import decode_stream_ranks
+    from triton_dist.layers.amd.sp_flash_decode_layer import SpGQAFlashDecodeAttention
+    announce("decode ranks: results of another width")
+    q, cache = torch.zeros((1, 8, 128), dtype=torch.bfloat16, device=cuda), torch.zeros((4, 16, 8, 128), dtype=torch.bfloat16, device=cuda)
+    table, lens = torch.zeros((1, 4), dtype=torch.int32, device=cuda), torch.full((2, 1), 16, dtype=torch.int32, device=cuda)
+    for heads, width in ((8, 64), (4, 128)):
+        rows, lse = torch.zeros((2, 1, heads, width), dtype=torch.bfloat16, device=cuda), torch.zeros((2, 1, heads), device=cuda)
+        layer = SpGQAFlashDecodeAttention(0, 0, 2, 1, heads, heads, 128, width, page_size=16, scale=1.0)
+        for peers in ((rows, lse), (rows, lse.to(torch.float64))):
+            with pytest.raises(AssertionError):
+                layer(q, cache, cache, lens, table, peers)
+        with pytest.raises(AssertionError):
+            decode_stream_ranks(q, cache, cache, lens, table, 1.0, 0.0, 0, rows, lse)
+    rows, lse = torch.zeros((2, 1, 8, 128), dtype=torch.bfloat16, device=cuda), torch.zeros((2, 1, 8), device=cuda)
+    for rank in (-1, 2):
+        with pytest.raises(AssertionError):
+            decode_stream_ranks(q, cache, cache, lens, table, 1.0, 0.0, rank, rows, lse)

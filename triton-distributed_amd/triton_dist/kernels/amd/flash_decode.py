@@ -174,7 +174,8 @@ def decode_stream_ranks(q, k_cache, v_cache, global_kv_lens, block_table, scale,
         return None
     R = all_out.shape[0]
     _lib.require_cuda(all_out, all_lse)
-    assert all_lse.shape == (R, batch, q_heads) and all_out.stride(-1) == 1 and global_kv_lens.shape == (R, batch)
+    assert all_out.shape == (R, batch, q_heads, dv) and all_lse.shape == (R, batch, q_heads) and all_out.stride(-1) == 1
+    assert global_kv_lens.shape == (R, batch) and 0 <= rank < R
     qs, os = q.stride(), all_out.stride()
     need = _stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv, q.device.index)
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device)

@@ -47,6 +47,7 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         batch = q.shape[0]
         assert global_kv_lens.shape[0] == self.num_ranks
         assert global_kv_lens.shape[1] == batch
+        assert (q.shape[1], v_cache.shape[-1]) == (self.num_q_heads, self.v_head_dim), "the results' rows are sized by the layer"
         assert batch <= self.max_allowed_batch, f"Only support {self.max_allowed_batch} queries decode now"
         if self.num_ranks == 1:
             all_out = torch.empty((1, batch, self.num_q_heads, self.v_head_dim), dtype=torch.float32, device=q.device)
