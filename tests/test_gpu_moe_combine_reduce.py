@@ -34,3 +34,42 @@ def test_like_the_steps_one_by_one(cuda, W, m, topk, hidden):
         want = y.clone()
         want[own] = -3.0
         assert torch.equal(sums, want)
+
+
+def _layer(cuda, mpr=3, world=2, hidden=264):
+    from triton_dist.kernels.amd import create_moe_rs_context
+    g = torch.Generator().manual_seed(mpr)
+    logits = [torch.randn((mpr, 4), generator=g).to(cuda) for _ in range(world)]
+    ctx = create_moe_rs_context(None, 0, world, world, world * mpr, hidden, 4, 2, torch.bfloat16, torch.bfloat16, cuda, 128, logits[0], {1: logits[1]})
+    ctx.set_peer_partials({1: torch.randn((mpr, hidden), generator=g).to(cuda)})
+    a = torch.randn((world * mpr * 2, 192), generator=g).bfloat16().to(cuda)
+    return ctx, a, torch.randn((4, 192, hidden), generator=g).bfloat16().to(cuda)
+
+
+def test_what_the_layer_refuses_of_a_context(cuda):
+    """Buffers that the one launch cannot take, as the copy into a slice and the reduction behind it refused them."""
+    from triton_dist.kernels.amd import moe_reduce_rs
+    announce("moe reduce-rs: replaced buffers and types")
+    for make in (lambda b: torch.zeros((b.shape[0], b.shape[1] + 8), dtype=b.dtype, device=b.device)[:, :-8], lambda b: b[:-1]):
+        ctx, a, b = _layer(cuda)
+        ctx.rs_buffers[0] = make(ctx.rs_buffers[0])
+        with pytest.raises(NotImplementedError):
+            moe_reduce_rs(0, 2, 2, a, b, ctx)
+    ctx, a, b = _layer(cuda)
+    with pytest.raises(TypeError):
+        moe_reduce_rs(0, 2, 2, a.float(), b.float(), ctx)
+
+
+def test_a_world_that_does_not_divide_the_tokens(cuda):
+    """Whole slices are reduced; the tokens behind them are nobody's."""
+    from triton_dist.kernels.amd import moe_reduce_rs, moe_weighted_combine
+    from triton_dist.kernels.amd.gemm_reduce_scatter import ring_reduce_after_scatter
+    announce("moe reduce-rs: 6 tokens by 4 ranks")
+    ctx, a, b = _layer(cuda)
+    for rank in (0, 3):
+        partials = ctx.rs_buffers[0].normal_().clone()
+        got = moe_reduce_rs(rank, 4, 4, a, b, ctx)
+        index = torch.arange(12, dtype=torch.int32, device=cuda).view(6, 2)
+        y = moe_weighted_combine(None, ctx.final_output_buffer[:12], None, index, ctx.topk_weight_f32, from_slots=False)
+        partials[rank] = y[rank]
+        assert got.shape == (1, 264) and torch.equal(got, ring_reduce_after_scatter(rank, 4, partials[:4], None))

@@ -14,7 +14,7 @@ from typing import Dict, List, Optional
 import torch
 
 from triton_dist import _lib
-from triton_dist.kernels.amd.allgather_group_gemm import (_group_gemm, any_block_fits, group_gemm_gated, group_gemm_rows,
+from triton_dist.kernels.amd.allgather_group_gemm import (_GROUP_GEMM_ENTRY, _group_gemm, any_block_fits, group_gemm_gated, group_gemm_rows,
                                                           joined_row_blocks, sort_topk_ids_align_block_size)
 
 
@@ -141,7 +141,7 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local, and
     # blocks that run across the rank segments hold less padding
     b_nk, row_bytes, stream = _weight_nk(ctx, b), a.shape[1] * a.element_size(), _lib.stream_ptr()
-    any_block = a.is_contiguous() and a.data_ptr() % 16 == 0 and any_block_fits(a.shape[0], row_bytes, b_nk, a.element_size())
+    any_block = a.dtype in _GROUP_GEMM_ENTRY and a.is_contiguous() and a.data_ptr() % 16 == 0 and any_block_fits(a.shape[0], row_bytes, b_nk, a.element_size())
     blocks = joined_row_blocks(ctx.joined, pre.full_sorted_token_ids, pre.full_token_expert_ids, pre.full_num_tokens_post_padded_list, pre.BLOCK_M,
                                pre.full_numel, b.shape[0], hidden, row_bytes, stream, any_block=any_block,
                                sk_workspace=ctx.sk_workspace)
@@ -155,8 +155,9 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
                          pre.num_tokens_per_rank * topk, 0, None, rank, sk_workspace=ctx.sk_workspace)
     m_per = M // world_size
     buf = ctx.rs_buffers[ctx.rank]
-    if hidden != buf.shape[1] and not buf[:M, :hidden].is_contiguous():
-        raise NotImplementedError("hidden must equal the context's hidden_dim")
+    slab = buf[:M, :hidden]
+    if slab.shape != (M, hidden) or not slab.is_contiguous():
+        raise NotImplementedError("hidden must equal the context's hidden_dim, and the context have rows for %d tokens" % M)
     weight = ctx.topk_weight_f32
     _lib.require_cuda(out, weight, buf)
     assert weight.dtype == torch.float32 and weight.is_contiguous() and weight.shape == (M, topk)
@@ -166,6 +167,7 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     # tokens are what this rank would send on
     sums = torch.empty((M, hidden), dtype=torch.bfloat16, device=a.device)
     result = torch.empty((m_per, hidden), dtype=ctx.output_dtype, device=a.device)
-    _lib.call("tdist_moe_combine_reduce", out.data_ptr(), weight.data_ptr(), M, topk, hidden, rank, world_size, buf.data_ptr(),
+    # (tokens behind world_size whole slices belong to nobody)
+    _lib.call("tdist_moe_combine_reduce", out.data_ptr(), weight.data_ptr(), m_per * world_size, topk, hidden, rank, world_size, slab.data_ptr(),
               sums.data_ptr(), result.data_ptr(), stream)
     return result
