@@ -138,3 +138,29 @@ def test_a_long_sequence_over_many_ranges(cuda, num_heads, D, lens):
 def test_a_long_latent_sequence(cuda):
     announce("decode stream, many ranges, latent heads")
     check(cuda, (16, 1), (576, 512), torch.bfloat16, [21000, 40], 16, 0, True, 5)
+
+
+@pytest.mark.parametrize("hq", [16, 40])
+def test_a_query_that_is_no_number_has_no_lse_either(cuda, hq):
+    """Latent heads, a sequence in one range: the result and its LSE are no numbers, as the exact ones; other heads and sequences
+    are as they were. (-inf, of a sequence without keys, would have a merge with other ranks leave the result out unseen.)"""
+    from triton_dist.kernels.amd.flash_decode import decode_stream
+    announce("decode stream latent, a query of NaN, %d heads" % hq)
+    g = torch.Generator().manual_seed(hq)
+    lens = [40, 33, 64]
+    q = torch.randn((3, hq, 576), generator=g).bfloat16()
+    k, _, table = golden.make_paged_kv(3, 64, 1, 576, 16, torch.bfloat16, g, v_head_dim=512)
+    kd, td, ld = k.to(cuda), table.to(cuda), torch.tensor(lens, dtype=torch.int32, device=cuda)
+
+    def run(query):
+        out, lse = torch.zeros((3, hq, 512), device=cuda), torch.zeros((3, hq), device=cuda)
+        decode_stream(query.to(cuda), kd, kd[..., :512], ld, td, 576**-0.5, 0.0, out, lse)
+        return out.cpu(), lse.cpu()
+
+    out, lse = run(q)
+    q[1, 5] = float("nan")
+    bad_out, bad_lse = run(q)
+    assert bad_out[1, 5].isnan().all() and bad_lse[1, 5].isnan()
+    others = torch.ones((3, hq), dtype=torch.bool)
+    others[1, 5] = False
+    assert torch.equal(bad_out[others], out[others]) and torch.equal(bad_lse[others], lse[others])

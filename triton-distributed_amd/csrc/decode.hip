@@ -1611,8 +1611,9 @@ __global__ __launch_bounds__(LatentCfg<HB>::kThreads) void decode_latent_kernel(
         const float L = sum_lane_xor<32>(sum_lane_xor<16>(l_run));
         if (g == 0) {
           TDIST_AS3 float* e = s_end + (((i & 1) * HB + hb) * 16 + x) * 2;
-          e[0] = L > 0.f ? 1.f / L : 0.f;
-          e[1] = L > 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
+          // (a sum that is no number stays one, also as an LSE: -inf would take the sequence for one without keys)
+          e[0] = L != 0.f ? 1.f / L : 0.f;
+          e[1] = L != 0.f ? (m_run + log2f(L)) * kLn2 : -INFINITY;
         }
         begins = true;
       }
