@@ -1222,8 +1222,10 @@ constexpr int kMergeBatch = 16;   // partial results in flight per lane of the m
 // it is rounded there, and then the sums over the ranks as in decode_combine_kernel, in the same order and with the same bits.
 // The other ranks' rows and LSEs are asked for first. With that merge as a launch of its own (6 us) behind this one a sequence-parallel
 // layer of 1 x 1259 keys, 16 heads, 8 ranks took 27.6 us, 18.6 with it; 32 x 32768 keys 658 and 650.
+// (Without ranks the launch carries nothing about them: a single sequence's call is as long as its host work.)
+struct NoRanks {};
 template <int KEYS, int NW, bool kAlone, int kRanks>
-__global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm, const RankParams rk) {
+__global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const DecodeParams prm, const std::conditional_t<kRanks != 0, RankParams, NoRanks> rk) {
   constexpr int kBatch = kAlone ? kMergeBatch / 2 : kMergeBatch, kPieces = kAlone ? NW * 64 : 64;   // 16-byte pieces of a workgroup
   __shared__ float4v s_acc[kAlone ? 1 : NW][64];
   __shared__ float s_max[kAlone ? 1 : NW][64], s_sum[kAlone ? 1 : NW][64];
@@ -1255,22 +1257,24 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_merge_kernel(const Deco
   const int d = (at_vec - h * row_vecs) * 4;
   piece_t rank_x[kRankBatch];
   float rank_lse[kRankBatch];
-  auto load_ranks = [&](int r0) {
+  [[maybe_unused]] auto load_ranks = [&](int r0) {
+    if constexpr (kRanks != 0) {
 #pragma unroll
-    for (int u = 0; u < kRankBatch; ++u) {
-      const int r = min(r0 + u, rk.c.P - 1);
-      const unsigned char* at = rk.c.part + (r * rk.c.p_sp + seq * rk.c.p_sb + h * rk.c.p_sh + d) * (int64_t)(sizeof(piece_t) / 4);
-      if (rk.part_vec) {
-        rank_x[u] = *(const piece_t*)at;
-      } else if constexpr (kRanks == 2) {
+      for (int u = 0; u < kRankBatch; ++u) {
+        const int r = min(r0 + u, rk.c.P - 1);
+        const unsigned char* at = rk.c.part + (r * rk.c.p_sp + seq * rk.c.p_sb + h * rk.c.p_sh + d) * (int64_t)(sizeof(piece_t) / 4);
+        if (rk.part_vec) {
+          rank_x[u] = *(const piece_t*)at;
+        } else if constexpr (kRanks == 2) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) rank_x[u][e] = ((const float*)at)[e];
-      } else {
-        const unsigned short* a = (const unsigned short*)at;
-        rank_x[u] = int2v{(int)(a[0] | (uint32_t)a[1] << 16), (int)(a[2] | (uint32_t)a[3] << 16)};
+          for (int e = 0; e < 4; ++e) rank_x[u][e] = ((const float*)at)[e];
+        } else {
+          const unsigned short* a = (const unsigned short*)at;
+          rank_x[u] = int2v{(int)(a[0] | (uint32_t)a[1] << 16), (int)(a[2] | (uint32_t)a[3] << 16)};
+        }
+        // (a rank without keys of the sequence is left out)
+        rank_lse[u] = r0 + u < rk.c.P && r != rk.own && rk.c.lens[(int64_t)r * prm.B + seq] != 0 ? rk.c.lse[r * rk.c.l_sp + seq * rk.c.l_sb + h * rk.c.l_sh] : -INFINITY;
       }
-      // (a rank without keys of the sequence is left out)
-      rank_lse[u] = r0 + u < rk.c.P && r != rk.own && rk.c.lens[(int64_t)r * prm.B + seq] != 0 ? rk.c.lse[r * rk.c.l_sp + seq * rk.c.l_sb + h * rk.c.l_sh] : -INFINITY;
     }
   };
   if constexpr (kRanks != 0) {
@@ -1393,7 +1397,7 @@ static int launch_merge_cfg(const DecodeParams& prm, hipStream_t stream) {
     else hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 1>), grid, block, 0, stream, prm, *prm.ranks);
     return launch_status("tdist_decode_stream");
   }
-  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 0>), grid, block, 0, stream, prm, RankParams{});
+  hipLaunchKernelGGL((decode_stream_merge_kernel<KEYS, NW, kAlone, 0>), grid, block, 0, stream, prm, NoRanks{});
   if (int rc = launch_status("tdist_decode_stream")) return rc;
   return prm.ranks ? launch_combine(prm.ranks->c, stream) : TDIST_OK;
 }

@@ -207,17 +207,18 @@ def shards_in_reach(table, rows, row_bytes):
     return len(table) <= 16 and rows >= 2 and len(table) * rows * rows < 1 << 32 and max(table) - min(table) + rows * row_bytes < (1 << 32) - 4096
 
 
+_DTYPE_CODES = {}
+
+
 def dtype_code(dtype):
-    import torch
-    if dtype == torch.bfloat16:
-        return TDIST_BF16
-    if dtype == torch.float16:
-        return TDIST_F16
-    if dtype == torch.float8_e4m3fn:
-        return TDIST_F8E4M3
-    if dtype == torch.float32:
-        return TDIST_F32
-    raise TypeError("unsupported dtype %s" % dtype)
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        import torch
+        _DTYPE_CODES.update({torch.bfloat16: TDIST_BF16, torch.float16: TDIST_F16, torch.float8_e4m3fn: TDIST_F8E4M3, torch.float32: TDIST_F32})
+        code = _DTYPE_CODES.get(dtype)
+        if code is None:
+            raise TypeError("unsupported dtype %s" % dtype)
+    return code
 
 
 _bench_lib = None

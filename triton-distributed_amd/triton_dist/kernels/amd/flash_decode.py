@@ -138,7 +138,8 @@ def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, ou
         part, lse, kv_lens = _split_kv(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, S)
         return decode_combine(part, lse, S, 1, kv_lens, batch, q_heads, dv, (part.stride(2), part.stride(0), part.stride(1)),
                               (lse.stride(2), lse.stride(0), lse.stride(1)), out, lse_out)
-    need = _stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv, q.device.index)
+    key = (batch, q_heads, kv_heads, dk, dv, q.device.index)
+    need = _STREAM_PLANS.get(key) or _stream_workspace_bytes(key)
     if counters is not None:
         _check_counters(q, kv_heads, counters)
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
@@ -150,12 +151,10 @@ def decode_stream(q, k_cache, v_cache, kv_lens, block_table, scale, soft_cap, ou
     return out
 
 
-def _stream_workspace_bytes(*key):
-    need = _STREAM_PLANS.get(key)
-    if need is None:
-        if len(_STREAM_PLANS) >= 1024:
-            _STREAM_PLANS.clear()
-        need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(*key[:5])
+def _stream_workspace_bytes(key):
+    if len(_STREAM_PLANS) >= 1024:
+        _STREAM_PLANS.clear()
+    need = _STREAM_PLANS[key] = _lib.load().tdist_decode_stream_workspace_bytes(*key[:5])
     return need
 
 
@@ -177,7 +176,8 @@ def decode_stream_ranks(q, k_cache, v_cache, global_kv_lens, block_table, scale,
     assert all_out.shape == (R, batch, q_heads, dv) and all_lse.shape == (R, batch, q_heads) and all_out.stride(-1) == 1
     assert global_kv_lens.shape == (R, batch) and 0 <= rank < R
     qs, os = q.stride(), all_out.stride()
-    need = _stream_workspace_bytes(batch, q_heads, kv_heads, dk, dv, q.device.index)
+    key = (batch, q_heads, kv_heads, dk, dv, q.device.index)
+    need = _STREAM_PLANS.get(key) or _stream_workspace_bytes(key)
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     out = torch.empty((batch, q_heads, dv), dtype=q.dtype, device=q.device)
     dtype = _lib.dtype_code(q.dtype)
