@@ -43,7 +43,7 @@ MEASURED_TRAFFIC_BYTES = {
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "f5b639d6f2c93627",
-    "decode.hip": "eb3de310b59afb82",
+    "decode.hip": "3ac771befeb01e03",
     "gather.h": "3fd5e450cd06de4d",
     "gemm.hip": "1a895ba16559069c",
     "gemm_small.h": "ef635860051b59ae",

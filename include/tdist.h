@@ -592,7 +592,9 @@ int tdist_decode_fused(const void* q, const void* k_cache, const void* v_cache, 
  * the sequences that are spread over several ranges. out [B,Hq,Dv] of
  * out_dtype (strides out_stride_b, out_stride_h); lse_out fp32 [B,Hq] or NULL; a sequence of length 0 gets out = 0,
  * lse = -inf. counters, n_counters: not used (NULL, 0). workspace: plain device memory,
- * 16-byte aligned, of at least tdist_decode_stream_workspace_bytes() bytes (-1: bad sizes); its contents do not matter
+ * 16-byte aligned, of at least tdist_decode_stream_workspace_bytes() bytes (-1: bad sizes; with (576,512) and more than 16 query
+ * heads per kv head the room for partial results of one block of 16 heads per workgroup is taken too, as 16.8 MB instead of 33.6 for
+ * 128 / 1 heads, and the call is slower); its contents do not matter
  * before or after the call: nothing is kept between calls, which may be captured and replayed in any order. Calls that
  * share a workspace must not overlap. Head dimensions as
  * for tdist_decode_split_kv, except that (576,512) is taken only where the value is the first 512 columns of the key (the

@@ -164,3 +164,36 @@ def test_a_query_that_is_no_number_has_no_lse_either(cuda, hq):
     others = torch.ones((3, hq), dtype=torch.bool)
     others[1, 5] = False
     assert torch.equal(bad_out[others], out[others]) and torch.equal(bad_lse[others], lse[others])
+
+
+@pytest.mark.parametrize("hq,hkv,ranges", [(128, 1, 32), (24, 1, 128), (40, 2, 64)])
+def test_latent_heads_in_half_the_workspace(cuda, hq, hkv, ranges):
+    """The room for ``ranges`` ranges, as many as one block of 16 heads per workgroup has on 256 compute units, is enough; less is
+    refused."""
+    from triton_dist import _lib
+    lib = _lib.load()
+    lens = [3000, 0, 31, 700, 64]
+    announce("decode stream latent heads=%d/%d with %d ranges" % (hq, hkv, ranges))
+    g = torch.Generator().manual_seed(hq)
+    q = torch.randn((5, hq, 576), generator=g).bfloat16()
+    k, _, table = golden.make_paged_kv(5, 3000, hkv, 576, 16, torch.bfloat16, g, v_head_dim=512)
+    exact, exact_lse = golden.decode_exact(q, k, k[..., :512], lens, table, 576**-0.5, 0)
+    qd, kd, td, ld = q.to(cuda), k.to(cuda), table.to(cuda), torch.tensor(lens, dtype=torch.int32, device=cuda)
+    per_range = 2 * hq * 513 * 4
+    assert lib.tdist_num_cus() == 256 and lib.tdist_decode_stream_workspace_bytes(5, hq, hkv, 576, 512) > ranges * per_range
+    memory = torch.zeros(ranges * per_range + 64, dtype=torch.uint8, device=cuda)
+    memory[-64:] = 7
+
+    def call(nbytes):
+        out, lse = torch.zeros((5, hq, 512), device=cuda), torch.zeros((5, hq), device=cuda)
+        rc = lib.tdist_decode_stream(qd.data_ptr(), kd.data_ptr(), kd.data_ptr(), 576**-0.5, 0.0, td.data_ptr(), ld.data_ptr(), 5, hq, hkv,
+                                     576, 512, 16, *qd.stride()[:2], *kd.stride()[:3], *kd.stride()[:3], td.stride(0), _lib.TDIST_BF16, None, 0,
+                                     memory.data_ptr(), nbytes, out.data_ptr(), _lib.TDIST_F32, *out.stride()[:2], lse.data_ptr(), None)
+        torch.cuda.synchronize()
+        return rc, out.cpu().double(), lse.cpu().double()
+
+    assert call(ranges * per_range - 1)[0] == _lib.TDIST_ERR_WORKSPACE
+    rc, out, lse = call(ranges * per_range)
+    live = ~torch.isinf(exact_lse)
+    assert rc == _lib.TDIST_OK and bool((memory[-64:] == 7).all())
+    assert (out - exact).abs().max() <= ATOL and (lse[live] - exact_lse[live]).abs().max() <= ATOL and torch.equal(torch.isinf(lse), ~live)

@@ -1908,16 +1908,19 @@ static int stream_ranges(int64_t units, int64_t slots) {
 }
 // Ranges for a call, given its head counts and key dimension. Four waves with rings of up to four stages per compute unit (as much
 // in flight as eight waves of two, half the fixed work and half the partial results), a kv head and a block of 16 query heads each;
-// or, for latent attention, two workgroups, each a set of head blocks.
-static int stream_ranges_for(int q_heads, int kv_heads, int head_dim) {
+// or, for latent attention, a workgroup per compute unit with a set of head blocks. With two blocks in a set that is twice the
+// ranges, and twice the workspace, of one block per workgroup (128 / 1 heads: 64 ranges, 33.6 MB); a caller who comes with the room
+// for `fewest`, as many as there were with one block, gets that many (16 sequences up to 4096 keys 41.5 us a call, 32.6 with 64).
+static int stream_ranges_for(int q_heads, int kv_heads, int head_dim, bool fewest = false) {
   const int group = q_heads / kv_heads, cus = device_info().num_cus > 0 ? device_info().num_cus : 256;
-  if (head_dim > 256) return stream_ranges((int64_t)kv_heads * ceil_div(group, 16 * latent_head_blocks(group)), 1ll * cus);
+  if (head_dim > 256) return stream_ranges((int64_t)kv_heads * ceil_div(group, 16 * (fewest ? 1 : latent_head_blocks(group))), 1ll * cus);
   return stream_ranges((int64_t)kv_heads * ceil_div(group, 16), 4ll * cus);
 }
+// two partial results per range: rows of head_dim_v floats and one LSE per query head
+static int64_t partials_bytes(int ranges, int q_heads, int head_dim_v) { return 2ll * ranges * q_heads * (head_dim_v + 1) * 4; }
 static int64_t stream_workspace_bytes(int batch, int q_heads, int kv_heads, int head_dim, int head_dim_v) {
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || head_dim_v <= 0) return -1;
-  // two partial results per range: rows of head_dim_v floats and one LSE per query head
-  return 2ll * stream_ranges_for(q_heads, kv_heads, head_dim) * q_heads * (head_dim_v + 1) * 4;
+  return partials_bytes(stream_ranges_for(q_heads, kv_heads, head_dim), q_heads, head_dim_v);
 }
 
 static int run_decode(const DecodeCall& c, DecodeForm form) {
@@ -2013,10 +2016,14 @@ static int run_decode(const DecodeCall& c, DecodeForm form) {
     const bool latent = c.v_cache == c.k_cache && prm.v_sp == prm.k_sp && prm.v_st == prm.k_st && (prm.v_sh == prm.k_sh || c.kv_heads == 1);
     if (dk > 256 && !latent)
       return fail(TDIST_ERR_UNSUPPORTED, "%s: head dims (%d, %d) with a value that is no part of the key", who, dk, dv);
-    const int64_t need = stream_workspace_bytes(c.batch, c.q_heads, c.kv_heads, dk, dv);
-    if (c.workspace_bytes < need)
-      return fail(TDIST_ERR_WORKSPACE, "%s: %lld bytes of workspace given, %lld needed", who, (long long)c.workspace_bytes, (long long)need);
     prm.ranges = stream_ranges_for(c.q_heads, c.kv_heads, dk);
+    if (c.workspace_bytes < partials_bytes(prm.ranges, c.q_heads, dv)) {
+      const int fewest = stream_ranges_for(c.q_heads, c.kv_heads, dk, true);
+      if (fewest >= prm.ranges || c.workspace_bytes < partials_bytes(fewest, c.q_heads, dv))
+        return fail(TDIST_ERR_WORKSPACE, "%s: %lld bytes of workspace given, %lld needed", who, (long long)c.workspace_bytes,
+                    (long long)partials_bytes(prm.ranges, c.q_heads, dv));
+      prm.ranges = fewest;
+    }
     prm.out = (float*)c.workspace;
     prm.lse = prm.out + 2ll * prm.ranges * c.q_heads * dv;
 #define TDIST_STREAM(D_, DPE_, KEYS_, NW_, NST_, PAD_)                                                \
