@@ -166,6 +166,41 @@ def test_a_query_that_is_no_number_has_no_lse_either(cuda, hq):
     assert torch.equal(bad_out[others], out[others]) and torch.equal(bad_lse[others], lse[others])
 
 
+@pytest.mark.parametrize("dtype,group", [(torch.bfloat16, 2), (torch.float16, 17)])
+def test_latent_maxima_raised_within_a_range(cuda, dtype, group):
+    """Scores far above those before them, in the middle of a range: the sums so far, which other waves hold, are rescaled. A quarter of
+    the heads sees one such key each at a third, a half and two thirds of a sequence (it and the sequence's other keys weigh about the
+    same, so that a sum left as it was, or dropped, is seen), the last quarter scores that grow with every block of 32 keys."""
+    from triton_dist.kernels.amd.flash_decode import decode_stream
+    announce("decode stream latent, raised maxima, %s, %d heads per kv head" % (dtype, group))
+    g = torch.Generator().manual_seed(group)
+    hkv, B = 8, 24
+    lens = [384 - 5 * (i % 7) for i in range(B)]   # 12 blocks each over 32 ranges of 9: sequences straddle ranges, ranges hold several
+    q = torch.randn((B, hkv * group, 576), generator=g) * 0.25
+    k, _, table = golden.make_paged_kv(B, 384, hkv, 576, 16, torch.float32, g, v_head_dim=512)
+    kind = torch.arange(hkv * group) % 4
+    q[:, :, 512:516] = torch.nn.functional.one_hot(kind, 4) * 12.875
+    k[..., 512:516] = 0
+    for b, n in enumerate(lens):
+        for key in range(n):
+            k[table[b, key // 16], key % 16, :, 515] = 0.35 * key   # 6 more per block, in the scores' e-logarithm
+        for j, key in enumerate((n // 3, n // 2, 2 * n // 3)):
+            k[table[b, key // 16], key % 16, :, 512 + j] = 12.875     # 6.9
+    q, k = q.to(dtype), k.to(dtype)
+    exact, exact_lse = golden.decode_exact(q, k, k[..., :512], lens, table, 576**-0.5, 0)
+    # (on the oracle's side: without its one key, a head's other scores stay more than 8 in log2 below)
+    flat = q.clone()
+    flat[:, :, 512:515] = 0
+    most = torch.stack([(flat[b].double() @ golden._gather_kv(k, table.numpy()[b], 0, n)[:, 0].double().t()).max(1).values for b, n in enumerate(lens)])
+    raised = 6.9 - 576**-0.5 * most[:, (kind < 3) & (torch.arange(hkv * group) < group)] > 8 * 0.6931
+    assert raised.double().mean() > 0.8
+    kd = k.to(cuda)
+    out, lse = torch.empty((B, hkv * group, 512), device=cuda), torch.empty((B, hkv * group), device=cuda)
+    decode_stream(q.to(cuda), kd, kd[..., :512], torch.tensor(lens, dtype=torch.int32, device=cuda), table.to(cuda), 576**-0.5, 0.0, out, lse)
+    assert (out.cpu().double() - exact).abs().max() <= ATOL
+    assert (lse.cpu().double() - exact_lse).abs().max() <= ATOL
+
+
 @pytest.mark.parametrize("hq,hkv,ranges", [(128, 1, 32), (24, 1, 128), (40, 2, 64)])
 def test_latent_heads_in_half_the_workspace(cuda, hq, hkv, ranges):
     """The room for ``ranges`` ranges, as many as one block of 16 heads per workgroup has on 256 compute units, is enough; less is
