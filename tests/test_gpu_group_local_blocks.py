@@ -34,6 +34,7 @@ def _context(cuda, shards, w, ids, rank, E):
     (torch.bfloat16, 4, 150, 512, 2312, 6, 3), (torch.float16, 4, 301, 200, 4100, 5, 2), (torch.float8_e4m3fn, 4, 130, 384, 1288, 7, 2),
     (torch.float8_e4m3fn, 8, 96, 208, 8200, 3, 2), (torch.bfloat16, 2, 257, 64, 520, 4, 2), (torch.bfloat16, 2, 64, 40, 136, 4, 2)])
 def test_exact_and_like_the_gated_form(cuda, monkeypatch, block, dtype, world, mpr, K, N, E, topk):
+    from triton_dist import _lib
     from triton_dist.kernels.amd import ag_group_gemm_intra_node, allgather_group_gemm
     announce("local blocks %s block %d W=%d m=%d K=%d N=%d E=%d topk=%d" % (dtype, block, world, mpr, K, N, E, topk))
     monkeypatch.setattr(allgather_group_gemm, "_join_plan", lambda n, e, _: (block, (n + e * (block - 1)) // block))
@@ -41,12 +42,13 @@ def test_exact_and_like_the_gated_form(cuda, monkeypatch, block, dtype, world, m
     ctx, a, b = _context(cuda, shards, w, ids, world - 1, E)
     esz = a.element_size()
     if K * esz % 64 != 0 and K * esz <= 128:
-        from triton_dist import _lib
         with pytest.raises(_lib.TdistError):   # refused in either form
             ag_group_gemm_intra_node(a, b, ctx)
         return
-    c = ag_group_gemm_intra_node(a, b, ctx)
+    with _lib.debug_switch(_lib.TDIST_DEBUG_GEMM_TILE, 0 if block == 256 else 4):   # (the large tile of so many rows)
+        c = ag_group_gemm_intra_node(a, b, ctx)
     ctx.check_status()
+    assert {blocks.block_size for blocks in ctx.joined.values()} == {block}
     want = golden.ag_group_gemm_fp32(shards, w, ids)
     assert torch.equal(c.float().cpu(), want.to(c.dtype).float())
     ctx.gather_rows = False

@@ -1,5 +1,5 @@
 """The grouped GEMM on the small tiles: blocks of 64 and 128 rows with 128 columns, whole or in pieces of K, exactly as the oracle has
-it (whole numbers small enough for every sum); and the forms that take blocks of 128 and 256 rows, where the choice is left to them."""
+it (whole numbers small enough for every sum); and the large tiles in the blocks that are chosen where no estimate has them."""
 import pytest
 import torch
 
@@ -36,7 +36,7 @@ def test_small_tiles_exact(cuda, tile, pieces, dtype, world, mpr, K, N, E, topk)
 @pytest.mark.parametrize("block", [128, 256])
 @pytest.mark.parametrize("dtype,world,mpr,K,N,E,topk", [(torch.bfloat16, 4, 150, 512, 2312, 6, 3), (torch.float16, 2, 3, 192, 264, 64, 2),
                                                         (torch.float8_e4m3fn, 8, 96, 208, 8200, 3, 2)])
-def test_large_tiles_where_the_choice_is_left_to_them(cuda, monkeypatch, block, dtype, world, mpr, K, N, E, topk):
+def test_large_tiles_in_blocks_without_an_estimate(cuda, monkeypatch, block, dtype, world, mpr, K, N, E, topk):
     from triton_dist.kernels.amd import allgather_group_gemm
     monkeypatch.setattr(allgather_group_gemm, "_block_plan", lambda *_: None)
     local_blocks.test_exact_and_like_the_gated_form(cuda, monkeypatch, block, dtype, world, mpr, K, N, E, topk)

@@ -78,11 +78,13 @@ def test_shards_out_of_reach_are_gathered(cuda, case):
     assert torch.equal(got, want)
 
 
+# (tile 0: 256 x 256, 4: 128 x 256; the choice left to the call takes small ones at all of these sizes)
+@pytest.mark.parametrize("tile", [None, 0, 4])
 @pytest.mark.parametrize("W,m,topk,E,N,K", [(4, 7, 2, 8, 256, 512), (8, 130, 2, 4, 520, 1000), (2, 1024, 4, 8, 512, 256), (16, 33, 1, 3, 256, 264)])
-def test_grouped_rows_where_they_lie(cuda, monkeypatch, W, m, topk, E, N, K):
+def test_grouped_rows_where_they_lie(cuda, monkeypatch, W, m, topk, E, N, K, tile):
     from triton_dist import _lib
     from triton_dist.kernels.amd import ag_group_gemm_intra_node, create_ag_group_gemm_intra_node_context
-    announce("grouped shard rows W=%d m=%d E=%d" % (W, m, E))
+    announce("grouped shard rows W=%d m=%d E=%d tile=%s" % (W, m, E, tile))
     g = torch.Generator().manual_seed(W * m)
     shards = scattered(cuda, g, W, (m, K), torch.bfloat16)
     ids = torch.rand((W * m, E), generator=g).topk(topk, dim=1).indices.to(torch.int32).to(cuda)
@@ -94,8 +96,10 @@ def test_grouped_rows_where_they_lie(cuda, monkeypatch, W, m, topk, E, N, K):
         ctx.workspace_tensors[1].view(torch.uint8).fill_(0x7B)
         if gathered:
             monkeypatch.setattr(_lib, "shards_in_reach", lambda *_: False)
-        out.append(ag_group_gemm_intra_node(shards[1], w, ctx))
+        with _lib.debug_switch(_lib.TDIST_DEBUG_GEMM_TILE, tile):
+            out.append(ag_group_gemm_intra_node(shards[1], w, ctx))
         torch.cuda.synchronize()
+        assert tile is None or {blocks.block_size for blocks in ctx.joined.values()} == {256 if tile == 0 else 128}
     assert torch.equal(out[0], out[1])
     token = torch.cat(shards)[:, None, :].expand(-1, topk, -1).reshape(-1, K).float()
     rows = torch.arange(0, W * m * topk, max(1, W * m * topk // 50), device=cuda)
