@@ -74,7 +74,6 @@ class MoEReduceRSContext:
     rs_buffers: List[Optional[torch.Tensor]]   # [max_token_num, hidden]: row block r holds rank r's partial of this rank's tokens
     final_output_buffer: torch.Tensor          # [max_token_num * topk, hidden]: the grouped GEMM's rows
     topk_weight_f32: torch.Tensor              # the routing weights as the combine kernel takes them
-    identity_index: torch.Tensor               # int32 [M, topk]: row t*topk + k
     output_dtype: torch.dtype = torch.bfloat16
     weight_nk: Optional[torch.Tensor] = None
     weight_key: Optional[tuple] = None
@@ -105,15 +104,13 @@ def create_moe_rs_context(pg, local_rank, world_size, local_world_size, max_toke
     assert num_tokens_per_rank * world_size <= max_token_num and max_token_num % world_size == 0
     pre = precompute_context_helper(pg, world_size, topk, num_tokens_per_rank, num_experts, input_dtype, device,
                                     router_logits, BLOCK_M=moe_block_size, peer_router_logits=peer_router_logits, rank=rank)
-    M = num_tokens_per_rank * world_size
     rs_buffers: List[Optional[torch.Tensor]] = [None] * world_size
     rs_buffers[rank] = torch.zeros([max_token_num, hidden_dim], dtype=output_dtype, device=device)
     return MoEReduceRSContext(
         precompute_ctx=pre, rank=rank, world_size=world_size, rs_buffers=rs_buffers,
         final_output_buffer=torch.zeros((max_token_num * topk, hidden_dim), dtype=output_dtype, device=device),
         topk_weight_f32=pre.full_topk_weight.float().contiguous(),
-        identity_index=torch.arange(M * topk, dtype=torch.int32, device=device).view(M, topk), output_dtype=output_dtype,
-        sk_workspace=_lib.new_split_k_workspace(device) if split_k else None)
+        output_dtype=output_dtype, sk_workspace=_lib.new_split_k_workspace(device) if split_k else None)
 
 
 def _weight_nk(ctx, b):
