@@ -889,3 +889,21 @@ def test_walks_of_an_ungated_gemm(cuda, switches, tile, M, N):
         gated_gemm(a, None, 0, b, c, None, 0, 0, 1, sk_workspace=ws)
         torch.cuda.synchronize()
         assert torch.equal(c, want), split
+
+
+# a round of 256 x 128 tiles or of 128 x 192: as many K tiles as it takes and one less, a ragged K; few row tiles, and more of them in
+# even and odd number
+@pytest.mark.parametrize("M,dtype,K", [(1280, torch.bfloat16, 1280), (1280, torch.bfloat16, 1216), (1280, torch.float16, 1288), (1536, torch.bfloat16, 2048),
+                                       (1536, torch.bfloat16, 1984), (1536, torch.float8_e4m3fn, 4224), (1792, torch.bfloat16, 2048)])
+def test_one_round_of_either_tile(cuda, dtype, M, K):
+    from triton_dist.kernels.amd import gated_gemm
+    announce("gemm of one round %s M=%d K=%d" % (dtype, M, K))
+    g = torch.Generator().manual_seed(M + K)
+    a, b = (torch.randint(-2, 3, (n, K), generator=g).to(dtype).to(cuda) for n in (M, 328))
+    out_dtype = torch.bfloat16 if dtype == torch.float8_e4m3fn else dtype
+    want = (a.float() @ b.float().t()).to(out_dtype)   # (|sums| < 2^24: exact in fp32, rounded once)
+    for flags in (torch.ones(M // 256, dtype=torch.int32, device=cuda), None):
+        c = torch.full((M, 328), float("nan"), dtype=out_dtype, device=cuda)
+        gated_gemm(a, None, 0, b, c, flags, 256, 0, M // 256)
+        torch.cuda.synchronize()
+        assert torch.equal(c, want), flags is None

@@ -2120,6 +2120,16 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // (the margin lies between whole tiles and a split round, not between two tiles' split rounds)
   bool use_sk = pick_split >= 0 && (sk_mode == 1 || split_last < 0.95 * whole);
   if (use_sk) pick = pick_split;
+  // One round of 256 x 128 tiles in place of one of 128 x 192: the rates are those of many rounds, which end in as many prologues and
+  // epilogues, and the larger tile has fewer bytes to fetch per product. Rows of whole 128-byte lines, from 32 K tiles on (20 where the
+  // call has five row tiles or fewer): 4096 x 1536 x 4096 bf16 46.4 -> 44.8 us, with the rows to their owners 46.2 -> 44.7, behind flags
+  // 49.4 -> 48.6; 768 x 7168 x 3072 behind flags 50.1 -> 36.3; 200 such calls 9 % faster on average, 9 % slower at worst. With shorter rows or
+  // ragged ones it is behind (2560 x 776 x 576 f16 14.1 us, 12.8 on 128 x 192; 3072 x 1472 x 8048 bf16 116, 105), and so it is where a
+  // call that is no ungated one has an odd number of its row tiles beyond five (3840 x 1536 x 4608 e4m3 37.3, 35.3).
+  auto one_round = [&](int t) { return ceil_div(c.M, kChoices[t].bm) * ceil_div(c.N, kChoices[t].bn) <= cap_wgs; };
+  const int64_t row_bytes = (int64_t)c.K * esz, row_tiles = ceil_div(c.M, kChoices[1].bm);
+  if (!use_sk && pick == 3 && admissible(1) && one_round(1) && one_round(3) && row_bytes % 128 == 0 &&
+      row_bytes >= (row_tiles <= 5 ? 20 : 32) * 128 && (row_tiles <= 5 || row_tiles % 2 == 0 || !(c.flags || c.scatter_bufs))) pick = 1;
   const double best = use_sk ? split_last : whole;
   if (small.us > 0) {
     const double large_us = launch_us + best / 65536.0 * 1.1 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
