@@ -368,8 +368,9 @@ __device__ __forceinline__ int chunk_of(const GemmParams& p, int oc) {
 }
 
 // kPlain: an instance for calls without flags and without a local shard (the GEMM-RS producer, plain GEMMs): no gating
-// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly).
-template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
+// code at all, and the next tile's first loads go out before the current tile's epilogue (see kEarly). kShards: an instance for rows in
+// shards too (see launch_gemm_rows).
+template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true, bool kShards = true>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams p) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
   typedef TDIST_AS3 unsigned char* lds_u8;
@@ -771,7 +772,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
     // DMA sources: a wave-uniform base (first row of the tile, advanced along K in scalar registers) plus a
     // 32-bit per-lane offset, so that the load takes its address as SGPR base + VGPR offset and the K loop
     // carries no vector address arithmetic for it
-    const bool in_shards = !kGrouped && p.shards.rows != 0;
+    const bool in_shards = kShards && !kGrouped && p.shards.rows != 0;
     const int a_g0 = kGrouped || in_shards ? 0 : min(m0 - a_row_off, a_row_max), b_g0 = min(n0, p.N - 1);
     const unsigned char* const a_base = Arows + (int64_t)a_g0 * a_ld + (int64_t)ka * KB;
     const unsigned char* b_base_ = p.B + (int64_t)b_g0 * p.ldb_b + (int64_t)ka * KB;
@@ -796,7 +797,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       }
       a_off[t] = (uint32_t)(gr - a_g0) * (uint32_t)a_ld + (uint32_t)((dma_pos ^ swz<KB>(r)) << 4);
     }
-    if constexpr (!kGrouped) {
+    if constexpr (kShards && !kGrouped) {
       if (in_shards) shard_offsets(m0, a_off);
     }
 #pragma unroll
@@ -1290,7 +1291,9 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
           early = true;
           a_base_n = in_shards ? p.A : p.A + (int64_t)nm0 * p.lda_b;
           b_base_n = p.B + (int64_t)nn0 * p.ldb_b;
-          if (in_shards) shard_offsets(nm0, a_off);
+          if constexpr (kShards) {
+            if (in_shards) shard_offsets(nm0, a_off);
+          }
         }
       }
       // (wave-uniform by construction; said so to the compiler, which otherwise carries them in vector registers)
@@ -1785,7 +1788,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_kernel(const GemmParams 
       }
     }
   }
-  if constexpr (!kGrouped || kPlain) retire_beside(p.shards);   // (in front of the tiles its test held the first loads up: 0.4 of 53 us)
+  if constexpr (kShards && (!kGrouped || kPlain)) retire_beside(p.shards);   // (in front of the tiles its test held the first loads up: 0.4 of 53 us)
   // ---- the last workgroup out advances the workspace's tag base for the next launch --------------------------
   if (p.sk_mode != 0 && threadIdx.x == 0) {
     int32_t* const done = p.sk_ctrl + kSkCtrlDone;
@@ -1833,10 +1836,10 @@ struct GemmCall {
   ShardRows shards;   // rows != 0: A's rows lie in shards
 };
 
-template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
+template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true, bool kShards = true>
 static int launch_gemm_cfg(const GemmParams& prm, int grid, hipStream_t stream, const char* who) {
   typedef GemmCfg<E, BM, BN, KB, WM, WN, NST> C;
-  auto kern = gemm_kernel<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain, kHead>;
+  auto kern = gemm_kernel<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain, kHead, kShards>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes);
@@ -1845,6 +1848,15 @@ static int launch_gemm_cfg(const GemmParams& prm, int grid, hipStream_t stream, 
   }
   hipLaunchKernelGGL(kern, dim3(grid), dim3(C::kThreads), C::kLdsBytes, stream, prm);
   return launch_status(who);
+}
+
+// Rows in shards have instances of their own: the test for them, a register or two of every tile's addresses and the launch's end cost the
+// others up to 3 % (the same box, before / after: 16384 x 7168 x 8192 e4m3 behind flags 607.3 / 604.2 us, 8192 x 8192 x 3584 bf16 with its rows to
+// their owners 317.2 / 316.2, 4096 x 4096 x 4096 e4m3 behind flags 53.6 / 52.3, 7168 x 7128 x 3792 e4m3 ungated 185.0 / 182.6).
+template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
+static int launch_gemm_rows(const GemmParams& prm, int grid, hipStream_t stream, const char* who) {
+  return prm.shards.rows != 0 ? launch_gemm_cfg<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain, kHead, true>(prm, grid, stream, who)
+                              : launch_gemm_cfg<E, BM, BN, KB, WM, WN, NST, kScales, kGrouped, kPlain, kHead, false>(prm, grid, stream, who);
 }
 
 // ---- split-K workspace (the caller's, per call) ------------------------------------------------------------
@@ -2283,8 +2295,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     // no flags, no local shard: the instances without gating code (the GEMM-RS producer's, the headline shape's), with
     // and without a ragged first K tile (the test for one costs the headline shape 0.5 %)
 #define TDIST_PLAIN(E_, SC_)                                                                                        \
-  (p.k_head_bytes != 0 ? launch_gemm_cfg<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, true>(p, grid, c.stream, who)    \
-                       : launch_gemm_cfg<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, false>(p, grid, c.stream, who))
+  (p.k_head_bytes != 0 ? launch_gemm_rows<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, true>(p, grid, c.stream, who)    \
+                       : launch_gemm_rows<E_, 256, 256, 128, 2, 2, 5, SC_, false, true, false>(p, grid, c.stream, who))
     switch (elem) {
       case kElemBF16: return TDIST_PLAIN(ElemBF16N, false);
       case kElemF16: return TDIST_PLAIN(ElemF16N, false);
@@ -2294,47 +2306,47 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   }
   if (BM == 256 && BN == 256) {
     switch (elem) {
-      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 256, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
-      case kElemF16: return launch_gemm_cfg<ElemF16N, 256, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 256, 256, 128, 2, 2, 5, false, false, false, true, false>(p, grid, c.stream, who);
+      case kElemF16: return launch_gemm_cfg<ElemF16N, 256, 256, 128, 2, 2, 5, false, false, false, true, false>(p, grid, c.stream, who);
       default:
-        return scales ? launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, true>(p, grid, c.stream, who)
-                      : launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+        return scales ? launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, true, false, false, true, false>(p, grid, c.stream, who)
+                      : launch_gemm_cfg<ElemFP8N, 256, 256, 128, 2, 2, 5, false, false, false, true, false>(p, grid, c.stream, who);
     }
   }
   if (BM == 256) {
     switch (elem) {
-      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
-      case kElemF16: return launch_gemm_cfg<ElemF16N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemBF16: return launch_gemm_rows<ElemBF16N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemF16: return launch_gemm_rows<ElemF16N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
       default:
-        return scales ? launch_gemm_cfg<ElemFP8N, 256, 128, 128, 2, 2, 5, true>(p, grid, c.stream, who)
-                      : launch_gemm_cfg<ElemFP8N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+        return scales ? launch_gemm_rows<ElemFP8N, 256, 128, 128, 2, 2, 5, true>(p, grid, c.stream, who)
+                      : launch_gemm_rows<ElemFP8N, 256, 128, 128, 2, 2, 5, false>(p, grid, c.stream, who);
     }
   }
   if (BM == 128 && BN == 256) {  // 128 x 256: waves of 64 x 128 on the split ring
     switch (elem) {
-      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
-      case kElemF16: return launch_gemm_cfg<ElemF16N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemBF16: return launch_gemm_rows<ElemBF16N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemF16: return launch_gemm_rows<ElemF16N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
       default:
-        return scales ? launch_gemm_cfg<ElemFP8N, 128, 256, 128, 2, 2, 5, true>(p, grid, c.stream, who)
-                      : launch_gemm_cfg<ElemFP8N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+        return scales ? launch_gemm_rows<ElemFP8N, 128, 256, 128, 2, 2, 5, true>(p, grid, c.stream, who)
+                      : launch_gemm_rows<ElemFP8N, 128, 256, 128, 2, 2, 5, false>(p, grid, c.stream, who);
     }
   }
   if (BN == 192) {  // 128 x 192: waves of 64 x 96 on the split ring
     switch (elem) {
-      case kElemBF16: return launch_gemm_cfg<ElemBF16N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
-      case kElemF16: return launch_gemm_cfg<ElemF16N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemBF16: return launch_gemm_rows<ElemBF16N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+      case kElemF16: return launch_gemm_rows<ElemF16N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
       default:
-        return scales ? launch_gemm_cfg<ElemFP8N, 128, 192, 128, 2, 2, 5, true>(p, grid, c.stream, who)
-                      : launch_gemm_cfg<ElemFP8N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
+        return scales ? launch_gemm_rows<ElemFP8N, 128, 192, 128, 2, 2, 5, true>(p, grid, c.stream, who)
+                      : launch_gemm_rows<ElemFP8N, 128, 192, 128, 2, 2, 5, false>(p, grid, c.stream, who);
     }
   }
   // the 128 x 128 tile on a four-stage ring of 64-byte K tiles, 32-row MFMA blocks: every shape
   switch (elem) {
-    case kElemBF16: return launch_gemm_cfg<ElemBF16, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
-    case kElemF16: return launch_gemm_cfg<ElemF16, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
+    case kElemBF16: return launch_gemm_rows<ElemBF16, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
+    case kElemF16: return launch_gemm_rows<ElemF16, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
     default:
-      return scales ? launch_gemm_cfg<ElemFP8, 128, 128, 64, 2, 2, 4, true>(p, grid, c.stream, who)
-                    : launch_gemm_cfg<ElemFP8, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
+      return scales ? launch_gemm_rows<ElemFP8, 128, 128, 64, 2, 2, 4, true>(p, grid, c.stream, who)
+                    : launch_gemm_rows<ElemFP8, 128, 128, 64, 2, 2, 4, false>(p, grid, c.stream, who);
   }
 }
 
