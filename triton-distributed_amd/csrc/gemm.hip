@@ -2056,7 +2056,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // tiles, which the estimate takes since it counts this; 1536 x 4480 x 14848 bf16 286 -> 157 us for the same reason); small
   // groups make an XCD's block long and narrow: 3 % more at 2 x 16 tiles of 256 x 256 and 9 % at 1 x 32 than at 8 x 4
   // (16384 x 7168 x 8192 e4m3; 4 x 8 there, 28 column tiles, constant operands: 472 us against 455), and no round is faster
-  // than its panels come from the memory-side cache, 7.5 TB/s to all XCDs (128 x 256 tiles one row at a time: 1.2 us a K tile
+  // than its panels come from the memory-side cache, 7.5 TB/s to all XCDs at 1.2 us a K tile of 256 x 256 (128 x 256 tiles one row at a time: 1.2 us a K tile
   // instead of 0.75). Over 300 shapes the tile and walk taken are 1 % from the best ones on average, 4 % before.
   struct Walk { double cost; int rows; };
   auto walk = [&](int t, bool split_last) -> Walk {
@@ -2093,8 +2093,9 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
   // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
   // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us (9 where the rows go to their owners' buffers:
-  // 1024 x 7424 x 768 bf16 22.7 us on 256 x 128, 16.1 on 128 x 128; over 60 scatter calls 0.7 % behind the best tile), handing over a split round 25 us more
-  // (15 of them in its estimate already)
+  // 1024 x 7424 x 768 bf16 22.7 us on 256 x 128, 16.1 on 128 x 128), handing over a split round 23.75 us more (13.75 of them, 12.5 such K tiles,
+  // in its estimate already). Over 280 scatter calls 2 % behind the best tile on average (3072 x 2048 x 1792 f16: 30.1 us on the small tiles, 24.9 on
+  // 256 x 128); a time per round and tile beside the rate, fitted to the same calls, does no better.
   // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 14 us on 256 of 128 x 128; 200 x 1536 x 4096 bf16: 26 -> 12 us;
   // 768 x 4952 x 2448 f16 37 -> 26, 2560 x 776 x 5936 68 -> 56; 2048 x 2104 x 4080 stays on the large tiles, 53 us against 70). Most
   // calls that take them are told by a bound that needs no walk (a microsecond of host time less): every tile's work at its rate,
@@ -2124,7 +2125,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
-      // (and 15 us in the same units, 1.2 us per K tile of the 256 x 256 tile: what the exchange takes beside its bytes)
+      // (and 12.5 K tiles of the 256 x 256 tile, 13.75 us: what the exchange takes beside its bytes)
       const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / rate(t)) + 15.0 / 1.2 * 65536.0;
       if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
@@ -2134,10 +2135,10 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   if (use_sk) pick = pick_split;
   // One round of 256 x 128 tiles in place of one of 128 x 192: the rates are those of many rounds, which end in as many prologues and
   // epilogues, and the larger tile has fewer bytes to fetch per product. Rows of whole 128-byte lines, from 32 K tiles on (20 where the
-  // call has five row tiles or fewer): 4096 x 1536 x 4096 bf16 46.4 -> 44.8 us, with the rows to their owners 46.2 -> 44.7, behind flags
-  // 49.4 -> 48.6; 768 x 7168 x 3072 behind flags 50.1 -> 36.3; 200 such calls 9 % faster on average, 9 % slower at worst. With shorter rows or
-  // ragged ones it is behind (2560 x 776 x 576 f16 14.1 us, 12.8 on 128 x 192; 3072 x 1472 x 8048 bf16 116, 105), and so it is where a
-  // call that is no ungated one has an odd number of its row tiles beyond five (3840 x 1536 x 4608 e4m3 37.3, 35.3).
+  // call has five row tiles or fewer): 4096 x 1536 x 4096 bf16 behind flags 48.0 -> 45.7 us, with the rows to their owners 46.2 -> 45.3, ungated
+  // 46.4 -> 44.8; 768 x 7168 x 3072 behind flags 49.0 -> 35.2; 200 such calls 9 % faster on average, 9 % slower at worst. With shorter rows or
+  // ragged ones it is behind (2560 x 776 x 576 f16 14.0 us, 12.6 on 128 x 192; 3072 x 1472 x 8048 bf16 109, 94), and so it is where a
+  // call that is no ungated one has an odd number of its row tiles beyond five (3840 x 1536 x 4608 e4m3 36.9, 34.8).
   auto one_round = [&](int t) { return ceil_div(c.M, kChoices[t].bm) * ceil_div(c.N, kChoices[t].bn) <= cap_wgs; };
   const int64_t row_bytes = (int64_t)c.K * esz, row_tiles = ceil_div(c.M, kChoices[1].bm);
   if (!use_sk && pick == 3 && admissible(1) && one_round(1) && one_round(3) && row_bytes % 128 == 0 &&
