@@ -1911,13 +1911,18 @@ struct SmallPlan {
   bool deep;
   double us;
 };
-constexpr double kSmallPairUs[kNumSmallTiles] = {0.5, 0.85};   // a K tile of each of two workgroups on a compute unit
-static double small_tiles_us(int t, int64_t units, int per, int pieces, int cus, const double* pair_us = kSmallPairUs) {
+struct SmallTimes {
+  double launch, alone[kNumSmallTiles], one_round;     // a K tile of the only workgroup on a compute unit, and what is beside them
+  double pair[kNumSmallTiles], round[kNumSmallTiles];  // a K tile of each of two, and what a round of them has beside
+};
+constexpr SmallTimes kSmallPlain = {3.0, {0.225, 0.315}, 1.0, {0.5, 0.85}, {1.5, 1.5}};
+constexpr SmallTimes kSmallScatter = {0.7, {0.255, 0.385}, 4.0, {0.51, 0.85}, {3.0, 4.4}};   // rows to several owners' buffers
+static double small_tiles_us(int t, int64_t units, int per, int pieces, int cus, const SmallTimes& time) {
   const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn;
-  const double alone = t == 0 ? 0.225 : 0.315, stage_mb = (bm + bn) * 128 * 1e-6;
-  double us = 3.0;
-  if (units <= cus) us += per * std::max(alone, units * stage_mb / 24.0) + 1.0;
-  else us += (double)ceil_div(units, 2 * cus) * (per * pair_us[t] + 1.5);
+  const double stage_mb = (bm + bn) * 128 * 1e-6;
+  double us = time.launch;
+  if (units <= cus) us += per * std::max(time.alone[t], units * stage_mb / 24.0) + time.one_round;
+  else us += (double)ceil_div(units, 2 * cus) * (per * time.pair[t] + time.round[t]);
   if (pieces > 1) us += 1.2 + (t == 0 ? 0.25 : 0.6) * pieces + (double)units * bm * bn * 4 / 3.0e6;
   return us;
 }
@@ -1938,7 +1943,7 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
       if (sk > 1 && s != sk) continue;
       const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
       const int64_t units = tiles * pieces;
-      const double us = small_tiles_us(t, units, per, pieces, cus);
+      const double us = small_tiles_us(t, units, per, pieces, cus, c.scatter_bufs ? kSmallScatter : kSmallPlain);
       if (best.us == 0 || us < best.us) best = {t, pieces, per, units <= cus, us};
     }
   }
@@ -2036,6 +2041,13 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // (behind flags the 256x256 tile has gating code too, and the 256x128 one is nearer to it: 4096 x 5208 x 3008 bf16 134 us on the large tile,
   // 115 on three rounds of the other; 26 gated shapes are 0.9 % behind the best tile, 2.0 % with 0.70 and 5.5 % with 0.88)
   auto rate = [&](int t) { return t == 1 && c.flags ? 0.80 : kChoices[t].eff; };
+  // (with the rows to their owners' buffers a tile's prologue and epilogue weigh more and the smaller tiles keep up better: microseconds per
+  // 128 bytes of K and per round of every tile, fitted to 280 such calls of 256 to 16384 rows with the small tiles' above. The tile taken is 0.6 %
+  // behind the best on average and 15 % at worst, with the rates above and 9 us a launch 2.1 and 40 %: 10240 x 2304 x 1536 f16 91 -> 79 us,
+  // 3072 x 2048 x 1792 f16 30 -> 25, 5120 x 1024 x 1792 e4m3 23.8 -> 21.1 with their reductions)
+  static const double kScatterKTile[kNumChoices] = {1.075, 0.61, 0.60, 0.585, 0.70}, kScatterRound[kNumChoices] = {7.2, 5.0, 4.0, 5.2, 4.6};
+  constexpr double kKTileUs = 1.1, kUnits = 65536.0 / kKTileUs;   // a K tile of 256 x 256, which costs 65536 units; units of a microsecond
+  auto k_tile_units = [&](int t) { return c.scatter_bufs ? kScatterKTile[t] * kUnits : kChoices[t].bm * kChoices[t].bn / rate(t); };
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
   // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
@@ -2062,7 +2074,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   auto walk = [&](int t, bool split_last) -> Walk {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int tiles_m = (c.M + bm - 1) / bm, tiles_n = (c.N + bn - 1) / bn;
-    const double per_k_tile = (double)bm * bn / rate(t);
+    const double per_k_tile = c.scatter_bufs ? k_tile_units(t) * k_tile_bytes(t) / 128 : k_tile_units(t);
     auto rounds = [&](int64_t positions) -> double {
       const int64_t full = positions < 0x7fffffff ? (int)positions / cap_wgs : positions / cap_wgs, tail = positions - full * cap_wgs;
       if (tail == 0 || !split_last) return (double)(full + (tail != 0));
@@ -2091,26 +2103,24 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // costs 1/s of a round plus one exchange of the tile's accumulators, and that form is taken where it beats whole
   // tiles by a margin.
   const int sk_mode = sk_env(), forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
-  // The small tiles where their estimate is clearly the lower one. In the same microseconds: a 128-byte K tile of the
-  // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us (9 where the rows go to their owners' buffers:
-  // 1024 x 7424 x 768 bf16 22.7 us on 256 x 128, 16.1 on 128 x 128), handing over a split round 23.75 us more (13.75 of them, 12.5 such K tiles,
-  // in its estimate already). Over 280 scatter calls 2 % behind the best tile on average (3072 x 2048 x 1792 f16: 30.1 us on the small tiles, 24.9 on
-  // 256 x 128); a time per round and tile beside the rate, fitted to the same calls, does no better.
+  // The small tiles where their estimate is the lower one, clearly so but for rows to their owners. In the same microseconds: a 128-byte K tile of the
+  // 256 x 256 tile takes 1.1 us, a launch with one tile's prologue and epilogue 6 us (3.2 where the rounds have a time of their own), handing
+  // over a split round 23.75 us more (13.75 of them, 12.5 such K tiles, in its estimate already).
   // (1024 x 4096 x 1536 f16: 37 us on 128 split tiles of 128 x 256, 14 us on 256 of 128 x 128; 200 x 1536 x 4096 bf16: 26 -> 12 us;
   // 768 x 4952 x 2448 f16 37 -> 26, 2560 x 776 x 5936 68 -> 56; 2048 x 2104 x 4080 stays on the large tiles, 53 us against 70). Most
   // calls that take them are told by a bound that needs no walk (a microsecond of host time less): every tile's work at its rate,
   // no hand-over, no last round.
   const SmallPlan small = small_plan(c, esz, di.num_cus);
-  const double launch_us = c.scatter_bufs ? 9.0 : 6.0;
+  const double launch_us = c.scatter_bufs ? 3.2 : 6.0, margin = c.scatter_bufs ? 1.0 : 0.95;
   if (small.us > 0 && forced_tile < 0) {
     double least = 0;
     for (int t = 0; t < kNumChoices; ++t) {
       const int bm = kChoices[t].bm, bn = kChoices[t].bn;
       const double tiles = (double)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn), rounds = std::max(tiles / cap_wgs, 1.0 / kSkMaxSplit);
-      const double cost = rounds * bm * bn / rate(t) * c.K * esz / 128.0;
+      const double cost = rounds * k_tile_units(t) * c.K * esz / 128.0 + (c.scatter_bufs ? std::max(1.0, rounds) * kScatterRound[t] * kUnits : 0.0);
       if (admissible(t) && (least == 0 || cost < least)) least = cost;
     }
-    if (small.us < 0.95 * (launch_us + least / 65536.0 * 1.1)) return run_small(c, elem, esz, small, di);
+    if (small.us < margin * (launch_us + least / kUnits)) return run_small(c, elem, esz, small, di);
   }
   int pick = 2, pick_split = -1;
   double whole = 0, split_last = 0;
@@ -2119,14 +2129,15 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int64_t tiles = ceil_div(c.M, bm) * ceil_div(c.N, bn);
     const int64_t kt = ceil_div((int64_t)c.K * esz, k_tile_bytes(t));
-    const double cost = walk(t, false).cost * kt;
+    const double beside = c.scatter_bufs ? (double)ceil_div(tiles, cap_wgs) * kScatterRound[t] * kUnits : 0.0;
+    const double cost = walk(t, false).cost * kt + beside;
     if (whole == 0 || cost < whole) whole = cost, pick = t;
     const int64_t tail = tiles % cap_wgs;
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
       // (and 12.5 K tiles of the 256 x 256 tile, 13.75 us: what the exchange takes beside its bytes)
-      const double cost_sk = walk(t, true).cost * kt + sk_handover_k_tiles(bm, bn) * ((double)bm * bn / rate(t)) + 15.0 / 1.2 * 65536.0;
+      const double cost_sk = walk(t, true).cost * kt + beside + sk_handover_k_tiles(bm, bn) * k_tile_units(t) + 12.5 * 65536.0;
       if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
   }
@@ -2145,8 +2156,8 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       row_bytes >= (row_tiles <= 5 ? 20 : 32) * 128 && (row_tiles <= 5 || row_tiles % 2 == 0 || !(c.flags || c.scatter_bufs))) pick = 1;
   const double best = use_sk ? split_last : whole;
   if (small.us > 0) {
-    const double large_us = launch_us + best / 65536.0 * 1.1 * (pick == 2 ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
-    if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < 0.95 * large_us)) return run_small(c, elem, esz, small, di);
+    const double large_us = launch_us + best / kUnits * (pick == 2 && !c.scatter_bufs ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
+    if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < margin * large_us)) return run_small(c, elem, esz, small, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,
   // 4 = 128x256; a tile that the call's row blocks or K do not admit is not taken.
@@ -2405,7 +2416,7 @@ static double group_panels_us(const GroupShape& g, double bytes, double cache_by
 // On small tile t; `capacity`: blocks that there is room for. (A pair of workgroups takes longer than in an ungrouped GEMM: no two
 // of them share their weights.)
 static SmallPlan group_small_plan(const GroupShape& g, int t, int64_t capacity, int64_t workspace_bytes, int cus) {
-  constexpr double kPairUs[kNumSmallTiles] = {0.77, 1.18};
+  constexpr SmallTimes kTimes = {3.0, {0.225, 0.315}, 1.0, {0.77, 1.18}, {1.5, 1.5}};
   SmallPlan best = {t, 0, 0, false, 0};
   const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn, k_tiles = (int)ceil_div(g.k_bytes, 128), sk = debug_get(TDIST_DEBUG_GEMM_SPLIT_K);
   const int64_t tiles_n = ceil_div(g.N, bn), used = group_blocks(g, bm) * tiles_n, tiles = capacity * tiles_n;
@@ -2415,7 +2426,7 @@ static SmallPlan group_small_plan(const GroupShape& g, int t, int64_t capacity, 
                   workspace_bytes < kSkHeaderBytes + tiles * s * bm * bn * 4)) break;
     if (sk > 1 && s != sk && s != 1) continue;   // (a forced number of pieces that K does not allow: whole)
     const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
-    const double us = std::max(small_tiles_us(t, used * pieces, per, pieces, cus, kPairUs), panels);
+    const double us = std::max(small_tiles_us(t, used * pieces, per, pieces, cus, kTimes), panels);
     if (best.us == 0 || us < best.us || (sk > 1 && s == sk)) best = {t, pieces, per, used * pieces <= cus, us};
   }
   return best;
