@@ -45,7 +45,7 @@ MEASURED_SOURCE_DIGEST = {
     "common.h": "f5b639d6f2c93627",
     "decode.hip": "3ac771befeb01e03",
     "gather.h": "3fd5e450cd06de4d",
-    "gemm.hip": "8067bf3e0cc9629d",
+    "gemm.hip": "c08abbcdb78be098",
     "gemm_small.h": "ef635860051b59ae",
     "gemm_small.hip": "9f3cf4730167f9a0",
     "moe.hip": "b232f7830cc66aab",

@@ -2038,16 +2038,21 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // before: 2048 x 4304 x 3040 f16 79 -> 57 us, 7168 x 7128 x 3792 e4m3 241 -> 179; the smaller tiles fetch more operand bytes
   // per product, and the 256x256 tile alone has an instance without gating code)
   static const TileChoice kChoices[kNumChoices] = {{256, 256, 1.0}, {256, 128, 0.70}, {128, 128, 0.48}, {128, 192, 0.62}, {128, 256, 0.70}};
-  // (behind flags the 256x256 tile has gating code too, and the 256x128 one is nearer to it: 4096 x 5208 x 3008 bf16 134 us on the large tile,
-  // 115 on three rounds of the other; 26 gated shapes are 0.9 % behind the best tile, 2.0 % with 0.70 and 5.5 % with 0.88)
+  // (with the rows to their owners' buffers, or behind flags, a tile's prologue and epilogue weigh more and the smaller tiles keep up better:
+  // microseconds per 128 bytes of K and per round of every tile. Rows to their owners, fitted to 280 such calls of 256 to 16384 rows with
+  // the small tiles' above: the tile taken is 0.6 % behind the best on average and 15 % at worst, with the rates above and 9 us a launch 2.1
+  // and 40 %: 10240 x 2304 x 1536 f16 91 -> 79 us, 3072 x 2048 x 1792 f16 30 -> 25, 5120 x 1024 x 1792 e4m3 23.8 -> 21.1 with their reductions.
+  // Behind flags, fitted to 135 calls of whole 128-row chunks and K tiles, for which they stand: over 310 others 4 % faster on average than with the rates above and 0.80 for 256x128, 119 by more than
+  // 3 % (4096 x 1024 x 5632 f16 75 -> 57 us, 512 x 1536 x 5120 e4m3 39 -> 24), 5 slower by as much (768 x 4352 x 7936 bf16 80 -> 89))
+  struct TileTimes { double k_tile, round; };
+  static const TileTimes kScatterTimes[kNumChoices] = {{1.075, 7.2}, {0.61, 5.0}, {0.60, 4.0}, {0.585, 5.2}, {0.70, 4.6}};
+  static const TileTimes kGatedTimes[kNumChoices] = {{1.057, 9.3}, {0.542, 7.15}, {0.68, 5.7}, {0.57, 6.66}, {0.687, 5.88}};
+  const bool gated_times = c.flags && !ragged && (int64_t)c.K * esz % 128 == 0;
+  const TileTimes* const times = c.scatter_bufs ? kScatterTimes : gated_times ? kGatedTimes : nullptr;
+  // (for the other calls behind flags: 4096 x 5208 x 3008 bf16 115 us on three rounds of 256x128, 134 on 256x256)
   auto rate = [&](int t) { return t == 1 && c.flags ? 0.80 : kChoices[t].eff; };
-  // (with the rows to their owners' buffers a tile's prologue and epilogue weigh more and the smaller tiles keep up better: microseconds per
-  // 128 bytes of K and per round of every tile, fitted to 280 such calls of 256 to 16384 rows with the small tiles' above. The tile taken is 0.6 %
-  // behind the best on average and 15 % at worst, with the rates above and 9 us a launch 2.1 and 40 %: 10240 x 2304 x 1536 f16 91 -> 79 us,
-  // 3072 x 2048 x 1792 f16 30 -> 25, 5120 x 1024 x 1792 e4m3 23.8 -> 21.1 with their reductions)
-  static const double kScatterKTile[kNumChoices] = {1.075, 0.61, 0.60, 0.585, 0.70}, kScatterRound[kNumChoices] = {7.2, 5.0, 4.0, 5.2, 4.6};
   constexpr double kKTileUs = 1.1, kUnits = 65536.0 / kKTileUs;   // a K tile of 256 x 256, which costs 65536 units; units of a microsecond
-  auto k_tile_units = [&](int t) { return c.scatter_bufs ? kScatterKTile[t] * kUnits : kChoices[t].bm * kChoices[t].bn / rate(t); };
+  auto k_tile_units = [&](int t) { return times ? times[t].k_tile * kUnits : kChoices[t].bm * kChoices[t].bn / rate(t); };
   auto admissible = [&](int t) { return kChoices[t].bm == 256 ? rows256 : (kChoices[t].bn == 128 || k128); };
   auto k_tile_bytes = [&](int t) { return kChoices[t].bm == 256 || kChoices[t].bn != 128 ? 128 : 64; };
   // An XCD's workgroups (one in num_xcds of the grid) work on a block of rows x cols tiles at a time and fetch the
@@ -2074,7 +2079,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   auto walk = [&](int t, bool split_last) -> Walk {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int tiles_m = (c.M + bm - 1) / bm, tiles_n = (c.N + bn - 1) / bn;
-    const double per_k_tile = c.scatter_bufs ? k_tile_units(t) * k_tile_bytes(t) / 128 : k_tile_units(t);
+    const double per_k_tile = times ? k_tile_units(t) * k_tile_bytes(t) / 128 : k_tile_units(t);
     auto rounds = [&](int64_t positions) -> double {
       const int64_t full = positions < 0x7fffffff ? (int)positions / cap_wgs : positions / cap_wgs, tail = positions - full * cap_wgs;
       if (tail == 0 || !split_last) return (double)(full + (tail != 0));
@@ -2111,13 +2116,14 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // calls that take them are told by a bound that needs no walk (a microsecond of host time less): every tile's work at its rate,
   // no hand-over, no last round.
   const SmallPlan small = small_plan(c, esz, di.num_cus);
+  constexpr double kHandoverUs = 10.0;
   const double launch_us = c.scatter_bufs ? 3.2 : 6.0, margin = c.scatter_bufs ? 1.0 : 0.95;
   if (small.us > 0 && forced_tile < 0) {
     double least = 0;
     for (int t = 0; t < kNumChoices; ++t) {
       const int bm = kChoices[t].bm, bn = kChoices[t].bn;
       const double tiles = (double)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn), rounds = std::max(tiles / cap_wgs, 1.0 / kSkMaxSplit);
-      const double cost = rounds * k_tile_units(t) * c.K * esz / 128.0 + (c.scatter_bufs ? std::max(1.0, rounds) * kScatterRound[t] * kUnits : 0.0);
+      const double cost = rounds * k_tile_units(t) * c.K * esz / 128.0 + (times ? std::max(1.0, rounds) * times[t].round * kUnits : 0.0);
       if (admissible(t) && (least == 0 || cost < least)) least = cost;
     }
     if (small.us < margin * (launch_us + least / kUnits)) return run_small(c, elem, esz, small, di);
@@ -2129,15 +2135,16 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
     const int bm = kChoices[t].bm, bn = kChoices[t].bn;
     const int64_t tiles = ceil_div(c.M, bm) * ceil_div(c.N, bn);
     const int64_t kt = ceil_div((int64_t)c.K * esz, k_tile_bytes(t));
-    const double beside = c.scatter_bufs ? (double)ceil_div(tiles, cap_wgs) * kScatterRound[t] * kUnits : 0.0;
+    const double beside = times ? (double)ceil_div(tiles, cap_wgs) * times[t].round * kUnits : 0.0;
     const double cost = walk(t, false).cost * kt + beside;
     if (whole == 0 || cost < whole) whole = cost, pick = t;
     const int64_t tail = tiles % cap_wgs;
     const int split = tail > 0 ? sk_split_for(cap_wgs, (int)tail, (int)(kt < 0x7fffffff ? kt : 0x7fffffff)) : 1;
     // (the exchange of the split form is written for staged rows of a power-of-two width: not for the 128x192 tile)
     if (sk_mode != 0 && split >= 2 && bn != 192 && sk_workspace_fits(c.sk_workspace, c.sk_workspace_bytes, cap_wgs, bm, bn)) {
-      // (and 12.5 K tiles of the 256 x 256 tile, 13.75 us: what the exchange takes beside its bytes)
-      const double cost_sk = walk(t, true).cost * kt + beside + sk_handover_k_tiles(bm, bn) * k_tile_units(t) + 12.5 * 65536.0;
+      // (and 12.5 K tiles of the 256 x 256 tile, 13.75 us: what the exchange takes beside its bytes; all of the 23.75 behind flags, where 1536 x 5888 x 7936
+      // e4m3 was split with 13.75, 87 us, 73 on one round of 256 x 256; with rows to their owners 2816 x 3072 x 3840 f16 is 79 us split, 83 not)
+      const double cost_sk = walk(t, true).cost * kt + beside + sk_handover_k_tiles(bm, bn) * k_tile_units(t) + 12.5 * 65536.0 + (gated_times ? kHandoverUs * kUnits : 0.0);
       if (pick_split < 0 || cost_sk < split_last) split_last = cost_sk, pick_split = t;
     }
   }
@@ -2156,7 +2163,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
       row_bytes >= (row_tiles <= 5 ? 20 : 32) * 128 && (row_tiles <= 5 || row_tiles % 2 == 0 || !(c.flags || c.scatter_bufs))) pick = 1;
   const double best = use_sk ? split_last : whole;
   if (small.us > 0) {
-    const double large_us = launch_us + best / kUnits * (pick == 2 && !c.scatter_bufs ? 0.5 : 1.0) + (use_sk ? 10.0 : 0.0);
+    const double large_us = launch_us + best / kUnits * (pick == 2 && !c.scatter_bufs ? 0.5 : 1.0) + (use_sk && !gated_times ? kHandoverUs : 0.0);
     if (forced_tile >= kNumLargeTiles || (forced_tile < 0 && small.us < margin * large_us)) return run_small(c, elem, esz, small, di);
   }
   // TDIST_DEBUG_GEMM_TILE forces a tile (test and measurement aid): 0 = 256x256, 1 = 256x128, 2 = 128x128, 3 = 128x192,
