@@ -1851,7 +1851,7 @@ static int launch_gemm_cfg(const GemmParams& prm, int grid, hipStream_t stream, 
 }
 
 // Rows in shards have instances of their own: the test for them, a register or two of every tile's addresses and the launch's end cost the
-// others up to 3 % (the same box, before / after: 16384 x 7168 x 8192 e4m3 behind flags 607.3 / 604.2 us, 8192 x 8192 x 3584 bf16 with its rows to
+// others up to 3 % (both in turn, before / after: 16384 x 7168 x 8192 e4m3 behind flags 607.3 / 604.2 us, 8192 x 8192 x 3584 bf16 with its rows to
 // their owners 317.2 / 316.2, 4096 x 4096 x 4096 e4m3 behind flags 53.6 / 52.3, 7168 x 7128 x 3792 e4m3 ungated 185.0 / 182.6).
 template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true>
 static int launch_gemm_rows(const GemmParams& prm, int grid, hipStream_t stream, const char* who) {
