@@ -1447,6 +1447,9 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(const DecodePara
 // conflicts, none here): 128 / 1 heads, 16 sequences of 64 to 4096 keys 56.6 -> 27.1 us; 16 x 16384 keys 296 -> 144; 64 x 300
 // 44 -> 24; 1 x 1000 19.9 -> 17.0; 16 / 1 heads, 16 x 16384 68.5 -> 63 (4.8 TB/s). The output waves bringing the rows in as well:
 // 16 x 16384 166 us; 64 heads a workgroup: 132, but twice the partial results (the batch of 16 uneven ones 45 us against 41).
+// A score wave shares its SIMD with an output wave and goes first (s_setprio): 16 x 16384 keys 144 -> 130 us, the 16 uneven ones
+// 27.5 -> 26.6. What does not bound it: the rows asked for four blocks ahead by a wave of its own (134 us), or two output waves of 256
+// columns on the other SIMDs (127, but 38 us for 31.8 where many sequences end: 40 up to 2000 keys).
 template <int HB>
 struct LatentCfg {
   static constexpr int kKeys = 32, kDK = 576, kDV = 512;
@@ -1522,6 +1525,7 @@ __global__ __launch_bounds__(LatentCfg<HB>::kThreads) void decode_latent_kernel(
   lds_u8 const s_p = lds + C::kProbs + lane * 16;                         // [2][HB][2 key groups][64]
   // Step s: the scores of block s and the output product of block s - 1. Blocks 0 .. n - 1, steps 0 .. n: every wave meets n + 1 times.
   if (wave >= 4 && wave < 4 + HB) {
+    __builtin_amdgcn_s_setprio(2);   // (ahead of the output wave on the same SIMD: a block's time is this wave's chain)
     const int hb = wave - 4;
     const float scale_log2 = prm.sm_scale * kLog2e;
     // query: head x, columns 32s + 8g .. + 7; operand reads relative to the stage: chunk 4s + g of key x
