@@ -135,6 +135,13 @@ def test_a_long_sequence_over_many_ranges(cuda, num_heads, D, lens):
     check(cuda, num_heads, (D, D), torch.bfloat16, lens, 16, 0, False, D + len(lens))
 
 
+# partial results in tiles of 16 columns: one narrower tile alone, and one behind whole ones; blocks of 16 heads and of fewer
+@pytest.mark.parametrize("num_heads,D", [((20, 1), 8), ((34, 2), 24), ((3, 3), 200)])
+def test_narrow_tiles_of_partial_results(cuda, num_heads, D):
+    announce("decode stream, narrow tiles, heads=%s D=%d" % (num_heads, D))
+    check(cuda, num_heads, (D, D), torch.float16, [2500, 0, 70], 16, 0, False, D)
+
+
 def test_a_long_latent_sequence(cuda):
     announce("decode stream, many ranges, latent heads")
     check(cuda, (16, 1), (576, 512), torch.bfloat16, [21000, 40], 16, 0, True, 5)
