@@ -33,6 +33,13 @@ def test_small_tiles_exact(cuda, tile, pieces, dtype, world, mpr, K, N, E, topk)
         assert torch.equal(got.float().cpu(), want)
 
 
+# experts of enough row blocks that an XCD goes down 2, 4 and 8 of them before the next column, the last group shorter
+@pytest.mark.parametrize("mpr,E", [(141, 1), (600, 1), (600, 2), (601, 3)])
+@pytest.mark.parametrize("tile", [5, 6])
+def test_walk_down_several_row_blocks(cuda, tile, mpr, E):
+    test_small_tiles_exact(cuda, tile, None, torch.bfloat16, 4, mpr, 256, 1288, E, 1)
+
+
 @pytest.mark.parametrize("block", [128, 256])
 @pytest.mark.parametrize("dtype,world,mpr,K,N,E,topk", [(torch.bfloat16, 4, 150, 512, 2312, 6, 3), (torch.float16, 2, 3, 192, 264, 64, 2),
                                                         (torch.float8_e4m3fn, 8, 96, 208, 8200, 3, 2)])

@@ -2395,8 +2395,9 @@ struct GroupGemmCall {
 };
 
 // ---- estimates for the grouped GEMM, in microseconds -------------------------------------------------------------
-// Fitted to the times of all four forms (64 x 128 and 128 x 128 small tiles, 128 x 256 and 256 x 256 large ones) on 70 problems of 16
-// to 18731 rows over 8 to 64 experts: the form taken is 0.3 % behind the best on average (the block sizes of before: 39 %). Beside
+// Fitted to the times of all four forms (64 x 128 and 128 x 128 small tiles, 128 x 256 and 256 x 256 large ones) on 180 problems of 32
+// to 37056 rows over 8 to 64 experts: the form taken is 0.5 % behind the best on average (2.0 % with the figures fitted before the
+// small tiles' walk kept to few panels: 9444 rows over 8 experts, 1408 x 768, 52.7 us on 256 x 256 tiles, 43.4 on 128 x 128). Beside
 // the tiles' work it is the way of the weights that counts: once from memory, again from the caches for an expert's other blocks.
 struct GroupShape {
   int64_t rows;
@@ -2423,11 +2424,11 @@ static double group_panels_us(const GroupShape& g, double bytes, double cache_by
 // On small tile t; `capacity`: blocks that there is room for. (A pair of workgroups takes longer than in an ungrouped GEMM: no two
 // of them share their weights.)
 static SmallPlan group_small_plan(const GroupShape& g, int t, int64_t capacity, int64_t workspace_bytes, int cus) {
-  constexpr SmallTimes kTimes = {3.0, {0.225, 0.315}, 1.0, {0.77, 1.18}, {1.5, 1.5}};
+  constexpr SmallTimes kTimes = {2.5, {0.28, 0.64}, 0.8, {0.635, 1.18}, {1.2, 1.5}};
   SmallPlan best = {t, 0, 0, false, 0};
   const int bm = kSmallTiles[t].bm, bn = kSmallTiles[t].bn, k_tiles = (int)ceil_div(g.k_bytes, 128), sk = debug_get(TDIST_DEBUG_GEMM_SPLIT_K);
   const int64_t tiles_n = ceil_div(g.N, bn), used = group_blocks(g, bm) * tiles_n, tiles = capacity * tiles_n;
-  const double panels = 4.2 + group_panels_us(g, (double)used * k_tiles * bn * 128, 10.6e6);
+  const double panels = 3.9 + group_panels_us(g, (double)used * k_tiles * bn * 128, 11.4e6);
   for (int s = 1; s <= kSmallMaxSplits; s *= 2) {
     if (s > 1 && (sk == 0 || tiles > kSkSmallTiles || k_tiles / s < (sk > 1 ? 2 : kSmallMinPiece) ||
                   workspace_bytes < kSkHeaderBytes + tiles * s * bm * bn * 4)) break;
@@ -2442,11 +2443,11 @@ static SmallPlan group_small_plan(const GroupShape& g, int t, int64_t capacity, 
 static double group_large_us(const GroupShape& g, int block, bool split_last, int cus) {
   const int k_tiles = (int)ceil_div(g.k_bytes, 128);
   const int64_t tiles = group_blocks(g, block) * ceil_div(g.N, 256), full = tiles / cus, tail = tiles % cus;
-  const double k_tile = block == 256 ? 1.5 : 0.955;
-  double us = (double)(full + (tail != 0)) * k_tiles * k_tile;
+  const double k_tile = block == 256 ? 1.5 : 0.9, beside = block == 256 ? 5.8 : 3.2;   // a round's K tiles, and its tiles' ends
+  double us = (double)(full + (tail != 0)) * (k_tiles * k_tile + beside);
   const int s = split_last && tail != 0 && k_tiles >= 2 * kSkMinPiece ? sk_split_for(cus, (int)tail, k_tiles) : 1;
-  if (s > 1) us = (full + 1.0 / s) * k_tiles * k_tile + 24.0;
-  return 11.7 + std::max(us, group_panels_us(g, (double)tiles * k_tiles * (block + 256) * 128, 12.8e6));
+  if (s > 1) us = full * (k_tiles * k_tile + beside) + k_tiles * k_tile / s + 24.0;
+  return 11.0 + std::max(us, group_panels_us(g, (double)tiles * k_tiles * (block + 256) * 128, 13.0e6));
 }
 
 // The small tiles' plan for a call whose blocks have a small tile's rows (us = 0: it does not qualify).

@@ -26,6 +26,7 @@ struct SmallGemmParams {
   int m_per_rank, rank;
   int splits;         // workgroups that share a tile along K
   int tiles_per_split;  // K tiles of 128 bytes per workgroup
+  int walk_rows;      // an XCD's run of tiles goes down this many row tiles before the next column (set by launch_gemm_small)
   float* partials;    // splits > 1: fp32 accumulators, a tile per workgroup
   int32_t* counters;  // splits > 1: one per tile, zero, left zero
   int l2_local;       // workgroup i has been seen to run on XCD i % 8: the pieces of a tile meet in that XCD's L2
