@@ -24,6 +24,8 @@ LIB_NAME = "libtdist_hip.so"
 SOURCES = ["gemm.hip", "gemm_small.hip", "decode.hip", "moe.hip", "lib.hip", "reduce.hip"]
 BENCH_SOURCES = ["bench_probes.hip"]   # libtdist_bench.so: measurement helpers, not part of the product library
 BENCH_LIB_NAME = "libtdist_bench.so"
+TORCH_SOURCE = "torch_calls.cpp"       # tdist_torch.so: the calls on torch tensors, a Python extension module
+TORCH_LIB_NAME = "tdist_torch.so"
 
 # -packed-fp32-ops is removed from the device target on purpose: no v_pk_*_f32 in any kernel.
 HIPCC_FLAGS = [
@@ -48,6 +50,10 @@ def bench_lib_path():
     return os.path.join(OUT_DIR, BENCH_LIB_NAME)
 
 
+def torch_lib_path():
+    return os.path.join(OUT_DIR, TORCH_LIB_NAME)
+
+
 def _hipcc():
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(exe):
@@ -56,7 +62,7 @@ def _hipcc():
 
 
 def _inputs():
-    files = [os.path.join(CSRC, s) for s in SOURCES + BENCH_SOURCES]
+    files = [os.path.join(CSRC, s) for s in SOURCES + BENCH_SOURCES + [TORCH_SOURCE]]
     files += [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_small.h"), os.path.join(CSRC, "gather.h"),
               os.path.join(INCLUDE, "tdist.h"), os.path.join(INCLUDE, "tdist_bench.h")]
     return files
@@ -64,7 +70,7 @@ def _inputs():
 
 def is_stale():
     lib = lib_path()
-    if not os.path.exists(lib) or not os.path.exists(bench_lib_path()):
+    if not all(os.path.exists(f) for f in (lib, bench_lib_path(), torch_lib_path())):
         return True
     t = os.path.getmtime(lib)
     return any(os.path.getmtime(f) > t for f in _inputs())
@@ -177,9 +183,30 @@ def _link(hipcc, objs, out):
     os.replace(tmp, out)
 
 
+def _build_torch_module(hipcc):
+    """The extension module, host code only, linked to torch's libraries and to libtdist_hip.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    tmp = torch_lib_path() + ".tmp"
+    cmd = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", INCLUDE, "-isystem", sysconfig.get_paths()["include"]]
+    for path in include_paths() + ["/opt/rocm/include"]:
+        cmd += ["-isystem", path]
+    cmd += [os.path.join(CSRC, TORCH_SOURCE), "-o", tmp]
+    for path in library_paths():
+        cmd += ["-L", path]
+    cmd += ["-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10", "-L", OUT_DIR, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("hipcc failed on %s:\n%s" % (TORCH_SOURCE, res.stdout))
+    os.replace(tmp, torch_lib_path())
+
+
 def build(force=False, verbose=True):
-    """Compiles every source and links the two shared libraries: libtdist_hip.so (the product) and
-    libtdist_bench.so (measurement helpers for bench.py). Returns the product library's path."""
+    """Compiles every source and links the shared libraries: libtdist_hip.so (the product), libtdist_bench.so
+    (measurement helpers for bench.py) and tdist_torch.so (the calls on torch tensors). Returns the product library's path."""
     if not force and not is_stale():
         return lib_path()
     hipcc = _hipcc()
@@ -193,6 +220,7 @@ def build(force=False, verbose=True):
                 print(log, file=sys.stderr)
     _link(hipcc, [objs[s] for s in BENCH_SOURCES], bench_lib_path())
     _link(hipcc, [objs[s] for s in SOURCES], lib_path())
+    _build_torch_module(hipcc)
     if verbose:
         print("built", lib_path(), file=sys.stderr)
     return lib_path()

@@ -133,6 +133,30 @@ def load():
     return lib
 
 
+TORCH_LIB_PATH = os.path.join(_HERE, "_lib", "tdist_torch.so")
+_native = None
+
+
+def native():
+    """The extension module tdist_torch (csrc/torch_calls.cpp), loaded once: the ordinary form of the package's calls, checked,
+    allocated for and launched without the interpreter. Its functions return None, with nothing done, for a call of another form."""
+    global _native
+    if _native is None:
+        import importlib.machinery
+        import importlib.util
+
+        import torch  # noqa: F401  (the libraries it is linked against)
+        load()
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise RuntimeError("tdist_torch.so is missing at %s: build it with `python triton-distributed_amd/build.py`" % TORCH_LIB_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("tdist_torch", TORCH_LIB_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("tdist_torch", TORCH_LIB_PATH, loader=loader))
+        loader.exec_module(mod)
+        mod.set_error(TdistError)
+        _native = mod
+    return _native
+
+
 def last_error():
     msg = load().tdist_last_error_string()
     return msg.decode("utf-8", "replace") if msg else ""

@@ -492,13 +492,19 @@ def ag_gemm_intra_node(a, b, transe_b, ctx, *, row_scale=None, col_scale=None):
         raise RuntimeError("requires ctx for ipc handle")
     if transe_b:
         raise NotImplementedError("transpose weight is not yet supported")
+    at_hand = ctx.num_ranks > 1 and _rows_are_at_hand(a, ctx)
+    if at_hand:
+        C = _lib.native().ag_gemm(a, b, ctx.peer_shards, ctx.rank, ctx.num_ranks, ctx.workspace_tensors[ctx.rank], ctx.status, ctx.sk_workspace,
+                                  ctx.gemm_stream.cuda_stream, row_scale, col_scale)
+        if C is not None:
+            return C
     _lib.require_cuda(a, b)
     M_per_rank, K = a.shape
     N_per_rank = b.shape[0]
     out_dtype = a.dtype if a.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
     C = torch.empty([ctx.num_ranks * M_per_rank, N_per_rank], dtype=out_dtype, device=a.device)
 
-    shards = _lib.shard_table(a, ctx.peer_shards, ctx.rank, ctx.num_ranks) if ctx.num_ranks > 1 and _rows_are_at_hand(a, ctx) else None
+    shards = _lib.shard_table(a, ctx.peer_shards, ctx.rank, ctx.num_ranks) if at_hand else None
     if shards is not None and (M_per_rank * a.shape[1] * a.element_size()) % 16 == 0:
         assert a.shape[1] == b.shape[1], "Incompatible dimensions"
         assert a.dtype == b.dtype, "Incompatible dtypes"

@@ -67,6 +67,10 @@ def sort_topk_ids_align_block_size(
             at += (n + 3) // 4 * 4
         plan = _ALIGN_PLANS[key] = (ws_bytes, at, tuple(starts), sizes)
     ws_bytes, n_flat, starts, sizes = plan
+    if moe_stream is None:
+        out = _lib.native().align(topk_ids, num_experts, num_ranks, block_size, starts, sizes, n_flat, _lib.zeroed_scratch(ws_bytes, dev), ws_bytes)
+        if out is not None:
+            return out
     flat = torch.empty(n_flat, dtype=torch.int32, device=dev)
     sorted_ids, expert_ids, block_barrier_ids, rank_block_num, num_tokens_post_pad = [
         flat[a:a + n] for a, n in zip(starts, sizes)]
@@ -130,6 +134,9 @@ class RowBlocks:
     def __init__(self, sorted_ids, experts, segments, padded, num_blocks, block_size, memory=None):
         self.sorted_ids, self.experts, self.segments, self.padded = sorted_ids, experts, segments, padded
         self.num_blocks, self.block_size, self.memory = num_blocks, block_size, memory
+
+    def fields(self):
+        return self.sorted_ids, self.experts, self.segments, self.padded, self.num_blocks, self.block_size
 
 
 def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, block_size, entries, num_experts, n, row_bytes, stream, gather=None,
@@ -389,10 +396,18 @@ def ag_group_gemm_intra_node(a, b, ctx=None, full_topk_ids=None, num_experts=Non
     row t*topk + k is token t of the gathered A times the weights of its k-th expert."""
     if ctx is None:
         raise RuntimeError("one GPU holds a single rank: create the context first and hand it the peers' rows")
-    _lib.require_cuda(a, b)
     M_per_rank, K = a.shape
     E, _, N_per_rank = b.shape
     W, rank = ctx.num_ranks, ctx.rank
+    if W > 1 and ctx.gather_rows and not ctx.held_ranks and ctx.group_gemm_stream is None:
+        blocks = ctx.joined.get((ctx.full_num_tokens, E, N_per_rank, K * a.element_size()))   # (what _gather_and_multiply has made)
+        if blocks is not None:
+            C = _lib.native().ag_group_gemm(a, b, ctx.peer_shards, rank, W, ctx.topk, ctx.workspace_tensors[rank], ctx.status, ctx.sk_workspace,
+                                            ctx.sorted_topk_ids, ctx.aligned_expert_ids, ctx.aligned_num_tokens, ctx.BLOCK_M, ctx.full_num_tokens,
+                                            *blocks.fields())
+            if C is not None:
+                return C
+    _lib.require_cuda(a, b)
     missing = [r for r in range(W) if r != rank and r not in ctx.peer_shards]
     if missing:
         raise RuntimeError("hand the other ranks' token rows to the context first (ctx.set_peer_shards); missing %s" % missing)

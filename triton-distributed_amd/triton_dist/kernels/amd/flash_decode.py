@@ -208,6 +208,10 @@ def gqa_fwd_batch_decode(q, k_cache, v_cache, workspace, q_lens, kv_lens, block_
     lengths (``kv_split``, the reference's fixed number of splits per sequence, is accepted for its signature and
     changes nothing in the result). Returns ``output_combine`` [B,Hq,Dv] (default dtype: q's; the reference hard-codes
     float16, :784)."""
+    if output_combine is None and kv_split == -1:
+        out = _lib.native().decode(q, k_cache, v_cache, block_table, scale, soft_cap, kv_lens)
+        if out is not None:
+            return out
     _check_kv_split(kv_split)
     if output_combine is None:
         output_combine = torch.empty((q.shape[0], q.shape[1], v_cache.shape[-1]), dtype=q.dtype, device=q.device)

@@ -154,6 +154,10 @@ def gemm_rs_intra_node(a, b, ctx, *, row_scale=None, col_scale=None):
     Returns:
         c (torch.Tensor<bfloat16/float16>): shape [M // world_size, N]
     """
+    if ctx.fuse_scatter and not ctx.transpose_weight:
+        out = _lib.native().gemm_rs(a, b, ctx.rank, ctx.num_ranks, ctx.scatter_bufs[ctx.rank], ctx.scatter_bufs_ptr, ctx.sk_workspace, row_scale, col_scale)
+        if out is not None:
+            return out
     return gemm_rs_intra_node_op(a, b, ctx.output_dtype, ctx.rank, ctx.num_ranks, ctx.scatter_bufs,
                                  ctx.scatter_bufs_ptr, ctx.sync_bufs_ptr, ctx.fuse_scatter, ctx.transpose_weight,
                                  sk_workspace=ctx.sk_workspace, row_scale=row_scale, col_scale=col_scale)

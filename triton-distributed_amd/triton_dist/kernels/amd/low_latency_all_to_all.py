@@ -184,6 +184,10 @@ def moe_dispatch_preprocess(exp_indices: torch.Tensor, num_experts: int, want_to
     One kernel launch. With ``ctx`` the five tensors are the context's own (allocated on the first call for a shape,
     two sets used in turn like the receive buffers, so a result stays valid until the call after next) and the call
     allocates nothing. Returns (splits, split_cumsum, scatter_idx, gather_idx[, topk_idx])."""
+    if ctx is not None and not want_topk_index:
+        out = _lib.native().preprocess(ctx, exp_indices, num_experts)
+        if out is not None:
+            return out
     _lib.require_cuda(exp_indices)
     T, topk = exp_indices.shape
     n = T * topk
@@ -265,6 +269,15 @@ def fast_all_to_all(
     Returns [splits int32[G], recv [W*max_m, hidden], scales [W*max_m] | None] — views into the context's
     buffers, valid until the call after next.
     """
+    out = None
+    if gather_index is None:
+        if online_quant_fp8:
+            if expert_ids is None and send_scale is None:
+                out = _lib.native().dispatch_quant(ctx, send_tensor, send_split_cumsum, scatter_index)
+        elif expert_ids is not None and scatter_index is None and send_split_cumsum is None:
+            out = _lib.native().dispatch_ids(ctx, send_tensor, send_scale, expert_ids)
+    if out is not None:
+        return out
     _lib.require_cuda(send_tensor, send_split_cumsum, send_scale, gather_index, scatter_index, expert_ids)
     if expert_ids is not None:
         if online_quant_fp8 or gather_index is not None or scatter_index is not None:
@@ -399,6 +412,10 @@ def moe_weighted_combine(ctx: Optional[AllToAllContext], rows: torch.Tensor, row
 
     ``rows`` is the slot layout returned by fast_all_to_all (from_slots=True, needs ``ctx`` and
     ``split_cumsum``) or a compact expert-sorted [n, hidden] tensor (from_slots=False)."""
+    if from_slots and ctx is not None:
+        out = _lib.native().combine(ctx, rows, row_scale, scatter_idx, topk_weight, split_cumsum)
+        if out is not None:
+            return out
     _lib.require_cuda(rows, row_scale, scatter_idx, topk_weight, split_cumsum)
     T, topk = scatter_idx.shape
     hidden = rows.shape[1]

@@ -129,9 +129,18 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     Returns [M // world_size, hidden]: sum over k of weight[t,k] * (a[t*topk+k] @ b[expert]) for this rank's tokens,
     summed with the other ranks' partial results (reference :889-...; golden test/nvidia/test_moe_reduce_rs.py:103-133).
     The synchronisation arguments are accepted and unused: one stream runs the three steps in order."""
-    _lib.require_cuda(a, b)
     pre = ctx.precompute_ctx
     M, topk = pre.full_topk_ids.shape
+    weight = ctx.topk_weight_f32
+    if ctx.output_dtype == torch.bfloat16 and weight.shape == (M, topk):
+        blocks = ctx.joined.get((pre.full_numel, b.shape[0], b.shape[2], a.shape[1] * a.element_size()))   # (made by the call that saw the size first)
+        if blocks is not None:
+            result = _lib.native().reduce_rs(a, b, rank, world_size, weight, ctx.final_output_buffer, ctx.rs_buffers[ctx.rank], ctx.sk_workspace,
+                                             pre.full_sorted_token_ids, pre.full_token_expert_ids, pre.full_num_tokens_post_padded_list, pre.BLOCK_M,
+                                             pre.full_numel, *blocks.fields())
+            if result is not None:
+                return result
+    _lib.require_cuda(a, b)
     assert a.shape[0] == M * topk and a.dtype == b.dtype and a.shape[1] == b.shape[1]
     hidden = b.shape[2]
     out = ctx.final_output_buffer[:M * topk, :hidden]
@@ -155,7 +164,6 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
     slab = buf[:M, :hidden]
     if slab.shape != (M, hidden) or not slab.is_contiguous():
         raise NotImplementedError("hidden must equal the context's hidden_dim, and the context have rows for %d tokens" % M)
-    weight = ctx.topk_weight_f32
     _lib.require_cuda(out, weight, buf)
     assert weight.dtype == torch.float32 and weight.is_contiguous() and weight.shape == (M, topk)
     if out.dtype != torch.bfloat16 or buf.dtype != torch.bfloat16 or not out.is_contiguous():

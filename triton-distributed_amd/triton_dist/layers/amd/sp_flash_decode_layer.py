@@ -8,6 +8,7 @@ the gather has nobody to talk to: the partial results of the other ranks are pas
 """
 import torch
 
+from triton_dist import _lib
 from triton_dist.kernels.amd.flash_decode import decode_stream, decode_stream_ranks, gqa_fwd_batch_decode_inter_rank_combine
 
 
@@ -44,6 +45,11 @@ class SpGQAFlashDecodeAttention(torch.nn.Module):
         peer_partials: (out [num_ranks, batch, Hq, Dv], lse fp32 [num_ranks, batch, Hq]) holding the other
             ranks' results (row ``rank`` is overwritten with this rank's own); required when num_ranks > 1.
         """
+        if self.num_ranks > 1 and isinstance(peer_partials, tuple) and len(peer_partials) == 2:
+            out = _lib.native().decode_ranks(q, k_cache, v_cache, block_table, self.scale, self.soft_cap, global_kv_lens, self.rank, self.num_ranks,
+                                             self.num_q_heads, self.v_head_dim, self.max_allowed_batch, *peer_partials)
+            if out is not None:
+                return out
         batch = q.shape[0]
         assert global_kv_lens.shape[0] == self.num_ranks
         assert global_kv_lens.shape[1] == batch
