@@ -261,6 +261,14 @@ int tdist_gemm_rs_scatter_fp8e4m3(const void* A, int64_t lda, const void* B, int
 int tdist_reduce_slices(const void* c, int64_t slice_stride, int n_slices, int first_slice, int64_t n_elems,
                         void* out, int dtype, void* stream);
 
+/* Both steps of a rank whose buffer already holds the other ranks' rows: tdist_gemm_rs_scatter_* (dtype: the inputs'; scales for e4m3
+ * only; every buffer [M, N] without gaps) and tdist_reduce_slices over `own` = scatter_bufs[rank], from slice rank + 1 on, into
+ * out [M / world_size, N]. One launch where the product takes the small tiles, whose workgroups then add up the rows that they have
+ * just stored: the same bits, in the buffers too. */
+int tdist_gemm_rs(int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, void* const* scatter_bufs, const void* own,
+                  void* out, int M, int N, int K, const float* row_scale, const float* col_scale, int rank, int world_size,
+                  void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * (c) MoE low-latency dispatch / combine permute.
  *   replaces the test-side preprocessing  test/nvidia/test_all_to_all.py:42-96,314-329

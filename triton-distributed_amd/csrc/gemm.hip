@@ -1834,6 +1834,10 @@ struct GemmCall {
   hipStream_t stream;
   const char* who;
   ShardRows shards;   // rows != 0: A's rows lie in shards
+  // scatter calls whose own rows may be added up beside (rs_out != NULL; see SmallGemmParams): *rs_done says whether they were
+  const void* rs_own = nullptr;
+  void* rs_out = nullptr;
+  bool* rs_done = nullptr;
 };
 
 template <typename E, int BM, int BN, int KB, int WM, int WN, int NST, bool kScales, bool kGrouped = false, bool kPlain = false, bool kHead = true, bool kShards = true>
@@ -1926,6 +1930,20 @@ static double small_tiles_us(int t, int64_t units, int per, int pieces, int cus,
   if (pieces > 1) us += 1.2 + (t == 0 ? 0.25 : 0.6) * pieces + (double)units * bm * bn * 4 / 3.0e6;
   return us;
 }
+// Whether the small tiles add the own rows up themselves: whole 16-byte pieces, and few enough other ranks' rows for a tile's workgroup.
+static bool adds_beside(const GemmCall& c, int tile) {
+  return c.rs_out && (c.world_size - 1) * kSmallTiles[tile].bm <= kSmallSumRows && c.N % 8 == 0 && c.N < 1 << 20 && c.ldc % 8 == 0 && aligned16(c.rs_own) &&
+         aligned16(c.rs_out);
+}
+// Microseconds that adding up this rank's rows takes beside the product: a launch that moves world_size + 1 slices, or the small tiles' loads
+// (measured with and without, each of them in 20 calls of 2 to 8 ranks).
+static double reduce_launch_us(const GemmCall& c) {
+  return c.rs_out ? 2.4 + 0.1 * c.world_size + (c.world_size + 1) * ((double)(c.M / c.world_size) * c.N * 2e-6) / 7.0 : 0.0;
+}
+static double small_reduce_us(const GemmCall& c, int tile) {
+  return adds_beside(c, tile) ? 0.6 + (tile == 0 ? 0.35 : 0.8) * (c.world_size - 1) : reduce_launch_us(c);
+}
+
 static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
   SmallPlan best = {0, 0, 0, false, 0};
   if (c.flags || c.A_local || (int64_t)c.M * c.lda * esz >= (1ll << 31) || (int64_t)c.N * c.ldb * esz >= (1ll << 31)) return best;
@@ -1943,7 +1961,7 @@ static SmallPlan small_plan(const GemmCall& c, int esz, int cus) {
       if (sk > 1 && s != sk) continue;
       const int per = (int)ceil_div(k_tiles, s), pieces = (int)ceil_div(k_tiles, per);
       const int64_t units = tiles * pieces;
-      const double us = small_tiles_us(t, units, per, pieces, cus, c.scatter_bufs ? kSmallScatter : kSmallPlain);
+      const double us = small_tiles_us(t, units, per, pieces, cus, c.scatter_bufs ? kSmallScatter : kSmallPlain) + small_reduce_us(c, t);
       if (best.us == 0 || us < best.us) best = {t, pieces, per, units <= cus, us};
     }
   }
@@ -1968,6 +1986,10 @@ static int run_small(const GemmCall& c, GemmElem elem, int esz, const SmallPlan&
   q.k_bytes = c.K * esz;
   q.m_per_rank = c.scatter_bufs ? c.M / c.world_size : c.M;
   q.rank = c.rank;
+  q.world = c.world_size;
+  q.own = (const unsigned char*)c.rs_own;
+  q.out = adds_beside(c, plan.tile) ? (unsigned char*)c.rs_out : nullptr;
+  if (q.out) *c.rs_done = true;
   q.splits = plan.splits;
   q.tiles_per_split = plan.tiles_per_split;
   q.partials = plan.splits > 1 ? (float*)((unsigned char*)c.sk_workspace + kSkHeaderBytes) : nullptr;
@@ -2117,7 +2139,7 @@ static int run_gemm(const GemmCall& c, GemmElem elem) {
   // no hand-over, no last round.
   const SmallPlan small = small_plan(c, esz, di.num_cus);
   constexpr double kHandoverUs = 10.0;
-  const double launch_us = c.scatter_bufs ? 3.2 : 6.0, margin = c.scatter_bufs ? 1.0 : 0.95;
+  const double launch_us = (c.scatter_bufs ? 3.2 : 6.0) + reduce_launch_us(c), margin = c.scatter_bufs ? 1.0 : 0.95;
   if (small.us > 0 && forced_tile < 0) {
     double least = 0;
     for (int t = 0; t < kNumChoices; ++t) {
@@ -2484,6 +2506,9 @@ static int run_group_small(const GroupGemmCall& c, GemmElem elem, int esz, const
   q.k_bytes = c.K * esz;
   q.m_per_rank = q.M;
   q.rank = 0;
+  q.world = 1;
+  q.own = nullptr;
+  q.out = nullptr;
   q.splits = plan.splits;
   q.tiles_per_split = plan.tiles_per_split;
   q.partials = plan.splits > 1 ? (float*)((unsigned char*)c.sk_workspace + kSkHeaderBytes) : nullptr;
@@ -2686,10 +2711,20 @@ int tdist_gemm_chunk_gated_fp8e4m3(const void* A, int64_t lda, const void* A_loc
   TDIST_GATED_BODY(kElemFP8, row_scale, col_scale, "tdist_gemm_chunk_gated_fp8e4m3")
 }
 
+static int elem_of(int dtype, GemmElem& elem, const char* who) {
+  switch (dtype) {
+    case TDIST_BF16: elem = kElemBF16; return TDIST_OK;
+    case TDIST_F16: elem = kElemF16; return TDIST_OK;
+    case TDIST_F8E4M3: elem = kElemFP8; return TDIST_OK;
+    default: return fail(TDIST_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
+  }
+}
+
 static int gemm_rs_scatter(GemmElem elem, const void* A, int64_t lda, const void* B, int64_t ldb,
                            void* const* scatter_bufs, int64_t ldc, int M, int N, int K, int rank, int world_size,
                            void* sk_workspace, int64_t sk_workspace_bytes, void* stream, const char* who,
-                           const float* row_scale = nullptr, const float* col_scale = nullptr) {
+                           const float* row_scale = nullptr, const float* col_scale = nullptr, const void* rs_own = nullptr,
+                           void* rs_out = nullptr, bool* rs_done = nullptr) {
   if (!scatter_bufs) return fail(TDIST_ERR_INVALID, "%s: null scatter_bufs", who);
   GemmCall c;
   c.shards.rows = 0;
@@ -2699,7 +2734,24 @@ static int gemm_rs_scatter(GemmElem elem, const void* A, int64_t lda, const void
   c.chunk_order = nullptr; c.rank = rank; c.world_size = world_size; c.spin_limit = 0; c.status = nullptr;
   c.max_workgroups = 0; c.sk_workspace = sk_workspace; c.sk_workspace_bytes = sk_workspace_bytes;
   c.stream = (hipStream_t)stream; c.who = who;
+  c.rs_own = rs_own; c.rs_out = rs_out; c.rs_done = rs_done;
   return run_gemm(c, elem);
+}
+
+int tdist_gemm_rs(int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, void* const* scatter_bufs, const void* own, void* out, int M,
+                  int N, int K, const float* row_scale, const float* col_scale, int rank, int world_size, void* sk_workspace,
+                  int64_t sk_workspace_bytes, void* stream) {
+  const char* who = "tdist_gemm_rs";
+  GemmElem elem;
+  if (int rc = elem_of(dtype, elem, who)) return rc;
+  if (!own || !out) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (dtype != TDIST_F8E4M3 && (row_scale || col_scale)) return fail(TDIST_ERR_INVALID, "%s: scales are for e4m3 inputs", who);
+  bool done = false;
+  if (int rc = gemm_rs_scatter(elem, A, lda, B, ldb, scatter_bufs, N, M, N, K, rank, world_size, sk_workspace, sk_workspace_bytes, stream, who,
+                               row_scale, col_scale, own, out, &done)) return rc;
+  if (done) return TDIST_OK;
+  const int64_t slice = (int64_t)(M / world_size) * N;
+  return tdist_reduce_slices(own, slice, world_size, (rank + 1) % world_size, slice, out, dtype == TDIST_F16 ? TDIST_F16 : TDIST_BF16, stream);
 }
 
 int tdist_gemm_rs_scatter_bf16(const void* A, int64_t lda, const void* B, int64_t ldb, void* const* scatter_bufs,
@@ -2721,15 +2773,6 @@ int tdist_gemm_rs_scatter_fp8e4m3(const void* A, int64_t lda, const void* B, int
                                   int rank, int world_size, void* sk_workspace, int64_t sk_workspace_bytes, void* stream) {
   return gemm_rs_scatter(kElemFP8, A, lda, B, ldb, scatter_bufs, ldc, M, N, K, rank, world_size, sk_workspace,
                          sk_workspace_bytes, stream, "tdist_gemm_rs_scatter_fp8e4m3", row_scale, col_scale);
-}
-
-static int elem_of(int dtype, GemmElem& elem, const char* who) {
-  switch (dtype) {
-    case TDIST_BF16: elem = kElemBF16; return TDIST_OK;
-    case TDIST_F16: elem = kElemF16; return TDIST_OK;
-    case TDIST_F8E4M3: elem = kElemFP8; return TDIST_OK;
-    default: return fail(TDIST_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
-  }
 }
 
 int tdist_ag_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, void* workspace, const void* B, int64_t ldb,

@@ -23,7 +23,11 @@ struct SmallGemmParams {
   int64_t ldc;           // elements
   int M, N;              // grouped: M is the rows of all blocks
   int k_bytes;  // a multiple of 16
-  int m_per_rank, rank;
+  int m_per_rank, rank, world;
+  // GEMM-RS: this rank's rows are added up beside (out != NULL): its buffer, in which the other ranks' rows lie, and their sum [m_per_rank, N],
+  // N and ldc whole 16-byte pieces, all on 16 bytes
+  const unsigned char* own;
+  unsigned char* out;
   int splits;         // workgroups that share a tile along K
   int tiles_per_split;  // K tiles of 128 bytes per workgroup
   int walk_rows;      // an XCD's run of tiles goes down this many row tiles before the next column (set by launch_gemm_small)
@@ -37,6 +41,12 @@ struct SmallGemmTile { int bm, bn; };
 constexpr int kNumSmallTiles = 2;
 constexpr SmallGemmTile kSmallTiles[kNumSmallTiles] = {{64, 128}, {128, 128}};
 constexpr int kSmallMaxSplits = 16;
+// `out`: other ranks' rows that the workgroup of a tile adds up, at most. Only the own rows' tiles have them to load, among the stores of all
+// the others and with 112 KB in flight; the other calls are better off with the reduction's launch (3 to 5 us). Whole calls in a graph, one
+// launch and two: 64-row tiles of 8 ranks, 2048 x 1024 x 768 9.0 and 10.3 us, 5120 x 1280 x 1280 30.2 and 31.6; 128-row ones of 4 ranks,
+// 1024 x 3328 x 1792 19.2 and 19.7, of 2, 2048 x 2048 x 8192 63.5 and 65.1; of 8, 1024 x 4096 x 1536, 22.1 and 20.1. (With their lines brought
+// into the L2 first, or asked for in front of the products, they were no faster, and the other tiles slower.)
+constexpr int kSmallSumRows = 448;
 constexpr int kGroupedFewRows = kSmallTiles[0].bm;   // rows of the smallest blocks of the grouped form
 
 // `deep`: six stages instead of three, one workgroup per compute unit

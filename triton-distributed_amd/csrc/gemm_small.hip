@@ -18,6 +18,8 @@
 //    weights. 64 experts of 72 rows in all, 2 x 512 x 2176: 51 us a launch on tiles of 128 x 256 cut along K (86 tiles, a third
 //    of their loads rows that are not there), 21 on 64 x 128, or 5.4 TB/s; 311 rows over 16 experts, 1280 x 3200: 62 -> 30;
 //    1454 rows over 16, 3584 x 896: 37 -> 25 on 128 x 128;
+//  * GEMM-RS (rows to their owners' buffers): this rank's tiles add the other ranks' rows to what they store, where that is little for one
+//    workgroup (kSmallSumRows): 2 to 3 us less than a launch for it. 512 x 3840 x 2304 e4m3 of 2 ranks 11.6 -> 9.3 us, 1024 x 3584 x 768 bf16 of 4 12.7 -> 10.9;
 //  * with `splits` > 1 every workgroup leaves its fp32 accumulators in the workspace and bumps its tile's counter; the last
 //    to arrive adds the pieces up in their K order, so the result does not depend on timing and nobody waits. The pieces
 //    of a tile meet in one XCD's L2 where workgroup i is known to run on XCD i % 8 (written through to memory they cost
@@ -33,6 +35,7 @@ namespace tdist {
 static __device__ __align__(16) const unsigned char kZeroChunk16[16] = {0};
 
 struct SmallBF16 {
+  typedef BF16 store;   // the results' type
   static constexpr int kVecs = 1, kSteps = 2;  // 16-byte pieces per operand fragment, MFMA steps per 128 bytes of K
   typedef int4v frag;
   __device__ static __forceinline__ float4v mma(frag a, frag b, float4v c) {
@@ -41,12 +44,14 @@ struct SmallBF16 {
   __device__ static __forceinline__ uint32_t pack(float a, float b) { return pack_bf16x2(a, b); }
 };
 struct SmallF16 : SmallBF16 {
+  typedef F16 store;
   __device__ static __forceinline__ float4v mma(frag a, frag b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, a), __builtin_bit_cast(f16x8v, b), c, 0, 0, 0);
   }
   __device__ static __forceinline__ uint32_t pack(float a, float b) { return pack_f16x2(a, b); }
 };
 struct SmallFP8 {
+  typedef BF16 store;
   static constexpr int kVecs = 2, kSteps = 1;
   typedef int8v frag;
   __device__ static __forceinline__ float4v mma(frag a, frag b, float4v c) {
@@ -69,8 +74,8 @@ struct SmallCfg {
   static_assert((NST - 2) * kLoads < 64, "vmcnt is 6 bits");
 };
 
-// kRows: where A's rows lie (instances of their own: the test for shards alone costs the other calls 0.3 us of 21)
-enum SmallRows { kRowsPlain, kRowsShards, kRowsGrouped };
+// kRows: where A's rows lie, or the results' (instances of their own: the test for shards alone costs the other calls 0.3 us of 21)
+enum SmallRows { kRowsPlain, kRowsShards, kRowsGrouped, kRowsScatter };
 template <typename E, int BM, int BN, int NST, bool kScales, int kRows>
 __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParams p) {
   typedef SmallCfg<BM, BN, NST> C;
@@ -94,7 +99,18 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
   if (mine >= (tiles >> 3) + (xcd < (tiles & 7))) return;
   const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + mine;
   const int group = tile / (p.walk_rows * tiles_n), in_group = tile - group * p.walk_rows * tiles_n;
-  const int rows_g = min(p.walk_rows, tiles_m - group * p.walk_rows), tn = in_group / rows_g, tm = group * p.walk_rows + in_group - tn * rows_g;
+  const int rows_g = min(p.walk_rows, tiles_m - group * p.walk_rows), tn = in_group / rows_g;
+  int tm = group * p.walk_rows + in_group - tn * rows_g, owner = 0;
+  constexpr bool kScatter = kRows == kRowsScatter;
+  if constexpr (kScatter) {
+    // the owners in turn, this rank first: its tiles, which have the other ranks' rows to add, are spread evenly over the XCDs (8 x 1024
+    // rows by 1024 columns in the order of rows: all of them on one)
+    const int nth = tm / p.world;
+    owner = p.rank + tm - nth * p.world;
+    if (owner >= p.world) owner -= p.world;
+    tm = owner * (p.m_per_rank / BM) + nth;
+  }
+  const bool adds = kScatter && p.out != nullptr && owner == p.rank;   // the sum of this tile is this workgroup's
   const int m0 = tm * BM, n0 = tn * BN;
   const int k_tiles = (p.k_bytes + kSmallKB - 1) / kSmallKB;
   const int back = k_tiles * kSmallKB - p.k_bytes;   // bytes of the first K tile in front of the rows
@@ -175,6 +191,8 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     for (int i = 0; i < C::kBInstr; ++i) one(b_base, boff[i], (i * 4 + wave) * 8 + (lane >> 3), st + BM * kSmallKB + i * 4096);
   };
 
+  unsigned char* c_base = p.C;
+
   float4v acc[C::kTN][C::kTM];
   // operand reads: row x of block i, the chunks of a step (of 16-bit types; e4m3: chunks g and g + 4, the four groups of a read on
   // consecutive chunks, and the order of gemm.hip's sums) and lane group g, relative to the stage; blocks are 16 rows apart, which
@@ -206,6 +224,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 #pragma unroll
       for (int i = 0; i < C::kTM; ++i) acc[j][i] = float4v{0.f, 0.f, 0.f, 0.f};
     const int n_kt = kt1 - kt0;
+    if constexpr (kScatter) c_base = (unsigned char*)p.scatter_bufs[owner];   // (asked for here: its trip to memory is over long before the epilogue)
 #pragma unroll
     for (int i = 0; i < NST - 1; ++i) {
       if (i >= n_kt) break;
@@ -377,21 +396,89 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 #pragma unroll
     for (int i = 0; i < C::kTM; ++i) rs[i] = p.row_scale ? p.row_scale[min(m0 + wm * (BM / 2) + i * 16 + x, p.M - 1)] : 1.f;
   }
+  auto stage_tile = [&] {
 #pragma unroll
-  for (int i = 0; i < C::kTM; ++i) {
-    const int row = wm * (BM / 2) + i * 16 + x;
+    for (int i = 0; i < C::kTM; ++i) {
+      const int row = wm * (BM / 2) + i * 16 + x;
 #pragma unroll
-    for (int j = 0; j < C::kTN; ++j) {
-      const int col = wn * (BN / 2) + j * 16 + 4 * g;
-      float4v v = acc[j][i];
-      if constexpr (kScales) {
+      for (int j = 0; j < C::kTN; ++j) {
+        const int col = wn * (BN / 2) + j * 16 + 4 * g;
+        float4v v = acc[j][i];
+        if constexpr (kScales) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= rs[i] * cs[j][e];
+          for (int e = 0; e < 4; ++e) v[e] *= rs[i] * cs[j][e];
+        }
+        *(TDIST_AS3 int2v*)(ring + row * C::kEpiPitch + col * 2) = int2v{(int)E::pack(v[0], v[1]), (int)E::pack(v[2], v[3])};
       }
-      *(TDIST_AS3 int2v*)(ring + row * C::kEpiPitch + col * 2) = int2v{(int)E::pack(v[0], v[1]), (int)E::pack(v[2], v[3])};
+    }
+    __syncthreads();
+  };
+  if constexpr (kScatter) {
+    if (adds) {
+      // The sum over the ranks: the others' rows, four pieces of every slice in flight at a time, in the order rank + 1, rank + 2, ..., and
+      // the own ones last, as they are stored: the order and the bits of reduce.hip. No load is conditional (the compiler would wait for
+      // some of them in front of others): slices beyond the last are the last one again.
+      auto add_up = [&](auto slices_c) {
+        constexpr int kSlices = decltype(slices_c)::value, kBatch = 4;
+        static_assert(kStores % kBatch == 0, "whole batches");
+        int4v v[kSlices][kBatch];
+        auto ask = [&](auto u0_c) {
+#pragma unroll
+          for (int w = 0; w < kSlices; ++w) {
+            const int i = min(1 + w, p.world - 1), s = p.rank + i < p.world ? p.rank + i : p.rank + i - p.world;
+            const unsigned char* const src = p.own + ((int64_t)((s - p.rank) * p.m_per_rank + m0) * p.ldc + n0) * 2;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+              const int idx = (decltype(u0_c)::value + u) * 256 + threadIdx.x, row = idx / kPieces, col = min(idx % kPieces * 8, p.N - 8 - n0);
+              v[w][u] = *(const TDIST_AS1 int4v*)(src + ((int64_t)row * p.ldc + col) * 2);
+            }
+          }
+        };
+        ask(std::integral_constant<int, 0>{});
+        stage_tile();
+        static_for<kStores / kBatch>([&](auto b_c) {
+          constexpr int u0 = decltype(b_c)::value * kBatch;
+          float sum[kBatch][8];
+#pragma unroll
+          for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[u][e] = 0.f;
+          auto add = [&](int u, const int4v& x) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              sum[u][2 * e] += E::store::lo((uint32_t)x[e]);
+              sum[u][2 * e + 1] += E::store::hi((uint32_t)x[e]);
+            }
+          };
+#pragma unroll
+          for (int w = 0; w < kSlices; ++w) {
+            if (1 + w >= p.world) break;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) add(u, v[w][u]);
+          }
+          if constexpr (u0 + kBatch < kStores) ask(std::integral_constant<int, u0 + kBatch>{});
+#pragma unroll
+          for (int u = 0; u < kBatch; ++u) {
+            const int idx = (u0 + u) * 256 + threadIdx.x, row = idx / kPieces, col = idx % kPieces * 8;
+            if (n0 + col >= p.N) continue;
+            const int4v own = *(const TDIST_AS3 int4v*)(ring + row * C::kEpiPitch + col * 2);
+            *(int4v*)(c_base + ((int64_t)(m0 + row) * p.ldc + n0 + col) * 2) = own;
+            add(u, own);
+            int4v o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (int)E::store::pack(sum[u][2 * e], sum[u][2 * e + 1]);
+            *(int4v*)(p.out + ((int64_t)(m0 - p.rank * p.m_per_rank + row) * p.N + n0 + col) * 2) = o;
+          }
+        });
+      };
+      constexpr int kMost = kSmallSumRows / BM;   // other ranks
+      if (p.world <= 2) add_up(std::integral_constant<int, 1>{});
+      else if (kMost <= 3 || p.world <= 4) add_up(std::integral_constant<int, 3>{});
+      else if constexpr (kMost > 3) add_up(std::integral_constant<int, kMost>{});
+      return;
     }
   }
-  __syncthreads();
+  stage_tile();
   if constexpr (kGrouped) {
     const bool vec = (p.ldc % 8) == 0 && ((uintptr_t)p.C & 15) == 0;
 #pragma unroll
@@ -410,13 +497,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
     }
     return;
   }
-  unsigned char* c_base = p.C;
-  int row_shift = 0;
-  if (p.scatter_bufs) {
-    const int owner = m0 / p.m_per_rank;
-    c_base = (unsigned char*)p.scatter_bufs[owner];
-    row_shift = (p.rank - owner) * p.m_per_rank;
-  }
+  const int row_shift = kScatter ? (p.rank - owner) * p.m_per_rank : 0;
   const bool vec = (p.ldc % 8) == 0 && ((uintptr_t)c_base & 15) == 0;
   for (int idx = threadIdx.x; idx < BM * kPieces; idx += 256) {
     const int row = idx / kPieces, col = idx % kPieces * 8;
@@ -467,6 +548,7 @@ template <typename E, int BM, int BN, int NST, bool kScales>
 static int launch_cfg(const SmallGemmParams& p, hipStream_t stream, const char* who) {
   if constexpr (!kScales)
     if (p.sorted_ids) return launch_rows<E, BM, BN, NST, kScales, kRowsGrouped>(p, stream, who);
+  if (p.scatter_bufs) return launch_rows<E, BM, BN, NST, kScales, kRowsScatter>(p, stream, who);
   return p.shards.rows != 0 ? launch_rows<E, BM, BN, NST, kScales, kRowsShards>(p, stream, who) : launch_rows<E, BM, BN, NST, kScales, kRowsPlain>(p, stream, who);
 }
 

@@ -283,19 +283,10 @@ PyObject* gemm_rs(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
   TDIST_ORDINARY(optional_of(o[7], device, c10::ScalarType::Float, &row_scale) && optional_of(o[8], device, c10::ScalarType::Float, &col_scale));
   TDIST_ORDINARY(code == TDIST_F8E4M3 || (!row_scale && !col_scale));
   void* const stream = stream_of(device);
-  void* const* const bufs = (void* const*)addresses->data_ptr();
-  const auto scatter = code == TDIST_F16 ? tdist_gemm_rs_scatter_f16 : tdist_gemm_rs_scatter_bf16;
   at::Tensor out = empty_on(device, out_type, {M / ranks, N});
   if (!run([&] {
-        const int rc = code == TDIST_F8E4M3 ? tdist_gemm_rs_scatter_fp8e4m3(a->data_ptr(), K, b->data_ptr(), b->stride(0), bufs, N, (int)M, (int)N, (int)K,
-                                                                           (const float*)ptr(row_scale), (const float*)ptr(col_scale), rank, ranks, sk,
-                                                                           sk_bytes, stream)
-                                           : scatter(a->data_ptr(), K, b->data_ptr(), b->stride(0), bufs, N, (int)M, (int)N, (int)K, rank, ranks, sk,
-                                                     sk_bytes, stream);
-        if (rc != TDIST_OK) return rc;
-        const int64_t slice = M / ranks * N;
-        return tdist_reduce_slices(own->data_ptr(), slice, ranks, (rank + 1) % ranks, slice, out.data_ptr(),
-                                   out_type == c10::ScalarType::Half ? TDIST_F16 : TDIST_BF16, stream);
+        return tdist_gemm_rs(code, a->data_ptr(), K, b->data_ptr(), b->stride(0), (void* const*)addresses->data_ptr(), own->data_ptr(), out.data_ptr(),
+                             (int)M, (int)N, (int)K, (const float*)ptr(row_scale), (const float*)ptr(col_scale), rank, ranks, sk, sk_bytes, stream);
       })) return nullptr;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
