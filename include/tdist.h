@@ -446,6 +446,16 @@ int tdist_moe_join_blocks(const int32_t* sorted_token_ids, const int32_t* expert
                           const int32_t* num_tokens_post_padded, int num_blocks, int block_size, int num_valid_tokens,
                           int num_experts, int out_block, int32_t* out_sorted_ids, int64_t out_rows,
                           int32_t* out_expert_ids, int32_t* out_segment_ids, int32_t* out_post_padded, void* stream);
+/* The same with a second list for a GEMM of `columns` output columns in tiles of out_block x 256: an expert's last rows, where they are at
+ * most tail_most (below out_block), go into blocks of tail_block rows there (ids, an expert and a segment 0 to a block, the padded total;
+ * tail_rows: room for that many ids) instead of a block that they would fill in part; both blocks are powers of two. Decided on the device,
+ * from what the blocks hold: where that takes a round of tiles away and there is room for all, else every row is in the first list and
+ * tail_padded[0] = 0. */
+int tdist_moe_join_blocks_tails(const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_padded,
+                                int num_blocks, int block_size, int num_valid_tokens, int num_experts, int out_block,
+                                int32_t* out_sorted_ids, int64_t out_rows, int32_t* out_expert_ids, int32_t* out_segment_ids,
+                                int32_t* out_post_padded, int tail_most, int tail_block, int columns, int32_t* tail_ids, int64_t tail_rows,
+                                int32_t* tail_experts, int32_t* tail_segments, int32_t* tail_padded, void* stream);
 /* tdist_gather_shards and tdist_moe_join_blocks in one launch: what a grouped GEMM needs whose rows are all at hand. */
 int tdist_moe_gather_and_join(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes,
                               int32_t* status, int32_t* first_error, const int32_t* sorted_token_ids,
@@ -510,6 +520,16 @@ int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, 
                           const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,
                           int num_blocks, int block_size, int num_valid_tokens, int topk, int32_t* status,
                           int32_t* first_error, void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
+/* Rows of an expert's tail that are worth a block of 64 rows of their own (tdist_moe_join_blocks_tails) beside blocks of `block` rows, by an
+ * estimate for rows evenly at random over the experts; 0: none. */
+int tdist_group_gemm_tail_rows(int64_t rows, int num_experts, int N, int64_t k_bytes, int block);
+/* tdist_group_gemm_rows over both lists of tdist_moe_join_blocks_tails, the second in tail_blocks blocks of 64 rows at most: two launches. */
+int tdist_group_gemm_rows_tails(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+                                int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids,
+                                const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,
+                                int num_blocks, int block_size, int num_valid_tokens, int topk, const int32_t* tail_ids,
+                                const int32_t* tail_experts, const int32_t* tail_segments, const int32_t* tail_padded, int tail_blocks,
+                                int32_t* status, int32_t* first_error, void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Workspace of the GEMM entry points above (tdist_gemm_chunk_gated_*, tdist_gemm_rs_scatter_*,

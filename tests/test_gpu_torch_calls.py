@@ -57,7 +57,7 @@ def same(a, b):
 
 def test_nothing_is_taken_without_a_gpu():
     module, cpu = _lib.native(), torch.zeros(4, 4)
-    counts = dict(decode=7, decode_ranks=14, ag_gemm=11, gemm_rs=9, ag_group_gemm=20, reduce_rs=19, preprocess=3, dispatch_ids=4, dispatch_quant=4,
+    counts = dict(decode=7, decode_ranks=14, ag_gemm=11, gemm_rs=9, ag_group_gemm=23, reduce_rs=22, preprocess=3, dispatch_ids=4, dispatch_quant=4,
                   combine=6, align=9)
     for name in NAMES:
         fn = getattr(module, name)

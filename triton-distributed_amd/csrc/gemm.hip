@@ -2414,6 +2414,7 @@ struct GroupGemmCall {
   const char* who;
   ShardRows shards;   // rows != 0: A's rows lie in shards (calls without flags only)
   bool few_rows;      // blocks of kGroupedFewRows rows are taken as well (calls without flags or a local shard)
+  int tails_of = 0;   // != 0: the blocks hold the last rows of some of this many experts
 };
 
 // ---- estimates for the grouped GEMM, in microseconds -------------------------------------------------------------
@@ -2470,6 +2471,25 @@ static double group_large_us(const GroupShape& g, int block, bool split_last, in
   const int s = split_last && tail != 0 && k_tiles >= 2 * kSkMinPiece ? sk_split_for(cus, (int)tail, k_tiles) : 1;
   if (s > 1) us = full * (k_tiles * k_tile + beside) + k_tiles * k_tile / s + 24.0;
   return 11.0 + std::max(us, group_panels_us(g, (double)tiles * k_tiles * (block + 256) * 128, 13.0e6));
+}
+
+// Rows that an expert's last block may have to go into blocks of 64 rows of a launch of their own, where that is likely to take a round of
+// tiles from the others: half a block, which is two short ones. (What the routing is, and so whether it is done, is known on the device
+// only: moe_join_blocks_kernel.) A last round, whole or cut along K, takes 30 us and more, the other launch 10 to 20, and 2 with nothing to
+// do: 8192 tokens, top 2 of 8 experts, 1792 deep by 4096 columns: a layer 492 -> 472 us, and
+// 457 -> 460 where every expert has exactly eight blocks and the other launch finds nothing.
+static int group_tail_rows(const GroupShape& g, int block, int cus) {
+  const double used = std::max(1.0, groups_in_use(g)), mean = g.rows / used, dev = std::max(0.3, std::sqrt(mean));
+  const int most = block / 2;
+  if (mean < block) return 0;
+  double share = 0;   // of the experts whose last rows are that few
+  if (dev > block) share = 0.5;
+  else
+    for (int k = (int)std::max(0.0, (mean - 4 * dev) / block); k * block < mean + 4 * dev; ++k)
+      share += 0.5 * (std::erfc((k * block + 0.5 - mean) / dev * 0.70710678) - std::erfc((k * block + most + 0.5 - mean) / dev * 0.70710678));
+  const int64_t cols = ceil_div(g.N, 256), blocks = group_blocks(g, block), whole = blocks - (int64_t)(used * share + 0.5);
+  // (short blocks: one or two to an expert, one tile of 128 columns to a compute unit)
+  return ceil_div(whole * cols, cus) < ceil_div(blocks * cols, cus) && 1.5 * used * share * ceil_div(g.N, 128) <= cus ? most : 0;
 }
 
 // The small tiles' plan for a call whose blocks have a small tile's rows (us = 0: it does not qualify).
@@ -2545,7 +2565,11 @@ static int run_group_gemm(const GroupGemmCall& c, GemmElem elem) {
   const DeviceInfo& di = device_info();
   if (di.ok != 1) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
   // (experts: what the number of blocks leaves room for, every one pads block_size - 1 rows at most)
-  const GroupShape shape = {c.num_valid, (double)(((int64_t)c.num_blocks * c.block_size - c.num_valid) / (c.block_size - 1) + 1), c.N, (int64_t)c.K * esz};
+  // (tails: half of the experts with half of what a block of the others may leave)
+  const double tails = std::max(1.0, 0.5 * c.tails_of);
+  const GroupShape shape = c.tails_of ? GroupShape{(int64_t)(tails * kGroupedFewRows), tails, c.N, (int64_t)c.K * esz}
+                                      : GroupShape{c.num_valid, (double)(((int64_t)c.num_blocks * c.block_size - c.num_valid) / (c.block_size - 1) + 1),
+                                                   c.N, (int64_t)c.K * esz};
   const SmallPlan small = group_small_plan(c, shape, esz, di.num_cus);
   const int forced_tile = debug_get(TDIST_DEBUG_GEMM_TILE);
   if (few && small.us == 0)
@@ -2848,12 +2872,11 @@ int tdist_group_gemm_row_block(int64_t rows, int num_experts, int N, int64_t k_b
   return best;
 }
 
-int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+static int group_gemm_rows(const char* who, int tails_of, int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
                           int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                           const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded, int num_blocks, int block_size,
                           int num_valid_tokens, int topk, int32_t* status, int32_t* first_error, void* sk_workspace,
                           int64_t sk_workspace_bytes, void* stream) {
-  const char* who = "tdist_group_gemm_rows";
   GemmElem elem;
   if (int rc = elem_of(dtype, elem, who)) return rc;
   if (rows_per_rank <= 0 || K <= 0 || (int64_t)world_size * rows_per_rank > 0x7fffffff) return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
@@ -2872,7 +2895,40 @@ int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, 
   c.block_segment = block_barrier_ids; c.post_pad = num_tokens_post_padded; c.num_blocks = num_blocks; c.block_size = block_size;
   c.num_valid = num_valid_tokens; c.topk = topk; c.tokens_per_rank = c.a_rows; c.few_rows = true;
   c.sk_workspace = sk_workspace; c.sk_workspace_bytes = sk_workspace_bytes; c.stream = (hipStream_t)stream; c.who = who;
+  c.tails_of = tails_of;
   return run_group_gemm(c, elem);
+}
+
+int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+                          int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded, int num_blocks, int block_size,
+                          int num_valid_tokens, int topk, int32_t* status, int32_t* first_error, void* sk_workspace,
+                          int64_t sk_workspace_bytes, void* stream) {
+  return group_gemm_rows("tdist_group_gemm_rows", 0, dtype, shards, world_size, rows_per_rank, B, ldb, expert_stride, C, ldc, N, K, sorted_token_ids,
+                         expert_ids, block_barrier_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, topk, status, first_error,
+                         sk_workspace, sk_workspace_bytes, stream);
+}
+
+int tdist_group_gemm_tail_rows(int64_t rows, int num_experts, int N, int64_t k_bytes, int block) {
+  const DeviceInfo& di = device_info();
+  if (di.ok != 1 || rows <= 0 || num_experts <= 0 || N <= 0 || k_bytes <= 0 || block != 256) return 0;
+  return group_tail_rows({rows, (double)num_experts, N, k_bytes}, block, di.num_cus);
+}
+
+int tdist_group_gemm_rows_tails(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
+                          int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded, int num_blocks, int block_size,
+                          int num_valid_tokens, int topk, const int32_t* tail_ids, const int32_t* tail_experts, const int32_t* tail_segments,
+                                const int32_t* tail_padded, int tail_blocks, int32_t* status, int32_t* first_error, void* sk_workspace,
+                                int64_t sk_workspace_bytes, void* stream) {
+  const char* who = "tdist_group_gemm_rows_tails";
+  if (int rc = group_gemm_rows(who, 0, dtype, shards, world_size, rows_per_rank, B, ldb, expert_stride, C, ldc, N, K, sorted_token_ids, expert_ids,
+                               block_barrier_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, topk, status, first_error,
+                               sk_workspace, sk_workspace_bytes, stream)) return rc;
+  // (the launch before has retired the status)
+  return group_gemm_rows(who, std::max(1, tail_blocks / 2), dtype, shards, world_size, rows_per_rank, B, ldb, expert_stride, C, ldc, N, K,
+                         tail_ids, tail_experts, tail_segments, tail_padded, tail_blocks, kGroupedFewRows, num_valid_tokens, topk, nullptr, nullptr,
+                         sk_workspace, sk_workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -522,6 +522,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const SmallGemmParam
 // 16384 over 8, 4096 x 1792: 372 -> 296, with two rows 328). 90 calls of each kind: 4 and 3.5 % faster on average, 1 % behind the best of 1 to 32.
 static int64_t walk_rows(const SmallGemmParams& p, int bm) {
   if (!p.sorted_ids) return 8;
+  if ((int64_t)p.num_blocks * bm < p.num_valid) return 2;   // (experts' last rows: one block of each, or two)
   // (experts: what the number of blocks leaves room for, every one pads bm - 1 rows at most)
   const int64_t experts = ((int64_t)p.num_blocks * bm - p.num_valid) / (bm - 1) + 1, blocks = (p.num_valid / std::max<int64_t>(experts, 1) + bm / 2) / bm;
   return blocks >= 16 ? 8 : blocks >= 8 ? 4 : blocks >= 4 ? 2 : 1;

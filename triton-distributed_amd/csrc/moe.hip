@@ -1629,6 +1629,11 @@ struct JoinParams {
   const int32_t *sorted_ids, *expert_ids, *post_pad;
   int num_blocks, block_size, num_valid, E, out_block, out_rows;
   int32_t *out_ids, *out_experts, *out_segments, *out_padded;
+  // tail_most != 0: an expert's last rows, where they are at most that many, go into blocks of tail_block rows of a list of their own instead
+  // of a block of `out_block` that they would fill in part (both powers of two). Done where it takes a round away from a GEMM of `cols`
+  // tiles to a block on `cus` compute units and the list has room for all of them; else it is empty.
+  int tail_most, tail_block, cols, cus, tail_rows;
+  int32_t *tail_ids, *tail_experts, *tail_segments, *tail_padded;
 };
 // Workgroup `block` of `blocks`. kChunks: 64 rows each to a block; 0: any number.
 template <int kThreads, int kChunks>
@@ -1644,7 +1649,8 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
   int32_t* const s_total = s_mem;           // [E] entries per expert
   int32_t* const s_start = s_mem + E;       // [E] its first row
   int32_t* const s_block = s_mem + 2 * E;   // [num_blocks] expert and number of entries of each block
-  __shared__ int32_t s_part[kWaves];
+  int32_t* const s_tail = s_block + num_blocks;   // [E] with tails: the first row of the expert's last rows
+  __shared__ int32_t s_part[3][kWaves];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int chunks = kChunks > 0 ? kChunks : (block_size + 63) / 64;
   const int gwave = block * kWaves + wave, waves = blocks * kWaves;
@@ -1696,25 +1702,60 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
   // exclusive prefix of the experts' padded sizes: a thread takes `per` neighbours
   const int per = (E + kThreads - 1) / kThreads;
   auto padded = [&](int n) { return (n + out_block - 1) / out_block * out_block; };
-  int own = 0;
+  auto tail_padded = [&](int n) { return (n + p.tail_block - 1) & -p.tail_block; };
+  bool tails = p.tail_most > 0;
+  auto tail_of = [&](int total) {   // (rows of an expert in the list of tails)
+    const int rest = total & (out_block - 1);
+    return tails && rest <= p.tail_most ? rest : 0;
+  };
+  int own = 0, own_whole = 0, own_tail = 0;
   for (int i = 0; i < per; ++i) {
     const int e = threadIdx.x * per + i;
-    if (e < E) own += padded(s_total[e]);
+    if (e < E) {
+      const int total = s_total[e];
+      own += padded(total);
+      if (tails) own_whole += padded(total - tail_of(total)), own_tail += tail_padded(tail_of(total));
+    }
   }
   const int sum = wave_scan_add(own);
-  if (lane == 63) s_part[wave] = sum;
+  if (lane == 63) s_part[0][wave] = sum;
+  int sum_whole = 0, sum_tail = 0;
+  if (tails) {
+    sum_whole = wave_scan_add(own_whole);
+    sum_tail = wave_scan_add(own_tail);
+    if (lane == 63) s_part[1][wave] = sum_whole, s_part[2][wave] = sum_tail;
+  }
   __syncthreads();
-  int at = sum - own, all = 0;
+  int at = sum - own, all = 0, at_tail = 0, all_tail = 0;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
-    if (w < wave) at += s_part[w];
-    all += s_part[w];
+    if (w < wave) at += s_part[0][w];
+    all += s_part[0][w];
+  }
+  if (tails) {
+    int at_whole = sum_whole - own_whole, all_whole = 0;
+    at_tail = sum_tail - own_tail;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < wave) at_whole += s_part[1][w], at_tail += s_part[2][w];
+      all_whole += s_part[1][w];
+      all_tail += s_part[2][w];
+    }
+    auto rounds = [&](int rows) { return ((uint32_t)rows / (uint32_t)out_block * (uint32_t)p.cols + (uint32_t)p.cus - 1) / (uint32_t)p.cus; };
+    tails = all_tail <= p.tail_rows && rounds(all_whole) < rounds(all);
+    if (tails) at = at_whole, all = all_whole;
+    if (block == 0 && threadIdx.x == 0) p.tail_padded[0] = tails ? all_tail : 0;
   }
   for (int i = 0; i < per; ++i) {
     const int e = threadIdx.x * per + i;
     if (e < E) {
+      const int total = s_total[e], tail = tail_of(total);
       s_start[e] = at;
-      at += padded(s_total[e]);
+      at += padded(total - tail);
+      if (tails) {
+        s_tail[e] = at_tail;
+        at_tail += tail_padded(tail);
+      }
     }
   }
   if (block == 0 && threadIdx.x == 0) p.out_padded[0] = min(all, out_rows / out_block * out_block);
@@ -1727,11 +1768,18 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
       before += v >> kJoinCountBits == e ? v & kCountMask : 0;
     }
     before = wave_sum(before);
-    int row = s_start[e] + before;
+    const int start = s_start[e], total = s_total[e], whole = total - tail_of(total), tail_start = tails ? s_tail[e] : 0;
+    int row = before;   // of the expert's
     auto place = [&](int id) {
       const unsigned long long is = __ballot(valid(id));
-      const int to = row + __popcll(is & ((1ull << lane) - 1));
-      if (valid(id) && to < out_rows) out_ids[to] = id;
+      const int of = row + __popcll(is & ((1ull << lane) - 1));
+      if (valid(id)) {
+        if (of < whole) {
+          if (start + of < out_rows) out_ids[start + of] = id;
+        } else if (tails) {
+          p.tail_ids[tail_start + of - whole] = id;   // (all of them fit, or there are no tails)
+        }
+      }
       row += __popcll(is);
     };
     if (kChunks > 0 && b == gwave) {
@@ -1742,7 +1790,15 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
     }
   }
   for (int e = gwave; e < E; e += waves) {
-    const int total = s_total[e], lo = s_start[e], hi = min(lo + padded(total), out_rows);
+    const int all_rows = s_total[e], tail = tail_of(all_rows), total = all_rows - tail, lo = s_start[e], hi = min(lo + padded(total), out_rows);
+    if (tail > 0) {
+      const int first = s_tail[e], end = first + tail_padded(tail);
+      for (int r = first + tail + lane; r < end; r += 64) p.tail_ids[r] = num_valid;
+      for (int b = first / p.tail_block + lane; b < end / p.tail_block; b += 64) {
+        p.tail_experts[b] = e;
+        p.tail_segments[b] = 0;
+      }
+    }
     for (int r = lo + total + lane; r < hi; r += 64) out_ids[r] = num_valid;
     for (int b = lo / out_block + lane; b < hi / out_block; b += 64) {
       p.out_experts[b] = e;
@@ -2149,7 +2205,7 @@ static int join_launch(JoinLaunch& j, const char* who, TDIST_JOIN_ARGS) {
   if (block_size > kJoinMaxBlock || num_experts > kMoeMaxExperts || j.lds > kJoinLdsLimit || out_rows > 0x7fffffffll)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: %d blocks of %d rows, %d experts", who, num_blocks, block_size, num_experts);
   j.p = {sorted_token_ids, expert_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, num_experts, out_block,
-         (int)out_rows, out_sorted_ids, out_expert_ids, out_segment_ids, out_post_padded};
+         (int)out_rows, out_sorted_ids, out_expert_ids, out_segment_ids, out_post_padded, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr};
   j.threads = num_blocks <= kJoinFewBlocks ? 256 : 1024;
   const int64_t items = ceil_div(num_blocks > num_experts ? num_blocks : num_experts, j.threads / 64);
   j.grid = (int)(items < 32 ? items : 32);
@@ -2172,6 +2228,28 @@ int tdist_moe_join_blocks(TDIST_JOIN_ARGS, void* stream) {
   const char* who = "tdist_moe_join_blocks";
   JoinLaunch j;
   if (int rc = join_launch(j, who, TDIST_JOIN_NAMES)) return rc;
+  TDIST_JOIN_PICK(moe_join_blocks_kernel)
+  hipLaunchKernelGGL(kern, dim3((unsigned)j.grid), dim3(j.threads), (size_t)j.lds, (hipStream_t)stream, j.p);
+  return launch_status(who);
+}
+
+int tdist_moe_join_blocks_tails(TDIST_JOIN_ARGS, int tail_most, int tail_block, int columns, int32_t* tail_ids, int64_t tail_rows,
+                                int32_t* tail_experts, int32_t* tail_segments, int32_t* tail_padded, void* stream) {
+  const char* who = "tdist_moe_join_blocks_tails";
+  JoinLaunch j;
+  if (int rc = join_launch(j, who, TDIST_JOIN_NAMES)) return rc;
+  if (!tail_ids || !tail_experts || !tail_segments || !tail_padded) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (tail_most <= 0 || tail_most >= out_block || tail_block <= 0 || columns <= 0 || tail_rows < tail_block || tail_rows > 0x7fffffffll)
+    return fail(TDIST_ERR_INVALID, "%s: tails of %d rows in blocks of %d, %d columns", who, tail_most, tail_block, columns);
+  if ((out_block & (out_block - 1)) != 0 || (tail_block & (tail_block - 1)) != 0)
+    return fail(TDIST_ERR_INVALID, "%s: blocks of %d and %d rows (powers of two)", who, out_block, tail_block);
+  j.lds += 4ll * num_experts;
+  if (j.lds > kJoinLdsLimit || out_rows / out_block * ceil_div(columns, 256) > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: %d blocks, %d experts", who, num_blocks, num_experts);
+  const DeviceInfo& di = device_info();
+  if (di.ok != 1) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
+  j.p.tail_most = tail_most, j.p.tail_block = tail_block, j.p.cus = di.num_cus, j.p.tail_rows = (int)tail_rows;
+  j.p.cols = (int)ceil_div(columns, 256);
+  j.p.tail_ids = tail_ids, j.p.tail_experts = tail_experts, j.p.tail_segments = tail_segments, j.p.tail_padded = tail_padded;
   TDIST_JOIN_PICK(moe_join_blocks_kernel)
   hipLaunchKernelGGL(kern, dim3((unsigned)j.grid), dim3(j.threads), (size_t)j.lds, (hipStream_t)stream, j.p);
   return launch_status(who);

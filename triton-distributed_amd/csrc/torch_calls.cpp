@@ -299,8 +299,11 @@ struct Blocks {
   int block_size, entries;
   int64_t at[4];   // addresses: sorted ids, experts, segments, padded total
   int count, rows;
+  int tail_most, tail_count;   // experts' last rows in blocks of their own, of kTailBlock rows, one array behind the other from tail_ids on
+  int32_t *tail_ids, *tail_experts, *tail_segments, *tail_padded;
 };
-// o[0..4]: sorted ids, experts and padded total of the align / sort, its block size, entries; o[5..10]: a RowBlocks, field by field
+constexpr int kTailBlock = 64;
+// o[0..4]: sorted ids, experts and padded total of the align / sort, its block size, entries; o[5..13]: a RowBlocks, field by field
 bool blocks_of(PyObject* const* o, int device, Blocks& b) {
   b.sorted = tensor_of(o[0], device, c10::ScalarType::Int, 1), b.experts = tensor_of(o[1], device, c10::ScalarType::Int, 1);
   b.padded = tensor_of(o[2], device, c10::ScalarType::Int, 1);
@@ -308,6 +311,14 @@ bool blocks_of(PyObject* const* o, int device, Blocks& b) {
   if (!int_of(o[3], &b.block_size) || b.block_size <= 0 || !int_of(o[4], &b.entries) || !int_of(o[9], &b.count) || !int_of(o[10], &b.rows)) return false;
   for (int i = 0; i < 4; ++i)
     if (!PyLong_CheckExact(o[5 + i]) || (b.at[i] = PyLong_AsLongLong(o[5 + i])) <= 0) return PyErr_Clear(), false;
+  int64_t tail;
+  if (!int_of(o[11], &b.tail_most) || !int_of(o[13], &b.tail_count) || b.tail_most < 0 || b.tail_count < 0 || !PyLong_CheckExact(o[12]) ||
+      (tail = PyLong_AsLongLong(o[12])) < 0) return PyErr_Clear(), false;
+  b.tail_ids = (int32_t*)tail;
+  if ((b.tail_most > 0) != (tail != 0 && b.tail_count > 0)) return false;
+  b.tail_experts = b.tail_ids + (int64_t)b.tail_count * kTailBlock;
+  b.tail_segments = b.tail_experts + b.tail_count;
+  b.tail_padded = b.tail_segments + b.tail_count;
   return true;
 }
 // weights [E, K, N] whose rows are contiguous along K, for rows of `k` elements of this type
@@ -320,21 +331,30 @@ const at::Tensor* weights_of(PyObject* o, int device, const at::Tensor& a, int64
 }
 int join_and_multiply(const Blocks& k, int code, const void* const* shards, int ranks, int64_t rows, const at::Tensor& a, const at::Tensor& b, void* c, int topk,
                       int32_t* status, void* sk, int64_t sk_bytes, void* stream, bool* joined) {
-  int rc = tdist_moe_join_blocks(i32(k.sorted), i32(k.experts), i32(k.padded), (int)std::min(k.experts->numel(), k.sorted->numel() / k.block_size),
-                                 k.block_size, k.entries, (int)b.size(0), k.rows, (int32_t*)k.at[0], (int64_t)k.count * k.rows, (int32_t*)k.at[1],
-                                 (int32_t*)k.at[2], (int32_t*)k.at[3], stream);
+  const int blocks = (int)std::min(k.experts->numel(), k.sorted->numel() / k.block_size), N = (int)b.size(2);
+  int32_t *const ids = (int32_t*)k.at[0], *const experts = (int32_t*)k.at[1], *const segments = (int32_t*)k.at[2], *const padded = (int32_t*)k.at[3];
+  const int64_t room = (int64_t)k.count * k.rows;
+  int rc = k.tail_most > 0
+               ? tdist_moe_join_blocks_tails(i32(k.sorted), i32(k.experts), i32(k.padded), blocks, k.block_size, k.entries, (int)b.size(0), k.rows, ids, room,
+                                             experts, segments, padded, k.tail_most, kTailBlock, N, k.tail_ids, (int64_t)k.tail_count * kTailBlock,
+                                             k.tail_experts, k.tail_segments, k.tail_padded, stream)
+               : tdist_moe_join_blocks(i32(k.sorted), i32(k.experts), i32(k.padded), blocks, k.block_size, k.entries, (int)b.size(0), k.rows, ids, room,
+                                       experts, segments, padded, stream);
   *joined = rc != TDIST_ERR_UNSUPPORTED;   // (nothing has been launched then)
   if (rc != TDIST_OK) return *joined ? rc : TDIST_OK;
-  const int N = (int)b.size(2);
-  return tdist_group_gemm_rows(code, shards, ranks, (int)rows, b.data_ptr(), b.stride(2), b.stride(0), c, N, N, (int)a.size(1), (int32_t*)k.at[0],
-                               (int32_t*)k.at[1], (int32_t*)k.at[2], (int32_t*)k.at[3], k.count, k.rows, k.entries, topk, status,
-                               status ? status + 2 : nullptr, sk, sk_bytes, stream);
+  int32_t* const first_error = status ? status + 2 : nullptr;
+  if (k.tail_most > 0)
+    return tdist_group_gemm_rows_tails(code, shards, ranks, (int)rows, b.data_ptr(), b.stride(2), b.stride(0), c, N, N, (int)a.size(1), ids, experts,
+                                       segments, padded, k.count, k.rows, k.entries, topk, k.tail_ids, k.tail_experts, k.tail_segments, k.tail_padded,
+                                       k.tail_count, status, first_error, sk, sk_bytes, stream);
+  return tdist_group_gemm_rows(code, shards, ranks, (int)rows, b.data_ptr(), b.stride(2), b.stride(0), c, N, N, (int)a.size(1), ids, experts, segments,
+                               padded, k.count, k.rows, k.entries, topk, status, first_error, sk, sk_bytes, stream);
 }
 
 // ag_group_gemm(a, b, peer_shards, rank, num_ranks, topk, workspace, status, sk_workspace, blocks...) -> c, where the rows can be read where
 // they lie
 PyObject* ag_group_gemm(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
-  TDIST_ARGS(20, 0);
+  TDIST_ARGS(23, 0);
   const at::Tensor* a = tensor_of(o[0], device);
   int code, rank, ranks, topk;
   TDIST_ORDINARY(a && a->dim() == 2 && a->is_contiguous() && a->numel() > 0 && code_of(a->scalar_type(), &code) && int_of(o[3], &rank) &&
@@ -366,7 +386,7 @@ PyObject* ag_group_gemm(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
 
 // reduce_rs(a, b, rank, world, weights, rows_buffer, rank_buffer, sk_workspace, blocks...) -> this rank's rows of the sum
 PyObject* reduce_rs(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
-  TDIST_ARGS(19, 0);
+  TDIST_ARGS(22, 0);
   const at::Tensor *a = tensor_of(o[0], device), *weight = tensor_of(o[4], device, c10::ScalarType::Float, 2);
   const at::Tensor *rows = tensor_of(o[5], device, c10::ScalarType::BFloat16, 2), *slab = tensor_of(o[6], device, c10::ScalarType::BFloat16, 2);
   int code, rank, world;

@@ -75,12 +75,15 @@ PROTOTYPES = {
     "tdist_moe_align_workspace_bytes": (_L, [_L, _I, _I]),
     "tdist_moe_align_block_size": (_I, [_P, _I, _L, _I, _I, _L, _I, _P, _L, _P, _P, _P, _P, _P, _L, _P]),
     "tdist_moe_join_blocks": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _P]),
+    "tdist_moe_join_blocks_tails": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _I, _I, _I, _P, _L, _P, _P, _P, _P]),
     "tdist_moe_gather_and_join": (_I, [_P, _P, _I, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _P]),
     "tdist_group_gemm_gated_bf16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_f16": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_gated_fp8e4m3": (_I, [_P, _L, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _P, _L, _P]),
     "tdist_group_gemm_row_block": (_I, [_L, _I, _I, _L, _L]),
     "tdist_group_gemm_rows": (_I, [_I, _P, _I, _I, _P, _L, _L, _P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _L, _P]),
+    "tdist_group_gemm_tail_rows": (_I, [_L, _I, _I, _L, _I]),
+    "tdist_group_gemm_rows_tails": (_I, [_I, _P, _I, _I, _P, _L, _L, _P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P, _L, _P]),
     "tdist_gemm_split_k_workspace_bytes": (_L, []),
     "tdist_decode_split_kv": (_I, [_P, _P, _P, _P, _P, _F, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I,
                                    _L, _L, _L, _L, _L, _L, _L, _L, _L, _I, _P]),

@@ -126,17 +126,29 @@ def _block_plan(entries, num_experts, n, row_bytes, sk_workspace):
     return (block, (entries + min(num_experts, entries) * (block - 1)) // block) if block > 0 else None
 
 
+_TAIL_BLOCK = 64   # rows of the blocks for experts' last rows
+
+
 class RowBlocks:
     """Addresses of a grouped GEMM's row blocks (sorted ids, an expert and a segment per block, the padded total), their
     number and their rows; ``memory``: the tensor they lie in."""
-    __slots__ = ("sorted_ids", "experts", "segments", "padded", "num_blocks", "block_size", "memory")
+    __slots__ = ("sorted_ids", "experts", "segments", "padded", "num_blocks", "block_size", "memory", "tail", "tail_most")
 
     def __init__(self, sorted_ids, experts, segments, padded, num_blocks, block_size, memory=None):
         self.sorted_ids, self.experts, self.segments, self.padded = sorted_ids, experts, segments, padded
         self.num_blocks, self.block_size, self.memory = num_blocks, block_size, memory
+        self.tail, self.tail_most = None, 0   # experts' last rows in RowBlocks of their own, and how many of them at most (0: none)
+
+    @classmethod
+    def of(cls, memory, at, num_blocks, block_size):
+        """Blocks in int32 ``memory`` from element ``at`` on."""
+        base, rows = memory.data_ptr() + 4 * at, num_blocks * block_size
+        return cls(base, base + 4 * rows, base + 4 * (rows + num_blocks), base + 4 * (rows + 2 * num_blocks), num_blocks, block_size, memory)
 
     def fields(self):
-        return self.sorted_ids, self.experts, self.segments, self.padded, self.num_blocks, self.block_size
+        t = self.tail
+        return (self.sorted_ids, self.experts, self.segments, self.padded, self.num_blocks, self.block_size, self.tail_most,
+                0 if t is None else t.sorted_ids, 0 if t is None else t.num_blocks)
 
 
 def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, block_size, entries, num_experts, n, row_bytes, stream, gather=None,
@@ -157,20 +169,31 @@ def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, bloc
         return None
     _lib.require_cuda(sorted_ids, expert_ids, num_tokens_post_padded)
     key = (entries, num_experts, n, any_block and row_bytes)
+    if gather is not None:
+        key += ("gather", )   # (that launch makes no tails)
     out = made.get(key)
     if out is None:
         plan = _block_plan(entries, num_experts, n, row_bytes, sk_workspace) if any_block else None
         block, n_blocks = plan or _join_plan(entries, num_experts, n)
-        rows = n_blocks * block
-        memory = torch.empty(rows + 2 * n_blocks + 1, dtype=torch.int32, device=sorted_ids.device)
-        base = memory.data_ptr()
-        out = made[key] = RowBlocks(base, base + 4 * rows, base + 4 * (rows + n_blocks), base + 4 * (rows + 2 * n_blocks), n_blocks, block,
-                                    memory)
+        tail_most = _lib.load().tdist_group_gemm_tail_rows(entries, num_experts, n, row_bytes, block) if any_block and gather is None else 0
+        # (as many as leave two of their tiles of 128 columns to a compute unit; and with fewer places the GEMM would take K apart for them)
+        tail_blocks = min(min(num_experts, entries) * (tail_most // _TAIL_BLOCK), 2 * _lib.load().tdist_num_cus() // -(-n // 128))
+        size = n_blocks * (block + 2) + 1
+        memory = torch.empty(size + (tail_blocks * (_TAIL_BLOCK + 2) + 1 if tail_most else 0), dtype=torch.int32, device=sorted_ids.device)
+        out = made[key] = RowBlocks.of(memory, 0, n_blocks, block)
+        if tail_most:
+            out.tail, out.tail_most = RowBlocks.of(memory, size, tail_blocks, _TAIL_BLOCK), tail_most
     args = (sorted_ids.data_ptr(), expert_ids.data_ptr(), num_tokens_post_padded.data_ptr(),
             min(expert_ids.numel(), sorted_ids.numel() // block_size), block_size, entries, num_experts, out.block_size, out.sorted_ids,
-            out.num_blocks * out.block_size, out.experts, out.segments, out.padded, stream)
-    lib = _lib.load()
-    rc = lib.tdist_moe_join_blocks(*args) if gather is None else lib.tdist_moe_gather_and_join(*gather, *args)
+            out.num_blocks * out.block_size, out.experts, out.segments, out.padded)
+    lib, tail = _lib.load(), out.tail
+    if gather is not None:
+        rc = lib.tdist_moe_gather_and_join(*gather, *args, stream)
+    elif tail is not None:
+        rc = lib.tdist_moe_join_blocks_tails(*args, out.tail_most, _TAIL_BLOCK, n, tail.sorted_ids, tail.num_blocks * _TAIL_BLOCK, tail.experts,
+                                             tail.segments, tail.padded, stream)
+    else:
+        rc = lib.tdist_moe_join_blocks(*args, stream)
     if rc == _lib.TDIST_ERR_UNSUPPORTED:
         return None
     _lib.check(rc)
@@ -227,10 +250,15 @@ def group_gemm_rows(dtype, shards, num_shards, rows_per_shard, b_nk, c, blocks, 
         raise ValueError("A, B ([E, N, K]) and C need a contiguous last dimension")
     _, N, K = b_nk.shape
     assert c.shape[1] == N
-    _lib.call("tdist_group_gemm_rows", _lib.dtype_code(dtype), shards, num_shards, rows_per_shard, b_nk.data_ptr(), b_nk.stride(1),
-              b_nk.stride(0), c.data_ptr(), c.stride(0), N, K, blocks.sorted_ids, blocks.experts, blocks.segments, blocks.padded,
-              blocks.num_blocks, blocks.block_size, int(num_valid_tokens), int(topk), status, None if status is None else status + 8,
-              *_lib.workspace_args(sk_workspace), stream)
+    args = (_lib.dtype_code(dtype), shards, num_shards, rows_per_shard, b_nk.data_ptr(), b_nk.stride(1), b_nk.stride(0), c.data_ptr(), c.stride(0),
+            N, K, blocks.sorted_ids, blocks.experts, blocks.segments, blocks.padded, blocks.num_blocks, blocks.block_size, int(num_valid_tokens),
+            int(topk))
+    rest = (status, None if status is None else status + 8, *_lib.workspace_args(sk_workspace), stream)
+    tail = blocks.tail
+    if tail is None:
+        _lib.call("tdist_group_gemm_rows", *args, *rest)
+    else:
+        _lib.call("tdist_group_gemm_rows_tails", *args, tail.sorted_ids, tail.experts, tail.segments, tail.padded, tail.num_blocks, *rest)
     return c
 
 
