@@ -43,12 +43,12 @@ MEASURED_TRAFFIC_BYTES = {
 }
 MEASURED_SOURCE_DIGEST = {
     "common.h": "f5b639d6f2c93627",
-    "decode.hip": "3ac771befeb01e03",
+    "decode.hip": "86e8879aaf685690",
     "gather.h": "3fd5e450cd06de4d",
-    "gemm.hip": "c08abbcdb78be098",
-    "gemm_small.h": "ef635860051b59ae",
-    "gemm_small.hip": "9f3cf4730167f9a0",
-    "moe.hip": "b232f7830cc66aab",
+    "gemm.hip": "72031edd6254e04a",
+    "gemm_small.h": "1368c14b33b545a8",
+    "gemm_small.hip": "87b09035e69e02ec",
+    "moe.hip": "5159f846f7e03e55",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")
