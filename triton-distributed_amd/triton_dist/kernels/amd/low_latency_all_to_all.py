@@ -339,7 +339,12 @@ def _fast_all_to_all_from_ids(ctx, send_tensor, send_scale, expert_ids):
         splits_i, cumsum, scatter, gather = moe_dispatch_preprocess(expert_ids, G, ctx=ctx)
         ctx.last_index = (splits_i, cumsum, scatter, gather)
         return fast_all_to_all(ctx, send_tensor, cumsum, send_scale, scatter_index=scatter)
-    _ensure_index_sets(ctx, T, topk, G, send_tensor.device)
+    if ctx.index_key != (T, topk, G, send_tensor.device):
+        # (a shape that the context sees for the first time: its tensors are made here, and the call goes where the later ones go)
+        _ensure_index_sets(ctx, T, topk, G, send_tensor.device)
+        out = _lib.native().dispatch_ids(ctx, send_tensor, send_scale, expert_ids)
+        if out is not None:
+            return out
     wide = expert_ids.dtype == torch.int64 and expert_ids.is_contiguous()   # (torch.topk's ids, read as they are)
     ids = expert_ids if wide else _staged_ids(ctx, expert_ids)
     which = ctx.index_calls % 2
