@@ -69,6 +69,25 @@ def test_random_inputs_and_the_routing(cuda):
     assert (out2.float().cpu() - ref2).abs().max() / ref2.abs().max() <= 2e-2
 
 
+def test_float16_inputs_are_refused(cuda):
+    """Their products are float16 and the context's buffers hold bf16: refused before anything is launched, also where the context has the
+    memory for a call of that size already."""
+    from triton_dist.kernels.amd.moe_reduce_rs import moe_reduce_rs
+    announce("moe reduce-rs: float16")
+    world, mpr, K, hidden, E, topk = 2, 24, 192, 264, 4, 2
+    g = torch.Generator().manual_seed(4)
+    logits = [torch.randn((mpr, E), generator=g) for _ in range(world)]
+    ctx = make_ctx(cuda, world, 0, mpr, hidden, E, topk, 128, logits, torch.float16)
+    a = torch.randn((world * mpr * topk, K), generator=g).bfloat16().to(cuda)
+    w = torch.randn((E, hidden, K), generator=g).bfloat16().to(cuda).transpose(1, 2)    # K contiguous
+    for _ in range(2):
+        ctx.final_output_buffer.zero_()
+        with pytest.raises(TypeError, match="float16"):
+            moe_reduce_rs(0, world, world, a.half(), w.transpose(1, 2).half().transpose(1, 2), ctx)
+        assert not ctx.final_output_buffer.any()
+        moe_reduce_rs(0, world, world, a, w, ctx)
+
+
 def test_argument_errors(cuda):
     from triton_dist.kernels.amd.moe_reduce_rs import create_moe_rs_context, select_experts
     logits = torch.randn((16, 4), device=cuda)

@@ -265,6 +265,11 @@ def test_moe_layer(cuda, route, dtype):
             out = []
             for _ in range(3):
                 h = ag_group_gemm_intra_node(shards[rank], up, ag)
+                if dtype == torch.float16:   # (the reduction is of bf16 rows)
+                    with pytest.raises(TypeError):
+                        moe_reduce_rs(rank, W, W, h, down, rs)
+                    out += [h]
+                    continue
                 out += [h, moe_reduce_rs(rank, W, W, h.to(dtype), down, rs), rs.rs_buffers[rank].clone(), rs.final_output_buffer.clone()]
             ag.check_status()
             return out
@@ -272,7 +277,8 @@ def test_moe_layer(cuda, route, dtype):
 
     a, b, taken = route(run())
     same(a, b)
-    assert taken == ["align"] * 2 + ["ag_group_gemm", "reduce_rs"] * 2   # (the contexts' own; the first calls make the memory of the row blocks)
+    second = ["ag_group_gemm"] if dtype == torch.float16 else ["ag_group_gemm", "reduce_rs"]
+    assert taken == ["align"] * 2 + second * 2   # (the contexts' own; the first calls make the memory of the row blocks)
     a, c, taken = route(run(up=up.contiguous(), down=down.contiguous()))   # weights that are transposed first
     same(a, c)
     same(a, b)

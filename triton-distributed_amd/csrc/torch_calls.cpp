@@ -390,8 +390,9 @@ PyObject* reduce_rs(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
   const at::Tensor *a = tensor_of(o[0], device), *weight = tensor_of(o[4], device, c10::ScalarType::Float, 2);
   const at::Tensor *rows = tensor_of(o[5], device, c10::ScalarType::BFloat16, 2), *slab = tensor_of(o[6], device, c10::ScalarType::BFloat16, 2);
   int code, rank, world;
-  TDIST_ORDINARY(a && a->dim() == 2 && a->is_contiguous() && a->numel() > 0 && aligned16(*a) && code_of(a->scalar_type(), &code) && int_of(o[2], &rank) &&
-                 int_of(o[3], &world) && world > 0 && weight && weight->is_contiguous());
+  // (the products of f16 rows are f16, and the buffers hold bf16)
+  TDIST_ORDINARY(a && a->dim() == 2 && a->is_contiguous() && a->numel() > 0 && aligned16(*a) && code_of(a->scalar_type(), &code) && code != TDIST_F16 &&
+                 int_of(o[2], &rank) && int_of(o[3], &world) && world > 0 && weight && weight->is_contiguous());
   const int64_t M = weight->size(0), topk = weight->size(1), row_bytes = a->size(1) * a->element_size();
   TDIST_ORDINARY(a->size(0) == M * topk && M >= world && row_bytes > 128);
   const at::Tensor* b = weights_of(o[1], device, *a, M * topk);

@@ -125,7 +125,7 @@ def _weight_nk(ctx, b):
 
 def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, debug_sync=False, do_initial_sync=True,
                   do_final_sync=True):
-    """a [M * topk, K_per_rank] intermediate states, row t*topk + k for token t's k-th expert; b [E, K_per_rank, hidden].
+    """a [M * topk, K_per_rank] intermediate states (bf16 or e4m3), row t*topk + k for token t's k-th expert; b [E, K_per_rank, hidden].
     Returns [M // world_size, hidden]: sum over k of weight[t,k] * (a[t*topk+k] @ b[expert]) for this rank's tokens,
     summed with the other ranks' partial results (reference :889-...; golden test/nvidia/test_moe_reduce_rs.py:103-133).
     The synchronisation arguments are accepted and unused: one stream runs the three steps in order."""
@@ -142,6 +142,8 @@ def moe_reduce_rs(rank, world_size, local_world_size, a, b, ctx, dump_ir=False, 
                 return result
     _lib.require_cuda(a, b)
     assert a.shape[0] == M * topk and a.dtype == b.dtype and a.shape[1] == b.shape[1]
+    if a.dtype == torch.float16:   # (its products are float16, which nothing behind them could tell from bf16)
+        raise TypeError("the context's buffers hold bf16 rows: bf16 or e4m3 inputs, not float16")
     hidden = b.shape[2]
     out = ctx.final_output_buffer[:M * topk, :hidden]
     # every sorted id names its own row of ``a`` (topk = 1 for the gather), no flag to wait for: the rows are local, and
