@@ -52,6 +52,42 @@ def test_producer_budget_guard():
         build._check_producer_resources(report(PRODUCER, 26, 0, 0))
 
 
+def test_an_interrupted_build_is_seen(tmp_path, monkeypatch):
+    """The extension module is built last: where that fails, no older one stays beside the new library, and the next build does not
+    take the outputs for whole. An output older than a source is seen whichever it is."""
+    build = load_build()
+    monkeypatch.setattr(build, "OUT_DIR", str(tmp_path))
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path / "build"))
+    outputs = (build.lib_path(), build.bench_lib_path(), build.torch_lib_path())
+    newest = max(os.path.getmtime(f) for f in build._inputs())
+
+    def write(path, age):
+        with open(path, "w") as f:
+            f.write("built")
+        os.utime(path, (newest - age, newest - age))
+
+    for path in outputs:
+        write(path, -10)
+    assert not build.is_stale()
+    for path in outputs:
+        write(path, 10)
+        assert build.is_stale(), path
+        write(path, -10)
+
+    def fails(hipcc):
+        raise RuntimeError("the module does not compile")
+
+    monkeypatch.setattr(build, "_compile_one", lambda hipcc, src: ("", ""))
+    monkeypatch.setattr(build, "_link", lambda hipcc, objs, out: write(out, -20))
+    monkeypatch.setattr(build, "_build_torch_module", fails)
+    with pytest.raises(RuntimeError, match="does not compile"):
+        build.build(force=True, verbose=False)
+    assert not os.path.exists(build.torch_lib_path()) and build.is_stale()
+    monkeypatch.setattr(build, "_build_torch_module", lambda hipcc: write(build.torch_lib_path(), -20))
+    build.build(verbose=False)
+    assert not build.is_stale()
+
+
 def asm_kernel(name, body):
     return "%s:\n%s\n\ts_endpgm\n" % (name, "\n".join("\t" + l for l in body))
 

@@ -66,6 +66,13 @@ def test_nothing_is_taken_without_a_gpu():
             fn(cpu)
 
 
+def test_a_module_built_for_another_torch_is_refused(monkeypatch):
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    with pytest.raises(RuntimeError, match="0.0.0"):
+        _lib.native()
+
+
 class Subclass(torch.Tensor):
     pass
 

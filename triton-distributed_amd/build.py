@@ -69,10 +69,10 @@ def _inputs():
 
 
 def is_stale():
-    lib = lib_path()
-    if not all(os.path.exists(f) for f in (lib, bench_lib_path(), torch_lib_path())):
+    outputs = (lib_path(), bench_lib_path(), torch_lib_path())
+    if not all(os.path.exists(f) for f in outputs):
         return True
-    t = os.path.getmtime(lib)
+    t = min(os.path.getmtime(f) for f in outputs)
     return any(os.path.getmtime(f) > t for f in _inputs())
 
 
@@ -191,7 +191,7 @@ def _build_torch_module(hipcc):
     from torch.utils.cpp_extension import include_paths, library_paths
     tmp = torch_lib_path() + ".tmp"
     cmd = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", INCLUDE, "-isystem", sysconfig.get_paths()["include"]]
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, '-DTDIST_TORCH_VERSION="%s"' % torch.__version__, "-I", INCLUDE, "-isystem", sysconfig.get_paths()["include"]]
     for path in include_paths() + ["/opt/rocm/include"]:
         cmd += ["-isystem", path]
     cmd += [os.path.join(CSRC, TORCH_SOURCE), "-o", tmp]
@@ -218,6 +218,9 @@ def build(force=False, verbose=True):
             objs[src] = obj
             if verbose and log.strip():
                 print(log, file=sys.stderr)
+    # (the module calls the library's entry points by name: none built against an older tdist.h stays beside a newer library)
+    if os.path.exists(torch_lib_path()):
+        os.remove(torch_lib_path())
     _link(hipcc, [objs[s] for s in BENCH_SOURCES], bench_lib_path())
     _link(hipcc, [objs[s] for s in SOURCES], lib_path())
     _build_torch_module(hipcc)

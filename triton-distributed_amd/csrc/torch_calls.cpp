@@ -686,5 +686,7 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "tdist_torch", nullptr, -1, kMetho
 PyMODINIT_FUNC PyInit_tdist_torch() {
   for (int i = 0; i < kNumAttrs; ++i)
     if (!(g_attr[i] = PyUnicode_InternFromString(kAttrNames[i]))) return nullptr;
-  return PyModule_Create(&kModule);
+  PyObject* const m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TDIST_TORCH_VERSION) != 0) return Py_DECREF(m), nullptr;
+  return m;
 }

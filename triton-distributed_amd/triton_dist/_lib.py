@@ -149,13 +149,16 @@ def native():
         import importlib.machinery
         import importlib.util
 
-        import torch  # noqa: F401  (the libraries it is linked against)
+        import torch   # (the libraries it is linked against)
         load()
         if not os.path.exists(TORCH_LIB_PATH):
             raise RuntimeError("tdist_torch.so is missing at %s: build it with `python triton-distributed_amd/build.py`" % TORCH_LIB_PATH)
         loader = importlib.machinery.ExtensionFileLoader("tdist_torch", TORCH_LIB_PATH)
         mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("tdist_torch", TORCH_LIB_PATH, loader=loader))
         loader.exec_module(mod)
+        if mod.torch_version != str(torch.__version__):
+            raise RuntimeError("tdist_torch.so was built for torch %s, this is %s: run `python triton-distributed_amd/build.py --force`"
+                               % (mod.torch_version, torch.__version__))
         mod.set_error(TdistError)
         _native = mod
     return _native
