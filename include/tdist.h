@@ -450,7 +450,8 @@ int tdist_moe_join_blocks(const int32_t* sorted_token_ids, const int32_t* expert
  * most tail_most (below out_block), go into blocks of tail_block rows there (ids, an expert and a segment 0 to a block, the padded total;
  * tail_rows: room for that many ids) instead of a block that they would fill in part; both blocks are powers of two. Decided on the device,
  * from what the blocks hold: where that takes a round of tiles away and there is room for all, else every row is in the first list and
- * tail_padded[0] = 0. */
+ * tail_padded[0] = 0. (The last is also what calls get whose tails' places have no room in the LDS, num_blocks + 3 num_experts words; what
+ * tdist_moe_join_blocks takes, num_blocks + 2 num_experts, is taken here.) */
 int tdist_moe_join_blocks_tails(const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_padded,
                                 int num_blocks, int block_size, int num_valid_tokens, int num_experts, int out_block,
                                 int32_t* out_sorted_ids, int64_t out_rows, int32_t* out_expert_ids, int32_t* out_segment_ids,

@@ -94,6 +94,39 @@ def test_products_over_both_lists(cuda, dtype, K, counts, n, taken):
             assert torch.equal(c, want)
 
 
+def test_no_room_for_the_tails_places(cuda):
+    """Blocks and experts for which the plain join's words fill the LDS: the same first list as by it, and nothing in the second."""
+    from triton_dist import _lib
+    from triton_dist.kernels.amd import sort_topk_ids_align_block_size
+    announce("join with tails, the LDS full")
+    counts, block, out, n = CASES[0][0], 64, 256, 4096
+    E, entries, words = len(counts), sum(counts), (160 * 1024 - 256) // 4
+    ids = routing(counts, torch.Generator().manual_seed(5)).to(cuda)
+    sorted_ids, experts, _, _, padded = sort_topk_ids_align_block_size(ids, E, 1, entries, block)
+    n_blocks, n_tails = entries // out + E, 8
+    for num_blocks, room in ((words - 3 * E, True), (words - 3 * E + 1, False), (words - 2 * E, False)):
+        ids_in = torch.full((num_blocks * block, ), entries, dtype=torch.int32, device=cuda)
+        experts_in = torch.zeros(num_blocks, dtype=torch.int32, device=cuda)
+        used = min(experts.numel(), sorted_ids.numel() // block)
+        ids_in[:used * block], experts_in[:used] = sorted_ids[:used * block], experts[:used]
+
+        def outputs():
+            return [torch.full((size, ), -7, dtype=torch.int32, device=cuda) for size in (n_blocks * out, n_blocks, n_blocks, 1, n_tails * 64, n_tails, n_tails, 1)]
+
+        a, b = outputs(), outputs()
+        args = (ids_in.data_ptr(), experts_in.data_ptr(), padded.data_ptr(), num_blocks, block, entries, E, out)
+        p, q = [t.data_ptr() for t in a], [t.data_ptr() for t in b]
+        _lib.call("tdist_moe_join_blocks", *args, q[0], b[0].numel(), q[1], q[2], q[3], _lib.stream_ptr())
+        _lib.call("tdist_moe_join_blocks_tails", *args, p[0], a[0].numel(), p[1], p[2], p[3], 128, 64, n, p[4], a[4].numel(), p[5], p[6], p[7],
+                  _lib.stream_ptr())
+        torch.cuda.synchronize()
+        if room:
+            assert int(a[7]) > 0 or _lib.load().tdist_num_cus() != 256
+            continue
+        assert int(a[7]) == 0 and all((t == -7).all() for t in a[4:7])
+        assert all(torch.equal(x, y) for x, y in zip(a[:4], b[:4]))
+
+
 def test_what_the_join_with_tails_refuses(cuda):
     from triton_dist import _lib
     lib = _lib.load()

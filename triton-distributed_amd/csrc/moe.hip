@@ -1631,7 +1631,7 @@ struct JoinParams {
   int32_t *out_ids, *out_experts, *out_segments, *out_padded;
   // tail_most != 0: an expert's last rows, where they are at most that many, go into blocks of tail_block rows of a list of their own instead
   // of a block of `out_block` that they would fill in part (both powers of two). Done where it takes a round away from a GEMM of `cols`
-  // tiles to a block on `cus` compute units and the list has room for all of them; else it is empty.
+  // tiles to a block on `cus` compute units and the list has room for all of them; else it is empty. tail_padded (or NULL) is set either way.
   int tail_most, tail_block, cols, cus, tail_rows;
   int32_t *tail_ids, *tail_experts, *tail_segments, *tail_padded;
 };
@@ -1744,8 +1744,8 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
     auto rounds = [&](int rows) { return ((uint32_t)rows / (uint32_t)out_block * (uint32_t)p.cols + (uint32_t)p.cus - 1) / (uint32_t)p.cus; };
     tails = all_tail <= p.tail_rows && rounds(all_whole) < rounds(all);
     if (tails) at = at_whole, all = all_whole;
-    if (block == 0 && threadIdx.x == 0) p.tail_padded[0] = tails ? all_tail : 0;
   }
+  if (p.tail_padded && block == 0 && threadIdx.x == 0) p.tail_padded[0] = tails ? all_tail : 0;
   for (int i = 0; i < per; ++i) {
     const int e = threadIdx.x * per + i;
     if (e < E) {
@@ -2243,13 +2243,16 @@ int tdist_moe_join_blocks_tails(TDIST_JOIN_ARGS, int tail_most, int tail_block, 
     return fail(TDIST_ERR_INVALID, "%s: tails of %d rows in blocks of %d, %d columns", who, tail_most, tail_block, columns);
   if ((out_block & (out_block - 1)) != 0 || (tail_block & (tail_block - 1)) != 0)
     return fail(TDIST_ERR_INVALID, "%s: blocks of %d and %d rows (powers of two)", who, out_block, tail_block);
-  j.lds += 4ll * num_experts;
-  if (j.lds > kJoinLdsLimit || out_rows / out_block * ceil_div(columns, 256) > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: %d blocks, %d experts", who, num_blocks, num_experts);
   const DeviceInfo& di = device_info();
   if (di.ok != 1) return fail(TDIST_ERR_DEVICE, "%s: current device is not gfx950", who);
-  j.p.tail_most = tail_most, j.p.tail_block = tail_block, j.p.cus = di.num_cus, j.p.tail_rows = (int)tail_rows;
-  j.p.cols = (int)ceil_div(columns, 256);
-  j.p.tail_ids = tail_ids, j.p.tail_experts = tail_experts, j.p.tail_segments = tail_segments, j.p.tail_padded = tail_padded;
+  j.p.tail_padded = tail_padded;
+  // (no room for the tails' places, in the LDS or in 32 bits: the blocks are joined all the same, and no row goes into the second list)
+  if (j.lds + 4ll * num_experts <= kJoinLdsLimit && out_rows / out_block * ceil_div(columns, 256) <= 0x7fffffff) {
+    j.lds += 4ll * num_experts;
+    j.p.tail_most = tail_most, j.p.tail_block = tail_block, j.p.cus = di.num_cus, j.p.tail_rows = (int)tail_rows;
+    j.p.cols = (int)ceil_div(columns, 256);
+    j.p.tail_ids = tail_ids, j.p.tail_experts = tail_experts, j.p.tail_segments = tail_segments;
+  }
   TDIST_JOIN_PICK(moe_join_blocks_kernel)
   hipLaunchKernelGGL(kern, dim3((unsigned)j.grid), dim3(j.threads), (size_t)j.lds, (hipStream_t)stream, j.p);
   return launch_status(who);
