@@ -151,7 +151,7 @@ def test_contexts_made_in_inference_mode_and_rerouted_between_replays(cuda):
 
 # one entry; blocks that are full, short and of one row; an expert without rows; more experts than entries; a block size that is
 # no whole number of waves; more blocks than waves in the grid; experts that come back in a later block
-@pytest.mark.parametrize("entries,E,world,block,out_block", [(2, 4, 1, 128, 128), (1000, 3, 4, 128, 256), (64, 40, 2, 128, 128), (4000, 64, 8, 128, 256),
+@pytest.mark.parametrize("entries,E,world,block,out_block", [(2, 4, 1, 128, 128), (1000, 3, 4, 128, 256), (3000, 7, 4, 128, 192), (20000, 7, 4, 128, 192), (64, 40, 2, 128, 128), (4000, 64, 8, 128, 256),
                                                              (640, 5, 2, 96, 128), (20000, 9, 8, 32, 256), (300, 512, 4, 256, 128)])
 def test_joined_blocks_are_the_sort_without_segments(cuda, monkeypatch, entries, E, world, block, out_block):
     from triton_dist import _lib

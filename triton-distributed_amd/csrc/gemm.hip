@@ -2476,8 +2476,8 @@ static double group_large_us(const GroupShape& g, int block, bool split_last, in
 // Rows that an expert's last block may have to go into blocks of 64 rows of a launch of their own, where that is likely to take a round of
 // tiles from the others: half a block, which is two short ones. (What the routing is, and so whether it is done, is known on the device
 // only: moe_join_blocks_kernel.) A last round, whole or cut along K, takes 30 us and more, the other launch 10 to 20, and 2 with nothing to
-// do: 8192 tokens, top 2 of 8 experts, 1792 deep by 4096 columns: a layer 492 -> 472 us, and
-// 457 -> 460 where every expert has exactly eight blocks and the other launch finds nothing.
+// do, however few its workgroups: 8192 tokens, top 2 of 8 experts, 1792 deep by 4096 columns: a layer 476 -> 456 us, and
+// 442 -> 444 where every expert has exactly eight blocks and the other launch finds nothing.
 static int group_tail_rows(const GroupShape& g, int block, int cus) {
   const double used = std::max(1.0, groups_in_use(g)), mean = g.rows / used, dev = std::max(0.3, std::sqrt(mean));
   const int most = block / 2;

@@ -1622,13 +1622,14 @@ int moe_static_scratch_init() {
 // and the ids of the first block that a wave will place are all on their way before anything is waited for.
 // What bounds it: the launch, one trip to memory, four barriers. 64 blocks 4.5 us a launch with 4 waves to a workgroup (6.4 with
 // 16), 160 blocks 6.4 and 512 blocks 8.7 with 16 (7.2 and 14.6 with 4): 4 waves up to kJoinFewBlocks, 16 beyond. (In a graph,
-// where a launch that does nothing takes 2.1 us.)
+// where a launch that does nothing takes 2.1 us; since then 79 blocks 4.0, 191 5.6, 636 7.4, and with tails 4.5, 6.2, 7.7.)
 constexpr int kJoinFewBlocks = 96, kJoinMaxBlock = 512, kJoinCountBits = 10;
 constexpr int64_t kJoinLdsLimit = 160 * 1024 - 256;
 struct JoinParams {
   const int32_t *sorted_ids, *expert_ids, *post_pad;
   int num_blocks, block_size, num_valid, E, out_block, out_rows;
   int32_t *out_ids, *out_experts, *out_segments, *out_padded;
+  int out_shift;   // out_block = 1 << out_shift, or negative: no power of two
   // tail_most != 0: an expert's last rows, where they are at most that many, go into blocks of tail_block rows of a list of their own instead
   // of a block of `out_block` that they would fill in part (both powers of two). Done where it takes a round away from a GEMM of `cols`
   // tiles to a block on `cus` compute units and the list has room for all of them; else it is empty. tail_padded (or NULL) is set either way.
@@ -1701,7 +1702,9 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
   __syncthreads();
   // exclusive prefix of the experts' padded sizes: a thread takes `per` neighbours
   const int per = (E + kThreads - 1) / kThreads;
-  auto padded = [&](int n) { return (n + out_block - 1) / out_block * out_block; };
+  const int shift = p.out_shift;   // (a division by a number that is not known is twenty instructions in a row: 0.2 to 0.4 us of a join)
+  auto blocks_of = [&](int n) { return shift >= 0 ? n >> shift : n / out_block; };
+  auto padded = [&](int n) { return blocks_of(n + out_block - 1) * out_block; };
   auto tail_padded = [&](int n) { return (n + p.tail_block - 1) & -p.tail_block; };
   bool tails = p.tail_most > 0;
   auto tail_of = [&](int total) {   // (rows of an expert in the list of tails)
@@ -1726,23 +1729,34 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
     if (lane == 63) s_part[1][wave] = sum_whole, s_part[2][wave] = sum_tail;
   }
   __syncthreads();
-  int at = sum - own, all = 0, at_tail = 0, all_tail = 0;
+  // What the waves before this one have, and all of them. (16 waves: by a scan; three rows of 16 sums read one by one were most of
+  // what tails cost a join: 191 blocks 7.3 -> 6.6 us, without tails 6.1 -> 5.8. Four waves' sums are read as fast.)
+  auto over_waves = [&](const int32_t* part, int& before, int& all) {
+    if constexpr (kWaves > 4) {
+      const int v = lane < kWaves ? part[lane] : 0, upto = wave_scan_add(v);
+      before = __builtin_amdgcn_readlane(upto, wave) - __builtin_amdgcn_readlane(v, wave);
+      all = __builtin_amdgcn_readlane(upto, 63);
+    } else {
+      before = all = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    if (w < wave) at += s_part[0][w];
-    all += s_part[0][w];
-  }
-  if (tails) {
-    int at_whole = sum_whole - own_whole, all_whole = 0;
-    at_tail = sum_tail - own_tail;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      if (w < wave) at_whole += s_part[1][w], at_tail += s_part[2][w];
-      all_whole += s_part[1][w];
-      all_tail += s_part[2][w];
+      for (int w = 0; w < kWaves; ++w) {
+        before += w < wave ? part[w] : 0;
+        all += part[w];
+      }
     }
-    auto rounds = [&](int rows) { return ((uint32_t)rows / (uint32_t)out_block * (uint32_t)p.cols + (uint32_t)p.cus - 1) / (uint32_t)p.cus; };
-    tails = all_tail <= p.tail_rows && rounds(all_whole) < rounds(all);
+  };
+  int before_own, all, at_tail = 0, all_tail = 0;
+  over_waves(s_part[0], before_own, all);
+  int at = before_own + sum - own;
+  if (tails) {
+    int before_whole, before_tail, all_whole;
+    over_waves(s_part[1], before_whole, all_whole);
+    over_waves(s_part[2], before_tail, all_tail);
+    const int at_whole = before_whole + sum_whole - own_whole;
+    at_tail = before_tail + sum_tail - own_tail;
+    // (fewer rounds: the tiles that are left fill at most the whole rounds before the last one of all)
+    const uint32_t cus = p.cus, tiles = (uint32_t)blocks_of(all) * p.cols, left = (uint32_t)blocks_of(all_whole) * p.cols;
+    tails = all_tail <= p.tail_rows && tiles > 0 && left <= (tiles - 1) / cus * cus;
     if (tails) at = at_whole, all = all_whole;
   }
   if (p.tail_padded && block == 0 && threadIdx.x == 0) p.tail_padded[0] = tails ? all_tail : 0;
@@ -1758,7 +1772,7 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
       }
     }
   }
-  if (block == 0 && threadIdx.x == 0) p.out_padded[0] = min(all, out_rows / out_block * out_block);
+  if (block == 0 && threadIdx.x == 0) p.out_padded[0] = min(all, blocks_of(out_rows) * out_block);
   __syncthreads();
   for (int b = gwave; b < used; b += waves) {
     const int e = s_block[b] >> kJoinCountBits;
@@ -1800,7 +1814,7 @@ __device__ __forceinline__ void join_blocks(const JoinParams& p, int block, int 
       }
     }
     for (int r = lo + total + lane; r < hi; r += 64) out_ids[r] = num_valid;
-    for (int b = lo / out_block + lane; b < hi / out_block; b += 64) {
+    for (int b = blocks_of(lo) + lane; b < blocks_of(hi); b += 64) {
       p.out_experts[b] = e;
       p.out_segments[b] = 0;
     }
@@ -2205,7 +2219,8 @@ static int join_launch(JoinLaunch& j, const char* who, TDIST_JOIN_ARGS) {
   if (block_size > kJoinMaxBlock || num_experts > kMoeMaxExperts || j.lds > kJoinLdsLimit || out_rows > 0x7fffffffll)
     return fail(TDIST_ERR_UNSUPPORTED, "%s: %d blocks of %d rows, %d experts", who, num_blocks, block_size, num_experts);
   j.p = {sorted_token_ids, expert_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, num_experts, out_block,
-         (int)out_rows, out_sorted_ids, out_expert_ids, out_segment_ids, out_post_padded, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr};
+         (int)out_rows, out_sorted_ids, out_expert_ids, out_segment_ids, out_post_padded,
+         (out_block & (out_block - 1)) == 0 ? __builtin_ctz(out_block) : -1, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr};
   j.threads = num_blocks <= kJoinFewBlocks ? 256 : 1024;
   const int64_t items = ceil_div(num_blocks > num_experts ? num_blocks : num_experts, j.threads / 64);
   j.grid = (int)(items < 32 ? items : 32);
