@@ -46,9 +46,9 @@ MEASURED_SOURCE_DIGEST = {
     "decode.hip": "86e8879aaf685690",
     "gather.h": "3fd5e450cd06de4d",
     "gemm.hip": "72031edd6254e04a",
-    "gemm_small.h": "1368c14b33b545a8",
+    "gemm_small.h": "ceafc5b3b8b28bd1",
     "gemm_small.hip": "87b09035e69e02ec",
-    "moe.hip": "5159f846f7e03e55",
+    "moe.hip": "d6426776d5a3636c",
     "reduce.hip": "469689d34df1b205",
 }
 CSRC = os.path.join(ROOT, "triton-distributed_amd", "csrc")

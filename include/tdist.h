@@ -187,6 +187,9 @@ int tdist_producer_push_peers(void* workspace, const void* const* peer_src, int 
 #define TDIST_GATHER_MAX_RANKS 64
 int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
                         int32_t* first_error, void* stream);
+/* Whether shards of `rows` rows (rank_bytes in all) are read where they lie, 1 or 0: what tdist_group_gemm_rows takes, and tdist_ag_gemm_rows
+ * without a gather. */
+int tdist_shards_in_reach(const void* const* shards, int world_size, int rows, int64_t rank_bytes);
 
 /* C = the gathered rows x B^T for an all-gather whose shards all lie on this GPU: tdist_gather_shards and an ungated
  * tdist_gemm_chunk_gated_* in one call, of which the gather is left out where the GEMM can read the rows where they lie
@@ -363,6 +366,8 @@ int tdist_moe_dispatch_tokens_from_ids64(const void* tokens, int64_t row_bytes, 
                                          int experts_per_rank, int max_m, void* slot_rows, float* slot_scales,
                                          int32_t* splits_out, int32_t* splits, int32_t* cumsum, int32_t* scatter_idx,
                                          int32_t* gather_idx, void* stream);
+/* 0 where a call is too large for the two, in any of these sizes (tdist_moe_scatter_index and tdist_moe_dispatch_tokens take it), else 1. */
+int tdist_moe_dispatch_from_ids_takes(int64_t n_tokens, int topk, int64_t row_bytes, int num_experts);
 
 /* Compaction of the slots into one [sum, row_bytes] tensor in destination order
  * (all_to_all_post_process, low_latency_all_to_all.py:251-270): output row p comes from slot row
@@ -521,10 +526,12 @@ int tdist_group_gemm_rows(int dtype, const void* const* shards, int world_size, 
                           const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,
                           int num_blocks, int block_size, int num_valid_tokens, int topk, int32_t* status,
                           int32_t* first_error, void* sk_workspace, int64_t sk_workspace_bytes, void* stream);
-/* Rows of an expert's tail that are worth a block of 64 rows of their own (tdist_moe_join_blocks_tails) beside blocks of `block` rows, by an
+#define TDIST_GROUP_TAIL_BLOCK 64
+/* Rows of an expert's tail that are worth a block of TDIST_GROUP_TAIL_BLOCK rows of their own (tdist_moe_join_blocks_tails) beside blocks of `block` rows, by an
  * estimate for rows evenly at random over the experts; 0: none. */
 int tdist_group_gemm_tail_rows(int64_t rows, int num_experts, int N, int64_t k_bytes, int block);
-/* tdist_group_gemm_rows over both lists of tdist_moe_join_blocks_tails, the second in tail_blocks blocks of 64 rows at most: two launches. */
+/* tdist_group_gemm_rows over both lists of tdist_moe_join_blocks_tails, the second in tail_blocks blocks of TDIST_GROUP_TAIL_BLOCK rows at most: two
+ * launches. */
 int tdist_group_gemm_rows_tails(int dtype, const void* const* shards, int world_size, int rows_per_rank, const void* B, int64_t ldb,
                                 int64_t expert_stride, void* C, int64_t ldc, int N, int K, const int32_t* sorted_token_ids,
                                 const int32_t* expert_ids, const int32_t* block_barrier_ids, const int32_t* num_tokens_post_padded,

@@ -99,6 +99,13 @@ def test_null_pointers_are_rejected_without_touching_the_gpu():
     assert lib.tdist_moe_workspace_bytes(32768, 256) == (128 + 1) * 256 * 4 + 256
 
 
+@pytest.mark.parametrize("tokens,topk,row_bytes,experts,takes", [
+    (1, 1, 1, 1, 1), (8192, 8, 7168, 256, 1), (8193, 8, 7168, 256, 0), (0, 8, 7168, 256, 1), (16, 64, 16 * 8192, 4096, 1), (16, 65, 7168, 256, 0),
+    (16, 8, 16 * 8192 + 1, 256, 0), (16, 8, 2 * 8192 + 1, 256, 0), (16, 8, 3 * 8192 + 1, 256, 1), (16, 8, 7168, 4097, 0), (16, 8, 0, 256, 0)])
+def test_what_the_dispatch_from_ids_takes(tokens, topk, row_bytes, experts, takes):
+    assert _lib.load().tdist_moe_dispatch_from_ids_takes(tokens, topk, row_bytes, experts) == takes
+
+
 @pytest.mark.parametrize("entry,scales", [("tdist_gemm_rs_scatter_bf16", []), ("tdist_gemm_rs_scatter_f16", []),
                                           ("tdist_gemm_rs_scatter_fp8e4m3", [None, None])])
 @pytest.mark.parametrize("rows_per_rank", [128, 64, 192, 320, 2048])
@@ -141,6 +148,9 @@ def test_debug_switches_default_to_automatic_and_ignore_the_environment(monkeypa
                  "DECODE_SPLITS_PER_TEAM", "MOE_INDEX_FORM"):
         m = re.search(r"TDIST_DEBUG_%s\s*=\s*(\d+)" % name, text)
         assert m and int(m.group(1)) == getattr(_lib, "TDIST_DEBUG_" + name), name
+    for name in ("GATHER_MAX_RANKS", "GROUP_TAIL_BLOCK"):
+        m = re.search(r"#define TDIST_%s (\d+)" % name, text)
+        assert m and int(m.group(1)) == getattr(_lib, name), name
     import glob
     for src in glob.glob(os.path.join(ROOT, "triton-distributed_amd", "csrc", "*")):
         assert "getenv" not in open(src).read(), "%s reads the environment" % src

@@ -48,6 +48,7 @@ constexpr int kSmallMaxSplits = 16;
 // into the L2 first, or asked for in front of the products, they were no faster, and the other tiles slower.)
 constexpr int kSmallSumRows = 448;
 constexpr int kGroupedFewRows = kSmallTiles[0].bm;   // rows of the smallest blocks of the grouped form
+static_assert(kGroupedFewRows == TDIST_GROUP_TAIL_BLOCK, "experts' last rows come in the smallest blocks");
 
 // `deep`: six stages instead of three, one workgroup per compute unit
 int launch_gemm_small(const SmallGemmParams& p, SmallGemmElem elem, int tile, bool deep, hipStream_t stream, const char* who);

@@ -262,6 +262,12 @@ using namespace tdist;
 
 extern "C" {
 
+int tdist_shards_in_reach(const void* const* shards, int world_size, int rows, int64_t rank_bytes) {
+  ShardRows at;
+  const unsigned char* base;
+  return shards && shards_in_reach(shards, world_size, rows, rank_bytes, at, base);
+}
+
 int tdist_gather_shards(void* workspace, const void* const* shards, int world_size, int64_t rank_bytes, int32_t* status,
                         int32_t* first_error, void* stream) {
   const char* who = "tdist_gather_shards";

@@ -1935,6 +1935,19 @@ int tdist_moe_dispatch_tokens(const void* tokens, int64_t row_bytes, const float
   return launch_status("tdist_moe_dispatch_tokens");
 }
 
+// (+ a word per lane for what is not counted)
+static int64_t from_ids_lds(int64_t G, int topk) { return (3 * G + ((G + 1 + 3) & ~3ll) + kFdWaves * topk + 8 + 64) * 4; }
+// The sizes that the launch from ids takes.
+static bool from_ids_takes(int64_t n_tokens, int topk, int64_t row_bytes, int64_t G) {
+  const int64_t windows = ceil_div(row_bytes, 8192);
+  return n_tokens * topk <= kFusedDispatchMaxIds && topk <= 64 && G <= kMoeMaxExperts && windows >= 1 && windows <= kFdWaves &&
+         kFdWaves % windows == 0 && from_ids_lds(G, topk) <= 160 * 1024 - 256;
+}
+
+int tdist_moe_dispatch_from_ids_takes(int64_t n_tokens, int topk, int64_t row_bytes, int num_experts) {
+  return from_ids_takes(n_tokens, topk, row_bytes, num_experts);
+}
+
 static int dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const float* token_scales, const int32_t* ids,
                                     int ids_wide, int topk, int64_t n_tokens, int world_size, int experts_per_rank, int max_m,
                                     void* slot_rows, float* slot_scales, int32_t* splits_out, int32_t* splits, int32_t* cumsum,
@@ -1944,17 +1957,15 @@ static int dispatch_tokens_from_ids(const void* tokens, int64_t row_bytes, const
     return fail(TDIST_ERR_INVALID, "%s: token_scales and slot_scales go together", who);
   if (row_bytes <= 0 || n_tokens < 0 || world_size <= 0 || experts_per_rank <= 0 || max_m <= 0 || topk <= 0)
     return fail(TDIST_ERR_INVALID, "%s: bad sizes", who);
-  if (topk > 64) return fail(TDIST_ERR_UNSUPPORTED, "%s: topk > 64", who);
   const int64_t G64 = (int64_t)world_size * experts_per_rank;
-  if (G64 > kMoeMaxExperts) return fail(TDIST_ERR_UNSUPPORTED, "%s: num_experts %lld > %d", who, (long long)G64, kMoeMaxExperts);
   if ((int64_t)world_size * max_m > 0x7fffffff) return fail(TDIST_ERR_UNSUPPORTED, "%s: world_size * max_m too large", who);
+  if (!from_ids_takes(n_tokens, topk, row_bytes, G64))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: more than %lld ids, 64 of them to a token or %d experts, or rows above %d bytes (or no power-of-two "
+                "number of 8 KB windows): use tdist_moe_scatter_index + tdist_moe_dispatch_tokens", who, (long long)kFusedDispatchMaxIds,
+                kMoeMaxExperts, kFdWaves * 8192);
   const int G = (int)G64;
   int windows = (int)ceil_div(row_bytes, 8192);
-  const int64_t lds = ((int64_t)3 * G + ((G + 1 + 3) & ~3) + kFdWaves * topk + 8 + 64) * 4;   // (+ a word per lane for what is not counted)
-  if (n_tokens * topk > kFusedDispatchMaxIds || windows > kFdWaves || kFdWaves % windows != 0 || lds > 160 * 1024 - 256)
-    return fail(TDIST_ERR_UNSUPPORTED, "%s: more than %lld ids, rows above %d bytes (or no power-of-two number of 8 KB windows), or too "
-                "many experts for one workgroup's counters: use tdist_moe_scatter_index + tdist_moe_dispatch_tokens", who,
-                (long long)kFusedDispatchMaxIds, kFdWaves * 8192);
+  const int64_t lds = from_ids_lds(G, topk);
   // Few tokens: smaller windows, as long as there are fewer workgroups than a quarter of the compute units (every
   // workgroup counts all ids, so more of them is not free) and a window holds a KB.
   int vecs = 8;

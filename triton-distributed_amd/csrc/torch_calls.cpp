@@ -205,11 +205,9 @@ PyObject* decode_ranks(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
 }
 
 // ---- GEMMs ---------------------------------------------------------------------------------------------------
-constexpr int kMaxRanks = 64;
-
 // The table of every rank's shard: `own` at `rank`, the others from a dict rank -> tensor.
 bool shards_of(const at::Tensor& own, PyObject* peers, int rank, int ranks, int device, const void** table) {
-  if (!PyDict_CheckExact(peers) || ranks < 2 || ranks > kMaxRanks || rank < 0 || rank >= ranks || !aligned16(own)) return false;
+  if (!PyDict_CheckExact(peers) || ranks < 2 || ranks > TDIST_GATHER_MAX_RANKS || rank < 0 || rank >= ranks || !aligned16(own)) return false;
   int found = 1;
   table[rank] = own.data_ptr();
   PyObject *key, *value;
@@ -242,7 +240,7 @@ PyObject* ag_gemm(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
   int code, rank, ranks;
   c10::ScalarType out_type;
   TDIST_ORDINARY(operands_of(o[0], o[1], device, &a, &b, &code, &out_type) && int_of(o[3], &rank) && int_of(o[4], &ranks));
-  const void* shards[kMaxRanks];
+  const void* shards[TDIST_GATHER_MAX_RANKS];
   TDIST_ORDINARY(shards_of(*a, o[2], rank, ranks, device, shards));
   const at::Tensor *workspace = tensor_of(o[5], device), *status = tensor_of(o[6], device, c10::ScalarType::Int, 1);
   const int64_t bytes = a->numel() * a->element_size(), M = a->size(0), K = a->size(1), N = b->size(0);
@@ -299,10 +297,9 @@ struct Blocks {
   int block_size, entries;
   int64_t at[4];   // addresses: sorted ids, experts, segments, padded total
   int count, rows;
-  int tail_most, tail_count;   // experts' last rows in blocks of their own, of kTailBlock rows, one array behind the other from tail_ids on
+  int tail_most, tail_count;   // experts' last rows in blocks of their own, of TDIST_GROUP_TAIL_BLOCK rows, one array behind the other from tail_ids on
   int32_t *tail_ids, *tail_experts, *tail_segments, *tail_padded;
 };
-constexpr int kTailBlock = 64;
 // o[0..4]: sorted ids, experts and padded total of the align / sort, its block size, entries; o[5..13]: a RowBlocks, field by field
 bool blocks_of(PyObject* const* o, int device, Blocks& b) {
   b.sorted = tensor_of(o[0], device, c10::ScalarType::Int, 1), b.experts = tensor_of(o[1], device, c10::ScalarType::Int, 1);
@@ -316,7 +313,7 @@ bool blocks_of(PyObject* const* o, int device, Blocks& b) {
       (tail = PyLong_AsLongLong(o[12])) < 0) return PyErr_Clear(), false;
   b.tail_ids = (int32_t*)tail;
   if ((b.tail_most > 0) != (tail != 0 && b.tail_count > 0)) return false;
-  b.tail_experts = b.tail_ids + (int64_t)b.tail_count * kTailBlock;
+  b.tail_experts = b.tail_ids + (int64_t)b.tail_count * TDIST_GROUP_TAIL_BLOCK;
   b.tail_segments = b.tail_experts + b.tail_count;
   b.tail_padded = b.tail_segments + b.tail_count;
   return true;
@@ -336,7 +333,7 @@ int join_and_multiply(const Blocks& k, int code, const void* const* shards, int 
   const int64_t room = (int64_t)k.count * k.rows;
   int rc = k.tail_most > 0
                ? tdist_moe_join_blocks_tails(i32(k.sorted), i32(k.experts), i32(k.padded), blocks, k.block_size, k.entries, (int)b.size(0), k.rows, ids, room,
-                                             experts, segments, padded, k.tail_most, kTailBlock, N, k.tail_ids, (int64_t)k.tail_count * kTailBlock,
+                                             experts, segments, padded, k.tail_most, TDIST_GROUP_TAIL_BLOCK, N, k.tail_ids, (int64_t)k.tail_count * TDIST_GROUP_TAIL_BLOCK,
                                              k.tail_experts, k.tail_segments, k.tail_padded, stream)
                : tdist_moe_join_blocks(i32(k.sorted), i32(k.experts), i32(k.padded), blocks, k.block_size, k.entries, (int)b.size(0), k.rows, ids, room,
                                        experts, segments, padded, stream);
@@ -360,15 +357,12 @@ PyObject* ag_group_gemm(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
   TDIST_ORDINARY(a && a->dim() == 2 && a->is_contiguous() && a->numel() > 0 && code_of(a->scalar_type(), &code) && int_of(o[3], &rank) &&
                  int_of(o[4], &ranks) && int_of(o[5], &topk) && topk > 0);
   const int64_t M = a->size(0), row_bytes = a->size(1) * a->element_size();
-  const void* shards[kMaxRanks];
+  const void* shards[TDIST_GATHER_MAX_RANKS];
   TDIST_ORDINARY(shards_of(*a, o[2], rank, ranks, device, shards) && M * row_bytes % 16 == 0 && M * ranks <= INT_MAX);
   const at::Tensor *b = weights_of(o[1], device, *a, M * ranks), *workspace = tensor_of(o[6], device), *status = tensor_of(o[7], device, c10::ScalarType::Int, 1);
   TDIST_ORDINARY(b && workspace && workspace->numel() * workspace->element_size() >= ranks * M * row_bytes && status && status->numel() == 4 &&
                  status->is_contiguous());
-  // (what tdist_group_gemm_rows takes as rows in shards)
-  const auto span = std::minmax_element(shards, shards + ranks);
-  TDIST_ORDINARY(ranks <= 16 && M >= 2 && ranks * M * M < 1ll << 32 &&
-                 (const char*)*span.second - (const char*)*span.first + M * row_bytes < (1ll << 32) - 4096);
+  TDIST_ORDINARY(tdist_shards_in_reach(shards, ranks, (int)M, M * row_bytes));
   void* sk;
   int64_t sk_bytes;
   Blocks k;
@@ -564,10 +558,8 @@ PyObject* dispatch_ids(PyObject*, PyObject* const* o, Py_ssize_t nargs) {
   TDIST_ORDINARY(optional_of(o[2], device, c10::ScalarType::Float, &scale));
   Slots s;
   TDIST_ORDINARY(slots_of(ctx, device, s) && x->size(1) == s.hidden && x->scalar_type() == s.type);
-  const int64_t T = ids->size(0), topk = ids->size(1), row_bytes = (int64_t)s.hidden * s.ele, windows = (row_bytes + 8191) / 8192;
-  // (what the launch from ids takes, as the Python code states it)
-  TDIST_ORDINARY(T * topk <= 65536 && (windows == 1 || windows == 2 || windows == 4 || windows == 8 || windows == 16) && topk <= 64 &&
-                 (4 * (int64_t)s.experts + 16 * topk + 8) * 4 <= 160 * 1024 - 256);
+  const int64_t T = ids->size(0), topk = ids->size(1), row_bytes = (int64_t)s.hidden * s.ele;
+  TDIST_ORDINARY(tdist_moe_dispatch_from_ids_takes(T, (int)topk, row_bytes, s.experts));
   IndexSet set;
   TDIST_ORDINARY(index_set_of(ctx, device, T, topk, s.experts, set));
   const Ref last(PyTuple_GetSlice(set.set, 0, 4));

@@ -48,6 +48,7 @@ PROTOTYPES = {
     "tdist_producer_push_peers": (_I, [_P, _P, _I, _I, _L, _L, _P, _I, _P, _P, _P, _L, ctypes.c_uint32, _L, _I, _P]),
     "tdist_ag_gemm_rows": (_I, [_I, _P, _I, _I, _P, _P, _L, _P, _L, _I, _I, _P, _P, _P, _P, _P, _L, _P]),
     "tdist_gather_shards": (_I, [_P, _P, _I, _L, _P, _P, _P]),
+    "tdist_shards_in_reach": (_I, [_P, _I, _I, _L]),
     "tdist_producer_mark": (_I, [_P, _P]),
     "tdist_producer_wait_until": (_I, [_P, _L, _P]),
     "tdist_flag_set": (_I, [_P, _I, _P]),
@@ -67,6 +68,7 @@ PROTOTYPES = {
     "tdist_moe_dispatch_tokens": (_I, [_P, _L, _P, _P, _I, _P, _L, _I, _I, _I, _P, _P, _P, _P]),
     "tdist_moe_dispatch_tokens_from_ids": (_I, [_P, _L, _P, _P, _I, _L, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P]),
     "tdist_moe_dispatch_tokens_from_ids64": (_I, [_P, _L, _P, _P, _I, _L, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "tdist_moe_dispatch_from_ids_takes": (_I, [_L, _I, _L, _I]),
     "tdist_moe_post_process": (_I, [_P, _L, _P, _P, _L, _I, _I, _I, _P, _P, _P]),
     "tdist_moe_combine_reduce": (_I, [_P, _P, _L, _I, _I, _I, _I, _P, _P, _P, _P]),
     "tdist_moe_combine": (_I, [_P, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P, _P]),
@@ -210,7 +212,8 @@ def stream_ptr(stream=None):
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())   # (without a Stream object: 0.2 us for 1.3)
 
 
-GATHER_MAX_RANKS = 64
+GATHER_MAX_RANKS = 64   # TDIST_GATHER_MAX_RANKS
+GROUP_TAIL_BLOCK = 64   # TDIST_GROUP_TAIL_BLOCK: rows of the blocks for experts' last rows
 
 
 def shard_table(own, peer_shards, rank, num_ranks):
@@ -234,8 +237,10 @@ def address_table(tensor):
 
 
 def shards_in_reach(table, rows, row_bytes):
-    """Whether tdist_group_gemm_rows takes these shards where they lie (a host table of shard_table): see gather.h."""
-    return len(table) <= 16 and rows >= 2 and len(table) * rows * rows < 1 << 32 and max(table) - min(table) + rows * row_bytes < (1 << 32) - 4096
+    """Whether tdist_group_gemm_rows takes these shards where they lie (a host table of shard_table, or addresses)."""
+    if not isinstance(table, ctypes.Array):
+        table = (c_void_p * len(table))(*table)
+    return load().tdist_shards_in_reach(table, len(table), rows, rows * row_bytes) != 0
 
 
 _DTYPE_CODES = {}

@@ -126,9 +126,6 @@ def _block_plan(entries, num_experts, n, row_bytes, sk_workspace):
     return (block, (entries + min(num_experts, entries) * (block - 1)) // block) if block > 0 else None
 
 
-_TAIL_BLOCK = 64   # rows of the blocks for experts' last rows
-
-
 class RowBlocks:
     """Addresses of a grouped GEMM's row blocks (sorted ids, an expert and a segment per block, the padded total), their
     number and their rows; ``memory``: the tensor they lie in."""
@@ -177,12 +174,12 @@ def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, bloc
         block, n_blocks = plan or _join_plan(entries, num_experts, n)
         tail_most = _lib.load().tdist_group_gemm_tail_rows(entries, num_experts, n, row_bytes, block) if any_block and gather is None else 0
         # (as many as leave two of their tiles of 128 columns to a compute unit; and with fewer places the GEMM would take K apart for them)
-        tail_blocks = min(min(num_experts, entries) * (tail_most // _TAIL_BLOCK), 2 * _lib.load().tdist_num_cus() // -(-n // 128))
+        tail_blocks = min(min(num_experts, entries) * (tail_most // _lib.GROUP_TAIL_BLOCK), 2 * _lib.load().tdist_num_cus() // -(-n // 128))
         size = n_blocks * (block + 2) + 1
-        memory = torch.empty(size + (tail_blocks * (_TAIL_BLOCK + 2) + 1 if tail_most else 0), dtype=torch.int32, device=sorted_ids.device)
+        memory = torch.empty(size + (tail_blocks * (_lib.GROUP_TAIL_BLOCK + 2) + 1 if tail_most else 0), dtype=torch.int32, device=sorted_ids.device)
         out = made[key] = RowBlocks.of(memory, 0, n_blocks, block)
         if tail_most:
-            out.tail, out.tail_most = RowBlocks.of(memory, size, tail_blocks, _TAIL_BLOCK), tail_most
+            out.tail, out.tail_most = RowBlocks.of(memory, size, tail_blocks, _lib.GROUP_TAIL_BLOCK), tail_most
     args = (sorted_ids.data_ptr(), expert_ids.data_ptr(), num_tokens_post_padded.data_ptr(),
             min(expert_ids.numel(), sorted_ids.numel() // block_size), block_size, entries, num_experts, out.block_size, out.sorted_ids,
             out.num_blocks * out.block_size, out.experts, out.segments, out.padded)
@@ -190,7 +187,7 @@ def joined_row_blocks(made, sorted_ids, expert_ids, num_tokens_post_padded, bloc
     if gather is not None:
         rc = lib.tdist_moe_gather_and_join(*gather, *args, stream)
     elif tail is not None:
-        rc = lib.tdist_moe_join_blocks_tails(*args, out.tail_most, _TAIL_BLOCK, n, tail.sorted_ids, tail.num_blocks * _TAIL_BLOCK, tail.experts,
+        rc = lib.tdist_moe_join_blocks_tails(*args, out.tail_most, _lib.GROUP_TAIL_BLOCK, n, tail.sorted_ids, tail.num_blocks * _lib.GROUP_TAIL_BLOCK, tail.experts,
                                              tail.segments, tail.padded, stream)
     else:
         rc = lib.tdist_moe_join_blocks(*args, stream)

@@ -321,9 +321,6 @@ def fast_all_to_all(
     return out_lis
 
 
-FUSED_INDEX_MAX_IDS = 65536   # tdist_moe_dispatch_tokens_from_ids takes up to this many ids
-
-
 def _fast_all_to_all_from_ids(ctx, send_tensor, send_scale, expert_ids):
     if ctx.fp8_group_size:
         raise ValueError("a context with group scales takes its rows through online_quant_fp8=True")
@@ -332,10 +329,7 @@ def _fast_all_to_all_from_ids(ctx, send_tensor, send_scale, expert_ids):
     assert T == send_tensor.shape[0]
     G = ctx.num_tot_experts
     row_bytes = ctx.hidden * ctx.ele_size
-    windows = -(-row_bytes // 8192)
-    fused = (T * topk <= FUSED_INDEX_MAX_IDS and windows in (1, 2, 4, 8, 16) and topk <= 64
-             and (4 * G + 16 * topk + 8) * 4 <= 160 * 1024 - 256)
-    if not fused:
+    if not _lib.load().tdist_moe_dispatch_from_ids_takes(T, topk, row_bytes, G):
         splits_i, cumsum, scatter, gather = moe_dispatch_preprocess(expert_ids, G, ctx=ctx)
         ctx.last_index = (splits_i, cumsum, scatter, gather)
         return fast_all_to_all(ctx, send_tensor, cumsum, send_scale, scatter_index=scatter)
