@@ -290,3 +290,207 @@ def test_moe_layer(cuda, route, dtype):
     same(a, c)
     same(a, b)
     assert taken == ["align"] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_moe_layer_with_two_lists(cuda, route, dtype):
+    """Experts' last rows in a list of their own, by the module and by the Python code, whole numbers exactly: 512 rows per expert on average
+    and 4096 columns are two rounds of 256-row blocks with the last rows, one without."""
+    from triton_dist.kernels.amd import (ag_group_gemm_intra_node, create_ag_group_gemm_intra_node_context, create_moe_rs_context, moe_reduce_rs)
+    announce("torch calls, MoE layer with two lists %s" % dtype)
+    W, mpr, E, N, K, topk, rank = 4, 512, 8, 4096, 192, 2, 1
+    g = torch.Generator(device=cuda).manual_seed(11)
+
+    def whole(*shape):
+        return torch.randint(-1, 2, shape, generator=g, device=cuda).float().to(dtype)
+
+    shards, logits = [whole(mpr, K) for _ in range(W)], [torch.randn((mpr, E), generator=g, device=cuda) for _ in range(W)]
+    up, down, states = whole(E, N, K).transpose(1, 2), whole(E, N, K).transpose(1, 2), whole(W * mpr * topk, K)
+    peers = {r: t for r, t in enumerate(logits) if r != rank}
+    weight = torch.randint(1, 3, (W * mpr, topk), generator=g, device=cuda).float()
+    partials = [torch.randint(-8, 9, (mpr, N), generator=g, device=cuda).bfloat16() for _ in range(W)]
+    ids = torch.cat(logits).softmax(-1).topk(topk).indices.int()
+    made = []
+
+    def f():
+        ag = create_ag_group_gemm_intra_node_context(None, shards[rank], up, ids, E, max_M=W * mpr, rank=rank, num_ranks=W)
+        ag.set_peer_shards({r: s for r, s in enumerate(shards) if r != rank})
+        rs = create_moe_rs_context(None, rank, W, W, W * mpr, N, E, topk, torch.bfloat16, torch.bfloat16, cuda, 128, logits[rank], peers)
+        rs.topk_weight_f32 = weight
+        rs.set_peer_partials({r: t for r, t in enumerate(partials) if r != rank})
+        made.append((ag, rs))
+        out = []
+        for _ in range(3):
+            out += [ag_group_gemm_intra_node(shards[rank], up, ag), moe_reduce_rs(rank, W, W, states, down, rs)]
+        ag.check_status()
+        return out
+
+    with _lib.debug_switch(_lib.TDIST_DEBUG_GEMM_TILE, 0):   # (256-row blocks, whatever the estimate for so short a K)
+        a, b, taken = route(f)
+    same(a, b)
+    assert taken == ["align"] * 2 + ["ag_group_gemm", "reduce_rs"] * 2
+    for ctx in (c for pair in made for c in pair):
+        blocks, = ctx.joined.values()
+        assert blocks.block_size == 256 and blocks.tail_most > 0
+        at = (blocks.tail.padded - blocks.memory.data_ptr()) // 4
+        assert int(blocks.memory[at]) > 0 or _lib.load().tdist_num_cus() != 256
+    entry = torch.arange(W * mpr * topk, device=cuda)
+
+    def products(rows, w):
+        out = torch.empty((rows.shape[0], N), device=cuda)
+        for e in range(E):
+            of = entry[ids.view(-1) == e]
+            out[of] = rows[of].float() @ w[e].float()
+        return out
+
+    h = products(torch.cat([s.float() for s in shards]).repeat_interleave(topk, 0), up)
+    sums = (products(states, down).view(W * mpr, topk, N) * weight[:, :, None]).sum(1)[rank * mpr:(rank + 1) * mpr]
+    y = sum(t.float() for r, t in enumerate(partials) if r != rank) + sums
+    assert max(t.abs().max() for t in (h, sums, y)) <= 256   # every value is an integer that bf16 holds
+    for i in range(0, 6, 2):
+        assert torch.equal(a[i].float(), h) and torch.equal(a[i + 1].float(), y)
+
+
+@pytest.mark.gpu
+def test_modes(cuda, route):
+    """A mode that sees the calls of torch sees those of the Python code; states that change nothing for the call leave it to the module."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from triton_dist.kernels.amd import gqa_fwd_batch_decode
+    announce("torch calls, modes")
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = decode_inputs(cuda, (32, 8, 128, 128), torch.bfloat16)
+    want = gqa_fwd_batch_decode(x["q"], x["k"], x["v"], None, [1] * 3, x["lens"], x["table"], x["scale"], x["soft_cap"])
+
+    def f(mode):
+        def g():
+            with mode():
+                return gqa_fwd_batch_decode(x["q"], x["k"], x["v"], None, [1] * 3, x["lens"], x["table"], x["scale"], x["soft_cap"])
+        return g
+
+    for mode, by_module in ((Function, False), (Dispatch, False), (torch.inference_mode, True), (torch.no_grad, True), (torch.enable_grad, True),
+                            (lambda: torch.autocast("cuda"), True)):
+        a, b, taken = route(f(mode))
+        assert bool(taken) == by_module
+        assert a.is_inference() == b.is_inference()
+        with torch.inference_mode():
+            same(a, b)
+            same(a, want)
+
+
+@pytest.mark.gpu
+def test_captured(cuda, monkeypatch):
+    """Calls that the module takes while a graph is captured: every replay, on inputs that have changed, with eager calls between, against the
+    eager result."""
+    from triton_dist.kernels.amd import (ag_group_gemm_intra_node, create_ag_group_gemm_intra_node_context, create_all_to_all_context,
+                                         create_gemm_rs_intra_node_context, create_moe_rs_context, fast_all_to_all, gemm_rs_intra_node,
+                                         gqa_fwd_batch_decode, moe_reduce_rs, moe_weighted_combine, sort_topk_ids_align_block_size)
+    announce("torch calls, captured")
+    g, module = torch.Generator(device=cuda).manual_seed(13), _lib.native()
+    d = decode_inputs(cuda, (32, 8, 128, 128), torch.bfloat16)
+    T, topk, G, W, H = 48, 3, 16, 4, 1024
+    x, w = torch.randn((T, H), generator=g, device=cuda).bfloat16(), torch.rand((T, topk), generator=g, device=cuda)
+    ids = torch.rand((T, G), generator=g, device=cuda).topk(topk, dim=1).indices
+    contexts = [create_all_to_all_context(T * topk, H, 0, G, W, G // W) for _ in range(2)]
+    R, mpr, E, I, rank = 2, 24, 4, 192, 1
+    shards, logits = [torch.randn((mpr, 256), generator=g, device=cuda).bfloat16() for _ in range(R)], [torch.randn((mpr, E), generator=g, device=cuda) for _ in range(R)]
+    up, down = (torch.randn((E, *s), generator=g, device=cuda).bfloat16().transpose(1, 2) for s in ((I, 256), (256, I)))
+    rs = create_moe_rs_context(None, rank, R, R, R * mpr, 256, E, 2, torch.bfloat16, torch.bfloat16, cuda, 128, logits[rank], {0: logits[0]})
+    rs.set_peer_partials({0: torch.randn((mpr, 256), generator=g, device=cuda)})
+    ag = create_ag_group_gemm_intra_node_context(None, shards[rank], up, rs.precompute_ctx.full_topk_ids, E, max_M=R * mpr, rank=rank, num_ranks=R)
+    ag.set_peer_shards({0: shards[0]})
+    gemm = create_gemm_rs_intra_node_context(256, 512, torch.bfloat16, 1, 2, None)
+    gemm.set_peer_partials({0: torch.randn((128, 512), generator=g, device=cuda)})
+    a, b = (torch.randn(s, generator=g, device=cuda).bfloat16() for s in ((256, 256), (512, 256)))
+
+    def calls(ctx):
+        out = [gqa_fwd_batch_decode(d["q"], d["k"], d["v"], None, [1] * 3, d["lens"], d["table"], d["scale"], d["soft_cap"])]
+        splits, recv, _ = fast_all_to_all(ctx, x, None, None, expert_ids=ids)
+        _, cumsum, scatter, gather = ctx.last_index
+        out += [splits, cumsum, scatter, gather, moe_weighted_combine(ctx, recv, None, scatter, w, cumsum)]
+        rows, _, _, blocks, padded = sort_topk_ids_align_block_size(ids, G, W, T // W, 64)
+        h = ag_group_gemm_intra_node(shards[rank], up, ag)
+        return out + [rows, blocks, padded, h, moe_reduce_rs(rank, R, R, h, down, rs), gemm_rs_intra_node(a, b, gemm)]
+
+    for ctx in contexts:
+        calls(ctx)   # (what a context makes at its first call)
+    recorder = Recorder(module)
+    monkeypatch.setattr(_lib, "native", lambda: recorder)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = calls(contexts[0])
+    monkeypatch.setattr(_lib, "native", lambda: module)
+    assert recorder.taken == [(n, True) for n in ("decode", "dispatch_ids", "combine", "align", "ag_group_gemm", "reduce_rs", "gemm_rs")]
+    for turn in range(4):
+        for t in (d["q"], x, shards[rank], shards[0], a):
+            t.copy_(torch.randn(t.shape, generator=g, device=cuda))
+        ids.copy_(torch.rand((T, G), generator=g, device=cuda).topk(topk, dim=1).indices)
+        d["lens"].copy_(torch.tensor([turn, 128 - turn, 17 * turn], dtype=torch.int32))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        same(got, calls(contexts[1]))
+        torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_threads(cuda):
+    """Threads with contexts and streams of their own, their calls in flight together: the results of one thread alone."""
+    import threading
+
+    from triton_dist.kernels.amd import (create_all_to_all_context, fast_all_to_all, gqa_fwd_batch_decode, moe_weighted_combine,
+                                         sort_topk_ids_align_block_size)
+    announce("torch calls, threads")
+    T, topk, G, W, H = 64, 4, 16, 4, 512
+
+    def job(seed):
+        g = torch.Generator(device=cuda).manual_seed(seed)
+        d = decode_inputs(cuda, (32, 8, 128, 128), torch.bfloat16)
+        q = torch.randn(d["q"].shape, generator=g, device=cuda).bfloat16()
+        x, w = torch.randn((T, H), generator=g, device=cuda).bfloat16(), torch.rand((T, topk), generator=g, device=cuda)
+        ids = torch.rand((T, G), generator=g, device=cuda).topk(topk, dim=1).indices
+        ctx = create_all_to_all_context(T * topk, H, 0, G, W, G // W)
+
+        def calls():
+            out = [gqa_fwd_batch_decode(q, d["k"], d["v"], None, [1] * 3, d["lens"], d["table"], d["scale"], 0.0)]
+            splits, recv, _ = fast_all_to_all(ctx, x, None, None, expert_ids=ids)
+            _, cumsum, scatter, gather = ctx.last_index
+            out += [splits, cumsum, scatter, gather, moe_weighted_combine(ctx, recv, None, scatter, w, cumsum)]
+            rows, _, _, blocks, padded = sort_topk_ids_align_block_size(ids, G, W, T // W, 64)
+            return [t.clone() for t in out + [rows, blocks, padded]]
+        return calls
+
+    jobs = [job(seed) for seed in range(4)]
+    want = [calls() for calls in jobs]
+    torch.cuda.synchronize()
+    got, failed = [None] * len(jobs), []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                got[i] = [jobs[i]() for _ in range(20)]
+            stream.synchronize()
+        except Exception as e:   # (a thread's own exception would be lost)
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(i, )) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+    for i, results in enumerate(got):
+        for r in results:
+            same(r, want[i])
