@@ -44,6 +44,15 @@ def test_register_budget_guard():
         build._check_gemm_resources(report(LARGE_TILE, 140, 256, 0) + report(LARGE_TILE.replace("BF16N", "F16N"), 256, 256, 0))
 
 
+def test_small_tiles_spill_guard():
+    build = load_build()
+    name = "_ZN5tdist17gemm_small_kernelINS_9SmallBF16ELi128ELi128ELi4ELb0ELi3EEEvNS_15SmallGemmParamsE"
+    build._check_small_resources(report(name, 248, 0, 0))
+    build._check_small_resources(report(LARGE_TILE, 171, 256, 16))   # the other check's business
+    with pytest.raises(RuntimeError, match="spill"):
+        build._check_small_resources(report(name, 248, 0, 0) + report(name, 128, 128, 4))
+
+
 def test_producer_budget_guard():
     build = load_build()
     build._check_producer_resources(report(PRODUCER, 22, 0, 0))

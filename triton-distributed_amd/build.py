@@ -117,6 +117,14 @@ def _check_gemm_resources(report):
                            % (GEMM_REGISTER_BUDGET, "\n  ".join(offenders)))
 
 
+def _check_small_resources(report):
+    """Two workgroups of the small tiles share a compute unit: 256 registers to a lane, which the compiler keeps to by spilling."""
+    offenders = ["%s: %d bytes of scratch" % (name, scratch) for name, _, _, scratch in _resource_report(report)
+                 if "gemm_small_kernel" in name and scratch != 0]
+    if offenders:
+        raise RuntimeError("gemm_small.hip: instances that spill:\n  %s" % "\n  ".join(offenders))
+
+
 def _check_producer_resources(report):
     for name, vgprs, _, scratch in _resource_report(report):
         if "producer_push_kernel" in name and ((vgprs + 7) // 8 * 8 > PRODUCER_REGISTER_BUDGET or scratch != 0):
@@ -154,7 +162,7 @@ def _check_fixed_accumulators(asm_text):
 def _compile_one(hipcc, src, flags=None):
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
     cmd = [hipcc] + (flags or HIPCC_FLAGS) + ["-c", os.path.join(CSRC, src), "-o", obj]
-    if src in ("gemm.hip", "lib.hip"):
+    if src in ("gemm.hip", "gemm_small.hip", "lib.hip"):
         cmd += [_RESOURCE_FLAG, "-fno-caret-diagnostics"]   # (no source excerpt under each of the report's lines)
     if src == "gemm.hip":
         cmd += ["-save-temps=obj"]                          # keeps the device assembly next to the object
@@ -163,6 +171,8 @@ def _compile_one(hipcc, src, flags=None):
         _check_gemm_resources(res.stdout)
         with open(os.path.join(OBJ_DIR, "gemm-hip-amdgcn-amd-amdhsa-gfx950.s")) as f:
             _check_fixed_accumulators(f.read())
+    if res.returncode == 0 and src == "gemm_small.hip":
+        _check_small_resources(res.stdout)
     if res.returncode == 0 and src == "lib.hip":
         _check_producer_resources(res.stdout)
     # the host pass does not know the device-only target feature; that line is noise, and so is the resource report
