@@ -45,7 +45,7 @@ MEASURED_SOURCE_DIGEST = {
     "common.h": "f5b639d6f2c93627",
     "decode.hip": "86e8879aaf685690",
     "gather.h": "3fd5e450cd06de4d",
-    "gemm.hip": "72031edd6254e04a",
+    "gemm.hip": "bf653307ec066b7e",
     "gemm_small.h": "ceafc5b3b8b28bd1",
     "gemm_small.hip": "87b09035e69e02ec",
     "moe.hip": "d6426776d5a3636c",

@@ -127,6 +127,32 @@ def test_no_room_for_the_tails_places(cuda):
         assert all(torch.equal(x, y) for x, y in zip(a[:4], b[:4]))
 
 
+def test_a_second_list_that_is_refused_launches_nothing(cuda):
+    from triton_dist import _lib
+    announce("grouped GEMM with tails: refusals")
+    n, K, rows = 512, 256, 256
+    a, w = torch.ones((rows, K), dtype=torch.bfloat16, device=cuda), torch.ones((1, n, K), dtype=torch.bfloat16, device=cuda)
+    c = torch.full((rows, n), -3.0, dtype=torch.bfloat16, device=cuda)
+    ids, zero = torch.arange(rows, dtype=torch.int32, device=cuda), torch.zeros(64, dtype=torch.int32, device=cuda)
+    total = torch.full((1, ), rows, dtype=torch.int32, device=cuda)
+    z = zero.data_ptr()
+
+    def call(tail=(z, z, z, z), blocks=1, ldb=K):
+        return _lib.load().tdist_group_gemm_rows_tails(_lib.TDIST_BF16, _lib.address_table(a), 1, rows, w.data_ptr(), ldb, n * K, c.data_ptr(), n, n, K,
+                                                       ids.data_ptr(), z, z, total.data_ptr(), 1, 256, rows, 1, *tail, blocks, None, None, None, 0,
+                                                       _lib.stream_ptr())
+
+    for i in range(4):
+        assert call(tail=tuple(None if k == i else z for k in range(4))) == _lib.TDIST_ERR_INVALID
+    assert call(blocks=0) == _lib.TDIST_ERR_INVALID
+    assert call(ldb=1 << 21) == _lib.TDIST_ERR_UNSUPPORTED   # (4 MiB a row: an expert's weights would be 2 GiB)
+    torch.cuda.synchronize()
+    assert (c == -3).all()
+    assert call() == _lib.TDIST_OK
+    torch.cuda.synchronize()
+    assert (c == K).all()
+
+
 def test_what_the_join_with_tails_refuses(cuda):
     from triton_dist import _lib
     lib = _lib.load()

@@ -2492,12 +2492,16 @@ static int group_tail_rows(const GroupShape& g, int block, int cus) {
   return ceil_div(whole * cols, cus) < ceil_div(blocks * cols, cus) && 1.5 * used * share * ceil_div(g.N, 128) <= cus ? most : 0;
 }
 
+// Whether small tile t addresses such a product: an expert's weights, the entries' tokens and the grid.
+static bool small_tile_reaches(int t, int N, int64_t ldb, int esz, int num_valid, int topk, int num_blocks) {
+  return (int64_t)N * ldb * esz < (1ll << 31) && (int64_t)num_valid * topk < (1ll << 32) &&
+         (num_blocks * ceil_div(N, kSmallTiles[t].bn) + 8) * kSmallMaxSplits <= 0x7fffffff;
+}
 // The small tiles' plan for a call whose blocks have a small tile's rows (us = 0: it does not qualify).
 static SmallPlan group_small_plan(const GroupGemmCall& c, const GroupShape& g, int esz, int cus) {
   const int t = c.block_size == kSmallTiles[0].bm ? 0 : 1;
   if (kSmallTiles[t].bm != c.block_size || c.flags || c.A_local || (c.max_workgroups > 0 && c.max_workgroups < cus) ||
-      (int64_t)c.N * c.ldb * esz >= (1ll << 31) || (int64_t)c.num_valid * c.topk >= (1ll << 32) ||
-      (c.num_blocks * ceil_div(c.N, kSmallTiles[t].bn) + 8) * kSmallMaxSplits > 0x7fffffff) return {t, 0, 0, false, 0};
+      !small_tile_reaches(t, c.N, c.ldb, esz, c.num_valid, c.topk, c.num_blocks)) return {t, 0, 0, false, 0};
   return group_small_plan(g, t, c.num_blocks, c.sk_workspace ? c.sk_workspace_bytes : 0, cus);
 }
 
@@ -2922,6 +2926,12 @@ int tdist_group_gemm_rows_tails(int dtype, const void* const* shards, int world_
                                 const int32_t* tail_padded, int tail_blocks, int32_t* status, int32_t* first_error, void* sk_workspace,
                                 int64_t sk_workspace_bytes, void* stream) {
   const char* who = "tdist_group_gemm_rows_tails";
+  // (what the second launch would be refused for, before the first is made)
+  if (!tail_ids || !tail_experts || !tail_segments || !tail_padded) return fail(TDIST_ERR_INVALID, "%s: null pointer", who);
+  if (tail_blocks <= 0 || N <= 0) return fail(TDIST_ERR_INVALID, "%s: sizes must be positive", who);
+  if ((int64_t)tail_blocks * kGroupedFewRows > 0x7fffffff ||
+      !small_tile_reaches(0, N, ldb, dtype == TDIST_F8E4M3 ? 1 : 2, num_valid_tokens, topk, tail_blocks))
+    return fail(TDIST_ERR_UNSUPPORTED, "%s: blocks of %d rows take an expert's weights below 2 GiB", who, kGroupedFewRows);
   if (int rc = group_gemm_rows(who, 0, dtype, shards, world_size, rows_per_rank, B, ldb, expert_stride, C, ldc, N, K, sorted_token_ids, expert_ids,
                                block_barrier_ids, num_tokens_post_padded, num_blocks, block_size, num_valid_tokens, topk, status, first_error,
                                sk_workspace, sk_workspace_bytes, stream)) return rc;
