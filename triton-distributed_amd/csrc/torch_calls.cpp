@@ -449,6 +449,8 @@ bool int_is(PyObject* o, uintptr_t v) {
   return same;
 }
 
+// Places in AllToAllContext.halves: the halves, the buffers, their addresses, rows of a half and experts.
+enum Half { kHalfBufs = 2, kHalfAddresses = 5, kHalfRows = 8, kHalfExperts = 9, kHalfFields = 10 };
 struct Slots {
   int hidden, ele, max_m, world, per_rank, experts, calls, mod;
   c10::ScalarType type;
@@ -459,16 +461,16 @@ bool slots_of(PyObject* ctx, int device, Slots& s) {
       !get_int(ctx, kPerRank, &s.per_rank) || !get_int(ctx, kExperts, &s.experts) || !get_int(ctx, kCallCount, &s.calls) ||
       !get_int(ctx, kModValue, &s.mod) || s.mod <= 0 || s.calls < 0) return false;
   const Ref dtype(get(ctx, kDtype)), halves(get(ctx, kHalves));
-  if (!dtype.o || !THPDtype_Check(dtype) || !halves.o || !PyTuple_CheckExact(halves) || PyTuple_GET_SIZE(halves.o) != 10) return false;
+  if (!dtype.o || !THPDtype_Check(dtype) || !halves.o || !PyTuple_CheckExact(halves) || PyTuple_GET_SIZE(halves.o) != kHalfFields) return false;
   s.type = ((THPDtype*)dtype.o)->scalar_type;
   const Attr bufs[3] = {kSplitBuf, kRecvBuf, kScaleBuf};
   for (int i = 0; i < 3; ++i) {
     const Ref buf(get(ctx, bufs[i]));
-    if (!buf.o || buf != PyTuple_GET_ITEM(halves.o, 2 + i)) return false;
+    if (!buf.o || buf != PyTuple_GET_ITEM(halves.o, kHalfBufs + i)) return false;
     const at::Tensor* t = tensor_of(buf, device);
-    if (!t || !int_is(PyTuple_GET_ITEM(halves.o, 5 + i), (uintptr_t)t->data_ptr())) return false;
+    if (!t || !int_is(PyTuple_GET_ITEM(halves.o, kHalfAddresses + i), (uintptr_t)t->data_ptr())) return false;
   }
-  if (!int_is(PyTuple_GET_ITEM(halves.o, 8), (uintptr_t)s.world * s.max_m) || !int_is(PyTuple_GET_ITEM(halves.o, 9), s.experts)) return false;
+  if (!int_is(PyTuple_GET_ITEM(halves.o, kHalfRows), (uintptr_t)s.world * s.max_m) || !int_is(PyTuple_GET_ITEM(halves.o, kHalfExperts), s.experts)) return false;
   PyObject* const half = PyTuple_GET_ITEM(halves.o, s.calls % 2);
   if (!PyTuple_CheckExact(half) || PyTuple_GET_SIZE(half) != 3) return false;
   at::Tensor* const out[3] = {&s.splits, &s.recv, &s.scales};

@@ -95,6 +95,7 @@ class AllToAllContext:
         if not (h and h[2] is splits and h[3] is recv and h[4] is scales and h[5] == splits.data_ptr() and h[6] == recv.data_ptr()
                 and h[7] == scales.data_ptr() and h[8] == rows and h[9] == G):
             one, two = ((splits[i * G:(i + 1) * G], recv[i * rows:(i + 1) * rows], scales[i * rows:(i + 1) * rows]) for i in (0, 1))
+            # (read by place in csrc/torch_calls.cpp as well)
             h = self.halves = (one, two, splits, recv, scales, splits.data_ptr(), recv.data_ptr(), scales.data_ptr(), rows, G)
         splits, recv, scales = h[self.call_count % 2]
         return splits.detach(), recv.detach(), scales.detach()
